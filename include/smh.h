@@ -56,6 +56,10 @@ int smh_q40_quantize(const void *in, void *w, void *s, long groups, smh_stream_t
  * src_bf16 != 0 says they were bfloat16.  torch's roundings for those types: scale = fp16(T(absmax / 7)) with T the source
  * type, code = rint(x / scale) with the quotient in fp32. */
 int smh_q40_quantize_f32(const void *in, int src_bf16, void *w, void *s, long groups, smh_stream_t stream);
+/* smh_q40_quantize_t: quantize_q40 of the TRANSPOSE of a checkpoint weight in [N, K] (fp16_to_int4.py:173-176: v.t(), then
+ * groups of 64 along the outputs) in one pass, the bytes and scales smh_q40_quantize / smh_q40_quantize_f32 give for the
+ * transposed copy.  src_type 0: fp16, 1: bfloat16, 2: fp32, as the checkpoint holds it.  N % 128 == 0, any K. */
+int smh_q40_quantize_t(const void *in, int src_type, int N, int K, void *w, void *s, smh_stream_t stream);
 
 /* ---- Q4_0 matmul ---------------------------------------------------------------------------
  * c[M,N] = a[M,K] . deq(b_w, b_s)[K,N], fp16 operands, fp32 accumulation, one fp16 rounding;

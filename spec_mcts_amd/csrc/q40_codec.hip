@@ -3,6 +3,8 @@
 // Both kernels are pure streaming (HBM-bound): dequant reads 68 B and writes 256 B per row,
 // quantise reads 256 B and writes 68 B per row.  One lane owns 16 bytes of a row, so a row is
 // covered by 4 neighbouring lanes and every access is a 128-bit load/store.
+#include <type_traits>
+
 #include "q40_matmul.hpp"
 
 namespace smh {
@@ -49,6 +51,94 @@ __device__ __forceinline__ int q40_code(half_t x, float scale) {
     if (!(qf == qf)) return 0;
     return (int)__builtin_rintf(qf);
 }
+// ... of a value of a wider type: the quotient stays fp32
+__device__ __forceinline__ int q40_code_wide(float x, float scale) {
+    const float qf = x / scale;
+    return (qf == qf) ? (int)__builtin_rintf(qf) : 0;
+}
+
+// The same codes without a division per value.  For a group whose scale is a normal finite fp16 number, x * (1 / scale) in
+// fp32 lies within 2^-21 (relative) of the quotient and |quotient| < 8, so it rounds to the same code unless it lies that
+// close to a point where the code changes; such values (and groups with any other scale) take the division.  A division is
+// ~16 instructions of which two run at a quarter of the rate: a weight of 45 M values is 29 us of vector ALU with it, more
+// than its bytes cost.
+__device__ __forceinline__ bool q40_scale_is_plain(float scale) { return scale >= 6.103515625e-05f && scale <= 65504.0f; }
+// fp16 values: the code changes where the fp16 rounding of the quotient does, at midpoints between fp16 numbers - fp32 numbers
+// whose low 13 bits are 0x1000 (below 2^-14 the midpoints lie elsewhere, but there every code is 0)
+__device__ __forceinline__ int q40_code_near(half_t x, float inv, bool &doubt) {
+    const float q = (float)x * inv;
+    doubt = ((__builtin_bit_cast(uint32_t, q) + 0x1003u) & 0x1FFFu) <= 6u;
+    return (int)(short)__builtin_rintf16((half_t)q);
+}
+// fp32 quotients: the code changes at n + 1/2.  Adding 1.5 * 2^23 rounds to an integer that stands in the low bits of the sum.
+__device__ __forceinline__ int q40_code_near(float x, float inv, bool &doubt) {
+    constexpr float round = 12582912.0f;
+    const float t = __builtin_fmaf(x, inv, round), r = t - round;
+    doubt = fabsf(__builtin_fmaf(x, inv, -r)) > 0.5f - 7.62939453125e-06f;
+    return __builtin_bit_cast(int, t);
+}
+__device__ __forceinline__ int q40_code_exact(half_t x, float scale) { return q40_code(x, scale); }
+__device__ __forceinline__ int q40_code_exact(float x, float scale) { return q40_code_wide(x, scale); }
+
+// The codes of eight values; only the low four bits of each count.
+template <typename T>
+__device__ __forceinline__ void q40_codes8(const T (&x)[8], float scale, int (&code)[8]) {
+    if (q40_scale_is_plain(scale)) {
+        const float inv = 1.0f / scale;
+        bool doubt[8], any = false;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            code[i] = q40_code_near(x[i], inv, doubt[i]);
+            any |= doubt[i];
+        }
+        if (any) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (doubt[i]) code[i] = q40_code_exact(x[i], scale);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) code[i] = q40_code_exact(x[i], scale);
+    }
+}
+
+// codes of an even group (high nibbles) and of the odd group behind it (low nibbles) -> 4 bytes
+__device__ __forceinline__ uint32_t pack_codes4(int h0, int h1, int h2_, int h3, int l0, int l1, int l2, int l3) {
+    auto byte = [](int hi, int lo) { return ((uint32_t)hi << 4 & ~15u) | ((uint32_t)lo & 15u); };     // (bits above the byte: dropped below)
+    const uint32_t b01 = __builtin_amdgcn_perm(byte(h1, l1), byte(h0, l0), 0x0c0c0400u);
+    const uint32_t b23 = __builtin_amdgcn_perm(byte(h3, l3), byte(h2_, l2), 0x0c0c0400u);
+    return b01 | (b23 << 16);
+}
+__device__ __forceinline__ u32x2 pack_codes8(const int (&hi)[8], const int (&lo)[8]) {
+    return u32x2{pack_codes4(hi[0], hi[1], hi[2], hi[3], lo[0], lo[1], lo[2], lo[3]), pack_codes4(hi[4], hi[5], hi[6], hi[7], lo[4], lo[5], lo[6], lo[7])};
+}
+// eight codes -> value j in bits 4j .. 4j+3
+__device__ __forceinline__ uint32_t nibbles8(const int (&c)[8]) {
+    uint32_t v = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v |= (uint32_t)(c[j] & 15) << (4 * j);
+    return v;
+}
+__device__ __forceinline__ u32x2 pack_codes(uint32_t hi, uint32_t lo) {
+    uint32_t b0 = 0, b1 = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        b0 |= ((((hi >> (4 * j)) & 15) << 4) | ((lo >> (4 * j)) & 15)) << (8 * j);
+        b1 |= ((((hi >> (4 * j + 16)) & 15) << 4) | ((lo >> (4 * j + 16)) & 15)) << (8 * j);
+    }
+    return u32x2{b0, b1};
+}
+// largest value of the 8 lanes that share lane / 8
+__device__ __forceinline__ float max8(float v) {
+    v = fmaxf(v, dpp_move<DPP_QUAD_XOR1>(v));
+    v = fmaxf(v, dpp_move<DPP_QUAD_XOR2>(v));
+    return fmaxf(v, dpp_move<DPP_ROW_HALF_MIRROR>(v));
+}
+__device__ __forceinline__ uint32_t max8(uint32_t v) {       // (bit patterns below 2^31: compared as integers)
+    v = max(v, __builtin_bit_cast(uint32_t, dpp_move<DPP_QUAD_XOR1>(__builtin_bit_cast(float, v))));
+    v = max(v, __builtin_bit_cast(uint32_t, dpp_move<DPP_QUAD_XOR2>(__builtin_bit_cast(float, v))));
+    return max(v, __builtin_bit_cast(uint32_t, dpp_move<DPP_ROW_HALF_MIRROR>(__builtin_bit_cast(float, v))));
+}
 
 // Lane layout: 8 lanes per 64-value group (8 values = one 128-bit load each), so a wave covers
 // 8 groups = 4 packed rows.  absmax is reduced over the 8 lanes of a group with xor-shuffles.
@@ -75,28 +165,19 @@ __global__ __launch_bounds__(256) void q40_quantize_kernel(const u32x4 *__restri
         uint32_t m = max(a & 0xFFFFu, a >> 16);
         amax = max(amax, m);
     }
-#pragma unroll
-    for (int o = 4; o > 0; o >>= 1) amax = max(amax, (uint32_t)__shfl_xor((int)amax, o, 64));
+    amax = max8(amax);
     half_t amax_h = __builtin_bit_cast(half_t, (uint16_t)amax);
     half_t scale_h = (half_t)((float)amax_h / 7.0f);
     float scale = (float)scale_h;
-    uint32_t nib = 0;   // 8 codes, value j in bits 4j..4j+3
-#pragma unroll
-    for (int j = 0; j < 8; ++j) nib |= (uint32_t)(q40_code(x[j], scale) & 15) << (4 * j);
+    int code[8];
+    q40_codes8(x, scale, code);
+    const uint32_t nib = nibbles8(code);
     // the partner group (g ^ 1) sits 8 lanes away; even groups supply high nibbles
     uint32_t other = (uint32_t)__shfl_xor((int)nib, 8, 64);
     if (!live) return;
     if (c == 0) s[g] = scale_h;
     if ((g & 1) == 0) {
-        uint32_t hi = nib, lo = other;
-        uint32_t b0 = 0, b1 = 0;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            b0 |= ((((hi >> (4 * j)) & 15) << 4) | ((lo >> (4 * j)) & 15)) << (8 * j);
-            b1 |= ((((hi >> (4 * j + 16)) & 15) << 4) | ((lo >> (4 * j + 16)) & 15)) << (8 * j);
-        }
-        u32x2 *dst = reinterpret_cast<u32x2 *>(w + (g >> 1) * 64 + c * 8);
-        *dst = u32x2{b0, b1};
+        *reinterpret_cast<u32x2 *>(w + (g >> 1) * 64 + c * 8) = pack_codes(nib, other);
     }
 }
 
@@ -122,31 +203,115 @@ __global__ __launch_bounds__(256) void q40_quantize_f32_kernel(const f4 *__restr
     float amax = 0.f;
 #pragma unroll
     for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(x[j]));
-#pragma unroll
-    for (int o = 4; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+    amax = max8(amax);
     float q7 = amax / 7.0f;
     if (SRC_BF16) q7 = round_to_bf16(q7);
     const half_t scale_h = (half_t)q7;
     const float scale = (float)scale_h;
-    uint32_t nib = 0;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const float qf = x[j] / scale;
-        const int code = (qf == qf) ? (int)__builtin_rintf(qf) : 0;
-        nib |= (uint32_t)(code & 15) << (4 * j);
-    }
+    int code[8];
+    q40_codes8(x, scale, code);
+    const uint32_t nib = nibbles8(code);
     uint32_t other = (uint32_t)__shfl_xor((int)nib, 8, 64);
     if (!live) return;
     if (c == 0) s[g] = scale_h;
     if ((g & 1) == 0) {
-        uint32_t hi = nib, lo = other;
-        uint32_t b0 = 0, b1 = 0;
+        *reinterpret_cast<u32x2 *>(w + (g >> 1) * 64 + c * 8) = pack_codes(nib, other);
+    }
+}
+
+// ---- a checkpoint's linear weight [N, K] -> Q4_0 of its transpose, in one pass ------------------------------------------------
+// A workgroup takes 128 outputs n x 64 inputs k.  The tile is read along k (whole cache lines, 16 bytes a lane), turned in LDS
+// and quantised along n: eight lanes share input column k (two columns at a time for 16-bit types), lane o holding outputs
+// 8 o .. 8 o + 7 of either group of 64, so a lane's codes are 8 consecutive bytes of packed row (k, n / 128).
+// Neighbouring blocks of 128 outputs (halves of one 128-byte line of codes, parts of one line of scales) go to one XCD, one
+// after the other, so that its L2 joins them.  Bound by HBM (2 or 4 bytes read, 17/32 written per value) and the vector ALU.
+// Measured at 11008 x 4096: bfloat16 31 us (3.7 TB/s), fp16 38, fp32 52; rows of odd length the same.  A transposed copy, a
+// widened copy (bfloat16) and the flat quantiser in its place: 372 us for bfloat16.
+//   SRC 0: fp16, 1: bfloat16, 2: fp32.  P: dwords of an LDS row, odd so that the eight rows a wave reads at a time are 8 P = 8
+// (mod 64) banks apart.
+template <int SRC>
+__global__ __launch_bounds__(256) void q40_quantize_t_kernel(const uint8_t *__restrict__ in, int N, int K, uint8_t *__restrict__ w,
+                                                             half_t *__restrict__ s, int k_tiles) {
+    constexpr int ES = SRC == 2 ? 4 : 2;                     // bytes of a source value
+    constexpr int P = SRC == 2 ? 65 : 33;
+    __shared__ uint32_t tile[128 * P];
+    const int tid = threadIdx.x;
+    const int n_blocks = N / 128;
+    const long total = (long)n_blocks * k_tiles, per = (total + 7) / 8;
+    const long id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((long)(blockIdx.x >> 3) >= per || id >= total) return;
+    const int nb = (int)(id % n_blocks), k0 = (int)(id / n_blocks) * 64;
+    {
+        constexpr int VEC = 16 / ES;                         // values of a load
+        constexpr int LPR = 64 / VEC;                        // lanes a row
+        const int c = tid % LPR, r0 = tid / LPR;
+        const int k = k0 + c * VEC;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            b0 |= ((((hi >> (4 * j)) & 15) << 4) | ((lo >> (4 * j)) & 15)) << (8 * j);
-            b1 |= ((((hi >> (4 * j + 16)) & 15) << 4) | ((lo >> (4 * j + 16)) & 15)) << (8 * j);
+        for (int i = 0; i < 128 / (256 / LPR); ++i) {
+            const int r = r0 + i * (256 / LPR);
+            const uint8_t *src = in + ((long)(nb * 128 + r) * K + k) * ES;
+            uint32_t v[4] = {0, 0, 0, 0};
+            if (k + VEC <= K) {
+                __builtin_memcpy(v, src, 16);                // (rows of an odd K start at any multiple of the value's size)
+            } else {
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) {
+                    if (k + e >= K) continue;
+                    if constexpr (ES == 4) v[e] = *reinterpret_cast<const uint32_t *>(src + 4 * e);
+                    else v[e / 2] |= (uint32_t)*reinterpret_cast<const uint16_t *>(src + 2 * e) << (16 * (e & 1));
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) tile[r * P + 4 * c + q] = v[q];
         }
-        *reinterpret_cast<u32x2 *>(w + (g >> 1) * 64 + c * 8) = u32x2{b0, b1};
+    }
+    __syncthreads();
+    constexpr int KL = SRC == 2 ? 1 : 2;                     // input columns per LDS dword
+    const int o = tid & 7;
+#pragma unroll
+    for (int rep = 0; rep < 2 / KL; ++rep) {
+        const int kc = (tid >> 3) + 32 * rep;                // dword column
+        uint32_t d[2][8];
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) d[g][i] = tile[(64 * g + 8 * o + i) * P + kc];
+#pragma unroll
+        for (int h = 0; h < KL; ++h) {
+            const int k = k0 + KL * kc + h;
+            int code[2][8];
+            half_t sc[2];
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                std::conditional_t<SRC == 0, half_t, float> x[8];
+                float amax = 0.f;
+                if constexpr (SRC == 0) {
+                    uint32_t abits = 0;                      // |x| as a bit pattern: integer order is magnitude order
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        const uint32_t b = h == 0 ? d[g][i] & 0xFFFFu : d[g][i] >> 16;
+                        abits = max(abits, b & 0x7FFFu);
+                        x[i] = __builtin_bit_cast(half_t, (uint16_t)b);
+                    }
+                    amax = (float)__builtin_bit_cast(half_t, (uint16_t)max8(abits));
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        if constexpr (SRC == 1) x[i] = __builtin_bit_cast(float, h == 0 ? d[g][i] << 16 : d[g][i] & 0xFFFF0000u);
+                        else x[i] = __builtin_bit_cast(float, d[g][i]);
+                        amax = fmaxf(amax, fabsf(x[i]));
+                    }
+                    amax = max8(amax);
+                }
+                float q7 = amax / 7.0f;
+                if constexpr (SRC == 1) q7 = round_to_bf16(q7);
+                sc[g] = (half_t)q7;
+                q40_codes8(x, (float)sc[g], code[g]);
+            }
+            if (k >= K) continue;
+            *reinterpret_cast<u32x2 *>(w + ((long)k * n_blocks + nb) * 64 + 8 * o) = pack_codes8(code[0], code[1]);
+            if (o == 0) *reinterpret_cast<h2 *>(s + ((long)k * n_blocks + nb) * 2) = h2{sc[0], sc[1]};
+        }
     }
 }
 
@@ -326,5 +491,19 @@ extern "C" int smh_q40_quantize_f32(const void *in, int src_bf16, void *w, void 
     dim3 grid((unsigned)((threads + 255) / 256));
     if (src_bf16) hipLaunchKernelGGL(q40_quantize_f32_kernel<true>, grid, dim3(256), 0, (hipStream_t)stream, (const f4 *)in, (uint8_t *)w, (half_t *)s, groups);
     else hipLaunchKernelGGL(q40_quantize_f32_kernel<false>, grid, dim3(256), 0, (hipStream_t)stream, (const f4 *)in, (uint8_t *)w, (half_t *)s, groups);
+    return launch_status();
+}
+
+extern "C" int smh_q40_quantize_t(const void *in, int src_type, int N, int K, void *w, void *s, smh_stream_t stream) {
+    using namespace smh;
+    SMH_REQUIRE(src_type >= 0 && src_type <= 2, "smh_q40_quantize_t: src_type=%d (0 fp16, 1 bfloat16, 2 fp32)", src_type);
+    SMH_REQUIRE(N > 0 && N % 128 == 0 && K > 0, "smh_q40_quantize_t: N=%d (a positive multiple of 128) K=%d", N, K);
+    SMH_REQUIRE(in && w && s && ((uintptr_t)in & (src_type == 2 ? 3 : 1)) == 0 && ((uintptr_t)w & 7) == 0 && ((uintptr_t)s & 3) == 0,
+                "smh_q40_quantize_t: null or misaligned pointer");
+    const int k_tiles = (K + 63) / 64;
+    const long blocks = ((long)(N / 128) * k_tiles + 7) / 8 * 8;
+    SMH_REQUIRE(blocks < (1L << 31), "smh_q40_quantize_t: N=%d K=%d is too large for one launch", N, K);
+    const auto kern = src_type == 0 ? q40_quantize_t_kernel<0> : src_type == 1 ? q40_quantize_t_kernel<1> : q40_quantize_t_kernel<2>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, (const uint8_t *)in, N, K, (uint8_t *)w, (half_t *)s, k_tiles);
     return launch_status();
 }

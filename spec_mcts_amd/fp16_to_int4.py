@@ -106,13 +106,16 @@ def iter_checkpoint_tensors(model_dir: str):
 
 
 def quantize_linear_weight_gpu(v: torch.Tensor, device="cuda:0"):
-    """quantize_linear_weight on the GPU: the weight goes to the device in its own dtype, is transposed there and quantised
-    by the HIP kernel for that dtype (same bytes as the host quantiser).  Returns device tensors (w, s, shape)."""
+    """quantize_linear_weight on the GPU: the weight goes to the device in its own dtype, where one kernel transposes and
+    quantises it (same bytes as the host quantiser).  Returns device tensors (w, s, shape)."""
     from . import kernels as K
     if v.dim() != 2 or v.shape[0] % 128 != 0:
         raise ValueError(f"out_features must be a multiple of 128, got {tuple(v.shape)}")
-    vt = v.to(device).t().contiguous()
-    w, s = K.quantize_q40(vt, GROUP_SIZE)
+    v = v.to(device)
+    if v.dtype in K._SRC_TYPES and v.shape[1] > 0:
+        w, s = K.quantize_q40_t(v)
+    else:
+        w, s = K.quantize_q40(v.t().contiguous(), GROUP_SIZE)
     return w, s, torch.Size(v.shape)
 
 

@@ -440,6 +440,22 @@ def quantize_q40(w: torch.Tensor, group_size: int = GROUP_SIZE) -> Tuple[torch.T
     return quantize_q40_torch(w, group_size)
 
 
+_SRC_TYPES = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}
+
+
+def quantize_q40_t(v: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
+    """quantize_q40(v.t().contiguous()) for a checkpoint weight v [N, K] (fp16, bfloat16 or fp32) on the GPU, in one pass over v."""
+    lib = _lib.load()
+    _need_gpu(v)
+    assert v.dim() == 2 and v.shape[0] % 128 == 0 and v.dtype in _SRC_TYPES
+    v = v.contiguous()
+    N, Kd = v.shape
+    q = torch.empty((N * Kd // 128, 64), device=v.device, dtype=torch.int8)
+    s = torch.empty((N * Kd // 64, 1), device=v.device, dtype=torch.float16)
+    check(lib.smh_q40_quantize_t(v.data_ptr(), _SRC_TYPES[v.dtype], N, Kd, q.data_ptr(), s.data_ptr(), _stream()), "smh_q40_quantize_t")
+    return q, s
+
+
 dequantize_q40 = deq_int40
 triton_deq_int40 = deq_int40      # the reference's name for the same operator
 triton_q_int40 = q_int40

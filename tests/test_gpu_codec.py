@@ -82,3 +82,23 @@ def test_quantize_dispatch_host_tensor():
     w, s = K.quantize_q40(x, 64)
     w2, s2 = O.quantize_q40(x, 64)
     assert torch.equal(w, w2) and torch.equal(s, s2)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,Kd", [(128, 1), (128, 63), (256, 64), (384, 65), (640, 200), (1024, 129)])
+def test_quantize_of_the_transpose_matches_the_oracle(dtype, N, Kd):
+    """edges of the 128 x 64 tile, rows of odd length, zero groups, subnormal and infinite scales, quotients at rounding ties"""
+    from spec_mcts_amd import kernels as K
+    g = torch.Generator().manual_seed(N + Kd)
+    v = torch.randn((N, Kd), generator=g) * 0.02
+    v[:64, 0] = 0
+    v[64:128, -1] *= 1e-4
+    v[:17, Kd // 2] = torch.tensor([7.0, 0.5, -0.5, 1.5, -1.5, 2.5, -2.5, 3.5, 6.5, -6.5, 4.5, 5.5, 2.4995, 2.5005, 1.4995, 1.5005, 0.50012])
+    v[17:64, Kd // 2] = 0
+    v = v.to(dtype)
+    if dtype != torch.float16 and Kd > 2:
+        v[70, 1] = 1e6                                    # the scale overflows fp16
+    w_want, s_want = O.quantize_q40(v.t().contiguous(), 64)
+    w_got, s_got = K.quantize_q40_t(v.cuda())
+    assert np.array_equal(_bits(s_got).reshape(-1), _bits(s_want).reshape(-1))
+    assert torch.equal(w_got.cpu(), w_want)
