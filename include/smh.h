@@ -385,6 +385,44 @@ int smh_shared_prefix_attn_qkv(const void *qkv_partial, int ksplit, void *out, i
                                const int32_t *t_dev, const int32_t *pages, int pages_stride, int single_launch,
                                void *workspace, size_t workspace_bytes, smh_stream_t stream);
 
+/* ---- a transformer layer of a decode step in one call ----------------------------------------------------------------
+ * TransformerBlock.forward (hf_model_q40_kv_shared.py:439-467) for one token per branch, on tiled weights: the launches of
+ * the operators above in the order the model issues them, without the host work between them.
+ *   smh_layer   one layer: sizes, norms, tiled weights (smh_q40_tile), prompt K/V (prompt_len rows) and Q4_0 suffix caches
+ *   smh_pass    one pass over all layers: `rows` branches, the step's tables and counters as smh_shared_prefix_attn_qkv takes
+ *               them, pages (NULL, or int32 [rows, pages_stride] over cache_rows cache rows), the switches (rows up to which
+ *               RMSNorm / SiLU are made inside the linear that follows, 0 = never; SwiGLU inside w1|w3; attention from the
+ *               q|k|v product; attention in one launch), the workspaces of smh_shared_prefix_attn and of its one-launch form,
+ *               and `scratch` of smh_decode_scratch_bytes(layer, rows) bytes.
+ *               In and out: h, the residual stream [rows, dim] (the embeddings before the first layer; the calls leave it at
+ *               a buffer inside scratch), and pending, 0 before the first layer.
+ *   smh_decode_finish   what follows the last layer: the residual add of its w2 and the final RMSNorm (:505-507). */
+typedef struct smh_layer {
+    int dim, ffn, heads, kv_heads;
+    float att_eps, ffn_eps;
+    const void *att_norm, *ffn_norm;
+    const void *wq, *wk, *wv, *wo, *w1, *w2, *w3;
+    void *prompt_k, *prompt_v;
+    void *cache_k, *cache_ks, *cache_v, *cache_vs;
+    int prompt_len;
+} smh_layer;
+typedef struct smh_pass {
+    int rows, smax, pages_stride;
+    int norm_in_rows, silu_in_rows, swiglu_in, attn_from_qkv, attn_one;
+    long cache_rows;
+    const void *cos_tab, *sin_tab;
+    const int32_t *pos_dev, *t_dev, *pages;
+    void *attn_ws, *attn_one_ws;
+    size_t attn_ws_bytes, attn_one_ws_bytes;
+    void *scratch;
+    size_t scratch_bytes;
+    void *h;
+    int pending;
+} smh_pass;
+size_t smh_decode_scratch_bytes(const smh_layer *layer, int rows);
+int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stream_t stream);
+int smh_decode_finish(const smh_layer *last, smh_pass *pass, const void *norm_weight, float eps, void *out, smh_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

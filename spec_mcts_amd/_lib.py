@@ -17,6 +17,23 @@ SMH_KV_NONE, SMH_KV_FP16, SMH_KV_Q40 = 0, 1, 2
 SMH_GEMV_MAX_M = 16
 
 _P = c_void_p
+
+
+class SmhLayer(ctypes.Structure):
+    """smh_layer of include/smh.h"""
+    _fields_ = ([(n, c_int) for n in ("dim", "ffn", "heads", "kv_heads")] + [(n, c_float) for n in ("att_eps", "ffn_eps")]
+                + [(n, _P) for n in ("att_norm", "ffn_norm", "wq", "wk", "wv", "wo", "w1", "w2", "w3", "prompt_k", "prompt_v",
+                                     "cache_k", "cache_ks", "cache_v", "cache_vs")] + [("prompt_len", c_int)])
+
+
+class SmhPass(ctypes.Structure):
+    """smh_pass of include/smh.h"""
+    _fields_ = ([(n, c_int) for n in ("rows", "smax", "pages_stride", "norm_in_rows", "silu_in_rows", "swiglu_in", "attn_from_qkv", "attn_one")]
+                + [("cache_rows", c_long)] + [(n, _P) for n in ("cos_tab", "sin_tab", "pos_dev", "t_dev", "pages", "attn_ws", "attn_one_ws")]
+                + [(n, c_size_t) for n in ("attn_ws_bytes", "attn_one_ws_bytes")] + [("scratch", _P), ("scratch_bytes", c_size_t), ("h", _P), ("pending", c_int)])
+
+
+_LAYER, _PASS = ctypes.POINTER(SmhLayer), ctypes.POINTER(SmhPass)
 # name -> (restype, argtypes); must list every symbol of include/smh.h
 SIGNATURES = {
     "smh_version": (c_int, []),
@@ -79,6 +96,9 @@ SIGNATURES = {
     "smh_paged_prefix_attn": (c_int, [_P, _P, c_int, c_int, c_int, c_int, _P, _P, c_int, c_long, c_long,
                                       c_int, _P, _P, _P, _P, c_long, c_long, c_long, _P, c_int, c_long, c_int, _P, c_int, _P, _P, c_int,
                                       _P, c_size_t, _P]),
+    "smh_decode_scratch_bytes": (c_size_t, [_LAYER, c_int]),
+    "smh_decode_layer": (c_int, [_LAYER, _PASS, _P]),
+    "smh_decode_finish": (c_int, [_LAYER, _PASS, _P, c_float, _P, _P]),
     "smh_page_fork": (c_int, [_P, c_int, c_long, c_int, c_int, c_int, c_int, _P]),
 }
 

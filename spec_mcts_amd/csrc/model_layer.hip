@@ -1,0 +1,141 @@
+// One transformer layer of a decode step as ONE host call.
+//
+// Issued operator by operator from Python a decode layer costs ~90 us of host time (eight or nine operators, each with its
+// checks, its output tensors and a foreign call), which at one branch is more than the GPU needs for it: a step of the
+// 32-layer model took 3.0 ms where a captured graph of the same launches takes 2.0.  Here the layer's launches are issued one
+// behind the other (2-3 us each), out of buffers the caller allocated once for the whole pass.  The sequence, the operators
+// and their switches are those of Transformer._forward_fused in hf_model_q40_kv_shared.py.
+#include "smh_common.hpp"
+
+namespace smh {
+
+constexpr size_t align_up(size_t n) { return (n + 255) & ~(size_t)255; }
+
+// Buffers of a pass over `rows` rows, carved out of one allocation.
+struct LayerBuffers {
+    char *h[2], *xn, *q, *k, *v, *att, *act;   // fp16; the residual stream moves from one h to the other at every norm
+    float *sums, *slab_a, *slab_b;             // slabs of wq|wk|wv and w1|w3 (a), of wo and w2 (b)
+    size_t slab_a_bytes, slab_b_bytes, total;
+};
+
+static int slices(int M, int K, int nseg, const int *n) { return smh_q40_matmul_plan_tiled(M, K, nseg, n); }
+
+static int layer_buffers(const smh_layer &L, int M, char *base, LayerBuffers &b) {
+    const int nq = L.heads * 128, nkv = L.kv_heads * 128;
+    const int n_qkv[3] = {nq, nkv, nkv}, n_gu[2] = {L.ffn, L.ffn}, n_dim[1] = {L.dim};
+    const int ks_qkv = slices(M, L.dim, 3, n_qkv), ks_gu = slices(M, L.dim, 2, n_gu), ks_o = slices(M, nq, 1, n_dim), ks_d = slices(M, L.ffn, 1, n_dim);
+    if (ks_qkv < 1 || ks_gu < 1 || ks_o < 1 || ks_d < 1) return -1;
+    const size_t m = (size_t)M;
+    auto most = [](size_t x, size_t y) { return x > y ? x : y; };
+    b.slab_a_bytes = align_up(most(ks_qkv * m * (nq + 2 * (size_t)nkv), ks_gu * m * 2 * (size_t)L.ffn) * sizeof(float));
+    b.slab_b_bytes = align_up((size_t)most(ks_o, ks_d) * m * L.dim * sizeof(float));
+    size_t at = 0;
+    auto take = [&](size_t bytes) { char *p = base ? base + at : nullptr; at += align_up(bytes); return p; };
+    b.h[0] = take(m * L.dim * 2);
+    b.h[1] = take(m * L.dim * 2);
+    b.xn = take(m * L.dim * 2);
+    b.q = take(m * nq * 2);
+    b.k = take(m * nkv * 2);
+    b.v = take(m * nkv * 2);
+    b.att = take(m * nq * 2);
+    b.act = take(m * L.ffn * 2);
+    b.sums = (float *)take(m * 16 * sizeof(float));
+    b.slab_a = (float *)take(b.slab_a_bytes);
+    b.slab_b = (float *)take(b.slab_b_bytes);
+    b.total = at;
+    return 0;
+}
+
+}  // namespace smh
+
+using namespace smh;
+
+extern "C" size_t smh_decode_scratch_bytes(const smh_layer *layer, int rows) {
+    LayerBuffers b;
+    if (layer == nullptr || rows < 1 || layer_buffers(*layer, rows, nullptr, b) != 0) return 0;
+    return b.total;
+}
+
+extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stream_t stream) {
+    const char *who = "smh_decode_layer";
+    SMH_REQUIRE(layer && pass && pass->h, "%s: null pointer", who);
+    const smh_layer &L = *layer;
+    smh_pass &S = *pass;
+    const int M = S.rows, nq = L.heads * 128, nkv = L.kv_heads * 128;
+    SMH_REQUIRE(M >= 1 && L.heads > 0 && L.kv_heads > 0 && L.heads % L.kv_heads == 0, "%s: rows=%d heads=%d kv_heads=%d", who, M, L.heads, L.kv_heads);
+    LayerBuffers b;
+    if (layer_buffers(L, M, (char *)S.scratch, b) != 0) return -1;
+    SMH_REQUIRE(S.scratch && S.scratch_bytes >= b.total, "%s: scratch %zu < %zu bytes", who, S.scratch_bytes, b.total);
+    const int n_qkv[3] = {nq, nkv, nkv}, n_gu[2] = {L.ffn, L.ffn}, n_dim[1] = {L.dim};
+    const void *w_qkv[3] = {L.wq, L.wk, L.wv}, *w_o[1] = {L.wo}, *w_gu[2] = {L.w1, L.w3}, *w_d[1] = {L.w2};
+    int st = 0;
+    // S.h += the product of the linear before (S.pending slabs in slab_b), then its RMSNorm: to b.xn
+    auto norm = [&](const void *weight, float eps) -> int {
+        void *h_out = S.pending > 0 ? b.h[S.h == b.h[0]] : nullptr;
+        const int r = smh_partial_rmsnorm(S.pending > 0 ? b.slab_b : nullptr, S.pending > 0 ? S.pending : 1, M, L.dim, S.h, weight, eps, h_out, b.xn, stream);
+        if (h_out != nullptr) S.h = h_out;
+        S.pending = 0;
+        return r;
+    };
+    // ... and the linears behind it: to slab_a.  With few rows the RMSNorm is made inside the linears' launch.
+    auto norm_linears = [&](const void *weight, float eps, int nseg, const void *const *w, const int *n) -> int {
+        if (S.pending == 0 || M > S.norm_in_rows || smh_q40_norm_in_fits(M, L.dim, nseg, n) != 1) {
+            if (int r = norm(weight, eps)) return r;
+            return smh_q40_matmul_partial_tiled(b.xn, M, L.dim, L.dim, nseg, w, n, b.slab_a, b.slab_a_bytes, stream);
+        }
+        void *h_out = b.h[S.h == b.h[0]];
+        if (int r = smh_partial_residual_sumsq(b.slab_b, S.pending, M, L.dim, S.h, h_out, b.sums, stream)) return r;
+        S.h = h_out;
+        S.pending = 0;
+        return smh_q40_matmul_partial_tiled_norm(h_out, L.dim, b.sums, weight, eps, M, L.dim, nseg, w, n, b.slab_a, b.slab_a_bytes, stream);
+    };
+    // ---- attention ----
+    if ((st = norm_linears(L.att_norm, L.att_eps, 3, w_qkv, n_qkv))) return st;
+    const int ks_qkv = slices(M, L.dim, 3, n_qkv), rep = L.heads / L.kv_heads;
+    const int one = S.attn_one != 0 && M * rep <= 16;
+    void *ws = one ? S.attn_one_ws : S.attn_ws;
+    const size_t ws_bytes = one ? S.attn_one_ws_bytes : S.attn_ws_bytes;
+    if (S.attn_from_qkv != 0 && M <= SMH_GEMV_MAX_M && M * rep <= 128) {
+        st = smh_shared_prefix_attn_qkv(b.slab_a, ks_qkv, b.att, M, L.heads, L.kv_heads, 128, S.cos_tab, S.sin_tab, S.pos_dev, L.prompt_k, L.prompt_v,
+                                        L.prompt_len, L.cache_k, L.cache_ks, L.cache_v, L.cache_vs, S.smax, S.t_dev, S.pages, S.pages_stride, one, ws,
+                                        ws_bytes, stream);
+    } else {
+        st = smh_partial_rope_append_kv(b.slab_a, ks_qkv, M, L.heads, L.kv_heads, 128, b.q, b.k, b.v, S.cos_tab, S.sin_tab, S.pos_dev, L.cache_k,
+                                        L.cache_ks, L.cache_v, L.cache_vs, S.smax, S.t_dev, stream);
+        if (st == 0 && S.pages != nullptr)
+            st = smh_paged_prefix_attn(b.q, b.att, M, L.heads, L.kv_heads, 128, L.prompt_k, L.prompt_v, L.prompt_len, 0, 0, SMH_KV_Q40, L.cache_k,
+                                       L.cache_v, L.cache_ks, L.cache_vs, 0, 0, S.cache_rows, S.pages, 4, S.pages_stride, S.pages_stride, S.t_dev, 0,
+                                       b.k, b.v, one, ws, ws_bytes, stream);
+        else if (st == 0)
+            st = (one ? smh_shared_prefix_attn_one : smh_shared_prefix_attn)(b.q, b.att, M, L.heads, L.kv_heads, 128, L.prompt_k, L.prompt_v, L.prompt_len,
+                                                                             SMH_KV_Q40, L.cache_k, L.cache_v, L.cache_ks, L.cache_vs, S.smax, S.t_dev, 0,
+                                                                             b.k, b.v, ws, ws_bytes, stream);
+    }
+    if (st) return st;
+    if ((st = smh_q40_matmul_partial_tiled(b.att, M, nq, nq, 1, w_o, n_dim, b.slab_b, b.slab_b_bytes, stream))) return st;
+    S.pending = slices(M, nq, 1, n_dim);
+    // ---- feed forward ----
+    if (S.swiglu_in != 0 && smh_q40_swiglu_fits(M, L.dim, L.ffn)) {
+        if ((st = norm(L.ffn_norm, L.ffn_eps))) return st;
+        if ((st = smh_q40_matmul_tiled_swiglu(b.xn, M, L.dim, L.dim, L.w1, L.w3, L.ffn, b.act, L.ffn, stream))) return st;
+        st = smh_q40_matmul_partial_tiled(b.act, M, L.ffn, L.ffn, 1, w_d, n_dim, b.slab_b, b.slab_b_bytes, stream);
+    } else {
+        if ((st = norm_linears(L.ffn_norm, L.ffn_eps, 2, w_gu, n_gu))) return st;
+        const int ks_gu = slices(M, L.dim, 2, n_gu);
+        if (M <= S.silu_in_rows && L.ffn % 32 == 0)
+            st = smh_q40_matmul_partial_tiled_silu(b.slab_a, ks_gu, M, L.ffn, 1, w_d, n_dim, b.slab_b, b.slab_b_bytes, stream);
+        else if ((st = smh_partial_silu_mul(b.slab_a, ks_gu, M, L.ffn, b.act, stream)) == 0)
+            st = smh_q40_matmul_partial_tiled(b.act, M, L.ffn, L.ffn, 1, w_d, n_dim, b.slab_b, b.slab_b_bytes, stream);
+    }
+    S.pending = slices(M, L.ffn, 1, n_dim);
+    return st;
+}
+
+// The last layer's product added to the residual stream, and the final RMSNorm -> out [rows, dim].
+extern "C" int smh_decode_finish(const smh_layer *last, smh_pass *pass, const void *norm_weight, float eps, void *out, smh_stream_t stream) {
+    SMH_REQUIRE(last && pass && pass->h && out, "smh_decode_finish: null pointer");
+    LayerBuffers b;
+    if (layer_buffers(*last, pass->rows, (char *)pass->scratch, b) != 0) return -1;
+    return smh_partial_rmsnorm(pass->pending > 0 ? b.slab_b : nullptr, pass->pending > 0 ? pass->pending : 1, pass->rows, last->dim, pass->h, norm_weight,
+                               eps, nullptr, out, stream);
+}

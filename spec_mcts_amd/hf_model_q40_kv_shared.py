@@ -276,6 +276,8 @@ class TransformerBlock(nn.Module):
         self.layer_id = layer_id
         self.attention_norm = RMSNorm(args.dim, eps=args.norm_eps)
         self.ffn_norm = RMSNorm(args.dim, eps=args.norm_eps)
+        self.native = None            # Transformer._layer_struct
+        self.native_key = None
 
     def forward(self, x, start_pos, freqs_cis, mask, step_state=None, pages=None):
         # the residual adds are fused into the epilogues of wo and w2
@@ -361,6 +363,9 @@ class Transformer(nn.Module):
         bsz, seqlen = tokens.shape
         M = bsz * seqlen
         p = self.params
+        if start_pos != 0 and self.tiled_weights:
+            assert seqlen == 1, "decode steps take one token per branch"
+            return self._decode(tokens, step_state)
         h = K.embedding(tokens, self.tok_embeddings.weight).view(M, p.dim)
         cos, sin = self._tables(h.device)
         pending = None                      # product of the previous layer's w2, not yet added to h
@@ -431,6 +436,45 @@ class Transformer(nn.Module):
                 pending = K.matmul_q40_partial(act, [ff.w2.operand(tiled)])
         _, hn = K.partial_rmsnorm(pending, h, self.norm.weight, self.norm.eps, want_h=False)
         return self._lm_head(hn.view(bsz, seqlen, p.dim))
+
+    def _decode(self, tokens: torch.Tensor, step_state) -> torch.Tensor:
+        """A decode step on tiled weights: the launches of _forward_fused, a layer per library call (smh_decode_layer) instead of
+        an operator per call - at a few branches the host, not the GPU, is what the operators' way waits for."""
+        p = self.params
+        B = tokens.shape[0]
+        h = K.embedding(tokens, self.tok_embeddings.weight)
+        dev = h.device
+        cos, sin = self._tables(dev)
+        pages = self._pages(dev)
+        att0 = self.layers[0].attention
+        H, rep, P = att0.n_local_heads, att0.n_rep, att0.cache_prompt_len
+        one = self.attn_single_launch and B * rep <= 16
+        ws = K.attn_qkv_workspace(dev, B, H, P) if one else K.attn_workspace(dev, B, H, P)
+        d = K.DecodePass(self._layer_struct(self.layers[0]), B, h, cos, sin, step_state, ws, bool(one))
+        norm_in = self._norm_in(B, p.dim, [lin._tiled for lin in (att0.wq, att0.wk, att0.wv)])      # (the library asks again, launch by launch)
+        d.set(smax=p.max_seq_len, cache_rows=p.max_batch_size * p.max_seq_len, pages=pages, norm_in_rows=B if norm_in else 0,
+              silu_in_rows=K.SILU_IN_MAX_M if self.silu_in_matmul else 0, swiglu_in=self.swiglu_in_matmul,
+              attn_from_qkv=self.attn_from_qkv and not self.per_branch_kv)
+        for layer in self.layers:
+            s = self._layer_struct(layer)
+            d.layer(s)
+        return self._lm_head(d.finish(s, self.norm.weight, self.norm.eps).view(B, 1, p.dim))
+
+    def _layer_struct(self, layer):
+        """What smh_decode_layer reads of a layer, rebuilt when any of its tensors is another one than at the last step."""
+        att, ff = layer.attention, layer.feed_forward
+        lins = (att.wq, att.wk, att.wv, att.wo, ff.w1, ff.w2, ff.w3)
+        key = [att.cache_prompt_len, layer.attention_norm.weight.data_ptr(), layer.ffn_norm.weight.data_ptr(), att.cache_prompt_k.data_ptr(),
+               att.cache_prompt_v.data_ptr(), att.cache_k.data_ptr(), att.cache_k_s.data_ptr(), att.cache_v.data_ptr(), att.cache_v_s.data_ptr()]
+        for lin in lins:
+            key += (lin.w.data_ptr(), lin.s.data_ptr(), id(lin._tiled))
+        if layer.native is None or layer.native_key != key:
+            layer.native = K.layer_struct(self.params.dim, att.n_local_heads, att.n_local_kv_heads, layer.attention_norm.weight, layer.attention_norm.eps,
+                                          layer.ffn_norm.weight, layer.ffn_norm.eps, [lin.operand(True) for lin in lins], att.cache_prompt_k,
+                                          att.cache_prompt_v, att.cache_prompt_len, att.cache_k, att.cache_k_s, att.cache_v, att.cache_v_s)
+            key[9:] = [x for lin in lins for x in (lin.w.data_ptr(), lin.s.data_ptr(), id(lin._tiled))]
+            layer.native_key = key
+        return layer.native
 
     def quantize_lm_head(self, enable: bool = True):
         """Optional: run the vocabulary projection as a Q4_0 matmul.  The reference keeps `output` in fp16 because its format

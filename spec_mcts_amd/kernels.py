@@ -707,6 +707,79 @@ def embedding(tokens: torch.Tensor, table: torch.Tensor) -> torch.Tensor:
 
 
 # ---------------------------------------------------------------------------------------------
+# a decode step, layer by layer
+# ---------------------------------------------------------------------------------------------
+def layer_struct(dim: int, H: int, Hkv: int, att_norm: torch.Tensor, att_eps: float, ffn_norm: torch.Tensor, ffn_eps: float, tiled: Sequence[TiledQ40],
+                 prompt_k: torch.Tensor, prompt_v: torch.Tensor, prompt_len: int, cache_k: torch.Tensor, cache_ks: torch.Tensor,
+                 cache_v: torch.Tensor, cache_vs: torch.Tensor) -> "_lib.SmhLayer":
+    """smh_layer of one transformer layer; `tiled`: wq, wk, wv, wo, w1, w2, w3.  The caller keeps the tensors alive."""
+    wq, wk, wv, wo, w1, w2, w3 = tiled
+    ffn, D = w1.N, 128
+    assert all(isinstance(t, TiledQ40) for t in tiled)
+    assert [(t.K, t.N) for t in tiled] == [(dim, H * D), (dim, Hkv * D), (dim, Hkv * D), (H * D, dim), (dim, ffn), (ffn, dim), (dim, ffn)]
+    _need_gpu(att_norm, ffn_norm, prompt_k, prompt_v, cache_k, cache_ks, cache_v, cache_vs, *(t.buf for t in tiled))
+    for t in (att_norm, ffn_norm):
+        assert t.numel() == dim and t.dtype == torch.float16 and t.is_contiguous()
+    for t in (prompt_k, prompt_v):
+        assert t.is_contiguous() and t.dtype == torch.float16 and prompt_len * Hkv * D <= t.numel()
+    assert cache_k.dtype == torch.int8 and cache_v.dtype == torch.int8 and cache_ks.dtype == torch.float16 and cache_vs.dtype == torch.float16
+    assert cache_k.is_contiguous() and cache_v.is_contiguous() and cache_ks.is_contiguous() and cache_vs.is_contiguous()
+    s = _lib.SmhLayer()
+    s.dim, s.ffn, s.heads, s.kv_heads, s.att_eps, s.ffn_eps, s.prompt_len = dim, ffn, H, Hkv, att_eps, ffn_eps, prompt_len
+    s.att_norm, s.ffn_norm = att_norm.data_ptr(), ffn_norm.data_ptr()
+    s.wq, s.wk, s.wv, s.wo, s.w1, s.w2, s.w3 = (t.buf.data_ptr() for t in tiled)
+    s.prompt_k, s.prompt_v = prompt_k.data_ptr(), prompt_v.data_ptr()
+    s.cache_k, s.cache_ks, s.cache_v, s.cache_vs = cache_k.data_ptr(), cache_ks.data_ptr(), cache_v.data_ptr(), cache_vs.data_ptr()
+    return s
+
+
+class DecodePass:
+    """One decode step over `rows` branches (smh_pass): layer(struct) per layer, then finish() for the last residual add and the
+    final RMSNorm.  `h`: the embeddings [rows, dim]; `step_state`: (position, suffix index) on the device; `ws`: the workspace of
+    the attention (of its one-launch form with `one_launch`).  All other buffers are one allocation that lives as long as this."""
+
+    def __init__(self, first: "_lib.SmhLayer", rows: int, h: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, step_state, ws: torch.Tensor, one_launch: bool):
+        self.lib = _lib.load()
+        pos_dev, t_dev = step_state
+        _need_gpu(h, cos, sin, pos_dev, t_dev, ws)
+        assert h.dtype == torch.float16 and h.is_contiguous() and h.numel() == rows * first.dim
+        assert pos_dev.dtype == torch.int32 and t_dev.dtype == torch.int32
+        nbytes = int(self.lib.smh_decode_scratch_bytes(first, rows))
+        if nbytes == 0:
+            check(-1, "smh_decode_scratch_bytes")
+        self.scratch = torch.empty(nbytes, dtype=torch.uint8, device=h.device)
+        self.h, self.ws = h, ws
+        p = self.p = _lib.SmhPass()
+        p.rows, p.cos_tab, p.sin_tab, p.pos_dev, p.t_dev = rows, cos.data_ptr(), sin.data_ptr(), pos_dev.data_ptr(), t_dev.data_ptr()
+        if one_launch:
+            p.attn_one, p.attn_one_ws, p.attn_one_ws_bytes = 1, ws.data_ptr(), ws.numel()
+        else:
+            p.attn_ws, p.attn_ws_bytes = ws.data_ptr(), ws.numel()
+        p.scratch, p.scratch_bytes, p.h = self.scratch.data_ptr(), nbytes, h.data_ptr()
+        self.stream = _stream()
+
+    def set(self, smax: int, cache_rows: int, pages: Optional[torch.Tensor], norm_in_rows: int, silu_in_rows: int, swiglu_in: bool, attn_from_qkv: bool) -> None:
+        p = self.p
+        p.smax, p.cache_rows, p.norm_in_rows, p.silu_in_rows = smax, cache_rows, norm_in_rows, silu_in_rows
+        p.swiglu_in, p.attn_from_qkv = int(bool(swiglu_in)), int(bool(attn_from_qkv))
+        if pages is not None:
+            assert pages.is_cuda and pages.dtype == torch.int32 and pages.dim() == 2 and pages.stride(1) == 1
+            assert pages.shape[0] >= p.rows and pages.shape[1] >= smax
+            p.pages, p.pages_stride = pages.data_ptr(), pages.stride(0)
+
+    def layer(self, s: "_lib.SmhLayer") -> None:
+        st = self.lib.smh_decode_layer(s, self.p, self.stream)
+        if st:
+            check(st, "smh_decode_layer")
+
+    def finish(self, last: "_lib.SmhLayer", weight: torch.Tensor, eps: float) -> torch.Tensor:
+        assert weight.numel() == last.dim and weight.dtype == torch.float16
+        out = torch.empty((self.p.rows, last.dim), dtype=torch.float16, device=self.h.device)
+        check(self.lib.smh_decode_finish(last, self.p, weight.data_ptr(), float(eps), out.data_ptr(), self.stream), "smh_decode_finish")
+        return out
+
+
+# ---------------------------------------------------------------------------------------------
 # attention
 # ---------------------------------------------------------------------------------------------
 def shared_prefix_attn(q: torch.Tensor, prefix_k: Optional[torch.Tensor], prefix_v: Optional[torch.Tensor], P: int,
