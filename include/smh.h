@@ -123,11 +123,17 @@ int smh_q40_matmul_plan_tiled(int M, int K, int nseg, const int *n);
  * [K, n_half] - `F.silu(self.w1(x)) * self.w3(x)` of FeedForward.forward (hf_model_q40_kv_shared.py:434) in ONE launch, with
  * the roundings of smh_q40_matmul_partial_tiled + smh_partial_silu_mul (every linear rounded to fp16 first) and no slab
  * in between.  17 <= M <= 128, K a multiple of 64, n_half a multiple of 128 and at most 16384 (all of K in one workgroup,
- * one workgroup per compute unit).  smh_q40_swiglu_fits: 1 when the shape is supported AND wide enough (n_half >= 8192) for
+ * one workgroup per compute unit); or M > 128, K a multiple of 32, n_half a multiple of 128.  smh_q40_swiglu_fits: 1 when the shape is supported AND wide enough (n_half >= 8192) for
  * this to be the faster way; else use the two launches. */
 int smh_q40_swiglu_fits(int M, int K, int n_half);
 int smh_q40_matmul_tiled_swiglu(const void *a, int M, int K, long lda, const void *tiled_gate, const void *tiled_up, int n_half,
                                 void *out, long ldo, smh_stream_t stream);
+/* smh_q40_matmul_tiled_direct: LinearQ4_0.forward (:228-236) of up to 3 tiled weights that share the input, for more than 128
+ * rows whose launch needs no K-split (smh_q40_matmul_tiled_direct_fits: 1 / 0): out[i][M, n[i]] = fp16(a . w_i), contiguous
+ * and 16-byte aligned; with a residual [M, ldr] (one weight only) out = fp16(residual + fp16(a . w)).  No slabs. */
+int smh_q40_matmul_tiled_direct_fits(int M, int K, int nseg, const int *n);
+int smh_q40_matmul_tiled_direct(const void *a, int M, int K, long lda, int nseg, const void *const *tiled, const int *n, void *const *out,
+                                const void *residual, long ldr, smh_stream_t stream);
 int smh_q40_matmul_partial(const void *a, int M, int K, long lda, int nseg, const void *const *w,
                            const void *const *s, const int *n, void *partial, size_t partial_bytes,
                            smh_stream_t stream);
@@ -167,6 +173,10 @@ int smh_partial_reduce(const void *partial, int ksplit, int M, int n_total, int 
 int smh_partial_rmsnorm(const void *partial, int ksplit, int M, int N, const void *h_in,
                         const void *weight, float eps, void *h_out, void *xn_out, smh_stream_t stream);
 int smh_partial_silu_mul(const void *partial, int ksplit, int M, int n_half, void *out, smh_stream_t stream);
+/* smh_partial_rope_rows: the same for a prompt: row s of the product is token s at position pos0 + s; q [S,H,D], k, v [S,Hkv,D]
+ * (rows of the fp16 prompt cache, :320-324), nothing quantised */
+int smh_partial_rope_rows(const void *partial, int ksplit, int S, int H, int Hkv, int D, void *q, void *k, void *v, const void *cos_tab,
+                          const void *sin_tab, int pos0, smh_stream_t stream);
 int smh_partial_rope_append_kv(const void *partial, int ksplit, int B, int H, int Hkv, int D,
                                void *q, void *k, void *v, const void *cos_tab, const void *sin_tab,
                                const int32_t *pos_dev, void *cache_k, void *cache_ks, void *cache_v,
@@ -393,9 +403,12 @@ int smh_shared_prefix_attn_qkv(const void *qkv_partial, int ksplit, void *out, i
  *               them, pages (NULL, or int32 [rows, pages_stride] over cache_rows cache rows), the switches (rows up to which
  *               RMSNorm / SiLU are made inside the linear that follows, 0 = never; SwiGLU inside w1|w3; attention from the
  *               q|k|v product; attention in one launch), the workspaces of smh_shared_prefix_attn and of its one-launch form,
- *               and `scratch` of smh_decode_scratch_bytes(layer, rows) bytes.
+ *               and `scratch` of smh_decode_scratch_bytes(layer, rows, swiglu_in) bytes.
  *               In and out: h, the residual stream [rows, dim] (the embeddings before the first layer; the calls leave it at
  *               a buffer inside scratch), and pending, 0 before the first layer.
+ *   smh_prefill_layer   the same block for a prompt of `rows` tokens at start_pos 0 (:499-504): k and v become rows 0 .. rows-1 of
+ *               the layer's prompt cache (prompt_len is not read).  Of the pass it needs rows, the tables, scratch, swiglu_in, h
+ *               and pending.
  *   smh_decode_finish   what follows the last layer: the residual add of its w2 and the final RMSNorm (:505-507). */
 typedef struct smh_layer {
     int dim, ffn, heads, kv_heads;
@@ -419,8 +432,9 @@ typedef struct smh_pass {
     void *h;
     int pending;
 } smh_pass;
-size_t smh_decode_scratch_bytes(const smh_layer *layer, int rows);
+size_t smh_decode_scratch_bytes(const smh_layer *layer, int rows, int swiglu_in);
 int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stream_t stream);
+int smh_prefill_layer(const smh_layer *layer, smh_pass *pass, smh_stream_t stream);
 int smh_decode_finish(const smh_layer *last, smh_pass *pass, const void *norm_weight, float eps, void *out, smh_stream_t stream);
 
 #ifdef __cplusplus

@@ -96,7 +96,11 @@ SIGNATURES = {
     "smh_paged_prefix_attn": (c_int, [_P, _P, c_int, c_int, c_int, c_int, _P, _P, c_int, c_long, c_long,
                                       c_int, _P, _P, _P, _P, c_long, c_long, c_long, _P, c_int, c_long, c_int, _P, c_int, _P, _P, c_int,
                                       _P, c_size_t, _P]),
-    "smh_decode_scratch_bytes": (c_size_t, [_LAYER, c_int]),
+    "smh_decode_scratch_bytes": (c_size_t, [_LAYER, c_int, c_int]),
+    "smh_prefill_layer": (c_int, [_LAYER, _PASS, _P]),
+    "smh_q40_matmul_tiled_direct_fits": (c_int, [c_int, c_int, c_int, _P]),
+    "smh_q40_matmul_tiled_direct": (c_int, [_P, c_int, c_int, c_long, c_int, _P, _P, _P, _P, c_long, _P]),
+    "smh_partial_rope_rows": (c_int, [_P, c_int, c_int, c_int, c_int, c_int, _P, _P, _P, _P, _P, c_int, _P]),
     "smh_decode_layer": (c_int, [_LAYER, _PASS, _P]),
     "smh_decode_finish": (c_int, [_LAYER, _PASS, _P, c_float, _P, _P]),
     "smh_page_fork": (c_int, [_P, c_int, c_long, c_int, c_int, c_int, c_int, _P]),

@@ -1,4 +1,4 @@
-// One transformer layer of a decode step as ONE host call.
+// One transformer layer of a decode step or of a prefill as ONE host call.
 //
 // Issued operator by operator from Python a decode layer costs ~90 us of host time (eight or nine operators, each with its
 // checks, its output tensors and a foreign call), which at one branch is more than the GPU needs for it: a step of the
@@ -20,14 +20,16 @@ struct LayerBuffers {
 
 static int slices(int M, int K, int nseg, const int *n) { return smh_q40_matmul_plan_tiled(M, K, nseg, n); }
 
-static int layer_buffers(const smh_layer &L, int M, char *base, LayerBuffers &b) {
+static int layer_buffers(const smh_layer &L, int M, bool swiglu_in, char *base, LayerBuffers &b) {
     const int nq = L.heads * 128, nkv = L.kv_heads * 128;
     const int n_qkv[3] = {nq, nkv, nkv}, n_gu[2] = {L.ffn, L.ffn}, n_dim[1] = {L.dim};
     const int ks_qkv = slices(M, L.dim, 3, n_qkv), ks_gu = slices(M, L.dim, 2, n_gu), ks_o = slices(M, nq, 1, n_dim), ks_d = slices(M, L.ffn, 1, n_dim);
     if (ks_qkv < 1 || ks_gu < 1 || ks_o < 1 || ks_d < 1) return -1;
     const size_t m = (size_t)M;
     auto most = [](size_t x, size_t y) { return x > y ? x : y; };
-    b.slab_a_bytes = align_up(most(ks_qkv * m * (nq + 2 * (size_t)nkv), ks_gu * m * 2 * (size_t)L.ffn) * sizeof(float));
+    // (above 128 rows w1|w3 leaves no slabs where SwiGLU is made inside its launch: 4 bytes x rows x 2 ffn less)
+    const bool gu_slabs = !(M > 128 && swiglu_in && smh_q40_swiglu_fits(M, L.dim, L.ffn));
+    b.slab_a_bytes = align_up(most(ks_qkv * m * (nq + 2 * (size_t)nkv), gu_slabs ? ks_gu * m * 2 * (size_t)L.ffn : 0) * sizeof(float));
     b.slab_b_bytes = align_up((size_t)most(ks_o, ks_d) * m * L.dim * sizeof(float));
     size_t at = 0;
     auto take = [&](size_t bytes) { char *p = base ? base + at : nullptr; at += align_up(bytes); return p; };
@@ -50,9 +52,9 @@ static int layer_buffers(const smh_layer &L, int M, char *base, LayerBuffers &b)
 
 using namespace smh;
 
-extern "C" size_t smh_decode_scratch_bytes(const smh_layer *layer, int rows) {
+extern "C" size_t smh_decode_scratch_bytes(const smh_layer *layer, int rows, int swiglu_in) {
     LayerBuffers b;
-    if (layer == nullptr || rows < 1 || layer_buffers(*layer, rows, nullptr, b) != 0) return 0;
+    if (layer == nullptr || rows < 1 || layer_buffers(*layer, rows, swiglu_in != 0, nullptr, b) != 0) return 0;
     return b.total;
 }
 
@@ -64,7 +66,7 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
     const int M = S.rows, nq = L.heads * 128, nkv = L.kv_heads * 128;
     SMH_REQUIRE(M >= 1 && L.heads > 0 && L.kv_heads > 0 && L.heads % L.kv_heads == 0, "%s: rows=%d heads=%d kv_heads=%d", who, M, L.heads, L.kv_heads);
     LayerBuffers b;
-    if (layer_buffers(L, M, (char *)S.scratch, b) != 0) return -1;
+    if (layer_buffers(L, M, S.swiglu_in != 0, (char *)S.scratch, b) != 0) return -1;
     SMH_REQUIRE(S.scratch && S.scratch_bytes >= b.total, "%s: scratch %zu < %zu bytes", who, S.scratch_bytes, b.total);
     const int n_qkv[3] = {nq, nkv, nkv}, n_gu[2] = {L.ffn, L.ffn}, n_dim[1] = {L.dim};
     const void *w_qkv[3] = {L.wq, L.wk, L.wv}, *w_o[1] = {L.wo}, *w_gu[2] = {L.w1, L.w3}, *w_d[1] = {L.w2};
@@ -131,11 +133,67 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
     return st;
 }
 
+// One layer of a prefill of `rows` tokens (TransformerBlock.forward with start_pos == 0): k and v go straight to the prompt cache.
+// Above 128 rows the linears store their fp16 results themselves wherever their launch needs no K-split (the residual adds of
+// wo and w2 inside), and SiLU(gate) * up is made inside w1|w3's launch.
+extern "C" int smh_prefill_layer(const smh_layer *layer, smh_pass *pass, smh_stream_t stream) {
+    const char *who = "smh_prefill_layer";
+    SMH_REQUIRE(layer && pass && pass->h, "%s: null pointer", who);
+    const smh_layer &L = *layer;
+    smh_pass &S = *pass;
+    const int M = S.rows, nq = L.heads * 128, nkv = L.kv_heads * 128;
+    SMH_REQUIRE(M >= 1 && L.heads > 0 && L.kv_heads > 0 && L.heads % L.kv_heads == 0, "%s: rows=%d heads=%d kv_heads=%d", who, M, L.heads, L.kv_heads);
+    LayerBuffers b;
+    if (layer_buffers(L, M, S.swiglu_in != 0, (char *)S.scratch, b) != 0) return -1;
+    SMH_REQUIRE(S.scratch && S.scratch_bytes >= b.total, "%s: scratch %zu < %zu bytes", who, S.scratch_bytes, b.total);
+    const int n_qkv[3] = {nq, nkv, nkv}, n_gu[2] = {L.ffn, L.ffn}, n_dim[1] = {L.dim};
+    const void *w_qkv[3] = {L.wq, L.wk, L.wv}, *w_o[1] = {L.wo}, *w_gu[2] = {L.w1, L.w3}, *w_d[1] = {L.w2};
+    int st = 0;
+    auto norm = [&](const void *weight, float eps) -> int {
+        void *h_out = S.pending > 0 ? b.h[S.h == b.h[0]] : nullptr;
+        const int r = smh_partial_rmsnorm(S.pending > 0 ? b.slab_b : nullptr, S.pending > 0 ? S.pending : 1, M, L.dim, S.h, weight, eps, h_out, b.xn, stream);
+        if (h_out != nullptr) S.h = h_out;
+        S.pending = 0;
+        return r;
+    };
+    // S.h += x . w, at once or as slabs that the next norm adds
+    auto residual_linear = [&](const void *x, int K, const void *const *w) -> int {
+        if (smh_q40_matmul_tiled_direct_fits(M, K, 1, n_dim) == 1) {
+            void *out[1] = {b.h[S.h == b.h[0]]};
+            const int r = smh_q40_matmul_tiled_direct(x, M, K, K, 1, w, n_dim, out, S.h, L.dim, stream);
+            S.h = out[0];
+            return r;
+        }
+        S.pending = slices(M, K, 1, n_dim);
+        return smh_q40_matmul_partial_tiled(x, M, K, K, 1, w, n_dim, b.slab_b, b.slab_b_bytes, stream);
+    };
+    if ((st = norm(L.att_norm, L.att_eps))) return st;
+    if (smh_q40_matmul_tiled_direct_fits(M, L.dim, 3, n_qkv) == 1) {
+        void *out[3] = {b.q, L.prompt_k, L.prompt_v};
+        if ((st = smh_q40_matmul_tiled_direct(b.xn, M, L.dim, L.dim, 3, w_qkv, n_qkv, out, nullptr, 0, stream))) return st;
+        st = smh_rope(b.q, L.prompt_k, M, L.heads, L.kv_heads, 128, S.cos_tab, S.sin_tab, 0, stream);
+    } else {
+        if ((st = smh_q40_matmul_partial_tiled(b.xn, M, L.dim, L.dim, 3, w_qkv, n_qkv, b.slab_a, b.slab_a_bytes, stream))) return st;
+        st = smh_partial_rope_rows(b.slab_a, slices(M, L.dim, 3, n_qkv), M, L.heads, L.kv_heads, 128, b.q, L.prompt_k, L.prompt_v, S.cos_tab, S.sin_tab, 0,
+                                   stream);
+    }
+    if (st) return st;
+    if ((st = smh_prefill_attn(b.q, L.prompt_k, L.prompt_v, b.att, M, L.heads, L.kv_heads, 128, stream))) return st;
+    if ((st = residual_linear(b.att, nq, w_o))) return st;
+    if ((st = norm(L.ffn_norm, L.ffn_eps))) return st;
+    if (S.swiglu_in != 0 && smh_q40_swiglu_fits(M, L.dim, L.ffn)) {
+        st = smh_q40_matmul_tiled_swiglu(b.xn, M, L.dim, L.dim, L.w1, L.w3, L.ffn, b.act, L.ffn, stream);
+    } else if ((st = smh_q40_matmul_partial_tiled(b.xn, M, L.dim, L.dim, 2, w_gu, n_gu, b.slab_a, b.slab_a_bytes, stream)) == 0) {
+        st = smh_partial_silu_mul(b.slab_a, slices(M, L.dim, 2, n_gu), M, L.ffn, b.act, stream);
+    }
+    return st ? st : residual_linear(b.act, L.ffn, w_d);
+}
+
 // The last layer's product added to the residual stream, and the final RMSNorm -> out [rows, dim].
 extern "C" int smh_decode_finish(const smh_layer *last, smh_pass *pass, const void *norm_weight, float eps, void *out, smh_stream_t stream) {
     SMH_REQUIRE(last && pass && pass->h && out, "smh_decode_finish: null pointer");
     LayerBuffers b;
-    if (layer_buffers(*last, pass->rows, (char *)pass->scratch, b) != 0) return -1;
+    if (layer_buffers(*last, pass->rows, pass->swiglu_in != 0, (char *)pass->scratch, b) != 0) return -1;
     return smh_partial_rmsnorm(pass->pending > 0 ? b.slab_b : nullptr, pass->pending > 0 ? pass->pending : 1, pass->rows, last->dim, pass->h, norm_weight,
                                eps, nullptr, out, stream);
 }

@@ -220,6 +220,34 @@ __global__ __launch_bounds__(256) void partial_rope_append_kernel(const void *__
     }
 }
 
+// A prefill's q|k|v product -> q, and k, v as rows of the prompt cache (fp16): sums, one rounding, RoPE of q and k at position
+// row + pos0.  One thread owns four rotation pairs (d .. d+3, d+64 ..) of one head.
+__global__ __launch_bounds__(256) void partial_rope_rows_kernel(const void *__restrict__ partial, int ksplit, int S, int H, int Hkv,
+                                                                half_t *__restrict__ q, half_t *__restrict__ k, half_t *__restrict__ v,
+                                                                const half_t *__restrict__ cos_tab, const half_t *__restrict__ sin_tab, int pos0) {
+    const int heads = H + 2 * Hkv, s = blockIdx.y;
+    const int item = blockIdx.x * 256 + threadIdx.x, h = item >> 4, d = 4 * (item & 15);
+    if (h >= heads) return;
+    const int n_total = heads * 128;
+    const long at = (long)s * n_total + h * 128 + d, slab = (long)S * n_total;
+    const f4 lo = slab_sum4(partial, at, slab, ksplit), hi = slab_sum4(partial, at + 64, slab, ksplit);
+    h4 x1, x2;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) { x1[j] = (half_t)lo[j]; x2[j] = (half_t)hi[j]; }
+    if (h < H + Hkv) {
+        const h4 cs = *reinterpret_cast<const h4 *>(cos_tab + (long)(pos0 + s) * 64 + d), sn = *reinterpret_cast<const h4 *>(sin_tab + (long)(pos0 + s) * 64 + d);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            half_t a = x1[j], b = x2[j];
+            rope_pair2(a, b, cs[j], sn[j]);
+            x1[j] = a; x2[j] = b;
+        }
+    }
+    half_t *dst = h < H ? q + ((long)s * H + h) * 128 : h < H + Hkv ? k + ((long)s * Hkv + h - H) * 128 : v + ((long)s * Hkv + h - H - Hkv) * 128;
+    *reinterpret_cast<h4 *>(dst + d) = x1;
+    *reinterpret_cast<h4 *>(dst + 64 + d) = x2;
+}
+
 }  // namespace smh
 
 using namespace smh;
@@ -258,17 +286,45 @@ extern "C" int smh_q40_matmul_tiled_swiglu(const void *a, int M, int K, long lda
                                            void *out, long ldo, smh_stream_t stream) {
     const char *who = "smh_q40_matmul_tiled_swiglu";
     SMH_REQUIRE(gemm_swiglu_fits(M, K, n_half, false),
-                "%s: M=%d (17 .. 128) K=%d (a multiple of 64) n_half=%d (a multiple of 128, at most 16384)", who, M, K, n_half);
+                "%s: M=%d (17 .. 128) K=%d (a multiple of 64) n_half=%d (a multiple of 128, at most 16384); or M above 128 and K a multiple of 32", who, M, K, n_half);
     SMH_REQUIRE(a && tiled_gate && tiled_up && out, "%s: null pointer", who);
-    SMH_REQUIRE(lda >= K && lda % 8 == 0 && ldo >= n_half && ldo % 2 == 0, "%s: lda=%ld (>= K, a multiple of 8) ldo=%ld (>= n_half, even)", who, lda, ldo);
-    SMH_REQUIRE(((uintptr_t)a & 15) == 0 && ((uintptr_t)out & 3) == 0 && ((uintptr_t)tiled_gate & 127) == 0 && ((uintptr_t)tiled_up & 127) == 0,
+    SMH_REQUIRE(lda >= K && lda % 8 == 0 && ldo >= n_half && ldo % (M > 128 ? 4 : 2) == 0, "%s: lda=%ld (>= K, a multiple of 8) ldo=%ld (>= n_half, even; above 128 rows a multiple of 4)", who, lda, ldo);
+    SMH_REQUIRE(((uintptr_t)a & 15) == 0 && ((uintptr_t)out & (M > 128 ? 7 : 3)) == 0 && ((uintptr_t)tiled_gate & 127) == 0 && ((uintptr_t)tiled_up & 127) == 0,
                 "%s: misaligned pointer", who);
     MatmulParams p = MatmulParams{};
     p.a = (const half_t *)a; p.M = M; p.K = K; p.lda = lda; p.nseg = 2;
     p.seg[0].w = (const uint8_t *)tiled_gate; p.seg[0].N = n_half;
     p.seg[1].w = (const uint8_t *)tiled_up; p.seg[1].N = n_half;
-    p.c = (half_t *)out; p.ldc = ldo; p.tiled = 1;
-    return gemm_swiglu_launch(p, (hipStream_t)stream);
+    p.c = p.seg[0].c = (half_t *)out; p.ldc = p.seg[0].ldc = ldo; p.tiled = 1;
+    return M > 128 ? gemm_swiglu_rows_launch(p, (hipStream_t)stream) : gemm_swiglu_launch(p, (hipStream_t)stream);
+}
+
+extern "C" int smh_q40_matmul_tiled_direct_fits(int M, int K, int nseg, const int *n) {
+    MatmulParams p;
+    if (M <= 128) return 0;
+    const int st = fill_params(p, nullptr, M, K, (K + 7) / 8 * 8, nseg, nullptr, nullptr, n, "smh_q40_matmul_tiled_direct_fits", true);
+    return st < 0 ? st : (gemm_direct_fits(p) ? 1 : 0);
+}
+
+extern "C" int smh_q40_matmul_tiled_direct(const void *a, int M, int K, long lda, int nseg, const void *const *tiled, const int *n, void *const *out,
+                                           const void *residual, long ldr, smh_stream_t stream) {
+    const char *who = "smh_q40_matmul_tiled_direct";
+    MatmulParams p;
+    const int st = fill_params(p, a, M, K, lda, nseg, tiled, nullptr, n, who, true);
+    if (st) return st;
+    SMH_REQUIRE(gemm_direct_fits(p), "%s: M=%d (above 128) K=%d (a multiple of 32) nseg=%d: ask smh_q40_matmul_tiled_direct_fits first", who, M, K, nseg);
+    SMH_REQUIRE(a && tiled && out && ((uintptr_t)a & 15) == 0, "%s: null or misaligned pointer", who);
+    for (int i = 0; i < nseg; ++i) {
+        SMH_REQUIRE(tiled[i] && ((uintptr_t)tiled[i] & 127) == 0 && out[i] && ((uintptr_t)out[i] & 15) == 0, "%s: weight or output %d is null or misaligned", who, i);
+        p.seg[i].c = (half_t *)out[i];
+        p.seg[i].ldc = n[i];
+    }
+    SMH_REQUIRE(residual == nullptr || (nseg == 1 && ldr >= n[0]), "%s: a residual goes with one weight, ldr=%ld", who, ldr);
+    p.direct = 1;
+    p.epilogue = residual ? SMH_EPI_RESIDUAL : SMH_EPI_NONE;
+    p.resid = (const half_t *)residual;
+    p.ldr = ldr;
+    return gemm_launch(p, (hipStream_t)stream);
 }
 
 extern "C" int smh_q40_matmul_plan_tiled(int M, int K, int nseg, const int *n) {
@@ -415,7 +471,7 @@ static int matmul_fp16(const void *a, int M, int K, long lda, const void *b_w, c
     SMH_REQUIRE(epilogue != SMH_EPI_RESIDUAL || (residual && ldr >= N), "%s: residual missing", who);
     if (force == 2 && M <= SMH_GEMV_MAX_M) gemm_fill_plan(p);        // smh_q40_gemm on a small batch
     const bool gemm = (force == 2) || M > SMH_GEMV_MAX_M;
-    p.c = (half_t *)c; p.ldc = ldc; p.resid = (const half_t *)residual; p.ldr = ldr; p.epilogue = epilogue;
+    p.c = p.seg[0].c = (half_t *)c; p.ldc = p.seg[0].ldc = ldc; p.resid = (const half_t *)residual; p.ldr = ldr; p.epilogue = epilogue;
     if (p.ksplit == 1) {
         p.direct = 1;
         SMH_REQUIRE(!gemm || ldc % 8 == 0, "%s: ldc=%ld must be a multiple of 8 for M > 16", who, ldc);
@@ -493,5 +549,17 @@ extern "C" int smh_partial_rope_append_kv(const void *partial, int ksplit, int B
                        partial, ksplit, B, H, Hkv, (half_t *)q, (half_t *)k, (half_t *)v,
                        (const half_t *)cos_tab, (const half_t *)sin_tab, pos_dev, (uint8_t *)cache_k, (half_t *)cache_ks,
                        (uint8_t *)cache_v, (half_t *)cache_vs, Smax, t_dev);
+    return launch_status();
+}
+
+extern "C" int smh_partial_rope_rows(const void *partial, int ksplit, int S, int H, int Hkv, int D, void *q, void *k, void *v, const void *cos_tab,
+                                     const void *sin_tab, int pos0, smh_stream_t stream) {
+    SMH_REQUIRE(D == 128, "smh_partial_rope_rows: head dim %d (only 128)", D);
+    SMH_REQUIRE(ksplit >= 1 && ksplit <= SMH_MAX_KSPLIT, "smh_partial_rope_rows: ksplit=%d", ksplit);
+    SMH_REQUIRE(S >= 0 && S <= 65535 && H > 0 && Hkv > 0 && pos0 >= 0, "smh_partial_rope_rows: S=%d (at most 65535) H=%d Hkv=%d pos0=%d", S, H, Hkv, pos0);
+    if (S == 0) return 0;
+    SMH_REQUIRE(partial && q && k && v && cos_tab && sin_tab, "smh_partial_rope_rows: null pointer");
+    hipLaunchKernelGGL(partial_rope_rows_kernel, dim3((unsigned)(((H + 2 * Hkv) * 16 + 255) / 256), (unsigned)S), dim3(256), 0, (hipStream_t)stream, partial,
+                       ksplit, S, H, Hkv, (half_t *)q, (half_t *)k, (half_t *)v, (const half_t *)cos_tab, (const half_t *)sin_tab, pos0);
     return launch_status();
 }

@@ -88,7 +88,9 @@ __device__ __forceinline__ void gemm_barrier() { asm volatile("s_waitcnt lgkmcnt
 // `slice`.  zero_rest: the piece ends its unit, and the slabs past `slice` (the unit has no piece for them) are written as
 // zeros.  more: another piece follows in this workgroup (one more barrier, after which the ring may be refilled).
 // tid_bias: zero (a range cut passes one the compiler cannot see, see there).
-template <int TILES, bool RAGGED, bool TILED, int WAVES, int SLOTS, bool PRODUCER>
+// SWIGLU (eight waves, tiled): unit j is 128-column block j of the gate weight (seg[0], pieces 0 and 1 of a stage) next to block
+// j of the up weight (seg[1], pieces 2 and 3); all of K; the epilogue stores fp16(silu(fp16(gate))) * fp16(up).
+template <int TILES, bool RAGGED, bool TILED, int WAVES, int SLOTS, bool PRODUCER, bool SWIGLU = false>
 __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int mb, int slice, int step0, int step1, bool zero_rest, bool more,
                                            int tid_bias) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -103,12 +105,12 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
     const int c = lane & 15;
     const int g = lane >> 4;
     int sg = 0;
-    if (p.nseg > 1 && unit >= p.seg[1].unit0) sg = 1;
-    if (p.nseg > 2 && unit >= p.seg[2].unit0) sg = 2;
+    if (!SWIGLU && p.nseg > 1 && unit >= p.seg[1].unit0) sg = 1;
+    if (!SWIGLU && p.nseg > 2 && unit >= p.seg[2].unit0) sg = 2;
     const MatmulSegment seg = p.seg[sg];
-    const int pair = unit - seg.unit0;
-    const int col0 = pair * GEMM_COLS;
-    const bool two_blocks = col0 + 128 < seg.N;
+    const int pair = SWIGLU ? unit >> 1 : unit - seg.unit0;
+    const int col0 = SWIGLU ? unit * 128 : pair * GEMM_COLS;
+    const bool two_blocks = SWIGLU || col0 + 128 < seg.N;
     const int m0 = mb * p.block_rows;
     const int blk = wave >> 1;                 // block of the pair this wave decodes
     const int bp = wave & 1;                   // ... and its pair of byte positions
@@ -122,6 +124,16 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
     //  Address = uniform base of the step (scalar arithmetic) + a lane offset fixed for the whole kernel.
     const uint8_t *w_base = TILED ? seg.w + (long)pair * tiled_steps(p.K) * TILE_BYTES : seg.w + (long)pair * 128;
     const uint8_t *s_base = reinterpret_cast<const uint8_t *>(seg.s) + (long)pair * 8;
+    // SWIGLU: bytes from the gate weight's tiles to the up weight's, the gate's first piece and its first scale group in a tile
+    const long up = SWIGLU ? (long)((uintptr_t)p.seg[1].w - (uintptr_t)p.seg[0].w) : 0;
+    const int sw_piece = SWIGLU ? 2 * (unit & 1) : 0;
+    // ... and where lane l's dword of a step's 64 scale bytes of k-octet `oct` lies (groups 0, 1: gate, 2, 3: up)
+    auto scale_off = [&](int oct, int l) -> long {
+        if (!SWIGLU) return TILE_W_BYTES + (16 * oct + l) * 4;
+        const int grp = l >> 2;
+        return TILE_W_BYTES + oct * 64 + (2 * (unit & 1) + (grp & 1)) * 16 + (l & 3) * 4 + (grp >= 2 ? up : 0L);
+    };
+    auto piece_off = [&](int q) -> long { return SWIGLU ? (sw_piece + (q & 1)) * 1024L + (q >= 2 ? up : 0L) : q * 1024L; };
     const uint8_t *a_base = reinterpret_cast<const uint8_t *>(p.a);
     const int w_lrow = 8 * wave + (lane >> 3), w_lcol = 16 * (two_blocks ? (lane & 7) : (lane & 3));
     const int s_lrow = 8 * wave + ((lane & 15) >> 1), s_lcol = 4 * (two_blocks ? (lane & 1) : 0);
@@ -137,8 +149,8 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
     auto issue_ws8 = [&](int step, int slot_) {
         uint8_t *st = lds + slot_ * GS_BYTES;
         const uint8_t *tile = w_base + (long)step * TILE_BYTES;
-        if (hh == 0) __builtin_amdgcn_global_load_lds((gptr_t)(tile + wave * 1024 + lane * 16), (lptr_t)(st + wave * 1024), 16, 0, 0);
-        else if (lane < 16) __builtin_amdgcn_global_load_lds((gptr_t)(tile + TILE_W_BYTES + (16 * wave + lane) * 4), (lptr_t)(st + GS_W + wave * 64), 4, 0, 0);
+        if (hh == 0) __builtin_amdgcn_global_load_lds((gptr_t)(tile + piece_off(wave) + lane * 16), (lptr_t)(st + wave * 1024), 16, 0, 0);
+        else if (lane < 16) __builtin_amdgcn_global_load_lds((gptr_t)(tile + scale_off(wave, lane)), (lptr_t)(st + GS_W + wave * 64), 4, 0, 0);
     };
     auto issue_a8 = [&](int step, int slot_) {
         __builtin_amdgcn_global_load_lds((gptr_t)(a_base + (long)step * 64 + a_voff0), (lptr_t)(lds + slot_ * GS_BYTES + GS_W + GS_S + wave8 * 1024), 16, 0, 0);
@@ -149,8 +161,8 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
         if (TILED && WAVES == 8) {
             // two DMA instructions a wave: waves 0-3 their piece of the nibbles, waves 4-7 its scales; every wave 16 rows of A
             const uint8_t *tile = w_base + (long)step * TILE_BYTES;
-            if (hh == 0) __builtin_amdgcn_global_load_lds((gptr_t)(tile + wave * 1024 + lane * 16), (lptr_t)(st + wave * 1024), 16, 0, 0);
-            else if (lane < 16) __builtin_amdgcn_global_load_lds((gptr_t)(tile + TILE_W_BYTES + (16 * wave + lane) * 4), (lptr_t)(st + GS_W + wave * 64), 4, 0, 0);
+            if (hh == 0) __builtin_amdgcn_global_load_lds((gptr_t)(tile + piece_off(wave) + lane * 16), (lptr_t)(st + wave * 1024), 16, 0, 0);
+            else if (lane < 16) __builtin_amdgcn_global_load_lds((gptr_t)(tile + scale_off(wave, lane)), (lptr_t)(st + GS_W + wave * 64), 4, 0, 0);
             __builtin_amdgcn_global_load_lds((gptr_t)(a_base + k0 * 2 + a_voff0), (lptr_t)(st + GS_W + GS_S + wave8 * 1024), 16, 0, 0);
         } else if (TILED) {
             const uint8_t *tile = w_base + (long)step * TILE_BYTES;
@@ -213,8 +225,8 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
                 const uint8_t *arow = a_base + (long)fetch * 64;
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
-                    __builtin_amdgcn_global_load_lds((gptr_t)(tile + q * 1024 + lane * 16), (lptr_t)(st + q * 1024), 16, 0, 0);
-                __builtin_amdgcn_global_load_lds((gptr_t)(tile + TILE_W_BYTES + lane * 4), (lptr_t)(st + GS_W), 4, 0, 0);
+                    __builtin_amdgcn_global_load_lds((gptr_t)(tile + piece_off(q) + lane * 16), (lptr_t)(st + q * 1024), 16, 0, 0);
+                __builtin_amdgcn_global_load_lds((gptr_t)(tile + scale_off(lane >> 4, lane & 15)), (lptr_t)(st + GS_W), 4, 0, 0);
 #pragma unroll
                 for (int t = 0; t < TILES; ++t)
                     __builtin_amdgcn_global_load_lds((gptr_t)(arow + a_voff[t]), (lptr_t)(st + GS_W + GS_S + t * 1024), 16, 0, 0);
@@ -493,8 +505,21 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
         }
         gemm_barrier();
         const int m = m0 + 16 * t + o_row;
-        if (m < p.M) {
-            if (p.direct) {
+        if (SWIGLU || m < p.M) {
+            if constexpr (SWIGLU) {
+                // rows of 128 gate columns and the same 128 up columns: four of them a thread, with partial_silu_mul_kernel's roundings
+                const int cq = 4 * (tid & 31), row = (tid >> 5) & 15, mr = m0 + 16 * t + row;
+                if (mr < p.M) {
+                    const f4 gv = *reinterpret_cast<const f4 *>(otile + row * OP + cq), uv = *reinterpret_cast<const f4 *>(otile + row * OP + 128 + cq);
+                    h4 o;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float gf = (float)(half_t)gv[e];
+                        o[e] = (half_t)(gf / (1.0f + expf(-gf))) * (half_t)uv[e];
+                    }
+                    *reinterpret_cast<h4 *>(seg.c + (long)mr * seg.ldc + col0 + cq) = o;
+                }
+            } else if (p.direct) {
 #pragma unroll
                 for (int q = (WAVES == 8 ? o_half : 0); q < (WAVES == 8 ? o_half + 1 : 2); ++q) {
                     const int n_seg = col0 + 128 * q + 8 * o_lane;
@@ -508,7 +533,7 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
                             o[e] = matmul_epilogue(p, v0[e], m, n + e);
                             o[4 + e] = matmul_epilogue(p, v1[e], m, n + 4 + e);
                         }
-                        *reinterpret_cast<h8 *>(p.c + (long)m * p.ldc + n) = o;
+                        *reinterpret_cast<h8 *>(seg.c + (long)m * seg.ldc + n_seg) = o;
                     }
                 }
             } else {
@@ -547,8 +572,9 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
 // what the kernel needs).  SLOTS: slots of the ring.
 // RANGE (p.chunk > 0): the steps of all column units, laid end to end, are dealt in runs of p.chunk to the workgroups, one
 // workgroup per compute unit, so a workgroup may finish one unit and begin the next: up to two pieces, one after the other.
-template <int TILES, bool RAGGED, bool TILED, int WAVES, int SLOTS = GEMM_STAGES, bool PRODUCER = false, bool RANGE = false>
-__global__ __launch_bounds__(64 * (WAVES + (PRODUCER ? 1 : 0)), WAVES == 8 ? 1 : 2) void q40_gemm_kernel(MatmulParams p) {
+template <int TILES, bool RAGGED, bool TILED, int WAVES, int SLOTS = GEMM_STAGES, bool PRODUCER = false, bool RANGE = false, bool SWIGLU = false>
+// (SWIGLU without the DMA wave: at most 128 registers, so that two workgroups of eight waves fit a compute unit)
+__global__ __launch_bounds__(64 * (WAVES + (PRODUCER ? 1 : 0)), WAVES == 8 ? (SWIGLU && !PRODUCER ? 4 : 1) : 2) void q40_gemm_kernel(MatmulParams p) {
     static_assert(WAVES == 4 || (WAVES == 8 && TILED && !RAGGED), "eight waves: tiled weights, K a multiple of 32");
     static_assert(SLOTS >= 6 && SLOTS <= 10 && (SLOTS == GEMM_STAGES || PRODUCER) && (!PRODUCER || WAVES == 8), "ring depth");
     const int steps_total = (p.K + 31) / 32;
@@ -578,7 +604,7 @@ __global__ __launch_bounds__(64 * (WAVES + (PRODUCER ? 1 : 0)), WAVES == 8 ? 1 :
         const int mb = bid % p.mblocks;
         const int slice = bid / p.mblocks;
         const int s0 = slice * p.steps_per_slice;
-        gemm_piece<TILES, RAGGED, TILED, WAVES, SLOTS, PRODUCER>(p, unit, mb, slice, s0, min(s0 + p.steps_per_slice, steps_total), false, false, 0);
+        gemm_piece<TILES, RAGGED, TILED, WAVES, SLOTS, PRODUCER, SWIGLU>(p, unit, mb, slice, s0, min(s0 + p.steps_per_slice, steps_total), false, false, 0);
     }
 }
 
@@ -1017,6 +1043,34 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_swiglu_kernel(MatmulParams p)
     }
 }
 
+// Rows of a block when M > 128 rows are cut into blocks of at most 128: as even as whole tiles of 16 allow (130 rows are two
+// blocks of 80, not 128 and 2 rows of which both multiply 128).
+static int gemm_even_rows(int M) {
+    const int mblocks = (M + GEMM_BM - 1) / GEMM_BM;
+    return ((M + mblocks - 1) / mblocks + 15) / 16 * 16;
+}
+
+// K-slices of a launch with more than 128 rows: the split with the least estimated time.  A workgroup takes ~0.46 us a step at
+// 128 rows (0.09 + 0.37 of that in proportion to its rows) and ~5 us around its loop; the launch takes as many rounds as its
+// workgroups need compute units; every slice of a split writes fp32 slabs that the consumer reads back (8 bytes an output at
+// ~4.5 TB/s).  (A cap by rows alone gave 1024 rows of wo and w2 one slice, 128 workgroups on 256 compute units: 56 and 136 us.)
+static void gemm_plan_rows(MatmulParams &p, int steps) {
+    p.block_rows = gemm_even_rows(p.M);
+    p.mblocks = (p.M + p.block_rows - 1) / p.block_rows;
+    const long tiles = (long)p.units * p.mblocks;
+    int best = 1;
+    float best_us = 0.f;
+    for (int ks = 1; ks <= SMH_MAX_KSPLIT && (ks == 1 || (tiles * ks <= 512 && steps / ks >= GEMM_STAGES)); ++ks) {
+        const float rounds = (float)((tiles * ks + 255) / 256);
+        const float us = rounds * ((float)((steps + ks - 1) / ks) * (0.09f + 0.37f * p.block_rows / GEMM_BM) + 5.0f) +
+                         (ks > 1 ? (float)ks * p.M * p.n_total * 8.0f / 4.5e6f : 0.0f);
+        if (ks == 1 || us < best_us) { best = ks; best_us = us; }
+    }
+    p.steps_per_slice = (steps + best - 1) / best;
+    p.ksplit = (steps + p.steps_per_slice - 1) / p.steps_per_slice;
+    p.chunk = 0;
+}
+
 void gemm_fill_plan(MatmulParams &p) {
     int unit0 = 0, col0 = 0;
     for (int i = 0; i < p.nseg; ++i) {
@@ -1068,6 +1122,10 @@ void gemm_fill_plan(MatmulParams &p) {
     if (p.M > 64 && p.M <= 128 && p.units <= 16 && p.K % 32 == 0 && p.K <= 4096) p.block_rows = 64;
     p.mblocks = (p.M + p.block_rows - 1) / p.block_rows;
     const int steps = (p.K + 31) / 32;
+    if (p.M > GEMM_BM) {
+        gemm_plan_rows(p, steps);
+        return;
+    }
     const long tiles = (long)p.units * p.mblocks;
     // One round of workgroups.  One workgroup per compute unit when the column units divide the GPU well
     // (at least 200 of the 256 units busy): a second co-resident workgroup buys little there and doubles the
@@ -1179,12 +1237,16 @@ static int gemm_kg_launch(const MatmulParams &p, hipStream_t stream) {
     return launch_status();
 }
 
-// Can w1|w3 of these dimensions run with SwiGLU inside the launch, and is it the faster way?  17 .. 128 rows, K a multiple of
+// Can w1|w3 of these dimensions run with SwiGLU inside the launch, and is it the faster way?  Above 128 rows always (K a multiple
+// of 32; the two-launch form writes and reads 8 bytes of slabs per gate and up value: 62 of 426 us at 2047 rows of the 7B
+// shape).  17 .. 128 rows: K a multiple of
 // 64, two weights of n_half columns (a multiple of 128) whose 2 * n_half / 128 workgroups fit the compute units in one round;
 // `worth_it`: and fill at least half of them (narrower weights are faster as two kernels with a K-split), above 32 rows
 // (measured at the 7B shape, w1|w3 + SiLU: 38.1 against 44.9 us at 100 rows, 29.1 against 31.5 at 64, level at 32).
 bool gemm_swiglu_fits(int M, int K, int n_half, bool worth_it) {
-    if (M <= SMH_GEMV_MAX_M || M > 128 || K <= 0 || K % 64 != 0 || n_half <= 0 || n_half % 128 != 0) return false;
+    if (M <= SMH_GEMV_MAX_M || K <= 0 || n_half <= 0 || n_half % 128 != 0) return false;
+    if (M > GEMM_BM) return K % 32 == 0;                        // gemm_swiglu_rows_launch
+    if (K % 64 != 0) return false;
     const int wgs = 2 * (n_half / 128);
     return wgs <= 256 && (!worth_it || (wgs >= 128 && M > 32));
 }
@@ -1210,6 +1272,50 @@ int gemm_swiglu_launch(const MatmulParams &p, hipStream_t stream) {
     int tiles = (p.M + 15) / 16;
     if (tiles < 2) tiles = 2;
     hipLaunchKernelGGL(kern[tiles], dim3((unsigned)(2 * (p.seg[0].N / 128))), dim3(576), lds_bytes[tiles], stream, p);
+    return launch_status();
+}
+
+// More than 128 rows (a prefill) on tiled weights.  Without a K-split a launch stores fp16 results itself: no fp32 slabs (4 bytes
+// an output and slice written here and read behind) and no kernel to add them.
+static int gemm_rows_setup(MatmulParams &p, int units) {
+    p.units = units;
+    p.units_pad = (units + 7) / 8 * 8;
+    p.block_rows = gemm_even_rows(p.M);
+    p.mblocks = (p.M + p.block_rows - 1) / p.block_rows;
+    p.kgroups = 0;
+    p.chunk = 0;
+    p.ksplit = 1;
+    p.steps_per_slice = p.K / 32;
+    p.direct = 1;
+    return p.units * p.mblocks;
+}
+
+bool gemm_direct_fits(const MatmulParams &p) { return p.tiled && p.M > GEMM_BM && p.K % 32 == 0 && p.ksplit == 1; }
+
+int gemm_swiglu_rows_launch(MatmulParams p, hipStream_t stream) {
+    // (more than 128 rows in even blocks: five to eight tiles)
+    constexpr int S = GEMM_DMA_WAVE_SLOTS;
+    static const gemm_kernel_t plain[4] = {q40_gemm_kernel<5, false, true, 8, GEMM_STAGES, false, false, true>, q40_gemm_kernel<6, false, true, 8, GEMM_STAGES, false, false, true>,
+                                           q40_gemm_kernel<7, false, true, 8, GEMM_STAGES, false, false, true>, q40_gemm_kernel<8, false, true, 8, GEMM_STAGES, false, false, true>};
+    static const gemm_kernel_t dma_wave[4] = {q40_gemm_kernel<5, false, true, 8, S, true, false, true>, q40_gemm_kernel<6, false, true, 8, S, true, false, true>,
+                                              q40_gemm_kernel<7, false, true, 8, S, true, false, true>, q40_gemm_kernel<8, false, true, 8, S, true, false, true>};
+    static const hipError_t lds_ok = [] {
+        hipError_t e = hipSuccess;
+        for (int t = 0; t < 4 && e == hipSuccess; ++t) {
+            e = hipFuncSetAttribute((const void *)plain[t], hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS);
+            if (e == hipSuccess) e = hipFuncSetAttribute((const void *)dma_wave[t], hipFuncAttributeMaxDynamicSharedMemorySize, S * GS_BYTES);
+        }
+        return e;
+    }();
+    if (lds_ok != hipSuccess) {
+        set_error("q40 gemm: the kernels' LDS could not be reserved: %s", hipGetErrorString(lds_ok));
+        return (int)lds_ok;
+    }
+    SMH_REQUIRE((long)p.M * p.lda * 2 < (1L << 32), "q40 gemm: M x lda = %d x %ld exceeds the 32-bit lane offsets of A", p.M, p.lda);
+    const bool one_each = gemm_rows_setup(p, p.seg[0].N / 128) <= GEMM_DMA_WAVE_MAX_WGS;
+    const int t = p.block_rows / 16 - 5;
+    hipLaunchKernelGGL((one_each ? dma_wave : plain)[t], dim3((unsigned)((long)p.units_pad * p.mblocks)), dim3(512 + (one_each ? 64 : 0)),
+                       one_each ? S * GS_BYTES : GEMM_LDS, stream, p);
     return launch_status();
 }
 

@@ -44,11 +44,13 @@ struct MatmulSegment {
     int N;               // columns of this weight
     int col0;            // first output column
     int unit0;           // first work unit (column pair / column block) of this weight
+    half_t *c;           // direct output of this weight [M, ldc] (GEMM without K-split)
+    long ldc;
 };
 
 struct MatmulParams {
     const half_t *a;
-    half_t *c;               // direct output (ksplit == 1)
+    half_t *c;               // GEMV: direct output (ksplit == 1)
     const half_t *resid;
     float *partial;          // [ksplit][M][n_total]
     MatmulSegment seg[SMH_MAX_SEGMENTS];
@@ -88,5 +90,9 @@ void gemm_fill_plan(MatmulParams &p);
 int gemm_launch(const MatmulParams &p, hipStream_t stream);
 bool gemm_swiglu_fits(int M, int K, int n_half, bool worth_it);
 int gemm_swiglu_launch(const MatmulParams &p, hipStream_t stream);     // seg[0] = gate, seg[1] = up (tiled), c / ldc = the activations
+// more than 128 rows on tiled weights: can the launch write its fp16 results itself (no K-split, enough workgroups without one)
+bool gemm_direct_fits(const MatmulParams &p);
+// SiLU(gate) * up for more than 128 rows: seg[0] = gate, seg[1] = up (tiled), seg[0].c / ldc = the activations
+int gemm_swiglu_rows_launch(MatmulParams p, hipStream_t stream);
 
 }  // namespace smh

@@ -359,13 +359,18 @@ class Transformer(nn.Module):
         residual+RMSNorm | wq,wk,wv (one launch) | RoPE + Q4_0 KV append | attention | wo |
         residual+RMSNorm | w1,w3 (one launch) | SiLU*up | w2.  Every linear leaves fp32 K-slice
         slabs that the next small kernel adds and rounds to fp16 once, exactly where the
-        reference's matmul_q40 rounds."""
+        reference's matmul_q40 rounds.  On tiled weights decode steps and the prefill of the shared prompt run layer by layer
+        inside the library (_decode, _prefill: with a few rows more of the operators in one launch); what is left here is the
+        checkpoint layout and prompts of several rows or in the branches' own caches."""
         bsz, seqlen = tokens.shape
         M = bsz * seqlen
         p = self.params
-        if start_pos != 0 and self.tiled_weights:
+        tiled = self.tiled_weights
+        if tiled and start_pos != 0:
             assert seqlen == 1, "decode steps take one token per branch"
             return self._decode(tokens, step_state)
+        if tiled and bsz == 1 and not self.per_branch_kv:
+            return self._prefill(tokens)
         h = K.embedding(tokens, self.tok_embeddings.weight).view(M, p.dim)
         cos, sin = self._tables(h.device)
         pending = None                      # product of the previous layer's w2, not yet added to h
@@ -373,15 +378,8 @@ class Transformer(nn.Module):
         for layer in self.layers:
             att, ff = layer.attention, layer.feed_forward
             H, Hkv, D = att.n_local_heads, att.n_local_kv_heads, att.head_dim
-            tiled = self.tiled_weights
-            qkv_ops = [att.wq.operand(tiled), att.wk.operand(tiled), att.wv.operand(tiled)]
-            if pending is not None and self._norm_in(M, p.dim, qkv_ops):
-                # RMSNorm made inside the matmul: the launch before it only adds the slabs and leaves sums of squares
-                h, sums = K.partial_residual_sumsq(pending, h)
-                qkv = K.matmul_q40_partial_norm(h, sums, layer.attention_norm.weight, layer.attention_norm.eps, qkv_ops)
-            else:
-                h, xn = K.partial_rmsnorm(pending, h, layer.attention_norm.weight, layer.attention_norm.eps)
-                qkv = K.matmul_q40_partial(xn, qkv_ops)
+            h, xn = K.partial_rmsnorm(pending, h, layer.attention_norm.weight, layer.attention_norm.eps)
+            qkv = K.matmul_q40_partial(xn, [att.wq.operand(tiled), att.wk.operand(tiled), att.wv.operand(tiled)])
             if start_pos == 0:
                 xq = K.partial_reduce(qkv, 0, H * D).view(bsz, seqlen, H, D)
                 xk = K.partial_reduce(qkv, H * D, Hkv * D).view(bsz, seqlen, Hkv, D)
@@ -417,23 +415,13 @@ class Transformer(nn.Module):
                                                        att.cache_v, att.cache_v_s, p.max_seq_len, t_dev)
                     o = att.decode_attention(q, k, v, t_dev, pages, self.attn_single_launch and M * (H // Hkv) <= 16).view(M, H * D)
             po = K.matmul_q40_partial(o, [att.wo.operand(tiled)])
+            h, xn = K.partial_rmsnorm(po, h, layer.ffn_norm.weight, layer.ffn_norm.eps)
             gu_ops = [ff.w1.operand(tiled), ff.w3.operand(tiled)]
             if tiled and self.swiglu_in_matmul and K.swiglu_fits(M, p.dim, ff.w1.shape[0]):
-                # 33 .. 128 rows and a wide FFN: SiLU(gate) * up leaves w1|w3's launch as the activations of w2
-                h, xn = K.partial_rmsnorm(po, h, layer.ffn_norm.weight, layer.ffn_norm.eps)
-                pending = K.matmul_q40_partial(K.matmul_q40_swiglu(xn, gu_ops[0], gu_ops[1]), [ff.w2.operand(True)])
-                continue
-            if self._norm_in(M, p.dim, gu_ops):
-                h, sums = K.partial_residual_sumsq(po, h)
-                gu = K.matmul_q40_partial_norm(h, sums, layer.ffn_norm.weight, layer.ffn_norm.eps, gu_ops)
+                act = K.matmul_q40_swiglu(xn, gu_ops[0], gu_ops[1])
             else:
-                h, xn = K.partial_rmsnorm(po, h, layer.ffn_norm.weight, layer.ffn_norm.eps)
-                gu = K.matmul_q40_partial(xn, gu_ops)
-            if tiled and self.silu_in_matmul and M <= K.SILU_IN_MAX_M and ff.w2.shape[1] % 32 == 0 and ff.w2.w.is_cuda:
-                pending = K.matmul_q40_partial_silu(gu, [ff.w2.operand(True)])      # SiLU(gate)*up made inside w2's launch
-            else:
-                act = K.partial_silu_mul(gu)
-                pending = K.matmul_q40_partial(act, [ff.w2.operand(tiled)])
+                act = K.partial_silu_mul(K.matmul_q40_partial(xn, gu_ops))
+            pending = K.matmul_q40_partial(act, [ff.w2.operand(tiled)])
         _, hn = K.partial_rmsnorm(pending, h, self.norm.weight, self.norm.eps, want_h=False)
         return self._lm_head(hn.view(bsz, seqlen, p.dim))
 
@@ -444,36 +432,49 @@ class Transformer(nn.Module):
         B = tokens.shape[0]
         h = K.embedding(tokens, self.tok_embeddings.weight)
         dev = h.device
-        cos, sin = self._tables(dev)
-        pages = self._pages(dev)
         att0 = self.layers[0].attention
-        H, rep, P = att0.n_local_heads, att0.n_rep, att0.cache_prompt_len
-        one = self.attn_single_launch and B * rep <= 16
-        ws = K.attn_qkv_workspace(dev, B, H, P) if one else K.attn_workspace(dev, B, H, P)
-        d = K.DecodePass(self._layer_struct(self.layers[0]), B, h, cos, sin, step_state, ws, bool(one))
+        one = self.attn_single_launch and B * att0.n_rep <= 16
+        P = att0.cache_prompt_len
+        ws = K.attn_qkv_workspace(dev, B, att0.n_local_heads, P) if one else K.attn_workspace(dev, B, att0.n_local_heads, P)
+        run = K.LayerPass(self._layer_struct(self.layers[0]), B, h, *self._tables(dev), self.swiglu_in_matmul)
         norm_in = self._norm_in(B, p.dim, [lin._tiled for lin in (att0.wq, att0.wk, att0.wv)])      # (the library asks again, launch by launch)
-        d.set(smax=p.max_seq_len, cache_rows=p.max_batch_size * p.max_seq_len, pages=pages, norm_in_rows=B if norm_in else 0,
-              silu_in_rows=K.SILU_IN_MAX_M if self.silu_in_matmul else 0, swiglu_in=self.swiglu_in_matmul,
-              attn_from_qkv=self.attn_from_qkv and not self.per_branch_kv)
+        run.decode_step(step_state, ws, bool(one), p.max_seq_len, p.max_batch_size * p.max_seq_len, self._pages(dev), B if norm_in else 0,
+                        K.SILU_IN_MAX_M if self.silu_in_matmul else 0, self.attn_from_qkv and not self.per_branch_kv)
         for layer in self.layers:
             s = self._layer_struct(layer)
-            d.layer(s)
-        return self._lm_head(d.finish(s, self.norm.weight, self.norm.eps).view(B, 1, p.dim))
+            run.decode(s)
+        return self._lm_head(run.finish(s, self.norm.weight, self.norm.eps).view(B, 1, p.dim))
+
+    def _prefill(self, tokens: torch.Tensor) -> torch.Tensor:
+        """The prefill of one prompt on tiled weights, a layer per library call (smh_prefill_layer): its k and v become the rows
+        of the shared prompt cache."""
+        S = tokens.shape[1]
+        h = K.embedding(tokens, self.tok_embeddings.weight)
+        run = K.LayerPass(self._layer_struct(self.layers[0]), S, h, *self._tables(h.device), self.swiglu_in_matmul)
+        for layer in self.layers:
+            att = layer.attention
+            assert S <= att.cache_prompt_k.shape[1] and S <= att.cache_prompt_v.shape[1]
+            s = self._layer_struct(layer)
+            run.prefill(s)
+            att.cache_prompt_len = S
+        return self._lm_head(run.finish(s, self.norm.weight, self.norm.eps).view(1, S, self.params.dim))
 
     def _layer_struct(self, layer):
-        """What smh_decode_layer reads of a layer, rebuilt when any of its tensors is another one than at the last step."""
+        """What the library's layer calls read of a layer, rebuilt when any of its tensors is another one than at the last pass."""
         att, ff = layer.attention, layer.feed_forward
         lins = (att.wq, att.wk, att.wv, att.wo, ff.w1, ff.w2, ff.w3)
-        key = [att.cache_prompt_len, layer.attention_norm.weight.data_ptr(), layer.ffn_norm.weight.data_ptr(), att.cache_prompt_k.data_ptr(),
-               att.cache_prompt_v.data_ptr(), att.cache_k.data_ptr(), att.cache_k_s.data_ptr(), att.cache_v.data_ptr(), att.cache_v_s.data_ptr()]
+        key = [layer.attention_norm.weight.data_ptr(), layer.ffn_norm.weight.data_ptr(), att.cache_prompt_k.data_ptr(), att.cache_prompt_v.data_ptr(),
+               att.cache_k.data_ptr(), att.cache_k_s.data_ptr(), att.cache_v.data_ptr(), att.cache_v_s.data_ptr()]
         for lin in lins:
             key += (lin.w.data_ptr(), lin.s.data_ptr(), id(lin._tiled))
         if layer.native is None or layer.native_key != key:
             layer.native = K.layer_struct(self.params.dim, att.n_local_heads, att.n_local_kv_heads, layer.attention_norm.weight, layer.attention_norm.eps,
                                           layer.ffn_norm.weight, layer.ffn_norm.eps, [lin.operand(True) for lin in lins], att.cache_prompt_k,
-                                          att.cache_prompt_v, att.cache_prompt_len, att.cache_k, att.cache_k_s, att.cache_v, att.cache_v_s)
-            key[9:] = [x for lin in lins for x in (lin.w.data_ptr(), lin.s.data_ptr(), id(lin._tiled))]
+                                          att.cache_prompt_v, att.cache_k, att.cache_k_s, att.cache_v, att.cache_v_s)
+            key[8:] = [x for lin in lins for x in (lin.w.data_ptr(), lin.s.data_ptr(), id(lin._tiled))]
             layer.native_key = key
+        assert att.cache_prompt_len <= att.cache_prompt_k.shape[1]
+        layer.native.prompt_len = att.cache_prompt_len
         return layer.native
 
     def quantize_lm_head(self, enable: bool = True):

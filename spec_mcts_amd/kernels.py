@@ -197,7 +197,7 @@ def swiglu_fits(M: int, K: int, n_half: int) -> bool:
 def matmul_q40_swiglu(a: torch.Tensor, gate: "TiledQ40", up: "TiledQ40", out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """fp16(silu(fp16(a . gate))) * fp16(a . up) in one launch (FeedForward's `F.silu(self.w1(x)) * self.w3(x)`,
     hf_model_q40_kv_shared.py:434) for tiled weights: what partial_silu_mul(matmul_q40_partial(a, [gate, up])) returns, without
-    the slabs.  17 <= M <= 128, K a multiple of 64, n_half a multiple of 128 up to 16384."""
+    the slabs.  17 <= M <= 128, K a multiple of 64, n_half a multiple of 128 up to 16384; or M > 128, K a multiple of 32."""
     lib = _lib.load()
     assert a.is_contiguous() and a.dtype == torch.float16 and a.dim() == 2 and a.data_ptr() % 16 == 0
     _need_gpu(a)
@@ -209,6 +209,27 @@ def matmul_q40_swiglu(a: torch.Tensor, gate: "TiledQ40", up: "TiledQ40", out: Op
     check(lib.smh_q40_matmul_tiled_swiglu(a.data_ptr(), M, Kd, Kd, gate.buf.data_ptr(), up.buf.data_ptr(), gate.N, out.data_ptr(), gate.N,
                                           _stream()), "smh_q40_matmul_tiled_swiglu")
     return out
+
+
+def matmul_q40_direct(a: torch.Tensor, linears: Sequence["TiledQ40"], residual: Optional[torch.Tensor] = None):
+    """The fp16 products of a [M,K] with up to 3 tiled weights in one launch that leaves no slabs, for more than 128 rows where no
+    K-split is needed to fill the GPU; None where the shape does not allow it.  residual [M,N]: residual + product (one weight)."""
+    import ctypes
+    lib = _lib.load()
+    assert a.is_contiguous() and a.dtype == torch.float16 and a.dim() == 2 and a.data_ptr() % 16 == 0
+    _need_gpu(a)
+    M, Kd = a.shape
+    nseg = len(linears)
+    assert all(isinstance(t, TiledQ40) and t.K == Kd for t in linears)
+    na = (ctypes.c_int * nseg)(*[t.N for t in linears])
+    if lib.smh_q40_matmul_tiled_direct_fits(M, Kd, nseg, na) != 1:
+        return None
+    assert residual is None or (nseg == 1 and residual.shape == (M, linears[0].N) and residual.is_contiguous() and residual.dtype == torch.float16)
+    outs = [torch.empty((M, t.N), dtype=torch.float16, device=a.device) for t in linears]
+    tp = (ctypes.c_void_p * nseg)(*[t.buf.data_ptr() for t in linears])
+    op = (ctypes.c_void_p * nseg)(*[o.data_ptr() for o in outs])
+    check(lib.smh_q40_matmul_tiled_direct(a.data_ptr(), M, Kd, Kd, nseg, tp, na, op, _ptr(residual), linears[0].N, _stream()), "smh_q40_matmul_tiled_direct")
+    return outs
 
 
 SILU_IN_MAX_M = 2
@@ -707,12 +728,13 @@ def embedding(tokens: torch.Tensor, table: torch.Tensor) -> torch.Tensor:
 
 
 # ---------------------------------------------------------------------------------------------
-# a decode step, layer by layer
+# a decode step or a prefill, layer by layer
 # ---------------------------------------------------------------------------------------------
 def layer_struct(dim: int, H: int, Hkv: int, att_norm: torch.Tensor, att_eps: float, ffn_norm: torch.Tensor, ffn_eps: float, tiled: Sequence[TiledQ40],
-                 prompt_k: torch.Tensor, prompt_v: torch.Tensor, prompt_len: int, cache_k: torch.Tensor, cache_ks: torch.Tensor,
-                 cache_v: torch.Tensor, cache_vs: torch.Tensor) -> "_lib.SmhLayer":
-    """smh_layer of one transformer layer; `tiled`: wq, wk, wv, wo, w1, w2, w3.  The caller keeps the tensors alive."""
+                 prompt_k: torch.Tensor, prompt_v: torch.Tensor, cache_k: torch.Tensor, cache_ks: torch.Tensor, cache_v: torch.Tensor,
+                 cache_vs: torch.Tensor) -> "_lib.SmhLayer":
+    """smh_layer of one transformer layer; `tiled`: wq, wk, wv, wo, w1, w2, w3.  The caller keeps the tensors alive and sets
+    prompt_len (at most the rows of prompt_k and prompt_v)."""
     wq, wk, wv, wo, w1, w2, w3 = tiled
     ffn, D = w1.N, 128
     assert all(isinstance(t, TiledQ40) for t in tiled)
@@ -720,12 +742,11 @@ def layer_struct(dim: int, H: int, Hkv: int, att_norm: torch.Tensor, att_eps: fl
     _need_gpu(att_norm, ffn_norm, prompt_k, prompt_v, cache_k, cache_ks, cache_v, cache_vs, *(t.buf for t in tiled))
     for t in (att_norm, ffn_norm):
         assert t.numel() == dim and t.dtype == torch.float16 and t.is_contiguous()
-    for t in (prompt_k, prompt_v):
-        assert t.is_contiguous() and t.dtype == torch.float16 and prompt_len * Hkv * D <= t.numel()
+    assert prompt_k.is_contiguous() and prompt_v.is_contiguous() and prompt_k.dtype == torch.float16 and prompt_v.dtype == torch.float16
     assert cache_k.dtype == torch.int8 and cache_v.dtype == torch.int8 and cache_ks.dtype == torch.float16 and cache_vs.dtype == torch.float16
     assert cache_k.is_contiguous() and cache_v.is_contiguous() and cache_ks.is_contiguous() and cache_vs.is_contiguous()
     s = _lib.SmhLayer()
-    s.dim, s.ffn, s.heads, s.kv_heads, s.att_eps, s.ffn_eps, s.prompt_len = dim, ffn, H, Hkv, att_eps, ffn_eps, prompt_len
+    s.dim, s.ffn, s.heads, s.kv_heads, s.att_eps, s.ffn_eps = dim, ffn, H, Hkv, att_eps, ffn_eps
     s.att_norm, s.ffn_norm = att_norm.data_ptr(), ffn_norm.data_ptr()
     s.wq, s.wk, s.wv, s.wo, s.w1, s.w2, s.w3 = (t.buf.data_ptr() for t in tiled)
     s.prompt_k, s.prompt_v = prompt_k.data_ptr(), prompt_v.data_ptr()
@@ -733,44 +754,54 @@ def layer_struct(dim: int, H: int, Hkv: int, att_norm: torch.Tensor, att_eps: fl
     return s
 
 
-class DecodePass:
-    """One decode step over `rows` branches (smh_pass): layer(struct) per layer, then finish() for the last residual add and the
-    final RMSNorm.  `h`: the embeddings [rows, dim]; `step_state`: (position, suffix index) on the device; `ws`: the workspace of
-    the attention (of its one-launch form with `one_launch`).  All other buffers are one allocation that lives as long as this."""
+class LayerPass:
+    """One pass over all layers (smh_pass): a decode step over `rows` branches (after decode_step()) or the prefill of a prompt
+    of `rows` tokens.  decode(struct) or prefill(struct) per layer, then finish() for the last residual add and the final RMSNorm.
+    `h`: the embeddings [rows, dim].  All other buffers are one allocation that lives as long as this."""
 
-    def __init__(self, first: "_lib.SmhLayer", rows: int, h: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, step_state, ws: torch.Tensor, one_launch: bool):
+    def __init__(self, first: "_lib.SmhLayer", rows: int, h: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, swiglu_in: bool):
         self.lib = _lib.load()
-        pos_dev, t_dev = step_state
-        _need_gpu(h, cos, sin, pos_dev, t_dev, ws)
+        _need_gpu(h, cos, sin)
         assert h.dtype == torch.float16 and h.is_contiguous() and h.numel() == rows * first.dim
-        assert pos_dev.dtype == torch.int32 and t_dev.dtype == torch.int32
-        nbytes = int(self.lib.smh_decode_scratch_bytes(first, rows))
+        nbytes = int(self.lib.smh_decode_scratch_bytes(first, rows, int(bool(swiglu_in))))
         if nbytes == 0:
             check(-1, "smh_decode_scratch_bytes")
         self.scratch = torch.empty(nbytes, dtype=torch.uint8, device=h.device)
-        self.h, self.ws = h, ws
+        self.h = h
         p = self.p = _lib.SmhPass()
-        p.rows, p.cos_tab, p.sin_tab, p.pos_dev, p.t_dev = rows, cos.data_ptr(), sin.data_ptr(), pos_dev.data_ptr(), t_dev.data_ptr()
+        p.rows, p.cos_tab, p.sin_tab, p.swiglu_in = rows, cos.data_ptr(), sin.data_ptr(), int(bool(swiglu_in))
+        p.scratch, p.scratch_bytes, p.h = self.scratch.data_ptr(), nbytes, h.data_ptr()
+        self.stream = _stream()
+
+    def decode_step(self, step_state, ws: torch.Tensor, one_launch: bool, smax: int, cache_rows: int, pages: Optional[torch.Tensor], norm_in_rows: int,
+                    silu_in_rows: int, attn_from_qkv: bool) -> None:
+        """step_state: (position, suffix index) on the device; `ws`: the workspace of the attention (of its one-launch form with
+        `one_launch`); pages: int32 page table over cache_rows cache rows, or None."""
+        p = self.p
+        pos_dev, t_dev = step_state
+        _need_gpu(pos_dev, t_dev, ws)
+        assert pos_dev.dtype == torch.int32 and t_dev.dtype == torch.int32
+        p.pos_dev, p.t_dev = pos_dev.data_ptr(), t_dev.data_ptr()
+        self.ws = ws
         if one_launch:
             p.attn_one, p.attn_one_ws, p.attn_one_ws_bytes = 1, ws.data_ptr(), ws.numel()
         else:
             p.attn_ws, p.attn_ws_bytes = ws.data_ptr(), ws.numel()
-        p.scratch, p.scratch_bytes, p.h = self.scratch.data_ptr(), nbytes, h.data_ptr()
-        self.stream = _stream()
-
-    def set(self, smax: int, cache_rows: int, pages: Optional[torch.Tensor], norm_in_rows: int, silu_in_rows: int, swiglu_in: bool, attn_from_qkv: bool) -> None:
-        p = self.p
-        p.smax, p.cache_rows, p.norm_in_rows, p.silu_in_rows = smax, cache_rows, norm_in_rows, silu_in_rows
-        p.swiglu_in, p.attn_from_qkv = int(bool(swiglu_in)), int(bool(attn_from_qkv))
+        p.smax, p.cache_rows, p.norm_in_rows, p.silu_in_rows, p.attn_from_qkv = smax, cache_rows, norm_in_rows, silu_in_rows, int(bool(attn_from_qkv))
         if pages is not None:
             assert pages.is_cuda and pages.dtype == torch.int32 and pages.dim() == 2 and pages.stride(1) == 1
             assert pages.shape[0] >= p.rows and pages.shape[1] >= smax
             p.pages, p.pages_stride = pages.data_ptr(), pages.stride(0)
 
-    def layer(self, s: "_lib.SmhLayer") -> None:
+    def decode(self, s: "_lib.SmhLayer") -> None:
         st = self.lib.smh_decode_layer(s, self.p, self.stream)
         if st:
             check(st, "smh_decode_layer")
+
+    def prefill(self, s: "_lib.SmhLayer") -> None:
+        st = self.lib.smh_prefill_layer(s, self.p, self.stream)
+        if st:
+            check(st, "smh_prefill_layer")
 
     def finish(self, last: "_lib.SmhLayer", weight: torch.Tensor, eps: float) -> torch.Tensor:
         assert weight.numel() == last.dim and weight.dtype == torch.float16

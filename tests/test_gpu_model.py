@@ -216,3 +216,19 @@ def test_graph_decoder_refuses_to_run_past_the_caches():
         dec.decode(1)
     with pytest.raises(AssertionError, match="suffix cache exhausted"):
         model(torch.zeros((2, 1), dtype=torch.int64, device="cuda:0"), 9 + SMALL["max_seq_len"])
+
+
+@pytest.mark.parametrize("P", [15, 40, 129, 200])
+def test_prefill_lengths_match_the_oracle(P):
+    """prompts on either side of the sizes at which the prefill's linears change kernel: logits and the prompt cache's rows"""
+    cfg = dict(dim=512, n_layers=2, n_heads=4, n_kv_heads=2, vocab_size=384, multiple_of=128, max_batch_size=2, max_seq_len=8, max_prompt_seq_len=256)
+    oargs, sd, model = _build(cfg, 60)
+    prompt = torch.randint(0, cfg["vocab_size"], (1, P), generator=torch.Generator().manual_seed(61 + P))
+    oracle = O.OracleTransformer(oargs, sd, dense=True)
+    want = oracle.forward(prompt, 0)
+    got = model(prompt.cuda(), 0).cpu()
+    assert torch.allclose(got.float(), want.float(), rtol=2e-2, atol=2e-2)
+    assert all(layer.attention.cache_prompt_len == P for layer in model.layers)
+    model.fused = False
+    same = model(prompt.cuda(), 0).cpu()
+    assert torch.allclose(got.float(), same.float(), rtol=2e-2, atol=2e-2)

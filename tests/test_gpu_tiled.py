@@ -272,3 +272,35 @@ def test_model_logits_do_not_depend_on_where_rmsnorm_is_made():
         b = run()
         for x, y in zip(a, b):
             assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("M", [129, 130, 255, 300])
+@pytest.mark.parametrize("K,n_half", [(256, 384), (4096, 1024), (96, 128), (512, 11008)])
+def test_swiglu_inside_the_gate_up_launch_above_128_rows(M, K, n_half):
+    """even row blocks of five to eight tiles, an odd number of 128-column blocks, with and without the DMA wave"""
+    import torch.nn.functional as F
+    from spec_mcts_amd import kernels as Kn
+    w1, w3 = _weight(K, n_half, 990 + K), _weight(K, n_half, 991 + K)
+    x = (torch.randn((M, K), generator=torch.Generator().manual_seed(992 + M)) * 0.5).half()
+    assert Kn.swiglu_fits(M, K, n_half)
+    got = Kn.matmul_q40_swiglu(x.cuda(), Kn.tile_q40(w1[0].cuda(), w1[1].cuda(), K, n_half), Kn.tile_q40(w3[0].cuda(), w3[1].cuda(), K, n_half)).cpu()
+    want = F.silu(O.matmul_q40(x, w1[0], w1[1], (K, n_half)).float()).half() * O.matmul_q40(x, w3[0], w3[1], (K, n_half))
+    assert torch.allclose(got.float(), want.float(), rtol=1e-2, atol=2e-3)
+
+
+@pytest.mark.parametrize("M,K,ns", [(129, 256, [16384, 128, 384]), (300, 64, [128]), (2047, 512, [2048]), (700, 4096, [11008])])
+def test_direct_products(M, K, ns):
+    """launches without a K-split that store fp16 themselves: outputs per weight, a residual, rows past the last block's end"""
+    from spec_mcts_amd import kernels as Kn
+    ws = [_weight(K, n, 1000 + i + K) for i, n in enumerate(ns)]
+    tiled = [Kn.tile_q40(w.cuda(), s.cuda(), K, n) for (w, s), n in zip(ws, ns)]
+    a = (torch.randn((M, K), generator=torch.Generator().manual_seed(1001 + M)) * 0.5).half()
+    r = torch.randn((M, ns[0]), generator=torch.Generator().manual_seed(1002)).half() if len(ns) == 1 else None
+    got = Kn.matmul_q40_direct(a.cuda(), tiled, residual=r.cuda() if r is not None else None)
+    assert (got is not None) == (Kn.matmul_plan(M, K, ns, tiled=True) == 1)
+    if got is None:
+        return
+    for (w, s), n, o in zip(ws, ns, got):
+        want = O.matmul_q40(a, w, s, (K, n))
+        want = want.float() + r.float() if r is not None else want.float()
+        assert torch.allclose(o.cpu().float(), want, rtol=1e-2, atol=2e-3)
