@@ -320,147 +320,209 @@ __global__ __launch_bounds__(256) void attn_prefix_kernel(AttnParams p) {
 }
 
 // ---- causal attention of a prefill on the matrix cores ----------------------------------------------------------
-// grid (ceil(S / 64), H): a workgroup owns 64 consecutive query positions of one head, wave w the 16 of them from
-// 64 qb + 16 w.  It walks the key tiles (PF_TW rows, staged once per workgroup: K row-major, V transposed, as in
-// attn_prefix_body) from position 0 to its diagonal with an online softmax: per tile S^T = K . Q^T and
-// O^T += V^T . P^T on the matrix cores (the B operand of the second product is the accumulator layout of the first),
-// running maximum / sum / O^T in registers, so nothing but the fp16 result is written.  The next tile's K / V rows
-// are in flight (registers) while the current one is multiplied.  q [S,H,128], k, v [S,Hkv,128], out [S,H,128].
-constexpr int PF_TW = 64;
+// A workgroup owns 32 QG consecutive query positions of one head; its 2 QG waves are QG groups of 32 queries x two key groups
+// that take alternate key tiles (a wave alone on a SIMD waits for its own chain of products, exponentials and LDS reads; two
+// keep the matrix cores twice as busy and halve the longest walk).  A wave's 32 queries are the columns of
+// S^T = K . Q^T and of O^T += V^T . P^T, both in 32 x 32 x 16 products (an operand read from LDS feeds twice the multiply-adds
+// of a 16-column tile: with 16 queries a wave the LDS reads alone took twice the matrix time).  It walks key tiles of 64 up to
+// the diagonal with an online softmax; running maximum, sum and O^T stay in registers until the key groups are merged.  The accumulator of S^T
+// holds keys 8 i + 4 hi + j of query lane % 32 (hi = lane / 32), so a lane's eight probabilities of 16 keys are a B operand of
+// the second product if V^T lists its keys in that order (pv_slot).
+//   * K tiles go global -> LDS by DMA, 16-byte chunks XOR-swizzled by the row; V goes through registers into its transposed
+//     tile, swizzled so that neither the 8-byte stores nor the 16-byte reads pile up on a few banks.  Two buffers: the next
+//     tile is on its way while one is multiplied, one barrier a tile.
+//   * O^T is rescaled only when a maximum has grown by more than 2^8 (the probabilities are then at most 256, and the factor
+//     cancels in the end): the rescale would be a quarter of the vector instructions of a tile.
+//   * The longest walks are dispatched first.
+// Bound by the vector ALU (exponentials) and the matrix cores together.  2047 rows x 32 heads: 187 us with 16 queries a wave and
+// two barriers a tile, 68 with 32 queries and one key group, 56 (614 TFLOP/s) like this; 512 rows: 22.5 -> 13 us.
+// (The two chains of S^T products interleaved, 32-bit row offsets, a higher wave priority for one key group: no gain.)
+// q [S,H,128], k, v [S,Hkv,128], out [S,H,128].
+constexpr int PF_TW = 64;                                  // keys of a tile
+typedef float f16v __attribute__((ext_vector_type(16)));
+typedef const __attribute__((address_space(1))) void *att_gptr_t;
+typedef __attribute__((address_space(3))) void *att_lptr_t;
 struct PrefillParams {
     const half_t *q, *k, *v;
     half_t *out;
     int S, H, Hkv, n_rep;
     float scale_log2;
 };
+// half-word slot of key t (0 .. 63) of dim d in V^T's row d
+__device__ __forceinline__ int pv_slot(int t, int d) {
+    const int chunk = 2 * (t >> 4) + ((t >> 2) & 1);       // sixteen keys are two chunks: hi = 0, hi = 1
+    return ((chunk ^ (d & 7) ^ ((d >> 3) & 7)) << 3) + ((t >> 3) & 1) * 4 + (t & 3);
+}
 
-__global__ __launch_bounds__(256) void attn_prefill_kernel(PrefillParams p) {
-    __shared__ __attribute__((aligned(16))) half_t ks[PF_TW][ATT_KPITCH];
-    __shared__ __attribute__((aligned(16))) half_t vt[ATT_D][PF_TW + 8];
+template <int QG>
+__global__ __launch_bounds__(128 * QG, 1) void attn_prefill_kernel(PrefillParams p) {
+    constexpr int NW = 2 * QG;
+    constexpr int TILE = PF_TW * ATT_D;                    // halves of a K or V tile
+    extern __shared__ __attribute__((aligned(16))) half_t pf_lds[];       // [buffer 2][key group 2][K | V] tiles
     const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
-    const int qb = gridDim.x - 1 - blockIdx.x, h = blockIdx.y, hk = h / p.n_rep;     // longest walks are dispatched first
-    const int q_lo = 64 * qb + 16 * wave;                  // this wave's first query position
-    const int my_q = q_lo + c;                             // this lane's query (column c of the tiles)
-    const int last_key = min(64 * qb + 63, p.S - 1);       // the workgroup's diagonal
-    const int n_tiles = last_key / PF_TW + 1;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 31, hi = lane >> 5;
+    const int qg = wave % QG, kg = wave / QG;
+    const int n_qb = (p.S + 32 * QG - 1) / (32 * QG);
+    const int qb = n_qb - 1 - blockIdx.x / p.H, h = blockIdx.x % p.H, hk = h / p.n_rep;
+    const int q_lo = 32 * (QG * qb + qg);                  // this wave's first query position
+    const int my_q = q_lo + c;                             // this lane's query
+    const int last_key = min(32 * QG * (qb + 1), p.S) - 1; // the workgroup's diagonal
+    const int n_iter = last_key / (2 * PF_TW) + 1;         // pairs of tiles
+    auto k_tile = [&](int buf, int g) { return pf_lds + (2 * (2 * buf + g)) * TILE; };
+    auto v_tile = [&](int buf, int g) { return pf_lds + (2 * (2 * buf + g) + 1) * TILE; };
 
-    // B operand of S^T = K . Q^T: dims 32 k4 + 8g .. +7 of query row c
-    h8 qbop[4];
+    h8 qop[8];                                             // B operand of S^T: dims 16 k + 8 hi .. of query c
     {
-        const half_t *qp = p.q + ((long)min(my_q, p.S - 1) * p.H + h) * ATT_D + 8 * g;
+        const half_t *qp = p.q + ((long)min(my_q, p.S - 1) * p.H + h) * ATT_D + 8 * hi;
 #pragma unroll
-        for (int k4 = 0; k4 < 4; ++k4) qbop[k4] = *reinterpret_cast<const h8 *>(qp + 32 * k4);
+        for (int k = 0; k < 8; ++k) qop[k] = *reinterpret_cast<const h8 *>(qp + 16 * k);
     }
-    constexpr int PER = PF_TW * 16 / 256;                  // 16-byte pieces of K (and of V) per thread and tile
-    u32x4 kreg[PER], vreg[PER];
-    // a thread moves piece ch (8 dims) of FOUR consecutive keys, so that V goes to its transposed tile as 8-byte stores
-    static_assert(PER == 4, "four keys per thread");
-    auto tile_load = [&](int kt) {
+    const half_t *kbase = p.k + (long)hk * ATT_D, *vbase = p.v + (long)hk * ATT_D;
+    const long row_stride = (long)p.Hkv * ATT_D;
+    // K: instruction i of this wave moves four rows of the pair of tiles, lane -> (row lane / 16, slot lane % 16)
+    auto k_fetch = [&](int it, int buf) {
 #pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const int t = 4 * (tid >> 4) + i, ch = tid & 15;
-            const int row = kt * PF_TW + t;
-            kreg[i] = u32x4{0, 0, 0, 0}; vreg[i] = u32x4{0, 0, 0, 0};
-            if (row < p.S) {
-                const long off = ((long)row * p.Hkv + hk) * ATT_D + ch * 8;
-                kreg[i] = *reinterpret_cast<const u32x4 *>(p.k + off);
-                vreg[i] = *reinterpret_cast<const u32x4 *>(p.v + off);
-            }
+        for (int i = 0; i < 32 / NW; ++i) {
+            const int r4 = (32 / NW) * wave + i, r = 4 * r4 + (lane >> 4);             // row inside the pair
+            const int row = min(it * 2 * PF_TW + r, p.S - 1);
+            __builtin_amdgcn_global_load_lds((att_gptr_t)(kbase + (row * row_stride + 8 * ((lane & 15) ^ (r & 15)))),
+                                             (att_lptr_t)(k_tile(buf, r4 >> 4) + (r4 & 15) * 4 * ATT_D), 16, 0, 0);
         }
     };
-    auto tile_store = [&]() {
-        const int t0 = 4 * (tid >> 4), ch = tid & 15;
+    // V: a thread moves 8 dims of FOUR consecutive keys, which sit side by side in a row of V^T
+    constexpr int VG = 8 / NW;                             // groups of four keys per thread
+    u32x4 vreg[VG][4];
+    const int ch = tid & 15;
+    auto v_fetch = [&](int it) {
 #pragma unroll
-        for (int i = 0; i < PER; ++i) *reinterpret_cast<u32x4 *>(&ks[t0 + i][ch * 8]) = kreg[i];
-        const int pos = vt_pos(t0);                            // keys t0 .. t0+3 sit side by side in a row of vt
-        const h8 v0 = __builtin_bit_cast(h8, vreg[0]), v1 = __builtin_bit_cast(h8, vreg[1]);
-        const h8 v2 = __builtin_bit_cast(h8, vreg[2]), v3 = __builtin_bit_cast(h8, vreg[3]);
+        for (int g = 0; g < VG; ++g)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) *reinterpret_cast<h4 *>(&vt[ch * 8 + j][pos]) = h4{v0[j], v1[j], v2[j], v3[j]};
+            for (int i = 0; i < 4; ++i) {
+                const int row = min(it * 2 * PF_TW + 4 * ((tid >> 4) + 4 * NW * g) + i, p.S - 1);
+                vreg[g][i] = *reinterpret_cast<const u32x4 *>(vbase + (row * row_stride + 8 * ch));
+            }
+    };
+    auto v_store = [&](int buf) {
+#pragma unroll
+        for (int g = 0; g < VG; ++g) {
+            const int t = 4 * ((tid >> 4) + 4 * NW * g);
+            half_t *vt = v_tile(buf, t / PF_TW);
+            const h8 v0 = __builtin_bit_cast(h8, vreg[g][0]), v1 = __builtin_bit_cast(h8, vreg[g][1]);
+            const h8 v2 = __builtin_bit_cast(h8, vreg[g][2]), v3 = __builtin_bit_cast(h8, vreg[g][3]);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) *reinterpret_cast<h4 *>(&vt[(8 * ch + j) * PF_TW + pv_slot(t % PF_TW, 8 * ch + j)]) = h4{v0[j], v1[j], v2[j], v3[j]};
+        }
     };
 
-    float m_run = -INFINITY, l_run = 0.f;                  // of query c (the same in the four lane groups)
-    f4 ot[8];                                              // O^T: element r of ot[dt] is dim 16 dt + 4g + r of query c
+    float m_run = -INFINITY, l_run = 0.f;                  // maximum of query c's raw scores (both lanes of the query); sum over this lane's keys
+    f16v ot[4];                                            // O^T: element r of ot[d] is dim 32 d + 8 (r / 4) + 4 hi + r % 4 of query c
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt) ot[dt] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) ot[d][r] = 0.f;
 
-    tile_load(0);
-    for (int kt = 0; kt < n_tiles; ++kt) {
-        __syncthreads();                                   // everyone is done with the previous tile
-        tile_store();
+    k_fetch(0, 0);
+    v_fetch(0);
+    v_store(0);
+    __syncthreads();                                       // (waits for the DMA too)
+    for (int it = 0; it < n_iter; ++it) {
+        const int buf = it & 1, k_lo = (2 * it + kg) * PF_TW;
+        if (it + 1 < n_iter) {
+            k_fetch(it + 1, buf ^ 1);
+            v_fetch(it + 1);
+        }
+        if (k_lo <= q_lo + 31) {                           // (uniform over the wave) else every key lies after this wave's queries
+            const half_t *ks = k_tile(buf, kg), *vt = v_tile(buf, kg);
+            f16v st[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) st[j][r] = 0.f;
+                const int r = 32 * j + c;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const h8 ka = *reinterpret_cast<const h8 *>(&ks[r * ATT_D + 8 * ((2 * k + hi) ^ (r & 15))]);
+                    st[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qop[k], st[j], 0, 0, 0);
+                }
+            }
+            if (k_lo + PF_TW - 1 > q_lo) {                 // the diagonal runs through this tile
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int key = k_lo + 32 * j + 8 * (r >> 2) + 4 * hi + (r & 3);
+                        st[j][r] = key <= my_q ? st[j][r] : -INFINITY;
+                    }
+            }
+            float mx = fmaxf(st[0][0], st[1][0]);
+#pragma unroll
+            for (int r = 1; r < 16; ++r) mx = fmaxf(fmaxf(st[0][r], st[1][r]), mx);
+            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            const bool grown = (mx - m_run) * p.scale_log2 > 8.0f;       // (true at the first key, false while there is none: NaN)
+            if (__any(grown)) {
+                const float m_new = fmaxf(m_run, mx);
+                const float alpha = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m_run - m_new) * p.scale_log2);
+                m_run = m_new;
+                l_run *= alpha;
+#pragma unroll
+                for (int d = 0; d < 4; ++d)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) ot[d][r] *= alpha;
+            }
+            const float m_scaled = m_run == -INFINITY ? 0.0f : m_run * p.scale_log2;
+            h8 pb[4];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(st[j][r], p.scale_log2, -m_scaled));     // masked keys: exp2(-inf) = 0
+                    l_run += e;
+                    pb[2 * j + (r >> 3)][r & 7] = (half_t)e;
+                }
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {                  // sixteen keys at a time
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    const int row = 32 * d + c;
+                    const h8 va = *reinterpret_cast<const h8 *>(&vt[row * PF_TW + (((2 * b + hi) ^ (row & 7) ^ ((row >> 3) & 7)) << 3)]);
+                    ot[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pb[b], ot[d], 0, 0, 0);
+                }
+            }
+        }
+        if (it + 1 < n_iter) v_store(buf ^ 1);
         __syncthreads();
-        if (kt + 1 < n_tiles) tile_load(kt + 1);
-        const int k_lo = kt * PF_TW;
-        if (k_lo > q_lo + 15) continue;                    // every key of this tile lies after this wave's queries
-        // 16-row sub-tiles that hold a key <= the wave's last query
-        const int subs = min(PF_TW / 16, (q_lo + 15 - k_lo) / 16 + 1);
-        f4 st[PF_TW / 16];
-        float mx = -INFINITY;
-#pragma unroll
-        for (int j = 0; j < PF_TW / 16; ++j) {
-            st[j] = f4{0.f, 0.f, 0.f, 0.f};
-            if (j < subs) {
-#pragma unroll
-                for (int k4 = 0; k4 < 4; ++k4) {
-                    h8 ka = *reinterpret_cast<const h8 *>(&ks[16 * j + c][32 * k4 + 8 * g]);
-                    st[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qbop[k4], st[j], 0, 0, 0);
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int key = k_lo + 16 * j + 4 * g + r;
-                const float sv = (j < subs && key <= my_q && key < p.S) ? st[j][r] * p.scale_log2 : -INFINITY;
-                st[j][r] = sv;
-                mx = fmaxf(mx, sv);
-            }
-        }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        const float m_new = fmaxf(m_run, mx);              // finite from the first tile on: key 0 precedes every query
-        const float alpha = exp2f(m_run - m_new);          // exp2(-inf) = 0 on the first tile
-        float sum = 0.f;
-#pragma unroll
-        for (int j = 0; j < PF_TW / 16; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float e = exp2f(st[j][r] - m_new);
-                st[j][r] = e;
-                sum += e;
-            }
-        sum += __shfl_xor(sum, 16, 64);
-        sum += __shfl_xor(sum, 32, 64);
-        l_run = l_run * alpha + sum;
-        m_run = m_new;
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt) ot[dt] *= alpha;
-#pragma unroll
-        for (int jj = 0; jj < PF_TW / 32; ++jj) {
-            if (2 * jj < subs) {
-                h8 pb;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    pb[r] = (half_t)st[2 * jj][r];
-                    pb[4 + r] = (half_t)st[2 * jj + 1][r];
-                }
-#pragma unroll
-                for (int dt = 0; dt < 8; ++dt) {
-                    h8 va = *reinterpret_cast<const h8 *>(&vt[16 * dt + c][32 * jj + 8 * g]);
-                    ot[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pb, ot[dt], 0, 0, 0);
-                }
-            }
-        }
     }
+    // ---- the second key group's state through LDS (the tiles are no longer needed) ----
+    float *part = reinterpret_cast<float *>(pf_lds) + (long)qg * (66 * 64) + lane;
+    if (kg == 1) {
+        part[0] = m_run;
+        part[64] = l_run;
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) part[(2 + 16 * d + r) * 64] = ot[d][r];
+    }
+    __syncthreads();
+    if (kg == 1) return;
+    const float m2 = part[0], m_new = fmaxf(m_run, m2);    // (finite: key 0 is in the first group's first tile)
+    const float a1 = __builtin_amdgcn_exp2f((m_run - m_new) * p.scale_log2), a2 = __builtin_amdgcn_exp2f((m2 - m_new) * p.scale_log2);
+    l_run = l_run * a1 + part[64] * a2;
+    l_run += __shfl_xor(l_run, 32, 64);
     if (my_q < p.S) {
         const float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
-        half_t *op = p.out + ((long)my_q * p.H + h) * ATT_D;
+        half_t *op = p.out + ((long)my_q * p.H + h) * ATT_D + 4 * hi;
 #pragma unroll
-        for (int dt = 0; dt < 8; ++dt) {
-            const h4 o = {(half_t)(ot[dt][0] * inv), (half_t)(ot[dt][1] * inv), (half_t)(ot[dt][2] * inv), (half_t)(ot[dt][3] * inv)};
-            *reinterpret_cast<h4 *>(op + 16 * dt + 4 * g) = o;
-        }
+        for (int d = 0; d < 4; ++d)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                h4 o;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) o[j] = (half_t)((ot[d][4 * i + j] * a1 + part[(2 + 16 * d + 4 * i + j) * 64] * a2) * inv);
+                *reinterpret_cast<h4 *>(op + 32 * d + 8 * i) = o;
+            }
     }
 }
+constexpr int PF_LDS = 8 * PF_TW * ATT_D * 2;              // 128 KB: one workgroup a compute unit
 
 // One wave per (branch b, query head h): the query heads of one kv head walk the same suffix rows in different
 // waves (the rows come from the cache after the first), so a wave's chain of memory round trips does not grow with
@@ -1252,8 +1314,7 @@ extern "C" int smh_shared_prefix_attn_qkv(const void *qkv_partial, int ksplit, v
     return launch_status();
 }
 
-// Causal prefill attention, expressed as the suffix kernel with "branch" = query position:
-// query s attends to rows 0..s of the same K/V tensors (batch stride 0, no shared prefix).
+// Causal prefill attention: query s attends to rows 0..s of the same K/V tensors.
 extern "C" int smh_prefill_attn(const void *q, const void *k, const void *v, void *out, int S, int H, int Hkv,
                                 int D, smh_stream_t stream) {
     using namespace smh;
@@ -1265,6 +1326,15 @@ extern "C" int smh_prefill_attn(const void *q, const void *k, const void *v, voi
     p.q = (const half_t *)q; p.k = (const half_t *)k; p.v = (const half_t *)v; p.out = (half_t *)out;
     p.S = S; p.H = H; p.Hkv = Hkv; p.n_rep = H / Hkv;
     p.scale_log2 = LOG2E / sqrtf((float)D);
-    hipLaunchKernelGGL(attn_prefill_kernel, dim3((unsigned)((S + 63) / 64), (unsigned)H), dim3(256), 0, (hipStream_t)stream, p);
+    // four query groups (128 queries) a workgroup share a staged tile; two where that would leave compute units without a workgroup
+    const long blocks4 = (long)((S + 127) / 128) * H, blocks2 = (long)((S + 63) / 64) * H;
+    SMH_REQUIRE(blocks2 < (1L << 31), "smh_prefill_attn: S=%d H=%d", S, H);
+    static const hipError_t lds_ok = [] {
+        const hipError_t e = hipFuncSetAttribute((const void *)attn_prefill_kernel<4>, hipFuncAttributeMaxDynamicSharedMemorySize, PF_LDS);
+        return e != hipSuccess ? e : hipFuncSetAttribute((const void *)attn_prefill_kernel<2>, hipFuncAttributeMaxDynamicSharedMemorySize, PF_LDS);
+    }();
+    if (lds_ok != hipSuccess) { set_error("smh_prefill_attn: the kernel's LDS could not be reserved: %s", hipGetErrorString(lds_ok)); return (int)lds_ok; }
+    if (blocks4 >= 256) hipLaunchKernelGGL(attn_prefill_kernel<4>, dim3((unsigned)blocks4), dim3(512), PF_LDS, (hipStream_t)stream, p);
+    else hipLaunchKernelGGL(attn_prefill_kernel<2>, dim3((unsigned)blocks2), dim3(256), PF_LDS, (hipStream_t)stream, p);
     return launch_status();
 }
