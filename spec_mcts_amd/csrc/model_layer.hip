@@ -27,10 +27,12 @@ static int layer_buffers(const smh_layer &L, int M, bool swiglu_in, char *base, 
     if (ks_qkv < 1 || ks_gu < 1 || ks_o < 1 || ks_d < 1) return -1;
     const size_t m = (size_t)M;
     auto most = [](size_t x, size_t y) { return x > y ? x : y; };
-    // (above 128 rows w1|w3 leaves no slabs where SwiGLU is made inside its launch: 4 bytes x rows x 2 ffn less)
+    // (a prefill's launches that store fp16 themselves leave no slabs)
     const bool gu_slabs = !(M > 128 && swiglu_in && smh_q40_swiglu_fits(M, L.dim, L.ffn));
-    b.slab_a_bytes = align_up(most(ks_qkv * m * (nq + 2 * (size_t)nkv), gu_slabs ? ks_gu * m * 2 * (size_t)L.ffn : 0) * sizeof(float));
-    b.slab_b_bytes = align_up((size_t)most(ks_o, ks_d) * m * L.dim * sizeof(float));
+    const bool qkv_slabs = smh_q40_matmul_tiled_direct_fits(M, L.dim, 3, n_qkv) != 1, o_slabs = smh_q40_matmul_tiled_direct_fits(M, nq, 1, n_dim) != 1;
+    const bool d_slabs = smh_q40_matmul_tiled_direct_fits(M, L.ffn, 1, n_dim) != 1;
+    b.slab_a_bytes = align_up(most(qkv_slabs ? ks_qkv * m * (nq + 2 * (size_t)nkv) : 1, gu_slabs ? ks_gu * m * 2 * (size_t)L.ffn : 1) * sizeof(float));
+    b.slab_b_bytes = align_up((size_t)most(o_slabs ? ks_o : 0, d_slabs ? ks_d : 0) * m * L.dim * sizeof(float));
     size_t at = 0;
     auto take = [&](size_t bytes) { char *p = base ? base + at : nullptr; at += align_up(bytes); return p; };
     b.h[0] = take(m * L.dim * 2);

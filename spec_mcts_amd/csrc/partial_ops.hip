@@ -98,6 +98,45 @@ __global__ __launch_bounds__(1024) void partial_rmsnorm_kernel(const void *__res
     }
 }
 
+// RMSNorm of rows that are already fp16: one workgroup of 256 threads a row, eight elements a load, the row kept in registers
+// (CH loads a thread).  2047 rows of 4096: 7.2 us; 1024 threads of four elements 16.5.
+template <int CH>
+__global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const half_t *__restrict__ h, const half_t *__restrict__ wt, int N, float eps,
+                                                           half_t *__restrict__ xn_out) {
+    __shared__ float s_part[4];
+    const half_t *row = h + (long)blockIdx.x * N;
+    h8 hv[CH], wv[CH];
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+        const int n = (i * 256 + threadIdx.x) * 8;
+        if (n < N) {
+            hv[i] = *reinterpret_cast<const h8 *>(row + n);
+            wv[i] = *reinterpret_cast<const h8 *>(wt + n);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < CH; ++i)
+        if ((i * 256 + (int)threadIdx.x) * 8 < N) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) ss = sumsq_add(ss, (float)hv[i][j]);
+        }
+    ss = wave_sum(ss);
+    if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    const float r = rms_factor(s_part[0] + s_part[1] + s_part[2] + s_part[3], N, eps);
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+        const int n = (i * 256 + threadIdx.x) * 8;
+        if (n < N) {
+            h8 o;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) o[j] = scale_to_half(hv[i][j], r) * wv[i][j];
+            *reinterpret_cast<h8 *>(xn_out + (long)blockIdx.x * N + n) = o;
+        }
+    }
+}
+
 // ---- residual add + sums of squares (the first half of partial_rmsnorm_kernel, spread over 16 workgroups a row) ----
 // grid (16, M), one wave each: wave w of a row is wave w of partial_rmsnorm_kernel's workgroup (same columns per
 // thread, same order of additions), so sums[m][0..15] added in index order give that kernel's sum of squares bit
@@ -507,6 +546,11 @@ extern "C" int smh_partial_rmsnorm(const void *partial, int ksplit, int M, int N
     SMH_REQUIRE(partial != nullptr || h_in != nullptr, "smh_partial_rmsnorm: no input");
     if (M == 0) return 0;
     SMH_REQUIRE(weight && xn_out, "smh_partial_rmsnorm: null pointer");
+    if (partial == nullptr && h_out == nullptr && N % 8 == 0 && (((uintptr_t)h_in | (uintptr_t)weight | (uintptr_t)xn_out) & 15) == 0) {
+        const auto kern = N <= 4096 ? rmsnorm_rows_kernel<2> : N <= 8192 ? rmsnorm_rows_kernel<4> : rmsnorm_rows_kernel<8>;
+        hipLaunchKernelGGL(kern, dim3(M), dim3(256), 0, (hipStream_t)stream, (const half_t *)h_in, (const half_t *)weight, N, eps, (half_t *)xn_out);
+        return launch_status();
+    }
     hipLaunchKernelGGL(partial_rmsnorm_kernel, dim3(M), dim3(1024), 0, (hipStream_t)stream, partial, ksplit, M, N,
                        (const half_t *)h_in, (const half_t *)weight, eps, (half_t *)h_out, (half_t *)xn_out);
     return launch_status();

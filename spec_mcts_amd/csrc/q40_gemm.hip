@@ -1043,30 +1043,35 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_swiglu_kernel(MatmulParams p)
     }
 }
 
-// Rows of a block when M > 128 rows are cut into blocks of at most 128: as even as whole tiles of 16 allow (130 rows are two
-// blocks of 80, not 128 and 2 rows of which both multiply 128).
-static int gemm_even_rows(int M) {
-    const int mblocks = (M + GEMM_BM - 1) / GEMM_BM;
-    return ((M + mblocks - 1) / mblocks + 15) / 16 * 16;
+// Row blocks and K-slices of a launch with more than 128 rows: the pair with the least estimated time.  Measured on the 7B shapes
+// at 160 .. 2047 rows: a workgroup takes 0.18 us a step and 0.24 more at 128 rows (in proportion), 4 us around its loop; a launch
+// takes as many of these as its workgroups need rounds over 256 compute units, and at least 1.2 times its share of them when all
+// compute units are busy (the clock drops: two workgroups that share a compute unit take as long as one behind the other).  A
+// split's consumer reads 4 bytes an output and slice at ~4 TB/s.  Blocks are even (130 rows: two of 80, not 128 and 2).
+// (Before, 128-row blocks and at most 1600 / M slices: w1|w3 at 300 rows 108 us, now 85; wo and w2 at 1024 rows 56 and 136, now
+// 37 and 88; 700 rows of wq|wk|wv 108, now 89.)
+static float gemm_rows_us(long tiles, int rows, int steps) {
+    const float r = (float)tiles / 256.0f, rounds = (float)((tiles + 255) / 256);
+    return (rounds > 1.2f * r ? rounds : 1.2f * r) * ((float)steps * (0.18f + 0.24f * rows / GEMM_BM) + 4.0f);
 }
-
-// K-slices of a launch with more than 128 rows: the split with the least estimated time.  A workgroup takes ~0.46 us a step at
-// 128 rows (0.09 + 0.37 of that in proportion to its rows) and ~5 us around its loop; the launch takes as many rounds as its
-// workgroups need compute units; every slice of a split writes fp32 slabs that the consumer reads back (8 bytes an output at
-// ~4.5 TB/s).  (A cap by rows alone gave 1024 rows of wo and w2 one slice, 128 workgroups on 256 compute units: 56 and 136 us.)
-static void gemm_plan_rows(MatmulParams &p, int steps) {
-    p.block_rows = gemm_even_rows(p.M);
-    p.mblocks = (p.M + p.block_rows - 1) / p.block_rows;
-    const long tiles = (long)p.units * p.mblocks;
-    int best = 1;
-    float best_us = 0.f;
-    for (int ks = 1; ks <= SMH_MAX_KSPLIT && (ks == 1 || (tiles * ks <= 512 && steps / ks >= GEMM_STAGES)); ++ks) {
-        const float rounds = (float)((tiles * ks + 255) / 256);
-        const float us = rounds * ((float)((steps + ks - 1) / ks) * (0.09f + 0.37f * p.block_rows / GEMM_BM) + 5.0f) +
-                         (ks > 1 ? (float)ks * p.M * p.n_total * 8.0f / 4.5e6f : 0.0f);
-        if (ks == 1 || us < best_us) { best = ks; best_us = us; }
+static void gemm_plan_rows(MatmulParams &p, int steps, int max_ks) {
+    float best_us = -1.0f;
+    int ksplit = 1;
+    for (int mb = (p.M + GEMM_BM - 1) / GEMM_BM; mb <= p.M / 64; ++mb) {                // (blocks of 64 .. 128 rows)
+        const int rows = ((p.M + mb - 1) / mb + 15) / 16 * 16;
+        const int blocks = (p.M + rows - 1) / rows;
+        const long tiles = (long)p.units * blocks;
+        for (int ks = 1; ks <= max_ks && (ks == 1 || (tiles * ks <= 512 && steps / ks >= GEMM_STAGES)); ++ks) {
+            const float us = gemm_rows_us(tiles * ks, rows, (steps + ks - 1) / ks) + (ks > 1 ? (float)ks * p.M * p.n_total * 4.0f / 4.0e6f : 0.0f);
+            if (best_us < 0.0f || us < best_us) {
+                best_us = us;
+                ksplit = ks;
+                p.block_rows = rows;
+                p.mblocks = blocks;
+            }
+        }
     }
-    p.steps_per_slice = (steps + best - 1) / best;
+    p.steps_per_slice = (steps + ksplit - 1) / ksplit;
     p.ksplit = (steps + p.steps_per_slice - 1) / p.steps_per_slice;
     p.chunk = 0;
 }
@@ -1123,7 +1128,7 @@ void gemm_fill_plan(MatmulParams &p) {
     p.mblocks = (p.M + p.block_rows - 1) / p.block_rows;
     const int steps = (p.K + 31) / 32;
     if (p.M > GEMM_BM) {
-        gemm_plan_rows(p, steps);
+        gemm_plan_rows(p, steps, SMH_MAX_KSPLIT);
         return;
     }
     const long tiles = (long)p.units * p.mblocks;
@@ -1275,33 +1280,20 @@ int gemm_swiglu_launch(const MatmulParams &p, hipStream_t stream) {
     return launch_status();
 }
 
-// More than 128 rows (a prefill) on tiled weights.  Without a K-split a launch stores fp16 results itself: no fp32 slabs (4 bytes
+// More than 128 rows (a prefill) on tiled weights: without a K-split a launch stores fp16 results itself - no fp32 slabs (4 bytes
 // an output and slice written here and read behind) and no kernel to add them.
-static int gemm_rows_setup(MatmulParams &p, int units) {
-    p.units = units;
-    p.units_pad = (units + 7) / 8 * 8;
-    p.block_rows = gemm_even_rows(p.M);
-    p.mblocks = (p.M + p.block_rows - 1) / p.block_rows;
-    p.kgroups = 0;
-    p.chunk = 0;
-    p.ksplit = 1;
-    p.steps_per_slice = p.K / 32;
-    p.direct = 1;
-    return p.units * p.mblocks;
-}
-
 bool gemm_direct_fits(const MatmulParams &p) { return p.tiled && p.M > GEMM_BM && p.K % 32 == 0 && p.ksplit == 1; }
 
 int gemm_swiglu_rows_launch(MatmulParams p, hipStream_t stream) {
-    // (more than 128 rows in even blocks: five to eight tiles)
+    // (blocks of 64 .. 128 rows)
     constexpr int S = GEMM_DMA_WAVE_SLOTS;
-    static const gemm_kernel_t plain[4] = {q40_gemm_kernel<5, false, true, 8, GEMM_STAGES, false, false, true>, q40_gemm_kernel<6, false, true, 8, GEMM_STAGES, false, false, true>,
+    static const gemm_kernel_t plain[5] = {q40_gemm_kernel<4, false, true, 8, GEMM_STAGES, false, false, true>, q40_gemm_kernel<5, false, true, 8, GEMM_STAGES, false, false, true>, q40_gemm_kernel<6, false, true, 8, GEMM_STAGES, false, false, true>,
                                            q40_gemm_kernel<7, false, true, 8, GEMM_STAGES, false, false, true>, q40_gemm_kernel<8, false, true, 8, GEMM_STAGES, false, false, true>};
-    static const gemm_kernel_t dma_wave[4] = {q40_gemm_kernel<5, false, true, 8, S, true, false, true>, q40_gemm_kernel<6, false, true, 8, S, true, false, true>,
+    static const gemm_kernel_t dma_wave[5] = {q40_gemm_kernel<4, false, true, 8, S, true, false, true>, q40_gemm_kernel<5, false, true, 8, S, true, false, true>, q40_gemm_kernel<6, false, true, 8, S, true, false, true>,
                                               q40_gemm_kernel<7, false, true, 8, S, true, false, true>, q40_gemm_kernel<8, false, true, 8, S, true, false, true>};
     static const hipError_t lds_ok = [] {
         hipError_t e = hipSuccess;
-        for (int t = 0; t < 4 && e == hipSuccess; ++t) {
+        for (int t = 0; t < 5 && e == hipSuccess; ++t) {
             e = hipFuncSetAttribute((const void *)plain[t], hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS);
             if (e == hipSuccess) e = hipFuncSetAttribute((const void *)dma_wave[t], hipFuncAttributeMaxDynamicSharedMemorySize, S * GS_BYTES);
         }
@@ -1312,8 +1304,12 @@ int gemm_swiglu_rows_launch(MatmulParams p, hipStream_t stream) {
         return (int)lds_ok;
     }
     SMH_REQUIRE((long)p.M * p.lda * 2 < (1L << 32), "q40 gemm: M x lda = %d x %ld exceeds the 32-bit lane offsets of A", p.M, p.lda);
-    const bool one_each = gemm_rows_setup(p, p.seg[0].N / 128) <= GEMM_DMA_WAVE_MAX_WGS;
-    const int t = p.block_rows / 16 - 5;
+    p.units = p.seg[0].N / 128;
+    p.units_pad = (p.units + 7) / 8 * 8;
+    p.kgroups = 0;
+    gemm_plan_rows(p, p.K / 32, 1);
+    const bool one_each = (long)p.units * p.mblocks <= GEMM_DMA_WAVE_MAX_WGS;
+    const int t = p.block_rows / 16 - 4;
     hipLaunchKernelGGL((one_each ? dma_wave : plain)[t], dim3((unsigned)((long)p.units_pad * p.mblocks)), dim3(512 + (one_each ? 64 : 0)),
                        one_each ? S * GS_BYTES : GEMM_LDS, stream, p);
     return launch_status();
