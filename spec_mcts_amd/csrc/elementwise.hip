@@ -242,10 +242,16 @@ namespace smh {
 // probabilities p = fp16(softmax) as F.softmax on an fp16 tensor returns them, and one candidate is drawn by inverse
 // CDF with the caller's uniform number.
 constexpr int SAMPLE_MAX_K = 1024;
+constexpr int SAMPLE_PICK_MAX_K = 512;         // up to here the candidates are picked by the threads' maxima (above, they would be thousands)
 
 __device__ __forceinline__ uint32_t sample_key(half_t x) {
     const uint32_t b = __builtin_bit_cast(uint16_t, x);
     return (b & 0x8000u) ? (~b & 0xFFFFu) : (b | 0x8000u);       // larger value <=> larger key
+}
+// ... of two fp16 values in one word
+__device__ __forceinline__ uint32_t sample_keys2(uint32_t b) {
+    const uint32_t neg = ((b >> 15) & 0x00010001u) * 0xFFFFu;       // 0xFFFF in the halves that are negative
+    return b ^ (neg | 0x80008000u);
 }
 __device__ __forceinline__ half_t sample_unkey(uint32_t k) {
     const uint16_t b = (uint16_t)((k & 0x8000u) ? (k & 0x7FFFu) : (~k & 0xFFFFu));
@@ -286,9 +292,11 @@ __device__ __forceinline__ void sample_pick_bin(int *bins, int *s_w, int want, i
 
 // counts == nullptr: one draw per row, uniform[row] -> out[row].  Otherwise row r makes counts[r] draws with replacement from
 // its candidates, with the uniform numbers (and into the slots of out) that start at counts[0] + ... + counts[r-1].
-// Thread t owns the contiguous chunk of ceil(vocab / 1024) logits that starts at t times that.  Up to 32768 logits (a multiple
-// of 8, rows 16-byte aligned) the chunk is read ONCE, as four 16-byte loads, and its 32 sixteen-bit keys stay in registers for
-// the two histogram passes, the tie count and the gather; otherwise every pass reads the logits again.
+// Up to 32768 logits (a multiple of 8, rows 16-byte aligned) and k <= 512 the row is read once into registers and the candidates
+// are those not below the k-th largest of the threads' maxima (a handful more than k): no histogram of the whole row, whose LDS
+// atomics pile up on the few bins that logits fall into.  80 rows of 32016, k = 32: 35 us with histograms, 11 like this.
+// Otherwise, and where the maxima leave more than 1024 candidates (ordered or mostly equal logits), two histogram passes: thread
+// t owns the contiguous chunk of ceil(vocab / 1024) logits that starts at t times that.
 __global__ __launch_bounds__(1024) void sample_topk_kernel(const half_t *__restrict__ logits, int vocab, long ld, float temperature,
                                                            int top_k, const float *__restrict__ uniform, int64_t *__restrict__ out,
                                                            const int32_t *__restrict__ counts, const float *__restrict__ row_temps, int n_draws,
@@ -305,11 +313,11 @@ __global__ __launch_bounds__(1024) void sample_topk_kernel(const half_t *__restr
     const bool greedy_row = row_temps != nullptr && !(temperature > 0.f);
     if (greedy_row) temperature = 1.0f;
     __shared__ int bins[256];
-    __shared__ int wbins[256 * 16];
+    __shared__ __attribute__((aligned(16))) int wbins[256 * 16];
     __shared__ int s_wi[16];
     __shared__ float s_wf[16];
     __shared__ int s_bin, s_above, s_count;
-    __shared__ uint32_t c_key[SAMPLE_MAX_K];
+    __shared__ __attribute__((aligned(16))) uint32_t c_key[SAMPLE_MAX_K];
     __shared__ int c_idx[SAMPLE_MAX_K];
     __shared__ uint32_t o_key[SAMPLE_MAX_K];
     __shared__ int o_idx[SAMPLE_MAX_K];
@@ -319,13 +327,126 @@ __global__ __launch_bounds__(1024) void sample_topk_kernel(const half_t *__restr
     int k = min(top_k, vocab);
     auto key_of = [&](half_t x) { return sample_key(wide ? x : (half_t)((float)x / temperature)); };
     auto value_of = [&](uint32_t key) { return wide ? (float)sample_unkey(key) / temperature : (float)sample_unkey(key); };
+    const int wv = tid >> 6;
 
     constexpr int CH = 32;
     const bool in_regs = vocab <= 1024 * CH && vocab % 8 == 0 && (reinterpret_cast<uintptr_t>(row) & 15) == 0;     // (uniform)
-    const int chunk = in_regs ? CH : (vocab + 1023) / 1024;
+    bool found = false;                        // the candidates are in o_key / o_idx, in order
+    if (in_regs && k <= SAMPLE_PICK_MAX_K) {
+        // ---- candidates by the threads' maxima ----
+        // At least k logits are not below the k-th largest of the 1024 threads' own maxima, so the k largest are among those
+        // that are not (about k + k^2 / 64 of them for unordered logits).  Order and equality are those of the
+        // quotients; the quotient is monotonic, so the logits themselves are compared, down to the smallest one with the same
+        // quotient.
+        uint32_t raw[CH / 2];
+#pragma unroll
+        for (int q = 0; q < CH / 8; ++q) {
+            const int i = 8 * (tid + 1024 * q);
+            u32x4 v = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu};       // key 0: below every number
+            if (i < vocab) v = *reinterpret_cast<const u32x4 *>(row + i);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) raw[4 * q + j] = sample_keys2(v[j]);
+        }
+        uint32_t mx = 0;
+#pragma unroll
+        for (int j = 0; j < CH / 2; ++j) mx = max(mx, max(raw[j] & 0xFFFFu, raw[j] >> 16));
+        uint32_t *maxima = reinterpret_cast<uint32_t *>(wbins);
+        maxima[tid] = mx;
+        if (tid == 0) s_count = 0;
+        __syncthreads();
+        uint32_t mine[16];                     // every wave holds all the maxima ...
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const u32x4 v = *reinterpret_cast<const u32x4 *>(&maxima[256 * j + 4 * (tid & 63)]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) mine[4 * j + e] = v[e];
+        }
+        uint32_t thr = 0;
+#pragma unroll
+        for (int shift = 12; shift >= 0; shift -= 4) {         // ... and counts those at or above one value of the next four bits
+            const uint32_t t = thr | ((uint32_t)wv << shift);
+            int n = 0;
+#pragma unroll
+            for (int j = 0; j < 16; ++j) n += __popcll(__ballot(mine[j] >= t));
+            int *slot = bins + 16 * (shift >> 2);
+            if ((tid & 63) == 0) slot[wv] = n;
+            __syncthreads();
+            int d = 0;
+#pragma unroll
+            for (int w = 1; w < 16; ++w) d = slot[w] >= k ? w : d;
+            thr |= (uint32_t)d << shift;
+        }
+        bool small = true;
+        if (!wide) {
+            const uint32_t q = key_of(sample_unkey(thr));
+            int steps = 0;
+            while (thr > 0 && steps < 64 && key_of(sample_unkey(thr - 1)) == q) { --thr; ++steps; }
+            small = steps < 64;
+        }
+        int n = 0;
+        if (small) {
+#pragma unroll
+            for (int j = 0; j < CH / 2; ++j) n += ((raw[j] & 0xFFFFu) >= thr) + ((raw[j] >> 16) >= thr);
+            const bool real = thr > 0;                          // (key 0: also the slots past the row)
+            int at = n > 0 && real ? atomicAdd(&s_count, n) : 0;
+            if (!real) at = SAMPLE_MAX_K;
+            if (n > 0) {
+#pragma unroll
+                for (int j = 0; j < CH; ++j) {
+                    const uint32_t key = (raw[j >> 1] >> (16 * (j & 1))) & 0xFFFFu;
+                    if (key >= thr) {
+                        // key above 32767 - index: one comparison orders by value, then by index
+                        const uint32_t i = 8 * (tid + 1024 * (j >> 3)) + (j & 7);
+                        if (at < SAMPLE_MAX_K) c_key[at] = ((wide ? key : key_of(sample_unkey(key))) << 15) | (32767u - i);
+                        ++at;
+                    }
+                }
+            }
+            if (!real && tid == 0) s_count = SAMPLE_MAX_K + 1;
+            __syncthreads();
+            const int count = s_count;
+            if (count <= SAMPLE_MAX_K) {
+                // rank = number of candidates that come before.  1024 / (count, rounded up to a power of two) threads share a
+                // candidate, each comparing it with every so-many-th quad of the others (the same for all lanes of a wave).
+                int pow2 = 64;
+                while (pow2 < count) pow2 <<= 1;
+                const int cand = tid & (pow2 - 1), part = tid / pow2, parts = 1024 / pow2;
+                const uint32_t mine_c = cand < count ? c_key[cand] : 0u;
+                if (tid < 1024 - count) c_key[count + tid] = 0u;           // (below every candidate)
+                c_idx[tid] = 0;
+                __syncthreads();
+                int rank = 0;
+                for (int j = 4 * part; j < count; j += 4 * parts) {
+                    const u32x4 v = *reinterpret_cast<const u32x4 *>(&c_key[j]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) rank += v[e] > mine_c;
+                }
+                if (parts > 1) {
+                    if (cand < count && rank > 0) atomicAdd(&c_idx[cand], rank);
+                    __syncthreads();
+                    rank = c_idx[cand];
+                }
+                if (part == 0 && cand < count) {
+                    o_key[rank] = mine_c >> 15;
+                    o_idx[rank] = 32767 - (int)(mine_c & 32767u);
+                }
+                __syncthreads();
+                if (keep_ties) {                               // every value equal to the k-th
+                    const uint32_t kth = o_key[k - 1];
+                    k += __syncthreads_count(tid >= k && tid < count && o_key[tid] == kth);
+                }
+                found = true;
+            }
+        }
+    }
+    if (!found) {
+    // ---- by histograms: many candidates, or rows that cannot be held in registers ----
+    __syncthreads();
+    const bool hold = in_regs && top_k > SAMPLE_PICK_MAX_K;
+    const int chunk = hold ? CH : (vocab + 1023) / 1024;
     const int lo = min(tid * chunk, vocab), hi = min(vocab, lo + chunk);
-    uint32_t kr[CH / 2];                       // in_regs: keys of elements lo + 2 j (low half) and lo + 2 j + 1
-    if (in_regs) {
+    uint32_t kr[CH / 2];                       // hold: keys of elements lo + 2 j (low half) and lo + 2 j + 1
+    if (hold) {
         u32x4 raw[CH / 8];
 #pragma unroll
         for (int q = 0; q < CH / 8; ++q) {
@@ -342,7 +463,7 @@ __global__ __launch_bounds__(1024) void sample_topk_kernel(const half_t *__restr
     }
     // f(index, key) for every logit of this thread's chunk, in index order
     auto for_each = [&](auto f) {
-        if (in_regs) {
+        if (hold) {
 #pragma unroll
             for (int j = 0; j < CH; ++j)
                 if (lo + j < hi) f(lo + j, (kr[j >> 1] >> (16 * (j & 1))) & 0xFFFFu);
@@ -354,7 +475,6 @@ __global__ __launch_bounds__(1024) void sample_topk_kernel(const half_t *__restr
     // ---- the k-th largest key: high byte, then low byte ----
     // Atomics of different waves on one LDS word take turns, and logits crowd into a few high bytes: every wave counts into a
     // histogram of its own (word = bin * 16 + wave, the 16 copies of a bin in 16 banks), which are then added.
-    const int wv = tid >> 6;
     auto fold_bins = [&]() {
         if (tid < 256) {
             int n = 0;
@@ -416,34 +536,62 @@ __global__ __launch_bounds__(1024) void sample_topk_kernel(const half_t *__restr
     }
     __syncthreads();
 
+    }
+
     // ---- p = fp16(softmax) (fp32 with a row temperature or the filter form), inverse CDF ----
     const float xmax = value_of(o_key[0]);
     const float e = tid < k ? expf(value_of(o_key[tid]) - xmax) : 0.f;
-    cdf[tid] = sample_block_scan(e, s_wf);
-    __syncthreads();
-    const float total = cdf[k - 1];
-    __syncthreads();
-    const float pr = tid < k ? (wide ? e / total : (float)(half_t)(e / total)) : 0.f;
-    cdf[tid] = sample_block_scan(pr, s_wf);
-    __syncthreads();
+    const bool one_wave = k <= 64;             // every candidate in the first wave: the same sums without the workgroup's barriers
+    auto wave_scan = [&](float v) {
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const float u = __shfl_up(v, o, 64);
+            if ((tid & 63) >= o) v += u;
+        }
+        return v;
+    };
+    float upto, before, all;                   // cumulative probability with and without candidate tid, and of all
+    if (one_wave) {
+        if (tid >= 64) return;
+        const float total = __shfl(wave_scan(e), k - 1, 64);
+        const float pr = tid < k ? (wide ? e / total : (float)(half_t)(e / total)) : 0.f;
+        upto = wave_scan(pr);
+        all = __shfl(upto, k - 1, 64);
+        before = __shfl_up(upto, 1, 64);
+        if (tid == 0) before = 0.f;
+    } else {
+        cdf[tid] = sample_block_scan(e, s_wf);
+        __syncthreads();
+        const float total = cdf[k - 1];
+        __syncthreads();
+        const float pr = tid < k ? (wide ? e / total : (float)(half_t)(e / total)) : 0.f;
+        cdf[tid] = sample_block_scan(pr, s_wf);
+        __syncthreads();
+        upto = cdf[tid];
+        before = tid == 0 ? 0.f : cdf[tid - 1];
+        all = cdf[k - 1];
+    }
     long first = blockIdx.x;
     int draws = 1;
     if (counts != nullptr) {
-        first = 0;
-        for (int r = 0; r < (int)blockIdx.x; ++r) first += max(counts[r], 0);
+        // every wave adds the counts of the rows before this one (all loads together, not one behind the other)
+        int sum = 0;
+        for (int r = tid & 63; r < (int)blockIdx.x; r += 64) sum += max(counts[r], 0);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+        first = sum;
         draws = max(counts[blockIdx.x], 0);
         draws = (int)max(min((long)draws, (long)n_draws - first), 0L);       // counts that add up to more than the buffers hold are cut
     }
     if (greedy_row) {
-        for (int j = tid; j < draws; j += 1024) out[first + j] = o_idx[0];
+        for (int j = tid; j < draws; j += one_wave ? 64 : 1024) out[first + j] = o_idx[0];
         return;
     }
     if (tid < k) {
-        const float before = tid == 0 ? 0.f : cdf[tid - 1];
         for (int j = 0; j < draws; ++j) {
-            const float target = uniform[first + j] * cdf[k - 1];
+            const float target = uniform[first + j] * all;
             // first candidate whose cumulative probability exceeds the target (the last one if rounding leaves none)
-            if ((before <= target && target < cdf[tid]) || (tid == k - 1 && target >= cdf[tid])) out[first + j] = o_idx[tid];
+            if ((before <= target && target < upto) || (tid == k - 1 && target >= upto)) out[first + j] = o_idx[tid];
         }
     }
 }
@@ -635,6 +783,146 @@ __global__ __launch_bounds__(256) void tree_fork_kernel(const int64_t *__restric
     }
 }
 
+// The same step for batches and draws of at most 256: a thread is a branch, a draw, a row in turn.  Nothing is walked by one
+// thread: a draw finds its rank among its branch's distinct tokens by comparing it with its branch's other draws (one, once the
+// tree has its full batch), the rows of the forks come from a prefix sum (a branch's first new row is c0 + the forks of the
+// branches before it, cut at the batch), and everything that depends on no other load is requested at the start.  At 80
+// branches: 28 us for tree_fork_kernel (whose first thread reads the counts and the live flags one behind the other), 4.4 here.
+constexpr int TREE_SMALL = 256;
+__global__ __launch_bounds__(TREE_SMALL) void tree_small_kernel(const int64_t *__restrict__ draws, int n_draws, int32_t *__restrict__ tok, int32_t *__restrict__ cnt,
+                                                                uint8_t *__restrict__ alive, int32_t *__restrict__ curr_b, int batch_size,
+                                                                int64_t *__restrict__ results, long ld, int t,
+                                                                int32_t *__restrict__ pages, long pages_stride, int n_rows,
+                                                                int32_t *__restrict__ origin, const int32_t *__restrict__ t_dev, TreeFinish fin) {
+    __shared__ uint32_t d_tok[TREE_SMALL];         // token of draw i
+    __shared__ uint8_t d_head[TREE_SMALL];         // draw i is the first of its branch with its token
+    __shared__ int seg[TREE_SMALL + 1];            // first draw of branch i
+    __shared__ int uniq[TREE_SMALL], row0[TREE_SMALL];
+    __shared__ int r_tok[TREE_SMALL], r_cnt[TREE_SMALL], r_origin[TREE_SMALL];
+    __shared__ uint8_t r_set[TREE_SMALL], b_alive[TREE_SMALL];
+    __shared__ int s_w[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // inclusive prefix sum over the workgroup; every thread calls
+    auto block_scan = [&](int v) {
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int u = __shfl_up(v, o, 64);
+            if (lane >= o) v += u;
+        }
+        if (lane == 63) s_w[wave] = v;
+        __syncthreads();
+        for (int w = 0; w < wave; ++w) v += s_w[w];
+        __syncthreads();
+        return v;
+    };
+    const bool is_row = tid < batch_size;
+    const int c0 = min(max(*curr_b, 0), batch_size);             // (a counter outside the batch is cut, never followed)
+    if (t_dev != nullptr) t = *t_dev;
+    const int my_cnt = is_row ? cnt[tid] : 0;
+    const bool was = is_row && alive[tid] != 0;
+    const uint32_t my_tok = tid < n_draws ? (uint32_t)draws[tid] : 0u;
+    int32_t st = 0, len = 0;
+    if (is_row && fin.state != nullptr) { st = fin.state[tid]; len = fin.results_len[tid]; }
+    if (t_dev != nullptr) {
+        t = min(max(t, 0), (int)ld - 1);                         // (a counter outside the row is cut, never followed)
+        n_rows = (int)min((long)t, pages_stride);
+    }
+    const int64_t old_token = is_row ? results[(long)tid * ld + t] : 0;
+    const int64_t seq_token = is_row && fin.state != nullptr && st >= 0 && st < fin.seq_len ? fin.seq[st] : 0;
+
+    d_tok[tid] = my_tok;
+    uniq[tid] = 0;
+    r_set[tid] = 0;
+    r_origin[tid] = -1;
+    b_alive[tid] = was ? 1 : 0;
+    const int upto = block_scan(tid < c0 ? min(max(my_cnt, 0), TREE_MAX_BATCH) : 0);
+    seg[tid + 1] = upto;
+    if (tid == 0) seg[0] = 0;
+    __syncthreads();
+    const int total = min(seg[c0], n_draws);                     // draws the buffer does not hold do not exist
+    // ---- this thread's draw: its branch, whether it is the first with its token there, and how many are equal ----
+    int br = 0, lo = 0, hi = 0, mult = 0;
+    bool head = tid < total;
+    if (tid < total) {
+        int b1 = c0 - 1;
+        while (br < b1) {
+            const int mid = (br + b1 + 1) >> 1;
+            if (seg[mid] <= tid) br = mid; else b1 = mid - 1;
+        }
+        lo = min(seg[br], total);
+        hi = min(seg[br + 1], total);
+        for (int j = lo; j < hi; ++j) {
+            const bool same = d_tok[j] == my_tok;
+            mult += same;
+            if (same && j < tid) head = false;
+        }
+    }
+    d_head[tid] = head ? 1 : 0;
+    if (head) atomicAdd(&uniq[br], 1);
+    __syncthreads();
+    // ---- rows of the forks, branch by branch ----
+    const int forks = (tid < c0 && was && uniq[tid] > 0) ? uniq[tid] - 1 : 0;
+    const int end = block_scan(forks);
+    row0[tid] = c0 + end - forks;
+    if (tid == TREE_SMALL - 1) seg[TREE_SMALL] = end;            // (seg[256] is read only where 256 branches are live: before this scan)
+    __syncthreads();
+    const int c1 = min(batch_size, c0 + seg[TREE_SMALL]);
+    if (head && b_alive[br]) {
+        int rank = 0;                                            // distinct tokens of the branch below this one
+        for (int j = lo; j < hi; ++j) rank += d_head[j] && d_tok[j] < my_tok;
+        const int r = rank == 0 ? br : row0[br] + rank - 1;
+        if (r < batch_size) {
+            r_tok[r] = (int32_t)my_tok;
+            r_cnt[r] = mult;
+            r_set[r] = 1;
+            if (rank > 0) r_origin[r] = br;
+        }
+    }
+    __syncthreads();
+    // token histories (without this step's column) and page ids of the new rows
+    {
+        const int n_new = c1 - c0, n = n_new * (int)ld;
+        for (int i = tid; i < n; i += TREE_SMALL) {
+            const int r = c0 + i / (int)ld, j = i - (r - c0) * (int)ld;
+            if (j != t) results[(long)r * ld + j] = results[(long)r_origin[r] * ld + j];
+        }
+        if (pages != nullptr && n_rows > 0)
+            for (int i = tid; i < n_new * n_rows; i += TREE_SMALL) {
+                const int r = c0 + i / n_rows, j = i - (r - c0) * n_rows;
+                pages[(long)r * pages_stride + j] = pages[(long)r_origin[r] * pages_stride + j];
+            }
+    }
+    // ---- this thread's row ----
+    int ended = 0;
+    if (is_row) {
+        const bool set = r_set[tid] != 0;
+        if (set) { tok[tid] = r_tok[tid]; cnt[tid] = r_cnt[tid]; }
+        origin[tid] = r_origin[tid];
+        int64_t token = old_token;
+        if (tid >= c0 && tid < c1 && !set) token = 0;            // (never: every new row has been set)
+        if (!was) token = 0;
+        else if (set) token = (int64_t)r_tok[tid];
+        results[(long)tid * ld + t] = token;
+        if (fin.state != nullptr) {
+            // detectTerminal on the step's column (mcts.py:14-28, :162), lengths and mask (:163-164)
+            const int32_t match = (st >= 0 && st < fin.seq_len && seq_token == token) ? 1 : 0;
+            const int32_t nxt = (st + match) * match;
+            const bool done = nxt == fin.seq_len || token == fin.eos;
+            fin.state[tid] = done ? 0 : nxt;
+            fin.results_len[tid] = len + (was ? 1 : 0);
+            const bool now = was && !done;
+            alive[tid] = now ? 1 : 0;
+            ended = now ? 0 : 1;
+            fin.next_tokens[tid] = token;
+        }
+    }
+    if (tid == 0) *curr_b = c1;
+    if (fin.state != nullptr) {
+        const int n = __syncthreads_count(ended);
+        if (tid == 0) { fin.summary[0] = c1; fin.summary[1] = n; }
+    }
+}
+
 }  // namespace smh
 
 extern "C" int smh_sample_topk(const void *logits, int rows, int vocab, long ld, float temperature, int top_k,
@@ -696,8 +984,9 @@ extern "C" int smh_tree_fork(const int64_t *draws, int n_draws, int32_t *tok, in
     SMH_REQUIRE(draws && n_draws >= 0 && tok && cnt && alive && curr_b && results && origin, "smh_tree_fork: null pointer or n_draws=%d", n_draws);
     SMH_REQUIRE(ld >= 1 && t >= 0 && t < ld, "smh_tree_fork: column %d outside the %ld of a row", t, ld);
     SMH_REQUIRE(pages == nullptr || (pages_stride >= n_rows && n_rows >= 0), "smh_tree_fork: n_rows=%d pages_stride=%ld", n_rows, pages_stride);
-    hipLaunchKernelGGL(tree_fork_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, draws, n_draws, tok, cnt, const_cast<uint8_t *>(alive), curr_b, batch_size,
-                       results, ld, t, pages, pages_stride, n_rows, origin, (const int32_t *)nullptr, TreeFinish{});
+    const bool small = batch_size <= TREE_SMALL && n_draws <= TREE_SMALL && ld <= (1 << 20);
+    hipLaunchKernelGGL(small ? tree_small_kernel : tree_fork_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, draws, n_draws, tok, cnt,
+                       const_cast<uint8_t *>(alive), curr_b, batch_size, results, ld, t, pages, pages_stride, n_rows, origin, (const int32_t *)nullptr, TreeFinish{});
     return launch_status();
 }
 
@@ -711,8 +1000,9 @@ extern "C" int smh_tree_step(const int64_t *draws, int n_draws, int32_t *tok, in
     SMH_REQUIRE(ld >= 1 && (pages == nullptr || pages_stride >= 1), "smh_tree_step: ld=%ld pages_stride=%ld", ld, pages_stride);
     SMH_REQUIRE(state && terminal_seq && seq_len >= 1 && results_len && next_tokens && summary, "smh_tree_step: null pointer or seq_len=%d", seq_len);
     TreeFinish fin{state, terminal_seq, seq_len, eos, results_len, next_tokens, summary};
-    hipLaunchKernelGGL(tree_fork_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, draws, n_draws, tok, cnt, alive, curr_b, batch_size, results, ld, 0,
-                       pages, pages_stride, 0, origin, t_dev, fin);
+    const bool small = batch_size <= TREE_SMALL && n_draws <= TREE_SMALL && ld <= (1 << 20);      // (row x column products stay in 32 bits)
+    hipLaunchKernelGGL(small ? tree_small_kernel : tree_fork_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, draws, n_draws, tok, cnt, alive, curr_b,
+                       batch_size, results, ld, 0, pages, pages_stride, 0, origin, t_dev, fin);
     return launch_status();
 }
 

@@ -239,3 +239,26 @@ def test_detect_terminal_matches_the_oracle():
     # no branches: nothing to do
     e, s_ = K.detect_terminal(toks_d[:0, 0].contiguous(), st_d[:0], seq_d)
     assert e.numel() == 0 and s_.numel() == 0
+
+
+@pytest.mark.parametrize("rows,vocab,k,temperature", [(3, 32768, 64, 0.7), (3, 32768, 65, 1.0), (2, 32016, 512, 0.9), (2, 32016, 513, 0.9), (2, 1024, 512, 1.0),
+                                                      (3, 2000, 300, 5.0), (2, 4096, 32, 1e4)])
+def test_sampler_candidates_by_maxima_match_the_oracle(rows, vocab, k, temperature):
+    """the sizes at which the sampler changes how it finds its candidates, quotients that collapse or overflow, ascending rows and
+    rows of one value (more candidates than it holds)"""
+    from spec_mcts_amd import kernels as K
+    g = torch.Generator().manual_seed(vocab + k)
+    logits = (torch.randn((rows + 2, vocab), generator=g) * 2).half()
+    logits[rows] = torch.arange(vocab).float().div(64).half()
+    logits[rows + 1] = 1.5
+    p, idx = O.topk_probs(logits, temperature, k)
+    cdf = p.float().cumsum(-1)
+    for trial in range(3):
+        u = torch.rand(rows + 2, generator=g)
+        got = K.sample_topk(logits.cuda(), temperature, k, u.cuda()).cpu()
+        want = O.sample_topk(logits, temperature, k, u)
+        for r in range(rows + 2):
+            j = int((idx[r] == int(got[r])).nonzero()[0])                 # drawn candidate; a neighbour only where the sums round
+            target = float(u[r]) * float(cdf[r, -1])
+            edges = [float(cdf[r, j - 1]) if j else 0.0, float(cdf[r, j])]
+            assert int(got[r]) == int(want[r]) or min(abs(e - target) for e in edges) < 1e-5, (r, j, target, edges)
