@@ -326,7 +326,8 @@ int smh_prefill_attn(const void *q, const void *k, const void *v, void *out, int
  *                pages_stride); lens[b] is cut to pages_cols, so no id past a row's end is read;
  *                the pool has pool_rows rows: an id outside 0 .. pool_rows-1 is read as the nearest valid row (a wrong
  *                result for that branch, never an access outside the pool)
- *   lens         int32 [B] (lens_stride 1) or one shared int32 (lens_stride 0): pages of the branch that are valid
+ *   lens         int32 [B] (lens_stride 1) or one shared int32 (lens_stride 0): pages of the branch that are valid; NULL: all
+ *                pages_cols of them
  *   single_launch, workspace: as smh_shared_prefix_attn_one (counters zeroed once) when != 0, else as smh_shared_prefix_attn
  * smh_page_fork: table[curr + i, 0..n-1] = table[origin, 0..n-1] for i < forks; table int32 [rows, stride]. */
 int smh_paged_prefix_attn(const void *q, void *out, int B, int H, int Hkv, int D,

@@ -130,6 +130,23 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+_ops = None
+
+
+def ops():
+    """The operators of csrc/torch_ops.cpp, bound to the library."""
+    global _ops
+    if _ops is None:
+        path = os.path.join(HERE, "_ops.so")
+        if not os.path.exists(path):
+            raise SmhError(f"{path} not found: build it with `python -m spec_mcts_amd.build` (there is no fallback path)")
+        import torch  # noqa: F401  (its libraries resolve the module's symbols)
+        from . import _ops as m
+        m.connect(load()._handle, SmhError)
+        _ops = m
+    return _ops
+
+
 def check(status: int, what: str) -> None:
     if status != 0:
         msg = load().smh_last_error_string().decode()

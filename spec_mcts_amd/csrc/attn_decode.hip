@@ -56,7 +56,6 @@ struct AttnParams {
     int suffix_waves;                // waves that share one query's suffix rows (1, 2 or 4)
     int P, tw, splits;
     int suffix_format, lens_stride;
-    int causal;                      // prefill mode: branch b attends to suffix rows 0..b
     float scale_log2;                // log2(e) / sqrt(D)
     // FUSED kernels: q, the new token's k and v come straight from the fp32 K-slice slabs of the wq|wk|wv product
     // ([qkv_ks][B][(H + 2 Hkv) * 128]); RoPE, the fp16 rounding points and the Q4_0 append of k, v are those of
@@ -331,7 +330,7 @@ __global__ __launch_bounds__(256) void attn_prefix_kernel(AttnParams p) {
 //   * K tiles go global -> LDS by DMA, 16-byte chunks XOR-swizzled by the row; V goes through registers into its transposed
 //     tile, swizzled so that neither the 8-byte stores nor the 16-byte reads pile up on a few banks.  Two buffers: the next
 //     tile is on its way while one is multiplied, one barrier a tile.
-//   * O^T is rescaled only when a maximum has grown by more than 2^8 (the probabilities are then at most 256, and the factor
+//   * O^T is rescaled only when a maximum has grown by more than 2^4 (the probabilities are then at most 16, and the factor
 //     cancels in the end): the rescale would be a quarter of the vector instructions of a tile.
 //   * The longest walks are dispatched first.
 // Bound by the vector ALU (exponentials) and the matrix cores together.  2047 rows x 32 heads: 187 us with 16 queries a wave and
@@ -458,7 +457,7 @@ __global__ __launch_bounds__(128 * QG, 1) void attn_prefill_kernel(PrefillParams
 #pragma unroll
             for (int r = 1; r < 16; ++r) mx = fmaxf(fmaxf(st[0][r], st[1][r]), mx);
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            const bool grown = (mx - m_run) * p.scale_log2 > 8.0f;       // (true at the first key, false while there is none: NaN)
+            const bool grown = (mx - m_run) * p.scale_log2 > 4.0f;       // (true at the first key, false while there is none: NaN)
             if (__any(grown)) {
                 const float m_new = fmaxf(m_run, mx);
                 const float alpha = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m_run - m_new) * p.scale_log2);
@@ -552,7 +551,8 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
     const int wave = threadIdx.x >> 6;
     int len = 0;
     // a length beyond the branch's rows (a device counter that ran past the cache) is cut at the cache's end
-    if (p.suffix_format != SMH_KV_NONE) len = p.causal ? b + 1 : min(p.lens[(long)b * p.lens_stride], (int)p.suffix_batch_stride_rows);
+    // (no lengths: every branch has all its rows)
+    if (p.suffix_format != SMH_KV_NONE) len = p.lens == nullptr ? (int)p.suffix_batch_stride_rows : min(p.lens[(long)b * p.lens_stride], (int)p.suffix_batch_stride_rows);
     const int gg = g + 4 * sub, gstride = 4 * nsub;      // this group's first row and the distance to its next one
     const long row0 = (long)b * p.suffix_batch_stride_rows;     // first suffix row of this branch
     // pool row that holds suffix position t of this branch
@@ -1068,7 +1068,7 @@ static int shared_prefix_attn(const char *who, bool one, const void *q, void *ou
     SMH_REQUIRE(q && out, "%s: null q/out", who);
     SMH_REQUIRE(P == 0 || (prefix_k && prefix_v), "%s: null prefix", who);
     if (suffix_format != SMH_KV_NONE) {
-        SMH_REQUIRE(suffix_k && suffix_v && lens && Smax > 0 && (lens_stride == 0 || lens_stride == 1),
+        SMH_REQUIRE(suffix_k && suffix_v && (lens || ex.pages) && Smax > 0 && (lens_stride == 0 || lens_stride == 1),
                     "%s: suffix arguments incomplete", who);
         SMH_REQUIRE(suffix_format != SMH_KV_Q40 || (suffix_ks && suffix_vs), "%s: null suffix scales", who);
     }
@@ -1085,7 +1085,7 @@ static int shared_prefix_attn(const char *who, bool one, const void *q, void *ou
     p.pfx_row_stride = ex.pfx_row ? ex.pfx_row : (long)Hkv * ATT_D; p.pfx_head_stride = ex.pfx_head ? ex.pfx_head : ATT_D;
     p.sfx_row_stride = ex.sfx_row ? ex.sfx_row : (long)Hkv * ATT_D; p.sfx_head_stride = ex.sfx_head ? ex.sfx_head : ATT_D;
     p.B = B; p.H = H; p.Hkv = Hkv; p.n_rep = H / Hkv; p.Bq = B * p.n_rep;
-    p.P = P; p.suffix_format = suffix_format; p.causal = 0;
+    p.P = P; p.suffix_format = suffix_format;
     p.scale_log2 = LOG2E / sqrtf((float)D);
     int qgroups = 1;
     if (one) p.tw = min(attn_plan_tw(P, Hkv), ATT_ONE_TW);
@@ -1278,7 +1278,7 @@ extern "C" int smh_shared_prefix_attn_qkv(const void *qkv_partial, int ksplit, v
     p.pfx_row_stride = (long)Hkv * ATT_D; p.pfx_head_stride = ATT_D;
     p.sfx_row_stride = (long)Hkv * ATT_D; p.sfx_head_stride = ATT_D;
     p.B = B; p.H = H; p.Hkv = Hkv; p.n_rep = H / Hkv; p.Bq = B * p.n_rep;
-    p.P = P; p.suffix_format = SMH_KV_Q40; p.causal = 0;
+    p.P = P; p.suffix_format = SMH_KV_Q40;
     p.scale_log2 = LOG2E / sqrtf((float)D);
     int qgroups = 1;
     if (single_launch) p.tw = min(attn_plan_tw(P, Hkv), ATT_ONE_TW);

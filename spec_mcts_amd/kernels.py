@@ -24,7 +24,7 @@ _workspaces: Dict[Tuple[str, int], torch.Tensor] = {}
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())      # (2.6 us less than building a Stream object for it)
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -34,20 +34,6 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 def _need_gpu(*tensors: torch.Tensor) -> None:
     for t in tensors:
         assert t.is_cuda, "spec_mcts_amd kernels need GPU tensors (there is no CPU fallback)"
-
-
-def matmul_workspace(device: torch.device, max_m: int = 16, max_n: int = 0) -> torch.Tensor:
-    """Per-device scratch that carries the fp32 K-slice slabs from the matmul kernel to its reduce
-    kernel.  Shared by all calls on the device (calls run in stream order); calls issued on
-    different streams at the same time need their own workspace."""
-    lib = _lib.load()
-    need = lib.smh_q40_matmul_workspace_bytes(int(max_m), int(max_n))
-    key = ("matmul", device.index if device.index is not None else torch.cuda.current_device())
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < need:
-        ws = torch.empty(need, dtype=torch.uint8, device=device)
-        _workspaces[key] = ws
-    return ws
 
 
 def attn_workspace(device: torch.device, B: int, H: int, P: int) -> torch.Tensor:
@@ -81,27 +67,7 @@ def matmul_q40(a: torch.Tensor, b_w: torch.Tensor, b_s: torch.Tensor, b_shape: S
     """c[M,N] = a[M,K] . deq(b_w, b_s)[K,N] in fp16 with fp32 accumulation
     (reference: triton_kernels.py:471-500).  `residual` ([M,N] fp16) fuses the block's residual
     add: c = residual + fp16(a . deq)."""
-    lib = _lib.load()
-    assert a.is_contiguous(), "Matrix A must be contiguous"
-    assert a.dtype == torch.float16 and a.dim() == 2
-    M, K = a.shape
-    K_b, N = int(b_shape[0]), int(b_shape[1])
-    assert K == K_b, "Incompatible dimensions"
-    _need_gpu(a, b_w, b_s)
-    assert b_w.is_contiguous() and b_s.is_contiguous()
-    assert b_w.dtype == torch.int8 and b_w.numel() == K * N // 2, "packed weight does not match b_shape"
-    assert b_s.dtype == torch.float16 and b_s.numel() == K * N // 64, "scales do not match b_shape"
-    assert a.data_ptr() % 16 == 0
-    c = out if out is not None else torch.empty((M, N), device=a.device, dtype=DTYPE_torch)
-    assert c.shape == (M, N) and c.is_contiguous() and c.dtype == torch.float16
-    epi = SMH_EPI_NONE
-    if residual is not None:
-        assert residual.shape == (M, N) and residual.is_contiguous() and residual.dtype == torch.float16
-        epi = SMH_EPI_RESIDUAL
-    ws = matmul_workspace(a.device, M, N)
-    check(lib.smh_q40_matmul(a.data_ptr(), M, K, K, b_w.data_ptr(), b_s.data_ptr(), N, c.data_ptr(), N,
-                             epi, _ptr(residual), N, ws.data_ptr(), ws.numel(), _stream()), "smh_q40_matmul")
-    return c
+    return _lib.ops().matmul_q40(a, b_w, b_s, b_shape, residual, out)
 
 
 def matmul_plan(M: int, K: int, ns: Sequence[int], tiled: bool = False) -> int:
@@ -374,33 +340,16 @@ def partial_rope_append_kv(p: PartialProduct, H: int, Hkv: int, D: int, cos: tor
 # ---------------------------------------------------------------------------------------------
 def deq_int40(w: torch.Tensor, s: torch.Tensor, group_size: int, shape, ptdtype=DTYPE_torch) -> torch.Tensor:
     """Q4_0 -> fp16, bit-exact nibble*scale (reference: triton_kernels.py:93-107)."""
-    lib = _lib.load()
-    assert group_size == GROUP_SIZE and ptdtype == torch.float16
-    _need_gpu(w, s)
-    assert w.is_contiguous() and s.is_contiguous() and w.dtype == torch.int8 and s.dtype == torch.float16
-    n_elements = int(math.prod(shape))
-    assert n_elements % 128 == 0 and w.numel() == n_elements // 2 and s.numel() == n_elements // 64
-    out = torch.empty(n_elements, device=w.device, dtype=torch.float16)
-    check(lib.smh_q40_dequant(w.data_ptr(), s.data_ptr(), out.data_ptr(), n_elements // 128, _stream()),
-          "smh_q40_dequant")
-    return out.view(shape)
+    assert ptdtype == torch.float16
+    return _lib.ops().deq_int40(w, s, group_size, shape)
 
 
 def q_int40(w: torch.Tensor, group_size: int = GROUP_SIZE) -> Tuple[torch.Tensor, torch.Tensor]:
     """fp16 -> Q4_0 on the GPU with the rounding of the torch quantiser (round-half-even of the fp16
     quotient), NOT the +0.5-and-truncate of the reference's disabled Triton kernel
     (triton_kernels.py:134)."""
-    lib = _lib.load()
     assert group_size == GROUP_SIZE
-    _need_gpu(w)
-    assert w.dtype == torch.float16
-    w = w.contiguous()
-    n = w.numel()
-    assert n % 128 == 0
-    q = torch.empty((n // 128, 64), device=w.device, dtype=torch.int8)
-    s = torch.empty((n // 64, 1), device=w.device, dtype=torch.float16)
-    check(lib.smh_q40_quantize(w.data_ptr(), q.data_ptr(), s.data_ptr(), n // 64, _stream()), "smh_q40_quantize")
-    return q, s
+    return _lib.ops().q_int40(w.contiguous())
 
 
 def quantize_gq40(w: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
@@ -461,20 +410,12 @@ def quantize_q40(w: torch.Tensor, group_size: int = GROUP_SIZE) -> Tuple[torch.T
     return quantize_q40_torch(w, group_size)
 
 
-_SRC_TYPES = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}
+_SRC_TYPES = (torch.float16, torch.bfloat16, torch.float32)
 
 
 def quantize_q40_t(v: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     """quantize_q40(v.t().contiguous()) for a checkpoint weight v [N, K] (fp16, bfloat16 or fp32) on the GPU, in one pass over v."""
-    lib = _lib.load()
-    _need_gpu(v)
-    assert v.dim() == 2 and v.shape[0] % 128 == 0 and v.dtype in _SRC_TYPES
-    v = v.contiguous()
-    N, Kd = v.shape
-    q = torch.empty((N * Kd // 128, 64), device=v.device, dtype=torch.int8)
-    s = torch.empty((N * Kd // 64, 1), device=v.device, dtype=torch.float16)
-    check(lib.smh_q40_quantize_t(v.data_ptr(), _SRC_TYPES[v.dtype], N, Kd, q.data_ptr(), s.data_ptr(), _stream()), "smh_q40_quantize_t")
-    return q, s
+    return _lib.ops().quantize_q40_t(v.contiguous())
 
 
 dequantize_q40 = deq_int40
@@ -563,24 +504,7 @@ def sample_topk_counts(logits: torch.Tensor, temperature, top_k: int, counts: to
     [rows] and uniform fp32 [>= counts.sum()] on the device.  temperature: a positive number (logits / temperature stays
     fp16, as in torch) or a float32 tensor [rows] of positive numbers on the device (the sampler's per-branch ramp,
     mcts.py:110-114: a tensor divisor promotes to fp32, so quotients and probabilities are fp32)."""
-    lib = _lib.load()
-    _need_gpu(logits, counts, uniform)
-    assert logits.dim() == 2 and logits.dtype == torch.float16 and logits.stride(1) == 1
-    rows, vocab = logits.shape
-    assert counts.dtype == torch.int32 and counts.is_contiguous() and counts.numel() >= rows
-    assert uniform.dtype == torch.float32 and uniform.is_contiguous()
-    if out is None:
-        out = torch.zeros(uniform.numel(), device=logits.device, dtype=torch.int64)
-    assert out.dtype == torch.int64 and out.is_contiguous() and out.numel() >= uniform.numel()
-    if isinstance(temperature, torch.Tensor):
-        _need_gpu(temperature)
-        assert temperature.dtype == torch.float32 and temperature.is_contiguous() and temperature.numel() >= rows
-        check(lib.smh_sample_topk_rowtemp(logits.data_ptr(), rows, vocab, logits.stride(0), temperature.data_ptr(), int(min(top_k, vocab)),
-                                          uniform.data_ptr(), counts.data_ptr(), out.data_ptr(), uniform.numel(), _stream()), "smh_sample_topk_rowtemp")
-        return out
-    check(lib.smh_sample_topk_counts(logits.data_ptr(), rows, vocab, logits.stride(0), float(temperature), int(min(top_k, vocab)),
-                                     uniform.data_ptr(), counts.data_ptr(), out.data_ptr(), uniform.numel(), _stream()), "smh_sample_topk_counts")
-    return out
+    return _lib.ops().sample_topk_counts(logits, temperature, top_k, counts, uniform, out)
 
 
 def tree_fork(draws: torch.Tensor, output_counts: torch.Tensor, alive: torch.Tensor, curr_b: torch.Tensor, results: torch.Tensor, t: int,
@@ -613,24 +537,7 @@ def tree_step(draws: torch.Tensor, output_counts: torch.Tensor, alive: torch.Ten
     index read from the device (t_dev int32 [1]: the column of `results` and the suffix rows written so far), so that the
     launch can sit in a captured graph: tree_fork, then detect_terminal on the step's column, results_len += alive,
     alive &= ~ended, next_tokens = results[:, t], summary = (branches, ended rows).  alive is uint8 [batch]."""
-    lib = _lib.load()
-    _need_gpu(draws, output_counts, alive, curr_b, results, t_dev, origin, state, terminal_seq, results_len, next_tokens, summary)
-    B, ld = results.shape
-    assert draws.dtype == torch.int64 and draws.is_contiguous()
-    assert output_counts.dtype == torch.int32 and output_counts.shape == (2, B) and output_counts.is_contiguous()
-    assert alive.dtype == torch.uint8 and alive.numel() == B and alive.is_contiguous()
-    assert curr_b.dtype == torch.int32 and t_dev.dtype == torch.int32 and summary.dtype == torch.int32 and summary.numel() >= 2
-    assert results.dtype == torch.int64 and results.is_contiguous()
-    assert origin.dtype == torch.int32 and origin.numel() >= B and state.dtype == torch.int32 and state.numel() == B
-    assert results_len.dtype == torch.int32 and results_len.numel() == B and next_tokens.dtype == torch.int64 and next_tokens.numel() >= B
-    assert terminal_seq.dtype == torch.int64 and terminal_seq.is_contiguous()
-    if pages is not None:
-        _need_gpu(pages)
-        assert pages.dtype == torch.int32 and pages.dim() == 2 and pages.shape[0] >= B and pages.stride(1) == 1
-    check(lib.smh_tree_step(draws.data_ptr(), draws.numel(), output_counts[0].data_ptr(), output_counts[1].data_ptr(), alive.data_ptr(),
-                            curr_b.data_ptr(), B, results.data_ptr(), ld, t_dev.data_ptr(), _ptr(pages), pages.stride(0) if pages is not None else 0,
-                            origin.data_ptr(), state.data_ptr(), terminal_seq.data_ptr(), terminal_seq.numel(), int(eos), results_len.data_ptr(),
-                            next_tokens.data_ptr(), summary.data_ptr(), _stream()), "smh_tree_step")
+    _lib.ops().tree_step(draws, output_counts, alive, curr_b, results, t_dev, pages, origin, state, terminal_seq, results_len, next_tokens, summary, eos)
 
 
 def detect_terminal(token: torch.Tensor, state: torch.Tensor, terminal_seq: torch.Tensor, eos: int = 2):
@@ -826,6 +733,9 @@ def shared_prefix_attn(q: torch.Tensor, prefix_k: Optional[torch.Tensor], prefix
     single_launch: one launch instead of two (at most 128 queries per kv head; same result up to fp32
     summation order).  static_scratch: the two-launch form on the library's own static scratch array: with `out`
     given the call allocates nothing (smh_shared_prefix_attn_static)."""
+    if not single_launch and not static_scratch:
+        return _lib.ops().shared_prefix_attn(q, prefix_k, prefix_v, P, suffix_k, suffix_v, suffix_ks, suffix_vs, Smax, lens, lens_stride, cur_k, cur_v,
+                                             n_kv_heads, out)
     lib = _lib.load()
     _need_gpu(q)
     assert q.is_contiguous() and q.dtype == torch.float16 and q.dim() == 3
@@ -858,10 +768,11 @@ def shared_prefix_attn(q: torch.Tensor, prefix_k: Optional[torch.Tensor], prefix
                                                 _ptr(lens), int(lens_stride), _ptr(cur_k), _ptr(cur_v), _stream()),
               "smh_shared_prefix_attn_static")
         return out
-    one = bool(single_launch) and B * (H // Hkv) <= 128
-    ws = attn_qkv_workspace(q.device, B, H, P) if one else attn_workspace(q.device, B, H, P)
-    fn = lib.smh_shared_prefix_attn_one if one else lib.smh_shared_prefix_attn
-    check(fn(q.data_ptr(), out.data_ptr(), B, H, Hkv, D, _ptr(prefix_k), _ptr(prefix_v), int(P),
+    if B * (H // Hkv) > 128:
+        return _lib.ops().shared_prefix_attn(q, prefix_k, prefix_v, P, suffix_k, suffix_v, suffix_ks, suffix_vs, Smax, lens, lens_stride, cur_k, cur_v,
+                                             n_kv_heads, out)
+    ws = attn_qkv_workspace(q.device, B, H, P)
+    check(lib.smh_shared_prefix_attn_one(q.data_ptr(), out.data_ptr(), B, H, Hkv, D, _ptr(prefix_k), _ptr(prefix_v), int(P),
              fmt, _ptr(suffix_k), _ptr(suffix_v), _ptr(suffix_ks), _ptr(suffix_vs), int(Smax),
              _ptr(lens), int(lens_stride), _ptr(cur_k), _ptr(cur_v),
              ws.data_ptr(), ws.numel(), _stream()), "smh_shared_prefix_attn")
@@ -930,7 +841,7 @@ def flash_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, B: int, L: int
                               n_kv_heads=H)
 
 
-def paged_prefix_attn(q: torch.Tensor, pages: torch.Tensor, lens: torch.Tensor, pool_k: torch.Tensor, pool_v: torch.Tensor,
+def paged_prefix_attn(q: torch.Tensor, pages: torch.Tensor, lens: Optional[torch.Tensor], pool_k: torch.Tensor, pool_v: torch.Tensor,
                       pool_ks: Optional[torch.Tensor] = None, pool_vs: Optional[torch.Tensor] = None, head_major: bool = False,
                       prefix_k: Optional[torch.Tensor] = None, prefix_v: Optional[torch.Tensor] = None, P: int = 0,
                       prefix_head_major: bool = False, cur_k: Optional[torch.Tensor] = None, cur_v: Optional[torch.Tensor] = None,
@@ -939,13 +850,16 @@ def paged_prefix_attn(q: torch.Tensor, pages: torch.Tensor, lens: torch.Tensor, 
     pages[b, :lens[b]] || cur_k[b].  The rows are looked up inside the kernel (nothing is gathered or copied).
     pool: fp16 [rows, Hkv, D] (or [Hkv, rows, D] with head_major) or Q4_0 rows int8 [rows, Hkv, 64] + scales fp16
     [rows, Hkv, 2]; pages: int16 / int32 / int64 [B, L] (possibly a column slice of a wider table); lens int32 on the device,
-    cut to L inside the kernel."""
+    cut to L inside the kernel, or None (every branch has its L pages)."""
+    if not single_launch or q.shape[0] * q.shape[1] > 128 * (pool_k.shape[0] if head_major else pool_k.shape[1]):
+        return _lib.ops().paged_prefix_attn(q, pages, lens, pool_k, pool_v, pool_ks, pool_vs, head_major, prefix_k, prefix_v, P, prefix_head_major, cur_k, cur_v,
+                                            lens_stride)
     lib = _lib.load()
-    _need_gpu(q, pages, lens, pool_k, pool_v)
+    _need_gpu(q, pages, pool_k, pool_v)
     assert q.is_contiguous() and q.dtype == torch.float16 and q.dim() == 3
     B, H, D = q.shape
     assert pages.dim() == 2 and pages.shape[0] >= B and pages.stride(1) == 1 and pages.dtype in (torch.int16, torch.int32, torch.int64)
-    assert lens.dtype == torch.int32
+    assert lens is None or (lens.is_cuda and lens.dtype == torch.int32)
     assert pool_k.is_contiguous() and pool_v.is_contiguous() and pool_k.shape == pool_v.shape
     if pool_k.dtype == torch.float16:
         fmt = SMH_KV_FP16
@@ -975,12 +889,11 @@ def paged_prefix_attn(q: torch.Tensor, pages: torch.Tensor, lens: torch.Tensor, 
     if cur_k is not None:
         assert cur_k.is_contiguous() and cur_v.is_contiguous() and cur_k.dtype == torch.float16 and cur_k.shape == (B, Hkv, D)
     out = torch.empty_like(q)
-    one = bool(single_launch) and B * (H // Hkv) <= 128
-    ws = attn_qkv_workspace(q.device, B, H, P) if one else attn_workspace(q.device, B, H, P)
+    ws = attn_qkv_workspace(q.device, B, H, P)
     check(lib.smh_paged_prefix_attn(q.data_ptr(), out.data_ptr(), B, H, Hkv, D, _ptr(prefix_k) if P else None, _ptr(prefix_v) if P else None,
                                     int(P), p_row, p_head, fmt, pool_k.data_ptr(), pool_v.data_ptr(), _ptr(pool_ks), _ptr(pool_vs),
                                     row_stride, head_stride, int(rows), pages.data_ptr(), pages.element_size(), pages.stride(0), pages.shape[1],
-                                    lens.data_ptr(), int(lens_stride), _ptr(cur_k), _ptr(cur_v), int(one), ws.data_ptr(), ws.numel(), _stream()),
+                                    _ptr(lens), int(lens_stride), _ptr(cur_k), _ptr(cur_v), 1, ws.data_ptr(), ws.numel(), _stream()),
           "smh_paged_prefix_attn")
     return out
 
@@ -1003,8 +916,7 @@ def page_flash_attn(p: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.
     reference keeps them in fp16)."""
     _need_gpu(p, q, k, v)
     assert p.shape == (B, L) and q.shape == (B, H, D) and k.shape == (H, P, D) and v.shape == (H, P, D)
-    lens = torch.full((1,), L, dtype=torch.int32, device=q.device)
-    return paged_prefix_attn(q.contiguous(), p if p.stride(1) == 1 else p.contiguous(), lens, k.contiguous(), v.contiguous(),
+    return paged_prefix_attn(q.contiguous(), p if p.stride(1) == 1 else p.contiguous(), None, k.contiguous(), v.contiguous(),
                              head_major=True, lens_stride=0)
 
 
