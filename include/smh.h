@@ -328,7 +328,9 @@ int smh_prefill_attn(const void *q, const void *k, const void *v, void *out, int
  *                result for that branch, never an access outside the pool)
  *   lens         int32 [B] (lens_stride 1) or one shared int32 (lens_stride 0): pages of the branch that are valid; NULL: all
  *                pages_cols of them
- *   single_launch, workspace: as smh_shared_prefix_attn_one (counters zeroed once) when != 0, else as smh_shared_prefix_attn
+ *   single_launch, workspace: as smh_shared_prefix_attn_one (counters zeroed once) when != 0, else as smh_shared_prefix_attn;
+ *                with smh_paged_attn_workspace_bytes(...) bytes (never fewer) fp16 pages that neighbouring branches share are
+ *                read once for them instead of once per branch (P = 0, lens = NULL)
  * smh_page_fork: table[curr + i, 0..n-1] = table[origin, 0..n-1] for i < forks; table int32 [rows, stride]. */
 int smh_paged_prefix_attn(const void *q, void *out, int B, int H, int Hkv, int D,
                           const void *prefix_k, const void *prefix_v, int P, long prefix_row_stride, long prefix_head_stride,
@@ -337,6 +339,7 @@ int smh_paged_prefix_attn(const void *q, void *out, int B, int H, int Hkv, int D
                           const void *pages, int page_bytes, long pages_stride, int pages_cols, const int32_t *lens, int lens_stride,
                           const void *cur_k, const void *cur_v, int single_launch,
                           void *workspace, size_t workspace_bytes, smh_stream_t stream);
+size_t smh_paged_attn_workspace_bytes(int B, int H, int Hkv, int P, int pages_cols);
 int smh_page_fork(int32_t *table, int rows, long stride, int origin, int curr, int forks, int n, smh_stream_t stream);
 
 /* smh_shared_prefix_attn_static: smh_shared_prefix_attn (same arguments without the workspace, same kernels, bit-identical

@@ -82,6 +82,7 @@ SIGNATURES = {
     "smh_f16_linear": (c_int, [_P, c_int, c_int, c_long, _P, c_int, _P, c_long, _P]),
     "smh_embedding": (c_int, [_P, c_int, _P, c_int, c_int, _P, _P]),
     "smh_attn_workspace_bytes": (c_size_t, [c_int, c_int, c_int]),
+    "smh_paged_attn_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
     "smh_shared_prefix_attn": (c_int, [_P, _P, c_int, c_int, c_int, c_int, _P, _P, c_int, c_int, _P, _P, _P, _P, c_int,
                                        _P, c_int, _P, _P, _P, c_size_t, _P]),
     "smh_shared_prefix_attn_one": (c_int, [_P, _P, c_int, c_int, c_int, c_int, _P, _P, c_int, c_int, _P, _P, _P, _P, c_int,

@@ -69,6 +69,7 @@ struct AttnParams {
     const int32_t *app_t;
     int app_smax;
     uint32_t *counters;              // one-launch variant: arrivals per kv head (zero between launches)
+    uint8_t *tile_done;              // [Hkv][query tiles][splits]: 1 where attn_page_tile_kernel has left the partials of a slice
 };
 
 // x / n_rep and x % n_rep for the query heads per kv head; 1 (multi-head attention) needs no division
@@ -318,6 +319,150 @@ __global__ __launch_bounds__(256) void attn_prefix_kernel(AttnParams p) {
     attn_prefix_body<FUSED, false, ATT_TW_MAX>(p, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z);
 }
 
+// ---- pages that the branches of a query tile share ---------------------------------------------------------------
+// Branches of a tree share their ancestors' pages, so the same page stands at the same position of many rows of the table
+// (the prompt's in all of them).  Workgroup (kv head, slice of 64 positions, tile of 16 queries): where the tile's branches
+// have the same ids throughout the slice, its rows are staged in LDS once for the 16 queries and multiplied on the matrix
+// cores - wave w scores positions 16 w .. + 15 and then makes dims 32 w .. + 31 of the outputs - and a partial (max, sum,
+// o[128]) is left per query; tile_done says so and attn_suffix_kernel skips the slice.  Where they differ, or a staged value
+// is infinite or NaN, the slice is left to attn_suffix_kernel.  Probabilities enter the product as two fp16 terms (the second
+// 2^11 times what the first leaves over), 22 bits: against 64-bit sums the result is no further off than the fp32 walk's.
+// Bound by the walk of what is not shared.  32 heads, 512 positions, half of them a prompt: 99 branches 150 -> 100 us a call, 50: 80 -> 60,
+// 27: 45 -> 37, 8: 32 -> 20; 460 shared positions and 99 branches: 111 -> 39 us (error against 64 bits 2.1e-4 before and after: the
+// output's fp16).  Where nothing is shared the pass costs its 3 us (100 positions, 99 branches: 29.7 -> 26.5 with the walk's gain).
+constexpr int PT_TW = 64;
+constexpr int PT_MAX_SLICES = 64;          // one bit a slice in the suffix kernel's mask
+__device__ __forceinline__ long page_at(const AttnParams &p, long i) {
+    if (p.page_bytes == 4) return reinterpret_cast<const int32_t *>(p.pages)[i];
+    if (p.page_bytes == 2) return reinterpret_cast<const int16_t *>(p.pages)[i];
+    return reinterpret_cast<const int64_t *>(p.pages)[i];
+}
+__global__ __launch_bounds__(256) void attn_page_tile_kernel(AttnParams p) {
+    __shared__ __attribute__((aligned(16))) half_t ks[PT_TW][ATT_KPITCH];
+    __shared__ __attribute__((aligned(16))) half_t vt[ATT_D][PT_TW + 8];
+    __shared__ __attribute__((aligned(16))) half_t ps[2][16][PT_TW + 8];      // probabilities of the 16 queries, both terms, in vt_pos order
+    __shared__ long s_row[PT_TW];
+    __shared__ float s_max[4][16], s_sum[4][16];
+    const int hk = blockIdx.x, split = blockIdx.y, tile = blockIdx.z;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
+    const int t0 = split * PT_TW, cnt = min(PT_TW, (int)p.suffix_batch_stride_rows - t0);
+    const int b_lo = div_rep(p, tile * 16), b_hi = div_rep(p, min(tile * 16 + 15, p.Bq - 1));
+    // ---- does every branch of the tile have the first one's ids? ----
+    bool same = true;
+    {
+        const int pos = t0 + min(lane, cnt - 1);
+        const long id0 = page_at(p, (long)b_lo * p.pages_stride + pos);
+        for (int b = b_lo + 1 + wave; b <= b_hi; b += 4) same &= page_at(p, (long)b * p.pages_stride + pos) == id0;
+        if (wave == 0) s_row[lane] = min(max(id0, 0L), p.pool_rows - 1);
+    }
+    uint8_t *done = p.tile_done + ((long)hk * gridDim.z + tile) * p.splits + split;
+    if (!__syncthreads_and(same)) {
+        if (tid == 0) *done = 0;
+        return;
+    }
+    // ---- the query tile (B operand of S^T), then the rows: K row-major, V transposed, as in attn_prefix_body ----
+    const int qrow = tile * 16 + c, qr = min(qrow, p.Bq - 1);
+    h8 qb[4];
+    {
+        const half_t *qp = p.q + ((long)div_rep(p, qr) * p.H + hk * p.n_rep + mod_rep(p, qr)) * ATT_D + 8 * g;
+#pragma unroll
+        for (int k4 = 0; k4 < 4; ++k4) qb[k4] = *reinterpret_cast<const h8 *>(qp + 32 * k4);
+    }
+    uint32_t bad = 0;
+    {
+        const int ch = tid & 15, kg = tid >> 4;
+        u32x4 kv[4], vv[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const long off = s_row[4 * kg + e] * p.sfx_row_stride + (long)hk * p.sfx_head_stride + ch * 8;
+            const half_t *kp = (const half_t *)p.suffix_k + off, *vp = (const half_t *)p.suffix_v + off;
+            // (8-byte loads: a pool's rows are only that much aligned)
+            const u32x2 k0 = *reinterpret_cast<const u32x2 *>(kp), k1 = *reinterpret_cast<const u32x2 *>(kp + 4);
+            const u32x2 v0 = *reinterpret_cast<const u32x2 *>(vp), v1 = *reinterpret_cast<const u32x2 *>(vp + 4);
+            kv[e] = u32x4{k0[0], k0[1], k1[0], k1[1]};
+            vv[e] = u32x4{v0[0], v0[1], v1[0], v1[1]};
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {          // (an exponent of all ones carries into the sign bit)
+                bad |= (kv[e][i] & 0x7fff7fffu) + 0x04000400u;
+                bad |= (vv[e][i] & 0x7fff7fffu) + 0x04000400u;
+            }
+            *reinterpret_cast<u32x4 *>(&ks[4 * kg + e][ch * 8]) = kv[e];
+        }
+        const int pos = vt_pos(4 * kg);
+        const h8 v0 = __builtin_bit_cast(h8, vv[0]), v1 = __builtin_bit_cast(h8, vv[1]);
+        const h8 v2 = __builtin_bit_cast(h8, vv[2]), v3 = __builtin_bit_cast(h8, vv[3]);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) *reinterpret_cast<h4 *>(&vt[ch * 8 + j][pos]) = h4{v0[j], v1[j], v2[j], v3[j]};
+    }
+    const bool finite = !__syncthreads_or((bad & 0x80008000u) != 0);
+    if (tid == 0) *done = finite ? 1 : 0;
+    if (!finite) return;
+    // ---- scores: element r of st is position 16 wave + 4 g + r (past the end: a repeated row, masked), column (query) c ----
+    f4 st = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k4 = 0; k4 < 4; ++k4)
+        st = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const h8 *>(&ks[16 * wave + c][32 * k4 + 8 * g]), qb[k4], st, 0, 0, 0);
+    float mx = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        st[r] = 16 * wave + 4 * g + r < cnt ? st[r] * p.scale_log2 : -INFINITY;
+        mx = fmaxf(mx, st[r]);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    if (g == 0) s_max[wave][c] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(s_max[0][c], s_max[1][c]), fmaxf(s_max[2][c], s_max[3][c]));
+    float sum = 0.f;
+    h4 p_hi, p_lo;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const float e = exp2f(st[r] - mx);
+        sum += e;
+        p_hi[r] = (half_t)e;
+        p_lo[r] = (half_t)((e - (float)p_hi[r]) * 2048.f);
+    }
+    {
+        const int at = 32 * (wave >> 1) + 8 * g + 4 * (wave & 1);
+        *reinterpret_cast<h4 *>(&ps[0][c][at]) = p_hi;
+        *reinterpret_cast<h4 *>(&ps[1][c][at]) = p_lo;
+    }
+    sum += __shfl_xor(sum, 16, 64);
+    sum += __shfl_xor(sum, 32, 64);
+    if (g == 0) s_sum[wave][c] = sum;
+    __syncthreads();
+    // ---- O^T: element r of o[i] is dim 32 wave + 16 i + 4 g + r, column (query) c ----
+    f4 o_hi[2], o_lo[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) { o_hi[i] = f4{0.f, 0.f, 0.f, 0.f}; o_lo[i] = f4{0.f, 0.f, 0.f, 0.f}; }
+#pragma unroll
+    for (int jj = 0; jj < PT_TW / 32; ++jj) {
+        const h8 ph = *reinterpret_cast<const h8 *>(&ps[0][c][32 * jj + 8 * g]), pl = *reinterpret_cast<const h8 *>(&ps[1][c][32 * jj + 8 * g]);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const h8 va = *reinterpret_cast<const h8 *>(&vt[32 * wave + 16 * i + c][32 * jj + 8 * g]);
+            o_hi[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, ph, o_hi[i], 0, 0, 0);
+            o_lo[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pl, o_lo[i], 0, 0, 0);
+        }
+    }
+    if (qrow >= p.Bq) return;
+    const long base = ((long)split * p.Hkv + hk) * p.Bq + qrow;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        f4 o;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = o_hi[i][r] + o_lo[i][r] * (1.f / 2048.f);
+        *reinterpret_cast<f4 *>(p.part_o + base * ATT_D + 32 * wave + 16 * i + 4 * g) = o;
+    }
+    if (wave == 0 && g == 0) {
+        p.part_ml[base * 2] = mx;
+        p.part_ml[base * 2 + 1] = s_sum[0][c] + s_sum[1][c] + s_sum[2][c] + s_sum[3][c];
+    }
+}
+
 // ---- causal attention of a prefill on the matrix cores ----------------------------------------------------------
 // A workgroup owns 32 QG consecutive query positions of one head; its 2 QG waves are QG groups of 32 queries x two key groups
 // that take alternate key tiles (a wave alone on a SIMD waits for its own chain of products, exponentials and LDS reads; two
@@ -531,8 +676,12 @@ constexpr int PF_LDS = 8 * PF_TW * ATT_D * 2;              // 128 KB: one workgr
 // nsub-th group of four rows, so that a long suffix is a single batch of loads per wave instead of a chain of
 // batches; the waves' results are folded through LDS (every wave of the workgroup must then make this call; a wave
 // without a query of its own passes a valid (b, h) and live = false, and writes nothing).
-template <bool FUSED, bool PARTIAL>
+// WALK: the rows' format where it is known - a kernel that holds both walks needs registers for the larger one.  WALK_TILES:
+// fp16, the slices that tile_done marks are skipped, and only their partials are folded in.
+enum { WALK_ANY, WALK_Q40, WALK_F16, WALK_TILES };
+template <bool FUSED, bool PARTIAL, int WALK = WALK_ANY>
 __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int h, int sub = 0, int nsub = 1, bool live = true) {
+    constexpr bool TILES = WALK == WALK_TILES;
     const int hk = div_rep(p, h);
     __shared__ __attribute__((aligned(16))) half_t s_kv[FUSED ? 4 : 1][3][ATT_D];     // FUSED: this wave's new k and v rows, its query
     __shared__ float s_fold[4][16][10];                                                 // nsub > 1: the waves' states (m, l, o[8])
@@ -558,12 +707,7 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
     // pool row that holds suffix position t of this branch
     auto row_of = [&](int t) -> long {
         if (p.pages == nullptr) return row0 + t;
-        const long i = (long)b * p.pages_stride + t;
-        long id;
-        if (p.page_bytes == 4) id = reinterpret_cast<const int32_t *>(p.pages)[i];
-        else if (p.page_bytes == 2) id = reinterpret_cast<const int16_t *>(p.pages)[i];
-        else id = reinterpret_cast<const int64_t *>(p.pages)[i];
-        return min(max(id, 0L), p.pool_rows - 1);
+        return min(max(page_at(p, (long)b * p.pages_stride + t), 0L), p.pool_rows - 1);
     };
     // ---- Q4_0 suffix rows: a wave takes Q4_ROWS rows per pass (row slot Q4_DW g + rl) and Q4_CH passes per chunk; wave
     // `sub` of the nsub that share a query takes every nsub-th pass.  All loads of a chunk are requested together, and
@@ -660,7 +804,7 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
         const int qrow = b * p.n_rep + (h - hk * p.n_rep);
         const bool has_cur = (FUSED || p.cur_k != nullptr) && g == 0 && sub == 0;
         RowRegs cur_kr = qr, cur_vr = qr;
-        if (has_cur) {
+        auto load_cur = [&]() {
             if (FUSED) {
                 cur_kr = row_from_fp16(&s_kv[wave][0][0], c);
                 cur_vr = row_from_fp16(&s_kv[wave][1][0], c);
@@ -669,10 +813,11 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
                 cur_kr = row_from_fp16(p.cur_k + off, c);
                 cur_vr = row_from_fp16(p.cur_v + off, c);
             }
-        }
-        constexpr int PRE = 2;
-        f4 pre_lo[PRE], pre_hi[PRE];
-        float pre_m[PRE], pre_l[PRE];
+        };
+        if (WALK < WALK_F16 && has_cur) load_cur();        // (the fp16 walk needs the registers)
+        constexpr int PRE = WALK < WALK_F16 ? 2 : 0;
+        f4 pre_lo[PRE + 1], pre_hi[PRE + 1];
+        float pre_m[PRE + 1], pre_l[PRE + 1];
 #pragma unroll
         for (int i = 0; i < PRE; ++i) {
             const int sp = gg + gstride * i;
@@ -685,21 +830,95 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
             }
         }
         // ---- this branch's suffix: group g takes rows g, g+4, ... in batches ----
-        if (p.suffix_format == SMH_KV_FP16) {
+        uint64_t tiles = 0;                                 // bit s: slice s is done
+        if (TILES) tiles = __ballot(lane < p.splits && p.tile_done[((long)hk * ((p.Bq + 15) / 16) + (qrow >> 4)) * p.splits + min(lane, p.splits - 1)] != 0);
+        if (WALK == WALK_F16 || TILES || (WALK == WALK_ANY && p.suffix_format == SMH_KV_FP16)) {
+            // Batches of U rows per group, the next one (and the ids of the one after it) on its way while this one is used; one
+            // maximum and one rescale a batch.
             constexpr int U = 4;
-            for (int t0 = gg; t0 < len; t0 += gstride * U) {
-                RowRegs kr[U], vr[U];
+            static_assert(PT_TW % (4 * 4 * U) == 0, "a batch of the waves of a query lies in one slice");
+            const int span = gstride * U, n_batches = (len + span - 1) / span;
+            auto next = [&](int i) {
+                ++i;
+                if (TILES) while (i < n_batches && ((tiles >> (i * span / PT_TW)) & 1) != 0) ++i;
+                return i;
+            };
+            struct Batch { u32x2 kl[U], kh[U], vl[U], vh[U]; };
+            int id[U];                                      // (rows of 256 bytes and more: their number fits)
+            auto ids = [&](int i) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) id[u] = (int)row_of(min(span * i + gg + gstride * u, len - 1));       // past the end: the last row again
+            };
+            auto rows = [&](Batch &r) {
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    const long off = row_of(min(t0 + gstride * u, len - 1)) * p.sfx_row_stride + (long)hk * p.sfx_head_stride;
-                    kr[u] = row_from_fp16((const half_t *)p.suffix_k + off, c);
-                    vr[u] = row_from_fp16((const half_t *)p.suffix_v + off, c);
+                    const long off = (long)id[u] * p.sfx_row_stride + (long)hk * p.sfx_head_stride + 4 * c;
+                    r.kl[u] = *reinterpret_cast<const u32x2 *>((const half_t *)p.suffix_k + off);
+                    r.kh[u] = *reinterpret_cast<const u32x2 *>((const half_t *)p.suffix_k + off + 64);
+                    r.vl[u] = *reinterpret_cast<const u32x2 *>((const half_t *)p.suffix_v + off);
+                    r.vh[u] = *reinterpret_cast<const u32x2 *>((const half_t *)p.suffix_v + off + 64);
                 }
-#pragma unroll
-                for (int u = 0; u < U; ++u)
-                    if (t0 + gstride * u < len) soft_add_row(st, row_dot(kr[u], qr) * p.scale_log2, vr[u]);
+            };
+            const u32x2 ql = {pack_lo16(as_u32(qr.a02), as_u32(qr.a13)), pack_hi16(as_u32(qr.a02), as_u32(qr.a13))};       // dims (0,1), (2,3)
+            const u32x2 qh = {pack_lo16(as_u32(qr.b02), as_u32(qr.b13)), pack_hi16(as_u32(qr.b02), as_u32(qr.b13))};
+            int i0 = next(-1), i1 = n_batches;
+            Batch cur;
+            if (i0 < n_batches) {
+                ids(i0);
+                rows(cur);
+                i1 = next(i0);
+                if (i1 < n_batches) ids(i1);
             }
-        } else if (q4_chunks > 0) {
+            while (i0 < n_batches) {
+                Batch nxt;
+                int i2 = n_batches;
+                if (i1 < n_batches) {
+                    rows(nxt);
+                    i2 = next(i1);
+                    if (i2 < n_batches) ids(i2);
+                }
+                float sc[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    float d = __builtin_amdgcn_fdot2(as_h2(cur.kl[u][0]), as_h2(ql[0]), 0.f, false);
+                    d = __builtin_amdgcn_fdot2(as_h2(cur.kl[u][1]), as_h2(ql[1]), d, false);
+                    d = __builtin_amdgcn_fdot2(as_h2(cur.kh[u][0]), as_h2(qh[0]), d, false);
+                    d = __builtin_amdgcn_fdot2(as_h2(cur.kh[u][1]), as_h2(qh[1]), d, false);
+                    sc[u] = row16_sum(d) * p.scale_log2;
+                }
+                if (span * (i0 + 1) > len) {                // (uniform) the last batch: a repeated row weighs nothing, also where it is infinite
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+                        if (span * i0 + gg + gstride * u >= len) {
+                            sc[u] = -INFINITY;
+                            cur.vl[u] = u32x2{0, 0};
+                            cur.vh[u] = u32x2{0, 0};
+                        }
+                }
+                float mx = sc[0];
+#pragma unroll
+                for (int u = 1; u < U; ++u) mx = fmaxf(mx, sc[u]);
+                const float m_new = fmaxf(st.m, mx), m_ref = m_new == -INFINITY ? 0.f : m_new;
+                const float corr = __builtin_amdgcn_exp2f(st.m - m_ref);
+                st.m = m_new;
+                st.l *= corr;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) st.o[k] *= corr;
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const float pr = __builtin_amdgcn_exp2f(sc[u] - m_ref);
+                    st.l += pr;
+                    const h2 v01 = as_h2(cur.vl[u][0]), v23 = as_h2(cur.vl[u][1]), w01 = as_h2(cur.vh[u][0]), w23 = as_h2(cur.vh[u][1]);
+                    st.o[0] += pr * (float)v01.x; st.o[2] += pr * (float)v01.y;
+                    st.o[1] += pr * (float)v23.x; st.o[3] += pr * (float)v23.y;
+                    st.o[4] += pr * (float)w01.x; st.o[6] += pr * (float)w01.y;
+                    st.o[5] += pr * (float)w23.x; st.o[7] += pr * (float)w23.y;
+                }
+                cur = nxt;
+                i0 = i1;
+                i1 = i2;
+            }
+        } else if (WALK <= WALK_Q40 && q4_chunks > 0) {
             if (!FUSED) q4_prime();
             RowRegs qj[Q4_DW];                              // the query's dims this lane holds of a row: pieces Q4_DW e + j
 #pragma unroll
@@ -786,6 +1005,7 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
             }
         }
         // ---- the new token's exact K/V (group 0 only) ----
+        if (WALK >= WALK_F16 && has_cur) load_cur();
         if (has_cur) soft_add_row(st, row_dot(cur_kr, qr) * p.scale_log2, cur_vr);
         // ---- prefix partials: the group folds in splits gg, gg + gstride, ... ----
 #pragma unroll
@@ -796,6 +1016,7 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
             }
         }
         for (int sp = gg + gstride * PRE; !PARTIAL && sp < p.splits; sp += gstride) {
+            if (TILES && ((tiles >> sp) & 1) == 0) continue;
             const long base = ((long)sp * p.Hkv + hk) * p.Bq + qrow;
             const f4 lo = *reinterpret_cast<const f4 *>(p.part_o + base * ATT_D + 4 * c);
             const f4 hi = *reinterpret_cast<const f4 *>(p.part_o + base * ATT_D + 64 + 4 * c);
@@ -840,12 +1061,15 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
     }
 }
 
-template <bool FUSED>
-__global__ __launch_bounds__(256) void attn_suffix_kernel(AttnParams p) {
+// (four waves a SIMD: with three, the 3168 waves of 99 branches x 32 heads left a second round of a few; 99 branches x 32 heads over 768
+// positions of a page table 171 -> 150 us)
+template <bool FUSED, int WALK>
+__global__ __launch_bounds__(256, FUSED ? 1 : 4) void attn_suffix_kernel(AttnParams p) {
     // suffix_waves (1, 2 or 4) waves per (branch, query head): more than one while branches x heads leave CUs idle.
     // Workgroups are dealt round-robin to the 8 XCDs (8 L2s); the heads of one branch share the 128-byte lines of that
     // branch's scales (2 fp16 per head and position), so ALL workgroups of a branch go to one XCD: workgroup L of the 1-D
     // grid sits on XCD L % 8 and takes branch 8 (L / 8 / per_branch) + L % 8, head group (L / 8) % per_branch.
+    // (Branches share pages: the queries of a kv head on one XCD instead measured 104 us against 100 at 99 branches x 512 positions.)
     const int wave = threadIdx.x >> 6, nsub = p.suffix_waves;
     const int per_branch = (p.H * nsub + 3) >> 2;              // workgroups (four waves) per branch
     const int L = blockIdx.x, j = L >> 3;
@@ -856,7 +1080,7 @@ __global__ __launch_bounds__(256) void attn_suffix_kernel(AttnParams p) {
     const int h = nsub == 4 ? hq >> 2 : (nsub == 2 ? hq >> 1 : hq);
     if (nsub == 1 && h >= p.H) return;
     // with shared queries every wave reaches the fold's barrier: one past the last head repeats it and writes nothing
-    attn_suffix_body<FUSED, false>(p, b, min(h, p.H - 1), hq & (nsub - 1), nsub, h < p.H);
+    attn_suffix_body<FUSED, false, WALK>(p, b, min(h, p.H - 1), hq & (nsub - 1), nsub, h < p.H);
 }
 
 // ---- the whole decode attention in ONE launch -----------------------------------------------------------------
@@ -1036,10 +1260,24 @@ static int attn_plan_suffix_waves(int splits, int Bq, int Hkv) {
 
 }  // namespace smh
 
+// Partials and marks of attn_page_tile_kernel for pages_cols positions, 0 where the pass does not pay or apply.
+static size_t attn_tiles_bytes(int B, int H, int Hkv, int cols) {
+    const size_t slices = (size_t)(cols + smh::PT_TW - 1) / smh::PT_TW, tiles = ((size_t)B * (H / Hkv) + 15) / 16;
+    if (B < 2 || slices > smh::PT_MAX_SLICES || tiles > 65535) return 0;
+    return slices * B * H * (smh::ATT_D + 2) * sizeof(float) + slices * tiles * Hkv;
+}
+
 extern "C" size_t smh_attn_workspace_bytes(int B, int H, int P) {
     if (P <= 0 || B <= 0 || H <= 0) return 256;
     size_t splits = (size_t)(P + 31) / 32;          // worst case: 32 rows per workgroup
     return splits * (size_t)B * (size_t)H * (smh::ATT_D + 2) * sizeof(float) + 256;
+}
+
+extern "C" size_t smh_paged_attn_workspace_bytes(int B, int H, int Hkv, int P, int pages_cols) {
+    const size_t least = smh_attn_workspace_bytes(B, H, P);
+    if (P > 0 || B <= 0 || H <= 0 || Hkv <= 0 || H % Hkv != 0 || pages_cols <= 0) return least;
+    const size_t tiles = attn_tiles_bytes(B, H, Hkv, pages_cols);
+    return tiles > least ? tiles : least;
 }
 
 constexpr size_t ATT_COUNTER_BYTES = 4096;     // one-launch variants: arrival counters at the start of the workspace
@@ -1113,7 +1351,21 @@ static int shared_prefix_attn(const char *who, bool one, const void *q, void *ou
     if (p.splits > 0)
         hipLaunchKernelGGL(attn_prefix_kernel<false>, dim3(p.splits, Hkv, qgroups), dim3(256), 0, (hipStream_t)stream, p);
     p.suffix_waves = attn_plan_suffix_waves_two((long)B * H);
-    hipLaunchKernelGGL(attn_suffix_kernel<false>, dim3((unsigned)(((H * p.suffix_waves + 3) / 4) * ((B + 7) / 8 * 8))), dim3(256), 0, (hipStream_t)stream, p);
+    const bool fp16_pages = p.pages != nullptr && suffix_format == SMH_KV_FP16;
+    const size_t tile_bytes = fp16_pages && P == 0 && lens == nullptr ? attn_tiles_bytes(B, H, Hkv, Smax) : 0;
+    const unsigned wgs = (unsigned)(((H * p.suffix_waves + 3) / 4) * ((B + 7) / 8 * 8));
+    if (tile_bytes > 0 && workspace && workspace_bytes >= tile_bytes) {
+        const int tiles = (p.Bq + 15) / 16;
+        p.splits = (Smax + PT_TW - 1) / PT_TW;
+        n_part = (size_t)p.splits * Hkv * p.Bq;
+        p.part_ml = p.part_o + n_part * ATT_D;
+        p.tile_done = (uint8_t *)(p.part_ml + n_part * 2);
+        hipLaunchKernelGGL(attn_page_tile_kernel, dim3(Hkv, p.splits, tiles), dim3(256), 0, (hipStream_t)stream, p);
+        hipLaunchKernelGGL((attn_suffix_kernel<false, WALK_TILES>), dim3(wgs), dim3(256), 0, (hipStream_t)stream, p);
+        return launch_status();
+    }
+    if (suffix_format == SMH_KV_FP16) hipLaunchKernelGGL((attn_suffix_kernel<false, WALK_F16>), dim3(wgs), dim3(256), 0, (hipStream_t)stream, p);
+    else hipLaunchKernelGGL((attn_suffix_kernel<false, WALK_Q40>), dim3(wgs), dim3(256), 0, (hipStream_t)stream, p);
     return launch_status();
 }
 
@@ -1310,7 +1562,7 @@ extern "C" int smh_shared_prefix_attn_qkv(const void *qkv_partial, int ksplit, v
     if (p.splits > 0)
         hipLaunchKernelGGL(attn_prefix_kernel<true>, dim3(p.splits, Hkv, qgroups), dim3(256), 0, (hipStream_t)stream, p);
     p.suffix_waves = attn_plan_suffix_waves_two((long)B * H);
-    hipLaunchKernelGGL(attn_suffix_kernel<true>, dim3((unsigned)(((H * p.suffix_waves + 3) / 4) * ((B + 7) / 8 * 8))), dim3(256), 0, (hipStream_t)stream, p);
+    hipLaunchKernelGGL((attn_suffix_kernel<true, WALK_Q40>), dim3((unsigned)(((H * p.suffix_waves + 3) / 4) * ((B + 7) / 8 * 8))), dim3(256), 0, (hipStream_t)stream, p);
     return launch_status();
 }
 

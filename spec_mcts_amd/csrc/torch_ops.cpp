@@ -29,6 +29,7 @@ struct Api {
     decltype(&smh_sample_topk_rowtemp) sample_rowtemp;
     decltype(&smh_tree_step) tree_step;
     decltype(&smh_attn_workspace_bytes) attn_bytes;
+    decltype(&smh_paged_attn_workspace_bytes) paged_bytes;
     decltype(&smh_shared_prefix_attn) shared_attn;
     decltype(&smh_paged_prefix_attn) paged_attn;
 } api;
@@ -335,7 +336,9 @@ PyObject *paged_prefix_attn(Args x) {
         need(ck.dim() == 3 && ck.size(0) == B && ck.size(1) == Hkv && ck.size(2) == D, "cur_k must be [B, Hkv, D]");
     }
     at::Tensor out = at::empty_like(q);
-    const size_t bytes = api.attn_bytes((int)B, (int)H, (int)P);
+    // (the partials of shared pages only where the call can use them)
+    const size_t bytes = fmt == SMH_KV_FP16 && lens == nullptr ? api.paged_bytes((int)B, (int)H, (int)Hkv, (int)P, (int)pages.size(1))
+                                                               : api.attn_bytes((int)B, (int)H, (int)P);
     at::Tensor ws = empty({(int64_t)bytes}, at::kByte, q);
     check(api.paged_attn(q.data_ptr(), out.data_ptr(), (int)B, (int)H, (int)Hkv, (int)D, P > 0 ? ptr(x[8]) : nullptr, P > 0 ? ptr(x[9]) : nullptr, (int)P, p_row, p_head,
                          fmt, pk.data_ptr(), pv.data_ptr(), ptr(x[5]), ptr(x[6]), row_stride, head_stride, rows, pages.data_ptr(), page_bytes, pages.stride(0),
@@ -375,6 +378,7 @@ PyObject *connect(PyObject *, PyObject *const *args, Py_ssize_t n) {
     find(api.sample_rowtemp, "smh_sample_topk_rowtemp");
     find(api.tree_step, "smh_tree_step");
     find(api.attn_bytes, "smh_attn_workspace_bytes");
+    find(api.paged_bytes, "smh_paged_attn_workspace_bytes");
     find(api.shared_attn, "smh_shared_prefix_attn");
     find(api.paged_attn, "smh_paged_prefix_attn");
     if (!ok) { PyErr_SetString(PyExc_RuntimeError, "the library lacks an entry point: build it again"); return nullptr; }

@@ -221,3 +221,29 @@ def test_lens_are_cut_to_the_columns_of_a_sliced_table():
     got = K.paged_prefix_attn(q.cuda(), tail, over, kp.cuda(), vp.cuda(), head_major=True).cpu().float()
     want = sdpa(q, pager[:, L - cols:], kp, vp)
     assert torch.allclose(got, want, atol=1e-2, rtol=0)
+
+
+@pytest.mark.parametrize("B,H,Hkv,L,shared", [(2, 8, 8, 64, 64), (17, 8, 8, 65, 40), (33, 16, 8, 129, 128), (16, 3, 3, 200, 192), (5, 32, 8, 63, 0),
+                                              (40, 8, 8, 4096, 4000), (3, 8, 8, 4097, 4000)])
+@pytest.mark.parametrize("odd", [False, True])
+def test_pages_shared_by_the_branches_of_a_tile(B, H, Hkv, L, shared, odd):
+    """Slices of 64 positions whose ids agree over the branches of 16 queries take the matrix-core pass: edges of slices and
+    tiles, GQA, one branch that differs in the middle of the shared run, infinite values in a shared page (left to the walk)."""
+    from spec_mcts_amd import kernels as K
+    g = torch.Generator().manual_seed(B * L)
+    rows = shared + B * (L - shared) + 1
+    pages = torch.zeros((B, L), dtype=torch.int32)
+    pages[:, :shared] = torch.randperm(shared, generator=g).int()
+    pages[:, shared:] = shared + torch.arange(B * (L - shared), dtype=torch.int32).view(B, L - shared)
+    k, v = (torch.empty((Hkv, rows, 128)).normal_(0.0, 0.5, generator=g).half() for _ in range(2))
+    q = torch.empty((B, H, 128)).normal_(0.0, 0.5, generator=g).half()
+    if odd:
+        pages[B // 2, shared // 2] = rows - 1
+        if shared:
+            v[0, pages[0, shared - 1]] = float("inf")
+    rep = lambda x: x.repeat_interleave(H // Hkv, 0)
+    want = sdpa(q, pages, rep(k), rep(v))
+    got = K.paged_prefix_attn(q.cuda(), pages.cuda(), None, k.cuda(), v.cuda(), head_major=True).cpu().float()
+    assert torch.equal(got.isinf(), want.isinf())
+    fin = want.isfinite()
+    assert bool(((got - want)[fin].abs() <= 2e-3 + 1e-2 * want[fin].abs()).all())
