@@ -1,7 +1,7 @@
 // Q4_0 dequant + matmul for large batches (decode at B = 100, prefill): c[M,N] = a[M,K] . deq(W)[K,N].
 //
-// A workgroup of 4 waves (8 on tiled weights, plus one that only issues DMA in launches with one workgroup per compute
-// unit, see the kernel) owns 128 rows of A, two adjacent 128-column blocks of the weight (one full 128-byte line of
+// A workgroup of 4 waves (8 plus one that only issues DMA in launches with one workgroup per compute unit, and 8 on tiled weights,
+// see the kernel) owns 128 rows of A, two adjacent 128-column blocks of the weight (one full 128-byte line of
 // packed nibbles per k) and a slice of K - or, under a range cut, a run of steps that may end one column unit and begin
 // the next; up to two workgroups share a compute unit.  Everything a 32-row step needs - 4 KB of nibbles, 256 B of scales, the 128 x 32 tile of A -
 // goes global -> LDS by DMA (global_load_lds) into a 6-slot ring shared by the workgroup; one bare s_barrier
@@ -33,7 +33,7 @@ namespace smh {
 // most K-slices of a launch = GEMM_KSCAP / rows (every slice leaves an fp32 slab of rows x columns)
 constexpr int GEMM_KSCAP = 1600;
 constexpr int GEMM_BM = 128;
-constexpr int GEMM_WAVES = 4;                  // checkpoint layout and ragged K; tiled weights run GEMM_TILED_WAVES
+constexpr int GEMM_WAVES = 4;                  // ragged K, and the checkpoint layout where workgroups share compute units; the rest runs GEMM_TILED_WAVES
 constexpr int GEMM_TILED_WAVES = 8;
 constexpr int GEMM_THREADS = GEMM_WAVES * 64;
 // slots of the DMA ring (with a barrier per step, four slots measured 2 % faster per launch at M=100 than six; with a
@@ -80,7 +80,7 @@ __device__ __forceinline__ void gemm_barrier() { asm volatile("s_waitcnt lgkmcnt
 // TILED: the weights are in the tiled layout (q40_matmul.hpp).  Wave w then moves and decodes piece w of a
 // tile (its two byte positions of its block, already paired by rows): one 16-byte LDS read instead of eight
 // dword reads, shifts instead of byte permutes, the scales already in operand order; rows past K hold zeros.
-// WAVES = 8 (tiled weights only): waves w and w + 4 share piece w of a tile; wave w multiplies the columns of its HIGH
+// WAVES = 8: waves w and w + 4 share piece w of a tile; wave w multiplies the columns of its HIGH
 // nibbles, wave w + 4 those of the low nibbles (two B operands and half the accumulators each, the same A tiles), so
 // that every SIMD holds two waves of the workgroup and the decode of one runs under the MFMAs of the other.
 //
@@ -148,6 +148,12 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
     // can go between the MFMAs of a step
     auto issue_ws8 = [&](int step, int slot_) {
         uint8_t *st = lds + slot_ * GS_BYTES;
+        if (!TILED) {
+            const long k0 = (long)step * 32;
+            if (hh == 0) __builtin_amdgcn_global_load_lds((gptr_t)(w_base + k0 * w_row + w_voff), (lptr_t)(st + wave * GS_WBLOCK), 16, 0, 0);
+            else if (lane < 16) __builtin_amdgcn_global_load_lds((gptr_t)(s_base + k0 * s_row + s_voff), (lptr_t)(st + GS_W + wave * 64), 4, 0, 0);
+            return;
+        }
         const uint8_t *tile = w_base + (long)step * TILE_BYTES;
         if (hh == 0) __builtin_amdgcn_global_load_lds((gptr_t)(tile + piece_off(wave) + lane * 16), (lptr_t)(st + wave * 1024), 16, 0, 0);
         else if (lane < 16) __builtin_amdgcn_global_load_lds((gptr_t)(tile + scale_off(wave, lane)), (lptr_t)(st + GS_W + wave * 64), 4, 0, 0);
@@ -158,12 +164,10 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
     auto issue = [&](int step, int slot_) {
         uint8_t *st = lds + slot_ * GS_BYTES;
         const long k0 = (long)step * 32;
-        if (TILED && WAVES == 8) {
+        if (WAVES == 8) {
             // two DMA instructions a wave: waves 0-3 their piece of the nibbles, waves 4-7 its scales; every wave 16 rows of A
-            const uint8_t *tile = w_base + (long)step * TILE_BYTES;
-            if (hh == 0) __builtin_amdgcn_global_load_lds((gptr_t)(tile + piece_off(wave) + lane * 16), (lptr_t)(st + wave * 1024), 16, 0, 0);
-            else if (lane < 16) __builtin_amdgcn_global_load_lds((gptr_t)(tile + scale_off(wave, lane)), (lptr_t)(st + GS_W + wave * 64), 4, 0, 0);
-            __builtin_amdgcn_global_load_lds((gptr_t)(a_base + k0 * 2 + a_voff0), (lptr_t)(st + GS_W + GS_S + wave8 * 1024), 16, 0, 0);
+            issue_ws8(step, slot_);
+            issue_a8(step, slot_);
         } else if (TILED) {
             const uint8_t *tile = w_base + (long)step * TILE_BYTES;
             __builtin_amdgcn_global_load_lds((gptr_t)(tile + wave * 1024 + lane * 16), (lptr_t)(st + wave * 1024), 16, 0, 0);
@@ -219,14 +223,24 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
 #pragma unroll
             for (int t = 0; t < TILES; ++t)
                 a_voff[t] = (uint32_t)((long)min(m0 + 16 * t + (lane >> 2), p.M - 1) * p.lda * 2 + 16 * a_chunk);
+            // checkpoint layout: lane l moves 16 bytes of row l / 8 of a piece and the dword l % 2 of row l / 2 of the scales
+            const uint32_t raw_w = (uint32_t)((lane >> 3) * w_row + w_lcol), raw_s = (uint32_t)((lane >> 1) * s_row + s_lcol);
             auto issue_all = [&](int slot_) {
                 uint8_t *st = lds + slot_ * GS_BYTES;
-                const uint8_t *tile = w_base + (long)fetch * TILE_BYTES;
                 const uint8_t *arow = a_base + (long)fetch * 64;
+                if (TILED) {
+                    const uint8_t *tile = w_base + (long)fetch * TILE_BYTES;
 #pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    __builtin_amdgcn_global_load_lds((gptr_t)(tile + piece_off(q) + lane * 16), (lptr_t)(st + q * 1024), 16, 0, 0);
-                __builtin_amdgcn_global_load_lds((gptr_t)(tile + scale_off(lane >> 4, lane & 15)), (lptr_t)(st + GS_W), 4, 0, 0);
+                    for (int q = 0; q < 4; ++q)
+                        __builtin_amdgcn_global_load_lds((gptr_t)(tile + piece_off(q) + lane * 16), (lptr_t)(st + q * 1024), 16, 0, 0);
+                    __builtin_amdgcn_global_load_lds((gptr_t)(tile + scale_off(lane >> 4, lane & 15)), (lptr_t)(st + GS_W), 4, 0, 0);
+                } else {
+                    const uint8_t *rows = w_base + (long)fetch * 32 * w_row;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        __builtin_amdgcn_global_load_lds((gptr_t)(rows + 8 * q * w_row + raw_w), (lptr_t)(st + q * GS_WBLOCK), 16, 0, 0);
+                    __builtin_amdgcn_global_load_lds((gptr_t)(s_base + (long)fetch * 32 * s_row + raw_s), (lptr_t)(st + GS_W), 4, 0, 0);
+                }
 #pragma unroll
                 for (int t = 0; t < TILES; ++t)
                     __builtin_amdgcn_global_load_lds((gptr_t)(arow + a_voff[t]), (lptr_t)(st + GS_W + GS_S + t * 1024), 16, 0, 0);
@@ -310,8 +324,23 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
     asm volatile("" : "+v"(nib_magic));                       // then ONE v_and_or_b32 (no literal operands there), not an AND and an OR
     const h2 nib_mul = hh == 0 ? h2{(half_t)0.0625f, (half_t)0.0625f} : h2{(half_t)1.0f, (half_t)1.0f};
     const h2 nib_off = hh == 0 ? h2{(half_t)-72.0f, (half_t)-72.0f} : h2{(half_t)-1032.0f, (half_t)-1032.0f};
+    // checkpoint layout: codes are two's complement, so the nibble's top bit is flipped in the same three-input operation
+    uint32_t raw_magic = MAGIC_1024 ^ (hh == 0 ? 0x00800080u : 0x00080008u);
+    const uint32_t raw_scale = hh == 0 ? 0x05040100u : 0x07060302u;        // the first or the second 64 columns' scale of two rows
     auto decode = [&](const uint32_t (&wv)[8], const uint32_t (&sv)[8], bool dead, h8 (&b)[NB]) {
         u32x4 v0h, v0l, v1h, v1l;
+        if (!TILED && WAVES == 8) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t pr0 = __builtin_amdgcn_perm(wv[2 * j + 1], wv[2 * j], sel0), pr1 = __builtin_amdgcn_perm(wv[2 * j + 1], wv[2 * j], sel1);
+                const h2 sc = as_h2(__builtin_amdgcn_perm(sv[2 * j + 1], sv[2 * j], raw_scale));
+                v0h[j] = as_u32(__builtin_elementwise_fma(as_h2((pr0 & nib_mask) ^ raw_magic), nib_mul, nib_off) * sc);
+                v1h[j] = as_u32(__builtin_elementwise_fma(as_h2((pr1 & nib_mask) ^ raw_magic), nib_mul, nib_off) * sc);
+            }
+            b[0] = __builtin_bit_cast(h8, v0h);
+            b[1] = __builtin_bit_cast(h8, v1h);
+            return;
+        }
         if (TILED && WAVES == 8) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -421,7 +450,7 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
             if constexpr (PRODUCER) {
                 one_step();
                 one_step();
-            } else if constexpr (TILED && WAVES == 8 && TILES < 8) {       // (with all 8 row tiles, the prefill, this form measured 5-8 % slower)
+            } else if constexpr (WAVES == 8 && TILES < 8) {       // (with all 8 row tiles, the prefill, this form measured 5-8 % slower)
                 // the nibbles and scales of the two refills now, their A rows from inside the steps: the address unit takes
                 // 16 cycles per instruction, and between MFMAs the wave has them to spare (2 % off a launch at 100 rows;
                 // the nibbles and scales too from inside the steps, behind their branches: 4 % slower)
@@ -575,7 +604,7 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
 template <int TILES, bool RAGGED, bool TILED, int WAVES, int SLOTS = GEMM_STAGES, bool PRODUCER = false, bool RANGE = false, bool SWIGLU = false>
 // (SWIGLU without the DMA wave: at most 128 registers, so that two workgroups of eight waves fit a compute unit)
 __global__ __launch_bounds__(64 * (WAVES + (PRODUCER ? 1 : 0)), WAVES == 8 ? (SWIGLU && !PRODUCER ? 4 : 1) : 2) void q40_gemm_kernel(MatmulParams p) {
-    static_assert(WAVES == 4 || (WAVES == 8 && TILED && !RAGGED), "eight waves: tiled weights, K a multiple of 32");
+    static_assert(WAVES == 4 || (WAVES == 8 && !RAGGED), "eight waves: K a multiple of 32");
     static_assert(SLOTS >= 6 && SLOTS <= 10 && (SLOTS == GEMM_STAGES || PRODUCER) && (!PRODUCER || WAVES == 8), "ring depth");
     const int steps_total = (p.K + 31) / 32;
     if constexpr (RANGE) {
@@ -1179,19 +1208,21 @@ static int gemm_launch_layout(const MatmulParams &p, hipStream_t stream) {
                                            q40_gemm_kernel<3, false, TILED, W>, q40_gemm_kernel<4, false, TILED, W>,
                                            q40_gemm_kernel<5, false, TILED, W>, q40_gemm_kernel<6, false, TILED, W>,
                                            q40_gemm_kernel<7, false, TILED, W>, q40_gemm_kernel<8, false, TILED, W>};
-    // one workgroup per compute unit: the variant with the DMA wave
-    constexpr bool HAS_DMA_WAVE = W == 8;
-    constexpr int PS = HAS_DMA_WAVE ? GEMM_DMA_WAVE_SLOTS : GEMM_STAGES;
+    // one workgroup per compute unit: eight waves and the DMA wave, on both layouts.  (Checkpoint layout, against four waves that
+    // leave every SIMD one: 100 rows x 11008 x 4096 31.9 -> 27.2 us, x 32128 61 -> 51, 20 x 28672 x 8192 66 -> 51, 160 x 28672 x
+    // 4096 96 -> 64.  Where two workgroups of four waves share a compute unit, eight re-read each nibble from LDS for nothing:
+    // 512 x 28672 x 8192 312-324 us against 314, 512 x 20480 x 12288 412 against 389.)
+    constexpr int WD = GEMM_TILED_WAVES, PS = GEMM_DMA_WAVE_SLOTS;
     static const gemm_kernel_t with_dma_wave[9] = {
-        nullptr, q40_gemm_kernel<2, false, TILED, W, PS, HAS_DMA_WAVE>, q40_gemm_kernel<2, false, TILED, W, PS, HAS_DMA_WAVE>,
-        q40_gemm_kernel<3, false, TILED, W, PS, HAS_DMA_WAVE>, q40_gemm_kernel<4, false, TILED, W, PS, HAS_DMA_WAVE>,
-        q40_gemm_kernel<5, false, TILED, W, PS, HAS_DMA_WAVE>, q40_gemm_kernel<6, false, TILED, W, PS, HAS_DMA_WAVE>,
-        q40_gemm_kernel<7, false, TILED, W, PS, HAS_DMA_WAVE>, q40_gemm_kernel<8, false, TILED, W, PS, HAS_DMA_WAVE>};
+        nullptr, q40_gemm_kernel<2, false, TILED, WD, PS, true>, q40_gemm_kernel<2, false, TILED, WD, PS, true>,
+        q40_gemm_kernel<3, false, TILED, WD, PS, true>, q40_gemm_kernel<4, false, TILED, WD, PS, true>,
+        q40_gemm_kernel<5, false, TILED, WD, PS, true>, q40_gemm_kernel<6, false, TILED, WD, PS, true>,
+        q40_gemm_kernel<7, false, TILED, WD, PS, true>, q40_gemm_kernel<8, false, TILED, WD, PS, true>};
     static const gemm_kernel_t range_cut[9] = {
-        nullptr, q40_gemm_kernel<2, false, TILED, W, PS, HAS_DMA_WAVE, true>, q40_gemm_kernel<2, false, TILED, W, PS, HAS_DMA_WAVE, true>,
-        q40_gemm_kernel<3, false, TILED, W, PS, HAS_DMA_WAVE, true>, q40_gemm_kernel<4, false, TILED, W, PS, HAS_DMA_WAVE, true>,
-        q40_gemm_kernel<5, false, TILED, W, PS, HAS_DMA_WAVE, true>, q40_gemm_kernel<6, false, TILED, W, PS, HAS_DMA_WAVE, true>,
-        q40_gemm_kernel<7, false, TILED, W, PS, HAS_DMA_WAVE, true>, q40_gemm_kernel<8, false, TILED, W, PS, HAS_DMA_WAVE, true>};
+        nullptr, q40_gemm_kernel<2, false, TILED, WD, PS, true, true>, q40_gemm_kernel<2, false, TILED, WD, PS, true, true>,
+        q40_gemm_kernel<3, false, TILED, WD, PS, true, true>, q40_gemm_kernel<4, false, TILED, WD, PS, true, true>,
+        q40_gemm_kernel<5, false, TILED, WD, PS, true, true>, q40_gemm_kernel<6, false, TILED, WD, PS, true, true>,
+        q40_gemm_kernel<7, false, TILED, WD, PS, true, true>, q40_gemm_kernel<8, false, TILED, WD, PS, true, true>};
     static const gemm_kernel_t ragged = q40_gemm_kernel<8, true, TILED, 4>;
     // more than 64 KB of dynamic LDS has to be allowed once per kernel (the attribute is not stream work,
     // so a launch under graph capture is not affected)
@@ -1199,7 +1230,7 @@ static int gemm_launch_layout(const MatmulParams &p, hipStream_t stream) {
         hipError_t e = hipFuncSetAttribute((const void *)ragged, hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS);
         for (int t = 2; t <= 8 && e == hipSuccess; ++t)
             e = hipFuncSetAttribute((const void *)exact[t], hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS);
-        for (int t = 2; t <= 8 && e == hipSuccess && HAS_DMA_WAVE; ++t)
+        for (int t = 2; t <= 8 && e == hipSuccess; ++t)
             e = hipFuncSetAttribute((const void *)with_dma_wave[t], hipFuncAttributeMaxDynamicSharedMemorySize, PS * GS_BYTES);
         for (int t = 2; t <= 8 && e == hipSuccess; ++t)
             e = hipFuncSetAttribute((const void *)range_cut[t], hipFuncAttributeMaxDynamicSharedMemorySize, PS * GS_BYTES);
@@ -1211,11 +1242,11 @@ static int gemm_launch_layout(const MatmulParams &p, hipStream_t stream) {
     }
     SMH_REQUIRE((long)p.M * p.lda * 2 < (1L << 32), "q40 gemm: M x lda = %d x %ld exceeds the 32-bit lane offsets of A", p.M, p.lda);
     const int tiles = p.mblocks > 1 ? p.block_rows / 16 : (p.M + 15) / 16;
-    const bool one_each = HAS_DMA_WAVE && p.K % 32 == 0 && (p.chunk > 0 || (long)p.units * p.mblocks * p.ksplit <= GEMM_DMA_WAVE_MAX_WGS);
+    const bool one_each = p.K % 32 == 0 && (p.chunk > 0 || (long)p.units * p.mblocks * p.ksplit <= GEMM_DMA_WAVE_MAX_WGS);
     const gemm_kernel_t kern = (p.K % 32 != 0) ? ragged : (p.chunk > 0 ? range_cut : one_each ? with_dma_wave : exact)[tiles < 2 ? 2 : tiles];
     const long total_steps = (long)p.units * ((p.K + 31) / 32);
     dim3 grid((unsigned)(p.chunk > 0 ? (total_steps + p.chunk - 1) / p.chunk : (long)p.units_pad * p.mblocks * p.ksplit));
-    hipLaunchKernelGGL(kern, grid, dim3(kern == ragged ? GEMM_THREADS : 64 * W + (one_each ? 64 : 0)), one_each ? PS * GS_BYTES : GEMM_LDS, stream, p);
+    hipLaunchKernelGGL(kern, grid, dim3(kern == ragged ? GEMM_THREADS : one_each ? 64 * (WD + 1) : 64 * W), one_each ? PS * GS_BYTES : GEMM_LDS, stream, p);
     return launch_status();
 }
 

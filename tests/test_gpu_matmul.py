@@ -121,6 +121,22 @@ def test_ragged_k_and_small_shapes(M, N, Kd):
     _check(got, O.matmul_q40(a, w, s, (Kd, N)))
 
 
+@pytest.mark.parametrize("M,N,Kd", [(17, 128, 32), (33, 384, 160), (48, 128, 4096), (64, 11008, 256), (81, 640, 1056), (100, 20224, 512),
+                                    (128, 384, 2048), (129, 128, 224), (250, 8192, 96), (300, 24704, 64)])
+def test_checkpoint_layout_by_workgroups(M, N, Kd):
+    """eight waves and the DMA wave (one workgroup a compute unit, range cut among them) or four waves: column units of one block,
+    few steps, edges of row tiles; fp32 sums of exact products, one rounding to fp16"""
+    from spec_mcts_amd import kernels as K
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    w, s = K.quantize_q40(torch.randn((Kd, N), device="cuda", generator=g).half())
+    x = torch.randn((M, Kd), device="cuda", generator=g).half()
+    d = K.deq_int40(w, s, 64, (Kd, N))
+    want = x.double() @ d.double()
+    got = K.matmul_q40(x, w, s, (Kd, N)).double()
+    bound = want.abs() * 2.0 ** -11 + 2.0 ** -24 + (x.double().abs() @ d.double().abs()) * Kd * 2.0 ** -24      # the rounding; sums of Kd terms
+    assert bool(((got - want).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("M", [4, 100])
 def test_residual_epilogue(M):
     from spec_mcts_amd import kernels as K
