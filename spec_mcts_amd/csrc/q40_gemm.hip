@@ -25,6 +25,7 @@
 // At M = 100 the work sits on the ridge of the roofline: 2*M*N*K flops against
 // N*K*0.53125 + 2*M*(K+N) bytes.
 #include <type_traits>
+#include <utility>
 
 #include "q40_matmul.hpp"
 
@@ -148,12 +149,6 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
     // can go between the MFMAs of a step
     auto issue_ws8 = [&](int step, int slot_) {
         uint8_t *st = lds + slot_ * GS_BYTES;
-        if (!TILED) {
-            const long k0 = (long)step * 32;
-            if (hh == 0) __builtin_amdgcn_global_load_lds((gptr_t)(w_base + k0 * w_row + w_voff), (lptr_t)(st + wave * GS_WBLOCK), 16, 0, 0);
-            else if (lane < 16) __builtin_amdgcn_global_load_lds((gptr_t)(s_base + k0 * s_row + s_voff), (lptr_t)(st + GS_W + wave * 64), 4, 0, 0);
-            return;
-        }
         const uint8_t *tile = w_base + (long)step * TILE_BYTES;
         if (hh == 0) __builtin_amdgcn_global_load_lds((gptr_t)(tile + piece_off(wave) + lane * 16), (lptr_t)(st + wave * 1024), 16, 0, 0);
         else if (lane < 16) __builtin_amdgcn_global_load_lds((gptr_t)(tile + scale_off(wave, lane)), (lptr_t)(st + GS_W + wave * 64), 4, 0, 0);
@@ -223,8 +218,12 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
 #pragma unroll
             for (int t = 0; t < TILES; ++t)
                 a_voff[t] = (uint32_t)((long)min(m0 + 16 * t + (lane >> 2), p.M - 1) * p.lda * 2 + 16 * a_chunk);
-            // checkpoint layout: lane l moves 16 bytes of row l / 8 of a piece and the dword l % 2 of row l / 2 of the scales
+            // checkpoint layout: lane l moves 16 bytes of row l / 8 of a piece and the dword l % 2 of row l / 2 of the scales.
+            // RAGGED: the last step has `left` = 8, 16 or 24 rows of k; what lies past them repeats valid ones (masked when decoded)
+            const int last = RAGGED ? (p.K - 1) / 32 : -1, left = p.K - 32 * last;
             const uint32_t raw_w = (uint32_t)((lane >> 3) * w_row + w_lcol), raw_s = (uint32_t)((lane >> 1) * s_row + s_lcol);
+            const uint32_t raw_s_last = RAGGED ? (uint32_t)(min(lane >> 1, left - 1) * s_row + s_lcol) : 0;
+            const uint32_t a_back = RAGGED ? (uint32_t)(2 * (8 * a_chunk - min(8 * a_chunk, left - 8))) : 0;
             auto issue_all = [&](int slot_) {
                 uint8_t *st = lds + slot_ * GS_BYTES;
                 const uint8_t *arow = a_base + (long)fetch * 64;
@@ -236,14 +235,17 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
                     __builtin_amdgcn_global_load_lds((gptr_t)(tile + scale_off(lane >> 4, lane & 15)), (lptr_t)(st + GS_W), 4, 0, 0);
                 } else {
                     const uint8_t *rows = w_base + (long)fetch * 32 * w_row;
+                    const bool at_end = RAGGED && fetch == last;
 #pragma unroll
                     for (int q = 0; q < 4; ++q)
-                        __builtin_amdgcn_global_load_lds((gptr_t)(rows + 8 * q * w_row + raw_w), (lptr_t)(st + q * GS_WBLOCK), 16, 0, 0);
-                    __builtin_amdgcn_global_load_lds((gptr_t)(s_base + (long)fetch * 32 * s_row + raw_s), (lptr_t)(st + GS_W), 4, 0, 0);
+                        __builtin_amdgcn_global_load_lds((gptr_t)(rows + (at_end && 8 * q >= left ? 0 : 8 * q) * w_row + raw_w),
+                                                         (lptr_t)(st + q * GS_WBLOCK), 16, 0, 0);
+                    __builtin_amdgcn_global_load_lds((gptr_t)(s_base + (long)fetch * 32 * s_row + (at_end ? raw_s_last : raw_s)), (lptr_t)(st + GS_W), 4, 0, 0);
                 }
 #pragma unroll
                 for (int t = 0; t < TILES; ++t)
-                    __builtin_amdgcn_global_load_lds((gptr_t)(arow + a_voff[t]), (lptr_t)(st + GS_W + GS_S + t * 1024), 16, 0, 0);
+                    __builtin_amdgcn_global_load_lds((gptr_t)(arow + (RAGGED && fetch == last ? a_voff[t] - a_back : a_voff[t])),
+                                                     (lptr_t)(st + GS_W + GS_S + t * 1024), 16, 0, 0);
                 fetch = fetch + 1 == step1 ? step0 : fetch + 1;
             };
 #pragma unroll
@@ -333,7 +335,9 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const uint32_t pr0 = __builtin_amdgcn_perm(wv[2 * j + 1], wv[2 * j], sel0), pr1 = __builtin_amdgcn_perm(wv[2 * j + 1], wv[2 * j], sel1);
-                const h2 sc = as_h2(__builtin_amdgcn_perm(sv[2 * j + 1], sv[2 * j], raw_scale));
+                uint32_t pair = __builtin_amdgcn_perm(sv[2 * j + 1], sv[2 * j], raw_scale);
+                if (RAGGED) pair = dead ? 0u : pair;           // k >= K: no contribution
+                const h2 sc = as_h2(pair);
                 v0h[j] = as_u32(__builtin_elementwise_fma(as_h2((pr0 & nib_mask) ^ raw_magic), nib_mul, nib_off) * sc);
                 v1h[j] = as_u32(__builtin_elementwise_fma(as_h2((pr1 & nib_mask) ^ raw_magic), nib_mul, nib_off) * sc);
             }
@@ -604,7 +608,7 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
 template <int TILES, bool RAGGED, bool TILED, int WAVES, int SLOTS = GEMM_STAGES, bool PRODUCER = false, bool RANGE = false, bool SWIGLU = false>
 // (SWIGLU without the DMA wave: at most 128 registers, so that two workgroups of eight waves fit a compute unit)
 __global__ __launch_bounds__(64 * (WAVES + (PRODUCER ? 1 : 0)), WAVES == 8 ? (SWIGLU && !PRODUCER ? 4 : 1) : 2) void q40_gemm_kernel(MatmulParams p) {
-    static_assert(WAVES == 4 || (WAVES == 8 && !RAGGED), "eight waves: K a multiple of 32");
+    static_assert(WAVES == 4 || (WAVES == 8 && (TILED ? !RAGGED : PRODUCER)), "eight waves: K a multiple of 32, or the checkpoint layout with a DMA wave");
     static_assert(SLOTS >= 6 && SLOTS <= 10 && (SLOTS == GEMM_STAGES || PRODUCER) && (!PRODUCER || WAVES == 8), "ring depth");
     const int steps_total = (p.K + 31) / 32;
     if constexpr (RANGE) {
@@ -1223,17 +1227,27 @@ static int gemm_launch_layout(const MatmulParams &p, hipStream_t stream) {
         q40_gemm_kernel<3, false, TILED, WD, PS, true, true>, q40_gemm_kernel<4, false, TILED, WD, PS, true, true>,
         q40_gemm_kernel<5, false, TILED, WD, PS, true, true>, q40_gemm_kernel<6, false, TILED, WD, PS, true, true>,
         q40_gemm_kernel<7, false, TILED, WD, PS, true, true>, q40_gemm_kernel<8, false, TILED, WD, PS, true, true>};
+    // K not a multiple of 32: on tiled weights one kernel for all row counts, on the checkpoint layout the two forms from above with
+    // a masked last step (against one four-wave kernel of eight row tiles: 33
+    // rows x 11008 x 4072 29.7 -> 19.4 us, 100 rows 34.5 -> 27.6, 20 x 28672 x 8200 103 -> 53, 512 x 4096 x 4104 50 -> 40)
     static const gemm_kernel_t ragged = q40_gemm_kernel<8, true, TILED, 4>;
+    static const gemm_kernel_t ragged_four[9] = {nullptr, q40_gemm_kernel<2, true, false, 4>, q40_gemm_kernel<2, true, false, 4>, q40_gemm_kernel<3, true, false, 4>,
+                                                 q40_gemm_kernel<4, true, false, 4>, q40_gemm_kernel<5, true, false, 4>, q40_gemm_kernel<6, true, false, 4>,
+                                                 q40_gemm_kernel<7, true, false, 4>, q40_gemm_kernel<8, true, false, 4>};
+    static const gemm_kernel_t ragged_dma_wave[9] = {
+        nullptr, q40_gemm_kernel<2, true, false, WD, PS, true>, q40_gemm_kernel<2, true, false, WD, PS, true>, q40_gemm_kernel<3, true, false, WD, PS, true>,
+        q40_gemm_kernel<4, true, false, WD, PS, true>, q40_gemm_kernel<5, true, false, WD, PS, true>, q40_gemm_kernel<6, true, false, WD, PS, true>,
+        q40_gemm_kernel<7, true, false, WD, PS, true>, q40_gemm_kernel<8, true, false, WD, PS, true>};
     // more than 64 KB of dynamic LDS has to be allowed once per kernel (the attribute is not stream work,
     // so a launch under graph capture is not affected)
     static const hipError_t lds_ok = [] {
         hipError_t e = hipFuncSetAttribute((const void *)ragged, hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS);
-        for (int t = 2; t <= 8 && e == hipSuccess; ++t)
-            e = hipFuncSetAttribute((const void *)exact[t], hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS);
-        for (int t = 2; t <= 8 && e == hipSuccess; ++t)
-            e = hipFuncSetAttribute((const void *)with_dma_wave[t], hipFuncAttributeMaxDynamicSharedMemorySize, PS * GS_BYTES);
-        for (int t = 2; t <= 8 && e == hipSuccess; ++t)
-            e = hipFuncSetAttribute((const void *)range_cut[t], hipFuncAttributeMaxDynamicSharedMemorySize, PS * GS_BYTES);
+        for (int t = 2; t <= 8 && e == hipSuccess; ++t) {
+            const std::pair<gemm_kernel_t, int> all[5] = {{exact[t], GEMM_LDS}, {ragged_four[t], GEMM_LDS}, {with_dma_wave[t], PS * GS_BYTES},
+                                                          {range_cut[t], PS * GS_BYTES}, {ragged_dma_wave[t], PS * GS_BYTES}};
+            for (int i = 0; i < 5 && e == hipSuccess; ++i)
+                e = hipFuncSetAttribute((const void *)all[i].first, hipFuncAttributeMaxDynamicSharedMemorySize, all[i].second);
+        }
         return e;
     }();
     if (lds_ok != hipSuccess) {
@@ -1241,12 +1255,15 @@ static int gemm_launch_layout(const MatmulParams &p, hipStream_t stream) {
         return (int)lds_ok;
     }
     SMH_REQUIRE((long)p.M * p.lda * 2 < (1L << 32), "q40 gemm: M x lda = %d x %ld exceeds the 32-bit lane offsets of A", p.M, p.lda);
-    const int tiles = p.mblocks > 1 ? p.block_rows / 16 : (p.M + 15) / 16;
-    const bool one_each = p.K % 32 == 0 && (p.chunk > 0 || (long)p.units * p.mblocks * p.ksplit <= GEMM_DMA_WAVE_MAX_WGS);
-    const gemm_kernel_t kern = (p.K % 32 != 0) ? ragged : (p.chunk > 0 ? range_cut : one_each ? with_dma_wave : exact)[tiles < 2 ? 2 : tiles];
+    const int tiles = max(2, p.mblocks > 1 ? p.block_rows / 16 : (p.M + 15) / 16);
+    const bool odd_k = p.K % 32 != 0;
+    const bool one_each = !(TILED && odd_k) && (p.chunk > 0 || (long)p.units * p.mblocks * p.ksplit <= GEMM_DMA_WAVE_MAX_WGS);
+    const bool four = odd_k ? !one_each : !TILED && !one_each;
+    const gemm_kernel_t kern = odd_k ? (TILED ? ragged : (one_each ? ragged_dma_wave : ragged_four)[tiles])
+                                     : (p.chunk > 0 ? range_cut : one_each ? with_dma_wave : exact)[tiles];
     const long total_steps = (long)p.units * ((p.K + 31) / 32);
     dim3 grid((unsigned)(p.chunk > 0 ? (total_steps + p.chunk - 1) / p.chunk : (long)p.units_pad * p.mblocks * p.ksplit));
-    hipLaunchKernelGGL(kern, grid, dim3(kern == ragged ? GEMM_THREADS : one_each ? 64 * (WD + 1) : 64 * W), one_each ? PS * GS_BYTES : GEMM_LDS, stream, p);
+    hipLaunchKernelGGL(kern, grid, dim3(one_each ? 64 * (WD + 1) : four ? GEMM_THREADS : 64 * W), one_each ? PS * GS_BYTES : GEMM_LDS, stream, p);
     return launch_status();
 }
 

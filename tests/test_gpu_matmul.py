@@ -122,7 +122,10 @@ def test_ragged_k_and_small_shapes(M, N, Kd):
 
 
 @pytest.mark.parametrize("M,N,Kd", [(17, 128, 32), (33, 384, 160), (48, 128, 4096), (64, 11008, 256), (81, 640, 1056), (100, 20224, 512),
-                                    (128, 384, 2048), (129, 128, 224), (250, 8192, 96), (300, 24704, 64)])
+                                    (128, 384, 2048), (129, 128, 224), (250, 8192, 96), (300, 24704, 64),
+                                    # K not a multiple of 32: 8, 16 and 24 rows of k in the last step, also as the only step of a slice
+                                    (17, 128, 8), (33, 384, 168), (64, 11008, 264), (81, 640, 1048), (100, 4096, 4088), (100, 20224, 520),
+                                    (128, 384, 2056), (129, 128, 232), (250, 8192, 88), (300, 24704, 72)])
 def test_checkpoint_layout_by_workgroups(M, N, Kd):
     """eight waves and the DMA wave (one workgroup a compute unit, range cut among them) or four waves: column units of one block,
     few steps, edges of row tiles; fp32 sums of exact products, one rounding to fp16"""
