@@ -99,7 +99,10 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
     const int one = S.attn_one != 0 && M * rep <= 16;
     void *ws = one ? S.attn_one_ws : S.attn_ws;
     const size_t ws_bytes = one ? S.attn_one_ws_bytes : S.attn_ws_bytes;
-    if (S.attn_from_qkv != 0 && M <= SMH_GEMV_MAX_M && M * rep <= 128) {
+    // (Only in one launch: in two, each of the 256 prefix workgroups adds up and rotates all queries of its kv head.  Grouped queries,
+    // three layers of 64 heads over 8 kv heads: 10 branches after 2047 rows 594 us a step so, 552 with the RoPE launch in front; 3
+    // branches 523 against 511, 16 branches 629 against 571.)
+    if (S.attn_from_qkv != 0 && one && M <= SMH_GEMV_MAX_M) {
         st = smh_shared_prefix_attn_qkv(b.slab_a, ks_qkv, b.att, M, L.heads, L.kv_heads, 128, S.cos_tab, S.sin_tab, S.pos_dev, L.prompt_k, L.prompt_v,
                                         L.prompt_len, L.cache_k, L.cache_ks, L.cache_v, L.cache_vs, S.smax, S.t_dev, S.pages, S.pages_stride, one, ws,
                                         ws_bytes, stream);

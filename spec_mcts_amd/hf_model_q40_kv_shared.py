@@ -313,9 +313,12 @@ class Transformer(nn.Module):
         self.attn_single_launch = True     # up to 16 queries per kv head: prefix slices, suffix passes and the merge in one launch
                                            # (above, the one workgroup that merges a kv head's query tiles takes longer than a launch)
         self.norm_in_matmul = True         # RMSNorm made by the matmul that consumes it (a shorter launch in between) ...
-        self.norm_in_max_rows = 2          # ... up to this many rows: at 10 rows the matmul's longer prologue costs more than it saves
+        # ... up to this many rows: at 10 rows of 4096 the matmul's longer prologue costs what it saves (2.364 against 2.358 ms a step);
+        # rows of 8192 are twice the work for the one workgroup that owns a row in the other form (3 layers, 3 branches: 499 against
+        # 511 us a step, 10: 546 against 552, 16: 568 against 571)
+        self.norm_in_max_rows = 2 if params.dim < 8192 else 16
         self._norm_in_ok = {}
-        self.attn_from_qkv = True          # up to 16 branches the attention takes the wq|wk|wv product itself, in one launch
+        self.attn_from_qkv = True          # where the attention is one launch it takes the wq|wk|wv product itself
         self._q40_output = None            # quantize_lm_head(): (w, s, padded vocab) of a Q4_0 vocabulary projection
         self.paged_kv = True               # fork = a copy of page ids: forked branches share their ancestor's suffix rows
         self._page_table = None            # int32 [max_batch_size, max_seq_len]: cache row that holds position j of branch b
@@ -403,12 +406,12 @@ class Transformer(nn.Module):
             else:
                 assert seqlen == 1, "decode steps take one token per branch"
                 pos_dev, t_dev = step_state
-                if self.attn_from_qkv and M <= K.SMH_GEMV_MAX_M and M * (H // Hkv) <= 128 and not self.per_branch_kv:
+                if self.attn_from_qkv and self.attn_single_launch and M * (H // Hkv) <= 16 and not self.per_branch_kv:
                     # RoPE and the KV append happen inside the attention kernels (one launch fewer)
                     o = K.shared_prefix_attn_qkv(qkv, H, Hkv, D, cos, sin, pos_dev, att.cache_prompt_k[0], att.cache_prompt_v[0],
                                                  att.cache_prompt_len, att.cache_k, att.cache_k_s, att.cache_v, att.cache_v_s,
                                                  p.max_seq_len, t_dev,
-                                                 single_launch=self.attn_single_launch and M * (H // Hkv) <= 16,
+                                                 single_launch=True,
                                                  pages=pages).view(M, H * D)
                 else:
                     q, k, v = K.partial_rope_append_kv(qkv, H, Hkv, D, cos, sin, pos_dev, att.cache_k, att.cache_k_s,
