@@ -40,9 +40,13 @@ constexpr int GEMM_THREADS = GEMM_WAVES * 64;
 // slots of the DMA ring (with a barrier per step, four slots measured 2 % faster per launch at M=100 than six; with a
 // barrier per two steps, six slots are 3 % faster than that)
 constexpr int GEMM_STAGES = 6;
-// slots of the ring in the variant with a DMA wave (eight measured like six) and the most workgroups of a launch that
-// takes it (one per compute unit)
-constexpr int GEMM_DMA_WAVE_SLOTS = 6;
+// slots of the ring in the variant with a DMA wave, by row tiles, and the most workgroups of a launch that takes it (one per
+// compute unit).  Up to 48 rows a step is over before its successors have come from memory: with eight slots a decode step of
+// three layers of the 70B architecture takes 618 us at 17 branches against 700, 699 against 736 at 33, of the 7B architecture
+// 2.62 ms against 2.73 and 2.99 against 3.00; twelve slots as eight.  At 64 rows and more (64 x 11008 x 4096: 22.5 us against
+// 21.3) and in the kernels whose stages hold two steps (7B at 33 .. 64 branches: 1 % slower) six are better.
+constexpr int gemm_dma_slots(int tiles) { return tiles <= 3 ? 8 : 6; }
+constexpr int GEMM_PAIR_SLOTS = 6;
 constexpr int GEMM_DMA_WAVE_MAX_WGS = 256;
 constexpr int GS_WBLOCK = 8 * 128 + 64;        // the 8 rows one wave fetches, padded by 16 banks: the four row groups a
                                                // ds_read_b32 touches (lanes 16g..16g+15 read row 8g+r) then sit in different banks
@@ -65,12 +69,13 @@ __device__ __forceinline__ void gemm_wait_vm() { asm volatile("s_waitcnt vmcnt(%
 template <int PER>
 __device__ __forceinline__ void gemm_wait_dma(int stages) {
     switch (stages) {
+        case 6: gemm_wait_vm<6 * PER>(); break;
         case 5: gemm_wait_vm<5 * PER>(); break;
         case 4: gemm_wait_vm<4 * PER>(); break;
         case 3: gemm_wait_vm<3 * PER>(); break;
         case 2: gemm_wait_vm<2 * PER>(); break;
         case 1: gemm_wait_vm<1 * PER>(); break;
-        default: gemm_wait_vm<0>(); break;
+        default: gemm_wait_vm<0>(); break;              // (waits for more than asked)
     }
 }
 
@@ -609,7 +614,7 @@ template <int TILES, bool RAGGED, bool TILED, int WAVES, int SLOTS = GEMM_STAGES
 // (SWIGLU without the DMA wave: at most 128 registers, so that two workgroups of eight waves fit a compute unit)
 __global__ __launch_bounds__(64 * (WAVES + (PRODUCER ? 1 : 0)), WAVES == 8 ? (SWIGLU && !PRODUCER ? 4 : 1) : 2) void q40_gemm_kernel(MatmulParams p) {
     static_assert(WAVES == 4 || (WAVES == 8 && (TILED ? !RAGGED : PRODUCER)), "eight waves: K a multiple of 32, or the checkpoint layout with a DMA wave");
-    static_assert(SLOTS >= 6 && SLOTS <= 10 && (SLOTS == GEMM_STAGES || PRODUCER) && (!PRODUCER || WAVES == 8), "ring depth");
+    static_assert(SLOTS >= 6 && SLOTS <= 8 && (SLOTS == GEMM_STAGES || PRODUCER) && (!PRODUCER || WAVES == 8), "ring depth");
     const int steps_total = (p.K + 31) / 32;
     if constexpr (RANGE) {
         int run0 = (int)blockIdx.x * p.chunk;                  // (units x steps is far below 2^31)
@@ -654,7 +659,7 @@ constexpr int KG_W = 4096;                     // [group kk][piece bp] x 1024
 constexpr int KG_S = 512;                      // [group kk] x 256 (the whole scale block of the step)
 template <int TILES> struct KgShape {
     static constexpr int STAGE = KG_W + KG_S + 2 * TILES * 1024;
-    static constexpr int SLOTS = GEMM_DMA_WAVE_SLOTS;
+    static constexpr int SLOTS = GEMM_PAIR_SLOTS;
     static constexpr int RING = SLOTS * STAGE;
     static constexpr int PER = 2 * (3 + TILES);                    // DMA instructions of a stage
     static constexpr int OP = 128 + 4;                             // floats per row of a group's sums in LDS
@@ -860,7 +865,7 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_kg_kernel(MatmulParams p) {
 template <int TILES> struct SwigluShape {
     static constexpr int SC = 1024;                                  // scales: [group kk][gate | up] x 256
     static constexpr int STAGE = KG_W + SC + 2 * TILES * 1024;
-    static constexpr int SLOTS = GEMM_DMA_WAVE_SLOTS;
+    static constexpr int SLOTS = GEMM_PAIR_SLOTS;
     static constexpr int LDS = SLOTS * STAGE;
     static constexpr int PER = 2 * (4 + TILES);
     static constexpr int RED = 4 * TILES * 2 * 1024;
@@ -1216,17 +1221,17 @@ static int gemm_launch_layout(const MatmulParams &p, hipStream_t stream) {
     // leave every SIMD one: 100 rows x 11008 x 4096 31.9 -> 27.2 us, x 32128 61 -> 51, 20 x 28672 x 8192 66 -> 51, 160 x 28672 x
     // 4096 96 -> 64.  Where two workgroups of four waves share a compute unit, eight re-read each nibble from LDS for nothing:
     // 512 x 28672 x 8192 312-324 us against 314, 512 x 20480 x 12288 412 against 389.)
-    constexpr int WD = GEMM_TILED_WAVES, PS = GEMM_DMA_WAVE_SLOTS;
+    constexpr int WD = GEMM_TILED_WAVES;
     static const gemm_kernel_t with_dma_wave[9] = {
-        nullptr, q40_gemm_kernel<2, false, TILED, WD, PS, true>, q40_gemm_kernel<2, false, TILED, WD, PS, true>,
-        q40_gemm_kernel<3, false, TILED, WD, PS, true>, q40_gemm_kernel<4, false, TILED, WD, PS, true>,
-        q40_gemm_kernel<5, false, TILED, WD, PS, true>, q40_gemm_kernel<6, false, TILED, WD, PS, true>,
-        q40_gemm_kernel<7, false, TILED, WD, PS, true>, q40_gemm_kernel<8, false, TILED, WD, PS, true>};
+        nullptr, q40_gemm_kernel<2, false, TILED, WD, gemm_dma_slots(2), true>, q40_gemm_kernel<2, false, TILED, WD, gemm_dma_slots(2), true>,
+        q40_gemm_kernel<3, false, TILED, WD, gemm_dma_slots(3), true>, q40_gemm_kernel<4, false, TILED, WD, gemm_dma_slots(4), true>,
+        q40_gemm_kernel<5, false, TILED, WD, gemm_dma_slots(5), true>, q40_gemm_kernel<6, false, TILED, WD, gemm_dma_slots(6), true>,
+        q40_gemm_kernel<7, false, TILED, WD, gemm_dma_slots(7), true>, q40_gemm_kernel<8, false, TILED, WD, gemm_dma_slots(8), true>};
     static const gemm_kernel_t range_cut[9] = {
-        nullptr, q40_gemm_kernel<2, false, TILED, WD, PS, true, true>, q40_gemm_kernel<2, false, TILED, WD, PS, true, true>,
-        q40_gemm_kernel<3, false, TILED, WD, PS, true, true>, q40_gemm_kernel<4, false, TILED, WD, PS, true, true>,
-        q40_gemm_kernel<5, false, TILED, WD, PS, true, true>, q40_gemm_kernel<6, false, TILED, WD, PS, true, true>,
-        q40_gemm_kernel<7, false, TILED, WD, PS, true, true>, q40_gemm_kernel<8, false, TILED, WD, PS, true, true>};
+        nullptr, q40_gemm_kernel<2, false, TILED, WD, gemm_dma_slots(2), true, true>, q40_gemm_kernel<2, false, TILED, WD, gemm_dma_slots(2), true, true>,
+        q40_gemm_kernel<3, false, TILED, WD, gemm_dma_slots(3), true, true>, q40_gemm_kernel<4, false, TILED, WD, gemm_dma_slots(4), true, true>,
+        q40_gemm_kernel<5, false, TILED, WD, gemm_dma_slots(5), true, true>, q40_gemm_kernel<6, false, TILED, WD, gemm_dma_slots(6), true, true>,
+        q40_gemm_kernel<7, false, TILED, WD, gemm_dma_slots(7), true, true>, q40_gemm_kernel<8, false, TILED, WD, gemm_dma_slots(8), true, true>};
     // K not a multiple of 32: on tiled weights one kernel for all row counts, on the checkpoint layout the two forms from above with
     // a masked last step (against one four-wave kernel of eight row tiles: 33
     // rows x 11008 x 4072 29.7 -> 19.4 us, 100 rows 34.5 -> 27.6, 20 x 28672 x 8200 103 -> 53, 512 x 4096 x 4104 50 -> 40)
@@ -1235,16 +1240,16 @@ static int gemm_launch_layout(const MatmulParams &p, hipStream_t stream) {
                                                  q40_gemm_kernel<4, true, false, 4>, q40_gemm_kernel<5, true, false, 4>, q40_gemm_kernel<6, true, false, 4>,
                                                  q40_gemm_kernel<7, true, false, 4>, q40_gemm_kernel<8, true, false, 4>};
     static const gemm_kernel_t ragged_dma_wave[9] = {
-        nullptr, q40_gemm_kernel<2, true, false, WD, PS, true>, q40_gemm_kernel<2, true, false, WD, PS, true>, q40_gemm_kernel<3, true, false, WD, PS, true>,
-        q40_gemm_kernel<4, true, false, WD, PS, true>, q40_gemm_kernel<5, true, false, WD, PS, true>, q40_gemm_kernel<6, true, false, WD, PS, true>,
-        q40_gemm_kernel<7, true, false, WD, PS, true>, q40_gemm_kernel<8, true, false, WD, PS, true>};
+        nullptr, q40_gemm_kernel<2, true, false, WD, gemm_dma_slots(2), true>, q40_gemm_kernel<2, true, false, WD, gemm_dma_slots(2), true>, q40_gemm_kernel<3, true, false, WD, gemm_dma_slots(3), true>,
+        q40_gemm_kernel<4, true, false, WD, gemm_dma_slots(4), true>, q40_gemm_kernel<5, true, false, WD, gemm_dma_slots(5), true>, q40_gemm_kernel<6, true, false, WD, gemm_dma_slots(6), true>,
+        q40_gemm_kernel<7, true, false, WD, gemm_dma_slots(7), true>, q40_gemm_kernel<8, true, false, WD, gemm_dma_slots(8), true>};
     // more than 64 KB of dynamic LDS has to be allowed once per kernel (the attribute is not stream work,
     // so a launch under graph capture is not affected)
     static const hipError_t lds_ok = [] {
         hipError_t e = hipFuncSetAttribute((const void *)ragged, hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS);
         for (int t = 2; t <= 8 && e == hipSuccess; ++t) {
-            const std::pair<gemm_kernel_t, int> all[5] = {{exact[t], GEMM_LDS}, {ragged_four[t], GEMM_LDS}, {with_dma_wave[t], PS * GS_BYTES},
-                                                          {range_cut[t], PS * GS_BYTES}, {ragged_dma_wave[t], PS * GS_BYTES}};
+            const std::pair<gemm_kernel_t, int> all[5] = {{exact[t], GEMM_LDS}, {ragged_four[t], GEMM_LDS}, {with_dma_wave[t], gemm_dma_slots(t) * GS_BYTES},
+                                                          {range_cut[t], gemm_dma_slots(t) * GS_BYTES}, {ragged_dma_wave[t], gemm_dma_slots(t) * GS_BYTES}};
             for (int i = 0; i < 5 && e == hipSuccess; ++i)
                 e = hipFuncSetAttribute((const void *)all[i].first, hipFuncAttributeMaxDynamicSharedMemorySize, all[i].second);
         }
@@ -1263,7 +1268,7 @@ static int gemm_launch_layout(const MatmulParams &p, hipStream_t stream) {
                                      : (p.chunk > 0 ? range_cut : one_each ? with_dma_wave : exact)[tiles];
     const long total_steps = (long)p.units * ((p.K + 31) / 32);
     dim3 grid((unsigned)(p.chunk > 0 ? (total_steps + p.chunk - 1) / p.chunk : (long)p.units_pad * p.mblocks * p.ksplit));
-    hipLaunchKernelGGL(kern, grid, dim3(one_each ? 64 * (WD + 1) : four ? GEMM_THREADS : 64 * W), one_each ? PS * GS_BYTES : GEMM_LDS, stream, p);
+    hipLaunchKernelGGL(kern, grid, dim3(one_each ? 64 * (WD + 1) : four ? GEMM_THREADS : 64 * W), one_each ? gemm_dma_slots(tiles) * GS_BYTES : GEMM_LDS, stream, p);
     return launch_status();
 }
 
@@ -1334,16 +1339,15 @@ bool gemm_direct_fits(const MatmulParams &p) { return p.tiled && p.M > GEMM_BM &
 
 int gemm_swiglu_rows_launch(MatmulParams p, hipStream_t stream) {
     // (blocks of 64 .. 128 rows)
-    constexpr int S = GEMM_DMA_WAVE_SLOTS;
     static const gemm_kernel_t plain[5] = {q40_gemm_kernel<4, false, true, 8, GEMM_STAGES, false, false, true>, q40_gemm_kernel<5, false, true, 8, GEMM_STAGES, false, false, true>, q40_gemm_kernel<6, false, true, 8, GEMM_STAGES, false, false, true>,
                                            q40_gemm_kernel<7, false, true, 8, GEMM_STAGES, false, false, true>, q40_gemm_kernel<8, false, true, 8, GEMM_STAGES, false, false, true>};
-    static const gemm_kernel_t dma_wave[5] = {q40_gemm_kernel<4, false, true, 8, S, true, false, true>, q40_gemm_kernel<5, false, true, 8, S, true, false, true>, q40_gemm_kernel<6, false, true, 8, S, true, false, true>,
-                                              q40_gemm_kernel<7, false, true, 8, S, true, false, true>, q40_gemm_kernel<8, false, true, 8, S, true, false, true>};
+    static const gemm_kernel_t dma_wave[5] = {q40_gemm_kernel<4, false, true, 8, gemm_dma_slots(4), true, false, true>, q40_gemm_kernel<5, false, true, 8, gemm_dma_slots(5), true, false, true>, q40_gemm_kernel<6, false, true, 8, gemm_dma_slots(6), true, false, true>,
+                                              q40_gemm_kernel<7, false, true, 8, gemm_dma_slots(7), true, false, true>, q40_gemm_kernel<8, false, true, 8, gemm_dma_slots(8), true, false, true>};
     static const hipError_t lds_ok = [] {
         hipError_t e = hipSuccess;
         for (int t = 0; t < 5 && e == hipSuccess; ++t) {
             e = hipFuncSetAttribute((const void *)plain[t], hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS);
-            if (e == hipSuccess) e = hipFuncSetAttribute((const void *)dma_wave[t], hipFuncAttributeMaxDynamicSharedMemorySize, S * GS_BYTES);
+            if (e == hipSuccess) e = hipFuncSetAttribute((const void *)dma_wave[t], hipFuncAttributeMaxDynamicSharedMemorySize, gemm_dma_slots(t + 4) * GS_BYTES);
         }
         return e;
     }();
@@ -1359,7 +1363,7 @@ int gemm_swiglu_rows_launch(MatmulParams p, hipStream_t stream) {
     const bool one_each = (long)p.units * p.mblocks <= GEMM_DMA_WAVE_MAX_WGS;
     const int t = p.block_rows / 16 - 4;
     hipLaunchKernelGGL((one_each ? dma_wave : plain)[t], dim3((unsigned)((long)p.units_pad * p.mblocks)), dim3(512 + (one_each ? 64 : 0)),
-                       one_each ? S * GS_BYTES : GEMM_LDS, stream, p);
+                       one_each ? gemm_dma_slots(t + 4) * GS_BYTES : GEMM_LDS, stream, p);
     return launch_status();
 }
 
