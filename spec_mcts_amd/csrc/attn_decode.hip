@@ -1083,6 +1083,174 @@ __global__ __launch_bounds__(256, FUSED ? 1 : 4) void attn_suffix_kernel(AttnPar
     attn_suffix_body<FUSED, false, WALK>(p, b, min(h, p.H - 1), hq & (nsub - 1), nsub, h < p.H);
 }
 
+// ---- prefix slices and suffix walks side by side, then a merge ------------------------------------------------------
+// The walk waits for memory, the prefix slices for their own chain of staging and products: in one launch they overlap, and
+// what is left for the second is to add the partials up.  Workgroups 0 .. prefix_wgs - 1 take (slice, 64 queries, kv head), the
+// others walk.  Both kinds share a compute unit, so a prefix workgroup may hold no more LDS than a quarter of it: K and then
+// V^T in the same 34 KB (V waits in registers), one tile of 16 queries a wave.
+// fp16 suffixes only.  Against the prefix launch and then the walk: 100 branches x 32 heads after 512 shared rows, suffixes of up
+// to 256 rows, 65.6 -> 59.0 us a call, 64 after 1024 45.5 -> 43.6, 16 after 512 15.6 -> 14.4, one branch 12.3 either way.  A walk over
+// Q4_0 rows is a quarter of the bytes and hides less than the merge costs: decode steps of the 7B architecture at 17, 64 and 100 branches 2.59,
+// 3.30 and 4.01 ms as two launches in turn, 2.64, 3.35 and 3.96 like this.
+constexpr int AP_PITCH = ATT_TW_MAX + 8;
+__device__ __forceinline__ void attn_prefix_round(const AttnParams &p, int split, int hk, int round) {
+    static_assert(ATT_KPITCH == AP_PITCH && ATT_D == ATT_TW_MAX, "K and V^T have one shape");
+    __shared__ __attribute__((aligned(16))) half_t kv_lds[ATT_D][AP_PITCH];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
+    const int t0 = split * p.tw, cnt = min(p.tw, p.P - t0), tw32 = (cnt + 31) & ~31, t_tiles = tw32 / 16;
+    const int qt = 4 * round + wave;
+    const bool live = qt * 16 < p.Bq;                        // (uniform over the wave)
+    h8 qb[4];
+    {
+        const int qr = min(qt * 16 + c, p.Bq - 1);
+        const half_t *qp = p.q + ((long)div_rep(p, qr) * p.H + hk * p.n_rep + mod_rep(p, qr)) * ATT_D + 8 * g;
+#pragma unroll
+        for (int k4 = 0; k4 < 4; ++k4) qb[k4] = *reinterpret_cast<const h8 *>(qp + 32 * k4);
+    }
+    const int ch = tid & 15;
+    u32x4 kr[2][4], vr[2][4];                                // this thread's 8 dims of rows 4 kg .. 4 kg + 3, kg = tid / 16 and 16 more
+    auto fetch = [&](const half_t *base, u32x4 (&r)[2][4]) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int t = 4 * ((tid >> 4) + 16 * i) + e;
+                r[i][e] = u32x4{0, 0, 0, 0};
+                if (t < cnt) r[i][e] = *reinterpret_cast<const u32x4 *>(base + (long)(t0 + t) * p.pfx_row_stride + (long)hk * p.pfx_head_stride + ch * 8);
+            }
+    };
+    fetch(p.prefix_k, kr);
+    fetch(p.prefix_v, vr);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int t = 4 * ((tid >> 4) + 16 * i) + e;
+            if (t < tw32) *reinterpret_cast<u32x4 *>(&kv_lds[t][ch * 8]) = kr[i][e];
+        }
+    __syncthreads();
+    f4 st[ATT_TW_MAX / 16];                                  // S^T: element r of st[j] is row 16 j + 4 g + r, column (query) c
+    float mx = -INFINITY, sum = 0.f;
+    if (live) {
+#pragma unroll
+        for (int j = 0; j < ATT_TW_MAX / 16; ++j) {
+            st[j] = f4{0.f, 0.f, 0.f, 0.f};
+            if (j < t_tiles) {
+#pragma unroll
+                for (int k4 = 0; k4 < 4; ++k4)
+                    st[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const h8 *>(&kv_lds[16 * j + c][32 * k4 + 8 * g]), qb[k4], st[j], 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    st[j][r] = 16 * j + 4 * g + r < cnt ? st[j][r] * p.scale_log2 : -INFINITY;
+                    mx = fmaxf(mx, st[j][r]);
+                }
+            }
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+#pragma unroll
+        for (int j = 0; j < ATT_TW_MAX / 16; ++j)
+            if (j < t_tiles) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    st[j][r] = exp2f(st[j][r] - mx);         // masked rows: exp2(-inf) = 0
+                    sum += st[j][r];
+                }
+            }
+        sum += __shfl_xor(sum, 16, 64);
+        sum += __shfl_xor(sum, 32, 64);
+    }
+    __syncthreads();                                         // every wave has read K
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int kg = (tid >> 4) + 16 * i;
+        if (4 * kg < tw32) {
+            const int pos = vt_pos(4 * kg);
+            const h8 v0 = __builtin_bit_cast(h8, vr[i][0]), v1 = __builtin_bit_cast(h8, vr[i][1]);
+            const h8 v2 = __builtin_bit_cast(h8, vr[i][2]), v3 = __builtin_bit_cast(h8, vr[i][3]);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) *reinterpret_cast<h4 *>(&kv_lds[ch * 8 + j][pos]) = h4{v0[j], v1[j], v2[j], v3[j]};
+        }
+    }
+    __syncthreads();
+    if (!live) return;
+    f4 ot[8];                                                // O^T: element r of ot[dt] is dim 16 dt + 4 g + r, column (query) c
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt) ot[dt] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int jj = 0; jj < ATT_TW_MAX / 32; ++jj)
+        if (2 * jj < t_tiles) {
+            h8 pb;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                pb[r] = (half_t)st[2 * jj][r];
+                pb[4 + r] = (half_t)st[2 * jj + 1][r];
+            }
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt)
+                ot[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const h8 *>(&kv_lds[16 * dt + c][32 * jj + 8 * g]), pb, ot[dt], 0, 0, 0);
+        }
+    const int qrow = qt * 16 + c;
+    if (qrow >= p.Bq) return;
+    const long base = ((long)split * p.Hkv + hk) * p.Bq + qrow;
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt) *reinterpret_cast<f4 *>(p.part_o + base * ATT_D + 16 * dt + 4 * g) = ot[dt];
+    if (g == 0) { p.part_ml[base * 2] = mx; p.part_ml[base * 2 + 1] = sum; }
+}
+
+// prefix_wgs: a multiple of 8, so that the others sit on the XCDs that attn_suffix_kernel's would
+__global__ __launch_bounds__(256, 4) void attn_parts_kernel(AttnParams p, int prefix_wgs, int rounds) {
+    int L = blockIdx.x;
+    if (L < prefix_wgs) {
+        const int hk = L % p.Hkv, rest = L / p.Hkv, split = rest / rounds;
+        if (split < p.splits) attn_prefix_round(p, split, hk, rest - split * rounds);
+        return;
+    }
+    L -= prefix_wgs;
+    const int wave = threadIdx.x >> 6, nsub = p.suffix_waves, per_branch = (p.H * nsub + 3) >> 2, j = L >> 3, grp = j / per_branch, b = 8 * grp + (L & 7);
+    if (b >= p.B) return;
+    const int hq = (j - grp * per_branch) * 4 + wave, h = nsub == 4 ? hq >> 2 : (nsub == 2 ? hq >> 1 : hq);
+    if (nsub == 1 && h >= p.H) return;
+    attn_suffix_body<false, true, WALK_F16>(p, b, min(h, p.H - 1), hq & (nsub - 1), nsub, h < p.H);
+}
+
+// One wave per query adds its splits + 1 partials up, in split order: lane d holds dims 2 d, 2 d + 1.
+__global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p) {
+    const int qi = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;       // kv head * Bq + query of the kv head
+    const int queries = p.Hkv * p.Bq;
+    if (qi >= queries) return;
+    float m = -INFINITY, l = 0.f;
+    f2 o = {0.f, 0.f};
+    constexpr int N = 8;                                     // partials on their way at a time
+    for (int s0 = 0; s0 <= p.splits; s0 += N) {
+        f2 v[N], ml[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            ml[i] = f2{-INFINITY, 0.f};
+            v[i] = f2{0.f, 0.f};
+            if (s0 + i <= p.splits) {
+                const long base = (long)(s0 + i) * queries + qi;
+                ml[i] = *reinterpret_cast<const f2 *>(p.part_ml + base * 2);
+                v[i] = *reinterpret_cast<const f2 *>(p.part_o + base * ATT_D + 2 * lane);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const float m_new = fmaxf(m, ml[i][0]);
+            if (m_new == -INFINITY) continue;                // nothing yet
+            const float c1 = exp2f(m - m_new), c2 = exp2f(ml[i][0] - m_new);
+            m = m_new;
+            l = l * c1 + ml[i][1] * c2;
+            o[0] = o[0] * c1 + v[i][0] * c2;
+            o[1] = o[1] * c1 + v[i][1] * c2;
+        }
+    }
+    const int hk = qi / p.Bq, qrow = qi - hk * p.Bq;
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    half_t *op = p.out + ((long)div_rep(p, qrow) * p.H + hk * p.n_rep + mod_rep(p, qrow)) * ATT_D + 2 * lane;
+    *reinterpret_cast<h2 *>(op) = h2{(half_t)(o[0] * inv), (half_t)(o[1] * inv)};
+}
+
 // ---- the whole decode attention in ONE launch -----------------------------------------------------------------
 // grid (splits + ceil(Bq / per_wg), kv heads): workgroups x < splits take a slice of the prefix, the others the suffix
 // + new token of per_wg = 1, 2 or 4 of the kv head's Bq = B x n_rep queries (4, 2 or 1 waves per query: with few
@@ -1269,7 +1437,7 @@ static size_t attn_tiles_bytes(int B, int H, int Hkv, int cols) {
 
 extern "C" size_t smh_attn_workspace_bytes(int B, int H, int P) {
     if (P <= 0 || B <= 0 || H <= 0) return 256;
-    size_t splits = (size_t)(P + 31) / 32;          // worst case: 32 rows per workgroup
+    size_t splits = (size_t)(P + 31) / 32 + 1;      // worst case: 32 rows per workgroup; the suffix's partial
     return splits * (size_t)B * (size_t)H * (smh::ATT_D + 2) * sizeof(float) + 256;
 }
 
@@ -1348,12 +1516,22 @@ static int shared_prefix_attn(const char *who, bool one, const void *q, void *ou
                 "%s: workspace %zu < %zu bytes", who, workspace_bytes, n_part * (ATT_D + 2) * sizeof(float));
     p.part_o = (float *)workspace;
     p.part_ml = p.part_o + n_part * ATT_D;
+    p.suffix_waves = attn_plan_suffix_waves_two((long)B * H);
+    const unsigned wgs = (unsigned)(((H * p.suffix_waves + 3) / 4) * ((B + 7) / 8 * 8));
+    const size_t n_parts = (size_t)(p.splits + 1) * Hkv * p.Bq;
+    const int rounds = ((p.Bq + 15) / 16 + 3) / 4;
+    const long prefix_wgs = ((long)p.splits * Hkv * rounds + 7) / 8 * 8;
+    if (p.splits > 0 && suffix_format == SMH_KV_FP16 && workspace_bytes >= n_parts * (ATT_D + 2) * sizeof(float) && prefix_wgs + wgs < (1L << 31)) {
+        p.part_ml = p.part_o + n_parts * ATT_D;
+        const dim3 grid((unsigned)(prefix_wgs + wgs));
+        hipLaunchKernelGGL(attn_parts_kernel, grid, dim3(256), 0, (hipStream_t)stream, p, (int)prefix_wgs, rounds);
+        hipLaunchKernelGGL(attn_merge_kernel, dim3((unsigned)(((long)Hkv * p.Bq + 3) / 4)), dim3(256), 0, (hipStream_t)stream, p);
+        return launch_status();
+    }
     if (p.splits > 0)
         hipLaunchKernelGGL(attn_prefix_kernel<false>, dim3(p.splits, Hkv, qgroups), dim3(256), 0, (hipStream_t)stream, p);
-    p.suffix_waves = attn_plan_suffix_waves_two((long)B * H);
     const bool fp16_pages = p.pages != nullptr && suffix_format == SMH_KV_FP16;
     const size_t tile_bytes = fp16_pages && P == 0 && lens == nullptr ? attn_tiles_bytes(B, H, Hkv, Smax) : 0;
-    const unsigned wgs = (unsigned)(((H * p.suffix_waves + 3) / 4) * ((B + 7) / 8 * 8));
     if (tile_bytes > 0 && workspace && workspace_bytes >= tile_bytes) {
         const int tiles = (p.Bq + 15) / 16;
         p.splits = (Smax + PT_TW - 1) / PT_TW;

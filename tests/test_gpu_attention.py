@@ -266,3 +266,34 @@ def test_one_launch_attention_matches_two_launches(B, H, Hkv, P, L):
         got = K.shared_prefix_attn(q, pk if P else None, pv if P else None, P, single_launch=True, **kw)
         torch.cuda.synchronize()
         assert torch.allclose(got.float(), want.float(), rtol=2e-3, atol=2e-3), f"call {rep}: {float((got.float() - want.float()).abs().max())}"
+
+
+@pytest.mark.parametrize("B,H,Hkv,P,S", [(1, 8, 8, 1, 5), (15, 8, 8, 31, 17), (16, 3, 3, 33, 64), (17, 16, 2, 127, 3), (65, 8, 8, 128, 33), (33, 16, 8, 129, 40),
+                                         (5, 32, 32, 1000, 12), (130, 8, 1, 300, 16)])
+@pytest.mark.parametrize("current", [False, True])
+def test_fp16_suffix_beside_the_prefix_slices(B, H, Hkv, P, S, current):
+    """slices and walks in one launch, then the merge: edges of slices (32 .. 128 rows) and of query tiles, grouped queries,
+    branches without rows of their own; the workspace of the older size takes the prefix launch and then the walk"""
+    from spec_mcts_amd import _lib, kernels as K
+    g = torch.Generator().manual_seed(B + P)
+    r = lambda *s: torch.randn(s, generator=g).half()
+    q, pk, pv, sk, sv, ck, cv = r(B, H, 128), r(P, Hkv, 128), r(P, Hkv, 128), r(B, S, Hkv, 128), r(B, S, Hkv, 128), r(B, Hkv, 128), r(B, Hkv, 128)
+    lens = torch.randint(0, S + 1, (B,), generator=g, dtype=torch.int32)
+    lens[0] = 0
+    want = torch.empty((B, H, 128), dtype=torch.float64)
+    for b in range(B):
+        parts = [(pk, pv), (sk[b, :lens[b]], sv[b, :lens[b]])] + ([(ck[b:b + 1], cv[b:b + 1])] if current else [])
+        k, v = (torch.cat([x[i] for x in parts]).double().repeat_interleave(H // Hkv, 1) for i in range(2))
+        p = torch.softmax(torch.einsum("hd,thd->ht", q[b].double(), k) / 128 ** 0.5, 1)
+        want[b] = torch.einsum("ht,thd->hd", p, v)
+    d = [t.cuda() for t in (q, pk, pv, sk, sv, lens, ck, cv)]
+    kw = dict(suffix_k=d[3], suffix_v=d[4], Smax=S, lens=d[5], lens_stride=1, **(dict(cur_k=d[6], cur_v=d[7]) if current else {}))
+    got = K.shared_prefix_attn(d[0], d[1], d[2], P, **kw).cpu().double()
+    tol = 2e-3 + 1e-2 * want.abs()                       # the bound of the other attention tests: fp16 probabilities of the prefix, fp16 output
+    assert bool(((got - want).abs() <= tol).all())
+    lib, splits = _lib.load(), -(-P // 32)
+    ws, out = torch.empty(splits * B * H * 130 * 4, dtype=torch.uint8, device="cuda"), torch.empty_like(d[0])
+    K.check(lib.smh_shared_prefix_attn(d[0].data_ptr(), out.data_ptr(), B, H, Hkv, 128, d[1].data_ptr(), d[2].data_ptr(), P, K.SMH_KV_FP16, d[3].data_ptr(),
+                                       d[4].data_ptr(), None, None, S, d[5].data_ptr(), 1, d[6].data_ptr() if current else None,
+                                       d[7].data_ptr() if current else None, ws.data_ptr(), ws.numel(), K._stream()), "smh_shared_prefix_attn")
+    assert bool(((out.cpu().double() - want).abs() <= tol).all())
