@@ -99,7 +99,7 @@ std::vector<int64_t> shape_of(PyObject *o) {
 bool is(const at::Tensor &t, at::ScalarType s) { return t.scalar_type() == s; }
 at::Tensor empty(at::IntArrayRef shape, at::ScalarType s, const at::Tensor &like) { return at::empty(shape, at::TensorOptions().dtype(s).device(like.device())); }
 smh_stream_t stream() { return (smh_stream_t)c10::hip::getCurrentHIPStream().stream(); }
-const void *ptr(PyObject *o) { return none(o) ? nullptr : THPVariable_Unpack(o).data_ptr(); }
+const void *ptr(PyObject *o) { return none(o) ? nullptr : gpu(o, "an optional argument").data_ptr(); }
 PyObject *give(const at::Tensor &t) { return THPVariable_Wrap(t); }
 void arity(Py_ssize_t n, Py_ssize_t want) {
     if (n != want) {
