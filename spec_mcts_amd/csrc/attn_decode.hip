@@ -12,6 +12,8 @@
 //  2. attn_suffix_kernel, one wave per (branch, query head): streams the branch's own suffix rows
 //     (HBM-bound; Q4_0 rows are decoded in registers), keeps an online softmax per 16-lane group,
 //     folds in the prefix partials and the new token, normalises and writes fp16.
+// With fp16 suffixes the slices and the walks are one launch and a merge follows (attn_parts_kernel); fp16 pages that neighbouring
+// branches share go through attn_page_tile_kernel before the walk.
 // Scores and softmax are fp32 throughout (exp2 of log2(e)-scaled scores); probabilities are rounded
 // to fp16 only as the operand of the P.V matrix product.
 //

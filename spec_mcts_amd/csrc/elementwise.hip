@@ -237,8 +237,8 @@ namespace smh {
 
 // ---- temperature / top-k sampling -----------------------------------------------------------------------------
 // One 1024-thread workgroup per row.  x = fp16(logit / temperature) (the reference divides fp16 tensors); the k largest
-// x, equal values taken lowest index first, are found with a two-pass radix select on an order-preserving 16-bit key
-// (256-bin histograms in LDS), gathered, ordered by (x descending, index ascending) with a rank sort, turned into
+// x, equal values taken lowest index first, are found by the threads' maxima (k above 512 and rows of mostly equal logits: with a
+// two-pass radix select, 256-bin histograms in LDS) on an order-preserving 16-bit key, gathered, ordered by (x descending, index ascending) with a rank sort, turned into
 // probabilities p = fp16(softmax) as F.softmax on an fp16 tensor returns them, and one candidate is drawn by inverse
 // CDF with the caller's uniform number.
 constexpr int SAMPLE_MAX_K = 1024;
