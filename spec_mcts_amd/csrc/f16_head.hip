@@ -199,41 +199,48 @@ __global__ __launch_bounds__(HEAD_WAVES * 64) void f16_head_kernel(HeadParams p)
 // way while one is multiplied, one barrier a stage.  Blocks of outputs are dealt to the XCDs (grid x is a multiple of 8), so
 // that an XCD's L2 sees an eighth of W, whatever the row block.
 // 32016 outputs of 4096 values, against blocks of 128 x 128: 2047 rows 873 -> 563 us (954 TFLOP/s), 1100 rows 496 -> 373, 512 rows
-// 251 -> 152, 257 rows 192 -> 147; of 8192 values, 2047 rows 1994 -> 1100.  With 256 rows or fewer half of the compute units would be idle.
+// 251 -> 152, 257 rows 192 -> 147; of 8192 values, 2047 rows 1994 -> 1100.  With 129 .. 256 rows such blocks would leave half of the compute
+// units idle: blocks of 256 x 128 there, 256 rows 124 -> 91 us, 129 rows 127 -> 85.
 constexpr int HEAD_ROWS = 256;
-constexpr int HEAD_ROWS_STAGE = 2 * HEAD_ROWS * 128;
+constexpr int head_rows_stage(int xb) { return (HEAD_ROWS + 64 * xb) * 128; }
 constexpr int HEAD_ROWS_LEAST_WGS = 192;
 typedef float f16v __attribute__((ext_vector_type(16)));
+template <int XB>                                            // 32-row tiles of x a wave: 4, or 2 (blocks of 128 rows, for 129 .. 256)
 __global__ __launch_bounds__(512, 2) void f16_head_rows_kernel(HeadParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    const int n0 = blockIdx.x * HEAD_ROWS, m0 = blockIdx.y * HEAD_ROWS;
+    const int n0 = blockIdx.x * HEAD_ROWS, m0 = blockIdx.y * (64 * XB);
     if (n0 >= p.N) return;                                   // (the padding of grid x)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, c = lane & 31, hi = lane >> 5;
-    const int wn = 64 * (wave & 3), wm = 128 * (wave >> 2);  // this wave's outputs and rows inside the block
-    // DMA: eight instructions a wave and stage, 8 rows of 128 bytes each: four of W, four of x; rows past the end repeat the last one
+    const int wn = 64 * (wave & 3), wm = 32 * XB * (wave >> 2);  // this wave's outputs and rows inside the block
+    // DMA: 4 + XB instructions a wave and stage, 8 rows of 128 bytes each: four of W, XB of x; rows past the end repeat the last one
     const int d_r = lane >> 3, d_q = lane & 7;
-    uint32_t w_off[4], x_off[4];
+    uint32_t w_off[4], x_off[XB];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int rr = 32 * wave + 8 * i + d_r, chunk = 8 * (d_q ^ ((rr >> 1) & 7));
-        w_off[i] = (uint32_t)(((long)(min(n0 + rr, p.N - 1) - n0) * p.K + chunk) * 2);
-        x_off[i] = (uint32_t)(((long)min(m0 + rr, p.M - 1) * p.ldx + chunk) * 2);
+        const int rr = 32 * wave + 8 * i + d_r;
+        w_off[i] = (uint32_t)(((long)(min(n0 + rr, p.N - 1) - n0) * p.K + 8 * (d_q ^ ((rr >> 1) & 7))) * 2);
+    }
+#pragma unroll
+    for (int i = 0; i < XB; ++i) {
+        const int rr = 8 * XB * wave + 8 * i + d_r;
+        x_off[i] = (uint32_t)(((long)min(m0 + rr, p.M - 1) * p.ldx + 8 * (d_q ^ ((rr >> 1) & 7))) * 2);
     }
     const uint8_t *w_base = reinterpret_cast<const uint8_t *>(p.w + (long)n0 * p.K), *x_base = reinterpret_cast<const uint8_t *>(p.x);
     auto issue = [&](int stage, int slot) {
-        uint8_t *st = lds + slot * HEAD_ROWS_STAGE + 32 * wave * 128;
+        uint8_t *st = lds + slot * head_rows_stage(XB);
         const long kb = (long)stage * HEAD_KS * 2;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            __builtin_amdgcn_global_load_lds((gptr_t)(w_base + kb + w_off[i]), (lptr_t)(st + i * 1024), 16, 0, 0);
-            __builtin_amdgcn_global_load_lds((gptr_t)(x_base + kb + x_off[i]), (lptr_t)(st + HEAD_ROWS * 128 + i * 1024), 16, 0, 0);
-        }
+        for (int i = 0; i < 4; ++i)
+            __builtin_amdgcn_global_load_lds((gptr_t)(w_base + kb + w_off[i]), (lptr_t)(st + (4 * wave + i) * 1024), 16, 0, 0);
+#pragma unroll
+        for (int i = 0; i < XB; ++i)
+            __builtin_amdgcn_global_load_lds((gptr_t)(x_base + kb + x_off[i]), (lptr_t)(st + HEAD_ROWS * 128 + (XB * wave + i) * 1024), 16, 0, 0);
     };
-    f16v acc[2][4];                                          // element r of acc[a][b], lane (hi, c): output wn + 32 a + 8 (r / 4) + 4 hi + r % 4 of row wm + 32 b + c
+    f16v acc[2][XB];                                         // element r of acc[a][b], lane (hi, c): output wn + 32 a + 8 (r / 4) + 4 hi + r % 4 of row wm + 32 b + c
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
+        for (int b = 0; b < XB; ++b)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
     const int n_stages = p.K / HEAD_KS;
@@ -243,28 +250,28 @@ __global__ __launch_bounds__(512, 2) void f16_head_rows_kernel(HeadParams p) {
         head_wait_dma<0>();                                              // stage i of this wave has landed ...
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); // ... and everyone's; everyone is done with stage i - 1
         if (i + 1 < n_stages) issue(i + 1, (i + 1) & 1);
-        const uint8_t *st = lds + (i & 1) * HEAD_ROWS_STAGE;
+        const uint8_t *st = lds + (i & 1) * head_rows_stage(XB);
 #pragma unroll
         for (int k = 0; k < HEAD_KS / 16; ++k) {
-            h8 wa[2], xb[4];
+            h8 wa[2], xb[XB];
 #pragma unroll
             for (int a = 0; a < 2; ++a) {
                 const int rr = wn + 32 * a + c;
                 wa[a] = *reinterpret_cast<const h8 *>(st + rr * 128 + (((2 * k + hi) ^ ((rr >> 1) & 7)) << 4));
             }
 #pragma unroll
-            for (int b = 0; b < 4; ++b) {
+            for (int b = 0; b < XB; ++b) {
                 const int rr = wm + 32 * b + c;
                 xb[b] = *reinterpret_cast<const h8 *>(st + HEAD_ROWS * 128 + rr * 128 + (((2 * k + hi) ^ ((rr >> 1) & 7)) << 4));
             }
 #pragma unroll
-            for (int b = 0; b < 4; ++b)
+            for (int b = 0; b < XB; ++b)
 #pragma unroll
                 for (int a = 0; a < 2; ++a) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wa[a], xb[b], acc[a][b], 0, 0, 0);
         }
     }
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
+    for (int b = 0; b < XB; ++b) {
         const int m = m0 + wm + 32 * b + c;
         if (m >= p.M) continue;
 #pragma unroll
@@ -314,7 +321,8 @@ extern "C" int smh_f16_linear(const void *x, int M, int K, long ldx, const void 
                                           f16_head_kernel<5>, f16_head_kernel<6>, f16_head_kernel<7>, f16_head_kernel<8>};
     // more than 64 KB of dynamic LDS has to be allowed once per kernel (not stream work: fine under graph capture)
     static const hipError_t lds_ok = [] {
-        hipError_t e = hipFuncSetAttribute((const void *)f16_head_rows_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * HEAD_ROWS_STAGE);
+        hipError_t e = hipFuncSetAttribute((const void *)f16_head_rows_kernel<4>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * head_rows_stage(4));
+        if (e == hipSuccess) e = hipFuncSetAttribute((const void *)f16_head_rows_kernel<2>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * head_rows_stage(2));
         for (int t = 1; t <= 8 && e == hipSuccess; ++t)
             e = hipFuncSetAttribute((const void *)kern[t], hipFuncAttributeMaxDynamicSharedMemorySize, head_stages(t) * (HEAD_W_BYTES + t * 16 * 128));
         return e;
@@ -324,11 +332,12 @@ extern "C" int smh_f16_linear(const void *x, int M, int K, long ldx, const void 
     p.x = (const half_t *)x; p.w = (const half_t *)w; p.out = (half_t *)out;
     p.ldx = ldx; p.ldo = ldo; p.M = M; p.N = N; p.K = K;
     p.vec_store = (ldo % 4 == 0) && (((uintptr_t)out & 7) == 0);
-    // more than two row blocks of the other kernel, and workgroups for most of the compute units
-    const long row_wgs = (long)((N + HEAD_ROWS - 1) / HEAD_ROWS) * ((M + HEAD_ROWS - 1) / HEAD_ROWS);
-    if (M > 2 * HEAD_BM && row_wgs >= HEAD_ROWS_LEAST_WGS && (long)HEAD_ROWS * K * 2 < (1L << 32)) {
-        const dim3 blocks((unsigned)((N + HEAD_ROWS - 1) / HEAD_ROWS + 7) / 8 * 8, (unsigned)((M + HEAD_ROWS - 1) / HEAD_ROWS));
-        hipLaunchKernelGGL(f16_head_rows_kernel, blocks, dim3(512), 2 * HEAD_ROWS_STAGE, (hipStream_t)stream, p);
+    // more rows than the other kernel's workgroup holds, and workgroups for most of the compute units
+    const int xb = M > HEAD_ROWS ? 4 : 2;
+    const long n_blocks = (N + HEAD_ROWS - 1) / HEAD_ROWS, m_blocks = (M + 64 * xb - 1) / (64 * xb);
+    if (M > HEAD_BM && n_blocks * m_blocks >= HEAD_ROWS_LEAST_WGS && (long)HEAD_ROWS * K * 2 < (1L << 32)) {
+        hipLaunchKernelGGL(xb == 4 ? f16_head_rows_kernel<4> : f16_head_rows_kernel<2>, dim3((unsigned)((n_blocks + 7) / 8 * 8), (unsigned)m_blocks), dim3(512),
+                           2 * head_rows_stage(xb), (hipStream_t)stream, p);
         return launch_status();
     }
     const int tiles = M >= HEAD_BM ? 8 : (M + 15) / 16;

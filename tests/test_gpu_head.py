@@ -35,7 +35,7 @@ def test_lm_head_at_vocab_32016(M):
 
 @pytest.mark.parametrize("M,N,K", [(1, 1, 64), (3, 320, 256), (16, 127, 128), (17, 129, 192), (130, 384, 512), (257, 200, 64), (5, 8192, 8192),
                                    # blocks of 256 outputs x 256 rows: one stage, edges of blocks, an odd number of outputs (no 8-byte stores)
-                                   (257, 24575, 64), (300, 32016, 128), (520, 24577, 192), (1024, 12288, 64)])
+                                   (129, 24831, 64), (192, 32016, 128), (256, 24577, 192), (257, 24575, 64), (300, 32016, 128), (520, 24577, 192), (1024, 12288, 64)])
 def test_lm_head_ragged_shapes(M, N, K):
     _check(M, N, K, 600 + M + N)
 
