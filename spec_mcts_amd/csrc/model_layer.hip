@@ -19,6 +19,9 @@ struct LayerBuffers {
 };
 
 static int slices(int M, int K, int nseg, const int *n) { return smh_q40_matmul_plan_tiled(M, K, nseg, n); }
+// A launch that stores its fp16 results itself (more than 128 rows, no K-split) leaves no slabs.  layer_buffers reserves none for it,
+// so every linear below asks here before it takes the slab form.
+static bool direct(int M, int K, int nseg, const int *n) { return smh_q40_matmul_tiled_direct_fits(M, K, nseg, n) == 1; }
 
 static int layer_buffers(const smh_layer &L, int M, bool swiglu_in, char *base, LayerBuffers &b) {
     const int nq = L.heads * 128, nkv = L.kv_heads * 128;
@@ -27,10 +30,8 @@ static int layer_buffers(const smh_layer &L, int M, bool swiglu_in, char *base, 
     if (ks_qkv < 1 || ks_gu < 1 || ks_o < 1 || ks_d < 1) return -1;
     const size_t m = (size_t)M;
     auto most = [](size_t x, size_t y) { return x > y ? x : y; };
-    // (a prefill's launches that store fp16 themselves leave no slabs)
     const bool gu_slabs = !(M > 128 && swiglu_in && smh_q40_swiglu_fits(M, L.dim, L.ffn));
-    const bool qkv_slabs = smh_q40_matmul_tiled_direct_fits(M, L.dim, 3, n_qkv) != 1, o_slabs = smh_q40_matmul_tiled_direct_fits(M, nq, 1, n_dim) != 1;
-    const bool d_slabs = smh_q40_matmul_tiled_direct_fits(M, L.ffn, 1, n_dim) != 1;
+    const bool qkv_slabs = !direct(M, L.dim, 3, n_qkv), o_slabs = !direct(M, nq, 1, n_dim), d_slabs = !direct(M, L.ffn, 1, n_dim);
     b.slab_a_bytes = align_up(most(qkv_slabs ? ks_qkv * m * (nq + 2 * (size_t)nkv) : 1, gu_slabs ? ks_gu * m * 2 * (size_t)L.ffn : 1) * sizeof(float));
     b.slab_b_bytes = align_up((size_t)most(o_slabs ? ks_o : 0, d_slabs ? ks_d : 0) * m * L.dim * sizeof(float));
     size_t at = 0;
@@ -50,6 +51,46 @@ static int layer_buffers(const smh_layer &L, int M, bool swiglu_in, char *base, 
     return 0;
 }
 
+// What a decode layer and a prefill layer share: the arguments checked, the buffers, and the residual stream on its way through them.
+struct LayerRun {
+    const smh_layer &L;
+    smh_pass &S;
+    smh_stream_t stream;
+    const int M, nq, nkv;
+    const int n_qkv[3], n_gu[2], n_dim[1];
+    const void *w_qkv[3], *w_o[1], *w_gu[2], *w_d[1];
+    LayerBuffers b;
+
+    LayerRun(const smh_layer &l, smh_pass &s, smh_stream_t st)
+        : L(l), S(s), stream(st), M(s.rows), nq(l.heads * 128), nkv(l.kv_heads * 128), n_qkv{nq, nkv, nkv}, n_gu{l.ffn, l.ffn}, n_dim{l.dim},
+          w_qkv{l.wq, l.wk, l.wv}, w_o{l.wo}, w_gu{l.w1, l.w3}, w_d{l.w2} {}
+    int begin(const char *who) {
+        SMH_REQUIRE(M >= 1 && L.heads > 0 && L.kv_heads > 0 && L.heads % L.kv_heads == 0, "%s: rows=%d heads=%d kv_heads=%d", who, M, L.heads, L.kv_heads);
+        if (layer_buffers(L, M, S.swiglu_in != 0, (char *)S.scratch, b) != 0) return -1;
+        SMH_REQUIRE(S.scratch && S.scratch_bytes >= b.total, "%s: scratch %zu < %zu bytes", who, S.scratch_bytes, b.total);
+        return 0;
+    }
+    // S.h += the product of the linear before (S.pending slabs in slab_b), then its RMSNorm: to b.xn
+    int norm(const void *weight, float eps) {
+        void *h_out = S.pending > 0 ? b.h[S.h == b.h[0]] : nullptr;
+        const int r = smh_partial_rmsnorm(S.pending > 0 ? b.slab_b : nullptr, S.pending > 0 ? S.pending : 1, M, L.dim, S.h, weight, eps, h_out, b.xn, stream);
+        if (h_out != nullptr) S.h = h_out;
+        S.pending = 0;
+        return r;
+    }
+    // S.h += x . w, at once or as slabs that the next norm adds
+    int residual_linear(const void *x, int K, const void *const *w) {
+        if (direct(M, K, 1, n_dim)) {
+            void *out[1] = {b.h[S.h == b.h[0]]};
+            const int r = smh_q40_matmul_tiled_direct(x, M, K, K, 1, w, n_dim, out, S.h, L.dim, stream);
+            S.h = out[0];
+            return r;
+        }
+        S.pending = slices(M, K, 1, n_dim);
+        return smh_q40_matmul_partial_tiled(x, M, K, K, 1, w, n_dim, b.slab_b, b.slab_b_bytes, stream);
+    }
+};
+
 }  // namespace smh
 
 using namespace smh;
@@ -63,28 +104,17 @@ extern "C" size_t smh_decode_scratch_bytes(const smh_layer *layer, int rows, int
 extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stream_t stream) {
     const char *who = "smh_decode_layer";
     SMH_REQUIRE(layer && pass && pass->h, "%s: null pointer", who);
+    LayerRun run(*layer, *pass, stream);
+    int st = run.begin(who);
+    if (st) return st;
     const smh_layer &L = *layer;
     smh_pass &S = *pass;
-    const int M = S.rows, nq = L.heads * 128, nkv = L.kv_heads * 128;
-    SMH_REQUIRE(M >= 1 && L.heads > 0 && L.kv_heads > 0 && L.heads % L.kv_heads == 0, "%s: rows=%d heads=%d kv_heads=%d", who, M, L.heads, L.kv_heads);
-    LayerBuffers b;
-    if (layer_buffers(L, M, S.swiglu_in != 0, (char *)S.scratch, b) != 0) return -1;
-    SMH_REQUIRE(S.scratch && S.scratch_bytes >= b.total, "%s: scratch %zu < %zu bytes", who, S.scratch_bytes, b.total);
-    const int n_qkv[3] = {nq, nkv, nkv}, n_gu[2] = {L.ffn, L.ffn}, n_dim[1] = {L.dim};
-    const void *w_qkv[3] = {L.wq, L.wk, L.wv}, *w_o[1] = {L.wo}, *w_gu[2] = {L.w1, L.w3}, *w_d[1] = {L.w2};
-    int st = 0;
-    // S.h += the product of the linear before (S.pending slabs in slab_b), then its RMSNorm: to b.xn
-    auto norm = [&](const void *weight, float eps) -> int {
-        void *h_out = S.pending > 0 ? b.h[S.h == b.h[0]] : nullptr;
-        const int r = smh_partial_rmsnorm(S.pending > 0 ? b.slab_b : nullptr, S.pending > 0 ? S.pending : 1, M, L.dim, S.h, weight, eps, h_out, b.xn, stream);
-        if (h_out != nullptr) S.h = h_out;
-        S.pending = 0;
-        return r;
-    };
-    // ... and the linears behind it: to slab_a.  With few rows the RMSNorm is made inside the linears' launch.
+    const LayerBuffers &b = run.b;
+    const int M = run.M, nq = run.nq;
+    // the RMSNorm of the residual stream and the linears behind it: to slab_a.  With few rows the RMSNorm is made inside the linears' launch.
     auto norm_linears = [&](const void *weight, float eps, int nseg, const void *const *w, const int *n) -> int {
         if (S.pending == 0 || M > S.norm_in_rows || smh_q40_norm_in_fits(M, L.dim, nseg, n) != 1) {
-            if (int r = norm(weight, eps)) return r;
+            if (int r = run.norm(weight, eps)) return r;
             return smh_q40_matmul_partial_tiled(b.xn, M, L.dim, L.dim, nseg, w, n, b.slab_a, b.slab_a_bytes, stream);
         }
         void *h_out = b.h[S.h == b.h[0]];
@@ -94,11 +124,20 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
         return smh_q40_matmul_partial_tiled_norm(h_out, L.dim, b.sums, weight, eps, M, L.dim, nseg, w, n, b.slab_a, b.slab_a_bytes, stream);
     };
     // ---- attention ----
-    if ((st = norm_linears(L.att_norm, L.att_eps, 3, w_qkv, n_qkv))) return st;
-    const int ks_qkv = slices(M, L.dim, 3, n_qkv), rep = L.heads / L.kv_heads;
+    const int rep = L.heads / L.kv_heads;
     const int one = S.attn_one != 0 && M * rep <= 16;
     void *ws = one ? S.attn_one_ws : S.attn_ws;
     const size_t ws_bytes = one ? S.attn_one_ws_bytes : S.attn_ws_bytes;
+    const bool qkv_direct = direct(M, L.dim, 3, run.n_qkv);
+    if (qkv_direct) {
+        if ((st = run.norm(L.att_norm, L.att_eps))) return st;
+        void *out[3] = {b.q, b.k, b.v};
+        st = smh_q40_matmul_tiled_direct(b.xn, M, L.dim, L.dim, 3, run.w_qkv, run.n_qkv, out, nullptr, 0, stream);
+    } else {
+        st = norm_linears(L.att_norm, L.att_eps, 3, run.w_qkv, run.n_qkv);
+    }
+    if (st) return st;
+    const int ks_qkv = slices(M, L.dim, 3, run.n_qkv);
     // (Only in one launch: in two, each of the 256 prefix workgroups adds up and rotates all queries of its kv head.  Grouped queries,
     // three layers of 64 heads over 8 kv heads: 10 branches after 2047 rows 594 us a step so, 552 with the RoPE launch in front; 3
     // branches 523 against 511, 16 branches 629 against 571.)
@@ -107,8 +146,10 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
                                         L.prompt_len, L.cache_k, L.cache_ks, L.cache_v, L.cache_vs, S.smax, S.t_dev, S.pages, S.pages_stride, one, ws,
                                         ws_bytes, stream);
     } else {
-        st = smh_partial_rope_append_kv(b.slab_a, ks_qkv, M, L.heads, L.kv_heads, 128, b.q, b.k, b.v, S.cos_tab, S.sin_tab, S.pos_dev, L.cache_k,
-                                        L.cache_ks, L.cache_v, L.cache_vs, S.smax, S.t_dev, stream);
+        st = qkv_direct ? smh_rope_append_kv(b.q, b.k, b.v, M, L.heads, L.kv_heads, 128, S.cos_tab, S.sin_tab, S.pos_dev, L.cache_k, L.cache_ks, L.cache_v,
+                                             L.cache_vs, S.smax, S.t_dev, stream)
+                        : smh_partial_rope_append_kv(b.slab_a, ks_qkv, M, L.heads, L.kv_heads, 128, b.q, b.k, b.v, S.cos_tab, S.sin_tab, S.pos_dev, L.cache_k,
+                                                     L.cache_ks, L.cache_v, L.cache_vs, S.smax, S.t_dev, stream);
         if (st == 0 && S.pages != nullptr)
             st = smh_paged_prefix_attn(b.q, b.att, M, L.heads, L.kv_heads, 128, L.prompt_k, L.prompt_v, L.prompt_len, 0, 0, SMH_KV_Q40, L.cache_k,
                                        L.cache_v, L.cache_ks, L.cache_vs, 0, 0, S.cache_rows, S.pages, 4, S.pages_stride, S.pages_stride, S.t_dev, 0,
@@ -119,23 +160,21 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
                                                                              b.k, b.v, ws, ws_bytes, stream);
     }
     if (st) return st;
-    if ((st = smh_q40_matmul_partial_tiled(b.att, M, nq, nq, 1, w_o, n_dim, b.slab_b, b.slab_b_bytes, stream))) return st;
-    S.pending = slices(M, nq, 1, n_dim);
+    if ((st = run.residual_linear(b.att, nq, run.w_o))) return st;
     // ---- feed forward ----
     if (S.swiglu_in != 0 && smh_q40_swiglu_fits(M, L.dim, L.ffn)) {
-        if ((st = norm(L.ffn_norm, L.ffn_eps))) return st;
+        if ((st = run.norm(L.ffn_norm, L.ffn_eps))) return st;
         if ((st = smh_q40_matmul_tiled_swiglu(b.xn, M, L.dim, L.dim, L.w1, L.w3, L.ffn, b.act, L.ffn, stream))) return st;
-        st = smh_q40_matmul_partial_tiled(b.act, M, L.ffn, L.ffn, 1, w_d, n_dim, b.slab_b, b.slab_b_bytes, stream);
-    } else {
-        if ((st = norm_linears(L.ffn_norm, L.ffn_eps, 2, w_gu, n_gu))) return st;
-        const int ks_gu = slices(M, L.dim, 2, n_gu);
-        if (M <= S.silu_in_rows && L.ffn % 32 == 0)
-            st = smh_q40_matmul_partial_tiled_silu(b.slab_a, ks_gu, M, L.ffn, 1, w_d, n_dim, b.slab_b, b.slab_b_bytes, stream);
-        else if ((st = smh_partial_silu_mul(b.slab_a, ks_gu, M, L.ffn, b.act, stream)) == 0)
-            st = smh_q40_matmul_partial_tiled(b.act, M, L.ffn, L.ffn, 1, w_d, n_dim, b.slab_b, b.slab_b_bytes, stream);
+        return run.residual_linear(b.act, L.ffn, run.w_d);
     }
-    S.pending = slices(M, L.ffn, 1, n_dim);
-    return st;
+    if ((st = norm_linears(L.ffn_norm, L.ffn_eps, 2, run.w_gu, run.n_gu))) return st;
+    const int ks_gu = slices(M, L.dim, 2, run.n_gu);
+    if (M <= S.silu_in_rows && L.ffn % 32 == 0) {
+        S.pending = slices(M, L.ffn, 1, run.n_dim);
+        return smh_q40_matmul_partial_tiled_silu(b.slab_a, ks_gu, M, L.ffn, 1, run.w_d, run.n_dim, b.slab_b, b.slab_b_bytes, stream);
+    }
+    if ((st = smh_partial_silu_mul(b.slab_a, ks_gu, M, L.ffn, b.act, stream))) return st;
+    return run.residual_linear(b.act, L.ffn, run.w_d);
 }
 
 // One layer of a prefill of `rows` tokens (TransformerBlock.forward with start_pos == 0): k and v go straight to the prompt cache.
@@ -144,54 +183,33 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
 extern "C" int smh_prefill_layer(const smh_layer *layer, smh_pass *pass, smh_stream_t stream) {
     const char *who = "smh_prefill_layer";
     SMH_REQUIRE(layer && pass && pass->h, "%s: null pointer", who);
+    LayerRun run(*layer, *pass, stream);
+    int st = run.begin(who);
+    if (st) return st;
     const smh_layer &L = *layer;
     smh_pass &S = *pass;
-    const int M = S.rows, nq = L.heads * 128, nkv = L.kv_heads * 128;
-    SMH_REQUIRE(M >= 1 && L.heads > 0 && L.kv_heads > 0 && L.heads % L.kv_heads == 0, "%s: rows=%d heads=%d kv_heads=%d", who, M, L.heads, L.kv_heads);
-    LayerBuffers b;
-    if (layer_buffers(L, M, S.swiglu_in != 0, (char *)S.scratch, b) != 0) return -1;
-    SMH_REQUIRE(S.scratch && S.scratch_bytes >= b.total, "%s: scratch %zu < %zu bytes", who, S.scratch_bytes, b.total);
-    const int n_qkv[3] = {nq, nkv, nkv}, n_gu[2] = {L.ffn, L.ffn}, n_dim[1] = {L.dim};
-    const void *w_qkv[3] = {L.wq, L.wk, L.wv}, *w_o[1] = {L.wo}, *w_gu[2] = {L.w1, L.w3}, *w_d[1] = {L.w2};
-    int st = 0;
-    auto norm = [&](const void *weight, float eps) -> int {
-        void *h_out = S.pending > 0 ? b.h[S.h == b.h[0]] : nullptr;
-        const int r = smh_partial_rmsnorm(S.pending > 0 ? b.slab_b : nullptr, S.pending > 0 ? S.pending : 1, M, L.dim, S.h, weight, eps, h_out, b.xn, stream);
-        if (h_out != nullptr) S.h = h_out;
-        S.pending = 0;
-        return r;
-    };
-    // S.h += x . w, at once or as slabs that the next norm adds
-    auto residual_linear = [&](const void *x, int K, const void *const *w) -> int {
-        if (smh_q40_matmul_tiled_direct_fits(M, K, 1, n_dim) == 1) {
-            void *out[1] = {b.h[S.h == b.h[0]]};
-            const int r = smh_q40_matmul_tiled_direct(x, M, K, K, 1, w, n_dim, out, S.h, L.dim, stream);
-            S.h = out[0];
-            return r;
-        }
-        S.pending = slices(M, K, 1, n_dim);
-        return smh_q40_matmul_partial_tiled(x, M, K, K, 1, w, n_dim, b.slab_b, b.slab_b_bytes, stream);
-    };
-    if ((st = norm(L.att_norm, L.att_eps))) return st;
-    if (smh_q40_matmul_tiled_direct_fits(M, L.dim, 3, n_qkv) == 1) {
+    const LayerBuffers &b = run.b;
+    const int M = run.M, nq = run.nq;
+    if ((st = run.norm(L.att_norm, L.att_eps))) return st;
+    if (direct(M, L.dim, 3, run.n_qkv)) {
         void *out[3] = {b.q, L.prompt_k, L.prompt_v};
-        if ((st = smh_q40_matmul_tiled_direct(b.xn, M, L.dim, L.dim, 3, w_qkv, n_qkv, out, nullptr, 0, stream))) return st;
+        if ((st = smh_q40_matmul_tiled_direct(b.xn, M, L.dim, L.dim, 3, run.w_qkv, run.n_qkv, out, nullptr, 0, stream))) return st;
         st = smh_rope(b.q, L.prompt_k, M, L.heads, L.kv_heads, 128, S.cos_tab, S.sin_tab, 0, stream);
     } else {
-        if ((st = smh_q40_matmul_partial_tiled(b.xn, M, L.dim, L.dim, 3, w_qkv, n_qkv, b.slab_a, b.slab_a_bytes, stream))) return st;
-        st = smh_partial_rope_rows(b.slab_a, slices(M, L.dim, 3, n_qkv), M, L.heads, L.kv_heads, 128, b.q, L.prompt_k, L.prompt_v, S.cos_tab, S.sin_tab, 0,
+        if ((st = smh_q40_matmul_partial_tiled(b.xn, M, L.dim, L.dim, 3, run.w_qkv, run.n_qkv, b.slab_a, b.slab_a_bytes, stream))) return st;
+        st = smh_partial_rope_rows(b.slab_a, slices(M, L.dim, 3, run.n_qkv), M, L.heads, L.kv_heads, 128, b.q, L.prompt_k, L.prompt_v, S.cos_tab, S.sin_tab, 0,
                                    stream);
     }
     if (st) return st;
     if ((st = smh_prefill_attn(b.q, L.prompt_k, L.prompt_v, b.att, M, L.heads, L.kv_heads, 128, stream))) return st;
-    if ((st = residual_linear(b.att, nq, w_o))) return st;
-    if ((st = norm(L.ffn_norm, L.ffn_eps))) return st;
+    if ((st = run.residual_linear(b.att, nq, run.w_o))) return st;
+    if ((st = run.norm(L.ffn_norm, L.ffn_eps))) return st;
     if (S.swiglu_in != 0 && smh_q40_swiglu_fits(M, L.dim, L.ffn)) {
         st = smh_q40_matmul_tiled_swiglu(b.xn, M, L.dim, L.dim, L.w1, L.w3, L.ffn, b.act, L.ffn, stream);
-    } else if ((st = smh_q40_matmul_partial_tiled(b.xn, M, L.dim, L.dim, 2, w_gu, n_gu, b.slab_a, b.slab_a_bytes, stream)) == 0) {
-        st = smh_partial_silu_mul(b.slab_a, slices(M, L.dim, 2, n_gu), M, L.ffn, b.act, stream);
+    } else if ((st = smh_q40_matmul_partial_tiled(b.xn, M, L.dim, L.dim, 2, run.w_gu, run.n_gu, b.slab_a, b.slab_a_bytes, stream)) == 0) {
+        st = smh_partial_silu_mul(b.slab_a, slices(M, L.dim, 2, run.n_gu), M, L.ffn, b.act, stream);
     }
-    return st ? st : residual_linear(b.act, L.ffn, w_d);
+    return st ? st : run.residual_linear(b.act, L.ffn, run.w_d);
 }
 
 // The last layer's product added to the residual stream, and the final RMSNorm -> out [rows, dim].

@@ -127,3 +127,24 @@ def test_converter_and_loader_host_logic():
     # the hot path refuses to run without a GPU instead of falling back
     with pytest.raises(AssertionError):
         model(torch.zeros((1, 4), dtype=torch.int64), 0)
+
+
+def test_layer_scratch_holds_every_slab_of_a_pass():
+    """smh_decode_scratch_bytes against the plans of the launches a layer makes: the fp16 buffers, and the slabs of every linear
+    whose launch does not store fp16 itself"""
+    from spec_mcts_amd import _lib
+    lib = _lib.load()
+
+    def slabs(M, K, *ns):
+        n = (ctypes.c_int * len(ns))(*ns)
+        return 0 if lib.smh_q40_matmul_tiled_direct_fits(M, K, len(ns), n) == 1 else lib.smh_q40_matmul_plan_tiled(M, K, len(ns), n) * M * sum(ns) * 4
+
+    for dim, heads, kv_heads, ffn in ((4096, 32, 32, 11008), (5120, 40, 40, 13824), (8192, 64, 8, 28672), (256, 2, 2, 768)):
+        layer = _lib.SmhLayer()
+        layer.dim, layer.heads, layer.kv_heads, layer.ffn = dim, heads, kv_heads, ffn
+        nq, nkv = heads * 128, kv_heads * 128
+        for swiglu in (0, 1):
+            for M in range(1, 1025):
+                gate_up = 0 if M > 128 and swiglu and lib.smh_q40_swiglu_fits(M, dim, ffn) else lib.smh_q40_matmul_plan_tiled(M, dim, 2, (ctypes.c_int * 2)(ffn, ffn)) * M * 2 * ffn * 4
+                need = 2 * M * (3 * dim + 2 * nq + 2 * nkv + ffn) + max(slabs(M, dim, nq, nkv, nkv), gate_up) + max(slabs(M, nq, dim), slabs(M, ffn, dim))
+                assert lib.smh_decode_scratch_bytes(layer, M, swiglu) >= need, (dim, swiglu, M)

@@ -69,3 +69,29 @@ def test_70b_architecture_layer(B, P):
     cfg = dict(ARCH_70B_LAYER, max_batch_size=max(B, 20), max_prompt_seq_len=max(P, 16))
     assert O.ffn_hidden_dim(cfg["dim"], cfg["multiple_of"], cfg["ffn_dim_multiplier"]) == 28672
     _steps(cfg, 74, B, P=P, std=0.02, rtol=1e-2, atol=1e-2, steps=2 if P > 100 else 3)
+
+
+LAYER_7B = dict(dim=4096, n_layers=2, n_heads=32, vocab_size=512, multiple_of=256, max_seq_len=8, max_prompt_seq_len=16)
+
+
+@pytest.mark.parametrize("cfg,B,swiglu", [(LAYER_7B, 129, True), (LAYER_7B, 257, True), (LAYER_7B, 257, False), (LAYER_7B, 400, True), (ARCH_70B_LAYER, 641, True)])
+def test_decode_above_128_branches(cfg, B, swiglu):
+    """Decode steps of more branches than one row block of the GEMM holds: from 257 rows of the 7B shape (385 of the 70B one) the
+    wq|wk|wv launch stores fp16 itself, from 641 rows of the 70B shape wo and w2 do too - no slabs are reserved for such launches."""
+    cfg = dict(cfg, max_batch_size=B)
+    P = 9
+    oargs, sd, model = _build(cfg, 75, 0.02)
+    model.swiglu_in_matmul = swiglu
+    oracle = O.OracleTransformer(oargs, sd, dense=True)
+    gen = torch.Generator().manual_seed(175)
+    prompt = torch.randint(0, cfg["vocab_size"], (1, P), generator=gen)
+    oracle.forward(prompt, 0)
+    model(prompt.cuda(), 0)
+    sync_prefix(model, oracle)
+    for step in range(2):
+        tok = torch.randint(0, cfg["vocab_size"], (B, 1), generator=gen)
+        want = oracle.forward(tok, P + step).float()
+        got = model(tok.cuda(), P + step).cpu().float()
+        print(f"B={B} step {step}: largest logit difference {float((got - want).abs().max()):.4f}", flush=True)
+        assert torch.allclose(got, want, rtol=1e-2, atol=1e-2)
+        sync_suffix_row(model, oracle, B, step)
