@@ -574,14 +574,15 @@ __global__ __launch_bounds__(1024) void sample_topk_kernel(const half_t *__restr
     long first = blockIdx.x;
     int draws = 1;
     if (counts != nullptr) {
-        // every wave adds the counts of the rows before this one (all loads together, not one behind the other)
-        int sum = 0;
-        for (int r = tid & 63; r < (int)blockIdx.x; r += 64) sum += max(counts[r], 0);
+        // every wave adds the counts of the rows before this one (all loads together, not one behind the other); every sum is cut at
+        // n_draws < 2^31 - counts that add up to more than the buffers hold are cut - so none of these unsigned sums wraps
+        const uint32_t most = (uint32_t)max(n_draws, 0);
+        uint32_t sum = 0;
+        for (int r = tid & 63; r < (int)blockIdx.x; r += 64) sum = min(sum + (uint32_t)max(counts[r], 0), most);
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+        for (int o = 32; o > 0; o >>= 1) sum = min(sum + (uint32_t)__shfl_xor((int)sum, o, 64), most);
         first = sum;
-        draws = max(counts[blockIdx.x], 0);
-        draws = (int)max(min((long)draws, (long)n_draws - first), 0L);       // counts that add up to more than the buffers hold are cut
+        draws = min(max(counts[blockIdx.x], 0), (int)(most - sum));
     }
     if (greedy_row) {
         for (int j = tid; j < draws; j += one_wave ? 64 : 1024) out[first + j] = o_idx[0];

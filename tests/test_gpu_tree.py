@@ -49,6 +49,29 @@ def test_counts_beyond_the_buffers_are_cut():
     assert int(results[0, 0]) == int(full[:6].min())              # branch 0 keeps its smallest distinct draw
 
 
+@pytest.mark.parametrize("big", [(1, 2**31 - 1), (2**31 - 1, 2**31 - 1, 7), (2**30, 2**30, 2**30, 2**30, 2**30), (-5, 3, -2**31, 2**31 - 1, 2**31 - 1)])
+@pytest.mark.parametrize("row_temps", [False, True])
+def test_counts_whose_sum_passes_32_bits_are_cut(big, row_temps):
+    """the rows' offsets are sums of counts cut at the buffer, so a sum beyond 2^31 (or 2^32) makes no draw outside it; the draws that
+    fit are those of counts cut on the host"""
+    from spec_mcts_amd import kernels as K
+    g = torch.Generator().manual_seed(83)
+    n, rows = 12, 70                                              # (more rows than lanes: a lane adds two counts)
+    logits = (torch.randn((rows, 4096), generator=g) * 2).half()
+    counts = torch.tensor(list(big) + [2**31 - 1] * (rows - len(big)), dtype=torch.int32)
+    left, cut = n, []
+    for c in counts.tolist():
+        cut.append(min(max(c, 0), left))
+        left -= cut[-1]
+    u = torch.rand(n, generator=g)
+    temp = torch.full((rows,), 0.7).cuda() if row_temps else 0.7
+    want = K.sample_topk_counts(logits.cuda(), temp, 16, torch.tensor(cut, dtype=torch.int32).cuda(), u.cuda()).cpu()
+    buf = torch.full((3 * n,), -1, dtype=torch.int64, device="cuda:0")
+    K.sample_topk_counts(logits.cuda(), temp, 16, counts.cuda(), u.cuda(), out=buf[n:2 * n])
+    assert torch.equal(buf[n:2 * n].cpu(), want)
+    assert bool((buf[:n] == -1).all()) and bool((buf[2 * n:] == -1).all())
+
+
 def test_row_temperature_sampler_matches_oracle():
     """The sampler's temp <= 0 mode: one temperature per branch, quotients and probabilities in float32."""
     from spec_mcts_amd import kernels as K
