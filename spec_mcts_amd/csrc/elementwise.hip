@@ -644,7 +644,7 @@ __global__ __launch_bounds__(256) void tree_fork_kernel(const int64_t *__restric
     const int c0 = min(max(*curr_b, 0), batch_size);             // (a counter outside the batch is cut, never followed)
     if (tid == 0) {
         int off = 0;
-        for (int i = 0; i < c0; ++i) { seg_off[i] = off; off = min(off + max(cnt[i], 0), TREE_MAX_BATCH); }
+        for (int i = 0; i < c0; ++i) { seg_off[i] = off; off = min(off + min(max(cnt[i], 0), TREE_MAX_BATCH), TREE_MAX_BATCH); }
         seg_off[c0] = off;
     }
     __syncthreads();

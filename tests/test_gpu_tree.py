@@ -262,3 +262,31 @@ def test_tree_fork_first_step_of_a_wide_search(seed):
         assert origin.cpu().tolist() == want_origin
         assert torch.equal(d_oc.cpu(), want_oc)
         assert torch.equal(d_res.cpu(), want_res)
+
+
+@pytest.mark.parametrize("B", [200, 255, 256, 257, 300])
+@pytest.mark.parametrize("huge", [False, True])
+def test_tree_step_on_either_side_of_the_small_batch_kernel(B, huge):
+    """Batches (and draws) of up to 256 take the one kernel, larger ones the other: both against the oracle, with rows that run out.
+    huge: the last live branch's multiplicity is 2^31 - 1, of which the draws that the buffer holds exist."""
+    from spec_mcts_amd import kernels as K
+    g = torch.Generator().manual_seed(1700 + B)
+    cur, steps, t = B // 3, 5, 3
+    cuts = torch.sort(torch.randperm(B - 1, generator=g)[: cur - 1] + 1).values.tolist()
+    cnt = [b - a for a, b in zip([0] + cuts, cuts + [B])]
+    oc = torch.zeros((2, B), dtype=torch.int32)
+    oc[1, :cur] = torch.tensor(cnt, dtype=torch.int32)
+    draws = torch.randint(0, 40, (B,), generator=g)
+    alive = torch.rand(B, generator=g) > 0.1
+    alive[cur - 1] = True
+    results = torch.zeros((B, steps), dtype=torch.int64)
+    results[:cur, :t] = torch.randint(1, 32016, (cur, t), generator=g)
+    want_oc, want_res = oc.clone(), results.clone()
+    want_cur, want_origin = O.tree_fork(draws, want_oc, alive, cur, B, want_res, t, None, 0)
+    d_oc = oc.clone()
+    if huge:
+        d_oc[1, cur - 1] = 2**31 - 1
+    d_oc, d_res, d_cur = d_oc.cuda(), results.cuda(), torch.tensor([cur], dtype=torch.int32).cuda()
+    origin = K.tree_fork(draws.cuda(), d_oc, alive.cuda(), d_cur, d_res, t)
+    assert int(d_cur) == want_cur and origin.cpu().tolist() == want_origin
+    assert torch.equal(d_oc.cpu(), want_oc) and torch.equal(d_res.cpu(), want_res)
