@@ -70,11 +70,13 @@ __device__ __forceinline__ int q40_code_near(half_t x, float inv, bool &doubt) {
     doubt = ((__builtin_bit_cast(uint32_t, q) + 0x1003u) & 0x1FFFu) <= 6u;
     return (int)(short)__builtin_rintf16((half_t)q);
 }
-// fp32 quotients: the code changes at n + 1/2.  Adding 1.5 * 2^23 rounds to an integer that stands in the low bits of the sum.
+// fp32 quotients: the code changes at n + 1/2.  Adding 1.5 * 2^23 rounds to an integer that stands in the low bits of the sum.  (A NaN
+// beside finite values leaves the group's scale plain: it is in doubt too and takes the division, code 0.  fp16 groups take their
+// largest magnitude from the bit patterns, so with a NaN their scale is one.)
 __device__ __forceinline__ int q40_code_near(float x, float inv, bool &doubt) {
     constexpr float round = 12582912.0f;
     const float t = __builtin_fmaf(x, inv, round), r = t - round;
-    doubt = fabsf(__builtin_fmaf(x, inv, -r)) > 0.5f - 7.62939453125e-06f;
+    doubt = !(fabsf(__builtin_fmaf(x, inv, -r)) <= 0.5f - 7.62939453125e-06f);
     return __builtin_bit_cast(int, t);
 }
 __device__ __forceinline__ int q40_code_exact(half_t x, float scale) { return q40_code(x, scale); }

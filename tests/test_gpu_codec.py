@@ -102,3 +102,33 @@ def test_quantize_of_the_transpose_matches_the_oracle(dtype, N, Kd):
     w_got, s_got = K.quantize_q40_t(v.cuda())
     assert np.array_equal(_bits(s_got).reshape(-1), _bits(s_want).reshape(-1))
     assert torch.equal(w_got.cpu(), w_want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_quantize_nan_values(dtype):
+    """A NaN has code 0, whatever its payload.  In a group of fp32 or bfloat16 values it does not count towards the scale (the bytes are
+    those of the group with a zero in its place); a group of fp16 values with a NaN has a NaN scale and codes 0."""
+    from spec_mcts_amd import kernels as K
+    g = torch.Generator().manual_seed(9)
+    v = (torch.randn((256, 70), generator=g) * 0.02).to(dtype)
+    bits = torch.int32 if dtype == torch.float32 else torch.int16
+    exponent = {torch.float16: 0x7C00, torch.bfloat16: 0x7F80, torch.float32: 0x7F800000}[dtype]
+    at = [(5, 0), (63, 0), (64, 7), (130, 33), (131, 33), (255, 69)]
+    for i, (n, k) in enumerate(at):
+        v.view(bits)[n, k] = exponent + 1 + 2 * i                 # payloads with low bits set
+    v.view(bits)[200, 50] = -1                                    # all ones
+    assert int(torch.isnan(v).sum()) == len(at) + 1
+    clean = torch.where(torch.isnan(v), torch.zeros_like(v), v)
+    w_want, s_want = O.quantize_q40(clean.t().contiguous(), 64)
+    forms = [K.quantize_q40_t(v.cuda()), K.quantize_q40(v.t().contiguous().cuda())]
+    if dtype == torch.float16:
+        groups = torch.isnan(v.t().reshape(-1, 64)).any(1)
+        nib = w_want.view(torch.uint8).clone().view(-1, 64)
+        nib[groups[0::2]] &= 15                                   # even groups: high nibbles
+        nib[groups[1::2]] &= 240
+        w_want = nib.view(torch.int8).view_as(w_want)
+        s_want = s_want.clone()
+        s_want.view(-1)[groups] = float("nan")
+    for w, s in forms:
+        assert torch.equal(w.cpu(), w_want)
+        assert _same_or_both_nan(_bits(s).reshape(-1), _bits(s_want).reshape(-1))
