@@ -344,9 +344,10 @@ int smh_page_fork(int32_t *table, int rows, long stride, int origin, int curr, i
 
 /* smh_shared_prefix_attn_static: smh_shared_prefix_attn (same arguments without the workspace, same kernels, bit-identical
  * results) for callers that cannot allocate device memory or pass a workspace: code under HIP graph capture, tight
- * serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the reference.  The prefix partials live in
- * a static device array of smh_attn_static_scratch_bytes() = 16 MiB that every GPU the library runs on holds until the
- * process ends; shapes that need more (prefix slices x B x H x 520 bytes) are rejected with an error.  The call allocates
+ * serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the reference.  The partials live in a static
+ * device array that every GPU the library runs on holds until the process ends: smh_attn_static_scratch_bytes() = 16 MiB
+ * for the prefix slices and as much again for the suffixes; shapes whose prefix slices need more (slices x B x H x 520 bytes)
+ * are rejected with an error.  The call allocates
  * and frees nothing; the first call on a device looks the array's address up (make that call outside a graph capture).
  * All calls on one GPU share the array: calls that overlap in time on one GPU race - keep them on one stream. */
 size_t smh_attn_static_scratch_bytes(void);

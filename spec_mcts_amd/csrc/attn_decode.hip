@@ -1608,8 +1608,11 @@ extern "C" int smh_page_fork(int32_t *table, int rows, long stride, int origin, 
 // The prefix partials of smh_shared_prefix_attn_static live in this array instead of a caller's workspace.  Every GPU
 // the library runs on holds its own copy at its own address for the life of the process; host code never uses the
 // array's name as an address, only what hipGetSymbolAddress returned for the current device.
+// ATT_STATIC_SCRATCH_BYTES limits the partials of the prefix slices; behind them the array has room for the suffixes' partials (as many
+// bytes as one slice's, so never more than the slices' together), so that a call takes the same launches as with a workspace of
+// smh_attn_workspace_bytes and returns the same bits.
 constexpr size_t ATT_STATIC_SCRATCH_BYTES = (size_t)16 << 20;
-static __device__ __align__(256) unsigned char scratch[ATT_STATIC_SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char scratch[2 * ATT_STATIC_SCRATCH_BYTES];
 constexpr int ATT_STATIC_MAX_DEVICES = 64;
 static std::mutex g_scratch_mutex;
 static void *g_scratch_ptr[ATT_STATIC_MAX_DEVICES] = {};
@@ -1662,7 +1665,7 @@ extern "C" int smh_shared_prefix_attn_static(const void *q, void *out, int B, in
     const int st = static_scratch(&ws);
     if (st) return st;
     return shared_prefix_attn(who, false, q, out, B, H, Hkv, D, prefix_k, prefix_v, P, suffix_format, suffix_k, suffix_v, suffix_ks, suffix_vs,
-                              Smax, lens, lens_stride, cur_k, cur_v, ws, ATT_STATIC_SCRATCH_BYTES, stream);
+                              Smax, lens, lens_stride, cur_k, cur_v, ws, sizeof(scratch), stream);
 }
 
 extern "C" int smh_shared_prefix_attn_one(const void *q, void *out, int B, int H, int Hkv, int D,

@@ -55,6 +55,19 @@ def test_static_scratch_entry_point_matches_workspace_entry_point():
             assert torch.equal(got.view(torch.int16), want.view(torch.int16)), f"round {rnd}: outputs differ"
 
 
+@pytest.mark.parametrize("B,H,Hkv,P", [(100, 32, 32, 1280), (98, 64, 8, 600), (32, 64, 8, 1900)])
+@pytest.mark.parametrize("q40", [False, True])
+def test_static_scratch_up_to_its_limit_equals_the_workspace_entry_point(B, H, Hkv, P, q40):
+    """shapes whose prefix partials fit the 16 MiB but not together with one more partial per query (what the fp16 launches leave)"""
+    from spec_mcts_amd import kernels as K
+    kw = _case(B, H, Hkv, P, 70, 14, q40)
+    names = ("q", "prefix_k", "prefix_v", "P")
+    rest = {k: v for k, v in kw.items() if k not in names}
+    want = K.shared_prefix_attn(*(kw[n] for n in names), **rest)
+    got = K.shared_prefix_attn(*(kw[n] for n in names), static_scratch=True, **rest)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
 def test_static_scratch_entry_point_rejects_shapes_beyond_its_array():
     from spec_mcts_amd import _lib, kernels as K
     kw = _case(2, 2, 2, 64, 4, 13, False)
