@@ -463,19 +463,21 @@ class Transformer(nn.Module):
         return self._lm_head(run.finish(s, self.norm.weight, self.norm.eps).view(1, S, self.params.dim))
 
     def _layer_struct(self, layer):
-        """What the library's layer calls read of a layer, rebuilt when any of its tensors is another one than at the last pass (the
-        tiled copies are compared as the objects they are, which the key keeps alive)."""
+        """What the library's layer calls read of a layer, rebuilt when any of its tensors or an eps is another one than at the last pass
+        (the tiled copies are compared as the objects they are, which the key keeps alive)."""
         att, ff = layer.attention, layer.feed_forward
         lins = (att.wq, att.wk, att.wv, att.wo, ff.w1, ff.w2, ff.w3)
         key = [layer.attention_norm.weight.data_ptr(), layer.ffn_norm.weight.data_ptr(), att.cache_prompt_k.data_ptr(), att.cache_prompt_v.data_ptr(),
-               att.cache_k.data_ptr(), att.cache_k_s.data_ptr(), att.cache_v.data_ptr(), att.cache_v_s.data_ptr()]
+               att.cache_k.data_ptr(), att.cache_k_s.data_ptr(), att.cache_v.data_ptr(), att.cache_v_s.data_ptr(), layer.attention_norm.eps,
+               layer.ffn_norm.eps]
+        n_fixed = len(key)
         for lin in lins:
             key += (lin.w.data_ptr(), lin.s.data_ptr(), lin._tiled)
         if layer.native is None or layer.native_key != key:
             layer.native = K.layer_struct(self.params.dim, att.n_local_heads, att.n_local_kv_heads, layer.attention_norm.weight, layer.attention_norm.eps,
                                           layer.ffn_norm.weight, layer.ffn_norm.eps, [lin.operand(True) for lin in lins], att.cache_prompt_k,
                                           att.cache_prompt_v, att.cache_k, att.cache_k_s, att.cache_v, att.cache_v_s)
-            key[8:] = [x for lin in lins for x in (lin.w.data_ptr(), lin.s.data_ptr(), lin._tiled)]
+            key[n_fixed:] = [x for lin in lins for x in (lin.w.data_ptr(), lin.s.data_ptr(), lin._tiled)]
             layer.native_key = key
         assert att.cache_prompt_len <= att.cache_prompt_k.shape[1]
         layer.native.prompt_len = att.cache_prompt_len

@@ -232,3 +232,27 @@ def test_prefill_lengths_match_the_oracle(P):
     model.fused = False
     same = model(prompt.cuda(), 0).cpu()
     assert torch.allclose(got.float(), same.float(), rtol=2e-2, atol=2e-2)
+
+
+def test_eps_changed_between_passes_takes_effect():
+    """the norms' eps are read at every pass (decode and prefill), not at the first one"""
+    prompt = torch.randint(0, GQA["vocab_size"], (1, 13), generator=torch.Generator().manual_seed(137)).cuda()
+    tok = prompt[:, :1].expand(3, 1).contiguous()
+
+    def passes(model):
+        model.resetSeq()
+        return model(prompt, 0), model(tok, 13)
+
+    def set_eps(model):
+        for i, layer in enumerate(model.layers):
+            layer.attention_norm.eps, layer.ffn_norm.eps = 0.05 * (i + 1), 0.2 * (i + 1)
+
+    _, _, used = _build(GQA, 37)
+    before = passes(used)
+    set_eps(used)
+    after = passes(used)
+    _, _, fresh = _build(GQA, 37)
+    set_eps(fresh)
+    want = passes(fresh)
+    for a, w, b in zip(after, want, before):
+        assert torch.equal(a, w) and not torch.equal(a, b)
