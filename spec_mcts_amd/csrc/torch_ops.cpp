@@ -61,33 +61,55 @@ const at::Tensor &gpu(PyObject *o, const char *what) {
     need(t.is_cuda(), "spec_mcts_amd kernels need GPU tensors (there is no CPU fallback)");
     return t;
 }
+PyObject *made(PyObject *o) {                  // a new object, or the error that kept it from being made
+    if (o == nullptr) throw Refused{};
+    return o;
+}
+// int(o) and float(o)
 long number(PyObject *o) {
-    const long v = PyLong_AsLong(o);
-    if (v == -1 && PyErr_Occurred()) {
-        // (an integer tensor or a numpy number)
-        PyErr_Clear();
-        PyObject *i = PyNumber_Index(o);
-        if (i == nullptr) throw Refused{};
-        const long w = PyLong_AsLong(i);
-        Py_DECREF(i);
-        if (w == -1 && PyErr_Occurred()) throw Refused{};
-        return w;
+    if (PyLong_CheckExact(o)) {
+        const long v = PyLong_AsLong(o);
+        if (v == -1 && PyErr_Occurred()) throw Refused{};
+        return v;
     }
+    PyObject *i = made(PyNumber_Long(o));
+    const long v = PyLong_AsLong(i);
+    Py_DECREF(i);
+    if (v == -1 && PyErr_Occurred()) throw Refused{};
     return v;
 }
 double real(PyObject *o) {
-    const double v = PyFloat_AsDouble(o);
-    if (v == -1.0 && PyErr_Occurred()) throw Refused{};
+    if (PyFloat_CheckExact(o)) return PyFloat_AS_DOUBLE(o);
+    PyObject *f = made(PyNumber_Float(o));
+    const double v = PyFloat_AS_DOUBLE(f);
+    Py_DECREF(f);
     return v;
 }
-std::vector<int64_t> shape_of(PyObject *o) {
-    PyObject *seq = PySequence_Fast(o, "a shape is a sequence of integers");
-    if (seq == nullptr) throw Refused{};
+// ... of whole numbers only
+long whole_number(PyObject *o) {
+    if (PyLong_CheckExact(o)) return number(o);
+    PyObject *i = made(PyNumber_Index(o));
+    const long v = PyLong_AsLong(i);
+    Py_DECREF(i);
+    if (v == -1 && PyErr_Occurred()) throw Refused{};
+    return v;
+}
+// o <op> v, on the number as it was given
+bool compares(PyObject *o, int op, long v) {
+    PyObject *i = made(PyLong_FromLong(v));
+    const int r = PyObject_RichCompareBool(o, i, op);
+    Py_DECREF(i);
+    if (r < 0) throw Refused{};
+    return r == 1;
+}
+std::vector<int64_t> shape_of(PyObject *o, bool whole) {      // whole: only whole numbers; else int() of each
+    PyObject *seq = made(PySequence_Fast(o, "a shape is a sequence of integers"));
     std::vector<int64_t> v;
     const Py_ssize_t n = PySequence_Fast_GET_SIZE(seq);
     for (Py_ssize_t i = 0; i < n; ++i) {
         try {
-            v.push_back(number(PySequence_Fast_GET_ITEM(seq, i)));
+            PyObject *x = PySequence_Fast_GET_ITEM(seq, i);
+            v.push_back(whole ? whole_number(x) : number(x));
         } catch (Refused &) {
             Py_DECREF(seq);
             throw;
@@ -114,7 +136,7 @@ PyObject *matmul_q40(Args x) {
     need(a.is_contiguous(), "Matrix A must be contiguous");
     need(is(a, at::kHalf) && a.dim() == 2, "A must be fp16 [M, K]");
     const int64_t M = a.size(0), K = a.size(1);
-    const std::vector<int64_t> bs = shape_of(x[3]);
+    const std::vector<int64_t> bs = shape_of(x[3], false);
     need(bs.size() >= 2 && bs[0] == K, "Incompatible dimensions");
     const int64_t N = bs[1];
     need(a.is_cuda() && w.is_cuda() && s.is_cuda(), "spec_mcts_amd kernels need GPU tensors (there is no CPU fallback)");
@@ -146,9 +168,9 @@ PyObject *matmul_q40(Args x) {
 // (w, s, group_size, shape)
 PyObject *deq_int40(Args x) {
     const at::Tensor &w = gpu(x[0], "w"), &s = gpu(x[1], "s");
-    need(number(x[2]) == 64, "group_size must be 64");
+    need(compares(x[2], Py_EQ, 64), "group_size must be 64");
     need(w.is_contiguous() && s.is_contiguous() && is(w, at::kChar) && is(s, at::kHalf), "w int8 and s fp16 must be contiguous");
-    const std::vector<int64_t> shape = shape_of(x[3]);
+    const std::vector<int64_t> shape = shape_of(x[3], true);
     int64_t n = 1;
     for (const int64_t d : shape) n *= d;
     need(n % 128 == 0 && w.numel() == n / 2 && s.numel() == n / 64, "w and s do not match the shape");
@@ -197,8 +219,7 @@ PyObject *sample_topk_counts(Args x) {
     need(is(uniform, at::kFloat) && uniform.is_contiguous(), "uniform must be contiguous fp32");
     at::Tensor out = none(x[5]) ? at::zeros({uniform.numel()}, at::TensorOptions().dtype(at::kLong).device(logits.device())) : gpu(x[5], "out");
     need(is(out, at::kLong) && out.is_contiguous() && out.numel() >= uniform.numel(), "out must be int64 with an entry per uniform number");
-    const long top_k = number(x[2]);
-    const int k = (int)(top_k < vocab ? top_k : vocab);
+    const int k = (int)(compares(x[2], Py_GT, vocab) ? vocab : number(x[2]));
     if (THPVariable_Check(x[1])) {
         const at::Tensor &temp = gpu(x[1], "temperature");
         need(is(temp, at::kFloat) && temp.is_contiguous() && temp.numel() >= rows, "temperature must be fp32 [rows]");
@@ -257,11 +278,11 @@ PyObject *shared_prefix_attn(Args x) {
     if (!none(x[1])) {
         const at::Tensor &k = gpu(x[1], "prefix_k");
         half_rows(k, x[2], "prefix_k and prefix_v must be contiguous fp16", &v);
-        need(k.dim() >= 3 && P <= k.size(-3), "P exceeds the prefix rows");
+        need(k.dim() >= 3 && compares(x[3], Py_LE, k.size(-3)), "P exceeds the prefix rows");
         Hkv = k.size(-2);
     } else {
-        need(P == 0, "P without a prefix");
-        Hkv = !none(x[13]) ? number(x[13]) : !none(x[11]) ? gpu(x[11], "cur_k").size(1) : H;
+        need(compares(x[3], Py_EQ, 0), "P without a prefix");
+        Hkv = !none(x[13]) ? whole_number(x[13]) : !none(x[11]) ? gpu(x[11], "cur_k").size(1) : H;
     }
     int fmt = SMH_KV_NONE;
     if (!none(x[4])) {
@@ -325,7 +346,7 @@ PyObject *paged_prefix_attn(Args x) {
     if (!none(x[8]) && P > 0) {
         const at::Tensor &k = gpu(x[8], "prefix_k");
         half_rows(k, x[9], "prefix_k and prefix_v must be contiguous fp16", &v);
-        need(k.dim() == 3 && k.size(prefix_head_major ? 0 : 1) == Hkv && P <= k.size(prefix_head_major ? 1 : 0), "the prefix does not match");
+        need(k.dim() == 3 && k.size(prefix_head_major ? 0 : 1) == Hkv && compares(x[10], Py_LE, k.size(prefix_head_major ? 1 : 0)), "the prefix does not match");
         if (prefix_head_major) { p_row = D; p_head = k.size(1) * D; }
     } else {
         P = 0;

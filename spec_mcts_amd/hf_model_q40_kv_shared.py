@@ -468,8 +468,8 @@ class Transformer(nn.Module):
         att, ff = layer.attention, layer.feed_forward
         lins = (att.wq, att.wk, att.wv, att.wo, ff.w1, ff.w2, ff.w3)
         key = [layer.attention_norm.weight.data_ptr(), layer.ffn_norm.weight.data_ptr(), att.cache_prompt_k.data_ptr(), att.cache_prompt_v.data_ptr(),
-               att.cache_k.data_ptr(), att.cache_k_s.data_ptr(), att.cache_v.data_ptr(), att.cache_v_s.data_ptr(), layer.attention_norm.eps,
-               layer.ffn_norm.eps]
+               att.cache_k.data_ptr(), att.cache_k_s.data_ptr(), att.cache_v.data_ptr(), att.cache_v_s.data_ptr(), float(layer.attention_norm.eps),
+               float(layer.ffn_norm.eps)]
         n_fixed = len(key)
         for lin in lins:
             key += (lin.w.data_ptr(), lin.s.data_ptr(), lin._tiled)

@@ -653,7 +653,7 @@ def layer_struct(dim: int, H: int, Hkv: int, att_norm: torch.Tensor, att_eps: fl
     assert cache_k.dtype == torch.int8 and cache_v.dtype == torch.int8 and cache_ks.dtype == torch.float16 and cache_vs.dtype == torch.float16
     assert cache_k.is_contiguous() and cache_v.is_contiguous() and cache_ks.is_contiguous() and cache_vs.is_contiguous()
     s = _lib.SmhLayer()
-    s.dim, s.ffn, s.heads, s.kv_heads, s.att_eps, s.ffn_eps = dim, ffn, H, Hkv, att_eps, ffn_eps
+    s.dim, s.ffn, s.heads, s.kv_heads, s.att_eps, s.ffn_eps = dim, ffn, H, Hkv, float(att_eps), float(ffn_eps)
     s.att_norm, s.ffn_norm = att_norm.data_ptr(), ffn_norm.data_ptr()
     s.wq, s.wk, s.wv, s.wo, s.w1, s.w2, s.w3 = (t.buf.data_ptr() for t in tiled)
     s.prompt_k, s.prompt_v = prompt_k.data_ptr(), prompt_v.data_ptr()

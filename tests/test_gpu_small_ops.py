@@ -262,3 +262,49 @@ def test_sampler_candidates_by_maxima_match_the_oracle(rows, vocab, k, temperatu
             target = float(u[r]) * float(cdf[r, -1])
             edges = [float(cdf[r, j - 1]) if j else 0.0, float(cdf[r, j])]
             assert int(got[r]) == int(want[r]) or min(abs(e - target) for e in edges) < 1e-5, (r, j, target, edges)
+
+
+def test_numbers_of_other_types():
+    """sizes and counts are taken as int() takes them (floats, numpy numbers, 0-d tensors), comparisons are made on the number as given"""
+    import math
+    from spec_mcts_amd import kernels as K
+    dev = "cuda:0"
+    logits = torch.randn((3, 512), generator=_g(20)).half().to(dev)
+    counts = torch.tensor([2, 1, 3], dtype=torch.int32, device=dev)
+    u = torch.rand(6, generator=_g(21)).to(dev)
+    want = K.sample_topk_counts(logits, 0.8, 8, counts, u)
+    for k in (8.0, np.int64(8), np.float32(8.5), torch.tensor(8)):
+        assert torch.equal(K.sample_topk_counts(logits, np.float64(0.8), k, counts, u), want)
+    want = K.sample_topk_counts(logits, 0.8, 512, counts, u)
+    for k in (600.5, math.inf, 10**30):
+        assert torch.equal(K.sample_topk_counts(logits, 0.8, k, counts, u), want)
+    with pytest.raises((ValueError, TypeError)):
+        K.sample_topk_counts(logits, 0.8, math.nan, counts, u)
+
+    B, H, P, S = 2, 4, 40, 6
+    q = torch.randn((B, H, 128), generator=_g(22)).half().to(dev)
+    pk, pv = (torch.randn((P, H, 128), generator=_g(23 + i)).half().to(dev) for i in range(2))
+    sk, sv = (torch.randn((B, S, H, 128), generator=_g(25 + i)).half().to(dev) for i in range(2))
+    lens = torch.tensor([6, 3], dtype=torch.int32, device=dev)
+    want = K.shared_prefix_attn(q, pk, pv, 33, suffix_k=sk, suffix_v=sv, Smax=S, lens=lens)
+    for p_, s_, l_ in ((33.0, 6.0, 1.0), (np.int32(33), np.int64(6), True), (torch.tensor(33), 6, 1)):
+        assert torch.equal(K.shared_prefix_attn(q, pk, pv, p_, suffix_k=sk, suffix_v=sv, Smax=s_, lens=lens, lens_stride=l_), want)
+    for p_ in (P + 1, P + 0.5):
+        with pytest.raises(AssertionError):
+            K.shared_prefix_attn(q, pk, pv, p_, suffix_k=sk, suffix_v=sv, Smax=S, lens=lens)
+    with pytest.raises(TypeError):
+        K.shared_prefix_attn(q, None, None, 0, suffix_k=sk, suffix_v=sv, Smax=S, lens=lens, n_kv_heads=4.0)
+    pages = torch.arange(B * S, dtype=torch.int32, device=dev).view(B, S)
+    paged = [K.paged_prefix_attn(q, pages, lens, sk.view(-1, H, 128), sv.view(-1, H, 128), prefix_k=pk, prefix_v=pv, P=p_, lens_stride=l_)
+             for p_, l_ in ((33, 1), (33.0, 1.0))]
+    assert torch.equal(paged[0], paged[1])
+
+    v = torch.randn((128, 64), generator=_g(28)).half()
+    w, s = K.quantize_q40(v.to(dev))
+    assert torch.equal(K.deq_int40(w, s, 64.0, (128, 64)), K.deq_int40(w, s, 64, (128, 64)))
+    with pytest.raises(AssertionError):
+        K.deq_int40(w, s, 64.5, (128, 64))
+    with pytest.raises(TypeError):
+        K.deq_int40(w, s, 64, (128.0, 64.0))
+    a = torch.randn((3, 64), generator=_g(29)).half().to(dev)
+    assert torch.equal(K.matmul_q40(a, w, s, (64.0, 128.0)), K.matmul_q40(a, w, s, (64, 128)))
