@@ -36,6 +36,20 @@ def _need_gpu(*tensors: torch.Tensor) -> None:
         assert t.is_cuda, "spec_mcts_amd kernels need GPU tensors (there is no CPU fallback)"
 
 
+def matmul_workspace(device: torch.device, max_m: int = 16, max_n: int = 0) -> torch.Tensor:
+    """Per-device scratch for callers of smh_q40_matmul (matmul_q40 takes its own from torch's allocator): the fp32 K-slice slabs
+    between the matmul kernel and its reduce kernel.  Shared by all who ask for it on the device; calls issued on different
+    streams at the same time need their own workspace."""
+    lib = _lib.load()
+    need = lib.smh_q40_matmul_workspace_bytes(int(max_m), int(max_n))
+    key = ("matmul", device.index if device.index is not None else torch.cuda.current_device())
+    ws = _workspaces.get(key)
+    if ws is None or ws.numel() < need:
+        ws = torch.empty(need, dtype=torch.uint8, device=device)
+        _workspaces[key] = ws
+    return ws
+
+
 def attn_workspace(device: torch.device, B: int, H: int, P: int) -> torch.Tensor:
     lib = _lib.load()
     need = lib.smh_attn_workspace_bytes(int(B), int(H), int(P))

@@ -240,3 +240,19 @@ def test_fused_rope_append_consumer_bit_exact():
     assert torch.equal(cv.cpu().view(B, Smax, Hkv, 64)[:, t], wv.view(B, Hkv, 64))
     assert torch.equal(cks.cpu().view(B, Smax, Hkv, 2)[:, t].view(torch.int16), sk.view(B, Hkv, 2).view(torch.int16))
     assert torch.equal(cvs.cpu().view(B, Smax, Hkv, 2)[:, t].view(torch.int16), sv.view(B, Hkv, 2).view(torch.int16))
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 100])
+def test_matmul_workspace_serves_the_c_entry_point(M):
+    """smh_q40_matmul on the workspace that matmul_workspace returns: what matmul_q40 returns, bit for bit"""
+    from spec_mcts_amd import _lib, kernels as K
+    N, Kd = 1024, 2048
+    g = torch.Generator().manual_seed(60 + M)
+    w, s = K.quantize_q40((torch.randn((Kd, N), generator=g) * 0.02).half().cuda())
+    a = torch.randn((M, Kd), generator=g).half().cuda()
+    ws = K.matmul_workspace(a.device, M, N)
+    assert ws.numel() >= _lib.load().smh_q40_matmul_workspace_bytes(M, N) and K.matmul_workspace(a.device, 1, 128) is ws
+    c = torch.empty((M, N), dtype=torch.float16, device=a.device)
+    K.check(_lib.load().smh_q40_matmul(a.data_ptr(), M, Kd, Kd, w.data_ptr(), s.data_ptr(), N, c.data_ptr(), N, K.SMH_EPI_NONE, None, N,
+                                       ws.data_ptr(), ws.numel(), K._stream()), "smh_q40_matmul")
+    assert torch.equal(c, K.matmul_q40(a, w, s, (Kd, N)))
