@@ -327,8 +327,9 @@ __global__ __launch_bounds__(256) void attn_prefix_kernel(AttnParams p) {
 // have the same ids throughout the slice, its rows are staged in LDS once for the 16 queries and multiplied on the matrix
 // cores - wave w scores positions 16 w .. + 15 and then makes dims 32 w .. + 31 of the outputs - and a partial (max, sum,
 // o[128]) is left per query; tile_done says so and attn_suffix_kernel skips the slice.  Where they differ, or a staged value
-// is infinite or NaN, the slice is left to attn_suffix_kernel.  Probabilities enter the product as two fp16 terms (the second
-// 2^11 times what the first leaves over), 22 bits: against 64-bit sums the result is no further off than the fp32 walk's.
+// is infinite or NaN, the slice is left to attn_suffix_kernel.  Probabilities enter the product as three fp16 terms of 2^15 p (the
+// second 2^11 times what the first leaves over, the third 2^11 times what the second does), in three accumulators: all 24 bits of
+// the fp32 probability down to 2^-38 of the slice's largest, 2^-62 of it absolutely below, so nothing of it is rounded away.
 // Bound by the walk of what is not shared.  32 heads, 512 positions, half of them a prompt: 99 branches 150 -> 100 us a call, 50: 80 -> 60,
 // 27: 45 -> 37, 8: 32 -> 20; 460 shared positions and 99 branches: 111 -> 39 us (error against 64 bits 2.1e-4 before and after: the
 // output's fp16).  Where nothing is shared the pass costs its 3 us (100 positions, 99 branches: 29.7 -> 26.5 with the walk's gain).
@@ -342,7 +343,7 @@ __device__ __forceinline__ long page_at(const AttnParams &p, long i) {
 __global__ __launch_bounds__(256) void attn_page_tile_kernel(AttnParams p) {
     __shared__ __attribute__((aligned(16))) half_t ks[PT_TW][ATT_KPITCH];
     __shared__ __attribute__((aligned(16))) half_t vt[ATT_D][PT_TW + 8];
-    __shared__ __attribute__((aligned(16))) half_t ps[2][16][PT_TW + 8];      // probabilities of the 16 queries, both terms, in vt_pos order
+    __shared__ __attribute__((aligned(16))) half_t ps[3][16][PT_TW + 8];      // probabilities of the 16 queries, the three terms, in vt_pos order
     __shared__ long s_row[PT_TW];
     __shared__ float s_max[4][16], s_sum[4][16];
     const int hk = blockIdx.x, split = blockIdx.y, tile = blockIdx.z;
@@ -419,35 +420,38 @@ __global__ __launch_bounds__(256) void attn_page_tile_kernel(AttnParams p) {
     __syncthreads();
     mx = fmaxf(fmaxf(s_max[0][c], s_max[1][c]), fmaxf(s_max[2][c], s_max[3][c]));
     float sum = 0.f;
-    h4 p_hi, p_lo;
+    h4 term[3];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const float e = exp2f(st[r] - mx);
         sum += e;
-        p_hi[r] = (half_t)e;
-        p_lo[r] = (half_t)((e - (float)p_hi[r]) * 2048.f);
+        float left = e * 32768.f;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {              // (the differences and the powers of two are exact)
+            term[i][r] = (half_t)left;
+            left = (left - (float)term[i][r]) * 2048.f;
+        }
     }
-    {
-        const int at = 32 * (wave >> 1) + 8 * g + 4 * (wave & 1);
-        *reinterpret_cast<h4 *>(&ps[0][c][at]) = p_hi;
-        *reinterpret_cast<h4 *>(&ps[1][c][at]) = p_lo;
-    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) *reinterpret_cast<h4 *>(&ps[i][c][32 * (wave >> 1) + 8 * g + 4 * (wave & 1)]) = term[i];
     sum += __shfl_xor(sum, 16, 64);
     sum += __shfl_xor(sum, 32, 64);
     if (g == 0) s_sum[wave][c] = sum;
     __syncthreads();
     // ---- O^T: element r of o[i] is dim 32 wave + 16 i + 4 g + r, column (query) c ----
-    f4 o_hi[2], o_lo[2];
+    f4 ot[3][2];                                   // by term
 #pragma unroll
-    for (int i = 0; i < 2; ++i) { o_hi[i] = f4{0.f, 0.f, 0.f, 0.f}; o_lo[i] = f4{0.f, 0.f, 0.f, 0.f}; }
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) ot[k][i] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int jj = 0; jj < PT_TW / 32; ++jj) {
-        const h8 ph = *reinterpret_cast<const h8 *>(&ps[0][c][32 * jj + 8 * g]), pl = *reinterpret_cast<const h8 *>(&ps[1][c][32 * jj + 8 * g]);
+        const h8 va[2] = {*reinterpret_cast<const h8 *>(&vt[32 * wave + c][32 * jj + 8 * g]), *reinterpret_cast<const h8 *>(&vt[32 * wave + 16 + c][32 * jj + 8 * g])};
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const h8 va = *reinterpret_cast<const h8 *>(&vt[32 * wave + 16 * i + c][32 * jj + 8 * g]);
-            o_hi[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, ph, o_hi[i], 0, 0, 0);
-            o_lo[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pl, o_lo[i], 0, 0, 0);
+        for (int k = 0; k < 3; ++k) {
+            const h8 pb = *reinterpret_cast<const h8 *>(&ps[k][c][32 * jj + 8 * g]);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) ot[k][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va[i], pb, ot[k][i], 0, 0, 0);
         }
     }
     if (qrow >= p.Bq) return;
@@ -456,7 +460,7 @@ __global__ __launch_bounds__(256) void attn_page_tile_kernel(AttnParams p) {
     for (int i = 0; i < 2; ++i) {
         f4 o;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = o_hi[i][r] + o_lo[i][r] * (1.f / 2048.f);
+        for (int r = 0; r < 4; ++r) o[r] = (ot[0][i][r] + (ot[1][i][r] + ot[2][i][r] * 0x1p-11f) * 0x1p-11f) * 0x1p-15f;
         *reinterpret_cast<f4 *>(p.part_o + base * ATT_D + 32 * wave + 16 * i + 4 * g) = o;
     }
     if (wave == 0 && g == 0) {

@@ -247,3 +247,24 @@ def test_pages_shared_by_the_branches_of_a_tile(B, H, Hkv, L, shared, odd):
     assert torch.equal(got.isinf(), want.isinf())
     fin = want.isfinite()
     assert bool(((got - want)[fin].abs() <= 2e-3 + 1e-2 * want[fin].abs()).all())
+
+
+def test_shared_pages_keep_fp32_probabilities():
+    """The matrix-core pass holds a probability's 24 bits: weights 2^-25 .. 2^-36 of the largest carry the whole result (the largest
+    one's row is zero), which is as far from 64-bit sums as fp16 output makes it (with two terms: 1.15 times as far)."""
+    from spec_mcts_amd import kernels as K
+    g = torch.Generator().manual_seed(3)
+    B, H, L, D = 16, 8, 256, 128
+    q = torch.zeros((B, H, D))
+    q[..., 0] = 8.0
+    k = torch.zeros((H, L, D))
+    k[..., 0] = -(25 + 11 * torch.rand((H, L), generator=g)) * 0.6931 * D ** 0.5 / 8
+    v = 30000 + 5000 * torch.randn((H, L, D), generator=g)
+    k[:, 5], v[:, 5] = 0, 0
+    q, k, v = q.half(), k.half(), v.half()
+    p = torch.softmax(torch.einsum("bhd,hld->bhl", q.double(), k.double()) / D ** 0.5, -1)
+    want = torch.einsum("bhl,hld->bhd", p, v.double())
+    pages = torch.arange(L, dtype=torch.int32)[None].expand(B, L).contiguous()
+    got = K.paged_prefix_attn(q.cuda(), pages.cuda(), None, k.cuda(), v.cuda(), head_major=True).cpu().double()
+    rounding = float((want.half().double() - want).norm())
+    assert float((got - want).norm()) <= 1.02 * rounding
