@@ -1242,10 +1242,8 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p) {
         }
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-            const float m_new = fmaxf(m, ml[i][0]);
-            if (m_new == -INFINITY) continue;                // nothing yet
-            const float c1 = exp2f(m - m_new), c2 = exp2f(ml[i][0] - m_new);
-            m = m_new;
+            float c1, c2;
+            m = soft_join(m, ml[i][0], c1, c2);
             l = l * c1 + ml[i][1] * c2;
             o[0] = o[0] * c1 + v[i][0] * c2;
             o[1] = o[1] * c1 + v[i][1] * c2;
@@ -1327,14 +1325,11 @@ __global__ __launch_bounds__(256, 2) void attn_one_kernel(AttnParams p) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) o[j] = 0.f;
         auto fold = [&](float pm, float pl, const float (&po)[8]) {
-            const float m_new = fmaxf(m, pm);
-            if (m_new != -INFINITY) {
-                const float c1 = exp2f(m - m_new), c2 = exp2f(pm - m_new);
-                m = m_new;
-                l = l * c1 + pl * c2;
+            float c1, c2;
+            m = soft_join(m, pm, c1, c2);
+            l = l * c1 + pl * c2;
 #pragma unroll
-                for (int j = 0; j < 8; ++j) o[j] = o[j] * c1 + po[j] * c2;
-            }
+            for (int j = 0; j < 8; ++j) o[j] = o[j] * c1 + po[j] * c2;
         };
         for (int s0 = si; live && s0 < n_part; s0 += 4 * sub) {
             f4 lo[4], hi[4];

@@ -297,3 +297,30 @@ def test_fp16_suffix_beside_the_prefix_slices(B, H, Hkv, P, S, current):
                                        d[4].data_ptr(), None, None, S, d[5].data_ptr(), 1, d[6].data_ptr() if current else None,
                                        d[7].data_ptr() if current else None, ws.data_ptr(), ws.numel(), K._stream()), "smh_shared_prefix_attn")
     assert bool(((out.cpu().double() - want).abs() <= tol).all())
+
+
+@pytest.mark.parametrize("B,H,Hkv,P,S,L", [(2, 4, 4, 64, 20, 20), (2, 4, 4, 0, 20, 20), (2, 4, 4, 64, 20, 0), (20, 8, 2, 300, 70, 64), (3, 8, 2, 200, 9, 5)])
+@pytest.mark.parametrize("q40", [False, True])
+@pytest.mark.parametrize("single_launch", [False, True])
+@pytest.mark.parametrize("current", [False, True])
+def test_nan_in_a_query_stays_visible(B, H, Hkv, P, S, L, q40, single_launch, current):
+    """a NaN in a query makes every score of it NaN: its output is NaN in every form of the attention (no partial has a maximum then),
+    all others are what they are without it"""
+    from spec_mcts_amd import kernels as K
+    g = _g(300 + B + P)
+    q = torch.randn((B, H, 128), generator=g).half()
+    pk, pv = (torch.randn((max(P, 1), Hkv, 128), generator=g).half().cuda() if P else None for _ in range(2))
+    kw = dict(Smax=S, lens=torch.full((B,), L, dtype=torch.int32).cuda(), n_kv_heads=Hkv, single_launch=single_launch)
+    if q40:
+        kw.update(zip(("suffix_k", "suffix_v"), (torch.randint(-128, 128, (B, S, Hkv, 64), generator=g, dtype=torch.int16).to(torch.int8).cuda() for _ in range(2))))
+        kw.update(zip(("suffix_ks", "suffix_vs"), ((torch.rand((B, S, Hkv, 2), generator=g) * 0.1).half().cuda() for _ in range(2))))
+    else:
+        kw.update(zip(("suffix_k", "suffix_v"), (torch.randn((B, S, Hkv, 128), generator=g).half().cuda() for _ in range(2))))
+    if current:
+        kw.update(zip(("cur_k", "cur_v"), (torch.randn((B, Hkv, 128), generator=g).half().cuda() for _ in range(2))))
+    clean = K.shared_prefix_attn(q.cuda(), pk, pv, P, **kw).cpu()
+    q[B - 1, H - 1, 5] = float("nan")
+    got = K.shared_prefix_attn(q.cuda(), pk, pv, P, **kw).cpu()
+    assert bool(got[B - 1, H - 1].isnan().all())
+    got[B - 1, H - 1] = clean[B - 1, H - 1] = 0
+    assert torch.equal(got, clean)

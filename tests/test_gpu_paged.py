@@ -268,3 +268,20 @@ def test_shared_pages_keep_fp32_probabilities():
     got = K.paged_prefix_attn(q.cuda(), pages.cuda(), None, k.cuda(), v.cuda(), head_major=True).cpu().double()
     rounding = float((want.half().double() - want).norm())
     assert float((got - want).norm()) <= 1.02 * rounding
+
+
+@pytest.mark.parametrize("shared", [False, True])
+def test_nan_in_a_query_stays_visible_through_pages(shared):
+    """pages of the branches' own and pages that all share (the matrix-core pass): a query with a NaN has a NaN output, the others do not"""
+    from spec_mcts_amd import kernels as K
+    g = torch.Generator().manual_seed(12)
+    B, H, L = 4, 4, 130
+    k, v = (torch.randn((H, B * L, 128), generator=g).half().cuda() for _ in range(2))
+    q = torch.randn((B, H, 128), generator=g).half()
+    pages = torch.arange(L, dtype=torch.int32)[None].expand(B, L).contiguous() if shared else torch.arange(B * L, dtype=torch.int32).view(B, L)
+    clean = K.paged_prefix_attn(q.cuda(), pages.cuda(), None, k, v, head_major=True).cpu()
+    q[1, 2, 5] = float("nan")
+    got = K.paged_prefix_attn(q.cuda(), pages.cuda(), None, k, v, head_major=True).cpu()
+    assert bool(got[1, 2].isnan().all())
+    got[1, 2] = clean[1, 2] = 0
+    assert torch.equal(got, clean)
