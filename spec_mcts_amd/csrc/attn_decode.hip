@@ -489,6 +489,7 @@ __global__ __launch_bounds__(256) void attn_page_tile_kernel(AttnParams p) {
 // (The two chains of S^T products interleaved, 32-bit row offsets, a higher wave priority for one key group: no gain.)
 // q [S,H,128], k, v [S,Hkv,128], out [S,H,128].
 constexpr int PF_TW = 64;                                  // keys of a tile
+constexpr int PF_BUFFER_WORD3 = 4 << 15;                   // last word of an untyped buffer's descriptor: data format "32"
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef const __attribute__((address_space(1))) void *att_gptr_t;
 typedef __attribute__((address_space(3))) void *att_lptr_t;
@@ -544,13 +545,15 @@ __global__ __launch_bounds__(128 * QG, 1) void attn_prefill_kernel(PrefillParams
     u32x4 vreg[VG][4];
     const int ch = tid & 15;
     auto v_fetch = [&](int it) {
+        // Buffer loads over the rows of this pair of tiles that there are: past them they read zeros.  (A repeated last row would be
+        // infinite where that row is, and its weight of 0 makes a NaN of it.)
+        const int left = min(p.S - it * 2 * PF_TW, 2 * PF_TW), pitch = (int)row_stride * 2;
+        const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(vbase) + (long)it * 2 * PF_TW * row_stride, 0,
+                                                                              (left - 1) * pitch + 2 * ATT_D, PF_BUFFER_WORD3);
 #pragma unroll
         for (int g = 0; g < VG; ++g)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int row = min(it * 2 * PF_TW + 4 * ((tid >> 4) + 4 * NW * g) + i, p.S - 1);
-                vreg[g][i] = *reinterpret_cast<const u32x4 *>(vbase + (row * row_stride + 8 * ch));
-            }
+            for (int i = 0; i < 4; ++i) vreg[g][i] = __builtin_amdgcn_raw_buffer_load_b128(rows, (4 * ((tid >> 4) + 4 * NW * g) + i) * pitch + 16 * ch, 0, 0);
     };
     auto v_store = [&](int buf) {
 #pragma unroll
@@ -631,6 +634,9 @@ __global__ __launch_bounds__(128 * QG, 1) void attn_prefill_kernel(PrefillParams
                 }
 #pragma unroll
             for (int b = 0; b < 4; ++b) {                  // sixteen keys at a time
+                // (the second half of a tile that begins at this wave's first query: its keys weigh 0, but 0 times an infinite or NaN
+                // value is NaN, so it stays out of the product)
+                if (b == 2 && k_lo == q_lo) break;
 #pragma unroll
                 for (int d = 0; d < 4; ++d) {
                     const int row = 32 * d + c;
@@ -1762,7 +1768,7 @@ extern "C" int smh_prefill_attn(const void *q, const void *k, const void *v, voi
     p.scale_log2 = LOG2E / sqrtf((float)D);
     // four query groups (128 queries) a workgroup share a staged tile; two where that would leave compute units without a workgroup
     const long blocks4 = (long)((S + 127) / 128) * H, blocks2 = (long)((S + 63) / 64) * H;
-    SMH_REQUIRE(blocks2 < (1L << 31), "smh_prefill_attn: S=%d H=%d", S, H);
+    SMH_REQUIRE(blocks2 < (1L << 31) && Hkv <= 65536, "smh_prefill_attn: S=%d H=%d Hkv=%d (at most 65536: a pair of tiles spans 31 bits)", S, H, Hkv);
     static const hipError_t lds_ok = [] {
         const hipError_t e = hipFuncSetAttribute((const void *)attn_prefill_kernel<4>, hipFuncAttributeMaxDynamicSharedMemorySize, PF_LDS);
         return e != hipSuccess ? e : hipFuncSetAttribute((const void *)attn_prefill_kernel<2>, hipFuncAttributeMaxDynamicSharedMemorySize, PF_LDS);

@@ -324,3 +324,21 @@ def test_nan_in_a_query_stays_visible(B, H, Hkv, P, S, L, q40, single_launch, cu
     assert bool(got[B - 1, H - 1].isnan().all())
     got[B - 1, H - 1] = clean[B - 1, H - 1] = 0
     assert torch.equal(got, clean)
+
+
+@pytest.mark.parametrize("S,H", [(97, 4), (130, 256)])
+@pytest.mark.parametrize("at", [5, 50, 96])
+def test_prefill_values_that_are_not_finite_reach_no_earlier_block(S, H, at):
+    """masked keys weigh 0, and 0 times an infinity is NaN: a value that is not finite must not reach the blocks of 32 queries before
+    its own, whose products leave it out"""
+    from spec_mcts_amd import kernels as K
+    g = _g(77)
+    q, k, v = (torch.randn((S, H, 128), generator=g).half() for _ in range(3))
+    clean = K.prefill_attn(q.cuda(), k.cuda(), v.cuda()).cpu()
+    v[at, 1, 3], v[at, 1, 4] = float("inf"), float("nan")
+    got = K.prefill_attn(q.cuda(), k.cuda(), v.cuda()).cpu()
+    assert torch.equal(got[: at // 32 * 32], clean[: at // 32 * 32])
+    assert bool(got[at:, 1, 3].isinf().all()) and bool(got[at:, 1, 4].isnan().all())
+    others = torch.ones((S, H, 128), dtype=torch.bool)
+    others[:, 1, 3:5] = False
+    assert torch.equal(got[others], clean[others])
