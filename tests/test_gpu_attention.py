@@ -342,3 +342,14 @@ def test_prefill_values_that_are_not_finite_reach_no_earlier_block(S, H, at):
     others = torch.ones((S, H, 128), dtype=torch.bool)
     others[:, 1, 3:5] = False
     assert torch.equal(got[others], clean[others])
+
+
+@pytest.mark.parametrize("S", [1, 31, 32, 33, 63, 64, 65, 95, 127, 128, 129, 191, 193, 255, 257, 385])
+@pytest.mark.parametrize("H,Hkv", [(256, 32), (2, 1)])
+def test_prefill_lengths_around_the_tiles(S, H, Hkv):
+    """every remainder class of the waves' 32 queries, the tiles of 64 keys and the workgroups' 64 and 128 queries: 256 heads fill the
+    GPU with four query groups a workgroup, 2 heads take two groups"""
+    from spec_mcts_amd import kernels as K
+    g = _g(500 + S)
+    q, k, v = (torch.randn((S, h, 128), generator=g).half() for h in (H, Hkv, Hkv))
+    _check(K.prefill_attn(q.cuda(), k.cuda(), v.cuda()), O.causal_attention(q, k, v))
