@@ -1083,13 +1083,17 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_swiglu_kernel(MatmulParams p)
 
 // Row blocks and K-slices of a launch with more than 128 rows: the pair with the least estimated time.  Measured on the 7B shapes
 // at 160 .. 2047 rows: a workgroup takes 0.18 us a step and 0.24 more at 128 rows (in proportion), 4 us around its loop; a launch
-// takes as many of these as its workgroups need rounds over 256 compute units, and at least 1.2 times its share of them when all
+// takes as many of these as the workgroups of the busiest XCD need rounds over its 32 compute units (whole column units go to an
+// XCD: of 20 units six XCDs get three, one two and one none), and at least 1.2 times its share of them when all
 // compute units are busy (the clock drops: two workgroups that share a compute unit take as long as one behind the other).  A
 // split's consumer reads 4 bytes an output and slice at ~4 TB/s.  Blocks are even (130 rows: two of 80, not 128 and 2).
 // (Before, 128-row blocks and at most 1600 / M slices: w1|w3 at 300 rows 108 us, now 85; wo and w2 at 1024 rows 56 and 136, now
-// 37 and 88; 700 rows of wq|wk|wv 108, now 89.)
-static float gemm_rows_us(long tiles, int rows, int steps) {
-    const float r = (float)tiles / 256.0f, rounds = (float)((tiles + 255) / 256);
+// 37 and 88; 700 rows of wq|wk|wv 108, now 89.  With rounds counted over the 256 compute units together: 5120 x 5120 at 1024 rows
+// 128 us, now 77, 5120 x 13824 at 512 rows 138, now 101.)
+// Against measurement at the 7B, 13B, 34B and 70B shapes, 160 .. 2047 rows: 0.87 to 1.17 times the estimate, 1.3 to 1.4 times it
+// for square weights at 160 rows (15 and 19 us: launches).
+static float gemm_rows_us(int units, long of_unit, int rows, int steps) {
+    const float r = (float)(units * of_unit) / 256.0f, rounds = (float)(((units + 7) / 8 * of_unit + 31) / 32);
     return (rounds > 1.2f * r ? rounds : 1.2f * r) * ((float)steps * (0.18f + 0.24f * rows / GEMM_BM) + 4.0f);
 }
 static void gemm_plan_rows(MatmulParams &p, int steps, int max_ks) {
@@ -1100,7 +1104,7 @@ static void gemm_plan_rows(MatmulParams &p, int steps, int max_ks) {
         const int blocks = (p.M + rows - 1) / rows;
         const long tiles = (long)p.units * blocks;
         for (int ks = 1; ks <= max_ks && (ks == 1 || (tiles * ks <= 512 && steps / ks >= GEMM_STAGES)); ++ks) {
-            const float us = gemm_rows_us(tiles * ks, rows, (steps + ks - 1) / ks) + (ks > 1 ? (float)ks * p.M * p.n_total * 4.0f / 4.0e6f : 0.0f);
+            const float us = gemm_rows_us(p.units, (long)blocks * ks, rows, (steps + ks - 1) / ks) + (ks > 1 ? (float)ks * p.M * p.n_total * 4.0f / 4.0e6f : 0.0f);
             if (best_us < 0.0f || us < best_us) {
                 best_us = us;
                 ksplit = ks;
@@ -1262,7 +1266,12 @@ static int gemm_launch_layout(const MatmulParams &p, hipStream_t stream) {
     SMH_REQUIRE((long)p.M * p.lda * 2 < (1L << 32), "q40 gemm: M x lda = %d x %ld exceeds the 32-bit lane offsets of A", p.M, p.lda);
     const int tiles = max(2, p.mblocks > 1 ? p.block_rows / 16 : (p.M + 15) / 16);
     const bool odd_k = p.K % 32 != 0;
-    const bool one_each = !(TILED && odd_k) && (p.chunk > 0 || (long)p.units * p.mblocks * p.ksplit <= GEMM_DMA_WAVE_MAX_WGS);
+    // (Whole column units go to an XCD, so with few of them an XCD can get more than its 32 workgroups although the launch has fewer than
+    // 256: those wait for a second round unless they share a compute unit, which four-wave workgroups do.  Where they are short that is
+    // the better way: 26 x 7168 x 1984 14.3 against 16.2 us, 93 x 5504 x 5792 26.1 against 29.1; from 25 steps on level or worse: 73 x
+    // 4736 x 15840 43.7 against 41.4, 45 x 21120 x 18728 152 against 141.)
+    const bool crowded = !TILED && (long)(p.units_pad / 8) * p.mblocks * p.ksplit > GEMM_DMA_WAVE_MAX_WGS / 8 && p.steps_per_slice <= 24;
+    const bool one_each = !(TILED && odd_k) && (p.chunk > 0 || ((long)p.units * p.mblocks * p.ksplit <= GEMM_DMA_WAVE_MAX_WGS && !crowded));
     const bool four = odd_k ? !one_each : !TILED && !one_each;
     const gemm_kernel_t kern = odd_k ? (TILED ? ragged : (one_each ? ragged_dma_wave : ragged_four)[tiles])
                                      : (p.chunk > 0 ? range_cut : one_each ? with_dma_wave : exact)[tiles];

@@ -256,3 +256,18 @@ def test_matmul_workspace_serves_the_c_entry_point(M):
     K.check(_lib.load().smh_q40_matmul(a.data_ptr(), M, Kd, Kd, w.data_ptr(), s.data_ptr(), N, c.data_ptr(), N, K.SMH_EPI_NONE, None, N,
                                        ws.data_ptr(), ws.numel(), K._stream()), "smh_q40_matmul")
     assert torch.equal(c, K.matmul_q40(a, w, s, (Kd, N)))
+
+
+@pytest.mark.parametrize("M,N,K", [(33, 4352, 2880), (100, 4352, 2888), (17, 6400, 1920), (96, 2304, 1032), (257, 2688, 1040), (300, 5120, 1024)])
+def test_matmul_with_few_column_units(M, N, K):
+    """Column units that do not divide by the eight XCDs: launches of at most 256 workgroups of which one XCD would get more than 32
+    (four waves a workgroup where its steps are few), K a multiple of 32 and not, and row blocks planned for the busiest XCD"""
+    from spec_mcts_amd import kernels as K_
+    w, s = _weights(N, K, seed=N + K)
+    a = _acts(M, K, seed=M)
+    r = _acts(M, N, seed=M + 1)
+    want = O.matmul_q40(a, w, s, (K, N)).float()
+    got = K_.matmul_q40(a.cuda(), w.cuda(), s.cuda(), (K, N)).cpu().float()
+    assert torch.allclose(got, want, rtol=RTOL, atol=ATOL)
+    got = K_.matmul_q40(a.cuda(), w.cuda(), s.cuda(), (K, N), residual=r.cuda()).cpu().float()
+    assert torch.allclose(got, r.float() + want, rtol=RTOL, atol=2 * ATOL)
