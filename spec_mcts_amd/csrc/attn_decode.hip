@@ -309,8 +309,8 @@ __device__ __forceinline__ void attn_prefix_body(const AttnParams &p, int split,
                 else *reinterpret_cast<f4 *>(po + 16 * dt + 4 * g) = ot[dt];
             }
             if (g == 0) {
-                if (COHERENT) { st_f32(p.part_ml + base * 2, mx); st_f32(p.part_ml + base * 2 + 1, sum); }
-                else { p.part_ml[base * 2] = mx; p.part_ml[base * 2 + 1] = sum; }
+                if (COHERENT) { st_f32(p.part_ml + base * 2, partial_max(mx, sum)); st_f32(p.part_ml + base * 2 + 1, sum); }
+                else { p.part_ml[base * 2] = partial_max(mx, sum); p.part_ml[base * 2 + 1] = sum; }
             }
         }
     }
@@ -464,8 +464,9 @@ __global__ __launch_bounds__(256) void attn_page_tile_kernel(AttnParams p) {
         *reinterpret_cast<f4 *>(p.part_o + base * ATT_D + 32 * wave + 16 * i + 4 * g) = o;
     }
     if (wave == 0 && g == 0) {
-        p.part_ml[base * 2] = mx;
-        p.part_ml[base * 2 + 1] = s_sum[0][c] + s_sum[1][c] + s_sum[2][c] + s_sum[3][c];
+        sum = s_sum[0][c] + s_sum[1][c] + s_sum[2][c] + s_sum[3][c];
+        p.part_ml[base * 2] = partial_max(mx, sum);
+        p.part_ml[base * 2 + 1] = sum;
     }
 }
 
@@ -1061,7 +1062,7 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
             const long base = ((long)p.splits * p.Hkv + hk) * p.Bq + qrow;
             st_f4(p.part_o + base * ATT_D + 4 * c, f4{st.o[0], st.o[2], st.o[1], st.o[3]});
             st_f4(p.part_o + base * ATT_D + 64 + 4 * c, f4{st.o[4], st.o[6], st.o[5], st.o[7]});
-            if (c == 0) { st_f32(p.part_ml + base * 2, st.m); st_f32(p.part_ml + base * 2 + 1, st.l); }
+            if (c == 0) { st_f32(p.part_ml + base * 2, partial_max(st.m, st.l)); st_f32(p.part_ml + base * 2 + 1, st.l); }
         } else if (g == 0 && sub == 0 && live) {
             const float inv = st.l > 0.f ? 1.0f / st.l : 0.f;
             half_t *op = p.out + ((long)b * p.H + h) * ATT_D;
@@ -1207,7 +1208,7 @@ __device__ __forceinline__ void attn_prefix_round(const AttnParams &p, int split
     const long base = ((long)split * p.Hkv + hk) * p.Bq + qrow;
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) *reinterpret_cast<f4 *>(p.part_o + base * ATT_D + 16 * dt + 4 * g) = ot[dt];
-    if (g == 0) { p.part_ml[base * 2] = mx; p.part_ml[base * 2 + 1] = sum; }
+    if (g == 0) { p.part_ml[base * 2] = partial_max(mx, sum); p.part_ml[base * 2 + 1] = sum; }
 }
 
 // prefix_wgs: a multiple of 8, so that the others sit on the XCDs that attn_suffix_kernel's would
@@ -1248,8 +1249,10 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p) {
         }
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-            float c1, c2;
-            m = soft_join(m, ml[i][0], c1, c2);
+            const float m_new = fmaxf(m, ml[i][0]);
+            if (m_new == -INFINITY) continue;                // nothing yet
+            const float c1 = exp2f(m - m_new), c2 = exp2f(ml[i][0] - m_new);
+            m = m_new;
             l = l * c1 + ml[i][1] * c2;
             o[0] = o[0] * c1 + v[i][0] * c2;
             o[1] = o[1] * c1 + v[i][1] * c2;
@@ -1331,11 +1334,14 @@ __global__ __launch_bounds__(256, 2) void attn_one_kernel(AttnParams p) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) o[j] = 0.f;
         auto fold = [&](float pm, float pl, const float (&po)[8]) {
-            float c1, c2;
-            m = soft_join(m, pm, c1, c2);
-            l = l * c1 + pl * c2;
+            const float m_new = fmaxf(m, pm);
+            if (m_new != -INFINITY) {
+                const float c1 = exp2f(m - m_new), c2 = exp2f(pm - m_new);
+                m = m_new;
+                l = l * c1 + pl * c2;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) o[j] = o[j] * c1 + po[j] * c2;
+                for (int j = 0; j < 8; ++j) o[j] = o[j] * c1 + po[j] * c2;
+            }
         };
         for (int s0 = si; live && s0 < n_part; s0 += 4 * sub) {
             f4 lo[4], hi[4];

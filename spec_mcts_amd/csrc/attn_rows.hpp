@@ -61,18 +61,15 @@ __device__ __forceinline__ void soft_add_row(SoftState &st, float score, const R
     st.o[6] = st.o[6] * corr + pr * (float)v.b13.x;
     st.o[7] = st.o[7] * corr + pr * (float)v.b13.y;
 }
-// The common maximum of two un-normalised partials and the factors that bring their sums to it.  Without a maximum in either (no
-// row yet, or nothing but NaN scores) both factors are 0, which leaves zeros zero and NaN NaN.
-__device__ __forceinline__ float soft_join(float m1, float m2, float &c1, float &c2) {
-    const float m = fmaxf(m1, m2), m_ref = m == -INFINITY ? 0.f : m;
-    c1 = exp2f(m1 - m_ref);
-    c2 = exp2f(m2 - m_ref);
-    return m;
-}
+// The maximum an un-normalised partial is handed on with.  -infinity: it holds no row, and whoever merges may pass it over.  Scores
+// that are all NaN have no maximum either, but a sum, which is NaN and has to arrive: the lowest finite number.
+__device__ __forceinline__ float partial_max(float m, float l) { return m == -INFINITY && !(l == 0.f) ? -3.402823466e38f : m; }
 // fold an un-normalised partial (m2, l2, o2) into st
 __device__ __forceinline__ void soft_merge(SoftState &st, float m2, float l2, const float *o2) {
-    float c1, c2;
-    st.m = soft_join(st.m, m2, c1, c2);
+    const float m_new = fmaxf(st.m, m2);
+    if (m_new == -INFINITY) return;                  // both empty
+    const float c1 = exp2f(st.m - m_new), c2 = exp2f(m2 - m_new);
+    st.m = m_new;
     st.l = st.l * c1 + l2 * c2;
 #pragma unroll
     for (int j = 0; j < 8; ++j) st.o[j] = st.o[j] * c1 + o2[j] * c2;
