@@ -14,8 +14,8 @@
 //     folds in the prefix partials and the new token, normalises and writes fp16.
 // With fp16 suffixes the slices and the walks are one launch and a merge follows (attn_parts_kernel); fp16 pages that neighbouring
 // branches share go through attn_page_tile_kernel before the walk.
-// Scores and softmax are fp32 throughout (exp2 of log2(e)-scaled scores); probabilities are rounded
-// to fp16 only as the operand of the P.V matrix product.
+// Scores and softmax are fp32 throughout (exp2 of log2(e)-scaled scores); probabilities are rounded to fp16 only as the operand of
+// the P.V matrix product of a shared prefix and of a prefill (walks and shared pages hold all their bits).
 //
 // Algorithmic HBM traffic: prefix 2*P*Hkv*D*2 B once + per branch its suffix rows
 // (512 B fp16 or 136 B Q4_0 per row and kv head) + q/out.
