@@ -440,6 +440,14 @@ typedef struct smh_pass {
 size_t smh_decode_scratch_bytes(const smh_layer *layer, int rows, int swiglu_in);
 int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stream_t stream);
 int smh_prefill_layer(const smh_layer *layer, smh_pass *pass, smh_stream_t stream);
+/* All layers of a decode step of a few branches in one launch (of up to 32 layers): what smh_decode_layer does layer by layer, with sums in
+ * another order.  smh_decode_stack_workspace_bytes: 0 where the sizes are not for it (1 .. 4 rows, as many kv heads as heads, widths that
+ * are multiples of 256, enough tiles for 256 workgroups).  ws: that many bytes, zero before the first call and left alone between
+ * calls (calls with other row counts may share it); calls that overlap need one each.  Of the pass it needs rows, the tables and
+ * counters, pages, scratch, h and pending (0).  The workgroups wait for one another, however many of them the GPU runs at a time; a wait
+ * of more than 5 seconds ends with NaN in h. */
+size_t smh_decode_stack_workspace_bytes(const smh_layer *layer, int rows);
+int smh_decode_stack(const smh_layer *const *layers, int n_layers, smh_pass *pass, void *ws, size_t ws_bytes, smh_stream_t stream);
 int smh_decode_finish(const smh_layer *last, smh_pass *pass, const void *norm_weight, float eps, void *out, smh_stream_t stream);
 
 #ifdef __cplusplus

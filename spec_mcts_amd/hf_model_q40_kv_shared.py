@@ -319,6 +319,8 @@ class Transformer(nn.Module):
         self.norm_in_max_rows = 2 if params.dim < 8192 else 16
         self._norm_in_ok = {}
         self.attn_from_qkv = True          # where the attention is one launch it takes the wq|wk|wv product itself
+        self.decode_stack = True           # up to 4 branches (multi-head attention): all layers of a decode step in one launch
+        self._stack_ws = None
         self._q40_output = None            # quantize_lm_head(): (w, s, padded vocab) of a Q4_0 vocabulary projection
         self.paged_kv = True               # fork = a copy of page ids: forked branches share their ancestor's suffix rows
         self._page_table = None            # int32 [max_batch_size, max_seq_len]: cache row that holds position j of branch b
@@ -443,10 +445,29 @@ class Transformer(nn.Module):
         norm_in = self._norm_in(B, p.dim, [lin._tiled for lin in (att0.wq, att0.wk, att0.wv)])      # (the library asks again, launch by launch)
         run.decode_step(step_state, ws, bool(one), p.max_seq_len, p.max_batch_size * p.max_seq_len, self._pages(dev), B if norm_in else 0,
                         K.SILU_IN_MAX_M if self.silu_in_matmul else 0, self.attn_from_qkv and not self.per_branch_kv)
-        for layer in self.layers:
-            s = self._layer_struct(layer)
-            run.decode(s)
+        structs = [self._layer_struct(layer) for layer in self.layers]
+        s = structs[-1]
+        stack_ws = self._stack_workspace(dev, structs[0], B)
+        if stack_ws is not None:
+            run.decode_stack(structs, stack_ws)
+        else:
+            for s in structs:
+                run.decode(s)
         return self._lm_head(run.finish(s, self.norm.weight, self.norm.eps).view(B, 1, p.dim))
+
+    def _stack_workspace(self, dev, first, B: int) -> Optional[torch.Tensor]:
+        """The workspace of a step whose layers are one launch, None where they are not.  The model's own, not the device's: its words belong
+        to one sequence of steps."""
+        if not (self.decode_stack and self.attn_single_launch and self.attn_from_qkv and self.norm_in_matmul and self.silu_in_matmul and not self.per_branch_kv):
+            return None
+        if K.decode_stack_bytes(first, B) == 0:
+            return None
+        if self._stack_ws is None or self._stack_ws.device != dev:
+            if torch.cuda.is_current_stream_capturing():        # (a graph's own memory is no place for what outlives its replay)
+                return None
+            # for every number of rows at once: a captured graph keeps its address
+            self._stack_ws = torch.zeros(max(K.decode_stack_bytes(first, r) for r in range(1, K.DECODE_STACK_MAX_ROWS + 1)), dtype=torch.uint8, device=dev)
+        return self._stack_ws
 
     def _prefill(self, tokens: torch.Tensor) -> torch.Tensor:
         """The prefill of one prompt on tiled weights, a layer per library call (smh_prefill_layer): its k and v become the rows

@@ -9,6 +9,7 @@ must live on the GPU and the library must be built.
 """
 from __future__ import annotations
 
+import ctypes
 import math
 from typing import Dict, Optional, Sequence, Tuple
 
@@ -675,6 +676,14 @@ def layer_struct(dim: int, H: int, Hkv: int, att_norm: torch.Tensor, att_eps: fl
     return s
 
 
+DECODE_STACK_MAX_ROWS = 4                      # csrc/decode_stack.hip
+
+
+def decode_stack_bytes(first: "_lib.SmhLayer", rows: int) -> int:
+    """Workspace of LayerPass.decode_stack, 0 where it is not for these sizes."""
+    return int(_lib.load().smh_decode_stack_workspace_bytes(first, rows))
+
+
 class LayerPass:
     """One pass over all layers (smh_pass): a decode step over `rows` branches (after decode_step()) or the prefill of a prompt
     of `rows` tokens.  decode(struct) or prefill(struct) per layer, then finish() for the last residual add and the final RMSNorm.
@@ -718,6 +727,11 @@ class LayerPass:
         st = self.lib.smh_decode_layer(s, self.p, self.stream)
         if st:
             check(st, "smh_decode_layer")
+
+    def decode_stack(self, structs: Sequence["_lib.SmhLayer"], ws: torch.Tensor) -> None:
+        """All layers in one launch (decode_stack_bytes() > 0)."""
+        arr = (ctypes.POINTER(_lib.SmhLayer) * len(structs))(*[ctypes.pointer(s) for s in structs])
+        check(self.lib.smh_decode_stack(arr, len(structs), self.p, ws.data_ptr(), ws.numel(), self.stream), "smh_decode_stack")
 
     def prefill(self, s: "_lib.SmhLayer") -> None:
         st = self.lib.smh_prefill_layer(s, self.p, self.stream)

@@ -1,0 +1,86 @@
+"""All layers of a decode step of a few branches in one launch (smh_decode_stack), against the oracle's dense restatement and
+the layer-by-layer launches."""
+import ctypes
+
+import pytest
+import torch
+
+from oracle import q40_oracle as O
+from tests.sync_state import sync_prefix, sync_suffix_row
+
+# layers, dim, ffn columns / 256 -> where it can go wrong
+CASES = [
+    (dict(dim=256, n_layers=33, n_heads=2), 1, 1, 3),       # more layers than a launch holds; runs of two tiles, most workgroups without any
+    (dict(dim=512, n_layers=2, n_heads=4), 2, 33, 4),       # two slices of the prompt, the second of one row
+    (dict(dim=1024, n_layers=2, n_heads=8), 3, 131, 3),     # runs that touch two column units
+    (dict(dim=1280, n_layers=1, n_heads=10), 4, 70, 3),     # the most rows; units that no number of equal runs divides
+    (dict(dim=2048, n_layers=1, n_heads=16), 1, 300, 30),   # more own rows than the attention's waves take at once
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,B,P,steps", CASES)
+def test_stack_matches_the_oracle(shape, B, P, steps, monkeypatch):
+    from spec_mcts_amd import ModelArgs, kernels as K
+    from spec_mcts_amd.load_q40 import load_q40
+    cfg = dict(shape, vocab_size=320, multiple_of=256, max_batch_size=5, max_seq_len=steps + 2, max_prompt_seq_len=320)
+    std = 0.8 / shape["dim"] ** 0.5
+    oargs = O.OracleArgs(**cfg)
+    sd = O.random_q40_state_dict(oargs, seed=B + P, std=std)
+    model = load_q40(dict(sd), ModelArgs(**cfg), device="cuda:0")
+    oracle = O.OracleTransformer(oargs, sd, dense=True)
+    calls = []
+    monkeypatch.setattr(K.LayerPass, "decode_stack", lambda self, structs, ws, _f=K.LayerPass.decode_stack: (calls.append(len(structs)), _f(self, structs, ws)))
+    gen = torch.Generator().manual_seed(P)
+    prompt = torch.randint(0, cfg["vocab_size"], (1, P), generator=gen)
+    oracle.forward(prompt, 0)
+    model(prompt.cuda(), 0)
+    sync_prefix(model, oracle)
+    for step in range(steps):
+        tok = torch.randint(0, cfg["vocab_size"], (B, 1), generator=gen)
+        want = oracle.forward(tok, P + step).float()
+        got = model(tok.cuda(), P + step)
+        assert calls.pop() == cfg["n_layers"]
+        model.decode_stack = False
+        layers = model(tok.cuda(), P + step).float().cpu()
+        model.decode_stack = True
+        again = model(tok.cuda(), P + step)
+        calls.clear()
+        assert torch.equal(got, again), "the order of the sums depends on nothing but the sizes"
+        got = got.float().cpu()
+        # Both round to fp16 at the same points and differ from the oracle in the order of fp32 sums alone, so by flipped roundings that
+        # add up over the layers: as far from the oracle as the layers' launches are, with room for the flips that fall the other way.
+        far, near = float((got - want).norm() / want.norm()), float((layers - want).norm() / want.norm())
+        print("step %d: from the oracle %.2e, layer by layer %.2e" % (step, far, near))
+        assert far <= 2 * near + 2e-3
+        sync_suffix_row(model, oracle, B, step)
+    # a fork: the branches share their ancestor's rows through the page table
+    model.fork(0, B, 1)
+    tok = tok[:1].expand(B + 1, 1).cuda()
+    if B < K.DECODE_STACK_MAX_ROWS:
+        got = model(tok, P + steps)
+        assert calls and torch.equal(got[0], got[B])
+
+
+def test_refused_sizes_and_arguments():
+    """No workspace, and an error instead of a launch, for what the kernel is not made for (no GPU needed)."""
+    from spec_mcts_amd import _lib
+    lib = _lib.load()
+
+    def layer(dim, heads, kv_heads, ffn, P=7):
+        s = _lib.SmhLayer()
+        s.dim, s.heads, s.kv_heads, s.ffn, s.prompt_len = dim, heads, kv_heads, ffn, P
+        return s
+
+    for rows in (1, 2, 3, 4):
+        for dim, heads, ffn in ((4096, 32, 11008), (5120, 40, 13824), (256, 2, 768)):
+            assert lib.smh_decode_stack_workspace_bytes(layer(dim, heads, heads, ffn), rows) > 0
+    for rows, s in ((0, layer(4096, 32, 32, 11008)), (5, layer(4096, 32, 32, 11008)), (1, layer(8192, 64, 8, 28672)), (1, layer(4096, 32, 32, 11008 + 32)),
+                    (1, layer(4096 + 128, 33, 33, 11008)), (1, layer(128, 1, 1, 256)), (1, layer(256, 0, 0, 256))):
+        assert lib.smh_decode_stack_workspace_bytes(s, rows) == 0
+        p = _lib.SmhPass()
+        p.rows, p.smax = rows, 8
+        for field in ("h", "pos_dev", "t_dev", "cos_tab", "sin_tab", "scratch"):
+            setattr(p, field, 256)                     # (never read: the sizes are refused first)
+        arr = (ctypes.POINTER(_lib.SmhLayer) * 1)(ctypes.pointer(s))
+        assert lib.smh_decode_stack(arr, 1, p, 256, 1 << 30, None) != 0
