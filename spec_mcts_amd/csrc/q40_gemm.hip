@@ -1081,6 +1081,204 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_swiglu_kernel(MatmulParams p)
     }
 }
 
+// ---- SwiGLU above 128 rows, three pieces a workgroup (tiled weights, all of K, one workgroup per compute unit) ----------------
+// q40_gemm_kernel<.., SWIGLU> with half as many columns again: pieces 3 u .. 3 u + 2 (64 columns each) of the gate weight and the
+// same of the up weight, 64 .. 128 rows of A, twelve multiplying waves - wave (nibble hh, slot s) has one piece's columns of one
+// nibble, two B operands, as there - and the DMA wave.  Bound by the matrix and vector pipes, which a third wave on each SIMD keeps
+// busier (0.55 us a step of 128 rows x 384 columns, where 1.5 steps of the 256-column units take 0.63), and by how well its workgroups
+// divide the compute units: 512 rows of the 7B shape are 232 of them, one round, where the 256-column units leave 344, two
+// rounds.  4096 -> 2 x 11008, before and now: 512 rows 112.9 us (818 TFLOP/s) and 90.1 (1025), 300 rows 85.3 and 65.2, 1024 rows 201
+// and 178, 2047 rows 375 (985) and 353 (1047); 8192 -> 2 x 28672 at 640 rows 609 and 515, 2047 rows 1834 and 1693.
+// A's rows lie in LDS with the chunk XOR (row / 2) % 4, which reads faster here: twelve waves ask for 96 KB a step.
+template <int TILES> struct WideShape {
+    static constexpr int W = 6 * 1024, SC = 6 * 128;             // [gate 0 .. 2 | up 0 .. 2]: nibbles; scales [octet][nibble][8 rows]
+    static constexpr int STAGE = W + SC + TILES * 1024;
+    static constexpr int SLOTS = 6;
+    static constexpr int LDS = SLOTS * STAGE;
+    static constexpr int PER = 9 + TILES;                        // DMA instructions of a stage
+    static constexpr int OP = 192 + 4;
+    static constexpr int OTILE = 2 * 16 * OP * 4;                // [gate | up][16][OP] fp32
+    static_assert(2 * OTILE <= LDS && LDS <= 160 * 1024, "two output tiles in the ring");
+};
+constexpr int WIDE_WAVES = 12;
+
+template <int TILES>
+__global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_swiglu_wide_kernel(MatmulParams p) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    typedef WideShape<TILES> S;
+    constexpr int SLOTS = S::SLOTS, PER = S::PER, STAGE = S::STAGE;
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63, c = lane & 15, g = lane >> 4;
+    // blockIdx -> (unit of three pieces, row block): each XCD takes a contiguous run of units
+    const int at = blockIdx.x % p.units_pad, mb = blockIdx.x / p.units_pad;
+    const int unit = (at & 7) * (p.units_pad >> 3) + (at >> 3);
+    if (unit >= p.units) return;
+    const int m0 = mb * p.block_rows, pieces = p.seg[0].N / 64;
+    const long tiles_per_pair = tiled_steps(p.K);
+    const int n_steps = p.K / 32;
+    const int rot = (unit * 5) % n_steps;                              // workgroups of a row block start at different steps
+    auto piece_of = [&](int k) { return min(3 * unit + k, pieces - 1); };      // (past the end: the last one again, not stored)
+
+    if (wave == WIDE_WAVES) {
+        // ---- the DMA wave ----
+        __builtin_amdgcn_s_setprio(3);
+        const int a_chunk = (lane & 3) ^ ((lane >> 3) & 3);
+        uint32_t a_voff[TILES];
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) a_voff[t] = (uint32_t)((long)min(m0 + 16 * t + (lane >> 2), p.M - 1) * p.lda * 2 + 16 * a_chunk);
+        const uint8_t *w[6], *sc[3];
+#pragma unroll
+        for (int s = 0; s < 6; ++s) {
+            const int P = piece_of(s % 3);
+            w[s] = p.seg[s / 3].w + (long)(P >> 2) * tiles_per_pair * TILE_BYTES + (P & 3) * 1024;
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {                                  // lanes 0 .. 31: slot 2 i's 128 bytes, the others slot 2 i + 1's
+            const int s = 2 * i + (lane >> 5), P = piece_of(s % 3), d = lane & 31;
+            sc[i] = (s < 3 ? p.seg[0].w : p.seg[1].w) + (long)(P >> 2) * tiles_per_pair * TILE_BYTES + TILE_W_BYTES + (d >> 3) * 64 + ((P & 3) >> 1) * 32 + (d & 7) * 4;
+        }
+        const uint8_t *a_base = reinterpret_cast<const uint8_t *>(p.a);
+        int fetch = rot;
+        auto issue_stage = [&](int slot_) {
+            uint8_t *st = lds + slot_ * STAGE;
+            const long off = (long)fetch * TILE_BYTES;
+            const uint8_t *arow = a_base + (long)fetch * 64;
+#pragma unroll
+            for (int s = 0; s < 6; ++s) __builtin_amdgcn_global_load_lds((gptr_t)(w[s] + off + lane * 16), (lptr_t)(st + s * 1024), 16, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 3; ++i) __builtin_amdgcn_global_load_lds((gptr_t)(sc[i] + off), (lptr_t)(st + S::W + i * 256), 4, 0, 0);
+#pragma unroll
+            for (int t = 0; t < TILES; ++t) __builtin_amdgcn_global_load_lds((gptr_t)(arow + a_voff[t]), (lptr_t)(st + S::W + S::SC + t * 1024), 16, 0, 0);
+            fetch = fetch + 1 == n_steps ? 0 : fetch + 1;
+        };
+#pragma unroll
+        for (int i = 0; i < SLOTS - 2; ++i)
+            if (i < n_steps) issue_stage(i);
+        gemm_wait_dma<PER>(min(SLOTS - 3, n_steps - 1));
+        gemm_barrier();
+        int slot = 0;
+        auto back = [&](int k) { return slot >= k ? slot - k : slot + SLOTS - k; };
+        int i = 0;
+#pragma unroll 1
+        for (; i + SLOTS - 1 < n_steps; i += 2) {
+            gemm_wait_vm<PER * (SLOTS - 5)>();
+            gemm_barrier();
+            issue_stage(back(2));
+            issue_stage(back(1));
+            slot = slot + 2 >= SLOTS ? slot + 2 - SLOTS : slot + 2;
+        }
+#pragma unroll 1
+        for (; i < n_steps; i += 2) {
+            gemm_wait_dma<PER>(max(0, min(n_steps - 1, i + SLOTS - 3) - (i + 2)));
+            gemm_barrier();
+            if (i + SLOTS - 2 < n_steps) issue_stage(back(2));
+            if (i + SLOTS - 1 < n_steps) issue_stage(back(1));
+            slot = slot + 2 >= SLOTS ? slot + 2 - SLOTS : slot + 2;
+        }
+        // the barriers of the epilogue: ring free, one per row tile
+#pragma unroll 1
+        for (int t = 0; t < 1 + TILES; ++t) gemm_barrier();
+        return;
+    }
+
+    const int hh = wave >= 6 ? 1 : 0, s = wave - 6 * hh, gu = s >= 3 ? 1 : 0, k3 = s - 3 * gu;       // nibble, slot, gate (0) or up (1), piece
+    const uint32_t nib_mask = hh == 0 ? 0x00F000F0u : 0x000F000Fu;
+    uint32_t nib_magic = MAGIC_1024;                             // (as in q40_gemm_swiglu_kernel)
+    asm volatile("" : "+v"(nib_magic));
+    const h2 nib_mul = hh == 0 ? h2{(half_t)0.0625f, (half_t)0.0625f} : h2{(half_t)1.0f, (half_t)1.0f};
+    const h2 nib_off = hh == 0 ? h2{(half_t)-72.0f, (half_t)-72.0f} : h2{(half_t)-1032.0f, (half_t)-1032.0f};
+    struct Raw { u32x4 wq, sc; };
+    const int ws_off = s * 1024 + lane * 16, sc_off = S::W + s * 128 + g * 32 + hh * 16, a_off = S::W + S::SC + c * 64 + ((g ^ ((c >> 1) & 3)) << 4);
+    auto load_ws = [&](const uint8_t *st, Raw &r) {
+        r.wq = *reinterpret_cast<const u32x4 *>(st + ws_off);
+        r.sc = *reinterpret_cast<const u32x4 *>(st + sc_off);
+    };
+    auto decode = [&](const Raw &r, h8 (&b)[2]) {
+        u32x4 v0, v1;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t pr0 = j < 2 ? r.wq[j] : r.wq[j - 2] >> 8;       // rows (2j, 2j+1) of byte 2bp, codes + 8
+            const uint32_t pr1 = j < 2 ? r.wq[2 + j] : r.wq[j] >> 8;       // ... of byte 2bp+1
+            const h2 sc = as_h2(r.sc[j]);
+            v0[j] = as_u32(__builtin_elementwise_fma(as_h2((pr0 & nib_mask) | nib_magic), nib_mul, nib_off) * sc);
+            v1[j] = as_u32(__builtin_elementwise_fma(as_h2((pr1 & nib_mask) | nib_magic), nib_mul, nib_off) * sc);
+        }
+        b[0] = __builtin_bit_cast(h8, v0);
+        b[1] = __builtin_bit_cast(h8, v1);
+    };
+    f4 acc[2][TILES];
+#pragma unroll
+    for (int o = 0; o < 2; ++o)
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) acc[o][t] = f4{0.f, 0.f, 0.f, 0.f};
+
+    h8 bq[2];
+    int slot = 0;
+    gemm_barrier();
+    {
+        Raw r;
+        load_ws(lds, r);
+        decode(r, bq);
+    }
+    auto one_step = [&]() {
+        const uint8_t *st = lds + slot * STAGE;
+        slot = slot == SLOTS - 1 ? 0 : slot + 1;
+        Raw r;
+        h8 av[TILES], bn[2];
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) av[t] = *reinterpret_cast<const h8 *>(st + a_off + t * 1024);
+        load_ws(lds + slot * STAGE, r);                        // (past the last step: stale bytes, decoded and never used)
+#pragma unroll
+        for (int t = 0; t < TILES; ++t)
+#pragma unroll
+            for (int o = 0; o < 2; ++o) acc[o][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[t], bq[o], acc[o][t], 0, 0, 0);
+        decode(r, bn);
+        bq[0] = bn[0];
+        bq[1] = bn[1];
+    };
+    int i = 0;
+#pragma unroll 1
+    for (; i + 1 < n_steps; i += 2) {
+        gemm_barrier();
+        one_step();
+        one_step();
+    }
+    if (i < n_steps) {
+        gemm_barrier();
+        one_step();
+    }
+
+    // rows of 192 columns: local column 64 k3 + 32 hh + 2 c + o is column 128 (P / 2) + 64 hh + 4 c + 2 (P % 2) + o, P the piece
+    constexpr int OP = S::OP;
+    const int o_row = tid / 48, o_lane = tid % 48, P = 3 * unit + (o_lane >> 4), q = o_lane & 15;
+    const bool mine = P < pieces;
+    const int out_col = 128 * (P >> 1) + 64 * (q >> 3) + 8 * (q & 7) + 2 * (P & 1);
+    gemm_barrier();                                            // every wave has left the loop: the ring is free
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+        float *otile = reinterpret_cast<float *>(lds + (t & 1) * S::OTILE);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            *reinterpret_cast<f2 *>(&otile[gu * 16 * OP + (4 * g + r) * OP + 64 * k3 + 32 * hh + 2 * c]) = f2{acc[0][t][r], acc[1][t][r]};
+        gemm_barrier();
+        const int m = m0 + 16 * t + o_row;
+        if (m < p.M && mine) {
+            const f4 gv = *reinterpret_cast<const f4 *>(otile + o_row * OP + 4 * o_lane);
+            const f4 uv = *reinterpret_cast<const f4 *>(otile + 16 * OP + o_row * OP + 4 * o_lane);
+            half_t ov[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {                      // the roundings of partial_silu_mul_kernel
+                const float gf = (float)(half_t)gv[e];
+                ov[e] = (half_t)(gf / (1.0f + expf(-gf))) * (half_t)uv[e];
+            }
+            half_t *dst = p.seg[0].c + (long)m * p.seg[0].ldc + out_col;
+            *reinterpret_cast<h2 *>(dst) = h2{ov[0], ov[1]};
+            *reinterpret_cast<h2 *>(dst + 4) = h2{ov[2], ov[3]};
+        }
+    }
+}
+
 // Row blocks and K-slices of a launch with more than 128 rows: the pair with the least estimated time.  Measured on the 7B shapes
 // at 160 .. 2047 rows: a workgroup takes 0.18 us a step and 0.24 more at 128 rows (in proportion), 4 us around its loop; a launch
 // takes as many of these as the workgroups of the busiest XCD need rounds over its 32 compute units (whole column units go to an
@@ -1092,11 +1290,17 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_swiglu_kernel(MatmulParams p)
 // 128 us, now 77, 5120 x 13824 at 512 rows 138, now 101.)
 // Against measurement at the 7B, 13B, 34B and 70B shapes, 160 .. 2047 rows: 0.87 to 1.17 times the estimate, 1.3 to 1.4 times it
 // for square weights at 160 rows (15 and 19 us: launches).
-static float gemm_rows_us(int units, long of_unit, int rows, int steps) {
+struct RowsCost { float step, per_rows, around, busy; };       // us a step, us more a step at 128 rows, us around the loop, and that factor
+constexpr RowsCost ROWS_256 = {0.18f, 0.24f, 4.0f, 1.2f};
+// SwiGLU with three pieces a workgroup (384 columns): fitted to the shapes of 7B, 13B, 34B and 70B at 130 .. 2047 rows, within 4 % in
+// the mean.  Taking it where its estimate is the smaller was never slower there than the 256-column units (0.72 .. 0.99 of their time).
+constexpr RowsCost ROWS_384 = {0.21f, 0.37f, 4.0f, 1.15f};
+static float gemm_rows_us(const RowsCost &t, int units, long of_unit, int rows, int steps) {
     const float r = (float)(units * of_unit) / 256.0f, rounds = (float)(((units + 7) / 8 * of_unit + 31) / 32);
-    return (rounds > 1.2f * r ? rounds : 1.2f * r) * ((float)steps * (0.18f + 0.24f * rows / GEMM_BM) + 4.0f);
+    return (rounds > t.busy * r ? rounds : t.busy * r) * ((float)steps * (t.step + t.per_rows * rows / GEMM_BM) + t.around);
 }
-static void gemm_plan_rows(MatmulParams &p, int steps, int max_ks) {
+// (p.units on entry; returns the estimate)
+static float gemm_plan_rows(MatmulParams &p, int steps, int max_ks, const RowsCost &cost) {
     float best_us = -1.0f;
     int ksplit = 1;
     for (int mb = (p.M + GEMM_BM - 1) / GEMM_BM; mb <= p.M / 64; ++mb) {                // (blocks of 64 .. 128 rows)
@@ -1104,7 +1308,7 @@ static void gemm_plan_rows(MatmulParams &p, int steps, int max_ks) {
         const int blocks = (p.M + rows - 1) / rows;
         const long tiles = (long)p.units * blocks;
         for (int ks = 1; ks <= max_ks && (ks == 1 || (tiles * ks <= 512 && steps / ks >= GEMM_STAGES)); ++ks) {
-            const float us = gemm_rows_us(p.units, (long)blocks * ks, rows, (steps + ks - 1) / ks) + (ks > 1 ? (float)ks * p.M * p.n_total * 4.0f / 4.0e6f : 0.0f);
+            const float us = gemm_rows_us(cost, p.units, (long)blocks * ks, rows, (steps + ks - 1) / ks) + (ks > 1 ? (float)ks * p.M * p.n_total * 4.0f / 4.0e6f : 0.0f);
             if (best_us < 0.0f || us < best_us) {
                 best_us = us;
                 ksplit = ks;
@@ -1116,6 +1320,7 @@ static void gemm_plan_rows(MatmulParams &p, int steps, int max_ks) {
     p.steps_per_slice = (steps + ksplit - 1) / ksplit;
     p.ksplit = (steps + p.steps_per_slice - 1) / p.steps_per_slice;
     p.chunk = 0;
+    return best_us;
 }
 
 void gemm_fill_plan(MatmulParams &p) {
@@ -1170,7 +1375,7 @@ void gemm_fill_plan(MatmulParams &p) {
     p.mblocks = (p.M + p.block_rows - 1) / p.block_rows;
     const int steps = (p.K + 31) / 32;
     if (p.M > GEMM_BM) {
-        gemm_plan_rows(p, steps, SMH_MAX_KSPLIT);
+        gemm_plan_rows(p, steps, SMH_MAX_KSPLIT, ROWS_256);
         return;
     }
     const long tiles = (long)p.units * p.mblocks;
@@ -1352,10 +1557,14 @@ int gemm_swiglu_rows_launch(MatmulParams p, hipStream_t stream) {
                                            q40_gemm_kernel<7, false, true, 8, GEMM_STAGES, false, false, true>, q40_gemm_kernel<8, false, true, 8, GEMM_STAGES, false, false, true>};
     static const gemm_kernel_t dma_wave[5] = {q40_gemm_kernel<4, false, true, 8, gemm_dma_slots(4), true, false, true>, q40_gemm_kernel<5, false, true, 8, gemm_dma_slots(5), true, false, true>, q40_gemm_kernel<6, false, true, 8, gemm_dma_slots(6), true, false, true>,
                                               q40_gemm_kernel<7, false, true, 8, gemm_dma_slots(7), true, false, true>, q40_gemm_kernel<8, false, true, 8, gemm_dma_slots(8), true, false, true>};
+    static const gemm_kernel_t wide[5] = {q40_gemm_swiglu_wide_kernel<4>, q40_gemm_swiglu_wide_kernel<5>, q40_gemm_swiglu_wide_kernel<6>,
+                                          q40_gemm_swiglu_wide_kernel<7>, q40_gemm_swiglu_wide_kernel<8>};
+    static const int wide_lds[5] = {WideShape<4>::LDS, WideShape<5>::LDS, WideShape<6>::LDS, WideShape<7>::LDS, WideShape<8>::LDS};
     static const hipError_t lds_ok = [] {
         hipError_t e = hipSuccess;
         for (int t = 0; t < 5 && e == hipSuccess; ++t) {
-            e = hipFuncSetAttribute((const void *)plain[t], hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS);
+            e = hipFuncSetAttribute((const void *)wide[t], hipFuncAttributeMaxDynamicSharedMemorySize, wide_lds[t]);
+            if (e == hipSuccess) e = hipFuncSetAttribute((const void *)plain[t], hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS);
             if (e == hipSuccess) e = hipFuncSetAttribute((const void *)dma_wave[t], hipFuncAttributeMaxDynamicSharedMemorySize, gemm_dma_slots(t + 4) * GS_BYTES);
         }
         return e;
@@ -1365,10 +1574,18 @@ int gemm_swiglu_rows_launch(MatmulParams p, hipStream_t stream) {
         return (int)lds_ok;
     }
     SMH_REQUIRE((long)p.M * p.lda * 2 < (1L << 32), "q40 gemm: M x lda = %d x %ld exceeds the 32-bit lane offsets of A", p.M, p.lda);
+    p.kgroups = 0;
+    MatmulParams w = p;
     p.units = p.seg[0].N / 128;
     p.units_pad = (p.units + 7) / 8 * 8;
-    p.kgroups = 0;
-    gemm_plan_rows(p, p.K / 32, 1);
+    w.units = (p.seg[0].N / 64 + 2) / 3;
+    w.units_pad = (w.units + 7) / 8 * 8;
+    const float narrow_us = gemm_plan_rows(p, p.K / 32, 1, ROWS_256);
+    if (gemm_plan_rows(w, p.K / 32, 1, ROWS_384) < narrow_us) {
+        const int t = w.block_rows / 16 - 4;
+        hipLaunchKernelGGL(wide[t], dim3((unsigned)((long)w.units_pad * w.mblocks)), dim3(64 * (WIDE_WAVES + 1)), wide_lds[t], stream, w);
+        return launch_status();
+    }
     const bool one_each = (long)p.units * p.mblocks <= GEMM_DMA_WAVE_MAX_WGS;
     const int t = p.block_rows / 16 - 4;
     hipLaunchKernelGGL((one_each ? dma_wave : plain)[t], dim3((unsigned)((long)p.units_pad * p.mblocks)), dim3(512 + (one_each ? 64 : 0)),

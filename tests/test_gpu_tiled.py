@@ -288,6 +288,23 @@ def test_swiglu_inside_the_gate_up_launch_above_128_rows(M, K, n_half):
     assert torch.allclose(got.float(), want.float(), rtol=1e-2, atol=2e-3)
 
 
+@pytest.mark.parametrize("M,K,n_half", [(257, 32, 11008),       # one step; six row tiles, the last block of 65 rows; a last workgroup of one piece of three
+                                        (300, 96, 11264),       # three steps; seven row tiles; a last workgroup of two pieces
+                                        (352, 256, 11136),      # eight steps, more than the ring holds; eight row tiles; three pieces throughout
+                                        (130, 160, 22016),      # five steps; five row tiles
+                                        (256, 4096, 11008)])    # four row tiles
+def test_swiglu_three_pieces_a_workgroup(M, K, n_half):
+    """sizes that q40_gemm_swiglu_wide_kernel takes (its estimate is the smaller one), against the oracle's two matmuls"""
+    import torch.nn.functional as F
+    from spec_mcts_amd import kernels as Kn
+    w1, w3 = _weight(K, n_half, 1990 + K), _weight(K, n_half, 1991 + K)
+    x = (torch.randn((M, K), generator=torch.Generator().manual_seed(1992 + M)) * 0.5).half()
+    got = Kn.matmul_q40_swiglu(x.cuda(), Kn.tile_q40(w1[0].cuda(), w1[1].cuda(), K, n_half), Kn.tile_q40(w3[0].cuda(), w3[1].cuda(), K, n_half)).cpu()
+    want = F.silu(O.matmul_q40(x, w1[0], w1[1], (K, n_half)).float()).half() * O.matmul_q40(x, w3[0], w3[1], (K, n_half))
+    # gate, up, silu and the product round to fp16 (2^-11 each, and once more where a sum in another order falls the other way): 5e-3
+    assert torch.allclose(got.float(), want.float(), rtol=5e-3, atol=2e-3)
+
+
 @pytest.mark.parametrize("M,K,ns", [(129, 256, [16384, 128, 384]), (300, 64, [128]), (2047, 512, [2048]), (700, 4096, [11008])])
 def test_direct_products(M, K, ns):
     """launches without a K-split that store fp16 themselves: outputs per weight, a residual, rows past the last block's end"""
