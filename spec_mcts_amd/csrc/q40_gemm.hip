@@ -13,8 +13,7 @@
 //     the value the reference's dequantiser produces, born in the B-operand layout of
 //     v_mfma_f32_16x16x32_f16, so dequantised weights never travel through LDS or HBM;
 //   * it multiplies its four B operands (2 byte positions x high / low nibbles = columns c and c+64)
-//     with all TILES 16-row tiles of A, read from LDS with an XOR swizzle that keeps ds_read_b128
-//     conflict-free: one read of the A tile feeds four MFMAs;
+//     with all TILES 16-row tiles of A, read from LDS through an XOR swizzle (GS_A): one read of the A tile feeds four MFMAs;
 //   * the step is software-pipelined inside the wave: while the matrix pipe works through step i,
 //     the vector ALU decodes the B operands of step i+1 (one basic block, no branches: the number of
 //     row tiles and the ragged-K handling are template parameters), and the DMA addresses are a
@@ -52,7 +51,10 @@ constexpr int GS_WBLOCK = 8 * 128 + 64;        // the 8 rows one wave fetches, p
                                                // ds_read_b32 touches (lanes 16g..16g+15 read row 8g+r) then sit in different banks
 constexpr int GS_W = 4 * GS_WBLOCK;            // nibbles
 constexpr int GS_S = 32 * 8;                   // scales
-constexpr int GS_A = GEMM_BM * 64;             // A tile, 64 B per row, 16-byte chunks XOR-swizzled
+// A tile, 64 B per row; the 16-byte chunk k of row r lies at k ^ ((r / 2) % 4): a wave's 16 rows x 64 B by k-octet then reach 480 - 520 GB/s
+// a compute unit, with (r / 4) % 4 280 - 295.  (In turn: eight steps of 100 branches 33.67 -> 32.98 ms, prefill of 512 rows 9.44 -> 9.35 ms,
+// of 2047 rows 31.16 -> 30.86, 100 x 11008 x 4096 25.7 -> 25.3 us.)
+constexpr int GS_A = GEMM_BM * 64;
 constexpr int GS_BYTES = GS_W + GS_S + GS_A;               // 12800
 constexpr int GEMM_LDS = GEMM_STAGES * GS_BYTES;           // 76800
 constexpr int GEMM_COLS = 256;
@@ -143,7 +145,7 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
     const uint8_t *a_base = reinterpret_cast<const uint8_t *>(p.a);
     const int w_lrow = 8 * wave + (lane >> 3), w_lcol = 16 * (two_blocks ? (lane & 7) : (lane & 3));
     const int s_lrow = 8 * wave + ((lane & 15) >> 1), s_lcol = 4 * (two_blocks ? (lane & 1) : 0);
-    const int a_chunk = (lane & 3) ^ ((lane >> 4) & 3);                   // logical 16-byte chunk stored in slot lane&3
+    const int a_chunk = (lane & 3) ^ ((lane >> 3) & 3);                   // logical 16-byte chunk stored in slot lane&3
     const long a_r0 = (long)min(m0 + (WAVES == 8 ? 16 * wave8 : 32 * wave) + (lane >> 2), p.M - 1) * p.lda * 2;
     const long a_r1 = (long)min(m0 + 32 * wave + 16 + (lane >> 2), p.M - 1) * p.lda * 2;
     const uint32_t w_voff = (uint32_t)(w_lrow * w_row + w_lcol);
@@ -410,7 +412,7 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
             const int r = 16 * t + c;
-            av[t] = *reinterpret_cast<const h8 *>(at + r * 64 + ((g ^ ((r >> 2) & 3)) << 4));
+            av[t] = *reinterpret_cast<const h8 *>(at + r * 64 + ((g ^ ((r >> 1) & 3)) << 4));
         }
     };
     auto multiply = [&](const h8 (&av)[TILES], const h8 (&b)[NB]) {
@@ -701,7 +703,7 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_kg_kernel(MatmulParams p) {
     if (wave8 == 8) {
         // ---- the DMA wave ----
         __builtin_amdgcn_s_setprio(3);
-        const int a_chunk = (lane & 3) ^ ((lane >> 4) & 3);
+        const int a_chunk = (lane & 3) ^ ((lane >> 3) & 3);
         uint32_t a_voff[TILES];
 #pragma unroll
         for (int t = 0; t < TILES; ++t)
@@ -783,7 +785,7 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_kg_kernel(MatmulParams p) {
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
             const int r = 16 * t + c;
-            av[t] = *reinterpret_cast<const h8 *>(at + r * 64 + ((g ^ ((r >> 2) & 3)) << 4));
+            av[t] = *reinterpret_cast<const h8 *>(at + r * 64 + ((g ^ ((r >> 1) & 3)) << 4));
         }
     };
     f4 acc[2][TILES];
@@ -899,7 +901,7 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_swiglu_kernel(MatmulParams p)
     if (wave8 == 8) {
         // ---- the DMA wave ----
         __builtin_amdgcn_s_setprio(3);
-        const int a_chunk = (lane & 3) ^ ((lane >> 4) & 3);
+        const int a_chunk = (lane & 3) ^ ((lane >> 3) & 3);
         uint32_t a_voff[TILES];
 #pragma unroll
         for (int t = 0; t < TILES; ++t)
@@ -984,7 +986,7 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_swiglu_kernel(MatmulParams p)
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
             const int r = 16 * t + c;
-            av[t] = *reinterpret_cast<const h8 *>(at + r * 64 + ((g ^ ((r >> 2) & 3)) << 4));
+            av[t] = *reinterpret_cast<const h8 *>(at + r * 64 + ((g ^ ((r >> 1) & 3)) << 4));
         }
     };
     f4 acc[2][TILES];
@@ -1089,7 +1091,6 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_swiglu_kernel(MatmulParams p)
 // divide the compute units: 512 rows of the 7B shape are 232 of them, one round, where the 256-column units leave 344, two
 // rounds.  4096 -> 2 x 11008, before and now: 512 rows 112.9 us (818 TFLOP/s) and 90.1 (1025), 300 rows 85.3 and 65.2, 1024 rows 201
 // and 178, 2047 rows 375 (985) and 353 (1047); 8192 -> 2 x 28672 at 640 rows 609 and 515, 2047 rows 1834 and 1693.
-// A's rows lie in LDS with the chunk XOR (row / 2) % 4, which reads faster here: twelve waves ask for 96 KB a step.
 template <int TILES> struct WideShape {
     static constexpr int W = 6 * 1024, SC = 6 * 128;             // [gate 0 .. 2 | up 0 .. 2]: nibbles; scales [octet][nibble][8 rows]
     static constexpr int STAGE = W + SC + TILES * 1024;
