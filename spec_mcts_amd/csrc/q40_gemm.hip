@@ -1083,31 +1083,38 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_swiglu_kernel(MatmulParams p)
     }
 }
 
-// ---- SwiGLU above 128 rows, three pieces a workgroup (tiled weights, all of K, one workgroup per compute unit) ----------------
-// q40_gemm_kernel<.., SWIGLU> with half as many columns again: pieces 3 u .. 3 u + 2 (64 columns each) of the gate weight and the
-// same of the up weight, 64 .. 128 rows of A, twelve multiplying waves - wave (nibble hh, slot s) has one piece's columns of one
-// nibble, two B operands, as there - and the DMA wave.  Bound by the matrix and vector pipes, which a third wave on each SIMD keeps
-// busier (0.55 us a step of 128 rows x 384 columns, where 1.5 steps of the 256-column units take 0.63), and by how well its workgroups
-// divide the compute units: 512 rows of the 7B shape are 232 of them, one round, where the 256-column units leave 344, two
-// rounds.  4096 -> 2 x 11008, before and now: 512 rows 112.9 us (818 TFLOP/s) and 90.1 (1025), 300 rows 85.3 and 65.2, 1024 rows 201
-// and 178, 2047 rows 375 (985) and 353 (1047); 8192 -> 2 x 28672 at 640 rows 609 and 515, 2047 rows 1834 and 1693.
-template <int TILES> struct WideShape {
-    static constexpr int W = 6 * 1024, SC = 6 * 128;             // [gate 0 .. 2 | up 0 .. 2]: nibbles; scales [octet][nibble][8 rows]
-    static constexpr int STAGE = W + SC + TILES * 1024;
+// ---- above 128 rows, six slots of weights a workgroup (tiled weights, all of K, one workgroup per compute unit) -------------------
+// A workgroup owns 64 .. 128 rows of A; its twelve multiplying waves - wave (nibble hh, slot s) has one piece's columns of one nibble, two
+// B operands, as in q40_gemm_kernel - work on six pieces (64 columns x 32 rows) a stage:
+//   * SWIGLU: pieces 3 u .. 3 u + 2 of the gate weight and the same of the up weight: 384 columns, where q40_gemm_kernel has 256;
+//   * else pieces 3 u .. 3 u + 2 of the weights laid end to end, of two steps: 192 columns and two K-groups, added through LDS.
+// Bound by the matrix and vector pipes, which a third wave on each SIMD keeps busier (0.55 us a step of 128 rows x 384 columns,
+// where 1.5 steps of the 256-column units take 0.63), and by how well its workgroups divide the compute units: w1|w3 of the 7B shape is
+// 232 of them at 512 rows, one round, where 256-column units leave 344, two rounds; wq|wk|wv is 256, where those leave 192.
+// In us, before and now: w1|w3 4096 -> 2 x 11008 at 512 rows 112.9 (818 TFLOP/s) and 90.1 (1025), at 300 rows 85.3 and 65.2, 1024 rows 201
+// and 178, 2047 rows 375 (985) and 353 (1047); 8192 -> 2 x 28672 at 640 rows 609 and 515, 2047 rows 1834 and 1693.  wq|wk|wv 4096 -> 12288 at
+// 512 rows 60.3 (855 TFLOP/s) and 53.2 (969), 1024 rows 119 and 106; 8192 -> 10240 at 512 rows 99.6 and 86.8; 5120 -> 5120 at 2047 rows
+// 131 and 122.  The rule: gemm_plan_rows with the costs ROWS_384 and ROWS_192.
+template <int TILES, bool SWIGLU> struct WideShape {
+    static constexpr int STEPS = SWIGLU ? 1 : 2;                 // of a stage
+    static constexpr int W = 6 * 1024, SC = 6 * 128;             // of the six slots: nibbles; scales [octet][nibble][8 rows]
+    static constexpr int STAGE = W + SC + STEPS * TILES * 1024;
     static constexpr int SLOTS = 6;
-    static constexpr int LDS = SLOTS * STAGE;
-    static constexpr int PER = 9 + TILES;                        // DMA instructions of a stage
+    static constexpr int PER = 9 + STEPS * TILES;                // DMA instructions of a stage
     static constexpr int OP = 192 + 4;
-    static constexpr int OTILE = 2 * 16 * OP * 4;                // [gate | up][16][OP] fp32
-    static_assert(2 * OTILE <= LDS && LDS <= 160 * 1024, "two output tiles in the ring");
+    static constexpr int OTILE = 2 * 16 * OP * 4;                // SwiGLU: [gate | up][16][OP] fp32
+    static constexpr int SUMS = TILES * 16 * OP * 4;             // two K-groups: [row][OP] fp32
+    static constexpr int OUT = SWIGLU ? 2 * OTILE : SUMS;
+    static constexpr int LDS = SLOTS * STAGE > OUT ? SLOTS * STAGE : OUT;
+    static_assert(LDS <= 160 * 1024, "ring");
 };
 constexpr int WIDE_WAVES = 12;
 
-template <int TILES>
-__global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_swiglu_wide_kernel(MatmulParams p) {
+template <int TILES, bool SWIGLU>
+__global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_wide_kernel(MatmulParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    typedef WideShape<TILES> S;
-    constexpr int SLOTS = S::SLOTS, PER = S::PER, STAGE = S::STAGE;
+    typedef WideShape<TILES, SWIGLU> S;
+    constexpr int SLOTS = S::SLOTS, PER = S::PER, STAGE = S::STAGE, STEPS = S::STEPS;
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63, c = lane & 15, g = lane >> 4;
@@ -1115,11 +1122,17 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_swiglu_wide
     const int at = blockIdx.x % p.units_pad, mb = blockIdx.x / p.units_pad;
     const int unit = (at & 7) * (p.units_pad >> 3) + (at >> 3);
     if (unit >= p.units) return;
-    const int m0 = mb * p.block_rows, pieces = p.seg[0].N / 64;
-    const long tiles_per_pair = tiled_steps(p.K);
-    const int n_steps = p.K / 32;
-    const int rot = (unit * 5) % n_steps;                              // workgroups of a row block start at different steps
-    auto piece_of = [&](int k) { return min(3 * unit + k, pieces - 1); };      // (past the end: the last one again, not stored)
+    const int m0 = mb * p.block_rows, pieces = (SWIGLU ? p.seg[0].N : p.n_total) / 64;
+    const int n_st = p.K / (32 * STEPS);
+    const int rot = (unit * 5) % n_st;                                 // workgroups of a row block start at different stages
+    // a piece's weight and its number within the weight
+    auto segment_of = [&](int &P) {
+        int sg = 0;
+        if (!SWIGLU && p.nseg > 1 && P >= p.seg[1].col0 / 64) sg = 1;
+        if (!SWIGLU && p.nseg > 2 && P >= p.seg[2].col0 / 64) sg = 2;
+        if (!SWIGLU) P -= p.seg[sg].col0 / 64;
+        return sg;
+    };
 
     if (wave == WIDE_WAVES) {
         // ---- the DMA wave ----
@@ -1129,40 +1142,49 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_swiglu_wide
 #pragma unroll
         for (int t = 0; t < TILES; ++t) a_voff[t] = (uint32_t)((long)min(m0 + 16 * t + (lane >> 2), p.M - 1) * p.lda * 2 + 16 * a_chunk);
         const uint8_t *w[6], *sc[3];
+        int in_tile[6];
 #pragma unroll
         for (int s = 0; s < 6; ++s) {
-            const int P = piece_of(s % 3);
-            w[s] = p.seg[s / 3].w + (long)(P >> 2) * tiles_per_pair * TILE_BYTES + (P & 3) * 1024;
+            int P = min(3 * unit + s % 3, pieces - 1);                 // (past the end: the last one again, not stored)
+            const int sg = SWIGLU ? s / 3 : segment_of(P);
+            in_tile[s] = P & 3;
+            w[s] = p.seg[sg].w + ((long)(P >> 2) * tiled_steps(p.K) + (SWIGLU ? 0 : s / 3)) * TILE_BYTES;
         }
 #pragma unroll
         for (int i = 0; i < 3; ++i) {                                  // lanes 0 .. 31: slot 2 i's 128 bytes, the others slot 2 i + 1's
-            const int s = 2 * i + (lane >> 5), P = piece_of(s % 3), d = lane & 31;
-            sc[i] = (s < 3 ? p.seg[0].w : p.seg[1].w) + (long)(P >> 2) * tiles_per_pair * TILE_BYTES + TILE_W_BYTES + (d >> 3) * 64 + ((P & 3) >> 1) * 32 + (d & 7) * 4;
+            const bool odd = lane >= 32;
+            const int d = lane & 31;
+            sc[i] = (odd ? w[2 * i + 1] : w[2 * i]) + TILE_W_BYTES + (d >> 3) * 64 + ((odd ? in_tile[2 * i + 1] : in_tile[2 * i]) >> 1) * 32 + (d & 7) * 4;
         }
+#pragma unroll
+        for (int s = 0; s < 6; ++s) w[s] += in_tile[s] * 1024;
         const uint8_t *a_base = reinterpret_cast<const uint8_t *>(p.a);
         int fetch = rot;
         auto issue_stage = [&](int slot_) {
             uint8_t *st = lds + slot_ * STAGE;
-            const long off = (long)fetch * TILE_BYTES;
-            const uint8_t *arow = a_base + (long)fetch * 64;
+            const long off = (long)fetch * STEPS * TILE_BYTES;
+            const uint8_t *arow = a_base + (long)fetch * STEPS * 64;
 #pragma unroll
             for (int s = 0; s < 6; ++s) __builtin_amdgcn_global_load_lds((gptr_t)(w[s] + off + lane * 16), (lptr_t)(st + s * 1024), 16, 0, 0);
 #pragma unroll
             for (int i = 0; i < 3; ++i) __builtin_amdgcn_global_load_lds((gptr_t)(sc[i] + off), (lptr_t)(st + S::W + i * 256), 4, 0, 0);
 #pragma unroll
-            for (int t = 0; t < TILES; ++t) __builtin_amdgcn_global_load_lds((gptr_t)(arow + a_voff[t]), (lptr_t)(st + S::W + S::SC + t * 1024), 16, 0, 0);
-            fetch = fetch + 1 == n_steps ? 0 : fetch + 1;
+            for (int k = 0; k < STEPS; ++k)
+#pragma unroll
+                for (int t = 0; t < TILES; ++t)
+                    __builtin_amdgcn_global_load_lds((gptr_t)(arow + k * 64 + a_voff[t]), (lptr_t)(st + S::W + S::SC + (k * TILES + t) * 1024), 16, 0, 0);
+            fetch = fetch + 1 == n_st ? 0 : fetch + 1;
         };
 #pragma unroll
         for (int i = 0; i < SLOTS - 2; ++i)
-            if (i < n_steps) issue_stage(i);
-        gemm_wait_dma<PER>(min(SLOTS - 3, n_steps - 1));
+            if (i < n_st) issue_stage(i);
+        gemm_wait_dma<PER>(min(SLOTS - 3, n_st - 1));
         gemm_barrier();
         int slot = 0;
         auto back = [&](int k) { return slot >= k ? slot - k : slot + SLOTS - k; };
         int i = 0;
 #pragma unroll 1
-        for (; i + SLOTS - 1 < n_steps; i += 2) {
+        for (; i + SLOTS - 1 < n_st; i += 2) {
             gemm_wait_vm<PER * (SLOTS - 5)>();
             gemm_barrier();
             issue_stage(back(2));
@@ -1170,27 +1192,29 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_swiglu_wide
             slot = slot + 2 >= SLOTS ? slot + 2 - SLOTS : slot + 2;
         }
 #pragma unroll 1
-        for (; i < n_steps; i += 2) {
-            gemm_wait_dma<PER>(max(0, min(n_steps - 1, i + SLOTS - 3) - (i + 2)));
+        for (; i < n_st; i += 2) {
+            gemm_wait_dma<PER>(max(0, min(n_st - 1, i + SLOTS - 3) - (i + 2)));
             gemm_barrier();
-            if (i + SLOTS - 2 < n_steps) issue_stage(back(2));
-            if (i + SLOTS - 1 < n_steps) issue_stage(back(1));
+            if (i + SLOTS - 2 < n_st) issue_stage(back(2));
+            if (i + SLOTS - 1 < n_st) issue_stage(back(1));
             slot = slot + 2 >= SLOTS ? slot + 2 - SLOTS : slot + 2;
         }
-        // the barriers of the epilogue: ring free, one per row tile
+        // the barriers of the epilogue: ring free, one per row tile; ring free, the second group's sums in place, all sums
 #pragma unroll 1
-        for (int t = 0; t < 1 + TILES; ++t) gemm_barrier();
+        for (int t = 0; t < (SWIGLU ? 1 + TILES : 3); ++t) gemm_barrier();
         return;
     }
 
-    const int hh = wave >= 6 ? 1 : 0, s = wave - 6 * hh, gu = s >= 3 ? 1 : 0, k3 = s - 3 * gu;       // nibble, slot, gate (0) or up (1), piece
+    // nibble, slot; the slot's half - gate (0) or up (1), or K-group - and piece
+    const int hh = wave >= 6 ? 1 : 0, s = wave - 6 * hh, half = s >= 3 ? 1 : 0, k3 = s - 3 * half;
     const uint32_t nib_mask = hh == 0 ? 0x00F000F0u : 0x000F000Fu;
     uint32_t nib_magic = MAGIC_1024;                             // (as in q40_gemm_swiglu_kernel)
     asm volatile("" : "+v"(nib_magic));
     const h2 nib_mul = hh == 0 ? h2{(half_t)0.0625f, (half_t)0.0625f} : h2{(half_t)1.0f, (half_t)1.0f};
     const h2 nib_off = hh == 0 ? h2{(half_t)-72.0f, (half_t)-72.0f} : h2{(half_t)-1032.0f, (half_t)-1032.0f};
     struct Raw { u32x4 wq, sc; };
-    const int ws_off = s * 1024 + lane * 16, sc_off = S::W + s * 128 + g * 32 + hh * 16, a_off = S::W + S::SC + c * 64 + ((g ^ ((c >> 1) & 3)) << 4);
+    const int ws_off = s * 1024 + lane * 16, sc_off = S::W + s * 128 + g * 32 + hh * 16;
+    const int a_off = S::W + S::SC + (SWIGLU ? 0 : half * TILES * 1024) + c * 64 + ((g ^ ((c >> 1) & 3)) << 4);
     auto load_ws = [&](const uint8_t *st, Raw &r) {
         r.wq = *reinterpret_cast<const u32x4 *>(st + ws_off);
         r.sc = *reinterpret_cast<const u32x4 *>(st + sc_off);
@@ -1222,14 +1246,14 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_swiglu_wide
         load_ws(lds, r);
         decode(r, bq);
     }
-    auto one_step = [&]() {
+    auto one_stage = [&]() {
         const uint8_t *st = lds + slot * STAGE;
         slot = slot == SLOTS - 1 ? 0 : slot + 1;
         Raw r;
         h8 av[TILES], bn[2];
 #pragma unroll
         for (int t = 0; t < TILES; ++t) av[t] = *reinterpret_cast<const h8 *>(st + a_off + t * 1024);
-        load_ws(lds + slot * STAGE, r);                        // (past the last step: stale bytes, decoded and never used)
+        load_ws(lds + slot * STAGE, r);                        // (past the last stage: stale bytes, decoded and never used)
 #pragma unroll
         for (int t = 0; t < TILES; ++t)
 #pragma unroll
@@ -1240,42 +1264,84 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_swiglu_wide
     };
     int i = 0;
 #pragma unroll 1
-    for (; i + 1 < n_steps; i += 2) {
+    for (; i + 1 < n_st; i += 2) {
         gemm_barrier();
-        one_step();
-        one_step();
+        one_stage();
+        one_stage();
     }
-    if (i < n_steps) {
+    if (i < n_st) {
         gemm_barrier();
-        one_step();
+        one_stage();
     }
 
-    // rows of 192 columns: local column 64 k3 + 32 hh + 2 c + o is column 128 (P / 2) + 64 hh + 4 c + 2 (P % 2) + o, P the piece
+    // rows of 192 columns: local column 64 k3 + 32 hh + 2 c + o is column 128 (P / 2) + 64 hh + 4 c + 2 (P % 2) + o, P the piece;
+    // a thread stores local columns 4 o_lane .. + 3
     constexpr int OP = S::OP;
-    const int o_row = tid / 48, o_lane = tid % 48, P = 3 * unit + (o_lane >> 4), q = o_lane & 15;
+    const int o_row = tid / 48, o_lane = tid % 48, q = o_lane & 15;
+    int P = 3 * unit + (o_lane >> 4);
     const bool mine = P < pieces;
-    const int out_col = 128 * (P >> 1) + 64 * (q >> 3) + 8 * (q & 7) + 2 * (P & 1);
+    const int sg = segment_of(P), out_col = 128 * (P >> 1) + 64 * (q >> 3) + 8 * (q & 7) + 2 * (P & 1);
+    half_t *const out = (sg == 0 ? p.seg[0].c : sg == 1 ? p.seg[1].c : p.seg[2].c) + out_col;
+    const long ldc = sg == 0 ? p.seg[0].ldc : sg == 1 ? p.seg[1].ldc : p.seg[2].ldc;
     gemm_barrier();                                            // every wave has left the loop: the ring is free
+    if constexpr (SWIGLU) {
 #pragma unroll
-    for (int t = 0; t < TILES; ++t) {
-        float *otile = reinterpret_cast<float *>(lds + (t & 1) * S::OTILE);
+        for (int t = 0; t < TILES; ++t) {
+            float *otile = reinterpret_cast<float *>(lds + (t & 1) * S::OTILE);
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-            *reinterpret_cast<f2 *>(&otile[gu * 16 * OP + (4 * g + r) * OP + 64 * k3 + 32 * hh + 2 * c]) = f2{acc[0][t][r], acc[1][t][r]};
-        gemm_barrier();
-        const int m = m0 + 16 * t + o_row;
-        if (m < p.M && mine) {
-            const f4 gv = *reinterpret_cast<const f4 *>(otile + o_row * OP + 4 * o_lane);
-            const f4 uv = *reinterpret_cast<const f4 *>(otile + 16 * OP + o_row * OP + 4 * o_lane);
-            half_t ov[4];
+            for (int r = 0; r < 4; ++r)
+                *reinterpret_cast<f2 *>(&otile[half * 16 * OP + (4 * g + r) * OP + 64 * k3 + 32 * hh + 2 * c]) = f2{acc[0][t][r], acc[1][t][r]};
+            gemm_barrier();
+            const int m = m0 + 16 * t + o_row;
+            if (m < p.M && mine) {
+                const f4 gv = *reinterpret_cast<const f4 *>(otile + o_row * OP + 4 * o_lane);
+                const f4 uv = *reinterpret_cast<const f4 *>(otile + 16 * OP + o_row * OP + 4 * o_lane);
+                half_t ov[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {                      // the roundings of partial_silu_mul_kernel
-                const float gf = (float)(half_t)gv[e];
-                ov[e] = (half_t)(gf / (1.0f + expf(-gf))) * (half_t)uv[e];
+                for (int e = 0; e < 4; ++e) {                  // the roundings of partial_silu_mul_kernel
+                    const float gf = (float)(half_t)gv[e];
+                    ov[e] = (half_t)(gf / (1.0f + expf(-gf))) * (half_t)uv[e];
+                }
+                *reinterpret_cast<h2 *>(out + (long)m * ldc) = h2{ov[0], ov[1]};
+                *reinterpret_cast<h2 *>(out + (long)m * ldc + 4) = h2{ov[2], ov[3]};
             }
-            half_t *dst = p.seg[0].c + (long)m * p.seg[0].ldc + out_col;
-            *reinterpret_cast<h2 *>(dst) = h2{ov[0], ov[1]};
-            *reinterpret_cast<h2 *>(dst + 4) = h2{ov[2], ov[3]};
+        }
+    } else {
+        // the second K-group's sums, then both groups' (in their order), then whole rows
+        float *sums = reinterpret_cast<float *>(lds) + 64 * k3 + 32 * hh + 2 * c;
+        if (half == 1) {
+#pragma unroll
+            for (int t = 0; t < TILES; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) *reinterpret_cast<f2 *>(&sums[(16 * t + 4 * g + r) * OP]) = f2{acc[0][t][r], acc[1][t][r]};
+        }
+        gemm_barrier();
+        if (half == 0) {
+#pragma unroll
+            for (int t = 0; t < TILES; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    f2 *at_ = reinterpret_cast<f2 *>(&sums[(16 * t + 4 * g + r) * OP]);
+                    const f2 other = *at_;
+                    *at_ = f2{acc[0][t][r] + other[0], acc[1][t][r] + other[1]};
+                }
+        }
+        gemm_barrier();
+        const int n = p.seg[sg].col0 + out_col;
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            const int m = m0 + 16 * t + o_row;
+            if (m < p.M && mine) {
+                const f4 v = *reinterpret_cast<const f4 *>(reinterpret_cast<const float *>(lds) + (16 * t + o_row) * OP + 4 * o_lane);
+                if (p.direct) {
+                    *reinterpret_cast<h2 *>(out + (long)m * ldc) = h2{matmul_epilogue(p, v[0], m, n), matmul_epilogue(p, v[1], m, n + 1)};
+                    *reinterpret_cast<h2 *>(out + (long)m * ldc + 4) = h2{matmul_epilogue(p, v[2], m, n + 4), matmul_epilogue(p, v[3], m, n + 5)};
+                } else {
+                    float *slab = p.partial + (long)m * p.n_total + n;
+                    *reinterpret_cast<f2 *>(slab) = f2{v[0], v[1]};
+                    *reinterpret_cast<f2 *>(slab + 4) = f2{v[2], v[3]};
+                }
+            }
         }
     }
 }
@@ -1296,6 +1362,10 @@ constexpr RowsCost ROWS_256 = {0.18f, 0.24f, 4.0f, 1.2f};
 // SwiGLU with three pieces a workgroup (384 columns): fitted to the shapes of 7B, 13B, 34B and 70B at 130 .. 2047 rows, within 4 % in
 // the mean.  Taking it where its estimate is the smaller was never slower there than the 256-column units (0.72 .. 0.99 of their time).
 constexpr RowsCost ROWS_384 = {0.21f, 0.37f, 4.0f, 1.15f};
+// Three pieces and two K-groups a workgroup (192 columns), in the place of 256-column units without a K-split: fitted to wq|wk|wv, wo and
+// w2 of 7B, 13B and 70B at 130 .. 2047 rows, within 7 % in the mean.  Taken where it promises 3 %, it took 0.85 .. 0.97 of the time (once
+// 1.01: 300 rows of 4096 x 12288).  Where the 256-column units have a K-split they stay: launch and slabs are level or better.
+constexpr RowsCost ROWS_192 = {0.11f, 0.21f, 4.0f, 1.2f};
 static float gemm_rows_us(const RowsCost &t, int units, long of_unit, int rows, int steps) {
     const float r = (float)(units * of_unit) / 256.0f, rounds = (float)(((units + 7) / 8 * of_unit + 31) / 32);
     return (rounds > t.busy * r ? rounds : t.busy * r) * ((float)steps * (t.step + t.per_rows * rows / GEMM_BM) + t.around);
@@ -1376,7 +1446,14 @@ void gemm_fill_plan(MatmulParams &p) {
     p.mblocks = (p.M + p.block_rows - 1) / p.block_rows;
     const int steps = (p.K + 31) / 32;
     if (p.M > GEMM_BM) {
-        gemm_plan_rows(p, steps, SMH_MAX_KSPLIT, ROWS_256);
+        const float us = gemm_plan_rows(p, steps, SMH_MAX_KSPLIT, ROWS_256);
+        if (p.tiled && p.ksplit == 1 && p.K % 64 == 0) {                       // q40_gemm_wide_kernel: see ROWS_192
+            MatmulParams w = p;
+            w.units = (p.n_total / 64 + 2) / 3;
+            w.units_pad = (w.units + 7) / 8 * 8;
+            w.kgroups = 3;
+            if (gemm_plan_rows(w, steps, 1, ROWS_192) < 0.97f * us) p = w;
+        }
         return;
     }
     const long tiles = (long)p.units * p.mblocks;
@@ -1558,9 +1635,9 @@ int gemm_swiglu_rows_launch(MatmulParams p, hipStream_t stream) {
                                            q40_gemm_kernel<7, false, true, 8, GEMM_STAGES, false, false, true>, q40_gemm_kernel<8, false, true, 8, GEMM_STAGES, false, false, true>};
     static const gemm_kernel_t dma_wave[5] = {q40_gemm_kernel<4, false, true, 8, gemm_dma_slots(4), true, false, true>, q40_gemm_kernel<5, false, true, 8, gemm_dma_slots(5), true, false, true>, q40_gemm_kernel<6, false, true, 8, gemm_dma_slots(6), true, false, true>,
                                               q40_gemm_kernel<7, false, true, 8, gemm_dma_slots(7), true, false, true>, q40_gemm_kernel<8, false, true, 8, gemm_dma_slots(8), true, false, true>};
-    static const gemm_kernel_t wide[5] = {q40_gemm_swiglu_wide_kernel<4>, q40_gemm_swiglu_wide_kernel<5>, q40_gemm_swiglu_wide_kernel<6>,
-                                          q40_gemm_swiglu_wide_kernel<7>, q40_gemm_swiglu_wide_kernel<8>};
-    static const int wide_lds[5] = {WideShape<4>::LDS, WideShape<5>::LDS, WideShape<6>::LDS, WideShape<7>::LDS, WideShape<8>::LDS};
+    static const gemm_kernel_t wide[5] = {q40_gemm_wide_kernel<4, true>, q40_gemm_wide_kernel<5, true>, q40_gemm_wide_kernel<6, true>,
+                                          q40_gemm_wide_kernel<7, true>, q40_gemm_wide_kernel<8, true>};
+    static const int wide_lds[5] = {WideShape<4, true>::LDS, WideShape<5, true>::LDS, WideShape<6, true>::LDS, WideShape<7, true>::LDS, WideShape<8, true>::LDS};
     static const hipError_t lds_ok = [] {
         hipError_t e = hipSuccess;
         for (int t = 0; t < 5 && e == hipSuccess; ++t) {
@@ -1594,7 +1671,27 @@ int gemm_swiglu_rows_launch(MatmulParams p, hipStream_t stream) {
     return launch_status();
 }
 
+static int gemm_wide_launch(const MatmulParams &p, hipStream_t stream) {
+    static const gemm_kernel_t kern[5] = {q40_gemm_wide_kernel<4, false>, q40_gemm_wide_kernel<5, false>, q40_gemm_wide_kernel<6, false>,
+                                          q40_gemm_wide_kernel<7, false>, q40_gemm_wide_kernel<8, false>};
+    static const int lds_bytes[5] = {WideShape<4, false>::LDS, WideShape<5, false>::LDS, WideShape<6, false>::LDS, WideShape<7, false>::LDS, WideShape<8, false>::LDS};
+    static const hipError_t lds_ok = [] {
+        hipError_t e = hipSuccess;
+        for (int t = 0; t < 5 && e == hipSuccess; ++t) e = hipFuncSetAttribute((const void *)kern[t], hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes[t]);
+        return e;
+    }();
+    if (lds_ok != hipSuccess) {
+        set_error("q40 gemm: the kernels' LDS could not be reserved: %s", hipGetErrorString(lds_ok));
+        return (int)lds_ok;
+    }
+    SMH_REQUIRE((long)p.M * p.lda * 2 < (1L << 32), "q40 gemm: M x lda = %d x %ld exceeds the 32-bit lane offsets of A", p.M, p.lda);
+    const int t = p.block_rows / 16 - 4;
+    hipLaunchKernelGGL(kern[t], dim3((unsigned)((long)p.units_pad * p.mblocks)), dim3(64 * (WIDE_WAVES + 1)), lds_bytes[t], stream, p);
+    return launch_status();
+}
+
 int gemm_launch(const MatmulParams &p, hipStream_t stream) {
+    if (p.kgroups == 3 && p.tiled) return gemm_wide_launch(p, stream);
     if (p.kgroups == 2 && p.tiled) return gemm_kg_launch(p, stream);
     return p.tiled ? gemm_launch_layout<true>(p, stream) : gemm_launch_layout<false>(p, stream);
 }

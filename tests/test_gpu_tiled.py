@@ -321,3 +321,32 @@ def test_direct_products(M, K, ns):
         want = O.matmul_q40(a, w, s, (K, n))
         want = want.float() + r.float() if r is not None else want.float()
         assert torch.allclose(o.cpu().float(), want, rtol=1e-2, atol=2e-3)
+
+
+@pytest.mark.parametrize("M,K,ns", [(192, 64, [1152]),                     # one stage; four row tiles; three pieces throughout
+                                    (129, 64, [1280]),                     # five row tiles, the last block of 49 rows; a last workgroup of two pieces
+                                    (257, 128, [10624]),                   # two stages; six row tiles; one piece
+                                    (512, 704, [7040, 128, 896]),          # eleven stages; seven row tiles; workgroups across weights, odd 128-column blocks
+                                    (600, 448, [7808]),                    # seven stages, more than the ring holds; eight row tiles
+                                    (400, 4096, [4096, 4096, 4096])])
+def test_three_pieces_and_two_k_groups(M, K, ns):
+    """sizes above 128 rows that q40_gemm_wide_kernel takes (its estimate is the smaller one): fp16 results with and without a
+    residual, and the one slab of the same launch"""
+    from spec_mcts_amd import kernels as Kn
+    ws = [_weight(K, n, 2000 + i + K) for i, n in enumerate(ns)]
+    tiled = [Kn.tile_q40(w.cuda(), s.cuda(), K, n) for (w, s), n in zip(ws, ns)]
+    a = (torch.randn((M, K), generator=torch.Generator().manual_seed(2001 + M)) * 0.5).half()
+    r = torch.randn((M, ns[0]), generator=torch.Generator().manual_seed(2002)).half() if len(ns) == 1 else None
+    assert Kn.matmul_plan(M, K, ns, tiled=True) == 1
+    got = Kn.matmul_q40_direct(a.cuda(), tiled)
+    with_r = Kn.matmul_q40_direct(a.cuda(), tiled, residual=r.cuda()) if r is not None else got
+    slab = Kn.matmul_q40_partial(a.cuda(), tiled).buf[:M * sum(ns)].view(M, sum(ns)).cpu()
+    col = 0
+    for (w, s), n, o, o_r in zip(ws, ns, got, with_r):
+        want = O.matmul_q40(a, w, s, (K, n)).float()
+        # fp32 sums in another order, one rounding to fp16 each (2^-11): 1e-3 of the value; near zero the sums' own error
+        assert torch.allclose(o.cpu().float(), want, rtol=2e-3, atol=2e-3)
+        assert torch.equal(slab[:, col:col + n].half(), o.cpu())
+        if r is not None:
+            assert torch.equal(o_r.cpu(), (r.float() + o.cpu().float()).half())
+        col += n
