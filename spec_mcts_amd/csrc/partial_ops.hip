@@ -17,26 +17,34 @@
 namespace smh {
 
 // ---- plain reduce (+ residual) ------------------------------------------------------------------
-__global__ __launch_bounds__(256) void partial_reduce_kernel(const void *__restrict__ partial, int ksplit, int M, int n_total,
-                                                             int col0, int N, half_t *__restrict__ c, long ldc, int epilogue,
-                                                             const half_t *__restrict__ resid, long ldr) {
+// RES: a residual of this alignment (elements a load; 0: none)
+template <int KS, int RES>
+__global__ __launch_bounds__(256) void partial_reduce_kernel(const void *__restrict__ partial, int M, int n_total, int col0, int N,
+                                                             half_t *__restrict__ c, long ldc, const half_t *__restrict__ resid, long ldr) {
     const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
     if (i >= (long)M * N) return;
     const int m = (int)(i / N), n = (int)(i % N);          // N % 4 == 0: the 4 columns share a row
-    const f4 acc = slab_sum4(partial, (long)m * n_total + col0 + n, (long)M * n_total, ksplit);
+    f4 v[KS];
+    slab_load(partial, (long)m * n_total + col0 + n, (long)M * n_total, v);
+    h4 r;
+    if constexpr (RES == 4) r = *reinterpret_cast<const h4 *>(resid + (long)m * ldr + n);
+    if constexpr (RES == 1) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) r[j] = resid[(long)m * ldr + n + j];
+    }
+    const f4 acc = slab_add(v);
     h4 out;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        half_t v = (half_t)acc[j];
-        if (epilogue == SMH_EPI_RESIDUAL) v = (half_t)((float)resid[(long)m * ldr + n + j] + (float)v);
-        out[j] = v;
-    }
+    for (int j = 0; j < 4; ++j) out[j] = RES == 0 ? (half_t)acc[j] : (half_t)((float)r[j] + (float)(half_t)acc[j]);
     *reinterpret_cast<h4 *>(c + (long)m * ldc + n) = out;
 }
 
 // ---- residual add + RMSNorm ---------------------------------------------------------------------
 // one workgroup of 1024 threads per row; h_out = h_in + fp16(acc) (fp16 add), xn = fp16(fp16(h*r)*w)
-__global__ __launch_bounds__(1024) void partial_rmsnorm_kernel(const void *__restrict__ partial, int ksplit, int M, int N,
+// A chain of trips to memory bounds it, so everything is requested before the first sum: KS slabs (0: none), PASSES passes of four
+// columns a thread, the residual and the norm's weights.  Up to 64 registers two workgroups share a compute unit.
+template <int PASSES, int KS>
+__global__ __launch_bounds__(1024, PASSES * KS <= 8 ? 8 : 4) void partial_rmsnorm_kernel(const void *__restrict__ partial, int M, int N,
                                                                const half_t *__restrict__ h_in, const half_t *__restrict__ wt,
                                                                float eps, half_t *__restrict__ h_out, half_t *__restrict__ xn_out) {
     __shared__ float s_part[16];
@@ -44,35 +52,33 @@ __global__ __launch_bounds__(1024) void partial_rmsnorm_kernel(const void *__res
     const long slab = (long)M * N;
     float ss = 0.f;
     // each thread owns columns 4t, 4t+1, 4t+2, 4t+3 (+ 4096 per pass); values kept for the second pass
-    constexpr int MAXPASS = 4;      // N <= 16384
-    h4 hv[MAXPASS], wv[MAXPASS];
-    // the norm weights are not needed before the second pass: fetched now, they arrive with the slabs
+    constexpr int AHEAD = PASSES * KS <= 16 ? PASSES : 1;      // passes whose slabs are on their way together
+    h4 hv[PASSES], wv[PASSES];
+    f4 v[AHEAD][KS > 0 ? KS : 1];
+    const half_t *from = h_in != nullptr ? h_in + (long)m * N : wt;          // (without a residual: read, not used)
 #pragma unroll
-    for (int ps = 0; ps < MAXPASS; ++ps) {
-        const int n = (ps * 1024 + threadIdx.x) * 4;
-        if (n < N) wv[ps] = *reinterpret_cast<const h4 *>(wt + n);
-    }
-#pragma unroll
-    for (int ps = 0; ps < MAXPASS; ++ps) {
+    for (int ps = 0; ps < PASSES; ++ps) {
         const int n = (ps * 1024 + threadIdx.x) * 4;
         if (n < N) {
-            h4 v;
-            if (partial != nullptr) {
-                const f4 acc = slab_sum4(partial, (long)m * N + n, slab, ksplit);
+            if constexpr (KS > 0 && AHEAD == PASSES) slab_load(partial, (long)m * N + n, slab, v[ps % AHEAD]);
+            hv[ps] = *reinterpret_cast<const h4 *>(from + n);
+            wv[ps] = *reinterpret_cast<const h4 *>(wt + n);
+        }
+    }
 #pragma unroll
-                for (int j = 0; j < 4; ++j) v[j] = (half_t)acc[j];
-                if (h_in != nullptr) {
-                    const h4 r = *reinterpret_cast<const h4 *>(h_in + (long)m * N + n);
+    for (int ps = 0; ps < PASSES; ++ps) {
+        const int n = (ps * 1024 + threadIdx.x) * 4;
+        if (n < N) {
+            h4 &h = hv[ps];
+            if constexpr (KS > 0) {
+                if constexpr (AHEAD < PASSES) slab_load(partial, (long)m * N + n, slab, v[0]);
+                const f4 acc = slab_add(v[ps % AHEAD]);
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) v[j] = (half_t)((float)r[j] + (float)v[j]);
-                }
-            } else {
-                v = *reinterpret_cast<const h4 *>(h_in + (long)m * N + n);
+                for (int j = 0; j < 4; ++j) h[j] = h_in != nullptr ? (half_t)((float)h[j] + (float)(half_t)acc[j]) : (half_t)acc[j];
             }
-            hv[ps] = v;
-            if (h_out != nullptr) *reinterpret_cast<h4 *>(h_out + (long)m * N + n) = v;
+            if (h_out != nullptr) *reinterpret_cast<h4 *>(h_out + (long)m * N + n) = h;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) ss = sumsq_add(ss, (float)v[j]);
+            for (int j = 0; j < 4; ++j) ss = sumsq_add(ss, (float)h[j]);
         }
     }
     ss = wave_sum(ss);
@@ -83,7 +89,7 @@ __global__ __launch_bounds__(1024) void partial_rmsnorm_kernel(const void *__res
     for (int w = 0; w < 16; ++w) total += s_part[w];
     const float r = rms_factor(total, N, eps);
 #pragma unroll
-    for (int ps = 0; ps < MAXPASS; ++ps) {
+    for (int ps = 0; ps < PASSES; ++ps) {
         const int n = (ps * 1024 + threadIdx.x) * 4;
         if (n < N) {
             const h4 w = wv[ps];
@@ -141,32 +147,33 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const half_t *__restr
 // grid (16, M), one wave each: wave w of a row is wave w of partial_rmsnorm_kernel's workgroup (same columns per
 // thread, same order of additions), so sums[m][0..15] added in index order give that kernel's sum of squares bit
 // for bit.  The consumer (the matmul that follows, q40_gemv_kernel LAYOUT 3) normalises its own K-slice.
-__global__ __launch_bounds__(64) void partial_residual_sumsq_kernel(const void *__restrict__ partial, int ksplit, int M, int N,
+template <int PASSES, int KS>
+__global__ __launch_bounds__(64) void partial_residual_sumsq_kernel(const void *__restrict__ partial, int M, int N,
                                                                     const half_t *__restrict__ h_in, half_t *__restrict__ h_out,
                                                                     float *__restrict__ sums) {
     const int m = blockIdx.y;
     const int vt = blockIdx.x * 64 + threadIdx.x;      // thread index inside partial_rmsnorm_kernel's workgroup
     const long slab = (long)M * N;
-    constexpr int MAXPASS = 4;      // N <= 16384
-    f4 acc[MAXPASS];
-    h4 res[MAXPASS];
+    f4 acc[PASSES][KS];
+    h4 res[PASSES];
 #pragma unroll
-    for (int ps = 0; ps < MAXPASS; ++ps) {
+    for (int ps = 0; ps < PASSES; ++ps) {
         const int n = (ps * 1024 + vt) * 4;
         if (n < N) {
-            acc[ps] = slab_sum4(partial, (long)m * N + n, slab, ksplit);
+            slab_load(partial, (long)m * N + n, slab, acc[ps]);
             if (h_in != nullptr) res[ps] = *reinterpret_cast<const h4 *>(h_in + (long)m * N + n);
         }
     }
     float ss = 0.f;
 #pragma unroll
-    for (int ps = 0; ps < MAXPASS; ++ps) {
+    for (int ps = 0; ps < PASSES; ++ps) {
         const int n = (ps * 1024 + vt) * 4;
         if (n < N) {
+            const f4 sum = slab_add(acc[ps]);
             h4 v;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                v[j] = (half_t)acc[ps][j];
+                v[j] = (half_t)sum[j];
                 if (h_in != nullptr) v[j] = (half_t)((float)res[ps][j] + (float)v[j]);
             }
             *reinterpret_cast<h4 *>(h_out + (long)m * N + n) = v;
@@ -180,14 +187,17 @@ __global__ __launch_bounds__(64) void partial_residual_sumsq_kernel(const void *
 
 // ---- SwiGLU gate ------------------------------------------------------------------------------------
 // slabs hold [gate | up] (2 * n_half columns)
-__global__ __launch_bounds__(256) void partial_silu_mul_kernel(const void *__restrict__ partial, int ksplit, int M, int n_half,
+template <int KS>
+__global__ __launch_bounds__(256) void partial_silu_mul_kernel(const void *__restrict__ partial, int M, int n_half,
                                                                half_t *__restrict__ out) {
     // grid (quads of a row, rows): no division to find the row (a 64-bit one costs more than the rest of the arithmetic)
     const int m = blockIdx.y, n = (blockIdx.x * 256 + threadIdx.x) * 4;
     if (n >= n_half) return;
     const long slab = (long)M * 2 * n_half;
-    const f4 ga = slab_sum4(partial, (long)m * 2 * n_half + n, slab, ksplit);
-    const f4 ua = slab_sum4(partial, (long)m * 2 * n_half + n_half + n, slab, ksplit);
+    f4 gv[KS], uv[KS];
+    slab_load(partial, (long)m * 2 * n_half + n, slab, gv);
+    slab_load(partial, (long)m * 2 * n_half + n_half + n, slab, uv);
+    const f4 ga = slab_add(gv), ua = slab_add(uv);
     h4 o;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -200,7 +210,8 @@ __global__ __launch_bounds__(256) void partial_silu_mul_kernel(const void *__res
 
 // one wave per (branch, head); heads 0..H-1 queries, H..H+Hkv-1 keys, H+Hkv.. values.
 // slab columns: [q (H*128) | k (Hkv*128) | v (Hkv*128)]
-__global__ __launch_bounds__(256) void partial_rope_append_kernel(const void *__restrict__ partial, int ksplit, int B, int H, int Hkv,
+template <int KS>
+__global__ __launch_bounds__(256) void partial_rope_append_kernel(const void *__restrict__ partial, int B, int H, int Hkv,
                                                                   half_t *__restrict__ q, half_t *__restrict__ k, half_t *__restrict__ v,
                                                                   const half_t *__restrict__ cos_tab, const half_t *__restrict__ sin_tab,
                                                                   const int32_t *__restrict__ pos_dev,
@@ -219,12 +230,14 @@ __global__ __launch_bounds__(256) void partial_rope_append_kernel(const void *__
     const int n_total = heads * 128;
     // the slabs are read two adjacent columns per lane; the rotation pairs column i with i + 64, so the sums
     // change lanes through LDS
-    // the position and the rotation factors travel while the slabs are read
+    // the slabs first: the position, and behind it the rotation factors, travel under them
+    f2 parts[KS];
+    slab_load(partial, (long)b * n_total + (long)h * 128 + 2 * lane, (long)B * n_total, parts);
     const int t = (t_dev != nullptr) ? *t_dev : -1;
     const int pos = *pos_dev;
     const half_t cos_l = cos_tab[(long)pos * 64 + lane], sin_l = sin_tab[(long)pos * 64 + lane];
     if (live) {
-        const f2 sum = slab_sum2(partial, (long)b * n_total + (long)h * 128 + 2 * lane, (long)B * n_total, ksplit);
+        const f2 sum = slab_add(parts);
         *reinterpret_cast<f2 *>(&s_row[wave][2 * lane]) = sum;
     }
     __syncthreads();
@@ -261,7 +274,8 @@ __global__ __launch_bounds__(256) void partial_rope_append_kernel(const void *__
 
 // A prefill's q|k|v product -> q, and k, v as rows of the prompt cache (fp16): sums, one rounding, RoPE of q and k at position
 // row + pos0.  One thread owns four rotation pairs (d .. d+3, d+64 ..) of one head.
-__global__ __launch_bounds__(256) void partial_rope_rows_kernel(const void *__restrict__ partial, int ksplit, int S, int H, int Hkv,
+template <int KS>
+__global__ __launch_bounds__(256) void partial_rope_rows_kernel(const void *__restrict__ partial, int S, int H, int Hkv,
                                                                 half_t *__restrict__ q, half_t *__restrict__ k, half_t *__restrict__ v,
                                                                 const half_t *__restrict__ cos_tab, const half_t *__restrict__ sin_tab, int pos0) {
     const int heads = H + 2 * Hkv, s = blockIdx.y;
@@ -269,7 +283,10 @@ __global__ __launch_bounds__(256) void partial_rope_rows_kernel(const void *__re
     if (h >= heads) return;
     const int n_total = heads * 128;
     const long at = (long)s * n_total + h * 128 + d, slab = (long)S * n_total;
-    const f4 lo = slab_sum4(partial, at, slab, ksplit), hi = slab_sum4(partial, at + 64, slab, ksplit);
+    f4 lo_v[KS], hi_v[KS];
+    slab_load(partial, at, slab, lo_v);
+    slab_load(partial, at + 64, slab, hi_v);
+    const f4 lo = slab_add(lo_v), hi = slab_add(hi_v);
     h4 x1, x2;
 #pragma unroll
     for (int j = 0; j < 4; ++j) { x1[j] = (half_t)lo[j]; x2[j] = (half_t)hi[j]; }
@@ -290,6 +307,32 @@ __global__ __launch_bounds__(256) void partial_rope_rows_kernel(const void *__re
 }  // namespace smh
 
 using namespace smh;
+
+// kernels by the number of slabs
+static_assert(SMH_MAX_KSPLIT == 16, "tables");
+#define BY_SLABS(k, ...) {__VA_ARGS__, k(1), k(2), k(3), k(4), k(5), k(6), k(7), k(8), k(9), k(10), k(11), k(12), k(13), k(14), k(15), k(16)}
+typedef void (*reduce_kernel_t)(const void *, int, int, int, int, half_t *, long, const half_t *, long);
+typedef void (*rmsnorm_kernel_t)(const void *, int, int, const half_t *, const half_t *, float, half_t *, half_t *);
+typedef void (*sumsq_kernel_t)(const void *, int, int, const half_t *, half_t *, float *);
+#define K_OF(n) partial_reduce_kernel<n, RES>
+template <int RES> static const reduce_kernel_t REDUCE_KERNELS[17] = BY_SLABS(K_OF, nullptr);
+#undef K_OF
+#define K_OF(n) partial_rmsnorm_kernel<PASSES, n>
+template <int PASSES> static const rmsnorm_kernel_t RMSNORM_KERNELS[17] = BY_SLABS(K_OF, K_OF(0));
+#undef K_OF
+#define K_OF(n) partial_residual_sumsq_kernel<PASSES, n>
+template <int PASSES> static const sumsq_kernel_t SUMSQ_KERNELS[17] = BY_SLABS(K_OF, nullptr);
+#undef K_OF
+#define K_OF(n) partial_silu_mul_kernel<n>
+static const decltype(&partial_silu_mul_kernel<1>) SILU_KERNELS[17] = BY_SLABS(K_OF, nullptr);
+#undef K_OF
+#define K_OF(n) partial_rope_append_kernel<n>
+static const decltype(&partial_rope_append_kernel<1>) ROPE_APPEND_KERNELS[17] = BY_SLABS(K_OF, nullptr);
+#undef K_OF
+#define K_OF(n) partial_rope_rows_kernel<n>
+static const decltype(&partial_rope_rows_kernel<1>) ROPE_ROWS_KERNELS[17] = BY_SLABS(K_OF, nullptr);
+#undef K_OF
+#undef BY_SLABS
 
 // ---- host side: plan, produce, consume ----------------------------------------------------------------
 static int fill_params(MatmulParams &p, const void *a, int M, int K, long lda, int nseg, const void *const *w,
@@ -477,8 +520,10 @@ extern "C" int smh_q40_matmul_partial_tiled_norm(const void *h, long ldh, const 
 static int reduce_launch(const void *partial, int ksplit, int M, int n_total, int col0, int N, void *c, long ldc,
                          int epilogue, const void *residual, long ldr, hipStream_t stream) {
     long quads = ((long)M * N + 3) / 4;
-    hipLaunchKernelGGL(partial_reduce_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream,
-                       partial, ksplit, M, n_total, col0, N, (half_t *)c, ldc, epilogue, (const half_t *)residual, ldr);
+    const bool aligned = ldr % 4 == 0 && (uintptr_t)residual % 8 == 0;
+    const auto kern = (epilogue != SMH_EPI_RESIDUAL ? REDUCE_KERNELS<0> : aligned ? REDUCE_KERNELS<4> : REDUCE_KERNELS<1>)[ksplit];
+    hipLaunchKernelGGL(kern, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream, partial, M, n_total, col0, N, (half_t *)c, ldc,
+                       (const half_t *)residual, ldr);
     return launch_status();
 }
 
@@ -551,8 +596,10 @@ extern "C" int smh_partial_rmsnorm(const void *partial, int ksplit, int M, int N
         hipLaunchKernelGGL(kern, dim3(M), dim3(256), 0, (hipStream_t)stream, (const half_t *)h_in, (const half_t *)weight, N, eps, (half_t *)xn_out);
         return launch_status();
     }
-    hipLaunchKernelGGL(partial_rmsnorm_kernel, dim3(M), dim3(1024), 0, (hipStream_t)stream, partial, ksplit, M, N,
-                       (const half_t *)h_in, (const half_t *)weight, eps, (half_t *)h_out, (half_t *)xn_out);
+    const int ks = partial == nullptr ? 0 : ksplit;
+    const auto kern = N <= 4096 ? RMSNORM_KERNELS<1>[ks] : N <= 8192 ? RMSNORM_KERNELS<2>[ks] : RMSNORM_KERNELS<4>[ks];
+    hipLaunchKernelGGL(kern, dim3(M), dim3(1024), 0, (hipStream_t)stream, partial, M, N, (const half_t *)h_in, (const half_t *)weight, eps, (half_t *)h_out,
+                       (half_t *)xn_out);
     return launch_status();
 }
 
@@ -562,8 +609,8 @@ extern "C" int smh_partial_residual_sumsq(const void *partial, int ksplit, int M
     SMH_REQUIRE(M >= 0 && N > 0 && N % 4 == 0 && N <= 16384, "smh_partial_residual_sumsq: M=%d N=%d (N must be a multiple of 4, <= 16384)", M, N);
     if (M == 0) return 0;
     SMH_REQUIRE(h_out && sums, "smh_partial_residual_sumsq: null pointer");
-    hipLaunchKernelGGL(partial_residual_sumsq_kernel, dim3(SMH_NORM_SUMS, M), dim3(64), 0, (hipStream_t)stream, partial, ksplit, M, N,
-                       (const half_t *)h_in, (half_t *)h_out, (float *)sums);
+    const auto kern = N <= 4096 ? SUMSQ_KERNELS<1>[ksplit] : N <= 8192 ? SUMSQ_KERNELS<2>[ksplit] : SUMSQ_KERNELS<4>[ksplit];
+    hipLaunchKernelGGL(kern, dim3(SMH_NORM_SUMS, M), dim3(64), 0, (hipStream_t)stream, partial, M, N, (const half_t *)h_in, (half_t *)h_out, (float *)sums);
     return launch_status();
 }
 
@@ -573,8 +620,8 @@ extern "C" int smh_partial_silu_mul(const void *partial, int ksplit, int M, int 
     if (M == 0) return 0;
     SMH_REQUIRE(partial && out, "smh_partial_silu_mul: null pointer");
     SMH_REQUIRE(M <= 65535, "smh_partial_silu_mul: M=%d (at most 65535 rows per launch)", M);
-    hipLaunchKernelGGL(partial_silu_mul_kernel, dim3((unsigned)((n_half / 4 + 255) / 256), (unsigned)M), dim3(256), 0, (hipStream_t)stream,
-                       partial, ksplit, M, n_half, (half_t *)out);
+    hipLaunchKernelGGL(SILU_KERNELS[ksplit], dim3((unsigned)((n_half / 4 + 255) / 256), (unsigned)M), dim3(256), 0, (hipStream_t)stream,
+                       partial, M, n_half, (half_t *)out);
     return launch_status();
 }
 
@@ -589,8 +636,8 @@ extern "C" int smh_partial_rope_append_kv(const void *partial, int ksplit, int B
     SMH_REQUIRE(partial && q && k && v && cos_tab && sin_tab && pos_dev, "smh_partial_rope_append_kv: null pointer");
     SMH_REQUIRE(!cache_k || (cache_ks && cache_v && cache_vs && t_dev && Smax > 0), "smh_partial_rope_append_kv: cache arguments incomplete");
     SMH_REQUIRE(B <= 65535, "smh_partial_rope_append_kv: B=%d (at most 65535 branches per launch)", B);
-    hipLaunchKernelGGL(partial_rope_append_kernel, dim3((unsigned)((H + 2 * Hkv + 3) / 4), (unsigned)B), dim3(256), 0, (hipStream_t)stream,
-                       partial, ksplit, B, H, Hkv, (half_t *)q, (half_t *)k, (half_t *)v,
+    hipLaunchKernelGGL(ROPE_APPEND_KERNELS[ksplit], dim3((unsigned)((H + 2 * Hkv + 3) / 4), (unsigned)B), dim3(256), 0, (hipStream_t)stream,
+                       partial, B, H, Hkv, (half_t *)q, (half_t *)k, (half_t *)v,
                        (const half_t *)cos_tab, (const half_t *)sin_tab, pos_dev, (uint8_t *)cache_k, (half_t *)cache_ks,
                        (uint8_t *)cache_v, (half_t *)cache_vs, Smax, t_dev);
     return launch_status();
@@ -603,7 +650,7 @@ extern "C" int smh_partial_rope_rows(const void *partial, int ksplit, int S, int
     SMH_REQUIRE(S >= 0 && S <= 65535 && H > 0 && Hkv > 0 && pos0 >= 0, "smh_partial_rope_rows: S=%d (at most 65535) H=%d Hkv=%d pos0=%d", S, H, Hkv, pos0);
     if (S == 0) return 0;
     SMH_REQUIRE(partial && q && k && v && cos_tab && sin_tab, "smh_partial_rope_rows: null pointer");
-    hipLaunchKernelGGL(partial_rope_rows_kernel, dim3((unsigned)(((H + 2 * Hkv) * 16 + 255) / 256), (unsigned)S), dim3(256), 0, (hipStream_t)stream, partial,
-                       ksplit, S, H, Hkv, (half_t *)q, (half_t *)k, (half_t *)v, (const half_t *)cos_tab, (const half_t *)sin_tab, pos0);
+    hipLaunchKernelGGL(ROPE_ROWS_KERNELS[ksplit], dim3((unsigned)(((H + 2 * Hkv) * 16 + 255) / 256), (unsigned)S), dim3(256), 0, (hipStream_t)stream, partial,
+                       S, H, Hkv, (half_t *)q, (half_t *)k, (half_t *)v, (const half_t *)cos_tab, (const half_t *)sin_tab, pos0);
     return launch_status();
 }

@@ -5,38 +5,33 @@
 
 namespace smh {
 
-// Element `idx` of every slab (fp32), added in slice order.
-__device__ __forceinline__ float slab_sum(const void *partial, long idx, long slab_stride, int ksplit) {
+// Elements idx .. of KS slabs on their way: T is float, f2 or f4 (idx a multiple of 2 or 4).  Kernels that live by this are instantiated by
+// the number of slabs: with a condition on each load the compiler moves what it has between registers in between, and waits for it first
+// (two or three trips to memory one behind the other instead of one).  In turn: eight steps of 100 branches (7B) 31.85 -> 31.30 ms, 37 branches
+// 2986 -> 2942 us a step, 512-row prefill 8.64 -> 8.46 ms, 10 branches of three 70B layers 537 -> 528 us.
+template <typename T, int KS>
+__device__ __forceinline__ void slab_load(const void *partial, long idx, long slab_stride, T (&v)[KS]) {
     const float *p = reinterpret_cast<const float *>(partial) + idx;
-    float v[SMH_MAX_KSPLIT];
 #pragma unroll
-    for (int s = 0; s < SMH_MAX_KSPLIT; ++s) v[s] = (s < ksplit) ? p[s * slab_stride] : 0.f;
-    float tot = 0.f;
+    for (int s = 0; s < KS; ++s) v[s] = *reinterpret_cast<const T *>(p + s * slab_stride);
+}
+// ... added in slice order.
+template <typename T, int KS>
+__device__ __forceinline__ T slab_add(const T (&v)[KS]) {
+    float zero = 0.f;
+    asm("" : "+v"(zero));                                    // (a zero that the compiler knows it adds where the first slab is loaded, and waits there)
+    T tot = T{} + zero;
 #pragma unroll
-    for (int s = 0; s < SMH_MAX_KSPLIT; ++s) tot += v[s];
+    for (int s = 0; s < KS; ++s) tot += v[s];
     return tot;
 }
-// Two consecutive elements (idx % 2 == 0).
-__device__ __forceinline__ f2 slab_sum2(const void *partial, long idx, long slab_stride, int ksplit) {
-    const float *p = reinterpret_cast<const float *>(partial) + idx;
-    f2 v[SMH_MAX_KSPLIT];
-#pragma unroll
-    for (int s = 0; s < SMH_MAX_KSPLIT; ++s) v[s] = (s < ksplit) ? *reinterpret_cast<const f2 *>(p + s * slab_stride) : f2{0.f, 0.f};
-    f2 tot = {0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < SMH_MAX_KSPLIT; ++s) tot += v[s];
-    return tot;
-}
-// Four consecutive elements (idx % 4 == 0).
+// Four consecutive elements of `ksplit` slabs, added.
 __device__ __forceinline__ f4 slab_sum4(const void *partial, long idx, long slab_stride, int ksplit) {
     const float *p = reinterpret_cast<const float *>(partial) + idx;
     f4 v[SMH_MAX_KSPLIT];
 #pragma unroll
     for (int s = 0; s < SMH_MAX_KSPLIT; ++s) v[s] = (s < ksplit) ? *reinterpret_cast<const f4 *>(p + s * slab_stride) : f4{0.f, 0.f, 0.f, 0.f};
-    f4 tot = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < SMH_MAX_KSPLIT; ++s) tot += v[s];
-    return tot;
+    return slab_add(v);
 }
 
 }  // namespace smh
