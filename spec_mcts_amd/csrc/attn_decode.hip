@@ -20,6 +20,7 @@
 // Algorithmic HBM traffic: prefix 2*P*Hkv*D*2 B once + per branch its suffix rows
 // (512 B fp16 or 136 B Q4_0 per row and kv head) + q/out.
 #include <mutex>
+#include <type_traits>
 
 #include "attn_rows.hpp"
 #include "rope_kv.hpp"
@@ -335,11 +336,26 @@ __global__ __launch_bounds__(256) void attn_prefix_kernel(AttnParams p) {
 // output's fp16).  Where nothing is shared the pass costs its 3 us (100 positions, 99 branches: 29.7 -> 26.5 with the walk's gain).
 constexpr int PT_TW = 64;
 constexpr int PT_MAX_SLICES = 64;          // one bit a slice in the suffix kernel's mask
-__device__ __forceinline__ long page_at(const AttnParams &p, long i) {
+// PB: bytes of a page id, 0 without a page table; PB_ANY: what the parameters say.  Kernels that walk know it when they are compiled: a load
+// behind a branch on the width was waited for with everything else on its way, rows of the next batch among them.
+constexpr int PB_ANY = -1;
+template <int PB> using page_id_t = std::conditional_t<PB == 2 || PB == 4 || PB == 0, int, long>;
+template <int PB>
+__device__ __forceinline__ page_id_t<PB> page_at(const AttnParams &p, long i) {
+    if constexpr (PB == 4) return reinterpret_cast<const int32_t *>(p.pages)[i];
+    if constexpr (PB == 2) return reinterpret_cast<const int16_t *>(p.pages)[i];
+    if constexpr (PB == 8) return reinterpret_cast<const int64_t *>(p.pages)[i];
     if (p.page_bytes == 4) return reinterpret_cast<const int32_t *>(p.pages)[i];
     if (p.page_bytes == 2) return reinterpret_cast<const int16_t *>(p.pages)[i];
     return reinterpret_cast<const int64_t *>(p.pages)[i];
 }
+// the pool row of a page id (ids outside the pool are cut at its ends)
+template <int PB>
+__device__ __forceinline__ long page_row(const AttnParams &p, page_id_t<PB> id) {
+    if constexpr (PB == 2 || PB == 4) return min(max(id, 0), (int)min(p.pool_rows - 1, 0x7fffffffL));
+    return min(max((long)id, 0L), p.pool_rows - 1);
+}
+template <int PB>
 __global__ __launch_bounds__(256) void attn_page_tile_kernel(AttnParams p) {
     __shared__ __attribute__((aligned(16))) half_t ks[PT_TW][ATT_KPITCH];
     __shared__ __attribute__((aligned(16))) half_t vt[ATT_D][PT_TW + 8];
@@ -354,16 +370,14 @@ __global__ __launch_bounds__(256) void attn_page_tile_kernel(AttnParams p) {
     bool same = true;
     {
         const int pos = t0 + min(lane, cnt - 1);
-        const long id0 = page_at(p, (long)b_lo * p.pages_stride + pos);
-        for (int b = b_lo + 1 + wave; b <= b_hi; b += 4) same &= page_at(p, (long)b * p.pages_stride + pos) == id0;
-        if (wave == 0) s_row[lane] = min(max(id0, 0L), p.pool_rows - 1);
+        page_id_t<PB> id[5];                       // the first branch's, and those of every fourth other one (past the last: again)
+#pragma unroll
+        for (int i = 0; i < 5; ++i) id[i] = page_at<PB>(p, (long)(i == 0 ? b_lo : min(b_lo + 1 + wave + 4 * (i - 1), b_hi)) * p.pages_stride + pos);
+#pragma unroll
+        for (int i = 1; i < 5; ++i) same &= id[i] == id[0];
+        if (wave == 0) s_row[lane] = page_row<PB>(p, id[0]);
     }
-    uint8_t *done = p.tile_done + ((long)hk * gridDim.z + tile) * p.splits + split;
-    if (!__syncthreads_and(same)) {
-        if (tid == 0) *done = 0;
-        return;
-    }
-    // ---- the query tile (B operand of S^T), then the rows: K row-major, V transposed, as in attn_prefix_body ----
+    // the query tile (B operand of S^T)
     const int qrow = tile * 16 + c, qr = min(qrow, p.Bq - 1);
     h8 qb[4];
     {
@@ -371,6 +385,12 @@ __global__ __launch_bounds__(256) void attn_page_tile_kernel(AttnParams p) {
 #pragma unroll
         for (int k4 = 0; k4 < 4; ++k4) qb[k4] = *reinterpret_cast<const h8 *>(qp + 32 * k4);
     }
+    uint8_t *done = p.tile_done + ((long)hk * gridDim.z + tile) * p.splits + split;
+    if (!__syncthreads_and(same)) {
+        if (tid == 0) *done = 0;
+        return;
+    }
+    // ---- the rows: K row-major, V transposed, as in attn_prefix_body ----
     uint32_t bad = 0;
     {
         const int ch = tid & 15, kg = tid >> 4;
@@ -692,7 +712,7 @@ constexpr int PF_LDS = 8 * PF_TW * ATT_D * 2;              // 128 KB: one workgr
 // WALK: the rows' format where it is known - a kernel that holds both walks needs registers for the larger one.  WALK_TILES:
 // fp16, the slices that tile_done marks are skipped, and only their partials are folded in.
 enum { WALK_ANY, WALK_Q40, WALK_F16, WALK_TILES };
-template <bool FUSED, bool PARTIAL, int WALK = WALK_ANY>
+template <bool FUSED, bool PARTIAL, int WALK = WALK_ANY, int PB = PB_ANY>
 __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int h, int sub = 0, int nsub = 1, bool live = true) {
     constexpr bool TILES = WALK == WALK_TILES;
     const int hk = div_rep(p, h);
@@ -717,10 +737,21 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
     if (p.suffix_format != SMH_KV_NONE) len = p.lens == nullptr ? (int)p.suffix_batch_stride_rows : min(p.lens[(long)b * p.lens_stride], (int)p.suffix_batch_stride_rows);
     const int gg = g + 4 * sub, gstride = 4 * nsub;      // this group's first row and the distance to its next one
     const long row0 = (long)b * p.suffix_batch_stride_rows;     // first suffix row of this branch
-    // pool row that holds suffix position t of this branch
-    auto row_of = [&](int t) -> long {
-        if (p.pages == nullptr) return row0 + t;
-        return min(max(page_at(p, (long)b * p.pages_stride + t), 0L), p.pool_rows - 1);
+    // page id of suffix position t of this branch, as it comes from memory, and the pool row that it means
+    typedef page_id_t<PB> id_t;
+    auto id_of = [&](int t) -> id_t {
+        if constexpr (PB == PB_ANY) {
+            if (p.pages == nullptr) return row0 + t;
+            return page_row<PB>(p, page_at<PB>(p, (long)b * p.pages_stride + t));
+        } else {
+            if constexpr (PB == 0) return t;
+            else return page_at<PB>(p, (long)b * p.pages_stride + t);
+        }
+    };
+    auto row_of = [&](id_t id) -> long {
+        if constexpr (PB == PB_ANY) return id;
+        else if constexpr (PB == 0) return row0 + id;
+        else return page_row<PB>(p, id);
     };
     // ---- Q4_0 suffix rows: a wave takes Q4_ROWS rows per pass (row slot Q4_DW g + rl) and Q4_CH passes per chunk; wave
     // `sub` of the nsub that share a query takes every nsub-th pass.  All loads of a chunk are requested together, and
@@ -734,14 +765,14 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
     const int q4_mine = q4_passes > sub ? (q4_passes - sub + nsub - 1) / nsub : 0;                // passes of this wave
     const int q4_chunks = (q4_mine + Q4_CH - 1) / Q4_CH;
     auto q4_pos = [&](int n, int u) { return Q4_ROWS * (sub + nsub * (Q4_CH * n + u)) + Q4_DW * g + rl; };  // suffix position of this lane's row
-    auto q4_ids = [&](int n, long (&id)[Q4_CH]) {
+    auto q4_ids = [&](int n, id_t (&id)[Q4_CH]) {
 #pragma unroll
-        for (int u = 0; u < Q4_CH; ++u) id[u] = row_of(min(q4_pos(n, u), len - 1));               // rows past the end repeat the last one
+        for (int u = 0; u < Q4_CH; ++u) id[u] = id_of(min(q4_pos(n, u), len - 1));                // rows past the end repeat the last one
     };
-    auto q4_rows = [&](const long (&id)[Q4_CH], Q4Chunk &ck) {
+    auto q4_rows = [&](const id_t (&id)[Q4_CH], Q4Chunk &ck) {
 #pragma unroll
         for (int u = 0; u < Q4_CH; ++u) {
-            const long row = id[u] * p.Hkv + hk;
+            const long row = row_of(id[u]) * p.Hkv + hk;
             ck.k[u] = *reinterpret_cast<const q4_reg_t *>((const uint8_t *)p.suffix_k + row * 64 + 4 * Q4_DW * e);
             ck.v[u] = *reinterpret_cast<const q4_reg_t *>((const uint8_t *)p.suffix_v + row * 64 + 4 * Q4_DW * e);
             ck.ks[u] = *reinterpret_cast<const uint32_t *>(p.suffix_ks + row * 2);
@@ -749,7 +780,7 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
         }
     };
     Q4Chunk q4_first;                                       // chunk 0, requested as early as the length is known
-    long q4_next_id[Q4_CH];                                 // page ids of the chunk after the one in flight
+    id_t q4_next_id[Q4_CH];                                 // page ids of the chunk after the one in flight
     auto q4_prime = [&]() {
         if (q4_chunks > 0) {
             q4_ids(0, q4_next_id);
@@ -802,9 +833,21 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
     }
 
     {
-        RowRegs qr;
-        if (!FUSED) qr = row_from_fp16(p.q + ((long)b * p.H + h) * ATT_D, c);
-        else qr = q_first;
+        // Not FUSED: the query (in the walk over Q4_0 rows its dims this lane holds of a row, pieces Q4_DW e + j, c among them) and the new
+        // token's rows are requested here and used behind the first rows of the walk.
+        constexpr bool Q4_ONLY = WALK == WALK_Q40;
+        constexpr int NQ = Q4_ONLY ? Q4_DW : 1;
+        const half_t *q_ptr = FUSED ? nullptr : p.q + ((long)b * p.H + h) * ATT_D;
+        RawRow q_raw[NQ], cur_raw[2];
+        if constexpr (!FUSED) {
+#pragma unroll
+            for (int j = 0; j < NQ; ++j) q_raw[j] = raw_row(q_ptr, Q4_ONLY ? Q4_DW * e + j : c);
+            if constexpr (WALK < WALK_F16) {                // (the fp16 walk needs the registers)
+                const long off = ((long)b * p.Hkv + hk) * ATT_D;
+                cur_raw[0] = raw_row(p.cur_k != nullptr ? p.cur_k + off : q_ptr, c);
+                cur_raw[1] = raw_row(p.cur_k != nullptr ? p.cur_v + off : q_ptr, c);
+            }
+        }
         SoftState st;
         st.m = -INFINITY;
         st.l = 0.f;
@@ -816,18 +859,6 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
         // ---- loads for the end of the pass: the new token's exact K/V, the first two prefix partials ----
         const int qrow = b * p.n_rep + (h - hk * p.n_rep);
         const bool has_cur = (FUSED || p.cur_k != nullptr) && g == 0 && sub == 0;
-        RowRegs cur_kr = qr, cur_vr = qr;
-        auto load_cur = [&]() {
-            if (FUSED) {
-                cur_kr = row_from_fp16(&s_kv[wave][0][0], c);
-                cur_vr = row_from_fp16(&s_kv[wave][1][0], c);
-            } else {
-                const long off = ((long)b * p.Hkv + hk) * ATT_D;
-                cur_kr = row_from_fp16(p.cur_k + off, c);
-                cur_vr = row_from_fp16(p.cur_v + off, c);
-            }
-        };
-        if (WALK < WALK_F16 && has_cur) load_cur();        // (the fp16 walk needs the registers)
         constexpr int PRE = WALK < WALK_F16 ? 2 : 0;
         f4 pre_lo[PRE + 1], pre_hi[PRE + 1];
         float pre_m[PRE + 1], pre_l[PRE + 1];
@@ -857,23 +888,30 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
                 return i;
             };
             struct Batch { u32x2 kl[U], kh[U], vl[U], vh[U]; };
-            int id[U];                                      // (rows of 256 bytes and more: their number fits)
+            std::conditional_t<PB == PB_ANY, int, id_t> id[U];         // (rows of 256 bytes and more: their number fits)
             auto ids = [&](int i) {
 #pragma unroll
-                for (int u = 0; u < U; ++u) id[u] = (int)row_of(min(span * i + gg + gstride * u, len - 1));       // past the end: the last row again
+                for (int u = 0; u < U; ++u) id[u] = id_of(min(span * i + gg + gstride * u, len - 1));             // past the end: the last row again
             };
             auto rows = [&](Batch &r) {
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    const long off = (long)id[u] * p.sfx_row_stride + (long)hk * p.sfx_head_stride + 4 * c;
+                    const long off = row_of(id[u]) * p.sfx_row_stride + (long)hk * p.sfx_head_stride + 4 * c;
                     r.kl[u] = *reinterpret_cast<const u32x2 *>((const half_t *)p.suffix_k + off);
                     r.kh[u] = *reinterpret_cast<const u32x2 *>((const half_t *)p.suffix_k + off + 64);
                     r.vl[u] = *reinterpret_cast<const u32x2 *>((const half_t *)p.suffix_v + off);
                     r.vh[u] = *reinterpret_cast<const u32x2 *>((const half_t *)p.suffix_v + off + 64);
                 }
             };
-            const u32x2 ql = {pack_lo16(as_u32(qr.a02), as_u32(qr.a13)), pack_hi16(as_u32(qr.a02), as_u32(qr.a13))};       // dims (0,1), (2,3)
-            const u32x2 qh = {pack_lo16(as_u32(qr.b02), as_u32(qr.b13)), pack_hi16(as_u32(qr.b02), as_u32(qr.b13))};
+            // dims (0,1), (2,3)
+            u32x2 ql, qh;
+            if constexpr (FUSED) {
+                ql = u32x2{pack_lo16(as_u32(q_first.a02), as_u32(q_first.a13)), pack_hi16(as_u32(q_first.a02), as_u32(q_first.a13))};
+                qh = u32x2{pack_lo16(as_u32(q_first.b02), as_u32(q_first.b13)), pack_hi16(as_u32(q_first.b02), as_u32(q_first.b13))};
+            } else {
+                ql = q_raw[0].lo;
+                qh = q_raw[0].hi;
+            }
             int i0 = next(-1), i1 = n_batches;
             Batch cur;
             if (i0 < n_batches) {
@@ -936,7 +974,7 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
             RowRegs qj[Q4_DW];                              // the query's dims this lane holds of a row: pieces Q4_DW e + j
 #pragma unroll
             for (int j = 0; j < Q4_DW; ++j)
-                qj[j] = FUSED ? row_from_fp16(&s_kv[wave][2][0], Q4_DW * e + j) : row_from_fp16(p.q + ((long)b * p.H + h) * ATT_D, Q4_DW * e + j);
+                qj[j] = FUSED ? row_from_fp16(&s_kv[wave][2][0], Q4_DW * e + j) : Q4_ONLY ? row_of_raw(q_raw[j < NQ ? j : 0]) : row_from_fp16(q_ptr, Q4_DW * e + j);
             float m = -INFINITY, l = 0.f;                   // m: common to the group; l, o: of this lane's row slot
             float o[Q4_DW][8];
 #pragma unroll
@@ -1018,8 +1056,33 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
             }
         }
         // ---- the new token's exact K/V (group 0 only) ----
-        if (WALK >= WALK_F16 && has_cur) load_cur();
-        if (has_cur) soft_add_row(st, row_dot(cur_kr, qr) * p.scale_log2, cur_vr);
+        if (has_cur) {
+            RowRegs qr, kr, vr;
+            if constexpr (FUSED) {
+                qr = q_first;
+                kr = row_from_fp16(&s_kv[wave][0][0], c);
+                vr = row_from_fp16(&s_kv[wave][1][0], c);
+            } else {
+                RawRow q_c = q_raw[0];                      // piece c
+#pragma unroll
+                for (int j = 1; j < NQ; ++j)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        q_c.lo[i] = rl == j ? q_raw[j].lo[i] : q_c.lo[i];
+                        q_c.hi[i] = rl == j ? q_raw[j].hi[i] : q_c.hi[i];
+                    }
+                qr = row_of_raw(q_c);
+                if constexpr (WALK >= WALK_F16) {
+                    const long off = ((long)b * p.Hkv + hk) * ATT_D;
+                    kr = row_from_fp16(p.cur_k + off, c);
+                    vr = row_from_fp16(p.cur_v + off, c);
+                } else {
+                    kr = row_of_raw(cur_raw[0]);
+                    vr = row_of_raw(cur_raw[1]);
+                }
+            }
+            soft_add_row(st, row_dot(kr, qr) * p.scale_log2, vr);
+        }
         // ---- prefix partials: the group folds in splits gg, gg + gstride, ... ----
 #pragma unroll
         for (int i = 0; i < PRE; ++i) {
@@ -1076,7 +1139,7 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
 
 // (four waves a SIMD: with three, the 3168 waves of 99 branches x 32 heads left a second round of a few; 99 branches x 32 heads over 768
 // positions of a page table 171 -> 150 us)
-template <bool FUSED, int WALK>
+template <bool FUSED, int WALK, int PB>
 __global__ __launch_bounds__(256, FUSED ? 1 : 4) void attn_suffix_kernel(AttnParams p) {
     // suffix_waves (1, 2 or 4) waves per (branch, query head): more than one while branches x heads leave CUs idle.
     // Workgroups are dealt round-robin to the 8 XCDs (8 L2s); the heads of one branch share the 128-byte lines of that
@@ -1093,7 +1156,7 @@ __global__ __launch_bounds__(256, FUSED ? 1 : 4) void attn_suffix_kernel(AttnPar
     const int h = nsub == 4 ? hq >> 2 : (nsub == 2 ? hq >> 1 : hq);
     if (nsub == 1 && h >= p.H) return;
     // with shared queries every wave reaches the fold's barrier: one past the last head repeats it and writes nothing
-    attn_suffix_body<FUSED, false, WALK>(p, b, min(h, p.H - 1), hq & (nsub - 1), nsub, h < p.H);
+    attn_suffix_body<FUSED, false, WALK, PB>(p, b, min(h, p.H - 1), hq & (nsub - 1), nsub, h < p.H);
 }
 
 // ---- prefix slices and suffix walks side by side, then a merge ------------------------------------------------------
@@ -1212,6 +1275,7 @@ __device__ __forceinline__ void attn_prefix_round(const AttnParams &p, int split
 }
 
 // prefix_wgs: a multiple of 8, so that the others sit on the XCDs that attn_suffix_kernel's would
+template <int PB>
 __global__ __launch_bounds__(256, 4) void attn_parts_kernel(AttnParams p, int prefix_wgs, int rounds) {
     int L = blockIdx.x;
     if (L < prefix_wgs) {
@@ -1224,7 +1288,7 @@ __global__ __launch_bounds__(256, 4) void attn_parts_kernel(AttnParams p, int pr
     if (b >= p.B) return;
     const int hq = (j - grp * per_branch) * 4 + wave, h = nsub == 4 ? hq >> 2 : (nsub == 2 ? hq >> 1 : hq);
     if (nsub == 1 && h >= p.H) return;
-    attn_suffix_body<false, true, WALK_F16>(p, b, min(h, p.H - 1), hq & (nsub - 1), nsub, h < p.H);
+    attn_suffix_body<false, true, WALK_F16, PB>(p, b, min(h, p.H - 1), hq & (nsub - 1), nsub, h < p.H);
 }
 
 // One wave per query adds its splits + 1 partials up, in split order: lane d holds dims 2 d, 2 d + 1.
@@ -1274,7 +1338,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p) {
 // FUSED: q and the new token's k, v come from the wq|wk|wv slabs (up to 16 branches); otherwise from p.q, p.cur_k/v.
 constexpr int ATT_ONE_MAX_TILES = ATT_FUSED_MAX_Q / 16;
 
-template <bool FUSED>
+template <bool FUSED, int PB>
 __global__ __launch_bounds__(256, 2) void attn_one_kernel(AttnParams p) {
     __shared__ uint32_t s_last[ATT_ONE_MAX_TILES];
     const int hk = blockIdx.y;
@@ -1289,7 +1353,7 @@ __global__ __launch_bounds__(256, 2) void attn_one_kernel(AttnParams p) {
         const int j = (int)blockIdx.x - p.splits, wave_ = tid >> 6;
         const int qrow = per_wg * j + (wave_ >> sw_shift);        // query of this kv head: branch qrow / n_rep, its query head qrow % n_rep
         const int qc = min(qrow, p.Bq - 1);
-        attn_suffix_body<FUSED, true>(p, div_rep(p, qc), hk * p.n_rep + mod_rep(p, qc), wave_ & (p.suffix_waves - 1), p.suffix_waves, qrow < p.Bq);
+        attn_suffix_body<FUSED, true, FUSED ? WALK_Q40 : WALK_ANY, PB>(p, div_rep(p, qc), hk * p.n_rep + mod_rep(p, qc), wave_ & (p.suffix_waves - 1), p.suffix_waves, qrow < p.Bq);
         tile_lo = tile_hi = (per_wg * j) / 16;  // a workgroup's 1, 2 or 4 consecutive queries never straddle a tile of 16
     }
     wait_vmem();                               // this wave's partials have reached memory ...
@@ -1521,7 +1585,7 @@ static int shared_prefix_attn(const char *who, bool one, const void *q, void *ou
         p.counters = (uint32_t *)workspace;
         p.part_o = (float *)((char *)workspace + ATT_COUNTER_BYTES);
         p.part_ml = p.part_o + n_part * ATT_D;
-        hipLaunchKernelGGL(attn_one_kernel<false>, dim3(p.splits + (p.Bq + 4 / p.suffix_waves - 1) / (4 / p.suffix_waves), Hkv), dim3(256), 0, (hipStream_t)stream, p);
+        hipLaunchKernelGGL((attn_one_kernel<false, PB_ANY>), dim3(p.splits + (p.Bq + 4 / p.suffix_waves - 1) / (4 / p.suffix_waves), Hkv), dim3(256), 0, (hipStream_t)stream, p);
         return launch_status();
     }
     size_t n_part = (size_t)p.splits * Hkv * p.Bq;
@@ -1531,13 +1595,15 @@ static int shared_prefix_attn(const char *who, bool one, const void *q, void *ou
     p.part_ml = p.part_o + n_part * ATT_D;
     p.suffix_waves = attn_plan_suffix_waves_two((long)B * H);
     const unsigned wgs = (unsigned)(((H * p.suffix_waves + 3) / 4) * ((B + 7) / 8 * 8));
+    const int pb = p.pages == nullptr ? 0 : p.page_bytes;
     const size_t n_parts = (size_t)(p.splits + 1) * Hkv * p.Bq;
     const int rounds = ((p.Bq + 15) / 16 + 3) / 4;
     const long prefix_wgs = ((long)p.splits * Hkv * rounds + 7) / 8 * 8;
     if (p.splits > 0 && suffix_format == SMH_KV_FP16 && workspace_bytes >= n_parts * (ATT_D + 2) * sizeof(float) && prefix_wgs + wgs < (1L << 31)) {
         p.part_ml = p.part_o + n_parts * ATT_D;
         const dim3 grid((unsigned)(prefix_wgs + wgs));
-        hipLaunchKernelGGL(attn_parts_kernel, grid, dim3(256), 0, (hipStream_t)stream, p, (int)prefix_wgs, rounds);
+        const auto parts = pb == 0 ? attn_parts_kernel<0> : pb == 2 ? attn_parts_kernel<2> : pb == 4 ? attn_parts_kernel<4> : attn_parts_kernel<8>;
+        hipLaunchKernelGGL(parts, grid, dim3(256), 0, (hipStream_t)stream, p, (int)prefix_wgs, rounds);
         hipLaunchKernelGGL(attn_merge_kernel, dim3((unsigned)(((long)Hkv * p.Bq + 3) / 4)), dim3(256), 0, (hipStream_t)stream, p);
         return launch_status();
     }
@@ -1551,12 +1617,17 @@ static int shared_prefix_attn(const char *who, bool one, const void *q, void *ou
         n_part = (size_t)p.splits * Hkv * p.Bq;
         p.part_ml = p.part_o + n_part * ATT_D;
         p.tile_done = (uint8_t *)(p.part_ml + n_part * 2);
-        hipLaunchKernelGGL(attn_page_tile_kernel, dim3(Hkv, p.splits, tiles), dim3(256), 0, (hipStream_t)stream, p);
-        hipLaunchKernelGGL((attn_suffix_kernel<false, WALK_TILES>), dim3(wgs), dim3(256), 0, (hipStream_t)stream, p);
+        const auto shared = pb == 2 ? attn_page_tile_kernel<2> : pb == 4 ? attn_page_tile_kernel<4> : attn_page_tile_kernel<8>;
+        const auto walk = pb == 2 ? attn_suffix_kernel<false, WALK_TILES, 2> : pb == 4 ? attn_suffix_kernel<false, WALK_TILES, 4> : attn_suffix_kernel<false, WALK_TILES, 8>;
+        hipLaunchKernelGGL(shared, dim3(Hkv, p.splits, tiles), dim3(256), 0, (hipStream_t)stream, p);
+        hipLaunchKernelGGL(walk, dim3(wgs), dim3(256), 0, (hipStream_t)stream, p);
         return launch_status();
     }
-    if (suffix_format == SMH_KV_FP16) hipLaunchKernelGGL((attn_suffix_kernel<false, WALK_F16>), dim3(wgs), dim3(256), 0, (hipStream_t)stream, p);
-    else hipLaunchKernelGGL((attn_suffix_kernel<false, WALK_Q40>), dim3(wgs), dim3(256), 0, (hipStream_t)stream, p);
+    const auto f16 = pb == 0 ? attn_suffix_kernel<false, WALK_F16, 0> : pb == 2 ? attn_suffix_kernel<false, WALK_F16, 2>
+                     : pb == 4 ? attn_suffix_kernel<false, WALK_F16, 4> : attn_suffix_kernel<false, WALK_F16, 8>;
+    const auto q40 = pb == 0 ? attn_suffix_kernel<false, WALK_Q40, 0> : pb == 2 ? attn_suffix_kernel<false, WALK_Q40, 2>
+                     : pb == 4 ? attn_suffix_kernel<false, WALK_Q40, 4> : attn_suffix_kernel<false, WALK_Q40, 8>;
+    hipLaunchKernelGGL(suffix_format == SMH_KV_FP16 ? f16 : q40, dim3(wgs), dim3(256), 0, (hipStream_t)stream, p);
     return launch_status();
 }
 
@@ -1745,7 +1816,7 @@ extern "C" int smh_shared_prefix_attn_qkv(const void *qkv_partial, int ksplit, v
         p.counters = (uint32_t *)workspace;
         p.part_o = (float *)((char *)workspace + ATT_COUNTER_BYTES);
         p.part_ml = p.part_o + n_part * ATT_D;
-        hipLaunchKernelGGL(attn_one_kernel<true>, dim3(p.splits + (p.Bq + 4 / p.suffix_waves - 1) / (4 / p.suffix_waves), Hkv), dim3(256), 0, (hipStream_t)stream, p);
+        hipLaunchKernelGGL((pages != nullptr ? attn_one_kernel<true, 4> : attn_one_kernel<true, 0>), dim3(p.splits + (p.Bq + 4 / p.suffix_waves - 1) / (4 / p.suffix_waves), Hkv), dim3(256), 0, (hipStream_t)stream, p);
         return launch_status();
     }
     size_t n_part = (size_t)p.splits * Hkv * p.Bq;
@@ -1756,7 +1827,7 @@ extern "C" int smh_shared_prefix_attn_qkv(const void *qkv_partial, int ksplit, v
     if (p.splits > 0)
         hipLaunchKernelGGL(attn_prefix_kernel<true>, dim3(p.splits, Hkv, qgroups), dim3(256), 0, (hipStream_t)stream, p);
     p.suffix_waves = attn_plan_suffix_waves_two((long)B * H);
-    hipLaunchKernelGGL((attn_suffix_kernel<true, WALK_Q40>), dim3((unsigned)(((H * p.suffix_waves + 3) / 4) * ((B + 7) / 8 * 8))), dim3(256), 0, (hipStream_t)stream, p);
+    hipLaunchKernelGGL((pages != nullptr ? attn_suffix_kernel<true, WALK_Q40, 4> : attn_suffix_kernel<true, WALK_Q40, 0>), dim3((unsigned)(((H * p.suffix_waves + 3) / 4) * ((B + 7) / 8 * 8))), dim3(256), 0, (hipStream_t)stream, p);
     return launch_status();
 }
 

@@ -13,16 +13,20 @@ namespace smh {
 // produces.
 struct RowRegs { h2 a02, a13, b02, b13; };   // a: dims 4c.., b: dims 64+4c..
 
-__device__ __forceinline__ RowRegs row_from_fp16(const half_t *row, int c) {
-    const u32x2 lo = *reinterpret_cast<const u32x2 *>(row + 4 * c);
-    const u32x2 hi = *reinterpret_cast<const u32x2 *>(row + 64 + 4 * c);
+// (as it comes from memory, so that a caller can request a row early and wait for it where it is used)
+struct RawRow { u32x2 lo, hi; };
+__device__ __forceinline__ RawRow raw_row(const half_t *row, int c) {
+    return RawRow{*reinterpret_cast<const u32x2 *>(row + 4 * c), *reinterpret_cast<const u32x2 *>(row + 64 + 4 * c)};
+}
+__device__ __forceinline__ RowRegs row_of_raw(const RawRow &t) {
     RowRegs r;
-    r.a02 = as_h2(pack_lo16(lo[0], lo[1]));
-    r.a13 = as_h2(pack_hi16(lo[0], lo[1]));
-    r.b02 = as_h2(pack_lo16(hi[0], hi[1]));
-    r.b13 = as_h2(pack_hi16(hi[0], hi[1]));
+    r.a02 = as_h2(pack_lo16(t.lo[0], t.lo[1]));
+    r.a13 = as_h2(pack_hi16(t.lo[0], t.lo[1]));
+    r.b02 = as_h2(pack_lo16(t.hi[0], t.hi[1]));
+    r.b13 = as_h2(pack_hi16(t.hi[0], t.hi[1]));
     return r;
 }
+__device__ __forceinline__ RowRegs row_from_fp16(const half_t *row, int c) { return row_of_raw(raw_row(row, c)); }
 // bytes: this lane's dword of the packed row; sc: (scale of dims 0..63, scale of dims 64..127)
 __device__ __forceinline__ RowRegs row_from_q40(uint32_t bytes, uint32_t sc) {
     const uint32_t u = bytes ^ NIBBLE_FLIP, u1 = u >> 8;
