@@ -336,6 +336,10 @@ __global__ __launch_bounds__(256) void attn_prefix_kernel(AttnParams p) {
 // output's fp16).  Where nothing is shared the pass costs its 3 us (100 positions, 99 branches: 29.7 -> 26.5 with the walk's gain).
 constexpr int PT_TW = 64;
 constexpr int PT_MAX_SLICES = 64;          // one bit a slice in the suffix kernel's mask
+// Waits for a wave's loads where a loop that keeps a batch on its way begins.  With the first batch still on its way there, the compiler, which
+// counts loads, waits in every pass for as much as the first one needs: for the next batch, too.
+__device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0f70); }       // vmcnt(0)
+
 // PB: bytes of a page id, 0 without a page table; PB_ANY: what the parameters say.  Kernels that walk know it when they are compiled: a load
 // behind a branch on the width was waited for with everything else on its way, rows of the next batch among them.
 constexpr int PB_ANY = -1;
@@ -920,6 +924,7 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
                 i1 = next(i0);
                 if (i1 < n_batches) ids(i1);
             }
+            wait_loads();
             while (i0 < n_batches) {
                 Batch nxt;
                 int i2 = n_batches;
@@ -982,6 +987,7 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
 #pragma unroll
                 for (int k = 0; k < 8; ++k) o[j][k] = 0.f;
             Q4Chunk cur = q4_first;
+            wait_loads();
             for (int n = 0; n < q4_chunks; ++n) {
                 Q4Chunk nxt;
                 if (n + 1 < q4_chunks) {
