@@ -79,46 +79,23 @@ struct AttnParams {
 __device__ __forceinline__ int div_rep(const AttnParams &p, int x) { return p.n_rep == 1 ? x : x / p.n_rep; }
 __device__ __forceinline__ int mod_rep(const AttnParams &p, int x) { return p.n_rep == 1 ? 0 : x % p.n_rep; }
 
-// column `col` of branch b in the fused q|k|v product: the slabs added in slice order, rounded once to fp16
-__device__ __forceinline__ half_t qkv_value(const AttnParams &p, int b, int col) {
-    const int cols = (p.H + 2 * p.Hkv) * ATT_D;
-    const float *src = p.qkv + (long)b * cols + col;
-    const long slab = (long)p.B * cols;
-    float v[16];
-#pragma unroll
-    for (int s_ = 0; s_ < 16; ++s_) v[s_] = (s_ < p.qkv_ks) ? src[s_ * slab] : 0.f;
-    float tot = 0.f;
-#pragma unroll
-    for (int s_ = 0; s_ < 16; ++s_) tot += v[s_];
-    return (half_t)tot;
-}
-// the same in two steps, so that a caller can request several columns before it waits for any of them
-struct SlabColumn { float v[16]; };
-__device__ __forceinline__ void qkv_request(const AttnParams &p, int b, int col, SlabColumn &c) {
+// Columns `col` .. (T: float or f4) of branch b in the fused q|k|v product, requested and then added in slice order; at most QKS slabs.  No
+// condition on a load (past the last slab: that one again, counted as zero): behind one the compiler waited for what it had before it
+// requested the rest.
+template <typename T, int QKS>
+__device__ __forceinline__ void qkv_request(const AttnParams &p, int b, int col, T (&v)[QKS]) {
     const int cols = (p.H + 2 * p.Hkv) * ATT_D;
     const float *src = p.qkv + (long)b * cols + col;
     const long slab = (long)p.B * cols;
 #pragma unroll
-    for (int s_ = 0; s_ < 16; ++s_) c.v[s_] = (s_ < p.qkv_ks) ? src[s_ * slab] : 0.f;
+    for (int s_ = 0; s_ < QKS; ++s_) v[s_] = *reinterpret_cast<const T *>(src + min(s_, p.qkv_ks - 1) * slab);
 }
-__device__ __forceinline__ half_t qkv_sum(const SlabColumn &c) {
-    float tot = 0.f;
+template <typename T, int QKS>
+__device__ __forceinline__ T qkv_sum(const AttnParams &p, const T (&v)[QKS]) {
+    T tot = T{};
 #pragma unroll
-    for (int s_ = 0; s_ < 16; ++s_) tot += c.v[s_];
-    return (half_t)tot;
-}
-// four consecutive columns (col % 4 == 0)
-__device__ __forceinline__ h4 qkv_value4(const AttnParams &p, int b, int col) {
-    const int cols = (p.H + 2 * p.Hkv) * ATT_D;
-    const float *src = p.qkv + (long)b * cols + col;
-    const long slab = (long)p.B * cols;
-    f4 v[16];
-#pragma unroll
-    for (int s_ = 0; s_ < 16; ++s_) v[s_] = (s_ < p.qkv_ks) ? *reinterpret_cast<const f4 *>(src + s_ * slab) : f4{0.f, 0.f, 0.f, 0.f};
-    f4 tot = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s_ = 0; s_ < 16; ++s_) tot += v[s_];
-    return h4{(half_t)tot[0], (half_t)tot[1], (half_t)tot[2], (half_t)tot[3]};
+    for (int s_ = 0; s_ < QKS; ++s_) tot += s_ < p.qkv_ks ? v[s_] : T{};
+    return tot;
 }
 
 // position of prefix row t (0..tw-1) inside an LDS row of V^T: within each block of 32 rows the
@@ -126,14 +103,17 @@ __device__ __forceinline__ h4 qkv_value4(const AttnParams &p, int b, int col) {
 // and of tile 2j+1) are 8 consecutive halves.
 // dims 4cc..4cc+3 (lo) and 64+4cc.. (hi) of the rotated query of head h, branch b: the rotation pairs d and d + 64
 // sit in the same lane
+template <int QKS>
 __device__ __forceinline__ void qkv_query(const AttnParams &p, int b, int h, int pos, int cc, h4 &lo, h4 &hi) {
-    lo = qkv_value4(p, b, h * ATT_D + 4 * cc);
-    hi = qkv_value4(p, b, h * ATT_D + 64 + 4 * cc);
+    f4 lo_v[QKS], hi_v[QKS];
+    qkv_request(p, b, h * ATT_D + 4 * cc, lo_v);
+    qkv_request(p, b, h * ATT_D + 64 + 4 * cc, hi_v);
     const h4 cs = *reinterpret_cast<const h4 *>(p.cos_tab + (long)pos * 64 + 4 * cc);
     const h4 sn = *reinterpret_cast<const h4 *>(p.sin_tab + (long)pos * 64 + 4 * cc);
+    const f4 lo_s = qkv_sum(p, lo_v), hi_s = qkv_sum(p, hi_v);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        half_t x1 = lo[j], x2 = hi[j];
+        half_t x1 = (half_t)lo_s[j], x2 = (half_t)hi_s[j];
         rope_pair2(x1, x2, cs[j], sn[j]);
         lo[j] = x1; hi[j] = x2;
     }
@@ -148,7 +128,8 @@ __device__ __forceinline__ int vt_pos(int t) {
 // COHERENT: the partials are read by another workgroup of the same launch (device-scope stores)
 // TWM: most prefix rows a workgroup takes (p.tw <= TWM), which sizes its LDS
 // qg, n_qg: this workgroup takes the query tiles of rounds qg, qg + n_qg, ... (a round = one tile per wave)
-template <bool FUSED, bool COHERENT, int TWM>
+// QKS: most slabs of the q|k|v product (FUSED)
+template <bool FUSED, bool COHERENT, int TWM, int QKS = 16>
 __device__ __forceinline__ void attn_prefix_body(const AttnParams &p, int split, int hk, int qg = 0, int n_qg = 1) {
     __shared__ __attribute__((aligned(16))) half_t ks[TWM][ATT_KPITCH];
     __shared__ __attribute__((aligned(16))) half_t vt[ATT_D][TWM + 8];
@@ -209,7 +190,7 @@ __device__ __forceinline__ void attn_prefix_body(const AttnParams &p, int split,
         const int pos = *p.pos_dev;
         for (int qr = tid >> 4; qr < p.Bq; qr += 16) {
             h4 lo, hi;
-            qkv_query(p, div_rep(p, qr), hk * p.n_rep + mod_rep(p, qr), pos, cc, lo, hi);
+            qkv_query<QKS>(p, div_rep(p, qr), hk * p.n_rep + mod_rep(p, qr), pos, cc, lo, hi);
             *reinterpret_cast<h4 *>(&qs[qr][4 * cc]) = lo;
             *reinterpret_cast<h4 *>(&qs[qr][64 + 4 * cc]) = hi;
         }
@@ -716,7 +697,7 @@ constexpr int PF_LDS = 8 * PF_TW * ATT_D * 2;              // 128 KB: one workgr
 // WALK: the rows' format where it is known - a kernel that holds both walks needs registers for the larger one.  WALK_TILES:
 // fp16, the slices that tile_done marks are skipped, and only their partials are folded in.
 enum { WALK_ANY, WALK_Q40, WALK_F16, WALK_TILES };
-template <bool FUSED, bool PARTIAL, int WALK = WALK_ANY, int PB = PB_ANY>
+template <bool FUSED, bool PARTIAL, int WALK = WALK_ANY, int PB = PB_ANY, int QKS = 16>
 __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int h, int sub = 0, int nsub = 1, bool live = true) {
     constexpr bool TILES = WALK == WALK_TILES;
     const int hk = div_rep(p, h);
@@ -804,7 +785,7 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
         // exact fp16 for the pass below.
         pos = *p.pos_dev;
         int t = -1;
-        SlabColumn cq1, cq2, ck1, ck2, cv1, cv2;
+        float cq1[QKS], cq2[QKS], ck1[QKS], ck2[QKS], cv1[QKS], cv2[QKS];
         qkv_request(p, b, h * ATT_D + lane, cq1);
         qkv_request(p, b, h * ATT_D + lane + 64, cq2);
         if (sub == 0) {                                            // the wave that owns the new token
@@ -815,9 +796,9 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
         }
         q4_prime();
         const half_t cos_l = p.cos_tab[(long)pos * 64 + lane], sin_l = p.sin_tab[(long)pos * 64 + lane];
-        half_t q1 = qkv_sum(cq1), q2 = qkv_sum(cq2);
+        half_t q1 = (half_t)qkv_sum(p, cq1), q2 = (half_t)qkv_sum(p, cq2);
         half_t k1 = q1, k2 = q1, v1 = q1, v2 = q1;
-        if (sub == 0) { k1 = qkv_sum(ck1); k2 = qkv_sum(ck2); v1 = qkv_sum(cv1); v2 = qkv_sum(cv2); }
+        if (sub == 0) { k1 = (half_t)qkv_sum(p, ck1); k2 = (half_t)qkv_sum(p, ck2); v1 = (half_t)qkv_sum(p, cv1); v2 = (half_t)qkv_sum(p, cv2); }
         rope_pair2(q1, q2, cos_l, sin_l);
         s_kv[wave][2][lane] = q1; s_kv[wave][2][lane + 64] = q2;
         asm volatile("" ::: "memory");                              // the reads below are of another type: keep them behind the writes
@@ -1344,7 +1325,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p) {
 // FUSED: q and the new token's k, v come from the wq|wk|wv slabs (up to 16 branches); otherwise from p.q, p.cur_k/v.
 constexpr int ATT_ONE_MAX_TILES = ATT_FUSED_MAX_Q / 16;
 
-template <bool FUSED, int PB>
+template <bool FUSED, int PB, int QKS = 16>
 __global__ __launch_bounds__(256, 2) void attn_one_kernel(AttnParams p) {
     __shared__ uint32_t s_last[ATT_ONE_MAX_TILES];
     const int hk = blockIdx.y;
@@ -1354,12 +1335,12 @@ __global__ __launch_bounds__(256, 2) void attn_one_kernel(AttnParams p) {
     const int per_wg = 4 >> sw_shift;          // queries of one suffix workgroup (suffix_waves = 1, 2 or 4 waves each)
     int tile_lo = 0, tile_hi = q_tiles - 1;    // query tiles this workgroup contributed to
     if ((int)blockIdx.x < p.splits) {
-        attn_prefix_body<FUSED, true, ATT_ONE_TW>(p, blockIdx.x, hk);
+        attn_prefix_body<FUSED, true, ATT_ONE_TW, QKS>(p, blockIdx.x, hk);
     } else {
-        const int j = (int)blockIdx.x - p.splits, wave_ = tid >> 6;
+        const int j = (int)blockIdx.x - p.splits, wave_ = __builtin_amdgcn_readfirstlane(tid >> 6);
         const int qrow = per_wg * j + (wave_ >> sw_shift);        // query of this kv head: branch qrow / n_rep, its query head qrow % n_rep
         const int qc = min(qrow, p.Bq - 1);
-        attn_suffix_body<FUSED, true, FUSED ? WALK_Q40 : WALK_ANY, PB>(p, div_rep(p, qc), hk * p.n_rep + mod_rep(p, qc), wave_ & (p.suffix_waves - 1), p.suffix_waves, qrow < p.Bq);
+        attn_suffix_body<FUSED, true, FUSED ? WALK_Q40 : WALK_ANY, PB, QKS>(p, div_rep(p, qc), hk * p.n_rep + mod_rep(p, qc), wave_ & (p.suffix_waves - 1), p.suffix_waves, qrow < p.Bq);
         tile_lo = tile_hi = (per_wg * j) / 16;  // a workgroup's 1, 2 or 4 consecutive queries never straddle a tile of 16
     }
     wait_vmem();                               // this wave's partials have reached memory ...
@@ -1822,7 +1803,10 @@ extern "C" int smh_shared_prefix_attn_qkv(const void *qkv_partial, int ksplit, v
         p.counters = (uint32_t *)workspace;
         p.part_o = (float *)((char *)workspace + ATT_COUNTER_BYTES);
         p.part_ml = p.part_o + n_part * ATT_D;
-        hipLaunchKernelGGL((pages != nullptr ? attn_one_kernel<true, 4> : attn_one_kernel<true, 0>), dim3(p.splits + (p.Bq + 4 / p.suffix_waves - 1) / (4 / p.suffix_waves), Hkv), dim3(256), 0, (hipStream_t)stream, p);
+        const auto kern = ksplit <= 8    ? (pages != nullptr ? attn_one_kernel<true, 4, 8> : attn_one_kernel<true, 0, 8>)
+                          : ksplit <= 12 ? (pages != nullptr ? attn_one_kernel<true, 4, 12> : attn_one_kernel<true, 0, 12>)
+                                         : (pages != nullptr ? attn_one_kernel<true, 4, 16> : attn_one_kernel<true, 0, 16>);
+        hipLaunchKernelGGL(kern, dim3(p.splits + (p.Bq + 4 / p.suffix_waves - 1) / (4 / p.suffix_waves), Hkv), dim3(256), 0, (hipStream_t)stream, p);
         return launch_status();
     }
     size_t n_part = (size_t)p.splits * Hkv * p.Bq;
