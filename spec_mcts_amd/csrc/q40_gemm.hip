@@ -1094,7 +1094,7 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_swiglu_kernel(MatmulParams p)
 // In us, before and now: w1|w3 4096 -> 2 x 11008 at 512 rows 112.9 (818 TFLOP/s) and 90.1 (1025), at 300 rows 85.3 and 65.2, 1024 rows 201
 // and 178, 2047 rows 375 (985) and 353 (1047); 8192 -> 2 x 28672 at 640 rows 609 and 515, 2047 rows 1834 and 1693.  wq|wk|wv 4096 -> 12288 at
 // 512 rows 60.3 (855 TFLOP/s) and 53.2 (969), 1024 rows 119 and 106; 8192 -> 10240 at 512 rows 99.6 and 86.8; 5120 -> 5120 at 2047 rows
-// 131 and 122.  The rule: gemm_plan_rows with the costs ROWS_384 and ROWS_192.
+// 131 and 122.  The rules: gemm_swiglu_rows_launch and gemm_wide_fits, with the costs ROWS_384 and ROWS_192.
 template <int TILES, bool SWIGLU> struct WideShape {
     static constexpr int STEPS = SWIGLU ? 1 : 2;                 // of a stage
     static constexpr int W = 6 * 1024, SC = 6 * 128;             // of the six slots: nibbles; scales [octet][nibble][8 rows]
@@ -1124,7 +1124,6 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_wide_kernel
     if (unit >= p.units) return;
     const int m0 = mb * p.block_rows, pieces = (SWIGLU ? p.seg[0].N : p.n_total) / 64;
     const int n_st = p.K / (32 * STEPS);
-    const int rot = (unit * 5) % n_st;                                 // workgroups of a row block start at different stages
     // a piece's weight and its number within the weight
     auto segment_of = [&](int &P) {
         int sg = 0;
@@ -1159,7 +1158,7 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_wide_kernel
 #pragma unroll
         for (int s = 0; s < 6; ++s) w[s] += in_tile[s] * 1024;
         const uint8_t *a_base = reinterpret_cast<const uint8_t *>(p.a);
-        int fetch = rot;
+        int fetch = 0;                                                 // (in K's order: a start of its own for each unit gains nothing here)
         auto issue_stage = [&](int slot_) {
             uint8_t *st = lds + slot_ * STAGE;
             const long off = (long)fetch * STEPS * TILE_BYTES;
@@ -1173,7 +1172,7 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_wide_kernel
 #pragma unroll
                 for (int t = 0; t < TILES; ++t)
                     __builtin_amdgcn_global_load_lds((gptr_t)(arow + k * 64 + a_voff[t]), (lptr_t)(st + S::W + S::SC + (k * TILES + t) * 1024), 16, 0, 0);
-            fetch = fetch + 1 == n_st ? 0 : fetch + 1;
+            ++fetch;
         };
 #pragma unroll
         for (int i = 0; i < SLOTS - 2; ++i)
@@ -1333,14 +1332,8 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_wide_kernel
             const int m = m0 + 16 * t + o_row;
             if (m < p.M && mine) {
                 const f4 v = *reinterpret_cast<const f4 *>(reinterpret_cast<const float *>(lds) + (16 * t + o_row) * OP + 4 * o_lane);
-                if (p.direct) {
-                    *reinterpret_cast<h2 *>(out + (long)m * ldc) = h2{matmul_epilogue(p, v[0], m, n), matmul_epilogue(p, v[1], m, n + 1)};
-                    *reinterpret_cast<h2 *>(out + (long)m * ldc + 4) = h2{matmul_epilogue(p, v[2], m, n + 4), matmul_epilogue(p, v[3], m, n + 5)};
-                } else {
-                    float *slab = p.partial + (long)m * p.n_total + n;
-                    *reinterpret_cast<f2 *>(slab) = f2{v[0], v[1]};
-                    *reinterpret_cast<f2 *>(slab + 4) = f2{v[2], v[3]};
-                }
+                *reinterpret_cast<h2 *>(out + (long)m * ldc) = h2{matmul_epilogue(p, v[0], m, n), matmul_epilogue(p, v[1], m, n + 1)};
+                *reinterpret_cast<h2 *>(out + (long)m * ldc + 4) = h2{matmul_epilogue(p, v[2], m, n + 4), matmul_epilogue(p, v[3], m, n + 5)};
             }
         }
     }
@@ -1446,14 +1439,7 @@ void gemm_fill_plan(MatmulParams &p) {
     p.mblocks = (p.M + p.block_rows - 1) / p.block_rows;
     const int steps = (p.K + 31) / 32;
     if (p.M > GEMM_BM) {
-        const float us = gemm_plan_rows(p, steps, SMH_MAX_KSPLIT, ROWS_256);
-        if (p.tiled && p.ksplit == 1 && p.K % 64 == 0) {                       // q40_gemm_wide_kernel: see ROWS_192
-            MatmulParams w = p;
-            w.units = (p.n_total / 64 + 2) / 3;
-            w.units_pad = (w.units + 7) / 8 * 8;
-            w.kgroups = 3;
-            if (gemm_plan_rows(w, steps, 1, ROWS_192) < 0.97f * us) p = w;
-        }
+        gemm_plan_rows(p, steps, SMH_MAX_KSPLIT, ROWS_256);
         return;
     }
     const long tiles = (long)p.units * p.mblocks;
@@ -1671,6 +1657,16 @@ int gemm_swiglu_rows_launch(MatmulParams p, hipStream_t stream) {
     return launch_status();
 }
 
+// The launch of a direct product whose plan has no K-split, with workgroups of 192 columns (w) where they promise more (slabs, whose
+// bits are those of the checkpoint layout's launch, stay with its kernel).
+static bool gemm_wide_fits(const MatmulParams &p, MatmulParams &w) {
+    if (!p.tiled || !p.direct || p.M <= GEMM_BM || p.ksplit != 1 || p.K % 64 != 0) return false;
+    w = p;
+    const float us = gemm_plan_rows(w, p.K / 32, 1, ROWS_256);
+    w.units = (p.n_total / 64 + 2) / 3;
+    w.units_pad = (w.units + 7) / 8 * 8;
+    return gemm_plan_rows(w, p.K / 32, 1, ROWS_192) < 0.97f * us;
+}
 static int gemm_wide_launch(const MatmulParams &p, hipStream_t stream) {
     static const gemm_kernel_t kern[5] = {q40_gemm_wide_kernel<4, false>, q40_gemm_wide_kernel<5, false>, q40_gemm_wide_kernel<6, false>,
                                           q40_gemm_wide_kernel<7, false>, q40_gemm_wide_kernel<8, false>};
@@ -1691,7 +1687,8 @@ static int gemm_wide_launch(const MatmulParams &p, hipStream_t stream) {
 }
 
 int gemm_launch(const MatmulParams &p, hipStream_t stream) {
-    if (p.kgroups == 3 && p.tiled) return gemm_wide_launch(p, stream);
+    MatmulParams w;
+    if (gemm_wide_fits(p, w)) return gemm_wide_launch(w, stream);
     if (p.kgroups == 2 && p.tiled) return gemm_kg_launch(p, stream);
     return p.tiled ? gemm_launch_layout<true>(p, stream) : gemm_launch_layout<false>(p, stream);
 }

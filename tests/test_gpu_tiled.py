@@ -330,8 +330,7 @@ def test_direct_products(M, K, ns):
                                     (600, 448, [7808]),                    # seven stages, more than the ring holds; eight row tiles
                                     (400, 4096, [4096, 4096, 4096])])
 def test_three_pieces_and_two_k_groups(M, K, ns):
-    """sizes above 128 rows that q40_gemm_wide_kernel takes (its estimate is the smaller one): fp16 results with and without a
-    residual, and the one slab of the same launch"""
+    """sizes above 128 rows that q40_gemm_wide_kernel takes (its estimate is the smaller one): fp16 results with and without a residual"""
     from spec_mcts_amd import kernels as Kn
     ws = [_weight(K, n, 2000 + i + K) for i, n in enumerate(ns)]
     tiled = [Kn.tile_q40(w.cuda(), s.cuda(), K, n) for (w, s), n in zip(ws, ns)]
@@ -340,13 +339,9 @@ def test_three_pieces_and_two_k_groups(M, K, ns):
     assert Kn.matmul_plan(M, K, ns, tiled=True) == 1
     got = Kn.matmul_q40_direct(a.cuda(), tiled)
     with_r = Kn.matmul_q40_direct(a.cuda(), tiled, residual=r.cuda()) if r is not None else got
-    slab = Kn.matmul_q40_partial(a.cuda(), tiled).buf[:M * sum(ns)].view(M, sum(ns)).cpu()
-    col = 0
     for (w, s), n, o, o_r in zip(ws, ns, got, with_r):
         want = O.matmul_q40(a, w, s, (K, n)).float()
         # fp32 sums in another order, one rounding to fp16 each (2^-11): 1e-3 of the value; near zero the sums' own error
         assert torch.allclose(o.cpu().float(), want, rtol=2e-3, atol=2e-3)
-        assert torch.equal(slab[:, col:col + n].half(), o.cpu())
         if r is not None:
             assert torch.equal(o_r.cpu(), (r.float() + o.cpu().float()).half())
-        col += n
