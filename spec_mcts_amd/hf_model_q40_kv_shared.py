@@ -445,13 +445,15 @@ class Transformer(nn.Module):
         norm_in = self._norm_in(B, p.dim, [lin._tiled for lin in (att0.wq, att0.wk, att0.wv)])      # (the library asks again, launch by launch)
         run.decode_step(step_state, ws, bool(one), p.max_seq_len, p.max_batch_size * p.max_seq_len, self._pages(dev), B if norm_in else 0,
                         K.SILU_IN_MAX_M if self.silu_in_matmul else 0, self.attn_from_qkv and not self.per_branch_kv)
-        structs = [self._layer_struct(layer) for layer in self.layers]
-        s = structs[-1]
-        stack_ws = self._stack_workspace(dev, structs[0], B)
+        s = self._layer_struct(self.layers[0])
+        stack_ws = self._stack_workspace(dev, s, B)
         if stack_ws is not None:
+            structs = [s] + [self._layer_struct(layer) for layer in self.layers[1:]]
+            s = structs[-1]
             run.decode_stack(structs, stack_ws)
-        else:
-            for s in structs:
+        else:                              # (layer by layer: the GPU works while the next one's arguments are gathered)
+            for i, layer in enumerate(self.layers):
+                s = self._layer_struct(layer) if i > 0 else s
                 run.decode(s)
         return self._lm_head(run.finish(s, self.norm.weight, self.norm.eps).view(B, 1, p.dim))
 
