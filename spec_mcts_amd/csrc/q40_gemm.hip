@@ -1086,39 +1086,44 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_swiglu_kernel(MatmulParams p)
 // ---- above 128 rows, six slots of weights a workgroup (tiled weights, all of K, one workgroup per compute unit) -------------------
 // A workgroup owns 64 .. 128 rows of A; its twelve multiplying waves - wave (nibble hh, slot s) has one piece's columns of one nibble, two
 // B operands, as in q40_gemm_kernel - work on six pieces (64 columns x 32 rows) a stage:
-//   * SWIGLU: pieces 3 u .. 3 u + 2 of the gate weight and the same of the up weight: 384 columns, where q40_gemm_kernel has 256;
-//   * else pieces 3 u .. 3 u + 2 of the weights laid end to end, of two steps: 192 columns and two K-groups, added through LDS.
+//   * WIDE_SWIGLU: pieces 3 u .. 3 u + 2 of the gate weight and the same of the up weight: 384 columns, where q40_gemm_kernel has 256;
+//   * WIDE_GROUPS: pieces 3 u .. 3 u + 2 of the weights laid end to end, of two steps: 192 columns and two K-groups, added through LDS;
+//   * WIDE_SIX: pieces 6 u .. 6 u + 5, 384 columns.
 // Bound by the matrix and vector pipes, which a third wave on each SIMD keeps busier (0.55 us a step of 128 rows x 384 columns,
 // where 1.5 steps of the 256-column units take 0.63), and by how well its workgroups divide the compute units: w1|w3 of the 7B shape is
 // 232 of them at 512 rows, one round, where 256-column units leave 344, two rounds; wq|wk|wv is 256, where those leave 192.
 // In us, before and now: w1|w3 4096 -> 2 x 11008 at 512 rows 112.9 (818 TFLOP/s) and 90.1 (1025), at 300 rows 85.3 and 65.2, 1024 rows 201
 // and 178, 2047 rows 375 (985) and 353 (1047); 8192 -> 2 x 28672 at 640 rows 609 and 515, 2047 rows 1834 and 1693.  wq|wk|wv 4096 -> 12288 at
 // 512 rows 60.3 (855 TFLOP/s) and 53.2 (969), 1024 rows 119 and 106; 8192 -> 10240 at 512 rows 99.6 and 86.8; 5120 -> 5120 at 2047 rows
-// 131 and 122.  The rules: gemm_swiglu_rows_launch and gemm_wide_fits, with the costs ROWS_384 and ROWS_192.
-template <int TILES, bool SWIGLU> struct WideShape {
-    static constexpr int STEPS = SWIGLU ? 1 : 2;                 // of a stage
+// 131 and 122.  With six pieces, against the faster of the others: 4096 -> 12288 at 1024 rows 101 and 93, 2047 rows 191 (1079) and 181 (1140);
+// 5120 -> 15360 at 1300 rows 226 and 192; 5120 -> 5120 at 2047 rows 120 and 112.  The rules: gemm_swiglu_rows_launch and gemm_wide_fits.
+enum { WIDE_SWIGLU, WIDE_GROUPS, WIDE_SIX };
+template <int TILES, int MODE> struct WideShape {
+    static constexpr int STEPS = MODE == WIDE_GROUPS ? 2 : 1;    // of a stage
+    static constexpr int PIECES = MODE == WIDE_SIX ? 6 : 3;      // of an output row
     static constexpr int W = 6 * 1024, SC = 6 * 128;             // of the six slots: nibbles; scales [octet][nibble][8 rows]
     static constexpr int STAGE = W + SC + STEPS * TILES * 1024;
     static constexpr int SLOTS = 6;
     static constexpr int PER = 9 + STEPS * TILES;                // DMA instructions of a stage
-    static constexpr int OP = 192 + 4;
-    static constexpr int OTILE = 2 * 16 * OP * 4;                // SwiGLU: [gate | up][16][OP] fp32
+    static constexpr int OP = 64 * PIECES + 4;
+    static constexpr int OTILE = (MODE == WIDE_SWIGLU ? 2 : 1) * 16 * OP * 4;      // [16][OP] fp32; SwiGLU: [gate | up][16][OP]
     static constexpr int SUMS = TILES * 16 * OP * 4;             // two K-groups: [row][OP] fp32
-    static constexpr int OUT = SWIGLU ? 2 * OTILE : SUMS;
+    static constexpr int OUT = MODE == WIDE_GROUPS ? SUMS : 2 * OTILE;
     static constexpr int LDS = SLOTS * STAGE > OUT ? SLOTS * STAGE : OUT;
     static_assert(LDS <= 160 * 1024, "ring");
 };
 constexpr int WIDE_WAVES = 12;
 
-template <int TILES, bool SWIGLU>
+template <int TILES, int MODE>
 __global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_wide_kernel(MatmulParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    typedef WideShape<TILES, SWIGLU> S;
-    constexpr int SLOTS = S::SLOTS, PER = S::PER, STAGE = S::STAGE, STEPS = S::STEPS;
+    typedef WideShape<TILES, MODE> S;
+    constexpr int SLOTS = S::SLOTS, PER = S::PER, STAGE = S::STAGE, STEPS = S::STEPS, PIECES = S::PIECES;
+    constexpr bool SWIGLU = MODE == WIDE_SWIGLU;
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63, c = lane & 15, g = lane >> 4;
-    // blockIdx -> (unit of three pieces, row block): each XCD takes a contiguous run of units
+    // blockIdx -> (unit of three or six pieces, row block): each XCD takes a contiguous run of units
     const int at = blockIdx.x % p.units_pad, mb = blockIdx.x / p.units_pad;
     const int unit = (at & 7) * (p.units_pad >> 3) + (at >> 3);
     if (unit >= p.units) return;
@@ -1144,10 +1149,10 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_wide_kernel
         int in_tile[6];
 #pragma unroll
         for (int s = 0; s < 6; ++s) {
-            int P = min(3 * unit + s % 3, pieces - 1);                 // (past the end: the last one again, not stored)
+            int P = min(PIECES * unit + s % PIECES, pieces - 1);       // (past the end: the last one again, not stored)
             const int sg = SWIGLU ? s / 3 : segment_of(P);
             in_tile[s] = P & 3;
-            w[s] = p.seg[sg].w + ((long)(P >> 2) * tiled_steps(p.K) + (SWIGLU ? 0 : s / 3)) * TILE_BYTES;
+            w[s] = p.seg[sg].w + ((long)(P >> 2) * tiled_steps(p.K) + (MODE == WIDE_GROUPS ? s / 3 : 0)) * TILE_BYTES;
         }
 #pragma unroll
         for (int i = 0; i < 3; ++i) {                                  // lanes 0 .. 31: slot 2 i's 128 bytes, the others slot 2 i + 1's
@@ -1200,12 +1205,12 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_wide_kernel
         }
         // the barriers of the epilogue: ring free, one per row tile; ring free, the second group's sums in place, all sums
 #pragma unroll 1
-        for (int t = 0; t < (SWIGLU ? 1 + TILES : 3); ++t) gemm_barrier();
+        for (int t = 0; t < (MODE == WIDE_GROUPS ? 3 : 1 + TILES); ++t) gemm_barrier();
         return;
     }
 
     // nibble, slot; the slot's half - gate (0) or up (1), or K-group - and piece
-    const int hh = wave >= 6 ? 1 : 0, s = wave - 6 * hh, half = s >= 3 ? 1 : 0, k3 = s - 3 * half;
+    const int hh = wave >= 6 ? 1 : 0, s = wave - 6 * hh, half = s >= PIECES ? 1 : 0, k3 = s - 3 * half;
     const uint32_t nib_mask = hh == 0 ? 0x00F000F0u : 0x000F000Fu;
     uint32_t nib_magic = MAGIC_1024;                             // (as in q40_gemm_swiglu_kernel)
     asm volatile("" : "+v"(nib_magic));
@@ -1213,7 +1218,7 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_wide_kernel
     const h2 nib_off = hh == 0 ? h2{(half_t)-72.0f, (half_t)-72.0f} : h2{(half_t)-1032.0f, (half_t)-1032.0f};
     struct Raw { u32x4 wq, sc; };
     const int ws_off = s * 1024 + lane * 16, sc_off = S::W + s * 128 + g * 32 + hh * 16;
-    const int a_off = S::W + S::SC + (SWIGLU ? 0 : half * TILES * 1024) + c * 64 + ((g ^ ((c >> 1) & 3)) << 4);
+    const int a_off = S::W + S::SC + (MODE == WIDE_GROUPS ? half * TILES * 1024 : 0) + c * 64 + ((g ^ ((c >> 1) & 3)) << 4);
     auto load_ws = [&](const uint8_t *st, Raw &r) {
         r.wq = *reinterpret_cast<const u32x4 *>(st + ws_off);
         r.sc = *reinterpret_cast<const u32x4 *>(st + sc_off);
@@ -1273,11 +1278,11 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_wide_kernel
         one_stage();
     }
 
-    // rows of 192 columns: local column 64 k3 + 32 hh + 2 c + o is column 128 (P / 2) + 64 hh + 4 c + 2 (P % 2) + o, P the piece;
+    // rows of 64 PIECES columns: local column 64 k3 + 32 hh + 2 c + o is column 128 (P / 2) + 64 hh + 4 c + 2 (P % 2) + o, P the piece;
     // a thread stores local columns 4 o_lane .. + 3
     constexpr int OP = S::OP;
     const int o_row = tid / 48, o_lane = tid % 48, q = o_lane & 15;
-    int P = 3 * unit + (o_lane >> 4);
+    int P = PIECES * unit + (o_lane >> 4);
     const bool mine = P < pieces;
     const int sg = segment_of(P), out_col = 128 * (P >> 1) + 64 * (q >> 3) + 8 * (q & 7) + 2 * (P & 1);
     half_t *const out = (sg == 0 ? p.seg[0].c : sg == 1 ? p.seg[1].c : p.seg[2].c) + out_col;
@@ -1303,6 +1308,32 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_wide_kernel
                 }
                 *reinterpret_cast<h2 *>(out + (long)m * ldc) = h2{ov[0], ov[1]};
                 *reinterpret_cast<h2 *>(out + (long)m * ldc + 4) = h2{ov[2], ov[3]};
+            }
+        }
+    } else if constexpr (MODE == WIDE_SIX) {
+        // two runs of four columns a thread: local columns 4 o_lane .. and 192 + 4 o_lane ..
+        int P2 = 6 * unit + 3 + (o_lane >> 4);
+        const bool mine2 = P2 < pieces;
+        const int sg2 = segment_of(P2), out_col2 = 128 * (P2 >> 1) + 64 * (q >> 3) + 8 * (q & 7) + 2 * (P2 & 1);
+        half_t *const out2 = (sg2 == 0 ? p.seg[0].c : sg2 == 1 ? p.seg[1].c : p.seg[2].c) + out_col2;
+        const long ldc2 = sg2 == 0 ? p.seg[0].ldc : sg2 == 1 ? p.seg[1].ldc : p.seg[2].ldc;
+        const int n = p.seg[sg].col0 + out_col, n2 = p.seg[sg2].col0 + out_col2;
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            float *otile = reinterpret_cast<float *>(lds + (t & 1) * S::OTILE);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) *reinterpret_cast<f2 *>(&otile[(4 * g + r) * OP + 64 * k3 + 32 * hh + 2 * c]) = f2{acc[0][t][r], acc[1][t][r]};
+            gemm_barrier();
+            const int m = m0 + 16 * t + o_row;
+            if (m < p.M && mine) {
+                const f4 v = *reinterpret_cast<const f4 *>(otile + o_row * OP + 4 * o_lane);
+                *reinterpret_cast<h2 *>(out + (long)m * ldc) = h2{matmul_epilogue(p, v[0], m, n), matmul_epilogue(p, v[1], m, n + 1)};
+                *reinterpret_cast<h2 *>(out + (long)m * ldc + 4) = h2{matmul_epilogue(p, v[2], m, n + 4), matmul_epilogue(p, v[3], m, n + 5)};
+            }
+            if (m < p.M && mine2) {
+                const f4 v = *reinterpret_cast<const f4 *>(otile + o_row * OP + 192 + 4 * o_lane);
+                *reinterpret_cast<h2 *>(out2 + (long)m * ldc2) = h2{matmul_epilogue(p, v[0], m, n2), matmul_epilogue(p, v[1], m, n2 + 1)};
+                *reinterpret_cast<h2 *>(out2 + (long)m * ldc2 + 4) = h2{matmul_epilogue(p, v[2], m, n2 + 4), matmul_epilogue(p, v[3], m, n2 + 5)};
             }
         }
     } else {
@@ -1350,18 +1381,23 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_wide_kernel
 // 128 us, now 77, 5120 x 13824 at 512 rows 138, now 101.)
 // Against measurement at the 7B, 13B, 34B and 70B shapes, 160 .. 2047 rows: 0.87 to 1.17 times the estimate, 1.3 to 1.4 times it
 // for square weights at 160 rows (15 and 19 us: launches).
-struct RowsCost { float step, per_rows, around, busy; };       // us a step, us more a step at 128 rows, us around the loop, and that factor
-constexpr RowsCost ROWS_256 = {0.18f, 0.24f, 4.0f, 1.2f};
+// (us a step, us more a step at 128 rows, us around the loop, that factor, and what the share of busy compute units adds to the rounds)
+struct RowsCost { float step, per_rows, around, busy, more; };
+constexpr RowsCost ROWS_256 = {0.18f, 0.24f, 4.0f, 1.2f, 0.0f};
 // SwiGLU with three pieces a workgroup (384 columns): fitted to the shapes of 7B, 13B, 34B and 70B at 130 .. 2047 rows, within 4 % in
 // the mean.  Taking it where its estimate is the smaller was never slower there than the 256-column units (0.72 .. 0.99 of their time).
-constexpr RowsCost ROWS_384 = {0.21f, 0.37f, 4.0f, 1.15f};
+constexpr RowsCost ROWS_384 = {0.21f, 0.37f, 4.0f, 1.15f, 0.0f};
 // Three pieces and two K-groups a workgroup (192 columns), in the place of 256-column units without a K-split: fitted to wq|wk|wv, wo and
 // w2 of 7B, 13B and 70B at 130 .. 2047 rows, within 7 % in the mean.  Taken where it promises 3 %, it took 0.85 .. 0.97 of the time (once
 // 1.01: 300 rows of 4096 x 12288).  Where the 256-column units have a K-split they stay: launch and slabs are level or better.
-constexpr RowsCost ROWS_192 = {0.11f, 0.21f, 4.0f, 1.2f};
+constexpr RowsCost ROWS_192 = {0.11f, 0.21f, 4.0f, 1.2f, 0.0f};
+// Six pieces of direct products (384 columns): the step of ROWS_384; with its `busy` a launch that nearly fills a round was estimated 10 to
+// 15 % short (8192 x 10240 at 1024 rows 173 us, 3 % more than with 192 columns).  Taken where it promises 3 % more than the others:
+// 0.85 .. 0.98 of their time, once 1.007 (1536 rows of 4096 x 12288).
+constexpr RowsCost ROWS_SIX = {0.21f, 0.37f, 4.0f, 1.0f, 0.15f};
 static float gemm_rows_us(const RowsCost &t, int units, long of_unit, int rows, int steps) {
     const float r = (float)(units * of_unit) / 256.0f, rounds = (float)(((units + 7) / 8 * of_unit + 31) / 32);
-    return (rounds > t.busy * r ? rounds : t.busy * r) * ((float)steps * (t.step + t.per_rows * rows / GEMM_BM) + t.around);
+    return ((rounds > t.busy * r ? rounds : t.busy * r) + t.more * r) * ((float)steps * (t.step + t.per_rows * rows / GEMM_BM) + t.around);
 }
 // (p.units on entry; returns the estimate)
 static float gemm_plan_rows(MatmulParams &p, int steps, int max_ks, const RowsCost &cost) {
@@ -1621,9 +1657,9 @@ int gemm_swiglu_rows_launch(MatmulParams p, hipStream_t stream) {
                                            q40_gemm_kernel<7, false, true, 8, GEMM_STAGES, false, false, true>, q40_gemm_kernel<8, false, true, 8, GEMM_STAGES, false, false, true>};
     static const gemm_kernel_t dma_wave[5] = {q40_gemm_kernel<4, false, true, 8, gemm_dma_slots(4), true, false, true>, q40_gemm_kernel<5, false, true, 8, gemm_dma_slots(5), true, false, true>, q40_gemm_kernel<6, false, true, 8, gemm_dma_slots(6), true, false, true>,
                                               q40_gemm_kernel<7, false, true, 8, gemm_dma_slots(7), true, false, true>, q40_gemm_kernel<8, false, true, 8, gemm_dma_slots(8), true, false, true>};
-    static const gemm_kernel_t wide[5] = {q40_gemm_wide_kernel<4, true>, q40_gemm_wide_kernel<5, true>, q40_gemm_wide_kernel<6, true>,
-                                          q40_gemm_wide_kernel<7, true>, q40_gemm_wide_kernel<8, true>};
-    static const int wide_lds[5] = {WideShape<4, true>::LDS, WideShape<5, true>::LDS, WideShape<6, true>::LDS, WideShape<7, true>::LDS, WideShape<8, true>::LDS};
+    static const gemm_kernel_t wide[5] = {q40_gemm_wide_kernel<4, WIDE_SWIGLU>, q40_gemm_wide_kernel<5, WIDE_SWIGLU>, q40_gemm_wide_kernel<6, WIDE_SWIGLU>,
+                                          q40_gemm_wide_kernel<7, WIDE_SWIGLU>, q40_gemm_wide_kernel<8, WIDE_SWIGLU>};
+    static const int wide_lds[5] = {WideShape<4, WIDE_SWIGLU>::LDS, WideShape<5, WIDE_SWIGLU>::LDS, WideShape<6, WIDE_SWIGLU>::LDS, WideShape<7, WIDE_SWIGLU>::LDS, WideShape<8, WIDE_SWIGLU>::LDS};
     static const hipError_t lds_ok = [] {
         hipError_t e = hipSuccess;
         for (int t = 0; t < 5 && e == hipSuccess; ++t) {
@@ -1657,23 +1693,40 @@ int gemm_swiglu_rows_launch(MatmulParams p, hipStream_t stream) {
     return launch_status();
 }
 
-// The launch of a direct product whose plan has no K-split, with workgroups of 192 columns (w) where they promise more (slabs, whose
-// bits are those of the checkpoint layout's launch, stay with its kernel).
-static bool gemm_wide_fits(const MatmulParams &p, MatmulParams &w) {
-    if (!p.tiled || !p.direct || p.M <= GEMM_BM || p.ksplit != 1 || p.K % 64 != 0) return false;
+// The launch of a direct product whose plan has no K-split, with workgroups of three pieces and two K-groups or of six pieces where they
+// promise more (slabs, whose bits are those of the checkpoint layout's launch, stay with its kernel).  Returns the pieces, 0: neither.
+static int gemm_wide_fits(const MatmulParams &p, MatmulParams &w) {
+    if (!p.tiled || !p.direct || p.M <= GEMM_BM || p.ksplit != 1 || p.K % 32 != 0) return 0;
+    int pieces = 0;
     w = p;
-    const float us = gemm_plan_rows(w, p.K / 32, 1, ROWS_256);
-    w.units = (p.n_total / 64 + 2) / 3;
-    w.units_pad = (w.units + 7) / 8 * 8;
-    return gemm_plan_rows(w, p.K / 32, 1, ROWS_192) < 0.97f * us;
+    float least = 0.97f * gemm_plan_rows(w, p.K / 32, 1, ROWS_256);
+    for (int n = 3; n <= 6; n += 3) {
+        if (n == 3 && p.K % 64 != 0) continue;
+        MatmulParams t = p;
+        t.units = (p.n_total / 64 + n - 1) / n;
+        t.units_pad = (t.units + 7) / 8 * 8;
+        const float us = gemm_plan_rows(t, p.K / 32, 1, n == 3 ? ROWS_192 : ROWS_SIX);
+        if (us < (n == 3 ? least : 0.97f * least)) {
+            least = us;
+            w = t;
+            pieces = n;
+        }
+    }
+    return pieces;
 }
-static int gemm_wide_launch(const MatmulParams &p, hipStream_t stream) {
-    static const gemm_kernel_t kern[5] = {q40_gemm_wide_kernel<4, false>, q40_gemm_wide_kernel<5, false>, q40_gemm_wide_kernel<6, false>,
-                                          q40_gemm_wide_kernel<7, false>, q40_gemm_wide_kernel<8, false>};
-    static const int lds_bytes[5] = {WideShape<4, false>::LDS, WideShape<5, false>::LDS, WideShape<6, false>::LDS, WideShape<7, false>::LDS, WideShape<8, false>::LDS};
+static int gemm_wide_launch(const MatmulParams &p, int pieces, hipStream_t stream) {
+    static const gemm_kernel_t kern[2][5] = {{q40_gemm_wide_kernel<4, WIDE_GROUPS>, q40_gemm_wide_kernel<5, WIDE_GROUPS>, q40_gemm_wide_kernel<6, WIDE_GROUPS>,
+                                              q40_gemm_wide_kernel<7, WIDE_GROUPS>, q40_gemm_wide_kernel<8, WIDE_GROUPS>},
+                                             {q40_gemm_wide_kernel<4, WIDE_SIX>, q40_gemm_wide_kernel<5, WIDE_SIX>, q40_gemm_wide_kernel<6, WIDE_SIX>,
+                                              q40_gemm_wide_kernel<7, WIDE_SIX>, q40_gemm_wide_kernel<8, WIDE_SIX>}};
+    static const int lds_bytes[2][5] = {{WideShape<4, WIDE_GROUPS>::LDS, WideShape<5, WIDE_GROUPS>::LDS, WideShape<6, WIDE_GROUPS>::LDS,
+                                         WideShape<7, WIDE_GROUPS>::LDS, WideShape<8, WIDE_GROUPS>::LDS},
+                                        {WideShape<4, WIDE_SIX>::LDS, WideShape<5, WIDE_SIX>::LDS, WideShape<6, WIDE_SIX>::LDS, WideShape<7, WIDE_SIX>::LDS,
+                                         WideShape<8, WIDE_SIX>::LDS}};
     static const hipError_t lds_ok = [] {
         hipError_t e = hipSuccess;
-        for (int t = 0; t < 5 && e == hipSuccess; ++t) e = hipFuncSetAttribute((const void *)kern[t], hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes[t]);
+        for (int t = 0; t < 10 && e == hipSuccess; ++t)
+            e = hipFuncSetAttribute((const void *)kern[t / 5][t % 5], hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes[t / 5][t % 5]);
         return e;
     }();
     if (lds_ok != hipSuccess) {
@@ -1681,14 +1734,14 @@ static int gemm_wide_launch(const MatmulParams &p, hipStream_t stream) {
         return (int)lds_ok;
     }
     SMH_REQUIRE((long)p.M * p.lda * 2 < (1L << 32), "q40 gemm: M x lda = %d x %ld exceeds the 32-bit lane offsets of A", p.M, p.lda);
-    const int t = p.block_rows / 16 - 4;
-    hipLaunchKernelGGL(kern[t], dim3((unsigned)((long)p.units_pad * p.mblocks)), dim3(64 * (WIDE_WAVES + 1)), lds_bytes[t], stream, p);
+    const int six = pieces == 6 ? 1 : 0, t = p.block_rows / 16 - 4;
+    hipLaunchKernelGGL(kern[six][t], dim3((unsigned)((long)p.units_pad * p.mblocks)), dim3(64 * (WIDE_WAVES + 1)), lds_bytes[six][t], stream, p);
     return launch_status();
 }
 
 int gemm_launch(const MatmulParams &p, hipStream_t stream) {
     MatmulParams w;
-    if (gemm_wide_fits(p, w)) return gemm_wide_launch(w, stream);
+    if (const int pieces = gemm_wide_fits(p, w)) return gemm_wide_launch(w, pieces, stream);
     if (p.kgroups == 2 && p.tiled) return gemm_kg_launch(p, stream);
     return p.tiled ? gemm_launch_layout<true>(p, stream) : gemm_launch_layout<false>(p, stream);
 }

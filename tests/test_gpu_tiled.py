@@ -328,9 +328,15 @@ def test_direct_products(M, K, ns):
                                     (257, 128, [10624]),                   # two stages; six row tiles; one piece
                                     (512, 704, [7040, 128, 896]),          # eleven stages; seven row tiles; workgroups across weights, odd 128-column blocks
                                     (600, 448, [7808]),                    # seven stages, more than the ring holds; eight row tiles
-                                    (400, 4096, [4096, 4096, 4096])])
-def test_three_pieces_and_two_k_groups(M, K, ns):
-    """sizes above 128 rows that q40_gemm_wide_kernel takes (its estimate is the smaller one): fp16 results with and without a residual"""
+                                    (400, 4096, [4096, 4096, 4096]),
+                                    # six pieces of one step
+                                    (700, 96, [10624]),                    # three steps; six row tiles, the last block of 28 rows; a last workgroup of four pieces
+                                    (1100, 32, [6272]),                    # one step; seven row tiles; two pieces
+                                    (700, 32, [5120, 128, 5120]),          # eight row tiles; workgroups across weights, an odd 128-column block; six pieces throughout
+                                    (1024, 4096, [4096, 4096, 4096])])
+def test_wide_workgroups(M, K, ns):
+    """sizes above 128 rows that q40_gemm_wide_kernel takes (three pieces and two K-groups, or six pieces, have the smaller
+    estimate): fp16 results with and without a residual"""
     from spec_mcts_amd import kernels as Kn
     ws = [_weight(K, n, 2000 + i + K) for i, n in enumerate(ns)]
     tiled = [Kn.tile_q40(w.cuda(), s.cuda(), K, n) for (w, s), n in zip(ws, ns)]
