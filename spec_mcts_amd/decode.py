@@ -61,7 +61,7 @@ class GraphDecoder:
     def _key(self):
         m = self.model
         return (self.prompt_len, self.B, m.fused, m.tiled_weights, m.silu_in_matmul, m.swiglu_in_matmul, m.norm_in_matmul, m.norm_in_max_rows,
-                m.attn_from_qkv, m.attn_single_launch, m.decode_stack, m.per_branch_kv, m._forked)
+                m.attn_from_qkv, m.attn_single_launch, m.decode_stack, m.decode_stack_min_prompt, m.per_branch_kv, m._forked)
 
     def _reset_state(self):
         self.state.copy_(torch.tensor([self.prompt_len, 0], dtype=torch.int32))
@@ -167,7 +167,7 @@ class BucketedForward:
     def _config(self):
         m = self.model
         return (self.prompt_len, m.fused, m.tiled_weights, m.silu_in_matmul, m.swiglu_in_matmul, m.norm_in_matmul, m.norm_in_max_rows, m.attn_from_qkv,
-                m.attn_single_launch, m.decode_stack, m.per_branch_kv)
+                m.attn_single_launch, m.decode_stack, m.decode_stack_min_prompt, m.per_branch_kv)
 
     def begin(self):
         """After the prefill: take the prompt length from the model, rewind the suffix, switch the page table on."""

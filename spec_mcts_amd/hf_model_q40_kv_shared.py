@@ -320,6 +320,10 @@ class Transformer(nn.Module):
         self._norm_in_ok = {}
         self.attn_from_qkv = True          # where the attention is one launch it takes the wq|wk|wv product itself
         self.decode_stack = True           # up to 4 branches (multi-head attention): all layers of a decode step in one launch
+        # ... behind a prompt of at least so many rows.  Its sums come in another order than the launches', and what that changes of a row's
+        # Q4_0 codes weighs by the row's share of the attention: after eight steps the two ways' logits differ by 2e-2 behind 64 shared rows
+        # (two forms of the attention alone by 1.5e-2), by 1.6e-2 behind 96, 0.9e-2 behind 256.
+        self.decode_stack_min_prompt = 96
         self._stack_ws = None
         self._q40_output = None            # quantize_lm_head(): (w, s, padded vocab) of a Q4_0 vocabulary projection
         self.paged_kv = True               # fork = a copy of page ids: forked branches share their ancestor's suffix rows
@@ -462,7 +466,7 @@ class Transformer(nn.Module):
         to one sequence of steps."""
         if not (self.decode_stack and self.attn_single_launch and self.attn_from_qkv and self.norm_in_matmul and self.silu_in_matmul and not self.per_branch_kv):
             return None
-        if K.decode_stack_bytes(first, B) == 0:
+        if first.prompt_len < self.decode_stack_min_prompt or K.decode_stack_bytes(first, B) == 0:
             return None
         if self._stack_ws is None or self._stack_ws.device != dev:
             if torch.cuda.is_current_stream_capturing():        # (a graph's own memory is no place for what outlives its replay)
