@@ -10,6 +10,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <cstring>
 #include <string>
 #include <vector>
 
@@ -367,6 +368,90 @@ PyObject *paged_prefix_attn(Args x) {
     return give(out);
 }
 
+// ---- what the layer calls read of a transformer block ----
+struct Ref {                                   // a reference of one's own
+    PyObject *o;
+    explicit Ref(PyObject *made_) : o(made(made_)) {}
+    Ref(Ref &&r) : o(r.o) { r.o = nullptr; }
+    Ref(const Ref &) = delete;
+    Ref &operator=(const Ref &) = delete;
+    ~Ref() { Py_XDECREF(o); }
+};
+struct Names {
+    PyObject *modules, *parameters, *attention, *feed_forward, *attention_norm, *ffn_norm, *weight, *eps, *prompt_len, *w, *s, *tiled, *buf;
+    PyObject *caches[6], *lin[7];
+    Names() {
+        auto in = [](const char *n) { return made(PyUnicode_InternFromString(n)); };
+        modules = in("_modules"); parameters = in("_parameters");
+        attention = in("attention"); feed_forward = in("feed_forward"); attention_norm = in("attention_norm"); ffn_norm = in("ffn_norm");
+        weight = in("weight"); eps = in("eps"); prompt_len = in("cache_prompt_len"); w = in("w"); s = in("s"); tiled = in("_tiled"); buf = in("buf");
+        const char *c[6] = {"cache_prompt_k", "cache_prompt_v", "cache_k", "cache_k_s", "cache_v", "cache_v_s"};
+        const char *l[7] = {"wq", "wk", "wv", "wo", "w1", "w2", "w3"};
+        for (int i = 0; i < 6; ++i) caches[i] = in(c[i]);
+        for (int i = 0; i < 7; ++i) lin[i] = in(l[i]);
+    }
+};
+Ref attribute(PyObject *o, PyObject *name) { return Ref(PyObject_GetAttr(o, name)); }
+// A submodule or parameter of an nn.Module, out of the dictionary that the module's own (Python) __getattr__ would look into.
+Ref member(PyObject *o, PyObject *kind, PyObject *name) {
+    PyObject *d = PyObject_GenericGetDict(o, nullptr);
+    if (d == nullptr) {
+        PyErr_Clear();
+    } else {
+        PyObject *of_kind = PyDict_GetItem(d, name) == nullptr ? PyDict_GetItem(d, kind) : nullptr;      // (borrowed)
+        PyObject *v = of_kind != nullptr && PyDict_Check(of_kind) ? PyDict_GetItem(of_kind, name) : nullptr;
+        Py_XINCREF(v);
+        Py_DECREF(d);
+        if (v != nullptr) return Ref(v);
+    }
+    return attribute(o, name);
+}
+constexpr int LAYER_WORDS = 2 + 2 + 6 + 7 * 4;
+
+// (block, key: bytearray of LAYER_WORDS 8-byte words) -> the rows of the block's prompt cache; -1 - rows where the key was another one.
+// The key is the addresses of all tensors that smh_layer takes from the block and of the checkpoint weights behind the tiled ones, the
+// norms' eps, and the tiled weights as the objects they are (the caller keeps them alive); it is brought up to date.
+PyObject *layer_state(Args x) {
+    static const Names n;
+    PyObject *block = x[0];
+    need(PyByteArray_Check(x[1]) && PyByteArray_GET_SIZE(x[1]) == LAYER_WORDS * 8, "the key of a layer is a bytearray of layer_key_bytes");
+    uint64_t now[LAYER_WORDS];
+    int at = 0;
+    auto address = [&](const Ref &t) { now[at++] = (uint64_t)(uintptr_t)tensor(t.o, "a layer's attribute").data_ptr(); };
+    auto number_of = [&](const Ref &f) {
+        const double v = real(f.o);
+        memcpy(&now[at++], &v, 8);
+    };
+    const Ref att = member(block, n.modules, n.attention), ff = member(block, n.modules, n.feed_forward);
+    for (PyObject *name : {n.attention_norm, n.ffn_norm}) {
+        const Ref norm = member(block, n.modules, name);
+        address(member(norm.o, n.parameters, n.weight));
+        number_of(attribute(norm.o, n.eps));
+    }
+    int64_t capacity = 0;
+    for (int i = 0; i < 6; ++i) {
+        const Ref t = attribute(att.o, n.caches[i]);
+        address(t);
+        if (i == 0) capacity = tensor(t.o, "cache_prompt_k").size(1);
+    }
+    for (int i = 0; i < 7; ++i) {
+        const Ref lin = member(i < 4 ? att.o : ff.o, n.modules, n.lin[i]);
+        address(attribute(lin.o, n.w));
+        address(attribute(lin.o, n.s));
+        const Ref tiled = attribute(lin.o, n.tiled);
+        now[at++] = (uint64_t)(uintptr_t)tiled.o;
+        if (none(tiled.o)) now[at++] = 0;
+        else address(attribute(tiled.o, n.buf));
+    }
+    const Ref rows_ = attribute(att.o, n.prompt_len);
+    const long rows = number(rows_.o);
+    need(rows >= 0 && rows <= capacity, "cache_prompt_len exceeds the prompt cache");
+    char *key = PyByteArray_AS_STRING(x[1]);
+    const bool same = memcmp(key, now, sizeof now) == 0;
+    if (!same) memcpy(key, now, sizeof now);
+    return PyLong_FromLong(same ? rows : -1 - rows);
+}
+
 template <PyObject *(*F)(Args), int N>
 PyObject *call(PyObject *, PyObject *const *args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
@@ -413,9 +498,16 @@ PyObject *connect(PyObject *, PyObject *const *args, Py_ssize_t n) {
 PyMethodDef methods[] = {
     {"connect", (PyCFunction)(void (*)(void))connect, METH_FASTCALL, nullptr},
     OP(matmul_q40, 6), OP(deq_int40, 4), OP(q_int40, 1), OP(quantize_q40_t, 1), OP(sample_topk_counts, 6), OP(tree_step, 14),
-    OP(shared_prefix_attn, 15), OP(paged_prefix_attn, 15), {nullptr, nullptr, 0, nullptr}};
+    OP(shared_prefix_attn, 15), OP(paged_prefix_attn, 15), OP(layer_state, 2), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_ops", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__ops(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__ops(void) {
+    PyObject *m = PyModule_Create(&module);
+    if (m != nullptr && PyModule_AddIntConstant(m, "layer_key_bytes", LAYER_WORDS * 8) != 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

@@ -278,6 +278,7 @@ class TransformerBlock(nn.Module):
         self.ffn_norm = RMSNorm(args.dim, eps=args.norm_eps)
         self.native = None            # Transformer._layer_struct
         self.native_key = None
+        self.native_tiled = None
 
     def forward(self, x, start_pos, freqs_cis, mask, step_state=None, pages=None):
         # the residual adds are fused into the epilogues of wo and w2
@@ -441,22 +442,25 @@ class Transformer(nn.Module):
         B = tokens.shape[0]
         h = K.embedding(tokens, self.tok_embeddings.weight)
         dev = h.device
-        att0 = self.layers[0].attention
-        one = self.attn_single_launch and B * att0.n_rep <= 16
-        P = att0.cache_prompt_len
-        ws = K.attn_qkv_workspace(dev, B, att0.n_local_heads, P) if one else K.attn_workspace(dev, B, att0.n_local_heads, P)
-        run = K.LayerPass(self._layer_struct(self.layers[0]), B, h, *self._tables(dev), self.swiglu_in_matmul)
-        norm_in = self._norm_in(B, p.dim, [lin._tiled for lin in (att0.wq, att0.wk, att0.wv)])      # (the library asks again, launch by launch)
-        run.decode_step(step_state, ws, bool(one), p.max_seq_len, p.max_batch_size * p.max_seq_len, self._pages(dev), B if norm_in else 0,
-                        K.SILU_IN_MAX_M if self.silu_in_matmul else 0, self.attn_from_qkv and not self.per_branch_kv)
-        s = self._layer_struct(self.layers[0])
-        stack_ws = self._stack_workspace(dev, s, B)
+        layers = list(self.layers)
+        first = s = self._layer_struct(layers[0])
+        run = K.LayerPass(first, B, h, *self._tables(dev), self.swiglu_in_matmul)
+        pages, smax, cache_rows = self._pages(dev), p.max_seq_len, p.max_batch_size * p.max_seq_len
+        stack_ws = self._stack_workspace(dev, first, B)
         if stack_ws is not None:
-            structs = [s] + [self._layer_struct(layer) for layer in self.layers[1:]]
+            run.decode_step(step_state, None, True, smax, cache_rows, pages, 0, 0, True)
+            structs = [first] + [self._layer_struct(layer) for layer in layers[1:]]
             s = structs[-1]
             run.decode_stack(structs, stack_ws)
         else:                              # (layer by layer: the GPU works while the next one's arguments are gathered)
-            for i, layer in enumerate(self.layers):
+            att0 = layers[0].attention
+            H, P = att0.n_local_heads, first.prompt_len
+            one = self.attn_single_launch and B * att0.n_rep <= 16
+            ws = K.attn_qkv_workspace(dev, B, H, P) if one else K.attn_workspace(dev, B, H, P)
+            norm_in = self._norm_in(B, p.dim, [lin._tiled for lin in (att0.wq, att0.wk, att0.wv)])  # (the library asks again, launch by launch)
+            run.decode_step(step_state, ws, bool(one), smax, cache_rows, pages, B if norm_in else 0, K.SILU_IN_MAX_M if self.silu_in_matmul else 0,
+                            self.attn_from_qkv and not self.per_branch_kv)
+            for i, layer in enumerate(layers):
                 s = self._layer_struct(layer) if i > 0 else s
                 run.decode(s)
         return self._lm_head(run.finish(s, self.norm.weight, self.norm.eps).view(B, 1, p.dim))
@@ -491,23 +495,21 @@ class Transformer(nn.Module):
 
     def _layer_struct(self, layer):
         """What the library's layer calls read of a layer, rebuilt when any of its tensors or an eps is another one than at the last pass
-        (the tiled copies are compared as the objects they are, which the key keeps alive)."""
-        att, ff = layer.attention, layer.feed_forward
-        lins = (att.wq, att.wk, att.wv, att.wo, ff.w1, ff.w2, ff.w3)
-        key = [layer.attention_norm.weight.data_ptr(), layer.ffn_norm.weight.data_ptr(), att.cache_prompt_k.data_ptr(), att.cache_prompt_v.data_ptr(),
-               att.cache_k.data_ptr(), att.cache_k_s.data_ptr(), att.cache_v.data_ptr(), att.cache_v_s.data_ptr(), float(layer.attention_norm.eps),
-               float(layer.ffn_norm.eps)]
-        n_fixed = len(key)
-        for lin in lins:
-            key += (lin.w.data_ptr(), lin.s.data_ptr(), lin._tiled)
-        if layer.native is None or layer.native_key != key:
+        (the tiled copies are compared as the objects they are, which the layer keeps alive).  The look is native: in Python it took 14 us
+        a layer, which a step in one launch waits for 32 times over."""
+        if layer.native_key is None:
+            layer.native_key = bytearray(K.layer_key_bytes())
+        rows = K.layer_state(layer, layer.native_key)
+        if rows < 0 or layer.native is None:
+            layer.native = None
+            att, ff = layer.attention, layer.feed_forward
+            layer.native_tiled = [lin.operand(True) for lin in (att.wq, att.wk, att.wv, att.wo, ff.w1, ff.w2, ff.w3)]
+            rows = K.layer_state(layer, layer.native_key)              # (of the tiled copies just made)
+            rows = rows if rows >= 0 else -1 - rows
             layer.native = K.layer_struct(self.params.dim, att.n_local_heads, att.n_local_kv_heads, layer.attention_norm.weight, layer.attention_norm.eps,
-                                          layer.ffn_norm.weight, layer.ffn_norm.eps, [lin.operand(True) for lin in lins], att.cache_prompt_k,
-                                          att.cache_prompt_v, att.cache_k, att.cache_k_s, att.cache_v, att.cache_v_s)
-            key[n_fixed:] = [x for lin in lins for x in (lin.w.data_ptr(), lin.s.data_ptr(), lin._tiled)]
-            layer.native_key = key
-        assert att.cache_prompt_len <= att.cache_prompt_k.shape[1]
-        layer.native.prompt_len = att.cache_prompt_len
+                                          layer.ffn_norm.weight, layer.ffn_norm.eps, layer.native_tiled, att.cache_prompt_k, att.cache_prompt_v,
+                                          att.cache_k, att.cache_k_s, att.cache_v, att.cache_v_s)
+        layer.native.prompt_len = rows
         return layer.native
 
     def quantize_lm_head(self, enable: bool = True):

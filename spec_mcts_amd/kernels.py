@@ -676,6 +676,17 @@ def layer_struct(dim: int, H: int, Hkv: int, att_norm: torch.Tensor, att_eps: fl
     return s
 
 
+def layer_key_bytes() -> int:
+    """Size of the key that layer_state keeps of a layer."""
+    return _lib.ops().layer_key_bytes
+
+
+def layer_state(block, key: bytearray) -> int:
+    """Rows of the block's prompt cache; -1 - rows if anything that layer_struct reads of the block is not what it was when the key was
+    written (the key is then brought up to date).  The caller keeps the block's tiled weights alive, whose identity is part of the key."""
+    return _lib.ops().layer_state(block, key)
+
+
 DECODE_STACK_MAX_ROWS = 4                      # csrc/decode_stack.hip
 
 
@@ -703,17 +714,19 @@ class LayerPass:
         p.scratch, p.scratch_bytes, p.h = self.scratch.data_ptr(), nbytes, h.data_ptr()
         self.stream = _stream()
 
-    def decode_step(self, step_state, ws: torch.Tensor, one_launch: bool, smax: int, cache_rows: int, pages: Optional[torch.Tensor], norm_in_rows: int,
+    def decode_step(self, step_state, ws: Optional[torch.Tensor], one_launch: bool, smax: int, cache_rows: int, pages: Optional[torch.Tensor], norm_in_rows: int,
                     silu_in_rows: int, attn_from_qkv: bool) -> None:
         """step_state: (position, suffix index) on the device; `ws`: the workspace of the attention (of its one-launch form with
-        `one_launch`); pages: int32 page table over cache_rows cache rows, or None."""
+        `one_launch`), None where all layers are one launch; pages: int32 page table over cache_rows cache rows, or None."""
         p = self.p
         pos_dev, t_dev = step_state
-        _need_gpu(pos_dev, t_dev, ws)
+        _need_gpu(pos_dev, t_dev)
         assert pos_dev.dtype == torch.int32 and t_dev.dtype == torch.int32
         p.pos_dev, p.t_dev = pos_dev.data_ptr(), t_dev.data_ptr()
         self.ws = ws
-        if one_launch:
+        if ws is None:
+            pass
+        elif one_launch:
             p.attn_one, p.attn_one_ws, p.attn_one_ws_bytes = 1, ws.data_ptr(), ws.numel()
         else:
             p.attn_ws, p.attn_ws_bytes = ws.data_ptr(), ws.numel()
