@@ -1074,15 +1074,42 @@ extern "C" size_t smh_decode_stack_workspace_bytes(const smh_layer *layer, int r
     return stack_space(rows, layer->dim, layer->ffn, layer->heads).bytes;
 }
 
+// Why a pass over these layers is not for the kernel, null: it is.  Alignments are those of its loads (the weights' of the DMA into LDS),
+// looked at layer by layer, for tensors may be views: the layers' own launches take what is refused here.
+static const char *stack_refuses(const smh_layer *const *layers, int n_layers, int rows, StackParams &p) {
+    if (layers == nullptr || n_layers < 1) return "no layers";
+    for (int i = 0; i < n_layers; ++i)
+        if (layers[i] == nullptr) return "a layer is null";
+    const smh_layer &L0 = *layers[0];
+    if (!stack_plan(L0, rows, p)) return "its rows, heads or widths are not for this call";
+    for (int i = 0; i < n_layers; ++i) {
+        const smh_layer &L = *layers[i];
+        if (L.dim != L0.dim || L.ffn != L0.ffn || L.heads != L0.heads || L.kv_heads != L0.kv_heads) return "layers of different sizes";
+        if (L.prompt_len < 0) return "a negative prompt length";
+        auto bad = [](const void *q, int align) { return q == nullptr || (uintptr_t)q % align != 0; };
+        for (const void *q : {L.wq, L.wk, L.wv, L.wo, L.w1, L.w2, L.w3})
+            if (bad(q, 16)) return "a weight is null or not 16-byte aligned";
+        for (const void *q : {L.prompt_k, L.prompt_v})
+            if (L.prompt_len > 0 && bad(q, 8)) return "a prompt cache is null or not 8-byte aligned";
+        for (const void *q : {(const void *)L.cache_k, (const void *)L.cache_v, (const void *)L.cache_ks, (const void *)L.cache_vs, L.att_norm, L.ffn_norm})
+            if (bad(q, 4)) return "a cache or the weight of a norm is null or not 4-byte aligned";
+    }
+    return nullptr;
+}
+
+extern "C" int smh_decode_stack_fits(const smh_layer *const *layers, int n_layers, int rows) {
+    StackParams p;
+    return stack_refuses(layers, n_layers, rows, p) == nullptr ? 1 : 0;
+}
+
 extern "C" int smh_decode_stack(const smh_layer *const *layers, int n_layers, smh_pass *pass, void *ws, size_t ws_bytes, smh_stream_t stream) {
     const char *who = "smh_decode_stack";
-    SMH_REQUIRE(layers && n_layers >= 1 && pass && pass->h && ws, "%s: null pointer or no layers", who);
-    for (int i = 0; i < n_layers; ++i) SMH_REQUIRE(layers[i] != nullptr, "%s: layer %d is null", who, i);
+    SMH_REQUIRE(pass && pass->h && ws, "%s: null pointer", who);
+    StackParams p;
+    const char *why = stack_refuses(layers, n_layers, pass->rows, p);
+    SMH_REQUIRE(why == nullptr, "%s: %s (%d rows)", who, why, pass->rows);
     const smh_layer &L0 = *layers[0];
     SMH_REQUIRE(pass->pos_dev && pass->t_dev && pass->cos_tab && pass->sin_tab && pass->smax >= 1, "%s: the step's tables and counters are missing", who);
-    StackParams p;
-    SMH_REQUIRE(stack_plan(L0, pass->rows, p), "%s: rows=%d heads=%d kv_heads=%d dim=%d ffn=%d are not for this call", who, pass->rows, L0.heads, L0.kv_heads,
-                L0.dim, L0.ffn);
     const size_t need = stack_space(pass->rows, p.dim, p.ffn, p.heads).bytes;
     SMH_REQUIRE(ws_bytes >= need, "%s: workspace %zu < %zu bytes", who, ws_bytes, need);
     const size_t rows_bytes = ((size_t)pass->rows * p.dim * 2 + 255) & ~(size_t)255;
@@ -1116,12 +1143,6 @@ extern "C" int smh_decode_stack(const smh_layer *const *layers, int n_layers, sm
         int count = 0;
         while (l0 + count < n_layers && count < DS_LAYERS) {
             const smh_layer &L = *layers[l0 + count];
-            SMH_REQUIRE(L.dim == L0.dim && L.ffn == L0.ffn && L.heads == L0.heads && L.kv_heads == L0.kv_heads, "%s: layers of different sizes", who);
-            const void *const need16[] = {L.wq, L.wk, L.wv, L.wo, L.w1, L.w3, L.w2, L.cache_k, L.cache_v, L.prompt_len > 0 ? L.prompt_k : L.wq,
-                                          L.prompt_len > 0 ? L.prompt_v : L.wq};
-            for (const void *q : need16) SMH_REQUIRE(q && (uintptr_t)q % 16 == 0, "%s: layer %d: a weight or cache is null or not 16-byte aligned", who, l0 + count);
-            SMH_REQUIRE(L.att_norm && L.ffn_norm && L.cache_ks && L.cache_vs && L.prompt_len >= 0, "%s: layer %d: null pointer or prompt_len=%d", who, l0 + count,
-                        L.prompt_len);
             if (L.att_eps != A.att_eps || L.ffn_eps != A.ffn_eps || L.prompt_len != A.prompt_len) break;
             p.layer[count++] = StackLayer{{(const uint8_t *)L.wq, (const uint8_t *)L.wk, (const uint8_t *)L.wv, (const uint8_t *)L.wo, (const uint8_t *)L.w1,
                                            (const uint8_t *)L.w3, (const uint8_t *)L.w2}, (const half_t *)L.att_norm, (const half_t *)L.ffn_norm,

@@ -446,12 +446,14 @@ class Transformer(nn.Module):
         first = s = self._layer_struct(layers[0])
         run = K.LayerPass(first, B, h, *self._tables(dev), self.swiglu_in_matmul)
         pages, smax, cache_rows = self._pages(dev), p.max_seq_len, p.max_batch_size * p.max_seq_len
-        stack_ws = self._stack_workspace(dev, first, B)
+        stack_ws, structs, stack = self._stack_workspace(dev, first, B), [], None
         if stack_ws is not None:
-            run.decode_step(step_state, None, True, smax, cache_rows, pages, 0, 0, True)
             structs = [first] + [self._layer_struct(layer) for layer in layers[1:]]
+            stack = K.decode_stack_layers(structs, B)
+        if stack is not None:
+            run.decode_step(step_state, None, True, smax, cache_rows, pages, 0, 0, True)
             s = structs[-1]
-            run.decode_stack(structs, stack_ws)
+            run.decode_stack(stack, stack_ws)
         else:                              # (layer by layer: the GPU works while the next one's arguments are gathered)
             att0 = layers[0].attention
             H, P = att0.n_local_heads, first.prompt_len

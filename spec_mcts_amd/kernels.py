@@ -695,6 +695,13 @@ def decode_stack_bytes(first: "_lib.SmhLayer", rows: int) -> int:
     return int(_lib.load().smh_decode_stack_workspace_bytes(first, rows))
 
 
+def decode_stack_layers(structs: Sequence["_lib.SmhLayer"], rows: int):
+    """What LayerPass.decode_stack takes of these layers (their structs must outlive it), None where it does not take them (a tensor that
+    is a view with an odd offset, layers of different sizes)."""
+    arr = (ctypes.c_void_p * len(structs))(*[ctypes.addressof(s) for s in structs])
+    return arr if _lib.load().smh_decode_stack_fits(arr, len(structs), rows) else None
+
+
 class LayerPass:
     """One pass over all layers (smh_pass): a decode step over `rows` branches (after decode_step()) or the prefill of a prompt
     of `rows` tokens.  decode(struct) or prefill(struct) per layer, then finish() for the last residual add and the final RMSNorm.
@@ -741,10 +748,9 @@ class LayerPass:
         if st:
             check(st, "smh_decode_layer")
 
-    def decode_stack(self, structs: Sequence["_lib.SmhLayer"], ws: torch.Tensor) -> None:
-        """All layers in one launch (decode_stack_bytes() > 0)."""
-        arr = (ctypes.POINTER(_lib.SmhLayer) * len(structs))(*[ctypes.pointer(s) for s in structs])
-        check(self.lib.smh_decode_stack(arr, len(structs), self.p, ws.data_ptr(), ws.numel(), self.stream), "smh_decode_stack")
+    def decode_stack(self, layers, ws: torch.Tensor) -> None:
+        """All layers (decode_stack_layers()) in one launch; `ws`: decode_stack_bytes() of them, the model's own."""
+        check(self.lib.smh_decode_stack(layers, len(layers), self.p, ws.data_ptr(), ws.numel(), self.stream), "smh_decode_stack")
 
     def prefill(self, s: "_lib.SmhLayer") -> None:
         st = self.lib.smh_prefill_layer(s, self.p, self.stream)

@@ -85,3 +85,66 @@ def test_refused_sizes_and_arguments():
             setattr(p, field, 256)                     # (never read: the sizes are refused first)
         arr = (ctypes.POINTER(_lib.SmhLayer) * 1)(ctypes.pointer(s))
         assert lib.smh_decode_stack(arr, 1, p, 256, 1 << 30, None) != 0
+
+
+def _pointers(dim=256, heads=2, ffn=768, P=7):
+    from spec_mcts_amd import _lib
+    s = _lib.SmhLayer()
+    s.dim, s.heads, s.kv_heads, s.ffn, s.prompt_len = dim, heads, heads, ffn, P
+    for i, (name, _) in enumerate(_lib.SmhLayer._fields_[6:-1]):
+        setattr(s, name, 1 << 20 | i << 12)            # (never read)
+    return s
+
+
+@pytest.mark.parametrize("name,align", [(n, 16) for n in ("wq", "wk", "wv", "wo", "w1", "w2", "w3")] + [("prompt_k", 8), ("prompt_v", 8)]
+                         + [(n, 4) for n in ("cache_k", "cache_v", "cache_ks", "cache_vs", "att_norm", "ffn_norm")])
+def test_alignments_that_the_stack_takes(name, align):
+    """... are asked for before the pass is built (no GPU needed): what is refused goes to the layers' own launches."""
+    from spec_mcts_amd import kernels as K
+    for at in (0, 1, 2):                               # in any layer
+        layers = [_pointers() for _ in range(3)]
+        assert K.decode_stack_layers(layers, 2) is not None
+        good = getattr(layers[at], name)
+        setattr(layers[at], name, good + align)
+        assert K.decode_stack_layers(layers, 2) is not None
+        setattr(layers[at], name, good + align // 2)
+        assert K.decode_stack_layers(layers, 2) is None
+        setattr(layers[at], name, None)
+        assert K.decode_stack_layers(layers, 2) is None
+    layers = [_pointers(P=0) for _ in range(2)]
+    if name.startswith("prompt"):                      # without a prompt there is no cache to read
+        setattr(layers[1], name, None)
+        assert K.decode_stack_layers(layers, 2) is not None
+    assert K.decode_stack_layers([_pointers(), _pointers(ffn=1024)], 2) is None
+    assert K.decode_stack_layers([_pointers(), _pointers(P=-1)], 2) is None
+
+
+def _offset(t, elements):
+    """the same values, so many elements behind an aligned address"""
+    buf = torch.empty(t.numel() + elements, dtype=t.dtype, device=t.device)
+    out = buf[elements:].view(t.shape)
+    out.copy_(t)
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,elements,stack", [("cache_k", 4, True), ("cache_v_s", 2, True), ("cache_prompt_k", 4, True), ("cache_prompt_v", 2, False)])
+def test_views_as_caches(name, elements, stack, monkeypatch):
+    """A cache that is a view at an offset runs, in one launch where the kernel's loads allow it, else layer by layer."""
+    from spec_mcts_amd import ModelArgs, kernels as K
+    from spec_mcts_amd.load_q40 import load_q40
+    cfg = dict(dim=512, n_layers=2, n_heads=4, vocab_size=320, multiple_of=256, max_batch_size=2, max_seq_len=4, max_prompt_seq_len=128)
+    model = load_q40(dict(O.random_q40_state_dict(O.OracleArgs(**cfg), seed=5, std=0.04)), ModelArgs(**cfg), device="cuda:0")
+    tokens = torch.randint(0, 320, (2, 101), generator=torch.Generator().manual_seed(7)).cuda()
+    model(tokens[:1, :100], 0)
+    calls = []
+    monkeypatch.setattr(K.LayerPass, "decode_stack", lambda self, layers, ws, _f=K.LayerPass.decode_stack: (calls.append(len(layers)), _f(self, layers, ws)))
+    one = model(tokens[:, 100:], 100)
+    assert calls == [2]
+    model.decode_stack = False
+    want = one if stack else model(tokens[:, 100:], 100)
+    model.decode_stack = True
+    att = model.layers[1].attention
+    setattr(att, name, _offset(getattr(att, name), elements))
+    got = model(tokens[:, 100:], 100)
+    assert calls == [2] + [2] * stack and torch.equal(got, want)
