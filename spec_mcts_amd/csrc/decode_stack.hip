@@ -1143,7 +1143,8 @@ extern "C" int smh_decode_stack(const smh_layer *const *layers, int n_layers, sm
         int count = 0;
         while (l0 + count < n_layers && count < DS_LAYERS) {
             const smh_layer &L = *layers[l0 + count];
-            if (L.att_eps != A.att_eps || L.ffn_eps != A.ffn_eps || L.prompt_len != A.prompt_len) break;
+            // (the first one always: a NaN differs from itself)
+            if (count > 0 && (L.att_eps != A.att_eps || L.ffn_eps != A.ffn_eps || L.prompt_len != A.prompt_len)) break;
             p.layer[count++] = StackLayer{{(const uint8_t *)L.wq, (const uint8_t *)L.wk, (const uint8_t *)L.wv, (const uint8_t *)L.wo, (const uint8_t *)L.w1,
                                            (const uint8_t *)L.w3, (const uint8_t *)L.w2}, (const half_t *)L.att_norm, (const half_t *)L.ffn_norm,
                                           (const half_t *)L.prompt_k, (const half_t *)L.prompt_v, (uint8_t *)L.cache_k, (uint8_t *)L.cache_v,

@@ -148,3 +148,24 @@ def test_views_as_caches(name, elements, stack, monkeypatch):
     setattr(att, name, _offset(getattr(att, name), elements))
     got = model(tokens[:, 100:], 100)
     assert calls == [2] + [2] * stack and torch.equal(got, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("eps", [(1e-5, 1e-3, 1e-3), (float("nan"), 1e-5, 1e-5), (1e-5, 1e-5, float("nan"))])
+def test_layers_of_different_eps(eps):
+    """take a launch each time it changes; one that is NaN (which equals nothing, itself included) a launch of its own"""
+    from spec_mcts_amd import ModelArgs
+    from spec_mcts_amd.load_q40 import load_q40
+    cfg = dict(dim=512, n_layers=3, n_heads=4, vocab_size=320, multiple_of=256, max_batch_size=2, max_seq_len=4, max_prompt_seq_len=128)
+    model = load_q40(dict(O.random_q40_state_dict(O.OracleArgs(**cfg), seed=6, std=0.04)), ModelArgs(**cfg), device="cuda:0")
+    tokens = torch.randint(0, 320, (2, 101), generator=torch.Generator().manual_seed(8)).cuda()
+    model(tokens[:1, :100], 0)
+    for layer, e in zip(model.layers, eps):
+        layer.ffn_norm.eps = e
+    got = model(tokens[:, 100:], 100).float()
+    model.decode_stack = False
+    want = model(tokens[:, 100:], 100).float()
+    if any(e != e for e in eps):
+        assert got.isnan().all() and want.isnan().all()
+    else:
+        assert float((got - want).norm() / want.norm()) < 4e-3
