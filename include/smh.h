@@ -446,10 +446,14 @@ int smh_prefill_layer(const smh_layer *layer, smh_pass *pass, smh_stream_t strea
  * calls (calls with other row counts may share it); calls that overlap need one each.  Of the pass it needs rows, the tables and
  * counters, pages, scratch, h and pending (0).  The workgroups wait for one another, however many of them the GPU runs at a time; a wait
  * of more than 5 seconds ends with NaN in h.  smh_decode_stack_fits: 1 where the call takes these layers, 0 where it refuses them: besides
- * the sizes, equal ones in all layers, the alignment of each tensor (weights 16 bytes, prompt caches 8, the others 4). */
+ * the sizes, equal ones in all layers, the alignment of each tensor (weights 16 bytes, prompt caches 8, the others 4).
+ * smh_decode_stack_of: with another number of workgroups (1 .. 256; fewer take several tasks each, the result is the same bit for bit) and
+ * another wait for workgroups that have not started (50 us in smh_decode_stack; the work is dealt to those that have). */
 size_t smh_decode_stack_workspace_bytes(const smh_layer *layer, int rows);
 int smh_decode_stack_fits(const smh_layer *const *layers, int n_layers, int rows);
 int smh_decode_stack(const smh_layer *const *layers, int n_layers, smh_pass *pass, void *ws, size_t ws_bytes, smh_stream_t stream);
+int smh_decode_stack_of(const smh_layer *const *layers, int n_layers, smh_pass *pass, void *ws, size_t ws_bytes, int workgroups, int join_us,
+                        smh_stream_t stream);
 int smh_decode_finish(const smh_layer *last, smh_pass *pass, const void *norm_weight, float eps, void *out, smh_stream_t stream);
 
 #ifdef __cplusplus

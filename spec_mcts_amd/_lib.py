@@ -106,6 +106,7 @@ SIGNATURES = {
     "smh_decode_stack_workspace_bytes": (c_size_t, [_LAYER, c_int]),
     "smh_decode_stack_fits": (c_int, [_P, c_int, c_int]),
     "smh_decode_stack": (c_int, [_P, c_int, _PASS, _P, c_size_t, _P]),
+    "smh_decode_stack_of": (c_int, [_P, c_int, _PASS, _P, c_size_t, c_int, c_int, _P]),
     "smh_decode_finish": (c_int, [_LAYER, _PASS, _P, c_float, _P, _P]),
     "smh_page_fork": (c_int, [_P, c_int, c_long, c_int, c_int, c_int, c_int, _P]),
 }

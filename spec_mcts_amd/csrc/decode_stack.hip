@@ -54,7 +54,7 @@ constexpr int DS_SUMS = 256;                   // room for a row's sums of squar
 constexpr int DS_PART = 132;                   // words of a partial: o[128], max, sum
 constexpr int DS_LDS = 160 * 1024;
 constexpr uint64_t DS_WAIT_LIMIT = 500000000; // 100 MHz: 5 s
-constexpr uint64_t DS_JOIN_LIMIT = 5000;       // 50 us
+constexpr int DS_JOIN_US = 50;                 // the first to sign in wait so long for the others
 
 struct StackLayer {
     const uint8_t *w[7];                       // wq, wk, wv, wo, w1, w3, w2
@@ -74,6 +74,7 @@ struct StackParams {
     const int32_t *pos_dev, *t_dev, *pages;
     uint8_t *ws;
     long cache_rows;
+    int workgroups, join_ticks;                // of the launch; DS_JOIN_US in ticks of 10 ns
     int layers, dim, ffn, heads, P, smax, pages_stride;
     int slices, slice_rows;                    // attention: the prompt's rows in `slices` tasks a head
     uint32_t by_att, by_red, by_act;           // quotients by the tasks of a head, by red_cols and by act_cols
@@ -976,7 +977,7 @@ __global__ __launch_bounds__(DS_THREADS) void decode_stack_kernel(StackParams p)
             const uint64_t since = ticks();
             uint32_t v = ld_u32(ctl);
             while ((v & CLOSED) == 0) {
-                if ((v & 0xfff) == DS_WGS || ticks() - since > DS_JOIN_LIMIT) {
+                if ((v & 0xfff) == (uint32_t)p.workgroups || ticks() - since > (uint64_t)p.join_ticks) {
                     const uint32_t closed = v | CLOSED | (v & 0xfff) << 12;
                     uint32_t want = v;
                     if (__hip_atomic_compare_exchange_strong(ctl, &want, closed, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) v = closed;
@@ -987,7 +988,7 @@ __global__ __launch_bounds__(DS_THREADS) void decode_stack_kernel(StackParams p)
             }
             const int n = (int)((v >> 12) & 0xfff);
             gates->n = n;
-            gates->id = n == DS_WGS ? (int)blockIdx.x : (int)(old & 0xfff);
+            gates->id = n == p.workgroups ? (int)blockIdx.x : (int)(old & 0xfff);
             gates->epoch = ld_u32(ctl + 128);
         }
     }
@@ -1008,7 +1009,7 @@ __global__ __launch_bounds__(DS_THREADS) void decode_stack_kernel(StackParams p)
         }
     }
     __syncthreads();
-    if (tid == 0 && __hip_atomic_fetch_add(ctl + 64, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == DS_WGS - 1) {
+    if (tid == 0 && __hip_atomic_fetch_add(ctl + 64, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)p.workgroups - 1) {
         // the last one out: nobody reads these any more, and the next launch starts behind this one
         const uint32_t e = ld_u32(ctl + 128);
         st_u32(ctl, 0u);
@@ -1103,7 +1104,14 @@ extern "C" int smh_decode_stack_fits(const smh_layer *const *layers, int n_layer
 }
 
 extern "C" int smh_decode_stack(const smh_layer *const *layers, int n_layers, smh_pass *pass, void *ws, size_t ws_bytes, smh_stream_t stream) {
+    return smh_decode_stack_of(layers, n_layers, pass, ws, ws_bytes, DS_WGS, DS_JOIN_US, stream);
+}
+
+extern "C" int smh_decode_stack_of(const smh_layer *const *layers, int n_layers, smh_pass *pass, void *ws, size_t ws_bytes, int workgroups, int join_us,
+                                   smh_stream_t stream) {
     const char *who = "smh_decode_stack";
+    SMH_REQUIRE(workgroups >= 1 && workgroups <= DS_WGS && join_us >= 0 && join_us <= 1000000, "%s: workgroups=%d (1 .. %d) join_us=%d (up to a second)", who,
+                workgroups, DS_WGS, join_us);
     SMH_REQUIRE(pass && pass->h && ws, "%s: null pointer", who);
     StackParams p;
     const char *why = stack_refuses(layers, n_layers, pass->rows, p);
@@ -1126,6 +1134,8 @@ extern "C" int smh_decode_stack(const smh_layer *const *layers, int n_layers, sm
     p.cache_rows = pass->cache_rows;
     p.smax = pass->smax;
     p.ws = (uint8_t *)ws;
+    p.workgroups = workgroups;
+    p.join_ticks = join_us * 100;
     // more than 64 KB of dynamic LDS has to be allowed once (not stream work: fine under graph capture)
     static void (*const kernels[DS_MAX_M])(StackParams) = {decode_stack_kernel<1>, decode_stack_kernel<2>, decode_stack_kernel<3>, decode_stack_kernel<4>};
     static const hipError_t lds_ok = [] {
@@ -1157,7 +1167,7 @@ extern "C" int smh_decode_stack(const smh_layer *const *layers, int n_layers, sm
         p.att_eps = A.att_eps;
         p.ffn_eps = A.ffn_eps;
         p.layers = count;
-        hipLaunchKernelGGL(kernels[pass->rows - 1], dim3(DS_WGS), dim3(DS_THREADS), (size_t)stack_lds(pass->rows, p.x_pitch).bytes, (hipStream_t)stream, p);
+        hipLaunchKernelGGL(kernels[pass->rows - 1], dim3((unsigned)workgroups), dim3(DS_THREADS), (size_t)stack_lds(pass->rows, p.x_pitch).bytes, (hipStream_t)stream, p);
         if (int st = launch_status()) return st;
         pass->h = out;
         l0 += count;

@@ -169,3 +169,140 @@ def test_layers_of_different_eps(eps):
         assert got.isnan().all() and want.isnan().all()
     else:
         assert float((got - want).norm() / want.norm()) < 4e-3
+
+
+def _model(cfg, seed, std=0.04):
+    from spec_mcts_amd import ModelArgs
+    from spec_mcts_amd.load_q40 import load_q40
+    oargs = O.OracleArgs(**cfg)
+    sd = O.random_q40_state_dict(oargs, seed=seed, std=std)
+    model = load_q40(dict(sd), ModelArgs(**cfg), device="cuda:0")
+    model.decode_stack_min_prompt = 0
+    return oargs, sd, model
+
+
+# workgroups launched, us the first wait for the others (0: the list is closed before most have started, and ids go by arrival)
+@pytest.mark.gpu
+@pytest.mark.parametrize("workgroups,join_us", [(1, 50), (2, 50), (7, 50), (100, 50), (255, 50), (256, 0), (40, 0), (256, 50)])
+def test_any_number_of_workgroups_finishes_the_work(workgroups, join_us, monkeypatch):
+    """Fewer workgroups than tasks deal themselves the rest: the same bits from however many took part."""
+    from spec_mcts_amd import kernels as K
+    from spec_mcts_amd._lib import check
+    _, _, model = _model(dict(dim=768, n_layers=2, n_heads=6, vocab_size=320, multiple_of=256, max_batch_size=4, max_seq_len=12, max_prompt_seq_len=128), seed=9)
+    tokens = torch.randint(0, 320, (3, 110), generator=torch.Generator().manual_seed(9)).cuda()
+    model(tokens[:1, :100], 0)
+    calls = []
+
+    def launch(self, layers, ws):
+        calls.append(workgroups)
+        check(self.lib.smh_decode_stack_of(layers, len(layers), self.p, ws.data_ptr(), ws.numel(), workgroups, join_us, self.stream), "smh_decode_stack_of")
+
+    for i in range(5):                                 # several steps on one workspace, between launches of all workgroups
+        want = model(tokens[:, 100 + i:101 + i], 100 + i)
+        caches = [model.layers[1].attention.cache_k.clone(), model.layers[1].attention.cache_v.clone()]
+        with monkeypatch.context() as m:
+            m.setattr(K.LayerPass, "decode_stack", launch)
+            got = model(tokens[:, 100 + i:101 + i], 100 + i)
+        assert calls.pop() == workgroups and torch.equal(got, want) and bool(got.isfinite().all())
+        assert torch.equal(caches[0], model.layers[1].attention.cache_k) and torch.equal(caches[1], model.layers[1].attention.cache_v)
+
+
+def test_number_of_workgroups_is_checked():
+    from spec_mcts_amd import _lib, kernels as K
+    p = _lib.SmhPass()
+    p.rows, p.smax, p.h = 2, 8, 256
+    layers = [_pointers()]
+    for workgroups, join_us in ((0, 50), (257, 50), (-1, 50), (256, -1), (256, 1000001)):
+        assert _lib.load().smh_decode_stack_of(K.decode_stack_layers(layers, 2), 1, p, 256, 1 << 30, workgroups, join_us, None) != 0
+        assert b"workgroups" in _lib.load().smh_last_error_string()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,forks", [(2, [(0, 1, 1)]), (3, [(0, 2, 1), (2, 1, 1)]), (4, [(1, 2, 2), (3, 0, 1)])])
+def test_rows_through_the_page_table_match_the_oracle(B, forks, monkeypatch):
+    """Branches that read their ancestors' rows through the page table, and their own behind them (as test_stack_matches_the_oracle)."""
+    from spec_mcts_amd import kernels as K
+    P, steps = 45, 2
+    cfg = dict(dim=512, n_layers=2, n_heads=4, vocab_size=320, multiple_of=256, max_batch_size=5, max_seq_len=40, max_prompt_seq_len=64)
+    oargs, sd, model = _model(cfg, seed=20 + B, std=0.8 / 512 ** 0.5)
+    oracle = O.OracleTransformer(oargs, sd, dense=True)
+    calls = []
+    monkeypatch.setattr(K.LayerPass, "decode_stack", lambda self, layers, ws, _f=K.LayerPass.decode_stack: (calls.append(len(layers)), _f(self, layers, ws)))
+    gen = torch.Generator().manual_seed(B)
+    prompt = torch.randint(0, 320, (1, P), generator=gen)
+    oracle.forward(prompt, 0)
+    model(prompt.cuda(), 0)
+    sync_prefix(model, oracle)
+    at = 0
+    for fork in [None] + forks:
+        if fork is not None:
+            model.fork(*fork)
+            oracle.fork(*fork)
+            assert model._pages(torch.device("cuda:0")) is not None
+        for _ in range(steps):
+            tok = torch.randint(0, 320, (B, 1), generator=gen)
+            want = oracle.forward(tok, P + at).float()
+            got = model(tok.cuda(), P + at)
+            assert calls.pop() == cfg["n_layers"]
+            model.decode_stack = False
+            layers = model(tok.cuda(), P + at).float().cpu()
+            model.decode_stack = True
+            got = got.float().cpu()
+            far, near = float((got - want).norm() / want.norm()), float((layers - want).norm() / want.norm())
+            print("row %d: from the oracle %.2e, layer by layer %.2e" % (at, far, near))
+            assert far <= 2 * near + 2e-3              # (as above)
+            sync_suffix_row(model, oracle, B, at)
+            at += 1
+
+
+def _poison(model, kind):
+    """Writes something that is not finite where one decode step reads it; returns the branches that must not notice."""
+    att, inf, nan = model.layers[0].attention, float("inf"), float("nan")
+    p, H = model.params, att.n_kv_heads
+    own = lambda c, w: c.view(p.max_batch_size, p.max_seq_len, H, w)
+    if kind == "query":                                # of branch 1: token 7's embedding
+        model.tok_embeddings.weight.data[7, 3] = nan
+    elif kind == "own_k_nan":
+        own(att.cache_k_s, 2)[1, 2, 1] = nan
+    elif kind == "own_v_inf":
+        own(att.cache_v_s, 2)[1, 2, 1] = inf
+    elif kind == "behind_the_rows":                    # rows that no branch has yet
+        own(att.cache_k_s, 2)[:, 4:], own(att.cache_v_s, 2)[:, 4:] = nan, inf
+        att.cache_prompt_k[0, 70:], att.cache_prompt_v[0, 70:] = nan, inf
+        return [0, 1, 2]
+    elif kind == "prompt_k_inf":                       # the last row of an odd number: a score of +inf or -inf, by the query's sign
+        att.cache_prompt_k[0, 69, 2, 5] = inf
+        return []
+    elif kind == "prompt_k_lowest":
+        att.cache_prompt_k[0, :, 2] = -65504.0
+        return []
+    elif kind == "prompt_v_inf":
+        att.cache_prompt_v[0, 33, 2, 5] = -inf
+        return []
+    return [0, 2]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["query", "own_k_nan", "own_v_inf", "behind_the_rows", "prompt_k_inf", "prompt_k_lowest", "prompt_v_inf"])
+def test_values_that_are_not_finite_stay_where_they_are(kind):
+    """A branch with a NaN or an infinity among what it reads has the result that the layers' launches give it; the others' bits do not move."""
+    cfg = dict(dim=512, n_layers=1, n_heads=4, vocab_size=320, multiple_of=256, max_batch_size=3, max_seq_len=8, max_prompt_seq_len=96)
+    _, _, model = _model(cfg, seed=31, std=0.8 / 512 ** 0.5)
+    gen = torch.Generator().manual_seed(31)
+    model(torch.randint(0, 320, (1, 70), generator=gen).cuda(), 0)
+    tokens = torch.tensor([[3], [7], [11]]).cuda()
+    for i in range(4):
+        clean = model(tokens, 70 + i)
+    untouched = _poison(model, kind)
+    got = model(tokens, 73)
+    model.decode_stack = False
+    want = model(tokens, 73)
+    for b in untouched:
+        assert torch.equal(got[b], clean[b]), b
+    finite = [bool(want[b].isfinite().all()) for b in range(3)]
+    print(kind, finite)
+    assert [bool(got[b].isfinite().all()) for b in range(3)] == finite
+    assert torch.equal(got.isnan(), want.isnan())
+    for b in range(3):
+        if finite[b]:
+            assert float((got[b].float() - want[b].float()).norm() / want[b].float().norm()) < 4e-3
