@@ -126,12 +126,16 @@ int smh_q40_matmul_plan_tiled(int M, int K, int nseg, const int *n);
  * one workgroup per compute unit); or M > 128, K a multiple of 32, n_half a multiple of 128.  smh_q40_swiglu_fits: 1 when the shape is supported AND wide enough (n_half >= 8192) for
  * this to be the faster way; else use the two launches. */
 int smh_q40_swiglu_fits(int M, int K, int n_half);
+/* columns of the two weights that a workgroup of that launch multiplies (128; above 128 rows 256 or 384, by an estimate); 0: not supported */
+int smh_q40_swiglu_columns(int M, int K, int n_half);
 int smh_q40_matmul_tiled_swiglu(const void *a, int M, int K, long lda, const void *tiled_gate, const void *tiled_up, int n_half,
                                 void *out, long ldo, smh_stream_t stream);
 /* smh_q40_matmul_tiled_direct: LinearQ4_0.forward (:228-236) of up to 3 tiled weights that share the input, for more than 128
  * rows whose launch needs no K-split (smh_q40_matmul_tiled_direct_fits: 1 / 0): out[i][M, n[i]] = fp16(a . w_i), contiguous
  * and 16-byte aligned; with a residual [M, ldr] (one weight only) out = fp16(residual + fp16(a . w)).  No slabs. */
 int smh_q40_matmul_tiled_direct_fits(int M, int K, int nseg, const int *n);
+/* columns that a workgroup of that launch multiplies (192, 256 or 384, by an estimate); 0 where it does not fit */
+int smh_q40_matmul_tiled_direct_columns(int M, int K, int nseg, const int *n);
 int smh_q40_matmul_tiled_direct(const void *a, int M, int K, long lda, int nseg, const void *const *tiled, const int *n, void *const *out,
                                 const void *residual, long ldr, smh_stream_t stream);
 int smh_q40_matmul_partial(const void *a, int M, int K, long lda, int nseg, const void *const *w,

@@ -388,6 +388,21 @@ extern "C" int smh_q40_matmul_tiled_direct_fits(int M, int K, int nseg, const in
     return st < 0 ? st : (gemm_direct_fits(p) ? 1 : 0);
 }
 
+extern "C" int smh_q40_matmul_tiled_direct_columns(int M, int K, int nseg, const int *n) {
+    MatmulParams p;
+    if (smh_q40_matmul_tiled_direct_fits(M, K, nseg, n) != 1) return 0;
+    const int st = fill_params(p, nullptr, M, K, (K + 7) / 8 * 8, nseg, nullptr, nullptr, n, "smh_q40_matmul_tiled_direct_columns", true);
+    return st < 0 ? st : gemm_direct_columns(p);
+}
+
+extern "C" int smh_q40_swiglu_columns(int M, int K, int n_half) {
+    if (!gemm_swiglu_fits(M, K, n_half, false)) return 0;
+    MatmulParams p = MatmulParams{};
+    p.M = M; p.K = K; p.nseg = 2;
+    p.seg[0].N = p.seg[1].N = n_half;
+    return gemm_swiglu_columns(p);
+}
+
 extern "C" int smh_q40_matmul_tiled_direct(const void *a, int M, int K, long lda, int nseg, const void *const *tiled, const int *n, void *const *out,
                                            const void *residual, long ldr, smh_stream_t stream) {
     const char *who = "smh_q40_matmul_tiled_direct";

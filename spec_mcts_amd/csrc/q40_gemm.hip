@@ -1651,6 +1651,21 @@ int gemm_swiglu_launch(const MatmulParams &p, hipStream_t stream) {
 // an output and slice written here and read behind) and no kernel to add them.
 bool gemm_direct_fits(const MatmulParams &p) { return p.tiled && p.M > GEMM_BM && p.K % 32 == 0 && p.ksplit == 1; }
 
+// Both forms of SwiGLU above 128 rows planned: p in workgroups of two pieces of each weight, w of three; true: w promises more.
+static bool gemm_swiglu_rows_plan(MatmulParams &p, MatmulParams &w) {
+    p.units = p.seg[0].N / 128;
+    p.units_pad = (p.units + 7) / 8 * 8;
+    w.units = (p.seg[0].N / 64 + 2) / 3;
+    w.units_pad = (w.units + 7) / 8 * 8;
+    const float narrow_us = gemm_plan_rows(p, p.K / 32, 1, ROWS_256);
+    return gemm_plan_rows(w, p.K / 32, 1, ROWS_384) < narrow_us;
+}
+int gemm_swiglu_columns(MatmulParams p) {
+    if (p.M <= GEMM_BM) return 128;
+    MatmulParams w = p;
+    return gemm_swiglu_rows_plan(p, w) ? 384 : 256;
+}
+
 int gemm_swiglu_rows_launch(MatmulParams p, hipStream_t stream) {
     // (blocks of 64 .. 128 rows)
     static const gemm_kernel_t plain[5] = {q40_gemm_kernel<4, false, true, 8, GEMM_STAGES, false, false, true>, q40_gemm_kernel<5, false, true, 8, GEMM_STAGES, false, false, true>, q40_gemm_kernel<6, false, true, 8, GEMM_STAGES, false, false, true>,
@@ -1676,12 +1691,7 @@ int gemm_swiglu_rows_launch(MatmulParams p, hipStream_t stream) {
     SMH_REQUIRE((long)p.M * p.lda * 2 < (1L << 32), "q40 gemm: M x lda = %d x %ld exceeds the 32-bit lane offsets of A", p.M, p.lda);
     p.kgroups = 0;
     MatmulParams w = p;
-    p.units = p.seg[0].N / 128;
-    p.units_pad = (p.units + 7) / 8 * 8;
-    w.units = (p.seg[0].N / 64 + 2) / 3;
-    w.units_pad = (w.units + 7) / 8 * 8;
-    const float narrow_us = gemm_plan_rows(p, p.K / 32, 1, ROWS_256);
-    if (gemm_plan_rows(w, p.K / 32, 1, ROWS_384) < narrow_us) {
+    if (gemm_swiglu_rows_plan(p, w)) {
         const int t = w.block_rows / 16 - 4;
         hipLaunchKernelGGL(wide[t], dim3((unsigned)((long)w.units_pad * w.mblocks)), dim3(64 * (WIDE_WAVES + 1)), wide_lds[t], stream, w);
         return launch_status();
@@ -1713,6 +1723,12 @@ static int gemm_wide_fits(const MatmulParams &p, MatmulParams &w) {
         }
     }
     return pieces;
+}
+int gemm_direct_columns(MatmulParams p) {
+    MatmulParams w;
+    p.direct = 1;
+    const int pieces = gemm_wide_fits(p, w);
+    return pieces > 0 ? 64 * pieces : GEMM_COLS;
 }
 static int gemm_wide_launch(const MatmulParams &p, int pieces, hipStream_t stream) {
     static const gemm_kernel_t kern[2][5] = {{q40_gemm_wide_kernel<4, WIDE_GROUPS>, q40_gemm_wide_kernel<5, WIDE_GROUPS>, q40_gemm_wide_kernel<6, WIDE_GROUPS>,

@@ -94,5 +94,8 @@ int gemm_swiglu_launch(const MatmulParams &p, hipStream_t stream);     // seg[0]
 bool gemm_direct_fits(const MatmulParams &p);
 // SiLU(gate) * up for more than 128 rows: seg[0] = gate, seg[1] = up (tiled), seg[0].c / ldc = the activations
 int gemm_swiglu_rows_launch(MatmulParams p, hipStream_t stream);
+// columns that a workgroup of these launches multiplies
+int gemm_direct_columns(MatmulParams p);
+int gemm_swiglu_columns(MatmulParams p);
 
 }  // namespace smh

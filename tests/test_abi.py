@@ -148,3 +148,23 @@ def test_layer_scratch_holds_every_slab_of_a_pass():
                 gate_up = 0 if M > 128 and swiglu and lib.smh_q40_swiglu_fits(M, dim, ffn) else lib.smh_q40_matmul_plan_tiled(M, dim, 2, (ctypes.c_int * 2)(ffn, ffn)) * M * 2 * ffn * 4
                 need = 2 * M * (3 * dim + 2 * nq + 2 * nkv + ffn) + max(slabs(M, dim, nq, nkv, nkv), gate_up) + max(slabs(M, nq, dim), slabs(M, ffn, dim))
                 assert lib.smh_decode_scratch_bytes(layer, M, swiglu) >= need, (dim, swiglu, M)
+
+
+def test_columns_of_a_workgroup_above_128_rows():
+    """which of the launches above 128 rows a shape takes (the GPU tests of each ask here), 0 where there is none"""
+    from spec_mcts_amd import _lib
+    lib = _lib.load()
+
+    def direct(M, K, *ns):
+        return lib.smh_q40_matmul_tiled_direct_columns(M, K, len(ns), (ctypes.c_int * len(ns))(*ns))
+
+    assert direct(128, 4096, 4096) == 0 and direct(512, 4096 + 8, 11008) == 0 and direct(512, 4096, 100) == 0
+    assert direct(2047, 4096, 11008 + 64) == 0
+    for M in (129, 300, 512, 1024, 2047):
+        for K, ns in ((4096, (4096, 4096, 4096)), (11008, (4096,)), (96, (10624,)), (8192, (8192, 1024, 1024))):
+            fits = lib.smh_q40_matmul_tiled_direct_fits(M, K, len(ns), (ctypes.c_int * len(ns))(*ns))
+            columns = direct(M, K, *ns)
+            assert columns in ((192, 256, 384) if fits else (0,)) and not (columns == 192 and K % 64)
+    assert lib.smh_q40_swiglu_columns(16, 4096, 11008) == 0 and lib.smh_q40_swiglu_columns(300, 4096 + 8, 11008) == 0
+    assert lib.smh_q40_swiglu_columns(100, 4096, 11008) == 128
+    assert {lib.smh_q40_swiglu_columns(M, 4096, 11008) for M in range(129, 600)} == {256, 384}

@@ -1,5 +1,7 @@
 """Tiled weight layout (smh_q40_tile, smh_q40_matmul_partial_tiled): the tiles against an element-by-element
 numpy statement of the layout, and the products against the checkpoint-layout kernels (bit for bit) and the oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -294,9 +296,10 @@ def test_swiglu_inside_the_gate_up_launch_above_128_rows(M, K, n_half):
                                         (130, 160, 22016),      # five steps; five row tiles
                                         (256, 4096, 11008)])    # four row tiles
 def test_swiglu_three_pieces_a_workgroup(M, K, n_half):
-    """sizes that q40_gemm_swiglu_wide_kernel takes (its estimate is the smaller one), against the oracle's two matmuls"""
+    """sizes that q40_gemm_wide_kernel takes (its estimate is the smaller one), against the oracle's two matmuls"""
     import torch.nn.functional as F
-    from spec_mcts_amd import kernels as Kn
+    from spec_mcts_amd import _lib, kernels as Kn
+    assert _lib.load().smh_q40_swiglu_columns(M, K, n_half) == 384
     w1, w3 = _weight(K, n_half, 1990 + K), _weight(K, n_half, 1991 + K)
     x = (torch.randn((M, K), generator=torch.Generator().manual_seed(1992 + M)) * 0.5).half()
     got = Kn.matmul_q40_swiglu(x.cuda(), Kn.tile_q40(w1[0].cuda(), w1[1].cuda(), K, n_half), Kn.tile_q40(w3[0].cuda(), w3[1].cuda(), K, n_half)).cpu()
@@ -323,26 +326,29 @@ def test_direct_products(M, K, ns):
         assert torch.allclose(o.cpu().float(), want, rtol=1e-2, atol=2e-3)
 
 
-@pytest.mark.parametrize("M,K,ns", [(192, 64, [1152]),                     # one stage; four row tiles; three pieces throughout
-                                    (129, 64, [1280]),                     # five row tiles, the last block of 49 rows; a last workgroup of two pieces
-                                    (257, 128, [10624]),                   # two stages; six row tiles; one piece
-                                    (512, 704, [7040, 128, 896]),          # eleven stages; seven row tiles; workgroups across weights, odd 128-column blocks
-                                    (600, 448, [7808]),                    # seven stages, more than the ring holds; eight row tiles
-                                    (400, 4096, [4096, 4096, 4096]),
-                                    # six pieces of one step
-                                    (700, 96, [10624]),                    # three steps; six row tiles, the last block of 28 rows; a last workgroup of four pieces
-                                    (1100, 32, [6272]),                    # one step; seven row tiles; two pieces
-                                    (700, 32, [5120, 128, 5120]),          # eight row tiles; workgroups across weights, an odd 128-column block; six pieces throughout
-                                    (1024, 4096, [4096, 4096, 4096])])
-def test_wide_workgroups(M, K, ns):
+WIDE = [(192, 64, [1152], 192),                     # one stage; four row tiles; three pieces throughout
+        (129, 64, [1280], 192),                     # five row tiles, the last block of 49 rows; a last workgroup of two pieces
+        (257, 128, [10624], 192),                   # two stages; six row tiles; one piece
+        (512, 704, [7040, 128, 896], 192),          # eleven stages; seven row tiles; workgroups across weights, odd 128-column blocks
+        (600, 448, [7808], 192),                    # seven stages, more than the ring holds; eight row tiles
+        (400, 4096, [4096, 4096, 4096], 192),
+        # six pieces of one step
+        (700, 96, [10624], 384),                    # three steps; six row tiles, the last block of 28 rows; a last workgroup of four pieces
+        (1100, 32, [6272], 384),                    # one step; seven row tiles; two pieces
+        (700, 32, [5120, 128, 5120], 384),          # eight row tiles; workgroups across weights, an odd 128-column block; six pieces throughout
+        (1024, 4096, [4096, 4096, 4096], 384)]
+
+
+@pytest.mark.parametrize("M,K,ns,columns", WIDE)
+def test_wide_workgroups(M, K, ns, columns):
     """sizes above 128 rows that q40_gemm_wide_kernel takes (three pieces and two K-groups, or six pieces, have the smaller
     estimate): fp16 results with and without a residual"""
-    from spec_mcts_amd import kernels as Kn
+    from spec_mcts_amd import _lib, kernels as Kn
+    assert _lib.load().smh_q40_matmul_tiled_direct_columns(M, K, len(ns), (ctypes.c_int * len(ns))(*ns)) == columns
     ws = [_weight(K, n, 2000 + i + K) for i, n in enumerate(ns)]
     tiled = [Kn.tile_q40(w.cuda(), s.cuda(), K, n) for (w, s), n in zip(ws, ns)]
     a = (torch.randn((M, K), generator=torch.Generator().manual_seed(2001 + M)) * 0.5).half()
     r = torch.randn((M, ns[0]), generator=torch.Generator().manual_seed(2002)).half() if len(ns) == 1 else None
-    assert Kn.matmul_plan(M, K, ns, tiled=True) == 1
     got = Kn.matmul_q40_direct(a.cuda(), tiled)
     with_r = Kn.matmul_q40_direct(a.cuda(), tiled, residual=r.cuda()) if r is not None else got
     for (w, s), n, o, o_r in zip(ws, ns, got, with_r):
