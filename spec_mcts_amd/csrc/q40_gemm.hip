@@ -1393,7 +1393,8 @@ constexpr RowsCost ROWS_384 = {0.21f, 0.37f, 4.0f, 1.15f, 0.0f};
 constexpr RowsCost ROWS_192 = {0.11f, 0.21f, 4.0f, 1.2f, 0.0f};
 // Six pieces of direct products (384 columns): the step of ROWS_384; with its `busy` a launch that nearly fills a round was estimated 10 to
 // 15 % short (8192 x 10240 at 1024 rows 173 us, 3 % more than with 192 columns).  Taken where it promises 3 % more than the others:
-// 0.85 .. 0.98 of their time, once 1.007 (1536 rows of 4096 x 12288).
+// 0.85 .. 0.98 of their time, once 1.007 (1536 rows of 4096 x 12288).  Where that is between 3 and 6 % against 256 columns: 0.85 .. 0.96 (us,
+// 4096 x 12288 at 1600 rows 179 -> 155, 5120 x 15360 at 1240 rows 222 -> 189, at 2047 305 -> 291, 4096 x 11008 at 1929 rows 186 -> 175).
 constexpr RowsCost ROWS_SIX = {0.21f, 0.37f, 4.0f, 1.0f, 0.15f};
 static float gemm_rows_us(const RowsCost &t, int units, long of_unit, int rows, int steps) {
     const float r = (float)(units * of_unit) / 256.0f, rounds = (float)(((units + 7) / 8 * of_unit + 31) / 32);
@@ -1709,14 +1710,14 @@ static int gemm_wide_fits(const MatmulParams &p, MatmulParams &w) {
     if (!p.tiled || !p.direct || p.M <= GEMM_BM || p.ksplit != 1 || p.K % 32 != 0) return 0;
     int pieces = 0;
     w = p;
-    float least = 0.97f * gemm_plan_rows(w, p.K / 32, 1, ROWS_256);
+    float least = gemm_plan_rows(w, p.K / 32, 1, ROWS_256);
     for (int n = 3; n <= 6; n += 3) {
         if (n == 3 && p.K % 64 != 0) continue;
         MatmulParams t = p;
         t.units = (p.n_total / 64 + n - 1) / n;
         t.units_pad = (t.units + 7) / 8 * 8;
         const float us = gemm_plan_rows(t, p.K / 32, 1, n == 3 ? ROWS_192 : ROWS_SIX);
-        if (us < (n == 3 ? least : 0.97f * least)) {
+        if (us < 0.97f * least) {
             least = us;
             w = t;
             pieces = n;

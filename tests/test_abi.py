@@ -165,6 +165,8 @@ def test_columns_of_a_workgroup_above_128_rows():
             fits = lib.smh_q40_matmul_tiled_direct_fits(M, K, len(ns), (ctypes.c_int * len(ns))(*ns))
             columns = direct(M, K, *ns)
             assert columns in ((192, 256, 384) if fits else (0,)) and not (columns == 192 and K % 64)
+    # six pieces where they promise 3 %, against whichever of the others promises most (here 256 columns; 4 % at these sizes)
+    assert direct(1600, 4096, 4096, 4096, 4096) == 384 and direct(1961, 5120, 5120, 5120, 5120) == 384 and direct(1929, 4096, 11008) == 384
     assert lib.smh_q40_swiglu_columns(16, 4096, 11008) == 0 and lib.smh_q40_swiglu_columns(300, 4096 + 8, 11008) == 0
     assert lib.smh_q40_swiglu_columns(100, 4096, 11008) == 128
     assert {lib.smh_q40_swiglu_columns(M, 4096, 11008) for M in range(129, 600)} == {256, 384}
