@@ -19,20 +19,20 @@ namespace smh {
 // ---- plain reduce (+ residual) ------------------------------------------------------------------
 // RES: a residual of this alignment (elements a load; 0: none)
 template <int KS, int RES>
-__global__ __launch_bounds__(256) void partial_reduce_kernel(const void *__restrict__ partial, int M, int n_total, int col0, int N,
+__global__ __launch_bounds__(256) void partial_reduce_kernel(const void *__restrict__ partial, int ks, int M, int n_total, int col0, int N,
                                                              half_t *__restrict__ c, long ldc, const half_t *__restrict__ resid, long ldr) {
     const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
     if (i >= (long)M * N) return;
     const int m = (int)(i / N), n = (int)(i % N);          // N % 4 == 0: the 4 columns share a row
     f4 v[KS];
-    slab_load(partial, (long)m * n_total + col0 + n, (long)M * n_total, v);
+    slab_load(partial, (long)m * n_total + col0 + n, (long)M * n_total, ks, v);
     h4 r;
     if constexpr (RES == 4) r = *reinterpret_cast<const h4 *>(resid + (long)m * ldr + n);
     if constexpr (RES == 1) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) r[j] = resid[(long)m * ldr + n + j];
     }
-    const f4 acc = slab_add(v);
+    const f4 acc = slab_add(v, ks);
     h4 out;
 #pragma unroll
     for (int j = 0; j < 4; ++j) out[j] = RES == 0 ? (half_t)acc[j] : (half_t)((float)r[j] + (float)(half_t)acc[j]);
@@ -44,7 +44,7 @@ __global__ __launch_bounds__(256) void partial_reduce_kernel(const void *__restr
 // A chain of trips to memory bounds it, so everything is requested before the first sum: KS slabs (0: none), PASSES passes of four
 // columns a thread, the residual and the norm's weights.  Up to 64 registers two workgroups share a compute unit.
 template <int PASSES, int KS>
-__global__ __launch_bounds__(1024, PASSES * KS <= 8 ? 8 : 4) void partial_rmsnorm_kernel(const void *__restrict__ partial, int M, int N,
+__global__ __launch_bounds__(1024, PASSES * KS <= 8 ? 8 : 4) void partial_rmsnorm_kernel(const void *__restrict__ partial, int ks, int M, int N,
                                                                const half_t *__restrict__ h_in, const half_t *__restrict__ wt,
                                                                float eps, half_t *__restrict__ h_out, half_t *__restrict__ xn_out) {
     __shared__ float s_part[16];
@@ -60,7 +60,7 @@ __global__ __launch_bounds__(1024, PASSES * KS <= 8 ? 8 : 4) void partial_rmsnor
     for (int ps = 0; ps < PASSES; ++ps) {
         const int n = (ps * 1024 + threadIdx.x) * 4;
         if (n < N) {
-            if constexpr (KS > 0 && AHEAD == PASSES) slab_load(partial, (long)m * N + n, slab, v[ps % AHEAD]);
+            if constexpr (KS > 0 && AHEAD == PASSES) slab_load(partial, (long)m * N + n, slab, ks, v[ps % AHEAD]);
             hv[ps] = *reinterpret_cast<const h4 *>(from + n);
             wv[ps] = *reinterpret_cast<const h4 *>(wt + n);
         }
@@ -71,8 +71,8 @@ __global__ __launch_bounds__(1024, PASSES * KS <= 8 ? 8 : 4) void partial_rmsnor
         if (n < N) {
             h4 &h = hv[ps];
             if constexpr (KS > 0) {
-                if constexpr (AHEAD < PASSES) slab_load(partial, (long)m * N + n, slab, v[0]);
-                const f4 acc = slab_add(v[ps % AHEAD]);
+                if constexpr (AHEAD < PASSES) slab_load(partial, (long)m * N + n, slab, ks, v[0]);
+                const f4 acc = slab_add(v[ps % AHEAD], ks);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) h[j] = h_in != nullptr ? (half_t)((float)h[j] + (float)(half_t)acc[j]) : (half_t)acc[j];
             }
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const half_t *__restr
 // thread, same order of additions), so sums[m][0..15] added in index order give that kernel's sum of squares bit
 // for bit.  The consumer (the matmul that follows, q40_gemv_kernel LAYOUT 3) normalises its own K-slice.
 template <int PASSES, int KS>
-__global__ __launch_bounds__(64) void partial_residual_sumsq_kernel(const void *__restrict__ partial, int M, int N,
+__global__ __launch_bounds__(64) void partial_residual_sumsq_kernel(const void *__restrict__ partial, int ks, int M, int N,
                                                                     const half_t *__restrict__ h_in, half_t *__restrict__ h_out,
                                                                     float *__restrict__ sums) {
     const int m = blockIdx.y;
@@ -160,7 +160,7 @@ __global__ __launch_bounds__(64) void partial_residual_sumsq_kernel(const void *
     for (int ps = 0; ps < PASSES; ++ps) {
         const int n = (ps * 1024 + vt) * 4;
         if (n < N) {
-            slab_load(partial, (long)m * N + n, slab, acc[ps]);
+            slab_load(partial, (long)m * N + n, slab, ks, acc[ps]);
             if (h_in != nullptr) res[ps] = *reinterpret_cast<const h4 *>(h_in + (long)m * N + n);
         }
     }
@@ -169,7 +169,7 @@ __global__ __launch_bounds__(64) void partial_residual_sumsq_kernel(const void *
     for (int ps = 0; ps < PASSES; ++ps) {
         const int n = (ps * 1024 + vt) * 4;
         if (n < N) {
-            const f4 sum = slab_add(acc[ps]);
+            const f4 sum = slab_add(acc[ps], ks);
             h4 v;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -188,16 +188,16 @@ __global__ __launch_bounds__(64) void partial_residual_sumsq_kernel(const void *
 // ---- SwiGLU gate ------------------------------------------------------------------------------------
 // slabs hold [gate | up] (2 * n_half columns)
 template <int KS>
-__global__ __launch_bounds__(256) void partial_silu_mul_kernel(const void *__restrict__ partial, int M, int n_half,
+__global__ __launch_bounds__(256) void partial_silu_mul_kernel(const void *__restrict__ partial, int ks, int M, int n_half,
                                                                half_t *__restrict__ out) {
     // grid (quads of a row, rows): no division to find the row (a 64-bit one costs more than the rest of the arithmetic)
     const int m = blockIdx.y, n = (blockIdx.x * 256 + threadIdx.x) * 4;
     if (n >= n_half) return;
     const long slab = (long)M * 2 * n_half;
     f4 gv[KS], uv[KS];
-    slab_load(partial, (long)m * 2 * n_half + n, slab, gv);
-    slab_load(partial, (long)m * 2 * n_half + n_half + n, slab, uv);
-    const f4 ga = slab_add(gv), ua = slab_add(uv);
+    slab_load(partial, (long)m * 2 * n_half + n, slab, ks, gv);
+    slab_load(partial, (long)m * 2 * n_half + n_half + n, slab, ks, uv);
+    const f4 ga = slab_add(gv, ks), ua = slab_add(uv, ks);
     h4 o;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -211,7 +211,7 @@ __global__ __launch_bounds__(256) void partial_silu_mul_kernel(const void *__res
 // one wave per (branch, head); heads 0..H-1 queries, H..H+Hkv-1 keys, H+Hkv.. values.
 // slab columns: [q (H*128) | k (Hkv*128) | v (Hkv*128)]
 template <int KS>
-__global__ __launch_bounds__(256) void partial_rope_append_kernel(const void *__restrict__ partial, int B, int H, int Hkv,
+__global__ __launch_bounds__(256) void partial_rope_append_kernel(const void *__restrict__ partial, int ks, int B, int H, int Hkv,
                                                                   half_t *__restrict__ q, half_t *__restrict__ k, half_t *__restrict__ v,
                                                                   const half_t *__restrict__ cos_tab, const half_t *__restrict__ sin_tab,
                                                                   const int32_t *__restrict__ pos_dev,
@@ -232,12 +232,12 @@ __global__ __launch_bounds__(256) void partial_rope_append_kernel(const void *__
     // change lanes through LDS
     // the slabs first: the position, and behind it the rotation factors, travel under them
     f2 parts[KS];
-    slab_load(partial, (long)b * n_total + (long)h * 128 + 2 * lane, (long)B * n_total, parts);
+    slab_load(partial, (long)b * n_total + (long)h * 128 + 2 * lane, (long)B * n_total, ks, parts);
     const int t = (t_dev != nullptr) ? *t_dev : -1;
     const int pos = *pos_dev;
     const half_t cos_l = cos_tab[(long)pos * 64 + lane], sin_l = sin_tab[(long)pos * 64 + lane];
     if (live) {
-        const f2 sum = slab_add(parts);
+        const f2 sum = slab_add(parts, ks);
         *reinterpret_cast<f2 *>(&s_row[wave][2 * lane]) = sum;
     }
     __syncthreads();
@@ -275,7 +275,7 @@ __global__ __launch_bounds__(256) void partial_rope_append_kernel(const void *__
 // A prefill's q|k|v product -> q, and k, v as rows of the prompt cache (fp16): sums, one rounding, RoPE of q and k at position
 // row + pos0.  One thread owns four rotation pairs (d .. d+3, d+64 ..) of one head.
 template <int KS>
-__global__ __launch_bounds__(256) void partial_rope_rows_kernel(const void *__restrict__ partial, int S, int H, int Hkv,
+__global__ __launch_bounds__(256) void partial_rope_rows_kernel(const void *__restrict__ partial, int ks, int S, int H, int Hkv,
                                                                 half_t *__restrict__ q, half_t *__restrict__ k, half_t *__restrict__ v,
                                                                 const half_t *__restrict__ cos_tab, const half_t *__restrict__ sin_tab, int pos0) {
     const int heads = H + 2 * Hkv, s = blockIdx.y;
@@ -284,9 +284,9 @@ __global__ __launch_bounds__(256) void partial_rope_rows_kernel(const void *__re
     const int n_total = heads * 128;
     const long at = (long)s * n_total + h * 128 + d, slab = (long)S * n_total;
     f4 lo_v[KS], hi_v[KS];
-    slab_load(partial, at, slab, lo_v);
-    slab_load(partial, at + 64, slab, hi_v);
-    const f4 lo = slab_add(lo_v), hi = slab_add(hi_v);
+    slab_load(partial, at, slab, ks, lo_v);
+    slab_load(partial, at + 64, slab, ks, hi_v);
+    const f4 lo = slab_add(lo_v, ks), hi = slab_add(hi_v, ks);
     h4 x1, x2;
 #pragma unroll
     for (int j = 0; j < 4; ++j) { x1[j] = (half_t)lo[j]; x2[j] = (half_t)hi[j]; }
@@ -308,12 +308,12 @@ __global__ __launch_bounds__(256) void partial_rope_rows_kernel(const void *__re
 
 using namespace smh;
 
-// kernels by the number of slabs
+// kernels by the number of slabs (least_slabs)
 static_assert(SMH_MAX_KSPLIT == 16, "tables");
-#define BY_SLABS(k, ...) {__VA_ARGS__, k(1), k(2), k(3), k(4), k(5), k(6), k(7), k(8), k(9), k(10), k(11), k(12), k(13), k(14), k(15), k(16)}
-typedef void (*reduce_kernel_t)(const void *, int, int, int, int, half_t *, long, const half_t *, long);
-typedef void (*rmsnorm_kernel_t)(const void *, int, int, const half_t *, const half_t *, float, half_t *, half_t *);
-typedef void (*sumsq_kernel_t)(const void *, int, int, const half_t *, half_t *, float *);
+#define BY_SLABS(k, ...) {__VA_ARGS__, k(1), k(2), k(3), k(4), k(5), k(6), k(8), k(8), k(10), k(10), k(12), k(12), k(16), k(16), k(16), k(16)}
+typedef void (*reduce_kernel_t)(const void *, int, int, int, int, int, half_t *, long, const half_t *, long);
+typedef void (*rmsnorm_kernel_t)(const void *, int, int, int, const half_t *, const half_t *, float, half_t *, half_t *);
+typedef void (*sumsq_kernel_t)(const void *, int, int, int, const half_t *, half_t *, float *);
 #define K_OF(n) partial_reduce_kernel<n, RES>
 template <int RES> static const reduce_kernel_t REDUCE_KERNELS[17] = BY_SLABS(K_OF, nullptr);
 #undef K_OF
@@ -537,7 +537,7 @@ static int reduce_launch(const void *partial, int ksplit, int M, int n_total, in
     long quads = ((long)M * N + 3) / 4;
     const bool aligned = ldr % 4 == 0 && (uintptr_t)residual % 8 == 0;
     const auto kern = (epilogue != SMH_EPI_RESIDUAL ? REDUCE_KERNELS<0> : aligned ? REDUCE_KERNELS<4> : REDUCE_KERNELS<1>)[ksplit];
-    hipLaunchKernelGGL(kern, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream, partial, M, n_total, col0, N, (half_t *)c, ldc,
+    hipLaunchKernelGGL(kern, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream, partial, ksplit, M, n_total, col0, N, (half_t *)c, ldc,
                        (const half_t *)residual, ldr);
     return launch_status();
 }
@@ -613,7 +613,7 @@ extern "C" int smh_partial_rmsnorm(const void *partial, int ksplit, int M, int N
     }
     const int ks = partial == nullptr ? 0 : ksplit;
     const auto kern = N <= 4096 ? RMSNORM_KERNELS<1>[ks] : N <= 8192 ? RMSNORM_KERNELS<2>[ks] : RMSNORM_KERNELS<4>[ks];
-    hipLaunchKernelGGL(kern, dim3(M), dim3(1024), 0, (hipStream_t)stream, partial, M, N, (const half_t *)h_in, (const half_t *)weight, eps, (half_t *)h_out,
+    hipLaunchKernelGGL(kern, dim3(M), dim3(1024), 0, (hipStream_t)stream, partial, ks, M, N, (const half_t *)h_in, (const half_t *)weight, eps, (half_t *)h_out,
                        (half_t *)xn_out);
     return launch_status();
 }
@@ -625,7 +625,7 @@ extern "C" int smh_partial_residual_sumsq(const void *partial, int ksplit, int M
     if (M == 0) return 0;
     SMH_REQUIRE(h_out && sums, "smh_partial_residual_sumsq: null pointer");
     const auto kern = N <= 4096 ? SUMSQ_KERNELS<1>[ksplit] : N <= 8192 ? SUMSQ_KERNELS<2>[ksplit] : SUMSQ_KERNELS<4>[ksplit];
-    hipLaunchKernelGGL(kern, dim3(SMH_NORM_SUMS, M), dim3(64), 0, (hipStream_t)stream, partial, M, N, (const half_t *)h_in, (half_t *)h_out, (float *)sums);
+    hipLaunchKernelGGL(kern, dim3(SMH_NORM_SUMS, M), dim3(64), 0, (hipStream_t)stream, partial, ksplit, M, N, (const half_t *)h_in, (half_t *)h_out, (float *)sums);
     return launch_status();
 }
 
@@ -636,7 +636,7 @@ extern "C" int smh_partial_silu_mul(const void *partial, int ksplit, int M, int 
     SMH_REQUIRE(partial && out, "smh_partial_silu_mul: null pointer");
     SMH_REQUIRE(M <= 65535, "smh_partial_silu_mul: M=%d (at most 65535 rows per launch)", M);
     hipLaunchKernelGGL(SILU_KERNELS[ksplit], dim3((unsigned)((n_half / 4 + 255) / 256), (unsigned)M), dim3(256), 0, (hipStream_t)stream,
-                       partial, M, n_half, (half_t *)out);
+                       partial, ksplit, M, n_half, (half_t *)out);
     return launch_status();
 }
 
@@ -652,7 +652,7 @@ extern "C" int smh_partial_rope_append_kv(const void *partial, int ksplit, int B
     SMH_REQUIRE(!cache_k || (cache_ks && cache_v && cache_vs && t_dev && Smax > 0), "smh_partial_rope_append_kv: cache arguments incomplete");
     SMH_REQUIRE(B <= 65535, "smh_partial_rope_append_kv: B=%d (at most 65535 branches per launch)", B);
     hipLaunchKernelGGL(ROPE_APPEND_KERNELS[ksplit], dim3((unsigned)((H + 2 * Hkv + 3) / 4), (unsigned)B), dim3(256), 0, (hipStream_t)stream,
-                       partial, B, H, Hkv, (half_t *)q, (half_t *)k, (half_t *)v,
+                       partial, ksplit, B, H, Hkv, (half_t *)q, (half_t *)k, (half_t *)v,
                        (const half_t *)cos_tab, (const half_t *)sin_tab, pos_dev, (uint8_t *)cache_k, (half_t *)cache_ks,
                        (uint8_t *)cache_v, (half_t *)cache_vs, Smax, t_dev);
     return launch_status();
@@ -665,7 +665,7 @@ extern "C" int smh_partial_rope_rows(const void *partial, int ksplit, int S, int
     SMH_REQUIRE(S >= 0 && S <= 65535 && H > 0 && Hkv > 0 && pos0 >= 0, "smh_partial_rope_rows: S=%d (at most 65535) H=%d Hkv=%d pos0=%d", S, H, Hkv, pos0);
     if (S == 0) return 0;
     SMH_REQUIRE(partial && q && k && v && cos_tab && sin_tab, "smh_partial_rope_rows: null pointer");
-    hipLaunchKernelGGL(ROPE_ROWS_KERNELS[ksplit], dim3((unsigned)(((H + 2 * Hkv) * 16 + 255) / 256), (unsigned)S), dim3(256), 0, (hipStream_t)stream, partial,
+    hipLaunchKernelGGL(ROPE_ROWS_KERNELS[ksplit], dim3((unsigned)(((H + 2 * Hkv) * 16 + 255) / 256), (unsigned)S), dim3(256), 0, (hipStream_t)stream, partial, ksplit,
                        S, H, Hkv, (half_t *)q, (half_t *)k, (half_t *)v, (const half_t *)cos_tab, (const half_t *)sin_tab, pos0);
     return launch_status();
 }

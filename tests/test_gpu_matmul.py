@@ -271,3 +271,41 @@ def test_matmul_with_few_column_units(M, N, K):
     assert torch.allclose(got, want, rtol=RTOL, atol=ATOL)
     got = K_.matmul_q40(a.cuda(), w.cuda(), s.cuda(), (K, N), residual=r.cuda()).cpu().float()
     assert torch.allclose(got, r.float() + want, rtol=RTOL, atol=2 * ATOL)
+
+
+@pytest.mark.parametrize("ks", range(1, 17))
+def test_consumers_at_every_number_of_slabs(ks):
+    """Each consumer of a product's slabs against itself on one slab that holds their sum: the sums in slice order and nothing else, at
+    numbers with a kernel of their own and at those between; what lies behind the last slab (NaN) is not added."""
+    from spec_mcts_amd import _lib, kernels as K
+    lib, dev = _lib.load(), "cuda:0"
+    g = torch.Generator(device=dev).manual_seed(ks)
+    for M, n in ((3, 768), (2, 5120), (2, 12288)):     # one, two and four passes of a row; two query heads and more, one kv head in three
+        buf = torch.full((17, M, n), float("nan"), device=dev)
+        buf[:ks] = torch.randn((ks, M, n), device=dev, generator=g)
+        total = torch.zeros((M, n), device=dev)
+        for s in range(ks):
+            total = total + buf[s]
+        both = K.PartialProduct(buf, ks, M, n), K.PartialProduct(total[None].contiguous(), 1, M, n)
+        h, w = torch.randn((M, n), device=dev, generator=g).half(), torch.randn(n, device=dev, generator=g).half()
+        odd = torch.empty(M * n + 1, dtype=torch.float16, device=dev)[1:].view(M, n).copy_(h)          # (a residual that is not aligned)
+        heads = n // 128
+        hkv = heads // 6
+        H = heads - 2 * hkv
+        angles = torch.randn((16, 64), device=dev, generator=g)
+        cos, sin = angles.cos().half(), angles.sin().half()
+        results = []
+        for p in both:
+            out = [K.partial_reduce(p), K.partial_reduce(p, 128, 256), K.partial_reduce(p, residual=h), K.partial_reduce(p, residual=odd)]
+            out += [*K.partial_rmsnorm(p, h, w, 1e-5), *K.partial_rmsnorm(p, None, w, 1e-5), *K.partial_residual_sumsq(p, h), *K.partial_residual_sumsq(p, None)]
+            out.append(K.partial_silu_mul(p))
+            ck, cks = torch.zeros((M * 4 * hkv, 64), dtype=torch.int8, device=dev), torch.zeros((M * 8 * hkv, 1), dtype=torch.float16, device=dev)
+            cv, cvs = ck.clone(), cks.clone()
+            st = torch.tensor([9, 2], dtype=torch.int32, device=dev)
+            out += [*K.partial_rope_append_kv(p, H, hkv, 128, cos, sin, st[0:1], ck, cks, cv, cvs, 4, st[1:2]), ck, cks, cv, cvs]
+            q, k, v = (torch.empty((M, x, 128), dtype=torch.float16, device=dev) for x in (H, hkv, hkv))
+            _lib.check(lib.smh_partial_rope_rows(p.buf.data_ptr(), p.ksplit, M, H, hkv, 128, q.data_ptr(), k.data_ptr(), v.data_ptr(), cos.data_ptr(),
+                                                 sin.data_ptr(), 1, K._stream()), "smh_partial_rope_rows")
+            results.append(out + [q, k, v])
+        for i, (a, b) in enumerate(zip(*results)):
+            assert bool(a.float().isfinite().all()) and torch.equal(a, b), (i, M, n)
