@@ -321,9 +321,12 @@ class Transformer(nn.Module):
         self._norm_in_ok = {}
         self.attn_from_qkv = True          # where the attention is one launch it takes the wq|wk|wv product itself
         self.decode_stack = True           # up to 4 branches (multi-head attention): all layers of a decode step in one launch
-        # ... behind a prompt of at least so many rows.  Its sums come in another order than the launches', and what that changes of a row's
-        # Q4_0 codes weighs by the row's share of the attention: after eight steps the two ways' logits differ by 2e-2 behind 64 shared rows
-        # (two forms of the attention alone by 1.5e-2), by 1.6e-2 behind 96, 0.9e-2 behind 256.
+        # ... behind a prompt of at least so many rows.  Not for precision: against 64 bits both ways are equally far off, a step 5.4e-3 .. 6.9e-3
+        # behind 16 .. 512 rows (stack and layers 0.92 .. 1.11 of each other), eight steps 8.9e-2 and 8.8e-2 behind 16, 5.0e-2 and 4.9e-2
+        # behind 64, 1.3e-2 and 1.3e-2 behind 512: each rounds to fp16 and quantises its own rows, which a short prompt gives much of
+        # the attention's weight.  That also takes the two ways apart, by 6.3e-2 after eight steps behind 16 rows, 2.1e-2 behind 64, 1.8e-2 behind
+        # 95: the line keeps what a search behind a short prompt returns within 2e-2 of what it returned layer by layer.  Where that
+        # does not matter, 0 takes one launch behind every prompt.
         self.decode_stack_min_prompt = 96
         self._stack_ws = None
         self._q40_output = None            # quantize_lm_head(): (w, s, padded vocab) of a Q4_0 vocabulary projection
