@@ -404,6 +404,15 @@ int smh_shared_prefix_attn_qkv(const void *qkv_partial, int ksplit, void *out, i
                                const int32_t *t_dev, const int32_t *pages, int pages_stride, int single_launch,
                                void *workspace, size_t workspace_bytes, smh_stream_t stream);
 
+/* smh_shared_prefix_attn_qkv_tiles: the same from any number of branches in ONE launch without a workspace: a workgroup has 16 queries of
+ * a kv head, reads the whole prefix for them and walks their branches' rows (the faster form where these workgroups fit the GPU in one
+ * round).  Equal to the other forms up to fp32 summation order.  pages: rows of a pool of cache_rows rows (not read without pages). */
+int smh_shared_prefix_attn_qkv_tiles(const void *qkv_partial, int ksplit, void *out, int B, int H, int Hkv, int D,
+                                     const void *cos_tab, const void *sin_tab, const int32_t *pos_dev,
+                                     const void *prefix_k, const void *prefix_v, int P,
+                                     void *cache_k, void *cache_ks, void *cache_v, void *cache_vs, int Smax,
+                                     const int32_t *t_dev, const int32_t *pages, int pages_stride, long cache_rows, smh_stream_t stream);
+
 /* ---- a transformer layer of a decode step in one call ----------------------------------------------------------------
  * TransformerBlock.forward (hf_model_q40_kv_shared.py:439-467) for one token per branch, on tiled weights: the launches of
  * the operators above in the order the model issues them, without the host work between them.

@@ -95,6 +95,8 @@ SIGNATURES = {
     "smh_attn_qkv_workspace_bytes": (c_size_t, [c_int, c_int, c_int]),
     "smh_shared_prefix_attn_qkv": (c_int, [_P, c_int, _P, c_int, c_int, c_int, c_int, _P, _P, _P, _P, _P, c_int,
                                            _P, _P, _P, _P, c_int, _P, _P, c_int, c_int, _P, c_size_t, _P]),
+    "smh_shared_prefix_attn_qkv_tiles": (c_int, [_P, c_int, _P, c_int, c_int, c_int, c_int, _P, _P, _P, _P, _P, c_int,
+                                                 _P, _P, _P, _P, c_int, _P, _P, c_int, c_long, _P]),
     "smh_paged_prefix_attn": (c_int, [_P, _P, c_int, c_int, c_int, c_int, _P, _P, c_int, c_long, c_long,
                                       c_int, _P, _P, _P, _P, c_long, c_long, c_long, _P, c_int, c_long, c_int, _P, c_int, _P, _P, c_int,
                                       _P, c_size_t, _P]),

@@ -15,7 +15,7 @@
 // With fp16 suffixes the slices and the walks are one launch and a merge follows (attn_parts_kernel); fp16 pages that neighbouring
 // branches share go through attn_page_tile_kernel before the walk.
 // Scores and softmax are fp32 throughout (exp2 of log2(e)-scaled scores); probabilities are rounded to fp16 only as the operand of
-// the P.V matrix product of a shared prefix and of a prefill (walks and shared pages hold all their bits).
+// the P.V matrix product of a shared prefix and of a prefill (walks and shared pages hold all their bits, attn_tile_kernel's prefix 22).
 //
 // Algorithmic HBM traffic: prefix 2*P*Hkv*D*2 B once + per branch its suffix rows
 // (512 B fp16 or 136 B Q4_0 per row and kv head) + q/out.
@@ -1449,6 +1449,451 @@ __global__ __launch_bounds__(256, 2) void attn_one_kernel(AttnParams p) {
     }
 }
 
+// ---- a step's attention in one launch, 16 queries of a kv head a workgroup ------------------------------------------
+// Wave w of eight has queries 2 w and 2 w + 1 of the tile, one in either half of its lanes: it adds up their q, k and v from the slabs of
+// wq|wk|wv, rotates, appends k and v, and walks the two branches' own rows.  In between all waves multiply the prefix for all 16 queries, 32 rows
+// at a time (a wave takes every eighth such chunk), with K and V in registers as they come from memory; the waves' partials meet in LDS, so nothing
+// but the output leaves the workgroup, and it waits for no other.
+//   S^T = K . Q^T: element r of tile i is prefix row 16 i + 4 g + r of query c.  O^T = V^T . P^T in eight products: lane (c, g) holds dims
+//   8 c .. + 7 of the eight rows whose probabilities it has, product e takes dims 8 c + e (a transpose of pairs of halves in registers), and
+//   lane (c, g) ends with dims 32 g .. 32 g + 31 of query c.
+// Workgroups of a kv head sit on one XCD (blockIdx.x), which then reads its prefix once, and neighbouring heads on the same one, which share
+// the lines of the scales (heads dealt to two or four XCDs: 1 and 6 % slower).
+// In place of the RoPE launch, the prefix slices and the walks (7B, 100 branches after 512 rows, 5 / 60 / 120 rows of their own: 26.0 / 34.1 /
+// 42.8 us -> 13.7 / 24.2 / 35; 37 branches, 221 and 40 rows, 20.5 -> 14.0; 64 heads over 8, 50 branches after 2047 rows 40 -> 25; a step of 100
+// branches 3.90 -> 3.58 ms, of 37 2.92 -> 2.77).  Which of them a layer takes: attn_way in model_layer.hip.
+// Bound by the vector ALU: ~2000 instructions a wave and 110 a pass of four rows for two queries, at 4.4 cycles, two waves a SIMD; and, before
+// that, by the compute unit's address unit and the latency of HBM (256 KB of K and V a workgroup: 5.5 us alone).
+// (16 waves of one query each spill their registers: 20 us, where eight took 17.)
+constexpr int AT_WAVES = 8, AT_CHUNK = 32;
+constexpr int AT_PITCH = ATT_D + 4;                        // floats of a partial: o[128], maximum, sum
+constexpr int AT_MINE = 16 * AT_PITCH;                     // floats of LDS of a wave: its partials, before that a chunk of K
+constexpr int AT_QPITCH = ATT_D + 8;
+constexpr int AT_LDS = AT_WAVES * AT_MINE * 4 + 3 * 16 * AT_QPITCH * 2;
+static_assert(AT_MINE * 4 >= AT_CHUNK * 256 && AT_LDS <= 160 * 1024, "K fits");
+__device__ __forceinline__ uint32_t row16_max_bits(uint32_t v) {
+    auto step = [&](auto ctrl) { v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, 0xf, 0xf, false)); };
+    step(std::integral_constant<int, DPP_QUAD_XOR1>());
+    step(std::integral_constant<int, DPP_QUAD_XOR2>());
+    step(std::integral_constant<int, DPP_ROW_HALF_MIRROR>());
+    step(std::integral_constant<int, DPP_ROW_ROR8>());
+    return v;
+}
+// Half a row of 32 lanes: lane hl holds dims 4 hl .. + 3, its partner of the rotation is lane hl ^ 16 (roundings of rope_pair2)
+__device__ __forceinline__ h4 rope_lanes(h4 x, h4 cs, h4 sn, bool lower) {
+#pragma clang fp contract(off)
+    const u32x2 mine = __builtin_bit_cast(u32x2, x);
+    const h4 other = __builtin_bit_cast(h4, u32x2{(uint32_t)__shfl_xor((int)mine[0], 16, 64), (uint32_t)__shfl_xor((int)mine[1], 16, 64)});
+    const h4 a = x * cs, b = (lower ? -other : other) * sn;
+    return a + b;
+}
+// kv_store_row2 in that layout; `store`: the half's row is one to be written.  Both quotients are those of its divisions: a reciprocal and one
+// correction by the remainder miss the correctly rounded quotient only where the exact one lies within 2^-46 of the middle between two
+// floats, and with 11 bits in numerator and denominator it is either that middle's neighbour by 2^-36 or a float itself.  Scales that are zero,
+// subnormal or not finite are left to the divisions.
+__device__ __forceinline__ float corrected_quotient(float a, float b, float rcp) {
+    const float q = a * rcp;
+    return __builtin_fmaf(__builtin_fmaf(-q, b, a), rcp, q);
+}
+__device__ __forceinline__ void kv_store_lanes(h4 x, uint8_t *row, half_t *scales, int hl, bool store) {
+    const u32x2 bits = __builtin_bit_cast(u32x2, x) & 0x7fff7fffu;
+    uint32_t big = max(max(bits[0] & 0xffffu, bits[0] >> 16), max(bits[1] & 0xffffu, bits[1] >> 16));
+    big = row16_max_bits(big);
+    const float top = (float)__builtin_bit_cast(half_t, (uint16_t)big);
+    half_t s = (half_t)corrected_quotient(top, 7.0f, 1.0f / 7.0f);
+    uint32_t codes = 0;
+    const uint32_t exponent = __builtin_bit_cast(uint16_t, s) & 0x7c00u;
+    if (__any(exponent == 0 || exponent == 0x7c00u)) {
+        s = (half_t)(top / 7.0f);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) codes |= (uint32_t)(kv_code2(x[j], (float)s) & 15) << (8 * j);
+    } else {
+        const float rcp = __builtin_amdgcn_rcpf((float)s);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const half_t q = __builtin_rintf16((half_t)corrected_quotient((float)x[j], (float)s, rcp));
+            codes |= ((uint32_t)(int)(short)q & 15u) << (8 * j);
+        }
+    }
+    const uint32_t upper = (uint32_t)__shfl_xor((int)codes, 16, 64);
+    if (store && hl < 16) reinterpret_cast<uint32_t *>(row)[hl] = codes << 4 | upper;
+    if (store && (hl & 15) == 0) scales[hl >> 4] = s;
+}
+
+// QKS: most slabs of the q|k|v product, LEAST: the fewest.  QT: queries of a workgroup, 16 or 8 (then a wave's halves share one query and take
+// its rows 16 at a time in turn).  Grid: (XCD, kv head of it, tile).
+template <bool PAGES, int LEAST, int QKS, int QT>
+__global__ __launch_bounds__(64 * AT_WAVES) void attn_tile_kernel(AttnParams p, int chunks) {
+    extern __shared__ __attribute__((aligned(16))) float at_lds[];
+    half_t *const s_q = reinterpret_cast<half_t *>(at_lds + AT_WAVES * AT_MINE), *const s_k = s_q + 16 * AT_QPITCH, *const s_v = s_k + 16 * AT_QPITCH;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int hk = blockIdx.x * gridDim.y + blockIdx.y, tile = blockIdx.z;
+    if (hk >= p.Hkv) return;
+    const int c = lane & 15, g = lane >> 4;                  // of the matrix products
+    const int hl = lane & 31, half = lane >> 5, qi = QT == 16 ? 2 * wave + half : wave;      // this half's lane and query
+    const int e = lane & 7, rs = (lane >> 3) & 3;            // of the walk: eight lanes a row, dims 8 e .. and 64 + 8 e ..; four rows a half
+    const int qrow = QT * tile + qi, qc = min(qrow, p.Bq - 1);
+    const int b = div_rep(p, qc), rep = mod_rep(p, qc), h = hk * p.n_rep + rep;
+    const bool live = qrow < p.Bq && (QT == 16 || half == 0);
+    auto meet = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+
+    // ---- requests: slabs, rotation factors, page ids, prefix ----
+    const int pos = *p.pos_dev, t = *p.app_t, len = min(max(t, 0), (int)p.suffix_batch_stride_rows);
+    const int cols = (p.H + 2 * p.Hkv) * ATT_D;
+    const long slab = (long)p.B * cols;
+    const float *src = p.qkv + (long)b * cols + 4 * hl;
+    // (QT == 8: k in the lower half of the lanes, v in the upper one)
+    f4 qv[QKS], kv[QKS], vv[QT == 16 ? QKS : 1];
+    auto slabs = [&](int col, f4 (&v)[QKS]) {
+#pragma unroll
+        for (int s = 0; s < QKS; ++s) v[s] = *reinterpret_cast<const f4 *>(src + (col + (s < LEAST ? s : min(s, p.qkv_ks - 1)) * slab));
+    };
+    slabs(h * ATT_D, qv);
+    slabs((p.H + hk + (QT == 8 && half == 1 ? p.Hkv : 0)) * ATT_D, kv);
+    if constexpr (QT == 16) slabs((p.H + p.Hkv + hk) * ATT_D, vv);
+    const h4 cs = *reinterpret_cast<const h4 *>(p.cos_tab + (long)pos * 64 + 4 * (hl & 15));
+    const h4 sn = *reinterpret_cast<const h4 *>(p.sin_tab + (long)pos * 64 + 4 * (hl & 15));
+    // a wave's turns of its walk: QT == 16: 16 rows of either half's query, 8: 32 of the one, 16 a half.  Four passes of four rows a half.
+    constexpr int TURN = QT == 16 ? 16 : 32;
+    const int turns = (len + TURN - 1) / TURN;
+    auto row_at = [&](int s, int u) { return QT == 16 ? 16 * s + 4 * u + rs : 32 * s + 16 * half + 4 * u + rs; };
+    const int32_t *ids = reinterpret_cast<const int32_t *>(p.pages) + (long)b * p.pages_stride;
+    auto ids_of = [&](int blk) { return ids[min(32 * blk + hl, len - 1)]; };           // of 32 positions, one a lane
+    int id_now = 0, id_next = 0;
+    if (PAGES && len > 0) {
+        id_now = ids_of(0);
+        if (len > 32) id_next = ids_of(1);
+    }
+
+    // This wave's chunks are kind, kind + 8, ..: the waves of different tiles begin at different ones (where they begin at the same, all wait for the
+    // same lines to come from HBM: 16.1 us instead of 14.3 at 100 branches after 512 rows), and every tile does the same sums in the same order.
+    const int kind = (wave + (int)(__brev((uint32_t)tile) >> 29)) & (AT_WAVES - 1);
+    char *const s_mine = reinterpret_cast<char *>(at_lds + kind * AT_MINE);
+    const uint32_t pfx_row = (uint32_t)p.pfx_row_stride * 2;
+    const char *kb = reinterpret_cast<const char *>(p.prefix_k + (long)hk * p.pfx_head_stride), *vb = reinterpret_cast<const char *>(p.prefix_v + (long)hk * p.pfx_head_stride);
+    const uint32_t k_off = g * pfx_row + 16 * c, v_off = 4 * g * pfx_row + 16 * c;
+    // whole rows a load (one whose neighbouring lanes are in different rows takes 64 cycles, not 16): K's row 4 i + g, V's 4 g + i, from 16 on for i >= 4
+    struct Chunk { u32x4 k[8], v[8]; };
+    auto fetch = [&](int j, Chunk &ck) {
+        if (AT_CHUNK * (j + 1) <= p.P) {
+            const long at = (long)(AT_CHUNK * j) * pfx_row;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) ck.k[i] = *reinterpret_cast<const u32x4 *>(kb + at + (long)(4 * i) * pfx_row + k_off);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) ck.v[i] = *reinterpret_cast<const u32x4 *>(vb + at + (long)(i < 4 ? i : 12 + i) * pfx_row + v_off);
+        } else {                                             // past the end: the last row again, which weighs nothing
+#pragma unroll
+            for (int i = 0; i < 8; ++i) ck.k[i] = *reinterpret_cast<const u32x4 *>(kb + ((uint32_t)min(AT_CHUNK * j + 4 * i + g, p.P - 1) * pfx_row + 16 * c));
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                ck.v[i] = *reinterpret_cast<const u32x4 *>(vb + ((uint32_t)min(AT_CHUNK * j + (i < 4 ? i : 12 + i) + 4 * g, p.P - 1) * pfx_row + 16 * c));
+        }
+    };
+    Chunk ck[2];
+    __builtin_amdgcn_sched_barrier(0);                       // (loads are waited for in their order: what the query needs comes first)
+    if (QKS <= 6 && kind < chunks) fetch(kind, ck[0]);
+
+    // ---- this branch's rows: a turn's four a request.  Half the lanes of a row have its K scales, half its V scales ----
+    struct Rows { u32x2 k[4], v[4]; uint32_t sc[4]; };
+    const char *sc_base = reinterpret_cast<const char *>(e < 4 ? p.suffix_ks : p.suffix_vs);
+    auto row_of = [&](int id) { return (uint32_t)min(max(id, 0), (int)p.pool_rows - 1) * (uint32_t)p.Hkv + hk; };
+    uint32_t row_now = PAGES ? 0u : (uint32_t)(b * (int)p.suffix_batch_stride_rows) * (uint32_t)p.Hkv + hk;
+    auto rows = [&](int s, Rows &r) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            // (past the end: the last row again)
+            const uint32_t row = PAGES ? (uint32_t)__shfl((int)row_now, (lane & 32) | (row_at(s, u) & 31), 64)
+                                       : row_now + (uint32_t)min(row_at(s, u), len - 1) * (uint32_t)p.Hkv;
+            r.k[u] = *reinterpret_cast<const u32x2 *>((const char *)p.suffix_k + (row * 64 + 8 * e));
+            r.v[u] = *reinterpret_cast<const u32x2 *>((const char *)p.suffix_v + (row * 64 + 8 * e));
+            r.sc[u] = *reinterpret_cast<const uint32_t *>(sc_base + (unsigned long)row * 4);
+        }
+    };
+    Rows cur;
+
+    // ---- q, k, v ----
+    {
+        auto total = [&](const f4 (&v)[QKS]) {
+            f4 tot = v[0];
+#pragma unroll
+            for (int s = 1; s < QKS; ++s) {
+                const f4 next = tot + v[s];
+                tot = s < LEAST || s < p.qkv_ks ? next : tot;
+            }
+            return h4{(half_t)tot[0], (half_t)tot[1], (half_t)tot[2], (half_t)tot[3]};
+        };
+        const bool lower = hl < 16;
+        const h4 q = rope_lanes(total(qv), cs, sn, lower), raw = total(kv), k = rope_lanes(raw, cs, sn, lower);
+        h4 v = raw;
+        if constexpr (QT == 16) v = total(vv);
+        *reinterpret_cast<h4 *>(s_q + qi * AT_QPITCH + 4 * hl) = q;
+        if constexpr (QT == 16) {
+            *reinterpret_cast<h4 *>(s_k + qi * AT_QPITCH + 4 * hl) = k;
+            *reinterpret_cast<h4 *>(s_v + qi * AT_QPITCH + 4 * hl) = v;
+        } else {
+            *reinterpret_cast<h4 *>((half == 0 ? s_k : s_v) + qi * AT_QPITCH + 4 * hl) = half == 0 ? k : v;
+        }
+        if (len > 0) {
+            if (PAGES) row_now = row_of(id_now);
+            rows(0, cur);
+        }
+        if (QKS > 6 && kind < chunks) fetch(kind, ck[0]);
+        meet();                                              // every query is in LDS
+        if (kind + AT_WAVES < chunks) fetch(kind + AT_WAVES, ck[1]);
+        if (t >= 0 && t < p.app_smax) {                      // (uniform) the first query head of a kv head appends the rows
+            const long row = ((long)b * p.app_smax + t) * p.Hkv + hk;
+            const bool store = qrow < p.Bq && rep == 0;
+            if constexpr (QT == 16) {
+                kv_store_lanes(k, p.app_k + row * 64, p.app_ks + row * 2, hl, store);
+                kv_store_lanes(v, p.app_v + row * 64, p.app_vs + row * 2, hl, store);
+            } else {
+                kv_store_lanes(half == 0 ? k : v, (half == 0 ? p.app_k : p.app_v) + row * 64, (half == 0 ? p.app_ks : p.app_vs) + row * 2, hl, store);
+            }
+        }
+    }
+
+    // ---- the prefix, two chunks at a time ----
+    if (kind < chunks) {
+        f4 o[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o[i] = f4{0.f, 0.f, 0.f, 0.f};
+        float m = -INFINITY, l = 0.f;                        // m: of query c, in all its lanes; l: over this lane's rows
+        auto scores = [&](int j, Chunk &ch, f4 *st) {
+            // K to the operand's layout through this wave's part of LDS: piece k of row r lies at k ^ (r % 16)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) *reinterpret_cast<u32x4 *>(s_mine + (4 * i + g) * 256 + 16 * (c ^ ((4 * i + g) & 15))) = ch.k[i];
+#pragma unroll
+            for (int k4 = 0; k4 < 4; ++k4) {
+                const h8 qb = *reinterpret_cast<const h8 *>(s_q + (c & (QT - 1)) * AT_QPITCH + 32 * k4 + 8 * g);
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    st[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const h8 *>(s_mine + (16 * i + c) * 256 + 16 * ((4 * k4 + g) ^ c)), qb, st[i], 0, 0, 0);
+            }
+            if (AT_CHUNK * (j + 1) > p.P) {                  // (uniform) the last chunk
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    if (AT_CHUNK * j + (i < 4 ? i : 12 + i) + 4 * g >= p.P) {
+                        st[i >> 2][i & 3] = -INFINITY;
+                        ch.v[i] = u32x4{0, 0, 0, 0};
+                    }
+            }
+        };
+        // Probabilities are 2^15 times themselves (the partial's maximum says so) and enter the product as two fp16 terms, 22 bits of them
+        struct Terms { h8 p, left; };
+        auto products = [&](const Chunk &ch, const Terms &pb) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                u32x4 va;
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    va[k] = (i & 1) == 0 ? pack_lo16(ch.v[2 * k][i >> 1], ch.v[2 * k + 1][i >> 1]) : pack_hi16(ch.v[2 * k][i >> 1], ch.v[2 * k + 1][i >> 1]);
+                o[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, va), pb.p, o[i], 0, 0, 0);
+                o[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, va), pb.left, o[i], 0, 0, 0);
+            }
+        };
+        for (int j = kind; j < chunks; j += 2 * AT_WAVES) {
+            const bool two = j + AT_WAVES < chunks;          // (uniform)
+            f4 st[4] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
+            scores(j, ck[0], st);
+            if (two) scores(j + AT_WAVES, ck[1], st + 2);
+            float mx = fmaxf(fmaxf(fmaxf(st[0][0], st[0][1]), fmaxf(st[0][2], st[0][3])), fmaxf(fmaxf(st[1][0], st[1][1]), fmaxf(st[1][2], st[1][3])));
+            if (two) mx = fmaxf(mx, fmaxf(fmaxf(fmaxf(st[2][0], st[2][1]), fmaxf(st[2][2], st[2][3])), fmaxf(fmaxf(st[3][0], st[3][1]), fmaxf(st[3][2], st[3][3]))));
+            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+            mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * p.scale_log2;
+            if (j != kind) {                                 // (uniform)
+                const float m_new = fmaxf(m, mx), corr = __builtin_amdgcn_exp2f(m - (m_new == -INFINITY ? 0.f : m_new));
+                l *= corr;
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) o[i][r] *= corr;
+                mx = m_new;
+            }
+            m = mx;
+            const float m_ref = (m == -INFINITY ? 0.f : m) - 15.f;
+            auto probabilities = [&](const f4 *s4) {
+                Terms pb;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const float pr = __builtin_amdgcn_exp2f(__builtin_fmaf(s4[i >> 2][i & 3], p.scale_log2, -m_ref));
+                    l += pr;
+                    pb.p[i] = (half_t)pr;
+                    pb.left[i] = (half_t)(pr - (float)pb.p[i]);
+                }
+                return pb;
+            };
+            products(ck[0], probabilities(st));
+            if (two) products(ck[1], probabilities(st + 2));
+            if (j + 2 * AT_WAVES < chunks) fetch(j + 2 * AT_WAVES, ck[0]);
+            if (j + 3 * AT_WAVES < chunks) fetch(j + 3 * AT_WAVES, ck[1]);
+        }
+        l += __shfl_xor(l, 16, 64);
+        l += __shfl_xor(l, 32, 64);
+        float *po = reinterpret_cast<float *>(s_mine) + c * AT_PITCH;
+        if (c < QT) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) *reinterpret_cast<f4 *>(po + 32 * g + 8 * r + 4 * i) = f4{o[4 * i][r], o[4 * i + 1][r], o[4 * i + 2][r], o[4 * i + 3][r]};
+            if (g == 0) *reinterpret_cast<f2 *>(po + ATT_D) = f2{m - 15.f, l};
+        }
+    }
+
+    // ---- the branch's own rows: m, l of this lane's row slot, o of its dims: as RowRegs orders them, first 8 e .., 64 + 8 e .., then 8 e + 4 .., 68 + 8 e .. ----
+    RowRegs q[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) q[j] = row_from_fp16(s_q + qi * AT_QPITCH, 2 * e + j);
+    float m, l, o[2][8];
+    auto score = [&](const RowRegs &k0, const RowRegs &k1) {
+        float d = 0.f;
+        const RowRegs *kr[2] = {&k0, &k1};
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            d = __builtin_amdgcn_fdot2(kr[j]->a02, q[j].a02, d, false);
+            d = __builtin_amdgcn_fdot2(kr[j]->a13, q[j].a13, d, false);
+            d = __builtin_amdgcn_fdot2(kr[j]->b02, q[j].b02, d, false);
+            d = __builtin_amdgcn_fdot2(kr[j]->b13, q[j].b13, d, false);
+        }
+        d += dpp_move<DPP_QUAD_XOR1>(d);
+        d += dpp_move<DPP_QUAD_XOR2>(d);
+        d += dpp_move<DPP_ROW_HALF_MIRROR>(d);
+        return d * p.scale_log2;
+    };
+    auto add = [&](float pr, int j, const RowRegs &v) {
+        o[j][0] += pr * (float)v.a02.x; o[j][1] += pr * (float)v.a02.y;
+        o[j][2] += pr * (float)v.a13.x; o[j][3] += pr * (float)v.a13.y;
+        o[j][4] += pr * (float)v.b02.x; o[j][5] += pr * (float)v.b02.y;
+        o[j][6] += pr * (float)v.b13.x; o[j][7] += pr * (float)v.b13.y;
+    };
+    // the state relative to another maximum; returned: what to subtract from scores
+    auto raise = [&](float m_new) {
+        const float m_ref = m_new == -INFINITY ? 0.f : m_new, corr = __builtin_amdgcn_exp2f(m - m_ref);
+        m = m_new;
+        l *= corr;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int k = 0; k < 8; ++k) o[j][k] *= corr;
+        return m_ref;
+    };
+    {
+        // the new token's exact row begins slot 0 (in the others an infinite value would weigh 0, and 0 times it is NaN)
+        const bool mine = rs == 0 && (QT == 16 || half == 0);
+        const float sc = score(row_from_fp16(s_k + qi * AT_QPITCH, 2 * e), row_from_fp16(s_k + qi * AT_QPITCH, 2 * e + 1));
+        m = mine ? fmaxf(sc, -INFINITY) : -INFINITY;
+        const float pr = __builtin_amdgcn_exp2f(sc - (m == -INFINITY ? 0.f : m));
+        l = 0.f;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int k = 0; k < 8; ++k) o[j][k] = 0.f;
+        if (mine) {
+            l = pr;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) add(pr, j, row_from_fp16(s_v + qi * AT_QPITCH, 2 * e + j));
+        }
+    }
+    // N passes from u0 on: one maximum, one rescale.  ends: some may lie past the last row
+    auto passes = [&](int s, auto N, int u0, bool ends) {
+        float sc[N];
+        uint32_t vs[N];
+        float mx = m;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const uint32_t mine = cur.sc[u0 + i], other = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mine, DPP_ROW_HALF_MIRROR, 0xf, 0xf, false);
+            const uint32_t ks = e < 4 ? mine : other;
+            vs[i] = e < 4 ? other : mine;
+            sc[i] = score(row_from_q40(cur.k[u0 + i][0], ks), row_from_q40(cur.k[u0 + i][1], ks));
+            if (ends && row_at(s, u0 + i) >= len) sc[i] = -INFINITY;
+            mx = fmaxf(mx, sc[i]);
+        }
+        const float m_ref = raise(mx);
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const float pr = __builtin_amdgcn_exp2f(sc[i] - m_ref);
+            l += pr;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) add(pr, j, row_from_q40(cur.v[u0 + i][j], vs[i]));
+        }
+    };
+    for (int s = 0; s < turns; ++s) {
+        Rows nxt;
+        if (s + 1 < turns) {
+            const int blk = TURN * (s + 1) / 32;
+            if (PAGES && TURN * (s + 1) % 32 == 0) {
+                row_now = row_of(id_next);
+                if (32 * (blk + 1) < len) id_next = ids_of(blk + 1);
+            }
+            rows(s + 1, nxt);
+        }
+        if (TURN * (s + 1) <= len) {                         // (uniform)
+            passes(s, std::integral_constant<int, 4>(), 0, false);
+        } else {
+            passes(s, std::integral_constant<int, 2>(), 0, true);
+            if (QT == 8 || TURN * s + 8 < len) passes(s, std::integral_constant<int, 2>(), 2, true);
+        }
+        cur = nxt;
+    }
+    meet();                                                  // the prefix's partials are in LDS
+    {
+        constexpr int N = AT_WAVES / 4 * QT / 16;            // of this slot
+        f4 part[N][2][2];
+        f2 ml[N];
+        float mx = m;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int sp = QT == 16 ? rs + 4 * i : 4 * half + rs;
+            ml[i] = f2{-INFINITY, 0.f};
+#pragma unroll
+            for (int j = 0; j < 2; ++j) part[i][j][0] = part[i][j][1] = f4{0.f, 0.f, 0.f, 0.f};
+            if (sp < chunks) {
+                const float *po = at_lds + sp * AT_MINE + qi * AT_PITCH;
+                ml[i] = *reinterpret_cast<const f2 *>(po + ATT_D);
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    part[i][j][0] = *reinterpret_cast<const f4 *>(po + 8 * e + 4 * j);
+                    part[i][j][1] = *reinterpret_cast<const f4 *>(po + 64 + 8 * e + 4 * j);
+                }
+            }
+            mx = fmaxf(mx, ml[i][0]);
+        }
+        // ... and the maximum of the slots of the query
+        mx = fmaxf(mx, dpp_move<DPP_ROW_ROR8>(mx));
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        if (QT == 8) mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const float m_ref = raise(mx);
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const float f = __builtin_amdgcn_exp2f(ml[i][0] - m_ref);
+            l += f * ml[i][1];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {                // (RowRegs order: dims 0, 2, 1, 3)
+                    o[j][k] += f * part[i][j][0][(k & 1) * 2 + (k >> 1)];
+                    o[j][4 + k] += f * part[i][j][1][(k & 1) * 2 + (k >> 1)];
+                }
+        }
+    }
+    // ---- the slots added up: slot (second, first bit) ends with dims 64 second + 8 e + 4 first .. + 3 ----
+    l += dpp_move<DPP_ROW_ROR8>(l);
+    l += __shfl_xor(l, 16, 64);
+    if (QT == 8) l += __shfl_xor(l, 32, 64);
+    const int first = rs & 1, second = rs >> 1;
+    float w[8], y[4];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) w[k] = (first ? o[1][k] : o[0][k]) + dpp_move<DPP_ROW_ROR8>(first ? o[0][k] : o[1][k]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        y[k] = (second ? w[4 + k] : w[k]) + __shfl_xor(second ? w[k] : w[4 + k], 16, 64);
+        if (QT == 8) y[k] += __shfl_xor(y[k], 32, 64);
+    }
+    if (!live) return;
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    *reinterpret_cast<h4 *>(p.out + ((long)b * p.H + h) * ATT_D + 64 * second + 8 * e + 4 * first) =
+        h4{(half_t)(y[0] * inv), (half_t)(y[2] * inv), (half_t)(y[1] * inv), (half_t)(y[3] * inv)};
+}
+
 static int attn_plan_tw(int P, int Hkv) {
     // rows of the prefix per workgroup: as large as fits while still giving the 256 CUs work
     int tw = ATT_TW_MAX;
@@ -1818,6 +2263,65 @@ extern "C" int smh_shared_prefix_attn_qkv(const void *qkv_partial, int ksplit, v
         hipLaunchKernelGGL(attn_prefix_kernel<true>, dim3(p.splits, Hkv, qgroups), dim3(256), 0, (hipStream_t)stream, p);
     p.suffix_waves = attn_plan_suffix_waves_two((long)B * H);
     hipLaunchKernelGGL((pages != nullptr ? attn_suffix_kernel<true, WALK_Q40, 4> : attn_suffix_kernel<true, WALK_Q40, 0>), dim3((unsigned)(((H * p.suffix_waves + 3) / 4) * ((B + 7) / 8 * 8))), dim3(256), 0, (hipStream_t)stream, p);
+    return launch_status();
+}
+
+extern "C" int smh_shared_prefix_attn_qkv_tiles(const void *qkv_partial, int ksplit, void *out, int B, int H, int Hkv, int D,
+                                                const void *cos_tab, const void *sin_tab, const int32_t *pos_dev,
+                                                const void *prefix_k, const void *prefix_v, int P,
+                                                void *cache_k, void *cache_ks, void *cache_v, void *cache_vs, int Smax,
+                                                const int32_t *t_dev, const int32_t *pages, int pages_stride, long cache_rows, smh_stream_t stream) {
+    using namespace smh;
+    const char *who = "smh_shared_prefix_attn_qkv_tiles";
+    SMH_REQUIRE(D == ATT_D, "%s: head dim %d (only 128)", who, D);
+    SMH_REQUIRE(B >= 0 && B <= 65535 && H > 0 && Hkv > 0 && H % Hkv == 0 && P >= 0, "%s: B=%d (at most 65535) H=%d Hkv=%d P=%d", who, B, H, Hkv, P);
+    SMH_REQUIRE(ksplit >= 1 && ksplit <= 16, "%s: ksplit=%d", who, ksplit);
+    if (B == 0) return 0;
+    SMH_REQUIRE(qkv_partial && out && cos_tab && sin_tab && pos_dev, "%s: null pointer", who);
+    SMH_REQUIRE(P == 0 || (prefix_k && prefix_v), "%s: null prefix", who);
+    SMH_REQUIRE(cache_k && cache_ks && cache_v && cache_vs && t_dev && Smax > 0, "%s: the suffix cache and its row counter are required", who);
+    SMH_REQUIRE(pages == nullptr || (pages_stride >= Smax && cache_rows >= 1), "%s: pages_stride=%d must cover the %d rows of a branch, cache_rows=%ld", who,
+                pages_stride, Smax, cache_rows);
+    AttnParams p{};
+    p.out = (half_t *)out;
+    p.prefix_k = (const half_t *)prefix_k; p.prefix_v = (const half_t *)prefix_v;
+    p.suffix_k = cache_k; p.suffix_v = cache_v;
+    p.suffix_ks = (const half_t *)cache_ks; p.suffix_vs = (const half_t *)cache_vs;
+    p.lens = t_dev; p.lens_stride = 0;
+    p.suffix_batch_stride_rows = Smax;
+    p.pages = pages; p.pages_stride = pages_stride; p.page_bytes = 4; p.pool_rows = cache_rows;
+    p.pfx_row_stride = (long)Hkv * ATT_D; p.pfx_head_stride = ATT_D;
+    p.sfx_row_stride = (long)Hkv * ATT_D; p.sfx_head_stride = ATT_D;
+    p.B = B; p.H = H; p.Hkv = Hkv; p.n_rep = H / Hkv; p.Bq = B * p.n_rep;
+    p.P = P; p.suffix_format = SMH_KV_Q40;
+    p.scale_log2 = LOG2E / sqrtf((float)D);
+    p.qkv = (const float *)qkv_partial; p.qkv_ks = ksplit;
+    p.cos_tab = (const half_t *)cos_tab; p.sin_tab = (const half_t *)sin_tab; p.pos_dev = pos_dev;
+    p.app_k = (uint8_t *)cache_k; p.app_v = (uint8_t *)cache_v;
+    p.app_ks = (half_t *)cache_ks; p.app_vs = (half_t *)cache_vs;
+    p.app_t = t_dev; p.app_smax = Smax;
+    typedef void (*kernel_t)(AttnParams, int);
+    static const kernel_t kern[2][2][3] = {{{attn_tile_kernel<false, 1, 2, 8>, attn_tile_kernel<false, 3, 6, 8>, attn_tile_kernel<false, 7, 16, 8>},
+                                            {attn_tile_kernel<true, 1, 2, 8>, attn_tile_kernel<true, 3, 6, 8>, attn_tile_kernel<true, 7, 16, 8>}},
+                                           {{attn_tile_kernel<false, 1, 2, 16>, attn_tile_kernel<false, 3, 6, 16>, attn_tile_kernel<false, 7, 16, 16>},
+                                            {attn_tile_kernel<true, 1, 2, 16>, attn_tile_kernel<true, 3, 6, 16>, attn_tile_kernel<true, 7, 16, 16>}}};
+    static const hipError_t lds_ok = [] {
+        hipError_t e = hipSuccess;
+        for (int i = 0; i < 12 && e == hipSuccess; ++i)
+            e = hipFuncSetAttribute((const void *)kern[i / 6][i / 3 % 2][i % 3], hipFuncAttributeMaxDynamicSharedMemorySize, AT_LDS);
+        return e;
+    }();
+    if (lds_ok != hipSuccess) { set_error("%s: the kernel's LDS could not be reserved: %s", who, hipGetErrorString(lds_ok)); return (int)lds_ok; }
+    SMH_REQUIRE((long)P * Hkv * ATT_D * 2 < (1L << 32), "%s: P=%d rows of %d heads exceed the 32-bit offsets of the prefix", who, P, Hkv);
+    const long rows = pages != nullptr ? cache_rows : (long)B * Smax;
+    SMH_REQUIRE(rows * Hkv * 64 < (1L << 32) && rows < (1L << 31), "%s: %ld cache rows of %d heads exceed the 32-bit offsets of the cache", who, rows, Hkv);
+    // Eight queries a workgroup while those fill one round of compute units, else 16 (us, 16 and 8: 32 heads, 64 branches after 512 rows 24.4 and
+    // 19.4, 17 20.5 and 14.2, 100, two rounds of eight, 24.1 and 30.6; 64 heads over 8, 30 branches after 2047 rows 26.3 and 23.7, 100 48.8 and 76.3)
+    const int qt = (long)Hkv * ((p.Bq + 7) / 8) <= 256 ? 8 : 16, tiles = (p.Bq + qt - 1) / qt;
+    SMH_REQUIRE(tiles <= 65535 && Hkv <= 8 * 65535, "%s: %d tiles of queries, %d heads", who, tiles, Hkv);
+    const int chunks = (P + AT_CHUNK - 1) / AT_CHUNK;
+    hipLaunchKernelGGL(kern[qt == 16][pages != nullptr][ksplit <= 2 ? 0 : ksplit <= 6 ? 1 : 2], dim3(8, (Hkv + 7) / 8, tiles), dim3(64 * AT_WAVES), AT_LDS,
+                       (hipStream_t)stream, p, chunks);
     return launch_status();
 }
 

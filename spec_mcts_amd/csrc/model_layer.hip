@@ -5,6 +5,8 @@
 // 32-layer model took 3.0 ms where a captured graph of the same launches takes 2.0.  Here the layer's launches are issued one
 // behind the other (2-3 us each), out of buffers the caller allocated once for the whole pass.  The sequence, the operators
 // and their switches are those of Transformer._forward_fused in hf_model_q40_kv_shared.py.
+#include <initializer_list>
+
 #include "smh_common.hpp"
 
 namespace smh {
@@ -22,6 +24,37 @@ static int slices(int M, int K, int nseg, const int *n) { return smh_q40_matmul_
 // A launch that stores its fp16 results itself (more than 128 rows, no K-split) leaves no slabs.  layer_buffers reserves none for it,
 // so every linear below asks here before it takes the slab form.
 static bool direct(int M, int K, int nseg, const int *n) { return smh_q40_matmul_tiled_direct_fits(M, K, nseg, n) == 1; }
+
+// The attention of a decode layer: in one launch whose last workgroups merge (ONE, up to 16 queries a kv head), in one launch of 8 or 16
+// queries a workgroup (TILES), or RoPE, prefix slices and walks (LAUNCHES).  us a call with RoPE and append, caches in HBM:
+//   32 heads, branches after prompt rows   ONE   TILES LAUNCHES  |  64 heads over 8                ONE   TILES LAUNCHES
+//     5 /  512                             12.8   14.9   15.1    |     1 /  512 (8 queries)        12.2   13.7   13.6
+//    16 /  256                             16.7   14.1   15.9    |     1 / 2047                    17.0   22.6   16.6
+//    10 /  768                             19.9   20.2   19.3    |     2 /  128 (16 queries)       10.7   11.2   12.7
+//    10 / 1024                             24.9   23.3   20.5    |     2 /  512                    15.6   13.7   14.1
+//    10 / 2047                             38.9   33.8   24.5    |     2 / 2047                    24.2   22.4   17.9
+//    17 /  512                               -    16.9   18.9    |     3 /  512                      -    11.8   14.9
+//    17 / 1024                               -    21.5   21.8    |     3 / 1024                      -    18.6   17.5
+//    17 / 2047                               -    29.3   26.0    |    10 / 1024                      -    18.0   21.4
+//    32 / 2047                               -    29.3   28.5    |    10 / 2047                      -    25.2   23.4
+//    48 / 2047                               -    31.5   32.0    |    16 / 2047                      -    24.4   26.3
+//   100 / 2047                               -    34.7   47.7    |   100 / 2047                      -    48.8   65.6
+//                                                                |  40 heads, 100 / 512 (two rounds) -   39.5   39.0
+// A long prompt wants more workgroups than few tiles are, and ONE's merge grows with the slices.  Behind fewer than 96 prompt rows results stay
+// where they are: there two evaluations that differ in one rounding drift 3e-2 (40 rows) to 6e-2 (16 rows) apart within eight steps of the 7B
+// architecture, 1.5e-2 behind 96.
+enum AttnWay { ATTN_ONE, ATTN_TILES, ATTN_LAUNCHES };
+constexpr int ATTN_TILES_MIN_PROMPT = 96;
+static AttnWay attn_way(int M, int heads, int kv_heads, int P, bool one, bool tiles, bool launches) {
+    const int rep = heads / kv_heads;
+    const long queries = (long)M * rep;                      // of a kv head
+    if (one && (rep == 1 ? P <= 768 : queries <= 8 || P <= 256)) return ATTN_ONE;
+    const bool round = (kv_heads + 7) / 8 * 8 * ((queries + 15) / 16) <= 256;
+    if (tiles && P >= ATTN_TILES_MIN_PROMPT && (rep > 1 || (M > SMH_GEMV_MAX_M && round)) &&
+        (P <= 512 || P <= kv_heads * ((queries + 7) / 8) * (rep == 1 ? 12 : 24)))
+        return ATTN_TILES;
+    return launches ? ATTN_LAUNCHES : one ? ATTN_ONE : ATTN_TILES;
+}
 
 static int layer_buffers(const smh_layer &L, int M, bool swiglu_in, char *base, LayerBuffers &b) {
     const int nq = L.heads * 128, nkv = L.kv_heads * 128;
@@ -125,10 +158,20 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
     };
     // ---- attention ----
     const int rep = L.heads / L.kv_heads;
-    const int one = S.attn_one != 0 && M * rep <= 16;
+    const bool qkv_direct = direct(M, L.dim, 3, run.n_qkv);
+    const long rows = S.pages != nullptr ? S.cache_rows : (long)M * S.smax;
+    auto aligned = [](std::initializer_list<const void *> list, uintptr_t to) {
+        for (const void *x : list)
+            if ((uintptr_t)x % to != 0) return false;
+        return true;
+    };
+    const bool can_tile = S.attn_from_qkv != 0 && !qkv_direct && aligned({L.prompt_k, L.prompt_v}, 16) && aligned({S.cos_tab, S.sin_tab, L.cache_k, L.cache_v}, 8) &&
+                          aligned({L.cache_ks, L.cache_vs}, 4) && (long)L.prompt_len * L.kv_heads * 256 < (1L << 32) && rows * L.kv_heads * 64 < (1L << 32);
+    const AttnWay way = attn_way(M, L.heads, L.kv_heads, L.prompt_len, S.attn_one != 0 && M * rep <= 16, can_tile,
+                                 S.attn_ws != nullptr || S.attn_one == 0 || M * rep > 16);
+    const int one = way == ATTN_ONE;
     void *ws = one ? S.attn_one_ws : S.attn_ws;
     const size_t ws_bytes = one ? S.attn_one_ws_bytes : S.attn_ws_bytes;
-    const bool qkv_direct = direct(M, L.dim, 3, run.n_qkv);
     if (qkv_direct) {
         if ((st = run.norm(L.att_norm, L.att_eps))) return st;
         void *out[3] = {b.q, b.k, b.v};
@@ -145,6 +188,10 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
         st = smh_shared_prefix_attn_qkv(b.slab_a, ks_qkv, b.att, M, L.heads, L.kv_heads, 128, S.cos_tab, S.sin_tab, S.pos_dev, L.prompt_k, L.prompt_v,
                                         L.prompt_len, L.cache_k, L.cache_ks, L.cache_v, L.cache_vs, S.smax, S.t_dev, S.pages, S.pages_stride, one, ws,
                                         ws_bytes, stream);
+    } else if (way == ATTN_TILES) {
+        st = smh_shared_prefix_attn_qkv_tiles(b.slab_a, ks_qkv, b.att, M, L.heads, L.kv_heads, 128, S.cos_tab, S.sin_tab, S.pos_dev, L.prompt_k, L.prompt_v,
+                                              L.prompt_len, L.cache_k, L.cache_ks, L.cache_v, L.cache_vs, S.smax, S.t_dev, S.pages, S.pages_stride,
+                                              S.cache_rows, stream);
     } else {
         st = qkv_direct ? smh_rope_append_kv(b.q, b.k, b.v, M, L.heads, L.kv_heads, 128, S.cos_tab, S.sin_tab, S.pos_dev, L.cache_k, L.cache_ks, L.cache_v,
                                              L.cache_vs, S.smax, S.t_dev, stream)

@@ -454,16 +454,16 @@ class Transformer(nn.Module):
             structs = [first] + [self._layer_struct(layer) for layer in layers[1:]]
             stack = K.decode_stack_layers(structs, B)
         if stack is not None:
-            run.decode_step(step_state, None, True, smax, cache_rows, pages, 0, 0, True)
+            run.decode_step(step_state, None, None, smax, cache_rows, pages, 0, 0, True)
             s = structs[-1]
             run.decode_stack(stack, stack_ws)
         else:                              # (layer by layer: the GPU works while the next one's arguments are gathered)
             att0 = layers[0].attention
             H, P = att0.n_local_heads, first.prompt_len
-            one = self.attn_single_launch and B * att0.n_rep <= 16
-            ws = K.attn_qkv_workspace(dev, B, H, P) if one else K.attn_workspace(dev, B, H, P)
+            ws = K.attn_workspace(dev, B, H, P)
+            ws_one = K.attn_qkv_workspace(dev, B, H, P) if self.attn_single_launch and B * att0.n_rep <= 16 else None
             norm_in = self._norm_in(B, p.dim, [lin._tiled for lin in (att0.wq, att0.wk, att0.wv)])  # (the library asks again, launch by launch)
-            run.decode_step(step_state, ws, bool(one), smax, cache_rows, pages, B if norm_in else 0, K.SILU_IN_MAX_M if self.silu_in_matmul else 0,
+            run.decode_step(step_state, ws, ws_one, smax, cache_rows, pages, B if norm_in else 0, K.SILU_IN_MAX_M if self.silu_in_matmul else 0,
                             self.attn_from_qkv and not self.per_branch_kv)
             for i, layer in enumerate(layers):
                 s = self._layer_struct(layer) if i > 0 else s

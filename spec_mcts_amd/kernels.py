@@ -721,21 +721,19 @@ class LayerPass:
         p.scratch, p.scratch_bytes, p.h = self.scratch.data_ptr(), nbytes, h.data_ptr()
         self.stream = _stream()
 
-    def decode_step(self, step_state, ws: Optional[torch.Tensor], one_launch: bool, smax: int, cache_rows: int, pages: Optional[torch.Tensor], norm_in_rows: int,
-                    silu_in_rows: int, attn_from_qkv: bool) -> None:
-        """step_state: (position, suffix index) on the device; `ws`: the workspace of the attention (of its one-launch form with
-        `one_launch`), None where all layers are one launch; pages: int32 page table over cache_rows cache rows, or None."""
+    def decode_step(self, step_state, ws: Optional[torch.Tensor], ws_one: Optional[torch.Tensor], smax: int, cache_rows: int, pages: Optional[torch.Tensor],
+                    norm_in_rows: int, silu_in_rows: int, attn_from_qkv: bool) -> None:
+        """step_state: (position, suffix index) on the device; `ws`: the workspace of the attention, `ws_one`: of its form in one launch, None where
+        it may not be that one (both None where all layers are one launch); pages: int32 page table over cache_rows cache rows, or None."""
         p = self.p
         pos_dev, t_dev = step_state
         _need_gpu(pos_dev, t_dev)
         assert pos_dev.dtype == torch.int32 and t_dev.dtype == torch.int32
         p.pos_dev, p.t_dev = pos_dev.data_ptr(), t_dev.data_ptr()
-        self.ws = ws
-        if ws is None:
-            pass
-        elif one_launch:
-            p.attn_one, p.attn_one_ws, p.attn_one_ws_bytes = 1, ws.data_ptr(), ws.numel()
-        else:
+        self.ws, self.ws_one = ws, ws_one
+        if ws_one is not None:
+            p.attn_one, p.attn_one_ws, p.attn_one_ws_bytes = 1, ws_one.data_ptr(), ws_one.numel()
+        if ws is not None:
             p.attn_ws, p.attn_ws_bytes = ws.data_ptr(), ws.numel()
         p.smax, p.cache_rows, p.norm_in_rows, p.silu_in_rows, p.attn_from_qkv = smax, cache_rows, norm_in_rows, silu_in_rows, int(bool(attn_from_qkv))
         if pages is not None:
@@ -856,6 +854,34 @@ def shared_prefix_attn_qkv(p: PartialProduct, H: int, Hkv: int, D: int, cos: tor
                                          t_dev.data_ptr(), _ptr(pages), pages.stride(0) if pages is not None else 0,
                                          int(bool(single_launch)), ws.data_ptr(), ws.numel(), _stream()),
           "smh_shared_prefix_attn_qkv")
+    return out
+
+
+def shared_prefix_attn_qkv_tiles(p: PartialProduct, H: int, Hkv: int, D: int, cos: torch.Tensor, sin: torch.Tensor,
+                                 pos_dev: torch.Tensor, prefix_k: Optional[torch.Tensor], prefix_v: Optional[torch.Tensor], P: int,
+                                 cache_k: torch.Tensor, cache_ks: torch.Tensor, cache_v: torch.Tensor, cache_vs: torch.Tensor,
+                                 Smax: int, t_dev: torch.Tensor, pages: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """shared_prefix_attn_qkv for any number of branches, in one launch whose workgroups have 16 queries of a kv head each and read the whole
+    prefix for them.  pages: int32 [>= B, >= Smax] ids of the caches' rows."""
+    lib = _lib.load()
+    B = p.M
+    if pages is not None:
+        assert pages.is_cuda and pages.dtype == torch.int32 and pages.dim() == 2 and pages.stride(1) == 1
+        assert pages.shape[0] >= B and pages.shape[1] >= Smax
+    assert p.n_total == (H + 2 * Hkv) * D and p.buf.dtype == torch.float32
+    _need_gpu(p.buf, cache_k, cache_v, cache_ks, cache_vs, t_dev, pos_dev)
+    if prefix_k is not None:
+        assert prefix_k.is_contiguous() and prefix_v.is_contiguous() and prefix_k.dtype == torch.float16 and P <= prefix_k.shape[-3]
+    else:
+        assert P == 0
+    assert cache_k.dtype == torch.int8 and cache_ks.dtype == torch.float16 and t_dev.dtype == torch.int32
+    out = torch.empty((B, H, D), dtype=torch.float16, device=p.buf.device)
+    check(lib.smh_shared_prefix_attn_qkv_tiles(p.buf.data_ptr(), p.ksplit, out.data_ptr(), B, H, Hkv, D, cos.data_ptr(), sin.data_ptr(),
+                                               pos_dev.data_ptr(), _ptr(prefix_k), _ptr(prefix_v), int(P),
+                                               cache_k.data_ptr(), cache_ks.data_ptr(), cache_v.data_ptr(), cache_vs.data_ptr(), int(Smax),
+                                               t_dev.data_ptr(), _ptr(pages), pages.stride(0) if pages is not None else 0,
+                                               cache_k.numel() // (64 * Hkv), _stream()),
+          "smh_shared_prefix_attn_qkv_tiles")
     return out
 
 
