@@ -7,12 +7,29 @@ device, replay again.  No hipMemsetAsync node is recorded (the matmul workspace 
 """
 from __future__ import annotations
 
+import contextlib
+import gc
 from typing import Optional
 
 import torch
 
 from . import kernels as K
 from .hf_model_q40_kv_shared import Transformer
+
+
+@contextlib.contextmanager
+def recording(graph: "torch.cuda.CUDAGraph"):
+    """torch.cuda.graph(graph) with no garbage collection inside: a collection that falls into a recording destroys whatever GPU objects wait for
+    one - the graphs of a search that its hook keeps in a cycle - and their destruction synchronises, which a recording stream
+    forbids: the process aborts."""
+    collects = gc.isenabled()
+    gc.disable()
+    try:
+        with torch.cuda.graph(graph):
+            yield
+    finally:
+        if collects:
+            gc.enable()
 
 
 class GraphDecoder:
@@ -86,7 +103,7 @@ class GraphDecoder:
             # they must outlive it even if a later, larger call replaces them in the operators' table
             self._pinned = list(K._workspaces.values())
             self.graph = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(self.graph):
+            with recording(self.graph):
                 self._step()
             self._graph_key = self._key()
             # the capture pass itself does not execute; state and tokens are untouched
@@ -231,7 +248,7 @@ class BucketedForward:
         # the warm-up grew the shared workspaces to what this bucket needs; the graph records their addresses
         self._pinned.extend(w for w in K._workspaces.values() if not any(w is q for q in self._pinned))
         g = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(g):
+        with recording(g):
             logits = self._run(bucket)
         self.graphs[bucket] = (g, logits)
         torch.cuda.synchronize()
