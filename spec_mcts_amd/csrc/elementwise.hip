@@ -242,6 +242,7 @@ namespace smh {
 // probabilities p = fp16(softmax) as F.softmax on an fp16 tensor returns them, and one candidate is drawn by inverse
 // CDF with the caller's uniform number.
 constexpr int SAMPLE_MAX_K = 1024;
+constexpr int SAMPLE_HOT_MAX = 576;            // threads whose logits are looked at again
 constexpr int SAMPLE_PICK_MAX_K = 512;         // up to here the candidates are picked by the threads' maxima (above, they would be thousands)
 
 __device__ __forceinline__ uint32_t sample_key(half_t x) {
@@ -249,8 +250,10 @@ __device__ __forceinline__ uint32_t sample_key(half_t x) {
     return (b & 0x8000u) ? (~b & 0xFFFFu) : (b | 0x8000u);       // larger value <=> larger key
 }
 // ... of two fp16 values in one word
+typedef int16_t s16x2 __attribute__((ext_vector_type(2)));
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t sample_keys2(uint32_t b) {
-    const uint32_t neg = ((b >> 15) & 0x00010001u) * 0xFFFFu;       // 0xFFFF in the halves that are negative
+    const uint32_t neg = __builtin_bit_cast(uint32_t, __builtin_bit_cast(s16x2, b) >> 15);       // 0xFFFF in the halves that are negative
     return b ^ (neg | 0x80008000u);
 }
 __device__ __forceinline__ half_t sample_unkey(uint32_t k) {
@@ -294,7 +297,10 @@ __device__ __forceinline__ void sample_pick_bin(int *bins, int *s_w, int want, i
 // its candidates, with the uniform numbers (and into the slots of out) that start at counts[0] + ... + counts[r-1].
 // Up to 32768 logits (a multiple of 8, rows 16-byte aligned) and k <= 512 the row is read once into registers and the candidates
 // are those not below the k-th largest of the threads' maxima (a handful more than k): no histogram of the whole row, whose LDS
-// atomics pile up on the few bins that logits fall into.  80 rows of 32016, k = 32: 35 us with histograms, 11 like this.
+// atomics pile up on the few bins that logits fall into.  80 rows of 32016, k = 32: 35 us with histograms, 7.9 like this.
+// Bound by its instructions (sixteen waves on a compute unit: 18 cycles each for all of them) and a chain of barriers.  So keys are made and
+// compared two to an instruction, only the few threads whose maximum reaches the bound hand their logits out, one to a thread, instead
+// of every wave looking through 32 (12.3 us with that), and what the draws need is on its way from the start.
 // Otherwise, and where the maxima leave more than 1024 candidates (ordered or mostly equal logits), two histogram passes: thread
 // t owns the contiguous chunk of ceil(vocab / 1024) logits that starts at t times that.
 __global__ __launch_bounds__(1024) void sample_topk_kernel(const half_t *__restrict__ logits, int vocab, long ld, float temperature,
@@ -313,10 +319,15 @@ __global__ __launch_bounds__(1024) void sample_topk_kernel(const half_t *__restr
     const bool greedy_row = row_temps != nullptr && !(temperature > 0.f);
     if (greedy_row) temperature = 1.0f;
     __shared__ int bins[256];
-    __shared__ __attribute__((aligned(16))) int wbins[256 * 16];
+    __shared__ __attribute__((aligned(16))) uint32_t hot_words[SAMPLE_HOT_MAX * 16];
+    __shared__ int hot_tid[SAMPLE_HOT_MAX];
+    int *const wbins = reinterpret_cast<int *>(hot_words);                 // [256 * 16]
+    static_assert(SAMPLE_HOT_MAX >= 256, "the histograms fit");
     __shared__ int s_wi[16];
     __shared__ float s_wf[16];
-    __shared__ int s_bin, s_above, s_count;
+    __shared__ int s_bin, s_above, s_count, s_hot;
+    __shared__ int s_first, s_draws;
+    __shared__ float s_uniform[64];
     __shared__ __attribute__((aligned(16))) uint32_t c_key[SAMPLE_MAX_K];
     __shared__ int c_idx[SAMPLE_MAX_K];
     __shared__ uint32_t o_key[SAMPLE_MAX_K];
@@ -327,7 +338,26 @@ __global__ __launch_bounds__(1024) void sample_topk_kernel(const half_t *__restr
     int k = min(top_k, vocab);
     auto key_of = [&](half_t x) { return sample_key(wide ? x : (half_t)((float)x / temperature)); };
     auto value_of = [&](uint32_t key) { return wide ? (float)sample_unkey(key) / temperature : (float)sample_unkey(key); };
-    const int wv = tid >> 6;
+    const int wv = tid >> 6, lane = tid & 63;
+
+    // The first wave: which draws are this row's (the counts of the rows before it added up, all loads together) and the uniform numbers of the
+    // first 64.  Every sum is cut at n_draws < 2^31 - counts that add up to more than the buffers hold are cut - so none of these
+    // unsigned sums wraps.
+    auto find_draws = [&]() {
+        int first = blockIdx.x, draws = 1;
+        if (counts != nullptr) {
+            const uint32_t most = (uint32_t)max(n_draws, 0);
+            uint32_t sum = 0;
+            for (int r = lane; r < (int)blockIdx.x; r += 64) sum = min(sum + (uint32_t)max(counts[r], 0), most);
+            const int own = counts[blockIdx.x];
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) sum = min(sum + (uint32_t)__shfl_xor((int)sum, o, 64), most);
+            first = (int)sum;
+            draws = min(max(own, 0), (int)(most - sum));
+        }
+        if (lane == 0) { s_first = first; s_draws = draws; }
+        if (!greedy_row && lane < draws) s_uniform[lane] = uniform[first + lane];
+    };
 
     constexpr int CH = 32;
     const bool in_regs = vocab <= 1024 * CH && vocab % 8 == 0 && (reinterpret_cast<uintptr_t>(row) & 15) == 0;     // (uniform)
@@ -339,25 +369,30 @@ __global__ __launch_bounds__(1024) void sample_topk_kernel(const half_t *__restr
         // quotients; the quotient is monotonic, so the logits themselves are compared, down to the smallest one with the same
         // quotient.
         uint32_t raw[CH / 2];
+        u32x4 from[CH / 8];
 #pragma unroll
         for (int q = 0; q < CH / 8; ++q) {
             const int i = 8 * (tid + 1024 * q);
-            u32x4 v = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu};       // key 0: below every number
-            if (i < vocab) v = *reinterpret_cast<const u32x4 *>(row + i);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) raw[4 * q + j] = sample_keys2(v[j]);
+            from[q] = u32x4{0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu};  // key 0: below every number
+            if (i < vocab) from[q] = *reinterpret_cast<const u32x4 *>(row + i);
         }
-        uint32_t mx = 0;
+        if (wv == 0) find_draws();
 #pragma unroll
-        for (int j = 0; j < CH / 2; ++j) mx = max(mx, max(raw[j] & 0xFFFFu, raw[j] >> 16));
-        uint32_t *maxima = reinterpret_cast<uint32_t *>(wbins);
+        for (int q = 0; q < CH / 8; ++q)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) raw[4 * q + j] = sample_keys2(from[q][j]);
+        u16x2 two = __builtin_bit_cast(u16x2, raw[0]);
+#pragma unroll
+        for (int j = 1; j < CH / 2; ++j) two = __builtin_elementwise_max(two, __builtin_bit_cast(u16x2, raw[j]));
+        const uint32_t mx = max((uint32_t)two[0], (uint32_t)two[1]);
+        uint32_t *maxima = hot_words;
         maxima[tid] = mx;
-        if (tid == 0) s_count = 0;
+        if (tid == 0) s_count = s_hot = 0;
         __syncthreads();
         uint32_t mine[16];                     // every wave holds all the maxima ...
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const u32x4 v = *reinterpret_cast<const u32x4 *>(&maxima[256 * j + 4 * (tid & 63)]);
+            const u32x4 v = *reinterpret_cast<const u32x4 *>(&maxima[256 * j + 4 * lane]);
 #pragma unroll
             for (int e = 0; e < 4; ++e) mine[4 * j + e] = v[e];
         }
@@ -369,40 +404,50 @@ __global__ __launch_bounds__(1024) void sample_topk_kernel(const half_t *__restr
 #pragma unroll
             for (int j = 0; j < 16; ++j) n += __popcll(__ballot(mine[j] >= t));
             int *slot = bins + 16 * (shift >> 2);
-            if ((tid & 63) == 0) slot[wv] = n;
+            if (lane == 0) slot[wv] = n;
             __syncthreads();
-            int d = 0;
-#pragma unroll
-            for (int w = 1; w < 16; ++w) d = slot[w] >= k ? w : d;
-            thr |= (uint32_t)d << shift;
+            // (the counts fall from wave to wave, and the first one's reaches k)
+            thr |= (uint32_t)(__popcll(__ballot(slot[lane & 15] >= k) & 0xFFFFull) - 1) << shift;
         }
         bool small = true;
-        if (!wide) {
-            const uint32_t q = key_of(sample_unkey(thr));
-            int steps = 0;
-            while (thr > 0 && steps < 64 && key_of(sample_unkey(thr - 1)) == q) { --thr; ++steps; }
-            small = steps < 64;
+        if (!wide) {                           // (one candidate a lane: thr - lane)
+            const bool same = key_of(sample_unkey(thr - min((uint32_t)lane, thr))) == key_of(sample_unkey(thr)) && (uint32_t)lane <= thr;
+            const int steps = __builtin_ctzll(~(__ballot(same) >> 1));
+            thr -= steps;
+            small = steps < 63;
         }
-        int n = 0;
-        if (small) {
+        const bool real = small && thr > 0;                     // (key 0: also the slots past the row)
+        // the threads whose maximum reaches the bound leave their keys, in any order
+        const bool hot = real && mx >= thr;
+        const uint64_t hots = __ballot(hot);
+        if (hots != 0) {                       // (uniform)
+            int at = 0;
+            if (lane == 0) at = atomicAdd(&s_hot, __popcll(hots));
+            at = __builtin_amdgcn_readfirstlane(at) + __popcll(hots & ((1ull << lane) - 1));
+            if (hot && at < SAMPLE_HOT_MAX) {
 #pragma unroll
-            for (int j = 0; j < CH / 2; ++j) n += ((raw[j] & 0xFFFFu) >= thr) + ((raw[j] >> 16) >= thr);
-            const bool real = thr > 0;                          // (key 0: also the slots past the row)
-            int at = n > 0 && real ? atomicAdd(&s_count, n) : 0;
-            if (!real) at = SAMPLE_MAX_K;
-            if (n > 0) {
-#pragma unroll
-                for (int j = 0; j < CH; ++j) {
-                    const uint32_t key = (raw[j >> 1] >> (16 * (j & 1))) & 0xFFFFu;
-                    if (key >= thr) {
-                        // key above 32767 - index: one comparison orders by value, then by index
-                        const uint32_t i = 8 * (tid + 1024 * (j >> 3)) + (j & 7);
-                        if (at < SAMPLE_MAX_K) c_key[at] = ((wide ? key : key_of(sample_unkey(key))) << 15) | (32767u - i);
-                        ++at;
-                    }
+                for (int j = 0; j < 4; ++j) *reinterpret_cast<u32x4 *>(&hot_words[16 * at + 4 * j]) = u32x4{raw[4 * j], raw[4 * j + 1], raw[4 * j + 2], raw[4 * j + 3]};
+                hot_tid[at] = tid;
+            }
+        }
+        __syncthreads();
+        const int n_hot = s_hot;
+        if (real && n_hot <= SAMPLE_HOT_MAX) {
+            for (int x0 = 0; x0 < 32 * n_hot; x0 += 1024) {
+                const int x = x0 + tid;
+                uint32_t key = 0;
+                if (x < 32 * n_hot) key = reinterpret_cast<const uint16_t *>(hot_words)[x];
+                const bool in = key >= thr;
+                const uint64_t ins = __ballot(in);
+                if (ins != 0) {                // (uniform)
+                    int at = 0;
+                    if (lane == 0) at = atomicAdd(&s_count, __popcll(ins));
+                    at = __builtin_amdgcn_readfirstlane(at) + __popcll(ins & ((1ull << lane) - 1));
+                    // key above 32767 - index: one comparison orders by value, then by index
+                    const uint32_t j = x & 31, i = 8 * (hot_tid[min(x >> 5, SAMPLE_HOT_MAX - 1)] + 1024 * (j >> 3)) + (j & 7);
+                    if (in && at < SAMPLE_MAX_K) c_key[at] = ((wide ? key : key_of(sample_unkey(key))) << 15) | (32767u - i);
                 }
             }
-            if (!real && tid == 0) s_count = SAMPLE_MAX_K + 1;
             __syncthreads();
             const int count = s_count;
             if (count <= SAMPLE_MAX_K) {
@@ -441,6 +486,7 @@ __global__ __launch_bounds__(1024) void sample_topk_kernel(const half_t *__restr
     }
     if (!found) {
     // ---- by histograms: many candidates, or rows that cannot be held in registers ----
+    if (wv == 0 && !(in_regs && k <= SAMPLE_PICK_MAX_K)) find_draws();
     __syncthreads();
     const bool hold = in_regs && top_k > SAMPLE_PICK_MAX_K;
     const int chunk = hold ? CH : (vocab + 1023) / 1024;
@@ -571,26 +617,15 @@ __global__ __launch_bounds__(1024) void sample_topk_kernel(const half_t *__restr
         before = tid == 0 ? 0.f : cdf[tid - 1];
         all = cdf[k - 1];
     }
-    long first = blockIdx.x;
-    int draws = 1;
-    if (counts != nullptr) {
-        // every wave adds the counts of the rows before this one (all loads together, not one behind the other); every sum is cut at
-        // n_draws < 2^31 - counts that add up to more than the buffers hold are cut - so none of these unsigned sums wraps
-        const uint32_t most = (uint32_t)max(n_draws, 0);
-        uint32_t sum = 0;
-        for (int r = tid & 63; r < (int)blockIdx.x; r += 64) sum = min(sum + (uint32_t)max(counts[r], 0), most);
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) sum = min(sum + (uint32_t)__shfl_xor((int)sum, o, 64), most);
-        first = sum;
-        draws = min(max(counts[blockIdx.x], 0), (int)(most - sum));
-    }
+    const long first = s_first;
+    const int draws = s_draws;
     if (greedy_row) {
         for (int j = tid; j < draws; j += one_wave ? 64 : 1024) out[first + j] = o_idx[0];
         return;
     }
     if (tid < k) {
         for (int j = 0; j < draws; ++j) {
-            const float target = uniform[first + j] * all;
+            const float target = (j < 64 ? s_uniform[j] : uniform[first + j]) * all;
             // first candidate whose cumulative probability exceeds the target (the last one if rounding leaves none)
             if ((before <= target && target < upto) || (tid == k - 1 && target >= upto)) out[first + j] = o_idx[tid];
         }

@@ -155,6 +155,36 @@ def test_sample_topk_ties_take_the_lowest_indices_and_frequencies_follow_p():
         assert abs(freq - pj) < 4 * (pj * (1 - pj) / n) ** 0.5 + 1e-3
 
 
+@pytest.mark.parametrize("k", [1, 32, 512])
+@pytest.mark.parametrize("hot", [1, 40, 575, 576, 577, 1000])
+@pytest.mark.parametrize("temperature", [0.7, 3000.0])
+def test_sample_topk_whatever_number_of_threads_holds_candidates(k, hot, temperature):
+    """The sampler looks again at the logits of the threads (eight in a row, every 8192) whose maximum reaches its bound: rows whose largest values,
+    some of them equal, sit in 1 .. 1000 of those, on either side of the 576 it keeps, and temperatures behind which many logits have one
+    quotient.  More draws than the 64 uniform numbers that are fetched ahead."""
+    from spec_mcts_amd import kernels as K
+    g = torch.Generator().manual_seed(7 * hot + k)
+    vocab = 32016
+    rows, per = 3, 70
+    logits = (torch.randn((rows, vocab), generator=g) * 0.5).half()
+    for r in range(rows):
+        for n, t in enumerate(torch.randperm(1000, generator=g)[:hot].tolist()):
+            logits[r, 8 * t + int(torch.randint(0, 8, (1,), generator=g))] = 6.0 + (n % 7) * 0.5
+            if hot <= 40:
+                logits[r, 8192 + 8 * t:8192 + 8 * t + 8] = 5.0 + 0.25 * r
+    counts = torch.full((rows,), per, dtype=torch.int32)
+    u = torch.rand(rows * per, generator=g)
+    p, idx = O.topk_probs(logits, temperature, k)
+    cdf = p.float().cumsum(-1)
+    got = K.sample_topk_counts(logits.cuda(), temperature, k, counts.cuda(), u.cuda()).cpu()
+    want = O.sample_topk_counts(logits, temperature, k, counts.tolist(), u)
+    for i in (got != want).nonzero().flatten().tolist():         # only where the number falls on a step (as above)
+        r, pos = i // per, (idx[i // per] == int(got[i])).nonzero()
+        assert len(pos) == 1, f"draw {i}: token {int(got[i])} is not a candidate"
+        j, target = int(pos[0]), float(u[i]) * float(cdf[r, -1])
+        assert min(abs(e - target) for e in (float(cdf[r, j - 1]) if j else 0.0, float(cdf[r, j]))) < 1e-5, f"draw {i}"
+
+
 @pytest.mark.parametrize("rows,vocab,k,temperature,grid", [(100, 32016, 32, 0.8, 0), (6, 32016, 32, 1.0, 8), (3, 320, 5, 1.0, 2),
                                                            (7, 1000, 1, 1.3, 4), (4, 50, 50, 2.0, 2), (5, 4096, 1000, 0.6, 0)])
 def test_sample_topk_filter_matches_the_oracle(rows, vocab, k, temperature, grid):
