@@ -300,6 +300,7 @@ __device__ __forceinline__ void attn_prefix_body(const AttnParams &p, int split,
 
 template <bool FUSED>
 __global__ __launch_bounds__(256) void attn_prefix_kernel(AttnParams p) {
+    args_ahead<sizeof(AttnParams)>();
     attn_prefix_body<FUSED, false, ATT_TW_MAX>(p, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z);
 }
 
@@ -342,6 +343,7 @@ __device__ __forceinline__ long page_row(const AttnParams &p, page_id_t<PB> id) 
 }
 template <int PB>
 __global__ __launch_bounds__(256) void attn_page_tile_kernel(AttnParams p) {
+    args_ahead<sizeof(AttnParams)>();
     __shared__ __attribute__((aligned(16))) half_t ks[PT_TW][ATT_KPITCH];
     __shared__ __attribute__((aligned(16))) half_t vt[ATT_D][PT_TW + 8];
     __shared__ __attribute__((aligned(16))) half_t ps[3][16][PT_TW + 8];      // probabilities of the 16 queries, the three terms, in vt_pos order
@@ -1128,6 +1130,7 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
 // positions of a page table 171 -> 150 us)
 template <bool FUSED, int WALK, int PB>
 __global__ __launch_bounds__(256, FUSED ? 1 : 4) void attn_suffix_kernel(AttnParams p) {
+    args_ahead<sizeof(AttnParams)>();
     // suffix_waves (1, 2 or 4) waves per (branch, query head): more than one while branches x heads leave CUs idle.
     // Workgroups are dealt round-robin to the 8 XCDs (8 L2s); the heads of one branch share the 128-byte lines of that
     // branch's scales (2 fp16 per head and position), so ALL workgroups of a branch go to one XCD: workgroup L of the 1-D
@@ -1136,7 +1139,7 @@ __global__ __launch_bounds__(256, FUSED ? 1 : 4) void attn_suffix_kernel(AttnPar
     const int wave = threadIdx.x >> 6, nsub = p.suffix_waves;
     const int per_branch = (p.H * nsub + 3) >> 2;              // workgroups (four waves) per branch
     const int L = blockIdx.x, j = L >> 3;
-    const int grp = j / per_branch;
+    const int grp = uniform_divmod(j, per_branch).q;
     const int b = 8 * grp + (L & 7);
     if (b >= p.B) return;
     const int hq = (j - grp * per_branch) * 4 + wave;
@@ -1264,14 +1267,15 @@ __device__ __forceinline__ void attn_prefix_round(const AttnParams &p, int split
 // prefix_wgs: a multiple of 8, so that the others sit on the XCDs that attn_suffix_kernel's would
 template <int PB>
 __global__ __launch_bounds__(256, 4) void attn_parts_kernel(AttnParams p, int prefix_wgs, int rounds) {
+    args_ahead<sizeof(AttnParams)>();
     int L = blockIdx.x;
     if (L < prefix_wgs) {
-        const int hk = L % p.Hkv, rest = L / p.Hkv, split = rest / rounds;
-        if (split < p.splits) attn_prefix_round(p, split, hk, rest - split * rounds);
+        const DivMod head = uniform_divmod(L, p.Hkv), slice = uniform_divmod(head.q, rounds);
+        if (slice.q < p.splits) attn_prefix_round(p, slice.q, head.r, slice.r);
         return;
     }
     L -= prefix_wgs;
-    const int wave = threadIdx.x >> 6, nsub = p.suffix_waves, per_branch = (p.H * nsub + 3) >> 2, j = L >> 3, grp = j / per_branch, b = 8 * grp + (L & 7);
+    const int wave = threadIdx.x >> 6, nsub = p.suffix_waves, per_branch = (p.H * nsub + 3) >> 2, j = L >> 3, grp = uniform_divmod(j, per_branch).q, b = 8 * grp + (L & 7);
     if (b >= p.B) return;
     const int hq = (j - grp * per_branch) * 4 + wave, h = nsub == 4 ? hq >> 2 : (nsub == 2 ? hq >> 1 : hq);
     if (nsub == 1 && h >= p.H) return;
@@ -1280,6 +1284,7 @@ __global__ __launch_bounds__(256, 4) void attn_parts_kernel(AttnParams p, int pr
 
 // One wave per query adds its splits + 1 partials up, in split order: lane d holds dims 2 d, 2 d + 1.
 __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p) {
+    args_ahead<sizeof(AttnParams)>();
     const int qi = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;       // kv head * Bq + query of the kv head
     const int queries = p.Hkv * p.Bq;
     if (qi >= queries) return;
@@ -1327,6 +1332,7 @@ constexpr int ATT_ONE_MAX_TILES = ATT_FUSED_MAX_Q / 16;
 
 template <bool FUSED, int PB, int QKS = 16>
 __global__ __launch_bounds__(256, 2) void attn_one_kernel(AttnParams p) {
+    args_ahead<sizeof(AttnParams)>();
     __shared__ uint32_t s_last[ATT_ONE_MAX_TILES];
     const int hk = blockIdx.y;
     const int tid = threadIdx.x;
@@ -1524,6 +1530,7 @@ __device__ __forceinline__ void kv_store_lanes(h4 x, uint8_t *row, half_t *scale
 // its rows 16 at a time in turn).  Grid: (XCD, kv head of it, tile).
 template <bool PAGES, int LEAST, int QKS, int QT>
 __global__ __launch_bounds__(64 * AT_WAVES) void attn_tile_kernel(AttnParams p, int chunks) {
+    args_ahead<sizeof(AttnParams)>();
     extern __shared__ __attribute__((aligned(16))) float at_lds[];
     half_t *const s_q = reinterpret_cast<half_t *>(at_lds + AT_WAVES * AT_MINE), *const s_k = s_q + 16 * AT_QPITCH, *const s_v = s_k + 16 * AT_QPITCH;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;

@@ -62,6 +62,7 @@ __device__ __forceinline__ void head_wait_stages(int left) {
 // TILES: 16-row tiles of x a workgroup multiplies (1..8); XD = DMA instructions of the x tile per wave and stage
 template <int TILES>
 __global__ __launch_bounds__(HEAD_WAVES * 64) void f16_head_kernel(HeadParams p) {
+    args_ahead<sizeof(HeadParams)>();
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     constexpr int X_BYTES = TILES * 16 * 128;
     constexpr int STAGE = HEAD_W_BYTES + X_BYTES;
@@ -106,7 +107,7 @@ __global__ __launch_bounds__(HEAD_WAVES * 64) void f16_head_kernel(HeadParams p)
     // channels: 59.6 us per launch at the 7B shape; staggered, 47.8 us (5.5 TB/s).  The order of the fp32 additions of an output
     // then depends on its block of 128 outputs, not on anything that varies between runs.
     const int n_stages = p.K / HEAD_KS;
-    const int rot = (int)(blockIdx.x % (unsigned)n_stages);
+    const int rot = uniform_divmod((int)blockIdx.x, n_stages).r;
     auto issue = [&](int stage_i, int slot) {
         uint8_t *st = lds + slot * STAGE;
         int stage_k = stage_i + rot;
@@ -207,6 +208,7 @@ constexpr int HEAD_ROWS_LEAST_WGS = 192;
 typedef float f16v __attribute__((ext_vector_type(16)));
 template <int XB>                                            // 32-row tiles of x a wave: 4, or 2 (blocks of 128 rows, for 129 .. 256)
 __global__ __launch_bounds__(512, 2) void f16_head_rows_kernel(HeadParams p) {
+    args_ahead<sizeof(HeadParams)>();
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int n0 = blockIdx.x * HEAD_ROWS, m0 = blockIdx.y * (64 * XB);
     if (n0 >= p.N) return;                                   // (the padding of grid x)

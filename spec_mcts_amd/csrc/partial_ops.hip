@@ -19,11 +19,12 @@ namespace smh {
 // ---- plain reduce (+ residual) ------------------------------------------------------------------
 // RES: a residual of this alignment (elements a load; 0: none)
 template <int KS, int RES>
-__global__ __launch_bounds__(256) void partial_reduce_kernel(const void *__restrict__ partial, int ks, int M, int n_total, int col0, int N,
+__global__ __launch_bounds__(256) void partial_reduce_kernel(const void *__restrict__ partial, int ks, int M, int m0, int n_total, int col0, int N,
                                                              half_t *__restrict__ c, long ldc, const half_t *__restrict__ resid, long ldr) {
-    const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
-    if (i >= (long)M * N) return;
-    const int m = (int)(i / N), n = (int)(i % N);          // N % 4 == 0: the 4 columns share a row
+    // grid (quads of a row, rows): no division to find the row (a 64-bit one, 150 instructions, was most of the launch)
+    args_ahead<96>();
+    const int m = m0 + (int)blockIdx.y, n = (int)(blockIdx.x * blockDim.x + threadIdx.x) * 4;
+    if (n >= N) return;
     f4 v[KS];
     slab_load(partial, (long)m * n_total + col0 + n, (long)M * n_total, ks, v);
     h4 r;
@@ -311,7 +312,7 @@ using namespace smh;
 // kernels by the number of slabs (least_slabs)
 static_assert(SMH_MAX_KSPLIT == 16, "tables");
 #define BY_SLABS(k, ...) {__VA_ARGS__, k(1), k(2), k(3), k(4), k(5), k(6), k(8), k(8), k(10), k(10), k(12), k(12), k(16), k(16), k(16), k(16)}
-typedef void (*reduce_kernel_t)(const void *, int, int, int, int, int, half_t *, long, const half_t *, long);
+typedef void (*reduce_kernel_t)(const void *, int, int, int, int, int, int, half_t *, long, const half_t *, long);
 typedef void (*rmsnorm_kernel_t)(const void *, int, int, int, const half_t *, const half_t *, float, half_t *, half_t *);
 typedef void (*sumsq_kernel_t)(const void *, int, int, int, const half_t *, half_t *, float *);
 #define K_OF(n) partial_reduce_kernel<n, RES>
@@ -534,11 +535,12 @@ extern "C" int smh_q40_matmul_partial_tiled_norm(const void *h, long ldh, const 
 
 static int reduce_launch(const void *partial, int ksplit, int M, int n_total, int col0, int N, void *c, long ldc,
                          int epilogue, const void *residual, long ldr, hipStream_t stream) {
-    long quads = ((long)M * N + 3) / 4;
+    const int quads = N / 4, threads = min(256, (quads + 63) / 64 * 64);       // of a row
     const bool aligned = ldr % 4 == 0 && (uintptr_t)residual % 8 == 0;
     const auto kern = (epilogue != SMH_EPI_RESIDUAL ? REDUCE_KERNELS<0> : aligned ? REDUCE_KERNELS<4> : REDUCE_KERNELS<1>)[ksplit];
-    hipLaunchKernelGGL(kern, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream, partial, ksplit, M, n_total, col0, N, (half_t *)c, ldc,
-                       (const half_t *)residual, ldr);
+    for (int m0 = 0; m0 < M; m0 += 65535)                    // (a grid has at most 65535 rows)
+        hipLaunchKernelGGL(kern, dim3((unsigned)((quads + threads - 1) / threads), (unsigned)min(M - m0, 65535)), dim3(threads), 0, stream, partial, ksplit, M, m0,
+                           n_total, col0, N, (half_t *)c, ldc, (const half_t *)residual, ldr);
     return launch_status();
 }
 

@@ -239,10 +239,11 @@ __global__ __launch_bounds__(256) void q40_quantize_t_kernel(const uint8_t *__re
     __shared__ uint32_t tile[128 * P];
     const int tid = threadIdx.x;
     const int n_blocks = N / 128;
-    const long total = (long)n_blocks * k_tiles, per = (total + 7) / 8;
-    const long id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    if ((long)(blockIdx.x >> 3) >= per || id >= total) return;
-    const int nb = (int)(id % n_blocks), k0 = (int)(id / n_blocks) * 64;
+    const int total = n_blocks * k_tiles, per = (total + 7) / 8;       // (of a grid: below 2^31 - 8)
+    const int id = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || id >= total) return;
+    const DivMod at = uniform_divmod(id, n_blocks);
+    const int nb = at.r, k0 = at.q * 64;
     {
         constexpr int VEC = 16 / ES;                         // values of a load
         constexpr int LPR = 64 / VEC;                        // lanes a row

@@ -115,7 +115,7 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
     int sg = 0;
     if (!SWIGLU && p.nseg > 1 && unit >= p.seg[1].unit0) sg = 1;
     if (!SWIGLU && p.nseg > 2 && unit >= p.seg[2].unit0) sg = 2;
-    const MatmulSegment seg = p.seg[sg];
+    const MatmulSegment seg = segment_at(p, sg);
     const int pair = SWIGLU ? unit >> 1 : unit - seg.unit0;
     const int col0 = SWIGLU ? unit * 128 : pair * GEMM_COLS;
     const bool two_blocks = SWIGLU || col0 + 128 < seg.N;
@@ -210,7 +210,7 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
     const int n_steps = max(step1 - step0, 0);
     // workgroups that share a K-slice read the same A tiles; each starts at a different step of the
     // slice (and wraps) so that they do not all pull the same L2 lines at the same time
-    const int rot = n_steps > 0 ? (unit * 5) % n_steps : 0;
+    const int rot = n_steps > 0 ? uniform_divmod(unit * 5, n_steps).r : 0;
     int fetch = step0 + rot;                   // next step to fetch
     auto fetch_next = [&](int slot_) {
         issue(fetch, slot_);
@@ -617,6 +617,7 @@ template <int TILES, bool RAGGED, bool TILED, int WAVES, int SLOTS = GEMM_STAGES
 __global__ __launch_bounds__(64 * (WAVES + (PRODUCER ? 1 : 0)), WAVES == 8 ? (SWIGLU && !PRODUCER ? 4 : 1) : 2) void q40_gemm_kernel(MatmulParams p) {
     static_assert(WAVES == 4 || (WAVES == 8 && (TILED ? !RAGGED : PRODUCER)), "eight waves: K a multiple of 32, or the checkpoint layout with a DMA wave");
     static_assert(SLOTS >= 6 && SLOTS <= 8 && (SLOTS == GEMM_STAGES || PRODUCER) && (!PRODUCER || WAVES == 8), "ring depth");
+    args_ahead<sizeof(MatmulParams)>();
     const int steps_total = (p.K + 31) / 32;
     if constexpr (RANGE) {
         int run0 = (int)blockIdx.x * p.chunk;                  // (units x steps is far below 2^31)
@@ -636,13 +637,12 @@ __global__ __launch_bounds__(64 * (WAVES + (PRODUCER ? 1 : 0)), WAVES == 8 ? (SW
             gemm_piece<TILES, RAGGED, TILED, WAVES, SLOTS, PRODUCER>(p, unit, 0, (int)blockIdx.x - first, s0, s1, s1 == steps_total, more, opaque_zero);
         }
     } else {
-        int bid = blockIdx.x;
-        // slot -> unit: each XCD (blockIdx % 8) takes a contiguous run of column units, which share scale lines
-        const int slot = bid % p.units_pad;  bid /= p.units_pad;
+        // blockIdx.x -> unit: each XCD (workgroups are dealt to them in turn) takes a contiguous run of column units, which share scale lines
+        const int slot = blockIdx.x;
         const int unit = (slot & 7) * (p.units_pad >> 3) + (slot >> 3);
         if (unit >= p.units) return;
-        const int mb = bid % p.mblocks;
-        const int slice = bid / p.mblocks;
+        const int mb = p.mb0 + (int)blockIdx.y;
+        const int slice = blockIdx.z;
         const int s0 = slice * p.steps_per_slice;
         gemm_piece<TILES, RAGGED, TILED, WAVES, SLOTS, PRODUCER, SWIGLU>(p, unit, mb, slice, s0, min(s0 + p.steps_per_slice, steps_total), false, false, 0);
     }
@@ -678,17 +678,17 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_kg_kernel(MatmulParams p) {
     const int tid = threadIdx.x;
     const int wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);       // 0..7 multiply, 8 issues the DMA
     const int lane = tid & 63, c = lane & 15, g = lane >> 4;
+    args_ahead<sizeof(MatmulParams)>();
     // blockIdx -> (128-column block, row block, K-slice); blocks of one unit are neighbours (same XCD every 8)
-    int bid = blockIdx.x;
-    const int hb = bid % (2 * p.units_pad);  bid /= 2 * p.units_pad;
+    const int hb = blockIdx.x;
     const int slot_u = hb >> 1, blk = hb & 1;
     const int unit = (slot_u & 7) * (p.units_pad >> 3) + (slot_u >> 3);
     if (unit >= p.units) return;
-    const int mb = bid % p.mblocks, slice = bid / p.mblocks;
+    const int mb = blockIdx.y, slice = blockIdx.z;
     int sg = 0;
     if (p.nseg > 1 && unit >= p.seg[1].unit0) sg = 1;
     if (p.nseg > 2 && unit >= p.seg[2].unit0) sg = 2;
-    const MatmulSegment seg = p.seg[sg];
+    const MatmulSegment seg = segment_at(p, sg);
     const int pair = unit - seg.unit0;
     const int col0 = pair * GEMM_COLS + 128 * blk;
     if (col0 >= seg.N) return;                                         // a weight with an odd number of 128-column blocks
@@ -698,7 +698,7 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_kg_kernel(MatmulParams p) {
     const int n_st = max(step1 - step0, 0) / 2;                        // stages (two steps each; slices are even)
     const uint8_t *w_base = seg.w + (long)pair * tiled_steps(p.K) * TILE_BYTES + (long)step0 * TILE_BYTES;
     const uint8_t *a_base = reinterpret_cast<const uint8_t *>(p.a) + (long)step0 * 64;
-    const int rot = n_st > 0 ? (hb * 5) % n_st : 0;                   // workgroups of a K-slice start at different stages
+    const int rot = n_st > 0 ? uniform_divmod(hb * 5, n_st).r : 0;             // workgroups of a K-slice start at different stages
 
     if (wave8 == 8) {
         // ---- the DMA wave ----
@@ -885,6 +885,7 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_swiglu_kernel(MatmulParams p)
     const int tid = threadIdx.x;
     const int wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);       // 0..7 multiply, 8 issues the DMA
     const int lane = tid & 63, c = lane & 15, g = lane >> 4;
+    args_ahead<sizeof(MatmulParams)>();
     // blockIdx -> (128-column block j of the gate and of the up weight, piece bp of that block)
     const int hb = blockIdx.x;
     const int blockj = hb >> 1, bp = hb & 1;
@@ -896,7 +897,7 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_swiglu_kernel(MatmulParams p)
     const uint8_t *w_gate = p.seg[0].w + (long)pair * tiled_steps(p.K) * TILE_BYTES;
     const uint8_t *w_up = p.seg[1].w + (long)pair * tiled_steps(p.K) * TILE_BYTES;
     const uint8_t *a_base = reinterpret_cast<const uint8_t *>(p.a);
-    const int rot = n_st > 0 ? (hb * 5) % n_st : 0;                   // workgroups of a K-slice start at different stages
+    const int rot = n_st > 0 ? uniform_divmod(hb * 5, n_st).r : 0;             // workgroups of a K-slice start at different stages
 
     if (wave8 == 8) {
         // ---- the DMA wave ----
@@ -1124,7 +1125,8 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_wide_kernel
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63, c = lane & 15, g = lane >> 4;
     // blockIdx -> (unit of three or six pieces, row block): each XCD takes a contiguous run of units
-    const int at = blockIdx.x % p.units_pad, mb = blockIdx.x / p.units_pad;
+    args_ahead<sizeof(MatmulParams)>();
+    const int at = blockIdx.x, mb = p.mb0 + (int)blockIdx.y;
     const int unit = (at & 7) * (p.units_pad >> 3) + (at >> 3);
     if (unit >= p.units) return;
     const int m0 = mb * p.block_rows, pieces = (SWIGLU ? p.seg[0].N : p.n_total) / 64;
@@ -1518,6 +1520,15 @@ void gemm_fill_plan(MatmulParams &p) {
 
 typedef void (*gemm_kernel_t)(MatmulParams);
 
+// Grid (units, row blocks, K-slices), by rows of at most 65535 row blocks
+static int gemm_launch_rows(gemm_kernel_t kern, MatmulParams p, int threads, int lds, hipStream_t stream) {
+    for (int mb = 0; mb < p.mblocks; mb += 65535) {
+        p.mb0 = mb;
+        hipLaunchKernelGGL(kern, dim3((unsigned)p.units_pad, (unsigned)min(p.mblocks - mb, 65535), (unsigned)p.ksplit), dim3(threads), lds, stream, p);
+    }
+    return launch_status();
+}
+
 template <bool TILED>
 static int gemm_launch_layout(const MatmulParams &p, hipStream_t stream) {
     // one instantiation per number of 16-row tiles (M <= 128) keeps the step free of branches; K % 32 != 0
@@ -1582,9 +1593,12 @@ static int gemm_launch_layout(const MatmulParams &p, hipStream_t stream) {
     const gemm_kernel_t kern = odd_k ? (TILED ? ragged : (one_each ? ragged_dma_wave : ragged_four)[tiles])
                                      : (p.chunk > 0 ? range_cut : one_each ? with_dma_wave : exact)[tiles];
     const long total_steps = (long)p.units * ((p.K + 31) / 32);
-    dim3 grid((unsigned)(p.chunk > 0 ? (total_steps + p.chunk - 1) / p.chunk : (long)p.units_pad * p.mblocks * p.ksplit));
-    hipLaunchKernelGGL(kern, grid, dim3(one_each ? 64 * (WD + 1) : four ? GEMM_THREADS : 64 * W), one_each ? gemm_dma_slots(tiles) * GS_BYTES : GEMM_LDS, stream, p);
-    return launch_status();
+    const int lds = one_each ? gemm_dma_slots(tiles) * GS_BYTES : GEMM_LDS, threads = one_each ? 64 * (WD + 1) : four ? GEMM_THREADS : 64 * W;
+    if (p.chunk > 0) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)((total_steps + p.chunk - 1) / p.chunk)), dim3(threads), lds, stream, p);
+        return launch_status();
+    }
+    return gemm_launch_rows(kern, p, threads, lds, stream);
 }
 
 typedef void (*gemm_kg_kernel_t)(MatmulParams);
@@ -1605,8 +1619,7 @@ static int gemm_kg_launch(const MatmulParams &p, hipStream_t stream) {
     SMH_REQUIRE((long)p.M * p.lda * 2 < (1L << 32), "q40 gemm: M x lda = %d x %ld exceeds the 32-bit lane offsets of A", p.M, p.lda);
     int tiles = p.mblocks > 1 ? p.block_rows / 16 : (p.M + 15) / 16;
     if (tiles < 2) tiles = 2;
-    dim3 grid((unsigned)(2L * p.units_pad * p.mblocks * p.ksplit));
-    hipLaunchKernelGGL(kern[tiles], grid, dim3(576), lds_bytes[tiles], stream, p);
+    hipLaunchKernelGGL(kern[tiles], dim3((unsigned)(2 * p.units_pad), (unsigned)p.mblocks, (unsigned)p.ksplit), dim3(576), lds_bytes[tiles], stream, p);
     return launch_status();
 }
 
@@ -1694,14 +1707,13 @@ int gemm_swiglu_rows_launch(MatmulParams p, hipStream_t stream) {
     MatmulParams w = p;
     if (gemm_swiglu_rows_plan(p, w)) {
         const int t = w.block_rows / 16 - 4;
-        hipLaunchKernelGGL(wide[t], dim3((unsigned)((long)w.units_pad * w.mblocks)), dim3(64 * (WIDE_WAVES + 1)), wide_lds[t], stream, w);
-        return launch_status();
+        w.ksplit = 1;
+        return gemm_launch_rows(wide[t], w, 64 * (WIDE_WAVES + 1), wide_lds[t], stream);
     }
     const bool one_each = (long)p.units * p.mblocks <= GEMM_DMA_WAVE_MAX_WGS;
     const int t = p.block_rows / 16 - 4;
-    hipLaunchKernelGGL((one_each ? dma_wave : plain)[t], dim3((unsigned)((long)p.units_pad * p.mblocks)), dim3(512 + (one_each ? 64 : 0)),
-                       one_each ? gemm_dma_slots(t + 4) * GS_BYTES : GEMM_LDS, stream, p);
-    return launch_status();
+    p.ksplit = 1;
+    return gemm_launch_rows((one_each ? dma_wave : plain)[t], p, 512 + (one_each ? 64 : 0), one_each ? gemm_dma_slots(t + 4) * GS_BYTES : GEMM_LDS, stream);
 }
 
 // The launch of a direct product whose plan has no K-split, with workgroups of three pieces and two K-groups or of six pieces where they
@@ -1752,8 +1764,7 @@ static int gemm_wide_launch(const MatmulParams &p, int pieces, hipStream_t strea
     }
     SMH_REQUIRE((long)p.M * p.lda * 2 < (1L << 32), "q40 gemm: M x lda = %d x %ld exceeds the 32-bit lane offsets of A", p.M, p.lda);
     const int six = pieces == 6 ? 1 : 0, t = p.block_rows / 16 - 4;
-    hipLaunchKernelGGL(kern[six][t], dim3((unsigned)((long)p.units_pad * p.mblocks)), dim3(64 * (WIDE_WAVES + 1)), lds_bytes[six][t], stream, p);
-    return launch_status();
+    return gemm_launch_rows(kern[six][t], p, 64 * (WIDE_WAVES + 1), lds_bytes[six][t], stream);
 }
 
 int gemm_launch(const MatmulParams &p, hipStream_t stream) {

@@ -256,15 +256,16 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void q40_gemv_kernel(MatmulParams 
     // Workgroups are dealt round-robin to the 8 XCDs (8 L2s).  Neighbouring column units share the 128-byte
     // lines of the scale rows, so each XCD takes a CONTIGUOUS run of units: a scale line is then fetched
     // from HBM by one L2, not by eight.
-    const int slot = blockIdx.x % p.units_pad;
+    args_ahead<sizeof(MatmulParams)>();
+    const int slot = blockIdx.x;
     const int unit = (slot & 7) * (p.units_pad >> 3) + (slot >> 3);
-    const int slice = blockIdx.x / p.units_pad;
+    const int slice = blockIdx.y;
     if (unit >= p.units) return;
     // which segment (weight) does this column pair belong to
     int sg = 0;
     if (p.nseg > 1 && unit >= p.seg[1].unit0) sg = 1;
     if (p.nseg > 2 && unit >= p.seg[2].unit0) sg = 2;
-    const MatmulSegment seg = p.seg[sg];
+    const MatmulSegment seg = segment_at(p, sg);
     const int pair = unit - seg.unit0;
 
     const int tid = threadIdx.x;
@@ -546,7 +547,7 @@ bool gemv_norm_in_fits(const MatmulParams &p) {
 
 int gemv_launch(const MatmulParams &p, hipStream_t stream) {
     constexpr int waves = GEMV_WAVES;
-    dim3 grid((unsigned)(p.units_pad * p.ksplit));
+    dim3 grid((unsigned)p.units_pad, (unsigned)p.ksplit);
     size_t lds = (size_t)waves * RING_BYTES;                       // rings, reused for the [waves][M][256] sums
     const size_t red = (size_t)waves * p.M * GEMV_COLS * sizeof(float);
     if (p.tiled && (p.gu_partial != nullptr || p.norm_w != nullptr))   // rings without activation tiles, xs (and r[]) behind them

@@ -58,6 +58,7 @@ struct MatmulParams {
     int M, K;
     int nseg, n_total;
     int units, units_pad;    // column units over all segments (GEMV: padded to a multiple of 8)
+    int mb0;                 // GEMM: row block of blockIdx.y == 0 (a grid has at most 65535 rows)
     int mblocks, block_rows; // GEMM: row blocks and the rows of one (128, or 64 where two blocks of a narrow matrix halve its K-slices)
     int ksplit, steps_per_slice;
     int kgroups;             // GEMM, 2: q40_gemm_kg_kernel (128-column blocks, two K-groups a workgroup)
@@ -76,6 +77,23 @@ struct MatmulParams {
     const float *norm_ss;
     float norm_eps;
 };
+
+// p.seg[sg] without a load that waits for sg
+__device__ __forceinline__ MatmulSegment segment_at(const MatmulParams &p, int sg) {
+    MatmulSegment r = p.seg[0];
+    auto pick = [&](auto member) { 
+        const auto a = held(p.seg[0].*member), b = held(p.seg[1].*member), c = held(p.seg[2].*member);
+        r.*member = sg == 0 ? a : sg == 1 ? b : c;
+    };
+    pick(&MatmulSegment::w);
+    pick(&MatmulSegment::s);
+    pick(&MatmulSegment::N);
+    pick(&MatmulSegment::col0);
+    pick(&MatmulSegment::unit0);
+    pick(&MatmulSegment::c);
+    pick(&MatmulSegment::ldc);
+    return r;
+}
 
 __device__ __forceinline__ half_t matmul_epilogue(const MatmulParams &p, float acc, int m, int n) {
     half_t v = (half_t)acc;

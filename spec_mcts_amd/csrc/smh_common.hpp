@@ -39,6 +39,33 @@ inline int launch_status() {
     return 0;
 }
 
+// Arguments of a kernel come by scalar loads, and the compiler asks for them where it needs them first: behind every early return and
+// every choice another trip to memory of ~0.35 us (three to nine of them before the matmuls' first request).  This asks for one word of each of the 64-byte
+// lines of the first BYTES at once, at the kernel's top; what is asked for later is in the scalar cache.  With the integer divisions
+// of the grids gone too (uniform_divmod, grids of two and three dimensions) a decode step of the 7B architecture took 2.64 ms instead of 2.73 at 37
+// branches, 3.45 instead of 3.56 at 100.
+template <int BYTES>
+__device__ __forceinline__ void args_ahead() {
+    static_assert(BYTES <= 384, "six lines");
+    auto k = (const __attribute__((address_space(4))) uint32_t *)__builtin_amdgcn_kernarg_segment_ptr();
+    constexpr int LAST = (BYTES - 1) / 64;
+    auto word = [&](int line) { return k[16 * (line < LAST ? line : LAST)]; };
+    asm volatile("" ::"s"(word(0)), "s"(word(1)), "s"(word(2)), "s"(word(3)), "s"(word(4)), "s"(word(5)));
+}
+// A value that the compiler has to have: it cannot turn a choice between two of them into a load from a chosen address
+template <class T>
+__device__ __forceinline__ T held(T v) {
+    asm("" : "+s"(v));
+    return v;
+}
+// i / n and i % n of non-negative numbers that all lanes share: eight instructions below 2^20, where the error of the float quotient stays under
+// the half that is added, instead of twenty-five
+struct DivMod { int q, r; };
+__device__ __forceinline__ DivMod uniform_divmod(int i, int n) {
+    const int q = i < 1 << 20 ? __builtin_amdgcn_readfirstlane((int)(((float)i + 0.5f) * __builtin_amdgcn_rcpf((float)n))) : i / n;
+    return DivMod{q, i - q * n};
+}
+
 // ---- bit casts ---------------------------------------------------------------------------------
 __device__ __forceinline__ h2 as_h2(uint32_t v) { return __builtin_bit_cast(h2, v); }
 __device__ __forceinline__ uint32_t as_u32(h2 v) { return __builtin_bit_cast(uint32_t, v); }
