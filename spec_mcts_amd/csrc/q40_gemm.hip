@@ -39,13 +39,13 @@ constexpr int GEMM_THREADS = GEMM_WAVES * 64;
 // slots of the DMA ring (with a barrier per step, four slots measured 2 % faster per launch at M=100 than six; with a
 // barrier per two steps, six slots are 3 % faster than that)
 constexpr int GEMM_STAGES = 6;
-// slots of the ring in the variant with a DMA wave, by row tiles, and the most workgroups of a launch that takes it (one per
-// compute unit).  Up to 48 rows a step is over before its successors have come from memory: with eight slots a decode step of
-// three layers of the 70B architecture takes 618 us at 17 branches against 700, 699 against 736 at 33, of the 7B architecture
-// 2.62 ms against 2.73 and 2.99 against 3.00; twelve slots as eight.  At 64 rows and more (64 x 11008 x 4096: 22.5 us against
-// 21.3) and in the kernels whose stages hold two steps (7B at 33 .. 64 branches: 1 % slower) six are better.
+// slots of the ring in the variant with DMA waves, by row tiles, and the most workgroups of a launch that takes it (one per
+// compute unit).  Up to 48 rows a step is over before its successors have come from memory: wq|wk|wv at 37 rows of the 7B shape takes 13.6 us with
+// six slots, 12.8 with eight and with twelve.  At 64 rows and more six are as good or better (wo, w2 at 512 rows 36.9, 37.4 and 37.7 us with six, eight and ten).
 constexpr int gemm_dma_slots(int tiles) { return tiles <= 3 ? 8 : 6; }
-constexpr int GEMM_PAIR_SLOTS = 6;
+// slots of the kernels whose stages hold two steps: up to `most`, as many as fit.  w1|w3 at 37 rows of the 7B shape 25.5 us with six, 21.6 with eight,
+// 22.0 with twelve; at 100 rows 30.0, 29.6.  The K-sliced kernel: at 37 rows 9.2 and 9.0, at 100 rows, where a slice has few stages, 16.6 and 17.0.
+constexpr int gemm_slots(int stage, int most) { return 160 * 1024 / stage < most ? 160 * 1024 / stage : most; }
 constexpr int GEMM_DMA_WAVE_MAX_WGS = 256;
 constexpr int GS_WBLOCK = 8 * 128 + 64;        // the 8 rows one wave fetches, padded by 16 banks: the four row groups a
                                                // ds_read_b32 touches (lanes 16g..16g+15 read row 8g+r) then sit in different banks
@@ -67,10 +67,15 @@ typedef __attribute__((address_space(3))) void *lptr_t;
 template <int N>
 __device__ __forceinline__ void gemm_wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N < 63 ? N : 63) : "memory"); }
 // ... at most `stages` younger stages of PER DMA instructions each (4 with four waves, 2 with eight, 5 + row tiles in
-// the DMA wave).
+// a DMA wave at most).
 template <int PER>
 __device__ __forceinline__ void gemm_wait_dma(int stages) {
     switch (stages) {
+        case 11: gemm_wait_vm<11 * PER>(); break;
+        case 10: gemm_wait_vm<10 * PER>(); break;
+        case 9: gemm_wait_vm<9 * PER>(); break;
+        case 8: gemm_wait_vm<8 * PER>(); break;
+        case 7: gemm_wait_vm<7 * PER>(); break;
         case 6: gemm_wait_vm<6 * PER>(); break;
         case 5: gemm_wait_vm<5 * PER>(); break;
         case 4: gemm_wait_vm<4 * PER>(); break;
@@ -84,6 +89,118 @@ __device__ __forceinline__ void gemm_wait_dma(int stages) {
 // A bare workgroup barrier.  Every LDS read this wave has issued has returned (lgkmcnt), so after the
 // barrier no wave still reads the stage that is refilled next.
 __device__ __forceinline__ void gemm_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// A DMA wave: it issues PER instructions of each of n stages (issue(slot): the next stage's) into a ring of SLOTS slots, waits for them and meets
+// the multiplying waves at their barriers, one per pair of stages (the protocol: gemm_piece).
+// A workgroup has GEMM_DMA_WAVES of these, each with a share of every stage.  One wave gets an instruction (1 KB) out every 32 - 40 cycles, two or more
+// together every 16, whatever rows the pieces lie in (measured from L2): with one, 22 instructions a stage of w1|w3 at 100 rows of
+// the 7B shape took 885 cycles, the same with the products taken out; with two 815, and 52 200 cycles for the 64 stages instead of 56 600.
+constexpr int GEMM_DMA_WAVES = 2;
+template <int PER, int SLOTS, class Issue>
+__device__ __forceinline__ void gemm_feed(int n, Issue issue) {
+    if (n <= 0) return;
+#pragma unroll 1
+    for (int i = 0; i < min(SLOTS - 2, n); ++i) issue(i);
+    gemm_wait_dma<PER>(min(SLOTS - 3, n - 1));
+    gemm_barrier();
+    int slot = 0;
+    auto back = [&](int k) { return slot >= k ? slot - k : slot + SLOTS - k; };
+    int i = 0;
+#pragma unroll 1
+    for (; i + SLOTS - 1 < n; i += 2) {
+        gemm_wait_vm<PER * (SLOTS - 5)>();
+        gemm_barrier();
+        issue(back(2));
+        issue(back(1));
+        slot = slot + 2 >= SLOTS ? slot + 2 - SLOTS : slot + 2;
+    }
+#pragma unroll 1
+    for (; i < n; i += 2) {
+        gemm_wait_dma<PER>(max(0, min(n - 1, i + SLOTS - 3) - (i + 2)));      // stages issued past stage i + 2
+        gemm_barrier();
+        if (i + SLOTS - 2 < n) issue(back(2));
+        if (i + SLOTS - 1 < n) issue(back(1));
+        slot = slot + 2 >= SLOTS ? slot + 2 - SLOTS : slot + 2;
+    }
+}
+template <int N> using int_constant = std::integral_constant<int, N>;
+
+// The products of one multiplying wave of the kernels below: n stages of a ring of SLOTS slots, B operands (one nibble of one piece, 16 columns of either
+// byte) x TILES row tiles.  A wave keeps the A rows and the B operands of ONE stage in registers.  As soon as a row tile's two products are
+// issued its registers take the next stage's rows, and the next nibbles, read first, are decoded between the products: no read is waited for where it
+// was issued.  Left to the compiler each pair of products waited for its own read - with the products 780 cycles a stage of 112 rows x 128 columns x 64,
+// 448 of them on the matrix pipe.
+// Stages go in pairs, one barrier a pair (gemm_feed): at the barrier before stages i, i + 1 the stages up to i + 2 have landed, whose rows
+// and nibbles stage i + 1 reads; past the last stage stale bytes are read, decoded and never used.
+template <int TILES, int SLOTS, int STAGE, bool SPREAD = true>
+__device__ __forceinline__ void gemm_multiply(const uint8_t *lds, int n, int hh, int ws_off, int sc_off, int a_off, f4 (&acc)[2][TILES]) {
+    const uint32_t nib_mask = hh == 0 ? 0x00F000F0u : 0x000F000Fu;
+    uint32_t nib_magic = MAGIC_1024;                             // in a register the compiler cannot see through: (bits & mask) | magic is
+    asm volatile("" : "+v"(nib_magic));                       // then ONE v_and_or_b32 (no literal operands there), not an AND and an OR
+    const h2 nib_mul = hh == 0 ? h2{(half_t)0.0625f, (half_t)0.0625f} : h2{(half_t)1.0f, (half_t)1.0f};
+    const h2 nib_off = hh == 0 ? h2{(half_t)-72.0f, (half_t)-72.0f} : h2{(half_t)-1032.0f, (half_t)-1032.0f};
+    // half a row pair of the operands: rows (2 j, 2 j + 1) of the piece's first (o = 0) or second byte, codes + 8 -> exact fp16 code * scale
+    auto decode = [&](const u32x4 &wq, const u32x4 &scales, int j, int o, u32x4 (&b)[2]) {
+        const uint32_t w = wq[(j & 1) + 2 * o], pr = j < 2 ? w : w >> 8;
+        b[o][j] = as_u32(__builtin_elementwise_fma(as_h2((pr & nib_mask) | nib_magic), nib_mul, nib_off) * as_h2(scales[j]));
+    };
+#pragma unroll
+    for (int o = 0; o < 2; ++o)
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) acc[o][t] = f4{0.f, 0.f, 0.f, 0.f};
+    if (n <= 0) return;
+    h8 av[TILES];
+    u32x4 bq[2];
+    gemm_barrier();
+    {
+        const u32x4 wq = *reinterpret_cast<const u32x4 *>(lds + ws_off), scales = *reinterpret_cast<const u32x4 *>(lds + sc_off);
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) av[t] = *reinterpret_cast<const h8 *>(lds + a_off + t * 1024);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) decode(wq, scales, u >> 1, u & 1, bq);
+    }
+    int slot = 0;
+    auto one_stage = [&]() {
+        slot = slot == SLOTS - 1 ? 0 : slot + 1;
+        const uint8_t *st = lds + slot * STAGE;                // of the next stage
+        const u32x4 wq = *reinterpret_cast<const u32x4 *>(st + ws_off), scales = *reinterpret_cast<const u32x4 *>(st + sc_off);
+        __builtin_amdgcn_sched_barrier(0);
+        u32x4 bn[2];
+        constexpr int FROM = TILES >= 4 ? 2 : TILES - 1;       // the row tile under whose products the decode begins
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+#pragma unroll
+            for (int o = 0; o < 2; ++o) acc[o][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[t], __builtin_bit_cast(h8, bq[o]), acc[o][t], 0, 0, 0);
+            av[t] = *reinterpret_cast<const h8 *>(st + a_off + t * 1024);
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (t == FROM + u * (TILES - FROM) / 8) {
+                    decode(wq, scales, u >> 1, u & 1, bn);
+                    if constexpr (SPREAD) asm volatile("" : "+v"(bn[u & 1][u >> 1]));      // (here, not where it is needed)
+                }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        bq[0] = bn[0];
+        bq[1] = bn[1];
+    };
+    // The slots that are refilled behind a barrier were read a stage ago, by reads older than the last stage's TILES + 2
+    auto meet = [] {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt lgkmcnt(%0)\n\ts_barrier" ::"n"(TILES + 2) : "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    int i = 0;
+#pragma unroll 1
+    for (; i + 1 < n; i += 2) {
+        meet();
+        one_stage();
+        one_stage();
+    }
+    if (i < n) {
+        meet();
+        one_stage();
+    }
+}
 
 // TILED: the weights are in the tiled layout (q40_matmul.hpp).  Wave w then moves and decodes piece w of a
 // tile (its two byte positions of its block, already paired by rows): one 16-byte LDS read instead of eight
@@ -217,10 +334,10 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
         fetch = fetch + 1 == step1 ? step0 : fetch + 1;
     };
     if constexpr (PRODUCER) {
-        if (wave8 == 8) {
-            // ---- the DMA wave: 5 + TILES instructions a stage (four pieces of nibbles, the scales, one per 16 rows of A) ----
-            constexpr int PER = 5 + TILES;
-            __builtin_amdgcn_s_setprio(3);      // its few instructions first: the others wait for what it requests (3 % of a launch)
+        if (wave8 >= 8) {
+            // ---- the DMA waves: 5 + TILES instructions a stage (four pieces of nibbles, the scales, one per 16 rows of A) ----
+            constexpr int A_FIRST = TILES > 5 ? (TILES - 5) / 2 : 0;   // row tiles that go with the weights, so that the two have as many to issue
+            __builtin_amdgcn_s_setprio(3);      // their few instructions first: the others wait for what they request (3 % of a launch)
             uint32_t a_voff[TILES];
 #pragma unroll
             for (int t = 0; t < TILES; ++t)
@@ -231,10 +348,14 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
             const uint32_t raw_w = (uint32_t)((lane >> 3) * w_row + w_lcol), raw_s = (uint32_t)((lane >> 1) * s_row + s_lcol);
             const uint32_t raw_s_last = RAGGED ? (uint32_t)(min(lane >> 1, left - 1) * s_row + s_lcol) : 0;
             const uint32_t a_back = RAGGED ? (uint32_t)(2 * (8 * a_chunk - min(8 * a_chunk, left - 8))) : 0;
-            auto issue_all = [&](int slot_) {
+            auto feed = [&](auto which) {
+            constexpr bool WEIGHTS = decltype(which)::value == 0;
+            constexpr int T0 = WEIGHTS ? 0 : A_FIRST, T1 = WEIGHTS ? A_FIRST : TILES;
+            gemm_feed<(WEIGHTS ? 5 : 0) + T1 - T0, SLOTS>(n_steps, [&](int slot_) {
                 uint8_t *st = lds + slot_ * GS_BYTES;
                 const uint8_t *arow = a_base + (long)fetch * 64;
-                if (TILED) {
+                if constexpr (!WEIGHTS) {
+                } else if (TILED) {
                     const uint8_t *tile = w_base + (long)fetch * TILE_BYTES;
 #pragma unroll
                     for (int q = 0; q < 4; ++q)
@@ -250,37 +371,14 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
                     __builtin_amdgcn_global_load_lds((gptr_t)(s_base + (long)fetch * 32 * s_row + (at_end ? raw_s_last : raw_s)), (lptr_t)(st + GS_W), 4, 0, 0);
                 }
 #pragma unroll
-                for (int t = 0; t < TILES; ++t)
+                for (int t = T0; t < T1; ++t)
                     __builtin_amdgcn_global_load_lds((gptr_t)(arow + (RAGGED && fetch == last ? a_voff[t] - a_back : a_voff[t])),
                                                      (lptr_t)(st + GS_W + GS_S + t * 1024), 16, 0, 0);
                 fetch = fetch + 1 == step1 ? step0 : fetch + 1;
+            });
             };
-#pragma unroll
-            for (int i = 0; i < SLOTS - 2; ++i)
-                if (i < n_steps) issue_all(i);
-            if (n_steps > 0) {
-                gemm_wait_dma<PER>(min(SLOTS - 3, n_steps - 1));
-                gemm_barrier();
-                int slot = 0;
-                auto back = [&](int k) { return slot >= k ? slot - k : slot + SLOTS - k; };
-                int i = 0;
-#pragma unroll 1
-                for (; i + SLOTS - 1 < n_steps; i += 2) {
-                    gemm_wait_vm<PER * (SLOTS - 5)>();
-                    gemm_barrier();
-                    issue_all(back(2));
-                    issue_all(back(1));
-                    slot = slot + 2 >= SLOTS ? slot + 2 - SLOTS : slot + 2;
-                }
-#pragma unroll 1
-                for (; i < n_steps; i += 2) {
-                    gemm_wait_dma<PER>(max(0, min(n_steps - 1, i + SLOTS - 3) - (i + 2)));      // stages issued past step i + 2
-                    gemm_barrier();
-                    if (i + SLOTS - 2 < n_steps) issue_all(back(2));
-                    if (i + SLOTS - 1 < n_steps) issue_all(back(1));
-                    slot = slot + 2 >= SLOTS ? slot + 2 - SLOTS : slot + 2;
-                }
-            }
+            if (wave8 == 8) feed(int_constant<0>{});
+            else feed(int_constant<1>{});
             // the barriers of the epilogue: one that frees the ring, one per row tile
 #pragma unroll 1
             for (int t = 0; t < 1 + TILES + (more ? 1 : 0); ++t) gemm_barrier();
@@ -422,11 +520,14 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
             for (int o = 0; o < NB; ++o) acc[o][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[t], b[o], acc[o][t], 0, 0, 0);
         }
     };
-    // Steps go in pairs: ONE wait + barrier per two steps.  With S slots (six; more only with the DMA wave): at the barrier
+    // Steps go in pairs: ONE wait + barrier per two steps.  With S slots (six; more only with the DMA waves): at the barrier
     // before steps i, i+1 the stages of steps i .. i+2 have landed (the B operands of step i+2 are decoded during step i+1),
     // steps i+3 .. i+S-3 may be in flight, and the slots of steps i-2, i-1 are refilled with steps i+S-2, i+S-1.  A stage has the same two steps of time to land as
     // with a barrier per step; the waves meet half as often.
-    if (n_steps > 0) {
+    if constexpr (PRODUCER && TILED && !RAGGED) {
+        gemm_multiply<TILES, SLOTS, GS_BYTES>(lds, n_steps, hh, wave * 1024 + lane * 16, GS_W + g * 64 + (2 * blk + hh) * 16,
+                                              GS_W + GS_S + c * 64 + ((g ^ ((c >> 1) & 3)) << 4), acc);
+    } else if (n_steps > 0) {
         h8 bq[NB];
         int cur = step0 + rot;                 // step being multiplied
         int slot = 0;                          // its ring slot
@@ -605,18 +706,18 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
     if (more) gemm_barrier();                   // the next piece refills the ring the last row tile left through
 }
 
-// PRODUCER (eight waves only): a ninth wave issues every DMA instruction of the workgroup and waits for them; the eight
-// others only meet it at the barriers.  The compute unit's address unit takes 16 cycles per DMA instruction, during which
+// PRODUCER (eight waves only): two more waves issue every DMA instruction of the workgroup and wait for them; the eight
+// others only meet them at the barriers.  The compute unit's address unit takes 16 cycles per DMA instruction, during which
 // the issuing wave stands still: ~0.28 us per pair of steps off the multiplying waves' path.  For launches with one
-// workgroup per compute unit (a ninth and tenth wave on a SIMD that already holds four would cap the registers below
+// workgroup per compute unit (more waves on a SIMD that already holds four would cap the registers below
 // what the kernel needs).  SLOTS: slots of the ring.
 // RANGE (p.chunk > 0): the steps of all column units, laid end to end, are dealt in runs of p.chunk to the workgroups, one
 // workgroup per compute unit, so a workgroup may finish one unit and begin the next: up to two pieces, one after the other.
 template <int TILES, bool RAGGED, bool TILED, int WAVES, int SLOTS = GEMM_STAGES, bool PRODUCER = false, bool RANGE = false, bool SWIGLU = false>
-// (SWIGLU without the DMA wave: at most 128 registers, so that two workgroups of eight waves fit a compute unit)
-__global__ __launch_bounds__(64 * (WAVES + (PRODUCER ? 1 : 0)), WAVES == 8 ? (SWIGLU && !PRODUCER ? 4 : 1) : 2) void q40_gemm_kernel(MatmulParams p) {
-    static_assert(WAVES == 4 || (WAVES == 8 && (TILED ? !RAGGED : PRODUCER)), "eight waves: K a multiple of 32, or the checkpoint layout with a DMA wave");
-    static_assert(SLOTS >= 6 && SLOTS <= 8 && (SLOTS == GEMM_STAGES || PRODUCER) && (!PRODUCER || WAVES == 8), "ring depth");
+// (SWIGLU without the DMA waves: at most 128 registers, so that two workgroups of eight waves fit a compute unit)
+__global__ __launch_bounds__(64 * (WAVES + (PRODUCER ? GEMM_DMA_WAVES : 0)), WAVES == 8 ? (SWIGLU && !PRODUCER ? 4 : 1) : 2) void q40_gemm_kernel(MatmulParams p) {
+    static_assert(WAVES == 4 || (WAVES == 8 && (TILED ? !RAGGED : PRODUCER)), "eight waves: K a multiple of 32, or the checkpoint layout with the DMA waves");
+    static_assert(SLOTS >= 6 && SLOTS <= 12 && (SLOTS == GEMM_STAGES || PRODUCER) && (!PRODUCER || WAVES == 8), "ring depth");
     args_ahead<sizeof(MatmulParams)>();
     const int steps_total = (p.K + 31) / 32;
     if constexpr (RANGE) {
@@ -661,9 +762,9 @@ constexpr int KG_W = 4096;                     // [group kk][piece bp] x 1024
 constexpr int KG_S = 512;                      // [group kk] x 256 (the whole scale block of the step)
 template <int TILES> struct KgShape {
     static constexpr int STAGE = KG_W + KG_S + 2 * TILES * 1024;
-    static constexpr int SLOTS = GEMM_PAIR_SLOTS;
+    static constexpr int SLOTS = gemm_slots(STAGE, TILES <= 4 ? 8 : 6);
     static constexpr int RING = SLOTS * STAGE;
-    static constexpr int PER = 2 * (3 + TILES);                    // DMA instructions of a stage
+    static constexpr int PER = 3 + TILES;                          // DMA instructions of a step
     static constexpr int OP = 128 + 4;                             // floats per row of a group's sums in LDS
     static constexpr int SUMS = TILES * 16 * OP * 4;               // one K-group's sums: [row][OP] fp32
     static constexpr int LDS = RING > 2 * SUMS ? RING : 2 * SUMS;
@@ -671,12 +772,12 @@ template <int TILES> struct KgShape {
 };
 
 template <int TILES>
-__global__ __launch_bounds__(576, 1) void q40_gemm_kg_kernel(MatmulParams p) {
+__global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_kg_kernel(MatmulParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     typedef KgShape<TILES> S;
     constexpr int SLOTS = S::SLOTS, PER = S::PER, STAGE = S::STAGE;
     const int tid = threadIdx.x;
-    const int wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);       // 0..7 multiply, 8 issues the DMA
+    const int wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);       // 0..7 multiply, the others issue the DMA
     const int lane = tid & 63, c = lane & 15, g = lane >> 4;
     args_ahead<sizeof(MatmulParams)>();
     // blockIdx -> (128-column block, row block, K-slice); blocks of one unit are neighbours (same XCD every 8)
@@ -700,8 +801,8 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_kg_kernel(MatmulParams p) {
     const uint8_t *a_base = reinterpret_cast<const uint8_t *>(p.a) + (long)step0 * 64;
     const int rot = n_st > 0 ? uniform_divmod(hb * 5, n_st).r : 0;             // workgroups of a K-slice start at different stages
 
-    if (wave8 == 8) {
-        // ---- the DMA wave ----
+    if (wave8 >= 8) {
+        // ---- the DMA waves: a K-group's steps each ----
         __builtin_amdgcn_s_setprio(3);
         const int a_chunk = (lane & 3) ^ ((lane >> 3) & 3);
         uint32_t a_voff[TILES];
@@ -709,10 +810,10 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_kg_kernel(MatmulParams p) {
         for (int t = 0; t < TILES; ++t)
             a_voff[t] = (uint32_t)((long)min(m0 + 16 * t + (lane >> 2), p.M - 1) * p.lda * 2 + 16 * a_chunk);
         int fetch = rot;
-        auto issue_stage = [&](int slot_) {
+        const int kk = wave8 - 8;
+        gemm_feed<PER, SLOTS>(n_st, [&](int slot_) {
             uint8_t *st = lds + slot_ * STAGE;
-#pragma unroll
-            for (int kk = 0; kk < 2; ++kk) {
+            {
                 const uint8_t *tile = w_base + (long)(2 * fetch + kk) * TILE_BYTES;
                 const uint8_t *arow = a_base + (long)(2 * fetch + kk) * 64;
 #pragma unroll
@@ -724,112 +825,16 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_kg_kernel(MatmulParams p) {
                     __builtin_amdgcn_global_load_lds((gptr_t)(arow + a_voff[t]), (lptr_t)(st + KG_W + KG_S + (kk * TILES + t) * 1024), 16, 0, 0);
             }
             fetch = fetch + 1 == n_st ? 0 : fetch + 1;
-        };
-#pragma unroll
-        for (int i = 0; i < SLOTS - 2; ++i)
-            if (i < n_st) issue_stage(i);
-        if (n_st > 0) {
-            gemm_wait_dma<PER>(min(SLOTS - 3, n_st - 1));
-            gemm_barrier();
-            int slot = 0;
-            auto back = [&](int k) { return slot >= k ? slot - k : slot + SLOTS - k; };
-            int i = 0;
-#pragma unroll 1
-            for (; i + SLOTS - 1 < n_st; i += 2) {
-                gemm_wait_vm<PER * (SLOTS - 5)>();
-                gemm_barrier();
-                issue_stage(back(2));
-                issue_stage(back(1));
-                slot = slot + 2 >= SLOTS ? slot + 2 - SLOTS : slot + 2;
-            }
-#pragma unroll 1
-            for (; i < n_st; i += 2) {
-                gemm_wait_dma<PER>(max(0, min(n_st - 1, i + SLOTS - 3) - (i + 2)));
-                gemm_barrier();
-                if (i + SLOTS - 2 < n_st) issue_stage(back(2));
-                if (i + SLOTS - 1 < n_st) issue_stage(back(1));
-                slot = slot + 2 >= SLOTS ? slot + 2 - SLOTS : slot + 2;
-            }
-        }
+        });
         gemm_barrier();                                        // the epilogue's two barriers: ring free, sums in place
         gemm_barrier();
         return;
     }
 
     const int kk = wave8 >> 2, hh = (wave8 >> 1) & 1, bp = wave8 & 1;
-    const uint32_t nib_mask = hh == 0 ? 0x00F000F0u : 0x000F000Fu;
-    uint32_t nib_magic = MAGIC_1024;                             // in a register the compiler cannot see through: (bits & mask) | magic is
-    asm volatile("" : "+v"(nib_magic));                       // then ONE v_and_or_b32 (no literal operands there), not an AND and an OR
-    const h2 nib_mul = hh == 0 ? h2{(half_t)0.0625f, (half_t)0.0625f} : h2{(half_t)1.0f, (half_t)1.0f};
-    const h2 nib_off = hh == 0 ? h2{(half_t)-72.0f, (half_t)-72.0f} : h2{(half_t)-1032.0f, (half_t)-1032.0f};
-    struct Raw { u32x4 wq, sc; };
-    auto load_ws = [&](const uint8_t *st, Raw &r) {
-        r.wq = *reinterpret_cast<const u32x4 *>(st + (2 * kk + bp) * 1024 + lane * 16);
-        r.sc = *reinterpret_cast<const u32x4 *>(st + KG_W + kk * 256 + g * 64 + (2 * blk + hh) * 16);
-    };
-    auto decode = [&](const Raw &r, h8 (&b)[2]) {
-        u32x4 v0, v1;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t pr0 = j < 2 ? r.wq[j] : r.wq[j - 2] >> 8;       // rows (2j, 2j+1) of byte 2bp, codes + 8
-            const uint32_t pr1 = j < 2 ? r.wq[2 + j] : r.wq[j] >> 8;       // ... of byte 2bp+1
-            const h2 sc = as_h2(r.sc[j]);
-            v0[j] = as_u32(__builtin_elementwise_fma(as_h2((pr0 & nib_mask) | nib_magic), nib_mul, nib_off) * sc);
-            v1[j] = as_u32(__builtin_elementwise_fma(as_h2((pr1 & nib_mask) | nib_magic), nib_mul, nib_off) * sc);
-        }
-        b[0] = __builtin_bit_cast(h8, v0);
-        b[1] = __builtin_bit_cast(h8, v1);
-    };
-    auto load_a = [&](const uint8_t *st, h8 (&av)[TILES]) {
-        const uint8_t *at = st + KG_W + KG_S + kk * TILES * 1024;
-#pragma unroll
-        for (int t = 0; t < TILES; ++t) {
-            const int r = 16 * t + c;
-            av[t] = *reinterpret_cast<const h8 *>(at + r * 64 + ((g ^ ((r >> 1) & 3)) << 4));
-        }
-    };
     f4 acc[2][TILES];
-#pragma unroll
-    for (int o = 0; o < 2; ++o)
-#pragma unroll
-        for (int t = 0; t < TILES; ++t) acc[o][t] = f4{0.f, 0.f, 0.f, 0.f};
-
-    if (n_st > 0) {
-        h8 bq[2];
-        int slot = 0;
-        gemm_barrier();
-        {
-            Raw r;
-            load_ws(lds, r);
-            decode(r, bq);
-        }
-        auto one_stage = [&]() {
-            const uint8_t *st = lds + slot * STAGE;
-            slot = slot == SLOTS - 1 ? 0 : slot + 1;
-            Raw r;
-            h8 av[TILES], bn[2];
-            load_a(st, av);
-            load_ws(lds + slot * STAGE, r);                    // (past the last stage: stale bytes, decoded and never used)
-#pragma unroll
-            for (int t = 0; t < TILES; ++t)
-#pragma unroll
-                for (int o = 0; o < 2; ++o) acc[o][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[t], bq[o], acc[o][t], 0, 0, 0);
-            decode(r, bn);
-            bq[0] = bn[0];
-            bq[1] = bn[1];
-        };
-        int i = 0;
-#pragma unroll 1
-        for (; i + 1 < n_st; i += 2) {
-            gemm_barrier();
-            one_stage();
-            one_stage();
-        }
-        if (i < n_st) {
-            gemm_barrier();
-            one_stage();
-        }
-    }
+    gemm_multiply<TILES, SLOTS, STAGE>(lds, n_st, hh, (2 * kk + bp) * 1024 + lane * 16, KG_W + kk * 256 + g * 64 + (2 * blk + hh) * 16,
+                                       KG_W + KG_S + kk * TILES * 1024 + c * 64 + ((g ^ ((c >> 1) & 3)) << 4), acc);
 
     // ---- both groups' sums as rows of 128 floats in LDS; then every thread adds group 0 + group 1 (a fixed order) for
     // 16-byte runs of whole rows and writes the slab: one pass, two barriers, all eight waves storing ----
@@ -867,23 +872,22 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_kg_kernel(MatmulParams p) {
 template <int TILES> struct SwigluShape {
     static constexpr int SC = 1024;                                  // scales: [group kk][gate | up] x 256
     static constexpr int STAGE = KG_W + SC + 2 * TILES * 1024;
-    static constexpr int SLOTS = GEMM_PAIR_SLOTS;
+    static constexpr int SLOTS = gemm_slots(STAGE, 8);
     static constexpr int LDS = SLOTS * STAGE;
-    static constexpr int PER = 2 * (4 + TILES);
-    static constexpr int RED = 4 * TILES * 2 * 1024;
-    static constexpr int OP = 64 + 4;
-    static constexpr int OTILE = 2 * 16 * OP * 4;
-    static_assert(RED + 2 * OTILE <= LDS, "the sums of the second group and two output tiles must fit in the ring");
+    static constexpr int PER = 4 + TILES;                            // DMA instructions of a step
+    static constexpr int OP = 128 + 4;                               // floats per row of a group's sums in LDS
+    static constexpr int SUMS = TILES * 16 * OP * 4;                 // one K-group's sums: [row][gate | up] fp32
+    static_assert(2 * SUMS <= LDS, "both groups' sums must fit in the ring");
     static_assert(PER * (SLOTS - 5) <= 63 && LDS <= 160 * 1024, "ring");
 };
 
 template <int TILES>
-__global__ __launch_bounds__(576, 1) void q40_gemm_swiglu_kernel(MatmulParams p) {
+__global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_swiglu_kernel(MatmulParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     typedef SwigluShape<TILES> S;
     constexpr int SLOTS = S::SLOTS, PER = S::PER, STAGE = S::STAGE;
     const int tid = threadIdx.x;
-    const int wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);       // 0..7 multiply, 8 issues the DMA
+    const int wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);       // 0..7 multiply, the others issue the DMA
     const int lane = tid & 63, c = lane & 15, g = lane >> 4;
     args_ahead<sizeof(MatmulParams)>();
     // blockIdx -> (128-column block j of the gate and of the up weight, piece bp of that block)
@@ -899,8 +903,8 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_swiglu_kernel(MatmulParams p)
     const uint8_t *a_base = reinterpret_cast<const uint8_t *>(p.a);
     const int rot = n_st > 0 ? uniform_divmod(hb * 5, n_st).r : 0;             // workgroups of a K-slice start at different stages
 
-    if (wave8 == 8) {
-        // ---- the DMA wave ----
+    if (wave8 >= 8) {
+        // ---- the DMA waves: a K-group's steps each ----
         __builtin_amdgcn_s_setprio(3);
         const int a_chunk = (lane & 3) ^ ((lane >> 3) & 3);
         uint32_t a_voff[TILES];
@@ -908,10 +912,10 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_swiglu_kernel(MatmulParams p)
         for (int t = 0; t < TILES; ++t)
             a_voff[t] = (uint32_t)((long)min(m0 + 16 * t + (lane >> 2), p.M - 1) * p.lda * 2 + 16 * a_chunk);
         int fetch = rot;
-        auto issue_stage = [&](int slot_) {
+        const int kk = wave8 - 8;
+        gemm_feed<PER, SLOTS>(n_st, [&](int slot_) {
             uint8_t *st = lds + slot_ * STAGE;
-#pragma unroll
-            for (int kk = 0; kk < 2; ++kk) {
+            {
                 const long off = (long)(2 * fetch + kk) * TILE_BYTES;
                 const uint8_t *arow = a_base + (long)(2 * fetch + kk) * 64;
 #pragma unroll
@@ -925,162 +929,47 @@ __global__ __launch_bounds__(576, 1) void q40_gemm_swiglu_kernel(MatmulParams p)
                     __builtin_amdgcn_global_load_lds((gptr_t)(arow + a_voff[t]), (lptr_t)(st + KG_W + S::SC + (kk * TILES + t) * 1024), 16, 0, 0);
             }
             fetch = fetch + 1 == n_st ? 0 : fetch + 1;
-        };
-#pragma unroll
-        for (int i = 0; i < SLOTS - 2; ++i)
-            if (i < n_st) issue_stage(i);
-        if (n_st > 0) {
-            gemm_wait_dma<PER>(min(SLOTS - 3, n_st - 1));
-            gemm_barrier();
-            int slot = 0;
-            auto back = [&](int k) { return slot >= k ? slot - k : slot + SLOTS - k; };
-            int i = 0;
-#pragma unroll 1
-            for (; i + SLOTS - 1 < n_st; i += 2) {
-                gemm_wait_vm<PER * (SLOTS - 5)>();
-                gemm_barrier();
-                issue_stage(back(2));
-                issue_stage(back(1));
-                slot = slot + 2 >= SLOTS ? slot + 2 - SLOTS : slot + 2;
-            }
-#pragma unroll 1
-            for (; i < n_st; i += 2) {
-                gemm_wait_dma<PER>(max(0, min(n_st - 1, i + SLOTS - 3) - (i + 2)));
-                gemm_barrier();
-                if (i + SLOTS - 2 < n_st) issue_stage(back(2));
-                if (i + SLOTS - 1 < n_st) issue_stage(back(1));
-                slot = slot + 2 >= SLOTS ? slot + 2 - SLOTS : slot + 2;
-            }
-        }
-        // the barriers of the epilogue: ring free, second group's sums in place, one per row tile
-#pragma unroll 1
-        for (int t = 0; t < 2 + TILES; ++t) gemm_barrier();
+        });
+        gemm_barrier();                                        // the epilogue's two barriers: ring free, sums in place
+        gemm_barrier();
         return;
     }
 
     const int kk = wave8 >> 2, hh = (wave8 >> 1) & 1, gu = wave8 & 1;       // K-group, nibble, gate (0) or up (1)
-    const uint32_t nib_mask = hh == 0 ? 0x00F000F0u : 0x000F000Fu;
-    uint32_t nib_magic = MAGIC_1024;                             // in a register the compiler cannot see through: (bits & mask) | magic is
-    asm volatile("" : "+v"(nib_magic));                       // then ONE v_and_or_b32 (no literal operands there), not an AND and an OR
-    const h2 nib_mul = hh == 0 ? h2{(half_t)0.0625f, (half_t)0.0625f} : h2{(half_t)1.0f, (half_t)1.0f};
-    const h2 nib_off = hh == 0 ? h2{(half_t)-72.0f, (half_t)-72.0f} : h2{(half_t)-1032.0f, (half_t)-1032.0f};
-    struct Raw { u32x4 wq, sc; };
-    auto load_ws = [&](const uint8_t *st, Raw &r) {
-        r.wq = *reinterpret_cast<const u32x4 *>(st + (2 * kk + gu) * 1024 + lane * 16);
-        r.sc = *reinterpret_cast<const u32x4 *>(st + KG_W + (2 * kk + gu) * 256 + g * 64 + (2 * blk + hh) * 16);
-    };
-    auto decode = [&](const Raw &r, h8 (&b)[2]) {
-        u32x4 v0, v1;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t pr0 = j < 2 ? r.wq[j] : r.wq[j - 2] >> 8;       // rows (2j, 2j+1) of byte 2bp, codes + 8
-            const uint32_t pr1 = j < 2 ? r.wq[2 + j] : r.wq[j] >> 8;       // ... of byte 2bp+1
-            const h2 sc = as_h2(r.sc[j]);
-            v0[j] = as_u32(__builtin_elementwise_fma(as_h2((pr0 & nib_mask) | nib_magic), nib_mul, nib_off) * sc);
-            v1[j] = as_u32(__builtin_elementwise_fma(as_h2((pr1 & nib_mask) | nib_magic), nib_mul, nib_off) * sc);
-        }
-        b[0] = __builtin_bit_cast(h8, v0);
-        b[1] = __builtin_bit_cast(h8, v1);
-    };
-    auto load_a = [&](const uint8_t *st, h8 (&av)[TILES]) {
-        const uint8_t *at = st + KG_W + S::SC + kk * TILES * 1024;
-#pragma unroll
-        for (int t = 0; t < TILES; ++t) {
-            const int r = 16 * t + c;
-            av[t] = *reinterpret_cast<const h8 *>(at + r * 64 + ((g ^ ((r >> 1) & 3)) << 4));
-        }
-    };
     f4 acc[2][TILES];
-#pragma unroll
-    for (int o = 0; o < 2; ++o)
-#pragma unroll
-        for (int t = 0; t < TILES; ++t) acc[o][t] = f4{0.f, 0.f, 0.f, 0.f};
+    gemm_multiply<TILES, SLOTS, STAGE>(lds, n_st, hh, (2 * kk + gu) * 1024 + lane * 16, KG_W + (2 * kk + gu) * 256 + g * 64 + (2 * blk + hh) * 16,
+                                       KG_W + S::SC + kk * TILES * 1024 + c * 64 + ((g ^ ((c >> 1) & 3)) << 4), acc);
 
-    if (n_st > 0) {
-        h8 bq[2];
-        int slot = 0;
-        gemm_barrier();
-        {
-            Raw r;
-            load_ws(lds, r);
-            decode(r, bq);
-        }
-        auto one_stage = [&]() {
-            const uint8_t *st = lds + slot * STAGE;
-            slot = slot == SLOTS - 1 ? 0 : slot + 1;
-            Raw r;
-            h8 av[TILES], bn[2];
-            load_a(st, av);
-            load_ws(lds + slot * STAGE, r);                    // (past the last stage: stale bytes, decoded and never used)
-#pragma unroll
-            for (int t = 0; t < TILES; ++t)
-#pragma unroll
-                for (int o = 0; o < 2; ++o) acc[o][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[t], bq[o], acc[o][t], 0, 0, 0);
-            decode(r, bn);
-            bq[0] = bn[0];
-            bq[1] = bn[1];
-        };
-        int i = 0;
-#pragma unroll 1
-        for (; i + 1 < n_st; i += 2) {
-            gemm_barrier();
-            one_stage();
-            one_stage();
-        }
-        if (i < n_st) {
-            gemm_barrier();
-            one_stage();
-        }
-    }
-
-    // ---- group 0 + group 1 through LDS, then the slab one row tile at a time ----
+    // ---- both groups' sums as rows of 64 gate and 64 up columns in LDS, then every thread adds group 0 + group 1 (a fixed order) of four columns ----
+    // local column 32 hh + 2 c + o is column 128 blockj + 64 hh + 4 c + 2 bp + o of the weights
     gemm_barrier();                                            // every wave has left the loop: the ring is free
-    if (kk == 1) {
-        uint8_t *dst = lds + (wave8 - 4) * (TILES * 2 * 1024) + lane * 16;
+    constexpr int OP = S::OP;
+    {
+        float *sums = reinterpret_cast<float *>(lds + kk * S::SUMS) + 64 * gu + 32 * hh + 2 * c;
 #pragma unroll
         for (int t = 0; t < TILES; ++t)
 #pragma unroll
-            for (int o = 0; o < 2; ++o) *reinterpret_cast<f4 *>(dst + (t * 2 + o) * 1024) = acc[o][t];
+            for (int r = 0; r < 4; ++r) *reinterpret_cast<f2 *>(&sums[(16 * t + 4 * g + r) * OP]) = f2{acc[0][t][r], acc[1][t][r]};
     }
     gemm_barrier();
-    if (kk == 1) {
-#pragma unroll 1
-        for (int t = 0; t < TILES; ++t) gemm_barrier();
-        return;
-    }
-    {
-        const uint8_t *src = lds + wave8 * (TILES * 2 * 1024) + lane * 16;
+    const float *sum0 = reinterpret_cast<const float *>(lds), *sum1 = reinterpret_cast<const float *>(lds + S::SUMS);
+    const int cq = 4 * (tid & 15), out_col = 128 * blockj + 64 * ((tid & 15) >> 3) + 4 * (2 * (tid & 7)) + 2 * bp;      // tid < 512 here
 #pragma unroll
-        for (int t = 0; t < TILES; ++t)
+    for (int row = tid >> 4; row < 16 * TILES; row += 32) {
+        if (row >= p.M) break;
+        const int at = row * OP + cq;
+        const f4 gv = *reinterpret_cast<const f4 *>(sum0 + at) + *reinterpret_cast<const f4 *>(sum1 + at);
+        const f4 uv = *reinterpret_cast<const f4 *>(sum0 + at + 64) + *reinterpret_cast<const f4 *>(sum1 + at + 64);
+        half_t ov[4];
 #pragma unroll
-            for (int o = 0; o < 2; ++o) acc[o][t] += *reinterpret_cast<const f4 *>(src + (t * 2 + o) * 1024);
-    }
-    // rows of 64 columns: local column 32 hh + 2 c + o is column 128 blockj + 64 hh + 4 c + 2 bp + o of the weights
-    constexpr int OP = S::OP;
-    const int o_row = tid >> 4, o_lane = tid & 15;            // tid < 256 here
-    const int st_hh = o_lane >> 3, st_c = 2 * (o_lane & 7);   // this thread's four local columns 4 o_lane .. + 3 when storing
-#pragma unroll
-    for (int t = 0; t < TILES; ++t) {
-        float *otile = reinterpret_cast<float *>(lds + S::RED + (t & 1) * S::OTILE);      // [gate | up][16][OP]
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-            *reinterpret_cast<f2 *>(&otile[gu * 16 * OP + (4 * g + r) * OP + 32 * hh + 2 * c]) = f2{acc[0][t][r], acc[1][t][r]};
-        gemm_barrier();
-        const int m = 16 * t + o_row;
-        if (m < p.M) {
-            const f4 gv = *reinterpret_cast<const f4 *>(otile + o_row * OP + 4 * o_lane);
-            const f4 uv = *reinterpret_cast<const f4 *>(otile + 16 * OP + o_row * OP + 4 * o_lane);
-            half_t ov[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {                      // the roundings of partial_silu_mul_kernel
-                const float gf = (float)(half_t)gv[e];
-                const half_t sl = (half_t)(gf / (1.0f + expf(-gf)));
-                ov[e] = sl * (half_t)uv[e];
-            }
-            half_t *dst = p.c + (long)m * p.ldc + 128 * blockj + 64 * st_hh + 4 * st_c + 2 * bp;
-            *reinterpret_cast<h2 *>(dst) = h2{ov[0], ov[1]};
-            *reinterpret_cast<h2 *>(dst + 4) = h2{ov[2], ov[3]};
+        for (int e = 0; e < 4; ++e) {                          // the roundings of partial_silu_mul_kernel
+            const float gf = (float)(half_t)gv[e];
+            const half_t sl = (half_t)(gf / (1.0f + expf(-gf)));
+            ov[e] = sl * (half_t)uv[e];
         }
+        half_t *dst = p.c + (long)row * p.ldc + out_col;
+        *reinterpret_cast<h2 *>(dst) = h2{ov[0], ov[1]};
+        *reinterpret_cast<h2 *>(dst + 4) = h2{ov[2], ov[3]};
     }
 }
 
@@ -1105,7 +994,6 @@ template <int TILES, int MODE> struct WideShape {
     static constexpr int W = 6 * 1024, SC = 6 * 128;             // of the six slots: nibbles; scales [octet][nibble][8 rows]
     static constexpr int STAGE = W + SC + STEPS * TILES * 1024;
     static constexpr int SLOTS = 6;
-    static constexpr int PER = 9 + STEPS * TILES;                // DMA instructions of a stage
     static constexpr int OP = 64 * PIECES + 4;
     static constexpr int OTILE = (MODE == WIDE_SWIGLU ? 2 : 1) * 16 * OP * 4;      // [16][OP] fp32; SwiGLU: [gate | up][16][OP]
     static constexpr int SUMS = TILES * 16 * OP * 4;             // two K-groups: [row][OP] fp32
@@ -1116,10 +1004,10 @@ template <int TILES, int MODE> struct WideShape {
 constexpr int WIDE_WAVES = 12;
 
 template <int TILES, int MODE>
-__global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_wide_kernel(MatmulParams p) {
+__global__ __launch_bounds__(64 * (WIDE_WAVES + GEMM_DMA_WAVES), 1) void q40_gemm_wide_kernel(MatmulParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     typedef WideShape<TILES, MODE> S;
-    constexpr int SLOTS = S::SLOTS, PER = S::PER, STAGE = S::STAGE, STEPS = S::STEPS, PIECES = S::PIECES;
+    constexpr int SLOTS = S::SLOTS, STAGE = S::STAGE, STEPS = S::STEPS, PIECES = S::PIECES;
     constexpr bool SWIGLU = MODE == WIDE_SWIGLU;
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1140,8 +1028,8 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_wide_kernel
         return sg;
     };
 
-    if (wave == WIDE_WAVES) {
-        // ---- the DMA wave ----
+    if (wave >= WIDE_WAVES) {
+        // ---- the DMA waves: the weights and the rows of A, or (WIDE_GROUPS) a step each ----
         __builtin_amdgcn_s_setprio(3);
         const int a_chunk = (lane & 3) ^ ((lane >> 3) & 3);
         uint32_t a_voff[TILES];
@@ -1166,45 +1054,30 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_wide_kernel
         for (int s = 0; s < 6; ++s) w[s] += in_tile[s] * 1024;
         const uint8_t *a_base = reinterpret_cast<const uint8_t *>(p.a);
         int fetch = 0;                                                 // (in K's order: a start of its own for each unit gains nothing here)
-        auto issue_stage = [&](int slot_) {
-            uint8_t *st = lds + slot_ * STAGE;
-            const long off = (long)fetch * STEPS * TILE_BYTES;
-            const uint8_t *arow = a_base + (long)fetch * STEPS * 64;
+        auto feed = [&](auto which) {
+            constexpr int D = decltype(which)::value;
+            constexpr bool GROUPS = MODE == WIDE_GROUPS;
+            constexpr int W0 = GROUPS ? 3 * D : 6 * D, W1 = GROUPS ? W0 + 3 : 6;             // slots, pairs of slots' scales and steps of A of this wave
+            constexpr int S0 = GROUPS ? 2 * D : 3 * D, S1 = GROUPS && D == 0 ? 2 : 3;
+            constexpr int K0 = GROUPS || D == 1 ? (GROUPS ? D : 0) : STEPS, K1 = GROUPS ? D + 1 : STEPS;
+            gemm_feed<W1 - W0 + S1 - S0 + (K1 - K0) * TILES, SLOTS>(n_st, [&](int slot_) {
+                uint8_t *st = lds + slot_ * STAGE;
+                const long off = (long)fetch * STEPS * TILE_BYTES;
+                const uint8_t *arow = a_base + (long)fetch * STEPS * 64;
 #pragma unroll
-            for (int s = 0; s < 6; ++s) __builtin_amdgcn_global_load_lds((gptr_t)(w[s] + off + lane * 16), (lptr_t)(st + s * 1024), 16, 0, 0);
+                for (int s = W0; s < W1; ++s) __builtin_amdgcn_global_load_lds((gptr_t)(w[s] + off + lane * 16), (lptr_t)(st + s * 1024), 16, 0, 0);
 #pragma unroll
-            for (int i = 0; i < 3; ++i) __builtin_amdgcn_global_load_lds((gptr_t)(sc[i] + off), (lptr_t)(st + S::W + i * 256), 4, 0, 0);
+                for (int i = S0; i < S1; ++i) __builtin_amdgcn_global_load_lds((gptr_t)(sc[i] + off), (lptr_t)(st + S::W + i * 256), 4, 0, 0);
 #pragma unroll
-            for (int k = 0; k < STEPS; ++k)
+                for (int k = K0; k < K1; ++k)
 #pragma unroll
-                for (int t = 0; t < TILES; ++t)
-                    __builtin_amdgcn_global_load_lds((gptr_t)(arow + k * 64 + a_voff[t]), (lptr_t)(st + S::W + S::SC + (k * TILES + t) * 1024), 16, 0, 0);
-            ++fetch;
+                    for (int t = 0; t < TILES; ++t)
+                        __builtin_amdgcn_global_load_lds((gptr_t)(arow + k * 64 + a_voff[t]), (lptr_t)(st + S::W + S::SC + (k * TILES + t) * 1024), 16, 0, 0);
+                ++fetch;
+            });
         };
-#pragma unroll
-        for (int i = 0; i < SLOTS - 2; ++i)
-            if (i < n_st) issue_stage(i);
-        gemm_wait_dma<PER>(min(SLOTS - 3, n_st - 1));
-        gemm_barrier();
-        int slot = 0;
-        auto back = [&](int k) { return slot >= k ? slot - k : slot + SLOTS - k; };
-        int i = 0;
-#pragma unroll 1
-        for (; i + SLOTS - 1 < n_st; i += 2) {
-            gemm_wait_vm<PER * (SLOTS - 5)>();
-            gemm_barrier();
-            issue_stage(back(2));
-            issue_stage(back(1));
-            slot = slot + 2 >= SLOTS ? slot + 2 - SLOTS : slot + 2;
-        }
-#pragma unroll 1
-        for (; i < n_st; i += 2) {
-            gemm_wait_dma<PER>(max(0, min(n_st - 1, i + SLOTS - 3) - (i + 2)));
-            gemm_barrier();
-            if (i + SLOTS - 2 < n_st) issue_stage(back(2));
-            if (i + SLOTS - 1 < n_st) issue_stage(back(1));
-            slot = slot + 2 >= SLOTS ? slot + 2 - SLOTS : slot + 2;
-        }
+        if (wave == WIDE_WAVES) feed(int_constant<0>{});
+        else feed(int_constant<1>{});
         // the barriers of the epilogue: ring free, one per row tile; ring free, the second group's sums in place, all sums
 #pragma unroll 1
         for (int t = 0; t < (MODE == WIDE_GROUPS ? 3 : 1 + TILES); ++t) gemm_barrier();
@@ -1213,72 +1086,10 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + 1), 1) void q40_gemm_wide_kernel
 
     // nibble, slot; the slot's half - gate (0) or up (1), or K-group - and piece
     const int hh = wave >= 6 ? 1 : 0, s = wave - 6 * hh, half = s >= PIECES ? 1 : 0, k3 = s - 3 * half;
-    const uint32_t nib_mask = hh == 0 ? 0x00F000F0u : 0x000F000Fu;
-    uint32_t nib_magic = MAGIC_1024;                             // (as in q40_gemm_swiglu_kernel)
-    asm volatile("" : "+v"(nib_magic));
-    const h2 nib_mul = hh == 0 ? h2{(half_t)0.0625f, (half_t)0.0625f} : h2{(half_t)1.0f, (half_t)1.0f};
-    const h2 nib_off = hh == 0 ? h2{(half_t)-72.0f, (half_t)-72.0f} : h2{(half_t)-1032.0f, (half_t)-1032.0f};
-    struct Raw { u32x4 wq, sc; };
-    const int ws_off = s * 1024 + lane * 16, sc_off = S::W + s * 128 + g * 32 + hh * 16;
-    const int a_off = S::W + S::SC + (MODE == WIDE_GROUPS ? half * TILES * 1024 : 0) + c * 64 + ((g ^ ((c >> 1) & 3)) << 4);
-    auto load_ws = [&](const uint8_t *st, Raw &r) {
-        r.wq = *reinterpret_cast<const u32x4 *>(st + ws_off);
-        r.sc = *reinterpret_cast<const u32x4 *>(st + sc_off);
-    };
-    auto decode = [&](const Raw &r, h8 (&b)[2]) {
-        u32x4 v0, v1;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t pr0 = j < 2 ? r.wq[j] : r.wq[j - 2] >> 8;       // rows (2j, 2j+1) of byte 2bp, codes + 8
-            const uint32_t pr1 = j < 2 ? r.wq[2 + j] : r.wq[j] >> 8;       // ... of byte 2bp+1
-            const h2 sc = as_h2(r.sc[j]);
-            v0[j] = as_u32(__builtin_elementwise_fma(as_h2((pr0 & nib_mask) | nib_magic), nib_mul, nib_off) * sc);
-            v1[j] = as_u32(__builtin_elementwise_fma(as_h2((pr1 & nib_mask) | nib_magic), nib_mul, nib_off) * sc);
-        }
-        b[0] = __builtin_bit_cast(h8, v0);
-        b[1] = __builtin_bit_cast(h8, v1);
-    };
     f4 acc[2][TILES];
-#pragma unroll
-    for (int o = 0; o < 2; ++o)
-#pragma unroll
-        for (int t = 0; t < TILES; ++t) acc[o][t] = f4{0.f, 0.f, 0.f, 0.f};
-
-    h8 bq[2];
-    int slot = 0;
-    gemm_barrier();
-    {
-        Raw r;
-        load_ws(lds, r);
-        decode(r, bq);
-    }
-    auto one_stage = [&]() {
-        const uint8_t *st = lds + slot * STAGE;
-        slot = slot == SLOTS - 1 ? 0 : slot + 1;
-        Raw r;
-        h8 av[TILES], bn[2];
-#pragma unroll
-        for (int t = 0; t < TILES; ++t) av[t] = *reinterpret_cast<const h8 *>(st + a_off + t * 1024);
-        load_ws(lds + slot * STAGE, r);                        // (past the last stage: stale bytes, decoded and never used)
-#pragma unroll
-        for (int t = 0; t < TILES; ++t)
-#pragma unroll
-            for (int o = 0; o < 2; ++o) acc[o][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[t], bq[o], acc[o][t], 0, 0, 0);
-        decode(r, bn);
-        bq[0] = bn[0];
-        bq[1] = bn[1];
-    };
-    int i = 0;
-#pragma unroll 1
-    for (; i + 1 < n_st; i += 2) {
-        gemm_barrier();
-        one_stage();
-        one_stage();
-    }
-    if (i < n_st) {
-        gemm_barrier();
-        one_stage();
-    }
+    // (seven row tiles: the decode where the compiler puts it; spread, these spill in the 128 registers of four waves a SIMD)
+    gemm_multiply<TILES, SLOTS, STAGE, SWIGLU || TILES != 7>(lds, n_st, hh, s * 1024 + lane * 16, S::W + s * 128 + g * 32 + hh * 16,
+                                       S::W + S::SC + (MODE == WIDE_GROUPS ? half * TILES * 1024 : 0) + c * 64 + ((g ^ ((c >> 1) & 3)) << 4), acc);
 
     // rows of 64 PIECES columns: local column 64 k3 + 32 hh + 2 c + o is column 128 (P / 2) + 64 hh + 4 c + 2 (P % 2) + o, P the piece;
     // a thread stores local columns 4 o_lane .. + 3
@@ -1538,7 +1349,7 @@ static int gemm_launch_layout(const MatmulParams &p, hipStream_t stream) {
                                            q40_gemm_kernel<3, false, TILED, W>, q40_gemm_kernel<4, false, TILED, W>,
                                            q40_gemm_kernel<5, false, TILED, W>, q40_gemm_kernel<6, false, TILED, W>,
                                            q40_gemm_kernel<7, false, TILED, W>, q40_gemm_kernel<8, false, TILED, W>};
-    // one workgroup per compute unit: eight waves and the DMA wave, on both layouts.  (Checkpoint layout, against four waves that
+    // one workgroup per compute unit: eight waves and the DMA waves, on both layouts.  (Checkpoint layout, against four waves that
     // leave every SIMD one: 100 rows x 11008 x 4096 31.9 -> 27.2 us, x 32128 61 -> 51, 20 x 28672 x 8192 66 -> 51, 160 x 28672 x
     // 4096 96 -> 64.  Where two workgroups of four waves share a compute unit, eight re-read each nibble from LDS for nothing:
     // 512 x 28672 x 8192 312-324 us against 314, 512 x 20480 x 12288 412 against 389.)
@@ -1593,7 +1404,7 @@ static int gemm_launch_layout(const MatmulParams &p, hipStream_t stream) {
     const gemm_kernel_t kern = odd_k ? (TILED ? ragged : (one_each ? ragged_dma_wave : ragged_four)[tiles])
                                      : (p.chunk > 0 ? range_cut : one_each ? with_dma_wave : exact)[tiles];
     const long total_steps = (long)p.units * ((p.K + 31) / 32);
-    const int lds = one_each ? gemm_dma_slots(tiles) * GS_BYTES : GEMM_LDS, threads = one_each ? 64 * (WD + 1) : four ? GEMM_THREADS : 64 * W;
+    const int lds = one_each ? gemm_dma_slots(tiles) * GS_BYTES : GEMM_LDS, threads = one_each ? 64 * (WD + GEMM_DMA_WAVES) : four ? GEMM_THREADS : 64 * W;
     if (p.chunk > 0) {
         hipLaunchKernelGGL(kern, dim3((unsigned)((total_steps + p.chunk - 1) / p.chunk)), dim3(threads), lds, stream, p);
         return launch_status();
@@ -1619,7 +1430,7 @@ static int gemm_kg_launch(const MatmulParams &p, hipStream_t stream) {
     SMH_REQUIRE((long)p.M * p.lda * 2 < (1L << 32), "q40 gemm: M x lda = %d x %ld exceeds the 32-bit lane offsets of A", p.M, p.lda);
     int tiles = p.mblocks > 1 ? p.block_rows / 16 : (p.M + 15) / 16;
     if (tiles < 2) tiles = 2;
-    hipLaunchKernelGGL(kern[tiles], dim3((unsigned)(2 * p.units_pad), (unsigned)p.mblocks, (unsigned)p.ksplit), dim3(576), lds_bytes[tiles], stream, p);
+    hipLaunchKernelGGL(kern[tiles], dim3((unsigned)(2 * p.units_pad), (unsigned)p.mblocks, (unsigned)p.ksplit), dim3(64 * (8 + GEMM_DMA_WAVES)), lds_bytes[tiles], stream, p);
     return launch_status();
 }
 
@@ -1657,7 +1468,7 @@ int gemm_swiglu_launch(const MatmulParams &p, hipStream_t stream) {
     SMH_REQUIRE((long)p.M * p.lda * 2 < (1L << 32), "q40 gemm: M x lda = %d x %ld exceeds the 32-bit lane offsets of A", p.M, p.lda);
     int tiles = (p.M + 15) / 16;
     if (tiles < 2) tiles = 2;
-    hipLaunchKernelGGL(kern[tiles], dim3((unsigned)(2 * (p.seg[0].N / 128))), dim3(576), lds_bytes[tiles], stream, p);
+    hipLaunchKernelGGL(kern[tiles], dim3((unsigned)(2 * (p.seg[0].N / 128))), dim3(64 * (8 + GEMM_DMA_WAVES)), lds_bytes[tiles], stream, p);
     return launch_status();
 }
 
@@ -1708,12 +1519,12 @@ int gemm_swiglu_rows_launch(MatmulParams p, hipStream_t stream) {
     if (gemm_swiglu_rows_plan(p, w)) {
         const int t = w.block_rows / 16 - 4;
         w.ksplit = 1;
-        return gemm_launch_rows(wide[t], w, 64 * (WIDE_WAVES + 1), wide_lds[t], stream);
+        return gemm_launch_rows(wide[t], w, 64 * (WIDE_WAVES + GEMM_DMA_WAVES), wide_lds[t], stream);
     }
     const bool one_each = (long)p.units * p.mblocks <= GEMM_DMA_WAVE_MAX_WGS;
     const int t = p.block_rows / 16 - 4;
     p.ksplit = 1;
-    return gemm_launch_rows((one_each ? dma_wave : plain)[t], p, 512 + (one_each ? 64 : 0), one_each ? gemm_dma_slots(t + 4) * GS_BYTES : GEMM_LDS, stream);
+    return gemm_launch_rows((one_each ? dma_wave : plain)[t], p, 512 + (one_each ? 64 * GEMM_DMA_WAVES : 0), one_each ? gemm_dma_slots(t + 4) * GS_BYTES : GEMM_LDS, stream);
 }
 
 // The launch of a direct product whose plan has no K-split, with workgroups of three pieces and two K-groups or of six pieces where they
@@ -1764,7 +1575,7 @@ static int gemm_wide_launch(const MatmulParams &p, int pieces, hipStream_t strea
     }
     SMH_REQUIRE((long)p.M * p.lda * 2 < (1L << 32), "q40 gemm: M x lda = %d x %ld exceeds the 32-bit lane offsets of A", p.M, p.lda);
     const int six = pieces == 6 ? 1 : 0, t = p.block_rows / 16 - 4;
-    return gemm_launch_rows(kern[six][t], p, 64 * (WIDE_WAVES + 1), lds_bytes[six][t], stream);
+    return gemm_launch_rows(kern[six][t], p, 64 * (WIDE_WAVES + GEMM_DMA_WAVES), lds_bytes[six][t], stream);
 }
 
 int gemm_launch(const MatmulParams &p, hipStream_t stream) {
