@@ -1253,8 +1253,11 @@ void gemm_fill_plan(MatmulParams &p) {
     // Tiled weights, 17 .. 128 rows, K a multiple of 64: 128-column blocks with two K-groups a workgroup (q40_gemm_kg_kernel)
     // where they fill at least two thirds of the compute units in one round - half the K-slices, or fewer, of the 256-column
     // units below for the same number of workgroups.  Narrow matrices (at most 32 blocks: wo, w2) at any such row count, and
-    // with two 64-row blocks per column block where K is short (wo at 65 .. 128 rows); wide ones (wq|wk|wv, w1|w3) above
-    // 64 rows only (below, the launch loses more than its consumer gains); K up to 16384 (a row of A is staged for 128 columns
+    // with two 64-row blocks per column block where K is short (wo at 65 .. 128 rows); wide ones (wq|wk|wv, w1|w3) above 64 rows,
+    // and below where K is still cut at least once (wq|wk|wv) above 32 rows or with K up to 4096.  (A step in us, 256-column units and this: 7B architecture,
+    // 24 branches 2349 and 2340, 32 2440 and 2414, 37 2523 and 2506, 48 2663 and 2618, 64 2926 and 2880; three layers of the 70B architecture, K = 8192,
+    // 24 branches 557 and 561, 40 630 and 624, 48 644 and 638.)  K up to 16384
+    // (a row of A is staged for 128 columns
     // instead of 256, which makes the loop ~12 % slower per step: with K = 28672 that outweighs the slabs).  Measured at 100
     // rows, launch + consumer: wo 15.8 against 17.5 us, w2 24.7 against 26.9, w1|w3 39.7 against 40.9; a decode step at 100
     // branches 4.06 against 4.29 ms.
@@ -1269,7 +1272,7 @@ void gemm_fill_plan(MatmulParams &p) {
         if (ks > cap) ks = cap;
         const int steps = p.K / 32;
         if (ks > steps / 8) ks = steps / 8;                    // at least four stages (of two steps) a slice
-        if (ks >= 1 && (narrow || p.M > 64) && (long)blocks * mblocks * ks >= 170) {
+        if (ks >= 1 && (narrow || p.M > 64 || (ks >= 2 && (p.M > 32 || p.K <= 4096))) && (long)blocks * mblocks * ks >= 170) {
             p.kgroups = 2;
             p.mblocks = mblocks;
             p.block_rows = mblocks == 2 ? 64 : GEMM_BM;

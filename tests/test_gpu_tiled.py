@@ -123,6 +123,22 @@ def test_range_cut_products(M, K, ns, slabs):
             col += nn
 
 
+@pytest.mark.parametrize("M,K,ns,slabs", [(17, 4096, [4096, 4096, 4096], 2), (32, 4096, [4096, 4096, 4096], 2), (64, 4096, [4096, 4096, 4096], 2),
+                                          (33, 8192, [8192, 1024, 1024], 3), (48, 8192, [8192, 1024, 1024], 3)])
+def test_wide_products_of_few_rows(M, K, ns, slabs):
+    """wq|wk|wv at 17 .. 64 rows on two K-groups a workgroup: the slab count, and the sum of the slabs as close to 64 bits as that of the
+    checkpoint layout's launch, whose fp32 sums have another order (either is below 2^-24 sqrt(K) of the result's norm)"""
+    from spec_mcts_amd import kernels as Kn
+    assert Kn.matmul_plan(M, K, ns, tiled=True) == slabs
+    ws = [_weight(K, n, 975 + i + K) for i, n in enumerate(ns)]
+    a = (torch.randn((M, K), generator=torch.Generator().manual_seed(976 + M)) * 0.5).half().cuda()
+    lin = [(w.cuda(), s.cuda(), n) for (w, s), n in zip(ws, ns)]
+    exact = torch.cat([a.double() @ Kn.deq_int40(w, s, 64, (K, n)).double() for w, s, n in lin], 1)
+    for p in (Kn.matmul_q40_partial(a, [Kn.tile_q40(w, s, K, n) for w, s, n in lin]), Kn.matmul_q40_partial(a, lin)):
+        got = p.buf[:p.ksplit * M * p.n_total].view(p.ksplit, M, p.n_total).double().sum(0)
+        assert float((got - exact).norm() / exact.norm()) < 2.0 ** -24 * K ** 0.5
+
+
 @pytest.mark.parametrize("M", [17, 33, 64, 100, 128])
 @pytest.mark.parametrize("K,n_half", [(4096, 11008), (256, 384), (8192, 1024), (128, 128), (1024, 16384)])
 def test_swiglu_inside_the_gate_up_launch(M, K, n_half):
