@@ -313,10 +313,15 @@ __global__ __launch_bounds__(256) void attn_prefix_kernel(AttnParams p) {
 // is infinite or NaN, the slice is left to attn_suffix_kernel.  Probabilities enter the product as three fp16 terms of 2^15 p (the
 // second 2^11 times what the first leaves over, the third 2^11 times what the second does), in three accumulators: all 24 bits of
 // the fp32 probability down to 2^-38 of the slice's largest, 2^-62 of it absolutely below, so nothing of it is rounded away.
+// A workgroup has PT_TILES tiles, one after the other, and stages rows again only where the ids differ from the last tile's.
 // Bound by the walk of what is not shared.  32 heads, 512 positions, half of them a prompt: 99 branches 150 -> 100 us a call, 50: 80 -> 60,
 // 27: 45 -> 37, 8: 32 -> 20; 460 shared positions and 99 branches: 111 -> 39 us (error against 64 bits 2.1e-4 before and after: the
 // output's fp16).  Where nothing is shared the pass costs its 3 us (100 positions, 99 branches: 29.7 -> 26.5 with the walk's gain).
+// Two tiles a workgroup where one a workgroup would be more than the 768 that run at a time (three a compute unit): 32 heads, 99 branches,
+// 512 positions, 256 of them a prompt 83.1 -> 80.7 us a call (this pass 16.3 -> 14.3), 460 of them 33.2 -> 30.9, 768 with a prompt of 600 68.2 -> 64.6;
+// 100 positions, 448 workgroups of one tile, 22.6 and 23.3 with two.  Three and four tiles: no faster, seven: slower.
 constexpr int PT_TW = 64;
+constexpr long PT_ROUND = 768;
 constexpr int PT_MAX_SLICES = 64;          // one bit a slice in the suffix kernel's mask
 // Waits for a wave's loads where a loop that keeps a batch on its way begins.  With the first batch still on its way there, the compiler, which
 // counts loads, waits in every pass for as much as the first one needs: for the next batch, too.
@@ -341,139 +346,168 @@ __device__ __forceinline__ long page_row(const AttnParams &p, page_id_t<PB> id) 
     if constexpr (PB == 2 || PB == 4) return min(max(id, 0), (int)min(p.pool_rows - 1, 0x7fffffffL));
     return min(max((long)id, 0L), p.pool_rows - 1);
 }
-template <int PB>
+template <int PB, int PT_TILES>
 __global__ __launch_bounds__(256) void attn_page_tile_kernel(AttnParams p) {
     args_ahead<sizeof(AttnParams)>();
     __shared__ __attribute__((aligned(16))) half_t ks[PT_TW][ATT_KPITCH];
     __shared__ __attribute__((aligned(16))) half_t vt[ATT_D][PT_TW + 8];
     __shared__ __attribute__((aligned(16))) half_t ps[3][16][PT_TW + 8];      // probabilities of the 16 queries, the three terms, in vt_pos order
-    __shared__ long s_row[PT_TW];
+    __shared__ long s_row[PT_TILES][PT_TW];        // rows of the tiles' first branches
     __shared__ float s_max[4][16], s_sum[4][16];
-    const int hk = blockIdx.x, split = blockIdx.y, tile = blockIdx.z;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
+    __shared__ uint32_t s_bits[4];
+    const int hk = blockIdx.x, split = blockIdx.y, tiles = (p.Bq + 15) / 16, tile0 = blockIdx.z * PT_TILES, n_tiles = min(PT_TILES, tiles - tile0);
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 15, g = lane >> 4;
     const int t0 = split * PT_TW, cnt = min(PT_TW, (int)p.suffix_batch_stride_rows - t0);
-    const int b_lo = div_rep(p, tile * 16), b_hi = div_rep(p, min(tile * 16 + 15, p.Bq - 1));
-    // ---- does every branch of the tile have the first one's ids? ----
-    bool same = true;
-    {
-        const int pos = t0 + min(lane, cnt - 1);
-        page_id_t<PB> id[5];                       // the first branch's, and those of every fourth other one (past the last: again)
-#pragma unroll
-        for (int i = 0; i < 5; ++i) id[i] = page_at<PB>(p, (long)(i == 0 ? b_lo : min(b_lo + 1 + wave + 4 * (i - 1), b_hi)) * p.pages_stride + pos);
-#pragma unroll
-        for (int i = 1; i < 5; ++i) same &= id[i] == id[0];
-        if (wave == 0) s_row[lane] = page_row<PB>(p, id[0]);
-    }
-    // the query tile (B operand of S^T)
-    const int qrow = tile * 16 + c, qr = min(qrow, p.Bq - 1);
-    h8 qb[4];
-    {
+    // a tile's queries (B operand of S^T)
+    auto queries = [&](int i, h8 (&qb)[4]) {
+        const int qr = min((tile0 + i) * 16 + c, p.Bq - 1);
         const half_t *qp = p.q + ((long)div_rep(p, qr) * p.H + hk * p.n_rep + mod_rep(p, qr)) * ATT_D + 8 * g;
 #pragma unroll
         for (int k4 = 0; k4 < 4; ++k4) qb[k4] = *reinterpret_cast<const h8 *>(qp + 32 * k4);
-    }
-    uint8_t *done = p.tile_done + ((long)hk * gridDim.z + tile) * p.splits + split;
-    if (!__syncthreads_and(same)) {
-        if (tid == 0) *done = 0;
-        return;
-    }
-    // ---- the rows: K row-major, V transposed, as in attn_prefix_body ----
-    uint32_t bad = 0;
+    };
+    // ---- bit i: every branch of tile i has the first one's ids; bit 8 + i: which are those of tile i - 1's first ----
+    uint32_t bits = 0;
+    h8 qn[4];
     {
-        const int ch = tid & 15, kg = tid >> 4;
-        u32x4 kv[4], vv[4];
+        const int pos = t0 + min(lane, cnt - 1);
+        page_id_t<PB> id[PT_TILES][5];             // a tile's first branch's, and those of every fourth other one (past the last: again)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const long off = s_row[4 * kg + e] * p.sfx_row_stride + (long)hk * p.sfx_head_stride + ch * 8;
-            const half_t *kp = (const half_t *)p.suffix_k + off, *vp = (const half_t *)p.suffix_v + off;
-            // (8-byte loads: a pool's rows are only that much aligned)
-            const u32x2 k0 = *reinterpret_cast<const u32x2 *>(kp), k1 = *reinterpret_cast<const u32x2 *>(kp + 4);
-            const u32x2 v0 = *reinterpret_cast<const u32x2 *>(vp), v1 = *reinterpret_cast<const u32x2 *>(vp + 4);
-            kv[e] = u32x4{k0[0], k0[1], k1[0], k1[1]};
-            vv[e] = u32x4{v0[0], v0[1], v1[0], v1[1]};
+        for (int i = 0; i < PT_TILES; ++i) {
+            const int b_lo = div_rep(p, min((tile0 + i) * 16, p.Bq - 1)), b_hi = div_rep(p, min((tile0 + i) * 16 + 15, p.Bq - 1));
+#pragma unroll
+            for (int j = 0; j < 5; ++j) id[i][j] = page_at<PB>(p, (long)(j == 0 ? b_lo : min(b_lo + 1 + wave + 4 * (j - 1), b_hi)) * p.pages_stride + pos);
         }
+        queries(0, qn);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
+        for (int i = 0; i < PT_TILES; ++i) {
+            bool same = true;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {          // (an exponent of all ones carries into the sign bit)
-                bad |= (kv[e][i] & 0x7fff7fffu) + 0x04000400u;
-                bad |= (vv[e][i] & 0x7fff7fffu) + 0x04000400u;
+            for (int j = 1; j < 5; ++j) same &= id[i][j] == id[i][0];
+            if (__all(same)) bits |= 1u << i;
+            if (i > 0 && __all(id[i][0] == id[i - 1][0])) bits |= 256u << i;
+            if (wave == i % 4) s_row[i][lane] = page_row<PB>(p, id[i][0]);
+        }
+    }
+    if (lane == 0) s_bits[wave] = bits;
+    __syncthreads();
+    bits = (uint32_t)__builtin_amdgcn_readfirstlane((int)(s_bits[0] & s_bits[1] & s_bits[2] & s_bits[3]));
+    bool staged = false, finite = false;           // rows in LDS: those of the tile in hand; whose values are finite
+#pragma unroll 1
+    for (int n = 0; n < n_tiles; ++n) {
+        uint8_t *done = p.tile_done + ((long)hk * tiles + tile0 + n) * p.splits + split;
+        const int qrow = (tile0 + n) * 16 + c;
+        staged = staged && ((bits >> (8 + n)) & 1) != 0;
+        h8 qb[4];
+#pragma unroll
+        for (int k4 = 0; k4 < 4; ++k4) qb[k4] = qn[k4];
+        if (n + 1 < n_tiles) queries(n + 1, qn);
+        if (((bits >> n) & 1) == 0) {
+            if (tid == 0) *done = 0;
+            continue;
+        }
+        if (!staged) {
+            if (n > 0) __syncthreads();                    // (the tile before has been multiplied)
+            // ---- the rows: K row-major, V transposed, as in attn_prefix_body ----
+            uint32_t bad = 0;
+            {
+                const int ch = tid & 15, kg = tid >> 4;
+                u32x4 kv[4], vv[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const long off = s_row[n][4 * kg + e] * p.sfx_row_stride + (long)hk * p.sfx_head_stride + ch * 8;
+                    const half_t *kp = (const half_t *)p.suffix_k + off, *vp = (const half_t *)p.suffix_v + off;
+                    // (8-byte loads: a pool's rows are only that much aligned)
+                    const u32x2 k0 = *reinterpret_cast<const u32x2 *>(kp), k1 = *reinterpret_cast<const u32x2 *>(kp + 4);
+                    const u32x2 v0 = *reinterpret_cast<const u32x2 *>(vp), v1 = *reinterpret_cast<const u32x2 *>(vp + 4);
+                    kv[e] = u32x4{k0[0], k0[1], k1[0], k1[1]};
+                    vv[e] = u32x4{v0[0], v0[1], v1[0], v1[1]};
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) {          // (an exponent of all ones carries into the sign bit)
+                        bad |= (kv[e][w] & 0x7fff7fffu) + 0x04000400u;
+                        bad |= (vv[e][w] & 0x7fff7fffu) + 0x04000400u;
+                    }
+                    *reinterpret_cast<u32x4 *>(&ks[4 * kg + e][ch * 8]) = kv[e];
+                }
+                const int pos = vt_pos(4 * kg);
+                const h8 v0 = __builtin_bit_cast(h8, vv[0]), v1 = __builtin_bit_cast(h8, vv[1]);
+                const h8 v2 = __builtin_bit_cast(h8, vv[2]), v3 = __builtin_bit_cast(h8, vv[3]);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) *reinterpret_cast<h4 *>(&vt[ch * 8 + j][pos]) = h4{v0[j], v1[j], v2[j], v3[j]};
             }
-            *reinterpret_cast<u32x4 *>(&ks[4 * kg + e][ch * 8]) = kv[e];
+            finite = !__syncthreads_or((bad & 0x80008000u) != 0);
+            staged = true;
         }
-        const int pos = vt_pos(4 * kg);
-        const h8 v0 = __builtin_bit_cast(h8, vv[0]), v1 = __builtin_bit_cast(h8, vv[1]);
-        const h8 v2 = __builtin_bit_cast(h8, vv[2]), v3 = __builtin_bit_cast(h8, vv[3]);
+        if (tid == 0) *done = finite ? 1 : 0;
+        if (!finite) continue;
+        // ---- scores: element r of st is position 16 wave + 4 g + r (past the end: a repeated row, masked), column (query) c ----
+        f4 st = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < 8; ++j) *reinterpret_cast<h4 *>(&vt[ch * 8 + j][pos]) = h4{v0[j], v1[j], v2[j], v3[j]};
-    }
-    const bool finite = !__syncthreads_or((bad & 0x80008000u) != 0);
-    if (tid == 0) *done = finite ? 1 : 0;
-    if (!finite) return;
-    // ---- scores: element r of st is position 16 wave + 4 g + r (past the end: a repeated row, masked), column (query) c ----
-    f4 st = {0.f, 0.f, 0.f, 0.f};
+        for (int k4 = 0; k4 < 4; ++k4)
+            st = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const h8 *>(&ks[16 * wave + c][32 * k4 + 8 * g]), qb[k4], st, 0, 0, 0);
+        float mx = -INFINITY;
 #pragma unroll
-    for (int k4 = 0; k4 < 4; ++k4)
-        st = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const h8 *>(&ks[16 * wave + c][32 * k4 + 8 * g]), qb[k4], st, 0, 0, 0);
-    float mx = -INFINITY;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        st[r] = 16 * wave + 4 * g + r < cnt ? st[r] * p.scale_log2 : -INFINITY;
-        mx = fmaxf(mx, st[r]);
-    }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    if (g == 0) s_max[wave][c] = mx;
-    __syncthreads();
-    mx = fmaxf(fmaxf(s_max[0][c], s_max[1][c]), fmaxf(s_max[2][c], s_max[3][c]));
-    float sum = 0.f;
-    h4 term[3];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const float e = exp2f(st[r] - mx);
-        sum += e;
-        float left = e * 32768.f;
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {              // (the differences and the powers of two are exact)
-            term[i][r] = (half_t)left;
-            left = (left - (float)term[i][r]) * 2048.f;
+        for (int r = 0; r < 4; ++r) {
+            st[r] = 16 * wave + 4 * g + r < cnt ? st[r] * p.scale_log2 : -INFINITY;
+            mx = fmaxf(mx, st[r]);
         }
-    }
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        if (g == 0) s_max[wave][c] = mx;
+        __syncthreads();
+        mx = fmaxf(fmaxf(s_max[0][c], s_max[1][c]), fmaxf(s_max[2][c], s_max[3][c]));
+        float sum = 0.f;
+        h4 term[3];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) *reinterpret_cast<h4 *>(&ps[i][c][32 * (wave >> 1) + 8 * g + 4 * (wave & 1)]) = term[i];
-    sum += __shfl_xor(sum, 16, 64);
-    sum += __shfl_xor(sum, 32, 64);
-    if (g == 0) s_sum[wave][c] = sum;
-    __syncthreads();
-    // ---- O^T: element r of o[i] is dim 32 wave + 16 i + 4 g + r, column (query) c ----
-    f4 ot[3][2];                                   // by term
+        for (int r = 0; r < 4; ++r) {
+            const float e = exp2f(st[r] - mx);
+            sum += e;
+            float left = e * 32768.f;
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) ot[k][i] = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int jj = 0; jj < PT_TW / 32; ++jj) {
-        const h8 va[2] = {*reinterpret_cast<const h8 *>(&vt[32 * wave + c][32 * jj + 8 * g]), *reinterpret_cast<const h8 *>(&vt[32 * wave + 16 + c][32 * jj + 8 * g])};
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const h8 pb = *reinterpret_cast<const h8 *>(&ps[k][c][32 * jj + 8 * g]);
-#pragma unroll
-            for (int i = 0; i < 2; ++i) ot[k][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va[i], pb, ot[k][i], 0, 0, 0);
+            for (int i = 0; i < 3; ++i) {              // (the differences and the powers of two are exact)
+                term[i][r] = (half_t)left;
+                left = (left - (float)term[i][r]) * 2048.f;
+            }
         }
-    }
-    if (qrow >= p.Bq) return;
-    const long base = ((long)split * p.Hkv + hk) * p.Bq + qrow;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        f4 o;
+        for (int i = 0; i < 3; ++i) *reinterpret_cast<h4 *>(&ps[i][c][32 * (wave >> 1) + 8 * g + 4 * (wave & 1)]) = term[i];
+        sum += __shfl_xor(sum, 16, 64);
+        sum += __shfl_xor(sum, 32, 64);
+        if (g == 0) s_sum[wave][c] = sum;
+        __syncthreads();
+        // ---- O^T: element r of o[i] is dim 32 wave + 16 i + 4 g + r, column (query) c ----
+        f4 ot[3][2];                                   // by term
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = (ot[0][i][r] + (ot[1][i][r] + ot[2][i][r] * 0x1p-11f) * 0x1p-11f) * 0x1p-15f;
-        *reinterpret_cast<f4 *>(p.part_o + base * ATT_D + 32 * wave + 16 * i + 4 * g) = o;
-    }
-    if (wave == 0 && g == 0) {
-        sum = s_sum[0][c] + s_sum[1][c] + s_sum[2][c] + s_sum[3][c];
-        p.part_ml[base * 2] = partial_max(mx, sum);
-        p.part_ml[base * 2 + 1] = sum;
+        for (int k = 0; k < 3; ++k)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) ot[k][i] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int jj = 0; jj < PT_TW / 32; ++jj) {
+            const h8 va[2] = {*reinterpret_cast<const h8 *>(&vt[32 * wave + c][32 * jj + 8 * g]), *reinterpret_cast<const h8 *>(&vt[32 * wave + 16 + c][32 * jj + 8 * g])};
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const h8 pb = *reinterpret_cast<const h8 *>(&ps[k][c][32 * jj + 8 * g]);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) ot[k][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va[i], pb, ot[k][i], 0, 0, 0);
+            }
+        }
+        if (qrow < p.Bq) {
+            const long base = ((long)split * p.Hkv + hk) * p.Bq + qrow;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                f4 o;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o[r] = (ot[0][i][r] + (ot[1][i][r] + ot[2][i][r] * 0x1p-11f) * 0x1p-11f) * 0x1p-15f;
+                *reinterpret_cast<f4 *>(p.part_o + base * ATT_D + 32 * wave + 16 * i + 4 * g) = o;
+            }
+            if (wave == 0 && g == 0) {
+                sum = s_sum[0][c] + s_sum[1][c] + s_sum[2][c] + s_sum[3][c];
+                p.part_ml[base * 2] = partial_max(mx, sum);
+                p.part_ml[base * 2 + 1] = sum;
+            }
+        }
     }
 }
 
@@ -2056,9 +2090,11 @@ static int shared_prefix_attn(const char *who, bool one, const void *q, void *ou
         n_part = (size_t)p.splits * Hkv * p.Bq;
         p.part_ml = p.part_o + n_part * ATT_D;
         p.tile_done = (uint8_t *)(p.part_ml + n_part * 2);
-        const auto shared = pb == 2 ? attn_page_tile_kernel<2> : pb == 4 ? attn_page_tile_kernel<4> : attn_page_tile_kernel<8>;
+        const int each = (long)Hkv * p.splits * tiles > PT_ROUND ? 2 : 1;
+        const auto one = pb == 2 ? attn_page_tile_kernel<2, 1> : pb == 4 ? attn_page_tile_kernel<4, 1> : attn_page_tile_kernel<8, 1>;
+        const auto two = pb == 2 ? attn_page_tile_kernel<2, 2> : pb == 4 ? attn_page_tile_kernel<4, 2> : attn_page_tile_kernel<8, 2>;
         const auto walk = pb == 2 ? attn_suffix_kernel<false, WALK_TILES, 2> : pb == 4 ? attn_suffix_kernel<false, WALK_TILES, 4> : attn_suffix_kernel<false, WALK_TILES, 8>;
-        hipLaunchKernelGGL(shared, dim3(Hkv, p.splits, tiles), dim3(256), 0, (hipStream_t)stream, p);
+        hipLaunchKernelGGL(each == 2 ? two : one, dim3(Hkv, p.splits, (tiles + each - 1) / each), dim3(256), 0, (hipStream_t)stream, p);
         hipLaunchKernelGGL(walk, dim3(wgs), dim3(256), 0, (hipStream_t)stream, p);
         return launch_status();
     }

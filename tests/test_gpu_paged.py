@@ -249,6 +249,36 @@ def test_pages_shared_by_the_branches_of_a_tile(B, H, Hkv, L, shared, odd):
     assert bool(((got - want)[fin].abs() <= 2e-3 + 1e-2 * want[fin].abs()).all())
 
 
+def test_two_query_tiles_of_a_workgroup():
+    """More workgroups of one tile than run at a time (32 heads x 9 slices x 3 tiles): a workgroup has two, and an odd one is left over.  Per
+    slice: both tiles the same rows; each its own; the first tile not shared; the second not; an infinite value in rows of both, of the
+    first alone, of the second alone; rows that differ by one id; the last slice has one position."""
+    from spec_mcts_amd import kernels as K
+    g = torch.Generator().manual_seed(7)
+    B, H, L = 40, 32, 8 * 64 + 1
+    rows = 4096
+    pages = torch.randperm(rows, generator=g).int()[:L].repeat(B, 1)
+    k, v = (torch.empty((H, rows, 128)).normal_(0.0, 0.5, generator=g).half() for _ in range(2))
+    other = torch.randperm(rows, generator=g).int()
+    sl = lambda i: slice(64 * i, 64 * i + 64)
+    pages[16:32, sl(1)] = other[:64]
+    pages[3, 64 * 2 + 5] = other[100]
+    pages[20, 64 * 3 + 63] = other[101]
+    v[0, pages[0, 64 * 4 + 1].item()] = float("inf")
+    pages[16:32, sl(5)] = other[200:264]
+    v[1, pages[0, 64 * 5].item()] = float("inf")
+    pages[16:32, sl(6)] = other[300:364]
+    v[2, other[310].item()] = float("inf")
+    pages[16:32, 64 * 7 + 31] = other[400]
+    q = torch.empty((B, H, 128)).normal_(0.0, 0.5, generator=g).half()
+    want = sdpa(q, pages, k, v)
+    for dtype in (torch.int16, torch.int32, torch.int64):
+        got = K.paged_prefix_attn(q.cuda(), pages.to(dtype).cuda(), None, k.cuda(), v.cuda(), head_major=True).cpu().float()
+        assert torch.equal(got.isinf(), want.isinf())
+        fin = want.isfinite()
+        assert bool(((got - want)[fin].abs() <= 2e-3 + 1e-2 * want[fin].abs()).all())
+
+
 def test_shared_pages_keep_fp32_probabilities():
     """The matrix-core pass holds a probability's 24 bits: weights 2^-25 .. 2^-36 of the largest carry the whole result (the largest
     one's row is zero), which is as far from 64-bit sums as fp16 output makes it (with two terms: 1.15 times as far)."""
