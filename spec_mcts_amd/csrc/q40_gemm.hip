@@ -1,6 +1,6 @@
 // Q4_0 dequant + matmul for large batches (decode at B = 100, prefill): c[M,N] = a[M,K] . deq(W)[K,N].
 //
-// A workgroup of 4 waves (8 plus one that only issues DMA in launches with one workgroup per compute unit, and 8 on tiled weights,
+// A workgroup of 4 waves (8 plus two that only issue DMA in launches with one workgroup per compute unit, and 8 on tiled weights,
 // see the kernel) owns 128 rows of A, two adjacent 128-column blocks of the weight (one full 128-byte line of
 // packed nibbles per k) and a slice of K - or, under a range cut, a run of steps that may end one column unit and begin
 // the next; up to two workgroups share a compute unit.  Everything a 32-row step needs - 4 KB of nibbles, 256 B of scales, the 128 x 32 tile of A -
@@ -125,6 +125,65 @@ __device__ __forceinline__ void gemm_feed(int n, Issue issue) {
 }
 template <int N> using int_constant = std::integral_constant<int, N>;
 
+// What a multiplying wave reads of a stage's weights, and half a row pair of its operands out of that: rows (2 j, 2 j + 1) of the piece's first
+// (o = 0) or second byte, the nibble (high: hh = 0, low) as fp16 code * scale.
+struct NibbleConsts {
+    uint32_t mask, magic;
+    h2 mul, off;
+    // flip: bits that turn a two's complement nibble into code + 8
+    __device__ __forceinline__ NibbleConsts(int hh, uint32_t flip)
+        : mask(hh == 0 ? 0x00F000F0u : 0x000F000Fu), magic(MAGIC_1024 ^ flip),
+          mul(hh == 0 ? h2{(half_t)0.0625f, (half_t)0.0625f} : h2{(half_t)1.0f, (half_t)1.0f}),
+          off(hh == 0 ? h2{(half_t)-72.0f, (half_t)-72.0f} : h2{(half_t)-1032.0f, (half_t)-1032.0f}) {
+        asm volatile("" : "+v"(magic));        // in a register the compiler cannot see through: (bits & mask) | magic is then ONE
+    }                                          // v_and_or_b32 (no literal operands there), not an AND and an OR
+    __device__ __forceinline__ h2 code(uint32_t bits) const { return __builtin_elementwise_fma(as_h2(bits), mul, off); }
+};
+struct TiledWeights {
+    static constexpr int READS = 2;            // LDS instructions of a load
+    NibbleConsts nib;
+    int w_off, s_off;
+    __device__ __forceinline__ TiledWeights(int hh, int w, int s) : nib(hh, 0), w_off(w), s_off(s) {}
+    struct Regs { u32x4 w, scales; };
+    __device__ __forceinline__ Regs load(const uint8_t *st, int) const {
+        return Regs{*reinterpret_cast<const u32x4 *>(st + w_off), *reinterpret_cast<const u32x4 *>(st + s_off)};
+    }
+    __device__ __forceinline__ uint32_t decode(const Regs &r, int j, int o) const {
+        const uint32_t w = r.w[(j & 1) + 2 * o], pr = j < 2 ? w : w >> 8;
+        return as_u32(nib.code((pr & nib.mask) | nib.magic) * as_h2(r.scales[j]));
+    }
+};
+// Checkpoint layout: row 8 g + r of a stage (GS_WBLOCK) and its scales (of the block's first, second 64 columns in a dword).
+// RAGGED: stage `last` is the end of K, where `dead` says that this lane's rows lie past it (their scales become zero).
+// (With reads that were waited for where they were issued, in us, before and now: 42 / 75 / 100 rows x 26880 x 9704 61.2 / 81.8 / 76.8 and 52.0 / 63.7 / 75.9,
+// 75 x 4096 x 11008 21.5 and 19.9, 100 x 11008 x 4096 23.9 and 23.2, 300 x 11008 x 4096 59 and 46.)
+template <bool RAGGED>
+struct RowWeights {
+    static constexpr int READS = 8;            // (pairs of dwords)
+    NibbleConsts nib;
+    int w_off, s_off;
+    uint32_t sel, half;                        // picks the first byte of two rows; the scales of the nibble
+    int last;
+    bool dead;
+    __device__ __forceinline__ RowWeights(int hh, int w, int s, uint32_t byte, int last_, bool dead_)
+        : nib(hh, hh == 0 ? 0x00800080u : 0x00080008u), w_off(w), s_off(s), sel(byte), half(hh == 0 ? 0x05040100u : 0x07060302u), last(last_), dead(dead_) {}
+    struct Regs { uint32_t w[8], s[8], keep; };
+    __device__ __forceinline__ Regs load(const uint8_t *st, int stage) const {
+        Regs x;
+        x.keep = RAGGED && stage == last && dead ? 0u : ~0u;
+#pragma unroll
+        for (int r = 0; r < 8; ++r) x.w[r] = *reinterpret_cast<const uint32_t *>(st + w_off + r * 128);
+#pragma unroll
+        for (int r = 0; r < 8; ++r) x.s[r] = *reinterpret_cast<const uint32_t *>(st + s_off + r * 8);
+        return x;
+    }
+    __device__ __forceinline__ uint32_t decode(const Regs &x, int j, int o) const {
+        const uint32_t pr = __builtin_amdgcn_perm(x.w[2 * j + 1], x.w[2 * j], o == 0 ? sel : sel + 0x00010001u);
+        const uint32_t pair = __builtin_amdgcn_perm(x.s[2 * j + 1], x.s[2 * j], half), sc = RAGGED ? pair & x.keep : pair;
+        return as_u32(nib.code((pr & nib.mask) ^ nib.magic) * as_h2(sc));
+    }
+};
+
 // The products of one multiplying wave of the kernels below: n stages of a ring of SLOTS slots, B operands (one nibble of one piece, 16 columns of either
 // byte) x TILES row tiles.  A wave keeps the A rows and the B operands of ONE stage in registers.  As soon as a row tile's two products are
 // issued its registers take the next stage's rows, and the next nibbles, read first, are decoded between the products: no read is waited for where it
@@ -132,18 +191,8 @@ template <int N> using int_constant = std::integral_constant<int, N>;
 // 448 of them on the matrix pipe.
 // Stages go in pairs, one barrier a pair (gemm_feed): at the barrier before stages i, i + 1 the stages up to i + 2 have landed, whose rows
 // and nibbles stage i + 1 reads; past the last stage stale bytes are read, decoded and never used.
-template <int TILES, int SLOTS, int STAGE, bool SPREAD = true>
-__device__ __forceinline__ void gemm_multiply(const uint8_t *lds, int n, int hh, int ws_off, int sc_off, int a_off, f4 (&acc)[2][TILES]) {
-    const uint32_t nib_mask = hh == 0 ? 0x00F000F0u : 0x000F000Fu;
-    uint32_t nib_magic = MAGIC_1024;                             // in a register the compiler cannot see through: (bits & mask) | magic is
-    asm volatile("" : "+v"(nib_magic));                       // then ONE v_and_or_b32 (no literal operands there), not an AND and an OR
-    const h2 nib_mul = hh == 0 ? h2{(half_t)0.0625f, (half_t)0.0625f} : h2{(half_t)1.0f, (half_t)1.0f};
-    const h2 nib_off = hh == 0 ? h2{(half_t)-72.0f, (half_t)-72.0f} : h2{(half_t)-1032.0f, (half_t)-1032.0f};
-    // half a row pair of the operands: rows (2 j, 2 j + 1) of the piece's first (o = 0) or second byte, codes + 8 -> exact fp16 code * scale
-    auto decode = [&](const u32x4 &wq, const u32x4 &scales, int j, int o, u32x4 (&b)[2]) {
-        const uint32_t w = wq[(j & 1) + 2 * o], pr = j < 2 ? w : w >> 8;
-        b[o][j] = as_u32(__builtin_elementwise_fma(as_h2((pr & nib_mask) | nib_magic), nib_mul, nib_off) * as_h2(scales[j]));
-    };
+template <int TILES, int SLOTS, int STAGE, bool SPREAD = true, class Weights>
+__device__ __forceinline__ void gemm_multiply(const uint8_t *lds, int n, const Weights &weights, int a_off, f4 (&acc)[2][TILES]) {
 #pragma unroll
     for (int o = 0; o < 2; ++o)
 #pragma unroll
@@ -153,17 +202,17 @@ __device__ __forceinline__ void gemm_multiply(const uint8_t *lds, int n, int hh,
     u32x4 bq[2];
     gemm_barrier();
     {
-        const u32x4 wq = *reinterpret_cast<const u32x4 *>(lds + ws_off), scales = *reinterpret_cast<const u32x4 *>(lds + sc_off);
+        const auto w = weights.load(lds, 0);
 #pragma unroll
         for (int t = 0; t < TILES; ++t) av[t] = *reinterpret_cast<const h8 *>(lds + a_off + t * 1024);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) decode(wq, scales, u >> 1, u & 1, bq);
+        for (int u = 0; u < 8; ++u) bq[u & 1][u >> 1] = weights.decode(w, u >> 1, u & 1);
     }
     int slot = 0;
-    auto one_stage = [&]() {
+    auto one_stage = [&](int next) {
         slot = slot == SLOTS - 1 ? 0 : slot + 1;
         const uint8_t *st = lds + slot * STAGE;                // of the next stage
-        const u32x4 wq = *reinterpret_cast<const u32x4 *>(st + ws_off), scales = *reinterpret_cast<const u32x4 *>(st + sc_off);
+        const auto w = weights.load(st, next);
         __builtin_amdgcn_sched_barrier(0);
         u32x4 bn[2];
         constexpr int FROM = TILES >= 4 ? 2 : TILES - 1;       // the row tile under whose products the decode begins
@@ -175,7 +224,7 @@ __device__ __forceinline__ void gemm_multiply(const uint8_t *lds, int n, int hh,
 #pragma unroll
             for (int u = 0; u < 8; ++u)
                 if (t == FROM + u * (TILES - FROM) / 8) {
-                    decode(wq, scales, u >> 1, u & 1, bn);
+                    bn[u & 1][u >> 1] = weights.decode(w, u >> 1, u & 1);
                     if constexpr (SPREAD) asm volatile("" : "+v"(bn[u & 1][u >> 1]));      // (here, not where it is needed)
                 }
             __builtin_amdgcn_sched_barrier(0);
@@ -183,22 +232,22 @@ __device__ __forceinline__ void gemm_multiply(const uint8_t *lds, int n, int hh,
         bq[0] = bn[0];
         bq[1] = bn[1];
     };
-    // The slots that are refilled behind a barrier were read a stage ago, by reads older than the last stage's TILES + 2
+    // The slots that are refilled behind a barrier were read a stage ago, by reads older than the last stage's TILES + READS
     auto meet = [] {
         __builtin_amdgcn_sched_barrier(0);
-        asm volatile("s_waitcnt lgkmcnt(%0)\n\ts_barrier" ::"n"(TILES + 2) : "memory");
+        asm volatile("s_waitcnt lgkmcnt(%0)\n\ts_barrier" ::"n"(TILES + Weights::READS < 15 ? TILES + Weights::READS : 15) : "memory");
         __builtin_amdgcn_sched_barrier(0);
     };
     int i = 0;
 #pragma unroll 1
     for (; i + 1 < n; i += 2) {
         meet();
-        one_stage();
-        one_stage();
+        one_stage(i + 1);
+        one_stage(i + 2);
     }
     if (i < n) {
         meet();
-        one_stage();
+        one_stage(i + 1);
     }
 }
 
@@ -524,15 +573,20 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
     // before steps i, i+1 the stages of steps i .. i+2 have landed (the B operands of step i+2 are decoded during step i+1),
     // steps i+3 .. i+S-3 may be in flight, and the slots of steps i-2, i-1 are refilled with steps i+S-2, i+S-1.  A stage has the same two steps of time to land as
     // with a barrier per step; the waves meet half as often.
-    if constexpr (PRODUCER && TILED && !RAGGED) {
-        gemm_multiply<TILES, SLOTS, GS_BYTES>(lds, n_steps, hh, wave * 1024 + lane * 16, GS_W + g * 64 + (2 * blk + hh) * 16,
-                                              GS_W + GS_S + c * 64 + ((g ^ ((c >> 1) & 3)) << 4), acc);
+    if constexpr (PRODUCER) {
+        // (the end of K is stage `at_end` of a slice that has it)
+        const int end = (p.K - 1) / 32 - step0, at_end = RAGGED && step1 > (p.K - 1) / 32 ? (end >= rot ? end - rot : end - rot + n_steps) : -1;
+        const auto weights = [&] {
+            if constexpr (TILED) return TiledWeights(hh, wave * 1024 + lane * 16, GS_W + g * 64 + (2 * blk + hh) * 16);
+            else return RowWeights<RAGGED>(hh, g * GS_WBLOCK + 64 * blk + 4 * c, GS_W + 64 * g + 4 * blk, sel0, at_end, (p.K - 1) / 32 * 32 + 8 * g >= p.K);
+        }();
+        gemm_multiply<TILES, SLOTS, GS_BYTES>(lds, n_steps, weights, GS_W + GS_S + c * 64 + ((g ^ ((c >> 1) & 3)) << 4), acc);
     } else if (n_steps > 0) {
         h8 bq[NB];
         int cur = step0 + rot;                 // step being multiplied
         int slot = 0;                          // its ring slot
         {
-            if constexpr (!PRODUCER) gemm_wait_dma<DMA_PER>(min(SLOTS - 3, n_steps - 1));
+            gemm_wait_dma<DMA_PER>(min(SLOTS - 3, n_steps - 1));
             gemm_barrier();
             uint32_t wv[8], sv[8];
             load_ws(lds, wv, sv);
@@ -557,12 +611,9 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
         int i = 0;
 #pragma unroll 1
         for (; i + SLOTS - 1 < n_steps; i += 2) {      // both refills exist: the body is one basic block
-            if constexpr (!PRODUCER) gemm_wait_vm<DMA_PER * (SLOTS - 5)>();
+            gemm_wait_vm<DMA_PER * (SLOTS - 5)>();
             gemm_barrier();
-            if constexpr (PRODUCER) {
-                one_step();
-                one_step();
-            } else if constexpr (WAVES == 8 && TILES < 8) {       // (with all 8 row tiles, the prefill, this form measured 5-8 % slower)
+            if constexpr (WAVES == 8 && TILES < 8) {       // (with all 8 row tiles, the prefill, this form measured 5-8 % slower)
                 // the nibbles and scales of the two refills now, their A rows from inside the steps: the address unit takes
                 // 16 cycles per instruction, and between MFMAs the wave has them to spare (2 % off a launch at 100 rows;
                 // the nibbles and scales too from inside the steps, behind their branches: 4 % slower)
@@ -604,12 +655,10 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
         }
 #pragma unroll 1
         for (; i < n_steps; i += 2) {
-            if constexpr (!PRODUCER) gemm_wait_dma<DMA_PER>(max(0, min(n_steps - 1, i + SLOTS - 3) - (i + 2)));      // stages issued past step i + 2
+            gemm_wait_dma<DMA_PER>(max(0, min(n_steps - 1, i + SLOTS - 3) - (i + 2)));      // stages issued past step i + 2
             gemm_barrier();
-            if constexpr (!PRODUCER) {
-                if (i + SLOTS - 2 < n_steps) fetch_next(back(2));
-                if (i + SLOTS - 1 < n_steps) fetch_next(back(1));
-            }
+            if (i + SLOTS - 2 < n_steps) fetch_next(back(2));
+            if (i + SLOTS - 1 < n_steps) fetch_next(back(1));
             one_step();
             if (i + 1 < n_steps) one_step();
         }
@@ -833,7 +882,7 @@ __global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_kg_kern
 
     const int kk = wave8 >> 2, hh = (wave8 >> 1) & 1, bp = wave8 & 1;
     f4 acc[2][TILES];
-    gemm_multiply<TILES, SLOTS, STAGE>(lds, n_st, hh, (2 * kk + bp) * 1024 + lane * 16, KG_W + kk * 256 + g * 64 + (2 * blk + hh) * 16,
+    gemm_multiply<TILES, SLOTS, STAGE>(lds, n_st, TiledWeights(hh, (2 * kk + bp) * 1024 + lane * 16, KG_W + kk * 256 + g * 64 + (2 * blk + hh) * 16),
                                        KG_W + KG_S + kk * TILES * 1024 + c * 64 + ((g ^ ((c >> 1) & 3)) << 4), acc);
 
     // ---- both groups' sums as rows of 128 floats in LDS; then every thread adds group 0 + group 1 (a fixed order) for
@@ -937,7 +986,7 @@ __global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_swiglu_
 
     const int kk = wave8 >> 2, hh = (wave8 >> 1) & 1, gu = wave8 & 1;       // K-group, nibble, gate (0) or up (1)
     f4 acc[2][TILES];
-    gemm_multiply<TILES, SLOTS, STAGE>(lds, n_st, hh, (2 * kk + gu) * 1024 + lane * 16, KG_W + (2 * kk + gu) * 256 + g * 64 + (2 * blk + hh) * 16,
+    gemm_multiply<TILES, SLOTS, STAGE>(lds, n_st, TiledWeights(hh, (2 * kk + gu) * 1024 + lane * 16, KG_W + (2 * kk + gu) * 256 + g * 64 + (2 * blk + hh) * 16),
                                        KG_W + S::SC + kk * TILES * 1024 + c * 64 + ((g ^ ((c >> 1) & 3)) << 4), acc);
 
     // ---- both groups' sums as rows of 64 gate and 64 up columns in LDS, then every thread adds group 0 + group 1 (a fixed order) of four columns ----
@@ -1088,7 +1137,7 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + GEMM_DMA_WAVES), 1) void q40_gem
     const int hh = wave >= 6 ? 1 : 0, s = wave - 6 * hh, half = s >= PIECES ? 1 : 0, k3 = s - 3 * half;
     f4 acc[2][TILES];
     // (seven row tiles: the decode where the compiler puts it; spread, these spill in the 128 registers of four waves a SIMD)
-    gemm_multiply<TILES, SLOTS, STAGE, SWIGLU || TILES != 7>(lds, n_st, hh, s * 1024 + lane * 16, S::W + s * 128 + g * 32 + hh * 16,
+    gemm_multiply<TILES, SLOTS, STAGE, SWIGLU || TILES != 7>(lds, n_st, TiledWeights(hh, s * 1024 + lane * 16, S::W + s * 128 + g * 32 + hh * 16),
                                        S::W + S::SC + (MODE == WIDE_GROUPS ? half * TILES * 1024 : 0) + c * 64 + ((g ^ ((c >> 1) & 3)) << 4), acc);
 
     // rows of 64 PIECES columns: local column 64 k3 + 32 hh + 2 c + o is column 128 (P / 2) + 64 hh + 4 c + 2 (P % 2) + o, P the piece;

@@ -309,3 +309,17 @@ def test_consumers_at_every_number_of_slabs(ks):
             results.append(out + [q, k, v])
         for i, (a, b) in enumerate(zip(*results)):
             assert bool(a.float().isfinite().all()) and torch.equal(a, b), (i, M, n)
+
+
+@pytest.mark.parametrize("M", [17, 61, 80, 100, 128, 300])
+@pytest.mark.parametrize("K,N", [(2056, 11008), (4112, 4096), (6168, 3712), (264, 8192), (8168, 16384), (4096, 4096), (224, 4096)])
+def test_checkpoint_products_at_the_end_of_k(M, K, N):
+    """17 rows and more on the checkpoint layout: the end of K (8, 16, 24 or 32 rows of its last step) lies in one slice of K, in whichever stage
+    of the ring that slice's start makes it, and adds nothing past K.  Against 64 bits: half a unit of fp16 and the fp32 sums"""
+    from spec_mcts_amd import kernels as Kn
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    w, s = Kn.quantize_q40(torch.randn((K, N), device="cuda", generator=g, dtype=torch.float16) * 0.02)
+    x = torch.randn((M, K), device="cuda", generator=g, dtype=torch.float16)
+    got = Kn.matmul_q40(x, w, s, (K, N)).double()
+    want = x.double() @ Kn.deq_int40(w, s, 64, (K, N)).double()
+    assert bool(((got - want).abs() <= want.abs() * 2.0 ** -11 + 2.0 ** -24 * K ** 0.5 * want.abs().max()).all())
