@@ -191,7 +191,8 @@ struct RowWeights {
 // 448 of them on the matrix pipe.
 // Stages go in pairs, one barrier a pair (gemm_feed): at the barrier before stages i, i + 1 the stages up to i + 2 have landed, whose rows
 // and nibbles stage i + 1 reads; past the last stage stale bytes are read, decoded and never used.
-template <int TILES, int SLOTS, int STAGE, bool SPREAD = true, class Weights>
+// Not AHEAD: a stage's rows are read in it, and the compiler puts reads and decode where it likes.
+template <int TILES, int SLOTS, int STAGE, bool AHEAD = true, class Weights>
 __device__ __forceinline__ void gemm_multiply(const uint8_t *lds, int n, const Weights &weights, int a_off, f4 (&acc)[2][TILES]) {
 #pragma unroll
     for (int o = 0; o < 2; ++o)
@@ -203,15 +204,33 @@ __device__ __forceinline__ void gemm_multiply(const uint8_t *lds, int n, const W
     gemm_barrier();
     {
         const auto w = weights.load(lds, 0);
+        if constexpr (AHEAD) {
 #pragma unroll
-        for (int t = 0; t < TILES; ++t) av[t] = *reinterpret_cast<const h8 *>(lds + a_off + t * 1024);
+            for (int t = 0; t < TILES; ++t) av[t] = *reinterpret_cast<const h8 *>(lds + a_off + t * 1024);
+        }
 #pragma unroll
         for (int u = 0; u < 8; ++u) bq[u & 1][u >> 1] = weights.decode(w, u >> 1, u & 1);
     }
     int slot = 0;
     auto one_stage = [&](int next) {
+        const uint8_t *here = lds + slot * STAGE;
         slot = slot == SLOTS - 1 ? 0 : slot + 1;
         const uint8_t *st = lds + slot * STAGE;                // of the next stage
+        if constexpr (!AHEAD) {
+            u32x4 bn[2];
+#pragma unroll
+            for (int t = 0; t < TILES; ++t) av[t] = *reinterpret_cast<const h8 *>(here + a_off + t * 1024);
+            const auto w = weights.load(st, next);
+#pragma unroll
+            for (int t = 0; t < TILES; ++t)
+#pragma unroll
+                for (int o = 0; o < 2; ++o) acc[o][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[t], __builtin_bit_cast(h8, bq[o]), acc[o][t], 0, 0, 0);
+#pragma unroll
+            for (int u = 0; u < 8; ++u) bn[u & 1][u >> 1] = weights.decode(w, u >> 1, u & 1);
+            bq[0] = bn[0];
+            bq[1] = bn[1];
+            return;
+        }
         const auto w = weights.load(st, next);
         __builtin_amdgcn_sched_barrier(0);
         u32x4 bn[2];
@@ -225,7 +244,7 @@ __device__ __forceinline__ void gemm_multiply(const uint8_t *lds, int n, const W
             for (int u = 0; u < 8; ++u)
                 if (t == FROM + u * (TILES - FROM) / 8) {
                     bn[u & 1][u >> 1] = weights.decode(w, u >> 1, u & 1);
-                    if constexpr (SPREAD) asm volatile("" : "+v"(bn[u & 1][u >> 1]));      // (here, not where it is needed)
+                    asm volatile("" : "+v"(bn[u & 1][u >> 1]));      // (here, not where it is needed)
                 }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -234,6 +253,7 @@ __device__ __forceinline__ void gemm_multiply(const uint8_t *lds, int n, const W
     };
     // The slots that are refilled behind a barrier were read a stage ago, by reads older than the last stage's TILES + READS
     auto meet = [] {
+        if constexpr (!AHEAD) return gemm_barrier();
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("s_waitcnt lgkmcnt(%0)\n\ts_barrier" ::"n"(TILES + Weights::READS < 15 ? TILES + Weights::READS : 15) : "memory");
         __builtin_amdgcn_sched_barrier(0);
@@ -1136,8 +1156,9 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + GEMM_DMA_WAVES), 1) void q40_gem
     // nibble, slot; the slot's half - gate (0) or up (1), or K-group - and piece
     const int hh = wave >= 6 ? 1 : 0, s = wave - 6 * hh, half = s >= PIECES ? 1 : 0, k3 = s - 3 * half;
     f4 acc[2][TILES];
-    // (seven row tiles: the decode where the compiler puts it; spread, these spill in the 128 registers of four waves a SIMD)
-    gemm_multiply<TILES, SLOTS, STAGE, SWIGLU || TILES != 7>(lds, n_st, TiledWeights(hh, s * 1024 + lane * 16, S::W + s * 128 + g * 32 + hh * 16),
+    // (Seven row tiles: reading ahead needs more than the 128 registers of four waves a SIMD, and does not gain what that costs.  In us, ahead and not:
+    // w1|w3 and wq|wk|wv of the 7B shape at 400 rows 90.1, 52.9 and 86.2, 49.3, w1|w3 of the 70B shape at 540 rows 551 and 524.)
+    gemm_multiply<TILES, SLOTS, STAGE, TILES != 7>(lds, n_st, TiledWeights(hh, s * 1024 + lane * 16, S::W + s * 128 + g * 32 + hh * 16),
                                        S::W + S::SC + (MODE == WIDE_GROUPS ? half * TILES * 1024 : 0) + c * 64 + ((g ^ ((c >> 1) & 3)) << 4), acc);
 
     // rows of 64 PIECES columns: local column 64 k3 + 32 hh + 2 c + o is column 128 (P / 2) + 64 hh + 4 c + 2 (P % 2) + o, P the piece;
