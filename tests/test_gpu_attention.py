@@ -298,6 +298,39 @@ def test_attention_of_sixteen_queries_a_workgroup_matches_the_three_launch_seque
         assert torch.equal(got_nan, got)
 
 
+@pytest.mark.parametrize("B,H,Hkv,P", [(17, 4, 4, 100), (20, 8, 2, 530), (100, 32, 32, 130), (40, 64, 8, 1030)])
+@pytest.mark.parametrize("where", ["first", "last", "one of many", "both signs"])
+def test_infinite_prompt_values_stay_infinite_in_one_launch(B, H, Hkv, P, where):
+    """An infinity in a row of the prompt's V: that dimension is infinite in every branch's output (NaN where +inf and -inf meet, as a
+    sum of the two is), all others are what they are with a finite value there - bit for bit but for what fp16 rounds off a probability (2^-11 of
+    a mean of values below 3).  With eight queries a workgroup and with 16."""
+    from spec_mcts_amd import kernels as K
+    dev, D, Smax, t = "cuda:0", 128, 8, 3
+    g = torch.Generator().manual_seed(40 + B)
+    half = lambda *shape, std=0.5: (torch.randn(shape, generator=g) * std).half().to(dev)
+    qkv = K.PartialProduct(torch.randn((2, B, (H + 2 * Hkv) * D), generator=g).to(dev), 2, B, (H + 2 * Hkv) * D)
+    cos, sin = half(64, 64), half(64, 64)
+    pos_dev, t_dev = (torch.tensor([x], dtype=torch.int32, device=dev) for x in (7, t))
+    pk, pv = half(P, Hkv, D), half(P, Hkv, D)
+    ck, cv = (torch.randint(-128, 128, (B, Smax, Hkv, 64), generator=g, dtype=torch.int16).to(torch.int8).to(dev) for _ in range(2))
+    cks, cvs = ((torch.rand((B, Smax, Hkv, 2), generator=g) * 0.1 + 0.01).half().to(dev) for _ in range(2))
+    run = lambda: K.shared_prefix_attn_qkv_tiles(qkv, H, Hkv, D, cos, sin, pos_dev, pk, pv, P, ck, cks, cv, cvs, Smax, t_dev)
+    inf, row = float("inf"), {"first": 0, "last": P - 1}.get(where, P // 2)
+    pv[row, 0, 77] = 1.0
+    clean = run().view(B, Hkv, H // Hkv, D)
+    pv[row, 0, 77] = -inf
+    if where == "both signs":
+        pv[row - 1, 0, 77] = inf
+    got = run().view(B, Hkv, H // Hkv, D)
+    torch.cuda.synchronize()
+    assert clean.isfinite().all()
+    hit = got[:, 0, :, 77]
+    assert hit.isnan().all() if where == "both signs" else (hit == -inf).all()
+    got[:, 0, :, 77] = clean[:, 0, :, 77]
+    assert torch.equal(got[:, 1:], clean[:, 1:])
+    assert torch.allclose(got.float(), clean.float(), rtol=2e-3, atol=2e-3)
+
+
 @pytest.mark.parametrize("B,H,Hkv,P,L", [(100, 4, 4, 150, 9), (33, 8, 2, 70, 4), (5, 4, 4, 0, 6), (128, 2, 2, 40, 0)])
 def test_one_launch_attention_matches_two_launches(B, H, Hkv, P, L):
     """smh_shared_prefix_attn_one against smh_shared_prefix_attn on the same inputs (Q4_0 suffix, new token):
