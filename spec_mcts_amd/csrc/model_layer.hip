@@ -53,7 +53,7 @@ static AttnWay attn_way(int M, int heads, int kv_heads, int P, bool one, bool ti
     if (tiles && P >= ATTN_TILES_MIN_PROMPT && (rep > 1 || (M > SMH_GEMV_MAX_M && round)) &&
         (P <= 512 || P <= kv_heads * ((queries + 7) / 8) * (rep == 1 ? 12 : 24)))
         return ATTN_TILES;
-    return launches ? ATTN_LAUNCHES : one ? ATTN_ONE : ATTN_TILES;
+    return one && !launches ? ATTN_ONE : ATTN_LAUNCHES;
 }
 
 static int layer_buffers(const smh_layer &L, int M, bool swiglu_in, char *base, LayerBuffers &b) {
@@ -165,10 +165,14 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
             if ((uintptr_t)x % to != 0) return false;
         return true;
     };
-    const bool can_tile = S.attn_from_qkv != 0 && !qkv_direct && aligned({L.prompt_k, L.prompt_v}, 16) && aligned({S.cos_tab, S.sin_tab, L.cache_k, L.cache_v}, 8) &&
-                          aligned({L.cache_ks, L.cache_vs}, 4) && (long)L.prompt_len * L.kv_heads * 256 < (1L << 32) && rows * L.kv_heads * 64 < (1L << 32);
-    const AttnWay way = attn_way(M, L.heads, L.kv_heads, L.prompt_len, S.attn_one != 0 && M * rep <= 16, can_tile,
-                                 S.attn_ws != nullptr || S.attn_one == 0 || M * rep > 16);
+    // What only some of the three ask for never decides whether a pass is taken.  A table of another width than a branch has rows: TILES and ONE cut the
+    // walks at the rows, LAUNCHES at the table.  TILES and LAUNCHES check page ids against cache_rows, LAUNCHES writes partials to attn_ws.
+    const bool may_one = S.attn_one != 0 && M * rep <= 16, table = S.pages == nullptr || (S.pages_stride == S.smax && S.cache_rows >= 1);
+    const bool can_launch = table && S.attn_ws != nullptr && S.attn_ws_bytes >= smh_attn_workspace_bytes(M, L.heads, L.prompt_len);
+    const bool can_tile = S.attn_from_qkv != 0 && !qkv_direct && table && aligned({L.prompt_k, L.prompt_v}, 16) &&
+                          aligned({S.cos_tab, S.sin_tab, L.cache_k, L.cache_v}, 8) && aligned({L.cache_ks, L.cache_vs}, 4) &&
+                          (long)L.prompt_len * L.kv_heads * 256 < (1L << 32) && rows * L.kv_heads * 64 < (1L << 32);
+    const AttnWay way = attn_way(M, L.heads, L.kv_heads, L.prompt_len, may_one, can_tile, can_launch);
     const int one = way == ATTN_ONE;
     void *ws = one ? S.attn_one_ws : S.attn_ws;
     const size_t ws_bytes = one ? S.attn_one_ws_bytes : S.attn_ws_bytes;

@@ -95,3 +95,47 @@ def test_decode_above_128_branches(cfg, B, swiglu):
         print(f"B={B} step {step}: largest logit difference {float((got - want).abs().max()):.4f}", flush=True)
         assert torch.allclose(got, want, rtol=1e-2, atol=1e-2)
         sync_suffix_row(model, oracle, B, step)
+
+
+def _layer_pass(model, h, t, pages, from_qkv=1, **fields):
+    """One decode step of a model of one layer by smh_decode_layer; fields: of its smh_pass, in place of the model's own."""
+    from spec_mcts_amd import kernels as K
+    p, B, dev = model.params, h.shape[0], h.device
+    s = model._layer_struct(model.layers[0])
+    run = K.LayerPass(s, B, h, *model._tables(dev), True)
+    state = torch.tensor([s.prompt_len + t, t], dtype=torch.int32, device=dev)
+    one = B * s.heads <= 16 * s.kv_heads
+    run.decode_step((state[:1], state[1:]), K.attn_workspace(dev, B, s.heads, s.prompt_len), K.attn_qkv_workspace(dev, B, s.heads, s.prompt_len) if one else None,
+                    p.max_seq_len, p.max_batch_size * p.max_seq_len, None, 0, 0, from_qkv)
+    if pages is not None:
+        run.p.pages, run.p.pages_stride = pages.data_ptr(), pages.stride(0)
+    for name, value in fields.items():
+        setattr(run.p, name, value)
+    run.decode(s)
+    return run.finish(s, model.norm.weight, model.norm.eps)
+
+
+@pytest.mark.parametrize("heads,kv_heads,B,P,change", [(2, 2, 17, 100, "narrow table"), (4, 2, 40, 300, "narrow table"), (2, 2, 10, 800, "no row count"), (4, 2, 5, 300, "no row count"),
+                                                       (2, 2, 10, 800, "small workspace"), (4, 2, 5, 900, "small workspace")])
+def test_passes_that_only_some_forms_of_the_attention_take(heads, kv_heads, B, P, change):
+    """A table of fewer columns than a branch has rows (t lies in it), no number of cache rows, a workspace for the one-launch form only: what the
+    forms a layer is usually given to ask for, and others do not.  The result is that of the form that takes it, bit for bit."""
+    cfg = dict(dim=128 * heads, n_layers=1, n_heads=heads, n_kv_heads=kv_heads, vocab_size=320, multiple_of=128, max_batch_size=B, max_seq_len=8, max_prompt_seq_len=1024)
+    _, _, model = _build(cfg, 90 + B, 0.05)
+    att, t = model.layers[0].attention, 3
+    g = torch.Generator(device="cuda:0").manual_seed(B)
+    normal = lambda *shape: torch.randn(shape, generator=g, device="cuda:0", dtype=torch.float16)
+    att.cache_prompt_k[0, :P], att.cache_prompt_v[0, :P] = normal(P, kv_heads, 128), normal(P, kv_heads, 128)
+    att.cache_prompt_len = P
+    h = normal(B, cfg["dim"])
+    rows = torch.arange(B, dtype=torch.int32, device="cuda:0")[:, None] * 8 + torch.arange(8, dtype=torch.int32, device="cuda:0")
+    for i in range(t):
+        _layer_pass(model, normal(B, cfg["dim"]), i, None)
+    if change == "narrow table":
+        want = _layer_pass(model, h, t, rows, from_qkv=0)
+        got = _layer_pass(model, h, t, rows[:, :6].contiguous())
+    else:                                              # (with neither, only the one-launch form takes it)
+        want = _layer_pass(model, h, t, rows, attn_ws=None, cache_rows=0)
+        got = _layer_pass(model, h, t, rows, **(dict(cache_rows=0) if change == "no row count" else dict(attn_ws_bytes=256)))
+    torch.cuda.synchronize()
+    assert want.isfinite().all() and torch.equal(got, want)
