@@ -624,11 +624,13 @@ __global__ __launch_bounds__(1024) void sample_topk_kernel(const half_t *__restr
         return;
     }
     if (tid < k) {
-        for (int j = 0; j < draws; ++j) {
-            const float target = (j < 64 ? s_uniform[j] : uniform[first + j]) * all;
-            // first candidate whose cumulative probability exceeds the target (the last one if rounding leaves none)
+        // first candidate whose cumulative probability exceeds the target (the last one if rounding leaves none)
+        auto draw = [&](int j, float target) {
             if ((before <= target && target < upto) || (tid == k - 1 && target >= upto)) out[first + j] = o_idx[tid];
-        }
+        };
+        // (two loops: one load from either address would be a flat one)
+        for (int j = 0; j < min(draws, 64); ++j) draw(j, s_uniform[j] * all);
+        for (int j = 64; j < draws; ++j) draw(j, uniform[first + j] * all);
     }
 }
 

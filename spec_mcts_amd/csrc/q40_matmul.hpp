@@ -81,7 +81,7 @@ struct MatmulParams {
 // p.seg[sg] without a load that waits for sg
 __device__ __forceinline__ MatmulSegment segment_at(const MatmulParams &p, int sg) {
     MatmulSegment r = p.seg[0];
-    auto pick = [&](auto member) { 
+    auto pick = [&](auto member) {
         const auto a = held(p.seg[0].*member), b = held(p.seg[1].*member), c = held(p.seg[2].*member);
         r.*member = sg == 0 ? a : sg == 1 ? b : c;
     };
