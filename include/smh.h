@@ -404,9 +404,11 @@ int smh_shared_prefix_attn_qkv(const void *qkv_partial, int ksplit, void *out, i
                                const int32_t *t_dev, const int32_t *pages, int pages_stride, int single_launch,
                                void *workspace, size_t workspace_bytes, smh_stream_t stream);
 
-/* smh_shared_prefix_attn_qkv_tiles: the same from any number of branches in ONE launch without a workspace: a workgroup has 16 queries of
+/* smh_shared_prefix_attn_qkv_tiles: the same from any number of branches in ONE launch without a workspace: a workgroup has 8 or 16 queries of
  * a kv head, reads the whole prefix for them and walks their branches' rows (the faster form where these workgroups fit the GPU in one
- * round).  Equal to the other forms up to fp32 summation order.  pages: rows of a pool of cache_rows rows (not read without pages). */
+ * round).  Equal to the other forms up to fp32 summation order.  pages: rows of a pool of cache_rows rows (not read without pages).
+ * Refused: slabs or prefix that are not 16-byte aligned, out, tables or codes not 8-byte, scales not 4-byte aligned; a prefix or a cache
+ * (codes) of 4 GiB and more. */
 int smh_shared_prefix_attn_qkv_tiles(const void *qkv_partial, int ksplit, void *out, int B, int H, int Hkv, int D,
                                      const void *cos_tab, const void *sin_tab, const int32_t *pos_dev,
                                      const void *prefix_k, const void *prefix_v, int P,

@@ -23,6 +23,7 @@
 #include <type_traits>
 
 #include "attn_rows.hpp"
+#include "attn_tiles.hpp"
 #include "rope_kv.hpp"
 
 namespace smh {
@@ -2335,6 +2336,9 @@ extern "C" int smh_shared_prefix_attn_qkv_tiles(const void *qkv_partial, int ksp
     SMH_REQUIRE(cache_k && cache_ks && cache_v && cache_vs && t_dev && Smax > 0, "%s: the suffix cache and its row counter are required", who);
     SMH_REQUIRE(pages == nullptr || (pages_stride >= Smax && cache_rows >= 1), "%s: pages_stride=%d must cover the %d rows of a branch, cache_rows=%ld", who,
                 pages_stride, Smax, cache_rows);
+    const char *const why = attn_tiles_refuse({qkv_partial, out, cos_tab, sin_tab, prefix_k, prefix_v, cache_k, cache_ks, cache_v, cache_vs, B, H, Hkv, P,
+                                               pages != nullptr ? cache_rows : (long)B * Smax});
+    SMH_REQUIRE(why == nullptr, "%s: %s", who, why);
     AttnParams p{};
     p.out = (half_t *)out;
     p.prefix_k = (const half_t *)prefix_k; p.prefix_v = (const half_t *)prefix_v;
@@ -2365,13 +2369,7 @@ extern "C" int smh_shared_prefix_attn_qkv_tiles(const void *qkv_partial, int ksp
         return e;
     }();
     if (lds_ok != hipSuccess) { set_error("%s: the kernel's LDS could not be reserved: %s", who, hipGetErrorString(lds_ok)); return (int)lds_ok; }
-    SMH_REQUIRE((long)P * Hkv * ATT_D * 2 < (1L << 32), "%s: P=%d rows of %d heads exceed the 32-bit offsets of the prefix", who, P, Hkv);
-    const long rows = pages != nullptr ? cache_rows : (long)B * Smax;
-    SMH_REQUIRE(rows * Hkv * 64 < (1L << 32) && rows < (1L << 31), "%s: %ld cache rows of %d heads exceed the 32-bit offsets of the cache", who, rows, Hkv);
-    // Eight queries a workgroup while those fill one round of compute units, else 16 (us, 16 and 8: 32 heads, 64 branches after 512 rows 24.4 and
-    // 19.4, 17 20.5 and 14.2, 100, two rounds of eight, 24.1 and 30.6; 64 heads over 8, 30 branches after 2047 rows 26.3 and 23.7, 100 48.8 and 76.3)
-    const int qt = (long)Hkv * ((p.Bq + 7) / 8) <= 256 ? 8 : 16, tiles = (p.Bq + qt - 1) / qt;
-    SMH_REQUIRE(tiles <= 65535 && Hkv <= 8 * 65535, "%s: %d tiles of queries, %d heads", who, tiles, Hkv);
+    const int qt = attn_tile_queries(p.Bq, Hkv), tiles = (p.Bq + qt - 1) / qt;
     const int chunks = (P + AT_CHUNK - 1) / AT_CHUNK;
     hipLaunchKernelGGL(kern[qt == 16][pages != nullptr][ksplit <= 2 ? 0 : ksplit <= 6 ? 1 : 2], dim3(8, (Hkv + 7) / 8, tiles), dim3(64 * AT_WAVES), AT_LDS,
                        (hipStream_t)stream, p, chunks);

@@ -5,9 +5,7 @@
 // 32-layer model took 3.0 ms where a captured graph of the same launches takes 2.0.  Here the layer's launches are issued one
 // behind the other (2-3 us each), out of buffers the caller allocated once for the whole pass.  The sequence, the operators
 // and their switches are those of Transformer._forward_fused in hf_model_q40_kv_shared.py.
-#include <initializer_list>
-
-#include "smh_common.hpp"
+#include "attn_tiles.hpp"
 
 namespace smh {
 
@@ -160,18 +158,13 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
     const int rep = L.heads / L.kv_heads;
     const bool qkv_direct = direct(M, L.dim, 3, run.n_qkv);
     const long rows = S.pages != nullptr ? S.cache_rows : (long)M * S.smax;
-    auto aligned = [](std::initializer_list<const void *> list, uintptr_t to) {
-        for (const void *x : list)
-            if ((uintptr_t)x % to != 0) return false;
-        return true;
-    };
     // What only some of the three ask for never decides whether a pass is taken.  A table of another width than a branch has rows: TILES and ONE cut the
     // walks at the rows, LAUNCHES at the table.  TILES and LAUNCHES check page ids against cache_rows, LAUNCHES writes partials to attn_ws.
     const bool may_one = S.attn_one != 0 && M * rep <= 16, table = S.pages == nullptr || (S.pages_stride == S.smax && S.cache_rows >= 1);
     const bool can_launch = table && S.attn_ws != nullptr && S.attn_ws_bytes >= smh_attn_workspace_bytes(M, L.heads, L.prompt_len);
-    const bool can_tile = S.attn_from_qkv != 0 && !qkv_direct && table && aligned({L.prompt_k, L.prompt_v}, 16) &&
-                          aligned({S.cos_tab, S.sin_tab, L.cache_k, L.cache_v}, 8) && aligned({L.cache_ks, L.cache_vs}, 4) &&
-                          (long)L.prompt_len * L.kv_heads * 256 < (1L << 32) && rows * L.kv_heads * 64 < (1L << 32);
+    const bool can_tile = S.attn_from_qkv != 0 && !qkv_direct && table &&
+                          attn_tiles_refuse({b.slab_a, b.att, S.cos_tab, S.sin_tab, L.prompt_k, L.prompt_v, L.cache_k, L.cache_ks, L.cache_v, L.cache_vs, M,
+                                             L.heads, L.kv_heads, L.prompt_len, rows}) == nullptr;
     const AttnWay way = attn_way(M, L.heads, L.kv_heads, L.prompt_len, may_one, can_tile, can_launch);
     const int one = way == ATTN_ONE;
     void *ws = one ? S.attn_one_ws : S.attn_ws;

@@ -861,20 +861,27 @@ def shared_prefix_attn_qkv_tiles(p: PartialProduct, H: int, Hkv: int, D: int, co
                                  pos_dev: torch.Tensor, prefix_k: Optional[torch.Tensor], prefix_v: Optional[torch.Tensor], P: int,
                                  cache_k: torch.Tensor, cache_ks: torch.Tensor, cache_v: torch.Tensor, cache_vs: torch.Tensor,
                                  Smax: int, t_dev: torch.Tensor, pages: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """shared_prefix_attn_qkv for any number of branches, in one launch whose workgroups have 16 queries of a kv head each and read the whole
+    """shared_prefix_attn_qkv for any number of branches, in one launch whose workgroups have 8 or 16 queries of a kv head each and read the whole
     prefix for them.  pages: int32 [>= B, >= Smax] ids of the caches' rows."""
     lib = _lib.load()
     B = p.M
+    half, rows = torch.float16, B * Smax * Hkv
     if pages is not None:
         assert pages.is_cuda and pages.dtype == torch.int32 and pages.dim() == 2 and pages.stride(1) == 1
         assert pages.shape[0] >= B and pages.shape[1] >= Smax
-    assert p.n_total == (H + 2 * Hkv) * D and p.buf.dtype == torch.float32
-    _need_gpu(p.buf, cache_k, cache_v, cache_ks, cache_vs, t_dev, pos_dev)
+    assert p.n_total == (H + 2 * Hkv) * D and p.buf.dtype == torch.float32 and p.buf.is_contiguous()
+    _need_gpu(p.buf, cache_k, cache_v, cache_ks, cache_vs, t_dev, pos_dev, cos, sin)
+    for c in (cos, sin):
+        assert c.is_contiguous() and c.dtype == half and c.shape[-1] == D // 2
     if prefix_k is not None:
-        assert prefix_k.is_contiguous() and prefix_v.is_contiguous() and prefix_k.dtype == torch.float16 and P <= prefix_k.shape[-3]
+        for c in (prefix_k, prefix_v):
+            assert c.is_contiguous() and c.dtype == half and tuple(c.shape[-2:]) == (Hkv, D) and P <= c.shape[-3]
     else:
         assert P == 0
-    assert cache_k.dtype == torch.int8 and cache_ks.dtype == torch.float16 and t_dev.dtype == torch.int32
+    for c, s in ((cache_k, cache_ks), (cache_v, cache_vs)):
+        assert c.is_contiguous() and c.dtype == torch.int8 and c.numel() >= 64 * rows and c.numel() % (64 * Hkv) == 0
+        assert s.is_contiguous() and s.dtype == half and s.numel() * 32 == cache_k.numel() and c.numel() == cache_k.numel()
+    assert t_dev.dtype == torch.int32 and pos_dev.dtype == torch.int32
     out = torch.empty((B, H, D), dtype=torch.float16, device=p.buf.device)
     check(lib.smh_shared_prefix_attn_qkv_tiles(p.buf.data_ptr(), p.ksplit, out.data_ptr(), B, H, Hkv, D, cos.data_ptr(), sin.data_ptr(),
                                                pos_dev.data_ptr(), _ptr(prefix_k), _ptr(prefix_v), int(P),

@@ -6,6 +6,7 @@ import shutil
 import subprocess
 
 import pytest
+import torch
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -55,6 +56,56 @@ def test_argument_errors_are_reported_without_a_gpu():
     st = lib.smh_shared_prefix_attn_static(None, None, 4096, 64, 64, 128, None, None, 4096, 0, None, None, None, None, 0, None, 0,
                                            None, None, None)
     assert st < 0 and b"static array holds" in lib.smh_last_error_string()
+
+
+@pytest.mark.parametrize("name,align", [("slabs", 16), ("prefix_k", 16), ("prefix_v", 16), ("out", 8), ("cos", 8), ("sin", 8), ("cache_k", 8), ("cache_v", 8), ("cache_ks", 4),
+                                        ("cache_vs", 4), ("P", 0), ("cache_rows", 0), ("B", 0)])
+def test_tile_attention_refuses_what_its_loads_cannot_take(name, align):
+    """... before anything touches the device: the alignment of every tensor, sizes past 32-bit offsets, more tiles than a grid has."""
+    from spec_mcts_amd import _lib
+    lib = _lib.load()
+    a = dict(slabs=1 << 20, ksplit=2, out=1 << 21, B=17, H=4, Hkv=4, D=128, cos=1 << 22, sin=1 << 22, pos=1 << 12, prefix_k=1 << 23, prefix_v=1 << 23, P=100,
+             cache_k=1 << 24, cache_ks=1 << 25, cache_v=1 << 24, cache_vs=1 << 25, Smax=8, t=1 << 12, pages=1 << 13, pages_stride=8, cache_rows=136, stream=None)
+    if align:
+        a[name] += align // 2
+    else:
+        a.update({"P": dict(P=1 << 22), "cache_rows": dict(cache_rows=1 << 24), "B": dict(B=65535, H=68, cache_rows=65535 * 8)}[name])
+    assert lib.smh_shared_prefix_attn_qkv_tiles(*a.values()) < 0
+    assert {"P": b"32-bit", "cache_rows": b"32-bit", "B": b"grid"}.get(name, b"%d-byte aligned" % align) in lib.smh_last_error_string()
+
+
+def _tile_tensors():
+    from spec_mcts_amd import kernels as K
+    half, i8, i32 = torch.float16, torch.int8, torch.int32
+    B, H, Hkv, P, Smax = 5, 4, 2, 9, 8
+    cache = lambda n, dtype: torch.zeros((B, Smax, Hkv, n), dtype=dtype)
+    return dict(p=K.PartialProduct(torch.zeros((2, B, (H + 2 * Hkv) * 128)), 2, B, (H + 2 * Hkv) * 128), H=H, Hkv=Hkv, D=128, cos=torch.zeros((64, 64), dtype=half),
+                sin=torch.zeros((64, 64), dtype=half), pos_dev=torch.zeros(1, dtype=i32), prefix_k=torch.zeros((P, Hkv, 128), dtype=half),
+                prefix_v=torch.zeros((P, Hkv, 128), dtype=half), P=P, cache_k=cache(64, i8), cache_ks=cache(2, half), cache_v=cache(64, i8), cache_vs=cache(2, half),
+                Smax=Smax, t_dev=torch.zeros(1, dtype=i32))
+
+
+@pytest.mark.parametrize("name,change", [(n, f) for n in ("cos", "sin") for f in ("float", "strided", "narrow")] + [("pos_dev", "long"), ("t_dev", "long")]
+                         + [(n, f) for n in ("prefix_k", "prefix_v") for f in ("float", "strided", "short", "narrow")]
+                         + [(n, f) for n in ("cache_k", "cache_v", "cache_ks", "cache_vs") for f in ("float", "strided", "short")] + [(None, None)])
+def test_tile_attention_checks_its_tensors(name, change, monkeypatch):
+    """kernels.shared_prefix_attn_qkv_tiles raises where a tensor is of another type, stride or size than the kernel reads (no GPU needed: the library is
+    stood in for)."""
+    from spec_mcts_amd import _lib, kernels as K
+    calls = []
+    monkeypatch.setattr(_lib, "load", lambda: type("Lib", (), {"smh_shared_prefix_attn_qkv_tiles": lambda self, *a: calls.append(a) or 0})())
+    monkeypatch.setattr(K, "_need_gpu", lambda *a: None)
+    monkeypatch.setattr(K, "_stream", lambda: None)
+    t = _tile_tensors()
+    if name is not None:
+        x = t[name]
+        t[name] = {"float": lambda: x.float(), "long": lambda: x.long(), "strided": lambda: torch.stack((x, x), -1)[..., 0], "short": lambda: x[:-1],
+                   "narrow": lambda: x[..., :-8].contiguous()}[change]()
+        with pytest.raises(AssertionError):
+            K.shared_prefix_attn_qkv_tiles(**t)
+        assert not calls
+    else:
+        assert K.shared_prefix_attn_qkv_tiles(**t).shape == (5, 4, 128) and len(calls) == 1
 
 
 def test_kernels_know_their_memory(tmp_path):
