@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import contextlib
 import gc
+import threading
 from typing import Optional
 
 import torch
@@ -17,19 +18,30 @@ from . import kernels as K
 from .hf_model_q40_kv_shared import Transformer
 
 
+_recordings_lock = threading.Lock()
+_recordings = 0                                # under way, in any thread
+_collects = False                              # the garbage collector was on before the first of them
+
+
 @contextlib.contextmanager
 def recording(graph: "torch.cuda.CUDAGraph"):
     """torch.cuda.graph(graph) with no garbage collection inside: a collection that falls into a recording destroys whatever GPU objects wait for
     one - the graphs of a search that its hook keeps in a cycle - and their destruction synchronises, which a recording stream
-    forbids: the process aborts."""
-    collects = gc.isenabled()
-    gc.disable()
+    forbids: the process aborts.  The collector is the process's: of recordings that overlap, the last to end turns it on again."""
+    global _recordings, _collects
+    with _recordings_lock:
+        if _recordings == 0:
+            _collects = gc.isenabled()
+            gc.disable()
+        _recordings += 1
     try:
         with torch.cuda.graph(graph):
             yield
     finally:
-        if collects:
-            gc.enable()
+        with _recordings_lock:
+            _recordings -= 1
+            if _recordings == 0 and _collects:
+                gc.enable()
 
 
 class GraphDecoder:

@@ -47,3 +47,23 @@ def test_no_collection_falls_into_a_recording(monkeypatch, enabled, fails):
         (gc.enable if was else gc.disable)()
         gc.collect()
     assert len(destroyed) == 50
+
+
+@pytest.mark.parametrize("enabled", [True, False])
+@pytest.mark.parametrize("first_out", [0, 1])
+def test_recordings_of_several_threads_overlap(monkeypatch, enabled, first_out):
+    """Each of two recordings that overlap keeps the collector off until both are over, whichever ends first; then it is as it was."""
+    monkeypatch.setattr(torch.cuda, "graph", lambda graph: contextlib.nullcontext())
+    was = gc.isenabled()
+    try:
+        (gc.enable if enabled else gc.disable)()
+        stacks = [contextlib.ExitStack() for _ in range(2)]
+        for s in stacks:
+            s.enter_context(decode.recording("g"))
+            assert not gc.isenabled()
+        stacks[first_out].close()
+        assert not gc.isenabled()
+        stacks[1 - first_out].close()
+        assert gc.isenabled() == enabled
+    finally:
+        (gc.enable if was else gc.disable)()
