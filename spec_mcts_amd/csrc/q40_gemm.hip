@@ -71,18 +71,12 @@ __device__ __forceinline__ void gemm_wait_vm() { asm volatile("s_waitcnt vmcnt(%
 template <int PER>
 __device__ __forceinline__ void gemm_wait_dma(int stages) {
     switch (stages) {
-        case 11: gemm_wait_vm<11 * PER>(); break;
-        case 10: gemm_wait_vm<10 * PER>(); break;
-        case 9: gemm_wait_vm<9 * PER>(); break;
-        case 8: gemm_wait_vm<8 * PER>(); break;
-        case 7: gemm_wait_vm<7 * PER>(); break;
-        case 6: gemm_wait_vm<6 * PER>(); break;
         case 5: gemm_wait_vm<5 * PER>(); break;
         case 4: gemm_wait_vm<4 * PER>(); break;
         case 3: gemm_wait_vm<3 * PER>(); break;
         case 2: gemm_wait_vm<2 * PER>(); break;
         case 1: gemm_wait_vm<1 * PER>(); break;
-        default: gemm_wait_vm<0>(); break;              // (waits for more than asked)
+        default: gemm_wait_vm<0>(); break;              // (a ring of eight slots asks for five at most; waits for more than asked)
     }
 }
 
@@ -494,31 +488,15 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
         }
     };
     // exact fp16 code * scale, as the four B operands (byte 2bp high / low, byte 2bp+1 high / low)
-    // eight waves: the nibble this wave decodes, as constants of one and-or + one packed fma (code = fp16 bits * mul + off)
+    // eight waves (tiled weights; the checkpoint layout's have the DMA waves and RowWeights): the nibble this wave decodes, as constants of one
+    // and-or + one packed fma (code = fp16 bits * mul + off)
     const uint32_t nib_mask = hh == 0 ? 0x00F000F0u : 0x000F000Fu;
     uint32_t nib_magic = MAGIC_1024;                             // in a register the compiler cannot see through: (bits & mask) | magic is
     asm volatile("" : "+v"(nib_magic));                       // then ONE v_and_or_b32 (no literal operands there), not an AND and an OR
     const h2 nib_mul = hh == 0 ? h2{(half_t)0.0625f, (half_t)0.0625f} : h2{(half_t)1.0f, (half_t)1.0f};
     const h2 nib_off = hh == 0 ? h2{(half_t)-72.0f, (half_t)-72.0f} : h2{(half_t)-1032.0f, (half_t)-1032.0f};
-    // checkpoint layout: codes are two's complement, so the nibble's top bit is flipped in the same three-input operation
-    uint32_t raw_magic = MAGIC_1024 ^ (hh == 0 ? 0x00800080u : 0x00080008u);
-    const uint32_t raw_scale = hh == 0 ? 0x05040100u : 0x07060302u;        // the first or the second 64 columns' scale of two rows
     auto decode = [&](const uint32_t (&wv)[8], const uint32_t (&sv)[8], bool dead, h8 (&b)[NB]) {
         u32x4 v0h, v0l, v1h, v1l;
-        if (!TILED && WAVES == 8) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t pr0 = __builtin_amdgcn_perm(wv[2 * j + 1], wv[2 * j], sel0), pr1 = __builtin_amdgcn_perm(wv[2 * j + 1], wv[2 * j], sel1);
-                uint32_t pair = __builtin_amdgcn_perm(sv[2 * j + 1], sv[2 * j], raw_scale);
-                if (RAGGED) pair = dead ? 0u : pair;           // k >= K: no contribution
-                const h2 sc = as_h2(pair);
-                v0h[j] = as_u32(__builtin_elementwise_fma(as_h2((pr0 & nib_mask) ^ raw_magic), nib_mul, nib_off) * sc);
-                v1h[j] = as_u32(__builtin_elementwise_fma(as_h2((pr1 & nib_mask) ^ raw_magic), nib_mul, nib_off) * sc);
-            }
-            b[0] = __builtin_bit_cast(h8, v0h);
-            b[1] = __builtin_bit_cast(h8, v1h);
-            return;
-        }
         if (TILED && WAVES == 8) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -786,7 +764,7 @@ template <int TILES, bool RAGGED, bool TILED, int WAVES, int SLOTS = GEMM_STAGES
 // (SWIGLU without the DMA waves: at most 128 registers, so that two workgroups of eight waves fit a compute unit)
 __global__ __launch_bounds__(64 * (WAVES + (PRODUCER ? GEMM_DMA_WAVES : 0)), WAVES == 8 ? (SWIGLU && !PRODUCER ? 4 : 1) : 2) void q40_gemm_kernel(MatmulParams p) {
     static_assert(WAVES == 4 || (WAVES == 8 && (TILED ? !RAGGED : PRODUCER)), "eight waves: K a multiple of 32, or the checkpoint layout with the DMA waves");
-    static_assert(SLOTS >= 6 && SLOTS <= 12 && (SLOTS == GEMM_STAGES || PRODUCER) && (!PRODUCER || WAVES == 8), "ring depth");
+    static_assert(SLOTS >= 6 && SLOTS <= 8 && (SLOTS == GEMM_STAGES || PRODUCER) && (!PRODUCER || WAVES == 8), "ring depth");
     args_ahead<sizeof(MatmulParams)>();
     const int steps_total = (p.K + 31) / 32;
     if constexpr (RANGE) {
