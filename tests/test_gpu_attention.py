@@ -241,6 +241,43 @@ def test_attention_fed_by_the_qkv_product_matches_the_three_launch_sequence(B, H
             assert torch.equal(a, b_), "appended cache rows differ"
 
 
+def _tiles_against_launches(qkv, H, Hkv, P, t, Smax, paged, g):
+    """smh_shared_prefix_attn_qkv_tiles and smh_partial_rope_append_kv + smh_shared_prefix_attn / smh_paged_prefix_attn on the same slabs and caches, of
+    which nobody's rows are alike: the same rows appended, outputs within the bound of the tests below.  Returns the call and its output."""
+    from spec_mcts_amd import kernels as K
+    dev, D, B = "cuda:0", 128, qkv.M
+    ang = torch.rand((64, 64), generator=g) * 6.28
+    cos, sin = torch.cos(ang).half().to(dev), torch.sin(ang).half().to(dev)
+    pos_dev = torch.tensor([P + t], dtype=torch.int32, device=dev) % 64
+    t_dev = torch.tensor([t], dtype=torch.int32, device=dev)
+    pk, pv = ((torch.randn((P + 5, Hkv, D), generator=g) * 0.5).half().to(dev) for _ in range(2))
+    ck, cv = (torch.randint(-128, 128, (B, Smax, Hkv, 64), generator=g, dtype=torch.int16).to(torch.int8).to(dev) for _ in range(2))
+    cks, cvs = ((torch.rand((B, Smax, Hkv, 2), generator=g) * 0.1 + 0.01).half().to(dev) for _ in range(2))
+    for past in (pk[P:], pv[P:], cks[:, max(t, 1):], cvs[:, max(t, 1):]):
+        past.fill_(float("nan"))
+    pages = None
+    if paged:                                      # rows of any branch, but for the new one
+        pages = torch.randint(0, B, (B, Smax), generator=g, dtype=torch.int32) * Smax + torch.randint(0, max(t, 1), (B, Smax), generator=g, dtype=torch.int32)
+        pages = pages.to(dev)
+    mine = [c.clone() for c in (ck, cks, cv, cvs)]
+    q, k, v = K.partial_rope_append_kv(qkv, H, Hkv, D, cos, sin, pos_dev, ck, cks, cv, cvs, Smax, t_dev)
+    common = dict(lens=t_dev, lens_stride=0, cur_k=k, cur_v=v)
+    prefix = (pk, pv) if P else (None, None)
+    if paged:
+        del common["lens"]
+        want = K.paged_prefix_attn(q, pages, t_dev, ck.view(-1, Hkv, 64), cv.view(-1, Hkv, 64), cks.view(-1, Hkv, 2), cvs.view(-1, Hkv, 2), False, *prefix, P, **common)
+    else:
+        want = K.shared_prefix_attn(q, *prefix, P, suffix_k=ck, suffix_v=cv, suffix_ks=cks, suffix_vs=cvs, Smax=Smax, n_kv_heads=Hkv, **common)
+    tiles = lambda: K.shared_prefix_attn_qkv_tiles(qkv, H, Hkv, D, cos, sin, pos_dev, *prefix, P, *mine, Smax, t_dev, pages=pages)
+    got = tiles()
+    torch.cuda.synchronize()
+    assert torch.isfinite(got).all()
+    assert torch.allclose(got.float(), want.float(), rtol=2e-3, atol=2e-3), f"{qkv.ksplit} slabs: {float((got.float() - want.float()).abs().max())}"
+    for a, b_ in zip((ck, cks, cv, cvs), mine):
+        assert torch.equal(a.nan_to_num(-1.0), b_.nan_to_num(-1.0)) if a.dtype == torch.float16 else torch.equal(a, b_), "appended cache rows differ"
+    return tiles, got
+
+
 @pytest.mark.parametrize("paged", [False, True])
 @pytest.mark.parametrize("B,H,Hkv,P,t", [(1, 4, 4, 31, 0), (16, 9, 9, 32, 1), (17, 4, 4, 33, 5), (33, 8, 2, 511, 15), (7, 6, 2, 513, 9), (40, 2, 2, 1030, 14), (5, 8, 8, 0, 3),
                                          (100, 3, 3, 100, 8)])
@@ -248,8 +285,8 @@ def test_attention_of_sixteen_queries_a_workgroup_matches_the_three_launch_seque
     """smh_shared_prefix_attn_qkv_tiles against smh_partial_rope_append_kv + smh_shared_prefix_attn / smh_paged_prefix_attn on the same slabs (as many
     as the plans of 256 to 2048 rows come to): the same rows appended; outputs equal up to the order of fp32 sums and to which fp16 a probability of
     the prefix is rounded to (relative to another maximum), 2^-11 of a mean of values below 3: 2e-3 as in the test above.  Prefixes around the
-    32 rows of a wave and the 512 of a workgroup's pass, tiles with one to sixteen queries, grouped heads that straddle a tile.  What lies past
-    the prefix and past a branch's rows is NaN; then one branch's query is, and nobody else's output."""
+    32 rows of a wave and the 512 of a workgroup's pass, tiles with one to eight queries (few heads: the form of eight), grouped heads that straddle a
+    tile.  What lies past the prefix and past a branch's rows is NaN; then one branch's query is, and nobody else's output."""
     from spec_mcts_amd import kernels as K
     dev = "cuda:0"
     D, Smax = 128, 16
@@ -262,40 +299,28 @@ def test_attention_of_sixteen_queries_a_workgroup_matches_the_three_launch_seque
             s = (torch.rand((dim * n // 64,), generator=g) * 0.02 + 0.005).half().to(dev)
             ws.append((w, s, n))
         qkv = K.matmul_q40_partial(x, ws)
-        ang = torch.rand((64, 64), generator=g) * 6.28
-        cos, sin = torch.cos(ang).half().to(dev), torch.sin(ang).half().to(dev)
-        pos_dev = torch.tensor([P + t], dtype=torch.int32, device=dev) % 64
-        t_dev = torch.tensor([t], dtype=torch.int32, device=dev)
-        pk, pv = ((torch.randn((P + 5, Hkv, D), generator=g) * 0.5).half().to(dev) for _ in range(2))
-        ck, cv = (torch.randint(-128, 128, (B, Smax, Hkv, 64), generator=g, dtype=torch.int16).to(torch.int8).to(dev) for _ in range(2))
-        cks, cvs = ((torch.rand((B, Smax, Hkv, 2), generator=g) * 0.1 + 0.01).half().to(dev) for _ in range(2))
-        for past in (pk[P:], pv[P:], cks[:, max(t, 1):], cvs[:, max(t, 1):]):
-            past.fill_(float("nan"))
-        pages = None
-        if paged:                                  # rows of any branch, but for the new one
-            pages = torch.randint(0, B, (B, Smax), generator=g, dtype=torch.int32) * Smax + torch.randint(0, max(t, 1), (B, Smax), generator=g, dtype=torch.int32)
-            pages = pages.to(dev)
-        mine = [c.clone() for c in (ck, cks, cv, cvs)]
-        q, k, v = K.partial_rope_append_kv(qkv, H, Hkv, D, cos, sin, pos_dev, ck, cks, cv, cvs, Smax, t_dev)
-        common = dict(lens=t_dev, lens_stride=0, cur_k=k, cur_v=v)
-        prefix = (pk, pv) if P else (None, None)
-        if paged:
-            del common["lens"]
-            want = K.paged_prefix_attn(q, pages, t_dev, ck.view(-1, Hkv, 64), cv.view(-1, Hkv, 64), cks.view(-1, Hkv, 2), cvs.view(-1, Hkv, 2), False, *prefix, P, **common)
-        else:
-            want = K.shared_prefix_attn(q, *prefix, P, suffix_k=ck, suffix_v=cv, suffix_ks=cks, suffix_vs=cvs, Smax=Smax, n_kv_heads=Hkv, **common)
-        tiles = lambda: K.shared_prefix_attn_qkv_tiles(qkv, H, Hkv, D, cos, sin, pos_dev, *prefix, P, *mine, Smax, t_dev, pages=pages)
-        got = tiles()
-        torch.cuda.synchronize()
-        assert torch.isfinite(got).all()
-        assert torch.allclose(got.float(), want.float(), rtol=2e-3, atol=2e-3), f"dim {dim}: {float((got.float() - want.float()).abs().max())}"
-        for a, b_ in zip((ck, cks, cv, cvs), mine):
-            assert torch.equal(a.nan_to_num(-1.0), b_.nan_to_num(-1.0)) if a.dtype == torch.float16 else torch.equal(a, b_), "appended cache rows differ"
+        tiles, got = _tiles_against_launches(qkv, H, Hkv, P, t, Smax, paged, g)
         qkv.buf.view(qkv.ksplit, B, -1)[0, B // 2, 3] = float("nan")
         got_nan = tiles()
         assert got_nan[B // 2, 0].isnan().all()
         got_nan[B // 2, 0] = got[B // 2, 0]
         assert torch.equal(got_nan, got)
+
+
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("B,H,Hkv,queries,ksplit,P,t", [
+    (100, 32, 32, 16, 2, 100, 65), (100, 32, 32, 16, 5, 512, 40), (65, 32, 32, 16, 1, 96, 127), (65, 32, 32, 16, 3, 222, 16), (33, 64, 8, 16, 6, 130, 33), (33, 64, 8, 16, 2, 600, 17),
+    (40, 64, 8, 16, 12, 129, 31), (73, 29, 29, 16, 7, 97, 64), (65, 32, 32, 16, 16, 1100, 1), (31, 64, 8, 8, 5, 2047, 110), (37, 32, 32, 8, 5, 221, 40), (37, 32, 32, 8, 2, 100, 64),
+    (17, 4, 4, 8, 16, 96, 127), (20, 8, 2, 8, 3, 222, 33), (64, 32, 32, 8, 1, 512, 32), (5, 64, 8, 8, 6, 500, 63)])
+def test_tile_attention_over_long_branches(B, H, Hkv, queries, ksplit, P, t, paged):
+    """Both numbers of queries a workgroup, each of their three kernels by the number of slabs, and branches of more rows than a turn of the walk (16 or 32)
+    and than one request of page ids (32): lengths around both, with and without a table, no two branches' rows alike."""
+    from spec_mcts_amd import kernels as K
+    assert (16 if Hkv * -(-B * (H // Hkv) // 8) > 256 else 8) == queries          # (the rule of the entry point)
+    g = torch.Generator().manual_seed(B + t)
+    n = (H + 2 * Hkv) * 128
+    qkv = K.PartialProduct((torch.randn((ksplit, B, n), generator=g) * 1.5 / ksplit ** 0.5).to("cuda:0"), ksplit, B, n)
+    _tiles_against_launches(qkv, H, Hkv, P, t, 128, paged, g)
 
 
 @pytest.mark.parametrize("B,H,Hkv,P", [(17, 4, 4, 100), (20, 8, 2, 530), (100, 32, 32, 130), (40, 64, 8, 1030)])

@@ -22,7 +22,7 @@ def _build(cfg, seed, std):
     return oargs, sd, model
 
 
-def _steps(cfg, seed, B, P, std, rtol, atol, steps=3):
+def _steps(cfg, seed, B, P, std, rtol, atol, steps=3, forks={}):
     oargs, sd, model = _build(cfg, seed, std)
     oracle = O.OracleTransformer(oargs, sd, dense=True)
     gen = torch.Generator().manual_seed(seed + 100)
@@ -34,6 +34,9 @@ def _steps(cfg, seed, B, P, std, rtol, atol, steps=3):
     # the tolerance: steps after the first read the suffix rows the earlier ones appended.
     sync_prefix(model, oracle)
     for step in range(steps):
+        if step in forks:                              # from here on the branches read an ancestor's rows through the page table
+            model.fork(*forks[step])
+            oracle.fork(*forks[step])
         tok = torch.randint(0, cfg["vocab_size"], (B, 1), generator=gen)
         want = oracle.forward(tok, P + step)
         got = model(tok.cuda(), P + step).cpu()
@@ -55,6 +58,17 @@ MANY_GQA = dict(dim=512, n_layers=2, n_heads=4, n_kv_heads=2, vocab_size=384, mu
 @pytest.mark.parametrize("cfg,seed,B", [(MANY, 70, 17), (MANY, 71, 40), (MANY_GQA, 72, 33), (MANY_GQA, 73, 100)])
 def test_decode_logits_above_16_branches(cfg, seed, B):
     _steps(cfg, seed, B, P=21, std=0.05, rtol=1e-2, atol=1e-2)
+
+
+@pytest.mark.parametrize("forks", [{}, {2: (3, 9, 6), 4: (16, 0, 3)}])
+@pytest.mark.parametrize("cfg,seed,B,P", [(MANY, 74, 17, 97), (MANY, 75, 37, 150), (MANY, 76, 40, 512), (MANY_GQA, 77, 65, 100), (MANY_GQA, 78, 100, 300), ("7b", 79, 70, 96),
+                                          ("7b", 80, 100, 130), ("70b", 81, 40, 100)])
+def test_decode_logits_behind_longer_prompts(cfg, seed, B, P, forks):
+    """From 96 prompt rows on, where such steps take their attention in one launch (eight queries a workgroup; 16 with the heads of the 7B and the 70B
+    architecture): per branch and step against the oracle, branches with rows of their own and branches that share an ancestor's."""
+    cfg = {"7b": LAYER_7B, "70b": ARCH_70B_LAYER}.get(cfg, cfg) if isinstance(cfg, str) else cfg
+    std = 0.05 if cfg["dim"] <= 512 else 0.02
+    _steps(dict(cfg, n_layers=min(cfg["n_layers"], 2), max_batch_size=B, max_prompt_seq_len=P), seed, B, P, std=std, rtol=1e-2, atol=1e-2, steps=6, forks=forks)
 
 
 ARCH_70B_LAYER = dict(dim=8192, n_layers=1, n_heads=64, n_kv_heads=8, vocab_size=512, multiple_of=4096,
