@@ -1490,10 +1490,10 @@ __global__ __launch_bounds__(256, 2) void attn_one_kernel(AttnParams p) {
     }
 }
 
-// ---- a step's attention in one launch, 16 queries of a kv head a workgroup ------------------------------------------
-// Wave w of eight has queries 2 w and 2 w + 1 of the tile, one in either half of its lanes: it adds up their q, k and v from the slabs of
-// wq|wk|wv, rotates, appends k and v, and walks the two branches' own rows.  In between all waves multiply the prefix for all 16 queries, 32 rows
-// at a time (a wave takes every eighth such chunk), with K and V in registers as they come from memory; the waves' partials meet in LDS, so nothing
+// ---- a step's attention in one launch, 16 or 8 queries of a kv head a workgroup -------------------------------------
+// (Of 16; of 8, a wave has one.)  Wave w of eight has queries 2 w and 2 w + 1 of the tile, one in either half of its lanes: it adds up their q, k and v
+// from the slabs of wq|wk|wv, rotates, appends k and v, and walks the two branches' own rows.  In between all waves multiply the prefix for all 16 queries,
+// 32 rows at a time (a wave takes every eighth such chunk), with K and V in registers as they come from memory; the waves' partials meet in LDS, so nothing
 // but the output leaves the workgroup, and it waits for no other.
 //   S^T = K . Q^T: element r of tile i is prefix row 16 i + 4 g + r of query c.  O^T = V^T . P^T in eight products: lane (c, g) holds dims
 //   8 c .. + 7 of the eight rows whose probabilities it has, product e takes dims 8 c + e (a transpose of pairs of halves in registers), and
@@ -1505,7 +1505,8 @@ __global__ __launch_bounds__(256, 2) void attn_one_kernel(AttnParams p) {
 // branches 3.90 -> 3.58 ms, of 37 2.92 -> 2.77).  Which of them a layer takes: attn_way in model_layer.hip.
 // Bound by the vector ALU: ~2000 instructions a wave and 110 a pass of four rows for two queries, at 4.4 cycles, two waves a SIMD; and, before
 // that, by the compute unit's address unit and the latency of HBM (256 KB of K and V a workgroup: 5.5 us alone).
-// (16 waves of one query each spill their registers: 20 us, where eight took 17.)
+// (16 waves of one query each spill their registers: 20 us, where eight took 17.  Eight waves of two queries with a page table keep three in 16 bytes of
+// scratch a lane.)
 constexpr int AT_WAVES = 8, AT_CHUNK = 32;
 constexpr int AT_PITCH = ATT_D + 4;                        // floats of a partial: o[128], maximum, sum
 constexpr int AT_MINE = 16 * AT_PITCH;                     // floats of LDS of a wave: its partials, before that a chunk of K

@@ -38,7 +38,9 @@ static bool direct(int M, int K, int nseg, const int *n) { return smh_q40_matmul
 //    48 / 2047                               -    31.5   32.0    |    16 / 2047                      -    24.4   26.3
 //   100 / 2047                               -    34.7   47.7    |   100 / 2047                      -    48.8   65.6
 //                                                                |  40 heads, 100 / 512 (two rounds) -   39.5   39.0
-// A long prompt wants more workgroups than few tiles are, and ONE's merge grows with the slices.  Behind fewer than 96 prompt rows results stay
+// A long prompt wants more workgroups than few tiles are, and ONE's merge grows with the slices.  Where the table has a faster form than the rule takes,
+// the line is not drawn yet: multi-head attention of 6 to 16 branches (TILES at 16 / 256, LAUNCHES at 10 / 768) and one grouped branch behind a long
+// prompt were measured at these sizes only, and stay with ONE.  Behind fewer than 96 prompt rows results stay
 // where they are: there two evaluations that differ in one rounding drift 3e-2 (40 rows) to 6e-2 (16 rows) apart within eight steps of the 7B
 // architecture, 1.5e-2 behind 96.
 enum AttnWay { ATTN_ONE, ATTN_TILES, ATTN_LAUNCHES };

@@ -1242,6 +1242,8 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + GEMM_DMA_WAVES), 1) void q40_gem
 // 128 us, now 77, 5120 x 13824 at 512 rows 138, now 101.)
 // Against measurement at the 7B, 13B, 34B and 70B shapes, 160 .. 2047 rows: 0.87 to 1.17 times the estimate, 1.3 to 1.4 times it
 // for square weights at 160 rows (15 and 19 us: launches).
+// All of these figures and constants are of the loop with one DMA wave whose products waited for their own reads; with two and the read-ahead launches are
+// faster (7B: w1|w3 at 512 rows 93.9 -> 90.6 us, at 2047 358.6 -> 346.8), and the constants have not been fitted again.
 // (us a step, us more a step at 128 rows, us around the loop, that factor, and what the share of busy compute units adds to the rounds)
 struct RowsCost { float step, per_rows, around, busy, more; };
 constexpr RowsCost ROWS_256 = {0.18f, 0.24f, 4.0f, 1.2f, 0.0f};

@@ -127,7 +127,7 @@ def test_ragged_k_and_small_shapes(M, N, Kd):
                                     (17, 128, 8), (33, 384, 168), (64, 11008, 264), (81, 640, 1048), (100, 4096, 4088), (100, 20224, 520),
                                     (128, 384, 2056), (129, 128, 232), (250, 8192, 88), (300, 24704, 72)])
 def test_checkpoint_layout_by_workgroups(M, N, Kd):
-    """eight waves and the DMA wave (one workgroup a compute unit, range cut among them) or four waves: column units of one block,
+    """eight waves and the DMA waves (one workgroup a compute unit, range cut among them) or four waves: column units of one block,
     few steps, edges of row tiles; fp32 sums of exact products, one rounding to fp16"""
     from spec_mcts_amd import kernels as K
     g = torch.Generator(device="cuda").manual_seed(M + N)

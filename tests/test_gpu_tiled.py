@@ -295,7 +295,7 @@ def test_model_logits_do_not_depend_on_where_rmsnorm_is_made():
 @pytest.mark.parametrize("M", [129, 130, 255, 300])
 @pytest.mark.parametrize("K,n_half", [(256, 384), (4096, 1024), (96, 128), (512, 11008)])
 def test_swiglu_inside_the_gate_up_launch_above_128_rows(M, K, n_half):
-    """even row blocks of five to eight tiles, an odd number of 128-column blocks, with and without the DMA wave"""
+    """even row blocks of five to eight tiles, an odd number of 128-column blocks, with and without the DMA waves"""
     import torch.nn.functional as F
     from spec_mcts_amd import kernels as Kn
     w1, w3 = _weight(K, n_half, 990 + K), _weight(K, n_half, 991 + K)
