@@ -1302,7 +1302,9 @@ __device__ __forceinline__ void attn_prefix_round(const AttnParams &p, int split
 // prefix_wgs: a multiple of 8, so that the others sit on the XCDs that attn_suffix_kernel's would
 template <int PB>
 __global__ __launch_bounds__(256, 4) void attn_parts_kernel(AttnParams p, int prefix_wgs, int rounds) {
-    args_ahead<sizeof(AttnParams)>();
+    // (No args_ahead: a walk's first request needs two of the arguments' six lines, and waiting for all of them costs more than the later trips.  us a call with
+    // the merge behind it, without and with: 64 heads over 8, 13 branches after 108 rows 12.1 and 12.6, 81 after 30 24.8 and 25.8; 32 heads, 40 after
+    // 500 25.8 and 26.8.  The merge has it.)
     int L = blockIdx.x;
     if (L < prefix_wgs) {
         const DivMod head = uniform_divmod(L, p.Hkv), slice = uniform_divmod(head.q, rounds);
