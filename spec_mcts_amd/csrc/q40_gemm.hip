@@ -295,7 +295,7 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
     int sg = 0;
     if (!SWIGLU && p.nseg > 1 && unit >= p.seg[1].unit0) sg = 1;
     if (!SWIGLU && p.nseg > 2 && unit >= p.seg[2].unit0) sg = 2;
-    const MatmulSegment seg = segment_at(p, sg);
+    const MatmulSegment seg = segment_at<true>(p, sg);
     const int pair = SWIGLU ? unit >> 1 : unit - seg.unit0;
     const int col0 = SWIGLU ? unit * 128 : pair * GEMM_COLS;
     const bool two_blocks = SWIGLU || col0 + 128 < seg.N;
@@ -836,7 +836,7 @@ __global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_kg_kern
     int sg = 0;
     if (p.nseg > 1 && unit >= p.seg[1].unit0) sg = 1;
     if (p.nseg > 2 && unit >= p.seg[2].unit0) sg = 2;
-    const MatmulSegment seg = segment_at(p, sg);
+    const MatmulSegment seg = segment_at<true>(p, sg);
     const int pair = unit - seg.unit0;
     const int col0 = pair * GEMM_COLS + 128 * blk;
     if (col0 >= seg.N) return;                                         // a weight with an odd number of 128-column blocks

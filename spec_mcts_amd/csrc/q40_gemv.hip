@@ -265,7 +265,7 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void q40_gemv_kernel(MatmulParams 
     int sg = 0;
     if (p.nseg > 1 && unit >= p.seg[1].unit0) sg = 1;
     if (p.nseg > 2 && unit >= p.seg[2].unit0) sg = 2;
-    const MatmulSegment seg = segment_at(p, sg);
+    const MatmulSegment seg = segment_at<false>(p, sg);
     const int pair = unit - seg.unit0;
 
     const int tid = threadIdx.x;

@@ -6,6 +6,8 @@
 // The slabs hold fp32 at every batch size.
 #pragma once
 
+#include <type_traits>
+
 #include "smh_common.hpp"
 
 #define SMH_MAX_KSPLIT 16
@@ -78,11 +80,17 @@ struct MatmulParams {
     float norm_eps;
 };
 
-// p.seg[sg] without a load that waits for sg
+// p.seg[sg] without a load that waits for sg.  GLOBAL: the kernel stores through c (held_global); one that does not schedules its first loads better
+// without (GEMV, 16 rows and fewer: 1 % of a call).
+template <bool GLOBAL>
 __device__ __forceinline__ MatmulSegment segment_at(const MatmulParams &p, int sg) {
     MatmulSegment r = p.seg[0];
+    auto hold = [](auto v) {
+        if constexpr (GLOBAL && std::is_pointer<decltype(v)>::value) return held_global(v);
+        else return held(v);
+    };
     auto pick = [&](auto member) {
-        const auto a = held(p.seg[0].*member), b = held(p.seg[1].*member), c = held(p.seg[2].*member);
+        const auto a = hold(p.seg[0].*member), b = hold(p.seg[1].*member), c = hold(p.seg[2].*member);
         r.*member = sg == 0 ? a : sg == 1 ? b : c;
     };
     pick(&MatmulSegment::w);

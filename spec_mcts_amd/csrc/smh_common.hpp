@@ -61,7 +61,7 @@ __device__ __forceinline__ T held(T v) {
 // ... a pointer to global memory, and known as one: stores through any other are flat ones, which every wait for LDS waits for, too (direct outputs of
 // 300 x 26880 x 9704, checkpoint layout: 276.6 us with flat stores, 272.7 with these)
 template <class T>
-__device__ __forceinline__ T *held(T *v) {
+__device__ __forceinline__ T *held_global(T *v) {
     auto at = (__attribute__((address_space(1))) T *)v;
     asm("" : "+s"(at));
     return (T *)at;
