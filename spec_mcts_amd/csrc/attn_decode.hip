@@ -1532,14 +1532,8 @@ __device__ __forceinline__ h4 rope_lanes(h4 x, h4 cs, h4 sn, bool lower) {
     const h4 a = x * cs, b = (lower ? -other : other) * sn;
     return a + b;
 }
-// kv_store_row2 in that layout; `store`: the half's row is one to be written.  Both quotients are those of its divisions: a reciprocal and one
-// correction by the remainder miss the correctly rounded quotient only where the exact one lies within 2^-46 of the middle between two
-// floats, and with 11 bits in numerator and denominator it is either that middle's neighbour by 2^-36 or a float itself.  Scales that are zero,
-// subnormal or not finite are left to the divisions.
-__device__ __forceinline__ float corrected_quotient(float a, float b, float rcp) {
-    const float q = a * rcp;
-    return __builtin_fmaf(__builtin_fmaf(-q, b, a), rcp, q);
-}
+// kv_store_row2 in that layout; `store`: the half's row is one to be written.  Both quotients are those of its divisions (corrected_quotient).  Scales
+// that are zero, subnormal or not finite are left to the divisions.
 __device__ __forceinline__ void kv_store_lanes(h4 x, uint8_t *row, half_t *scales, int hl, bool store) {
     const u32x2 bits = __builtin_bit_cast(u32x2, x) & 0x7fff7fffu;
     uint32_t big = max(max(bits[0] & 0xffffu, bits[0] >> 16), max(bits[1] & 0xffffu, bits[1] >> 16));

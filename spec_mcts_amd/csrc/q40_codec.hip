@@ -9,6 +9,8 @@
 
 namespace smh {
 
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+
 // out[row*128 + j]      = code(high nibble of byte j) * s[2*row]
 // out[row*128 + 64 + j] = code(low  nibble of byte j) * s[2*row+1]      (one fp16 multiply each)
 __global__ __launch_bounds__(256) void q40_dequant_kernel(const u32x4 *__restrict__ w,
@@ -104,16 +106,6 @@ __device__ __forceinline__ void q40_codes8(const T (&x)[8], float scale, int (&c
     }
 }
 
-// codes of an even group (high nibbles) and of the odd group behind it (low nibbles) -> 4 bytes
-__device__ __forceinline__ uint32_t pack_codes4(int h0, int h1, int h2_, int h3, int l0, int l1, int l2, int l3) {
-    auto byte = [](int hi, int lo) { return ((uint32_t)hi << 4 & ~15u) | ((uint32_t)lo & 15u); };     // (bits above the byte: dropped below)
-    const uint32_t b01 = __builtin_amdgcn_perm(byte(h1, l1), byte(h0, l0), 0x0c0c0400u);
-    const uint32_t b23 = __builtin_amdgcn_perm(byte(h3, l3), byte(h2_, l2), 0x0c0c0400u);
-    return b01 | (b23 << 16);
-}
-__device__ __forceinline__ u32x2 pack_codes8(const int (&hi)[8], const int (&lo)[8]) {
-    return u32x2{pack_codes4(hi[0], hi[1], hi[2], hi[3], lo[0], lo[1], lo[2], lo[3]), pack_codes4(hi[4], hi[5], hi[6], hi[7], lo[4], lo[5], lo[6], lo[7])};
-}
 // eight codes -> value j in bits 4j .. 4j+3
 __device__ __forceinline__ uint32_t nibbles8(const int (&c)[8]) {
     uint32_t v = 0;
@@ -221,37 +213,107 @@ __global__ __launch_bounds__(256) void q40_quantize_f32_kernel(const f4 *__restr
     }
 }
 
+// a / 7, correctly rounded, of a magnitude: the quotient by the reciprocal corrected by its remainder.  (Infinities and NaN, and what is so
+// large that the remainder might overflow, are left to the division.)
+__device__ __forceinline__ float seventh(float a) {
+    constexpr float r = 1.0f / 7.0f;
+    float q = a * r;
+    q = __builtin_fmaf(__builtin_fmaf(-q, 7.0f, a), r, q);
+    if (!(a < 3e38f)) q = a / 7.0f;
+    return q;
+}
+// The codes of eight values in the low halves of eight bytes (the high halves hold anything).
+// Values of at most 11 significant bits (fp16, bfloat16): the quotient is corrected by its remainder, which gives the division's (corrected_quotient).
+// With a doubt about the values next to a tie, as below, most waves divided: a bfloat16 weight has one value in 440 exactly on a tie.
+__device__ __forceinline__ u32x2 q40_bytes8(const half_t (&x)[8], float scale) {
+    u16x2 code[4];
+    if (q40_scale_is_plain(scale)) {
+        const float inv = __builtin_amdgcn_rcpf(scale);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {                        // rounded to fp16, then added to 1536, whose neighbours are one apart
+            const f2 q = {corrected_quotient((float)x[2 * i], scale, inv), corrected_quotient((float)x[2 * i + 1], scale, inv)};
+            code[i] = __builtin_bit_cast(u16x2, __builtin_convertvector(q, h2) + h2{(half_t)1536.0f, (half_t)1536.0f});
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) code[i >> 1][i & 1] = (uint16_t)q40_code(x[i], scale);
+    }
+    auto four = [&](int i) { return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, code[i + 1]), __builtin_bit_cast(uint32_t, code[i]), 0x06040200u); };
+    return u32x2{four(0), four(2)};
+}
+// (A NaN's low bits are zeros, and so is its code.)
+__device__ __forceinline__ u32x2 q40_bytes8_bf16(const float (&x)[8], float scale) {
+    uint32_t t[8];
+    if (q40_scale_is_plain(scale)) {
+        const float inv = __builtin_amdgcn_rcpf(scale);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) t[i] = __builtin_bit_cast(uint32_t, corrected_quotient(x[i], scale, inv) + 12582912.0f);      // 1.5 x 2^23
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) t[i] = (uint32_t)q40_code_wide(x[i], scale);
+    }
+    auto four = [&](int i) { return __builtin_amdgcn_perm(t[i + 1], t[i], 0x0c0c0400u) | __builtin_amdgcn_perm(t[i + 3], t[i + 2], 0x04000c0cu); };
+    return u32x2{four(0), four(4)};
+}
+// fp32 values: x / scale + 192.5 has 16 bits below the point, so that bits 16 .. 19 are the quotient rounded.  The sum is within 2^-16 of
+// the exact one, and a code is in doubt, and divided for, where the bits below the point say that a whole number is at most as far away: it or its
+// neighbours (one value in 20000; a NaN has zeros there or is found as one).  Whether any is: the least of eight distances, two to a register.
+__device__ __forceinline__ u32x2 q40_bytes8_f32(const float (&x)[8], float scale) {
+    uint32_t t[8];
+    bool all = !q40_scale_is_plain(scale);
+    const float inv = __builtin_amdgcn_rcpf(scale);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) t[i] = __builtin_bit_cast(uint32_t, __builtin_fmaf(x[i], inv, 192.5f));
+    auto near = [&](int i) { return __builtin_bit_cast(u16x2, pack_lo16(t[i], t[i + 1])) + u16x2{1, 1}; };
+    const u16x2 least = __builtin_elementwise_min(__builtin_elementwise_min(near(0), near(2)), __builtin_elementwise_min(near(4), near(6)));
+    // (finite values do not add up to a NaN)
+    const float sum = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+    if (all || min(least.x, least.y) < 3 || sum != sum) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (all || ((t[i] + 1) & 0xFFFFu) < 3 || x[i] != x[i]) t[i] = (uint32_t)q40_code_wide(x[i], scale) << 16;
+    }
+    auto four = [&](int i) { return __builtin_amdgcn_perm(t[i + 1], t[i], 0x0c0c0602u) | __builtin_amdgcn_perm(t[i + 3], t[i + 2], 0x06020c0cu); };
+    return u32x2{four(0), four(4)};
+}
+
 // ---- a checkpoint's linear weight [N, K] -> Q4_0 of its transpose, in one pass ------------------------------------------------
-// A workgroup takes 128 outputs n x 64 inputs k.  The tile is read along k (whole cache lines, 16 bytes a lane), turned in LDS
+// A workgroup takes 128 outputs n x 128 bytes of inputs k.  The tile is read along k (whole cache lines, 16 bytes a lane), turned in LDS
 // and quantised along n: eight lanes share input column k (two columns at a time for 16-bit types), lane o holding outputs
 // 8 o .. 8 o + 7 of either group of 64, so a lane's codes are 8 consecutive bytes of packed row (k, n / 128).
 // Neighbouring blocks of 128 outputs (halves of one 128-byte line of codes, parts of one line of scales) go to one XCD, one
-// after the other, so that its L2 joins them.  Bound by HBM (2 or 4 bytes read, 17/32 written per value) and the vector ALU.
-// Measured at 11008 x 4096: bfloat16 31 us (3.7 TB/s), fp16 38, fp32 52; rows of odd length the same.  A transposed copy, a
-// widened copy (bfloat16) and the flat quantiser in its place: 372 us for bfloat16.
+// after the other, so that its L2 joins them; `together` of them at a k (smh_q40_quantize_t).
+// Bound by HBM (2 or 4 bytes read, 17/32 written per value); loads alone take 18 us at 11008 x 4096 bfloat16, and the vector ALU, with no steady state
+// to hide it in (few tiles a compute unit), most of the rest.  In turn, us, with a division in every wave that has a value next to a tie, fp32 tiles of 256
+// bytes and all blocks of outputs at a k, and now: bfloat16 11008 x 4096 28.5 and 27.5 (4.2 TB/s), 8192 x 1024 7.9 and 6.8, 28672 x 8192 136 and 132 (4.5
+// TB/s); fp16 4096 x 4096 16.4 and 12.2, 19968 x 2111 40.1 and 29.7; fp32 8192 x 8192 91.4 and 65.1 (4.7 TB/s), 3072 x 3001 13.7 and 11.7.  (Tiles of 256
+// bytes: level.  Workgroups that stay and load the next tile under this one: 31 to 44 us at 11008 x 4096, where others wait they wait, too.)
 //   SRC 0: fp16, 1: bfloat16, 2: fp32.  P: dwords of an LDS row, odd so that the eight rows a wave reads at a time are 8 P = 8
 // (mod 64) banks apart.
+constexpr int QT_ROW = 128, QT_THREADS = 2 * QT_ROW;        // bytes of a tile's row; eight lanes to a dword of it
 template <int SRC>
-__global__ __launch_bounds__(256) void q40_quantize_t_kernel(const uint8_t *__restrict__ in, int N, int K, uint8_t *__restrict__ w,
-                                                             half_t *__restrict__ s, int k_tiles) {
+__global__ __launch_bounds__(QT_THREADS) void q40_quantize_t_kernel(const uint8_t *__restrict__ in, int N, int K, uint8_t *__restrict__ w,
+                                                                    half_t *__restrict__ s, int k_tiles, int together) {
     constexpr int ES = SRC == 2 ? 4 : 2;                     // bytes of a source value
-    constexpr int P = SRC == 2 ? 65 : 33;
+    constexpr int P = QT_ROW / 4 + 1;
     __shared__ uint32_t tile[128 * P];
     const int tid = threadIdx.x;
     const int n_blocks = N / 128;
     const int total = n_blocks * k_tiles, per = (total + 7) / 8;       // (of a grid: below 2^31 - 8)
+    constexpr int VEC = 16 / ES;                             // values of a load
+    constexpr int LPR = QT_ROW / 16;                         // lanes a row
+    constexpr int LOADS = 128 / (QT_THREADS / LPR);
     const int id = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
     if ((int)(blockIdx.x >> 3) >= per || id >= total) return;
-    const DivMod at = uniform_divmod(id, n_blocks);
-    const int nb = at.r, k0 = at.q * 64;
+    const DivMod of = uniform_divmod(id, together * k_tiles);
+    const int nb0 = of.q * together;
+    const DivMod at = uniform_divmod(of.r, min(together, n_blocks - nb0));
+    const int nb = nb0 + at.r, k0 = at.q * (QT_ROW / ES);
     {
-        constexpr int VEC = 16 / ES;                         // values of a load
-        constexpr int LPR = 64 / VEC;                        // lanes a row
-        const int c = tid % LPR, r0 = tid / LPR;
-        const int k = k0 + c * VEC;
+        const int c = tid % LPR, r0 = tid / LPR, k = k0 + c * VEC;
 #pragma unroll
-        for (int i = 0; i < 128 / (256 / LPR); ++i) {
-            const int r = r0 + i * (256 / LPR);
+        for (int i = 0; i < LOADS; ++i) {
+            const int r = r0 + i * (QT_THREADS / LPR);
             const uint8_t *src = in + ((long)(nb * 128 + r) * K + k) * ES;
             uint32_t v[4] = {0, 0, 0, 0};
             if (k + VEC <= K) {
@@ -271,9 +333,8 @@ __global__ __launch_bounds__(256) void q40_quantize_t_kernel(const uint8_t *__re
     __syncthreads();
     constexpr int KL = SRC == 2 ? 1 : 2;                     // input columns per LDS dword
     const int o = tid & 7;
-#pragma unroll
-    for (int rep = 0; rep < 2 / KL; ++rep) {
-        const int kc = (tid >> 3) + 32 * rep;                // dword column
+    {
+        const int kc = tid >> 3;                             // dword column
         uint32_t d[2][8];
 #pragma unroll
         for (int g = 0; g < 2; ++g)
@@ -282,37 +343,40 @@ __global__ __launch_bounds__(256) void q40_quantize_t_kernel(const uint8_t *__re
 #pragma unroll
         for (int h = 0; h < KL; ++h) {
             const int k = k0 + KL * kc + h;
-            int code[2][8];
+            u32x2 nib[2];                                    // codes in the low halves of the bytes, either group's
             half_t sc[2];
 #pragma unroll
             for (int g = 0; g < 2; ++g) {
-                std::conditional_t<SRC == 0, half_t, float> x[8];
-                float amax = 0.f;
                 if constexpr (SRC == 0) {
-                    uint32_t abits = 0;                      // |x| as a bit pattern: integer order is magnitude order
+                    uint32_t bits[8], abits = 0;             // |x| as a bit pattern: integer order is magnitude order
 #pragma unroll
                     for (int i = 0; i < 8; ++i) {
-                        const uint32_t b = h == 0 ? d[g][i] & 0xFFFFu : d[g][i] >> 16;
-                        abits = max(abits, b & 0x7FFFu);
-                        x[i] = __builtin_bit_cast(half_t, (uint16_t)b);
+                        bits[i] = h == 0 ? d[g][i] & 0xFFFFu : d[g][i] >> 16;
+                        abits = max(abits, bits[i] & 0x7FFFu);
                     }
-                    amax = (float)__builtin_bit_cast(half_t, (uint16_t)max8(abits));
+                    sc[g] = (half_t)seventh((float)__builtin_bit_cast(half_t, (uint16_t)max8(abits)));
+                    half_t x[8];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) x[i] = __builtin_bit_cast(half_t, (uint16_t)bits[i]);
+                    nib[g] = q40_bytes8(x, (float)sc[g]);
                 } else {
+                    float x[8], amax = 0.f;
 #pragma unroll
                     for (int i = 0; i < 8; ++i) {
                         if constexpr (SRC == 1) x[i] = __builtin_bit_cast(float, h == 0 ? d[g][i] << 16 : d[g][i] & 0xFFFF0000u);
                         else x[i] = __builtin_bit_cast(float, d[g][i]);
                         amax = fmaxf(amax, fabsf(x[i]));
                     }
-                    amax = max8(amax);
+                    float q7 = seventh(max8(amax));
+                    if constexpr (SRC == 1) q7 = round_to_bf16(q7);
+                    sc[g] = (half_t)q7;
+                    if constexpr (SRC == 1) nib[g] = q40_bytes8_bf16(x, (float)sc[g]);
+                    else nib[g] = q40_bytes8_f32(x, (float)sc[g]);
                 }
-                float q7 = amax / 7.0f;
-                if constexpr (SRC == 1) q7 = round_to_bf16(q7);
-                sc[g] = (half_t)q7;
-                q40_codes8(x, (float)sc[g], code[g]);
             }
             if (k >= K) continue;
-            *reinterpret_cast<u32x2 *>(w + ((long)k * n_blocks + nb) * 64 + 8 * o) = pack_codes8(code[0], code[1]);
+            const u32x2 both = (nib[0] << 4 & 0xF0F0F0F0u) | (nib[1] & 0x0F0F0F0Fu);
+            *reinterpret_cast<u32x2 *>(w + ((long)k * n_blocks + nb) * 64 + 8 * o) = both;
             if (o == 0) *reinterpret_cast<h2 *>(s + ((long)k * n_blocks + nb) * 2) = h2{sc[0], sc[1]};
         }
     }
@@ -503,10 +567,15 @@ extern "C" int smh_q40_quantize_t(const void *in, int src_type, int N, int K, vo
     SMH_REQUIRE(N > 0 && N % 128 == 0 && K > 0, "smh_q40_quantize_t: N=%d (a positive multiple of 128) K=%d", N, K);
     SMH_REQUIRE(in && w && s && ((uintptr_t)in & (src_type == 2 ? 3 : 1)) == 0 && ((uintptr_t)w & 7) == 0 && ((uintptr_t)s & 3) == 0,
                 "smh_q40_quantize_t: null or misaligned pointer");
-    const int k_tiles = (K + 63) / 64;
+    const int tile_k = QT_ROW / (src_type == 2 ? 4 : 2), k_tiles = (K + tile_k - 1) / tile_k;
     const long blocks = ((long)(N / 128) * k_tiles + 7) / 8 * 8;
     SMH_REQUIRE(blocks < (1L << 31), "smh_q40_quantize_t: N=%d K=%d is too large for one launch", N, K);
+    // Two blocks of outputs share a line of codes.  Where an XCD walks all blocks of outputs at one k, and there are more than run at a time, all it reads
+    // at a time lies at one offset of many rows, in few memory channels: from 64 on it takes two blocks along k instead.  us, all blocks and two: 11008 x
+    // 4096 bfloat16 30.9 and 28.8, 28672 x 8192 136 and 127, 8192 x 8192 fp32 99 and 64, fp16 43.4 and 44.0; below, 4096 x 4096 bfloat16 12.7 and 13.5,
+    // 4096 x 8192 fp16 23.3 and 25.6.
+    const int together = N / 128 >= 64 ? 2 : N / 128;
     const auto kern = src_type == 0 ? q40_quantize_t_kernel<0> : src_type == 1 ? q40_quantize_t_kernel<1> : q40_quantize_t_kernel<2>;
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, (const uint8_t *)in, N, K, (uint8_t *)w, (half_t *)s, k_tiles);
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(QT_THREADS), 0, (hipStream_t)stream, (const uint8_t *)in, N, K, (uint8_t *)w, (half_t *)s, k_tiles, together);
     return launch_status();
 }

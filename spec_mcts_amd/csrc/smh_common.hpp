@@ -162,6 +162,13 @@ __device__ __forceinline__ float rms_factor(float total, int n, float eps) {
     return 1.0f / sqrtf(shifted);
 }
 
+// a / b from b's reciprocal: it and one correction by the remainder miss the correctly rounded quotient only where the exact one lies within 2^-46
+// of the middle between two floats, and with 11 bits in numerator and denominator it is either that middle's neighbour by 2^-36 or a float itself.
+__device__ __forceinline__ float corrected_quotient(float a, float b, float rcp) {
+    const float q = a * rcp;
+    return __builtin_fmaf(__builtin_fmaf(-q, b, a), rcp, q);
+}
+
 // ---- cross-workgroup hand-off inside one launch ------------------------------------------------------
 // Data written by one workgroup and read by another (possibly on a different XCD, i.e. behind a different
 // L2) travels as device-scope relaxed atomics: such stores write through to the point of coherence and

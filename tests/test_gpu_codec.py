@@ -105,6 +105,26 @@ def test_quantize_of_the_transpose_matches_the_oracle(dtype, N, Kd):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,Kd", [(128, 31), (384, 33), (8192, 65), (8320, 70)])
+def test_quantize_of_the_transpose_next_to_ties(dtype, N, Kd):
+    """quotients on and next to points where a code changes, under scales from 2^-14 (the smallest that is multiplied by, not divided) to 2^7, in blocks
+    of outputs taken all or two at a time (65: the last one alone): the oracle's bytes"""
+    from spec_mcts_amd import kernels as K
+    g = torch.Generator().manual_seed(N + Kd)
+    half_steps = torch.randint(-14, 15, (N, Kd), generator=g).float() / 2
+    half_steps[::64] = 7.0
+    step = 2.0 ** torch.randint(-14, 8, (1, Kd), generator=g).float()
+    ulp = {torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7, torch.float32: 2.0 ** -23}[dtype]
+    near = 1 + torch.randint(-4, 5, (N, Kd), generator=g).float() * ulp
+    for v in (half_steps * step, half_steps * step * near, half_steps * step * 1.3717 * near):
+        v = v.to(dtype)
+        w_want, s_want = O.quantize_q40(v.t().contiguous(), 64)
+        w_got, s_got = K.quantize_q40_t(v.cuda())
+        assert np.array_equal(_bits(s_got).reshape(-1), _bits(s_want).reshape(-1))
+        assert torch.equal(w_got.cpu(), w_want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 def test_quantize_nan_values(dtype):
     """A NaN has code 0, whatever its payload.  In a group of fp32 or bfloat16 values it does not count towards the scale (the bytes are
     those of the group with a zero in its place); a group of fp16 values with a NaN has a NaN scale and codes 0."""
