@@ -578,10 +578,16 @@ static int matmul_fp16(const void *a, int M, int K, long lda, const void *b_w, c
         SMH_REQUIRE(!gemm || ldc % 8 == 0, "%s: ldc=%ld must be a multiple of 8 for M > 16", who, ldc);
         return gemm ? gemm_launch(p, (hipStream_t)stream) : gemv_launch(p, (hipStream_t)stream);
     }
-    size_t need = (size_t)p.ksplit * M * N * sizeof(float);
+    size_t need = (size_t)p.ksplit * M * N * sizeof(float);          // (what smh_q40_matmul_plan says; fewer slabs where q40_gemm_kg_kernel runs)
     SMH_REQUIRE(workspace && workspace_bytes >= need, "%s: workspace %zu < %zu bytes", who, workspace_bytes, need);
     p.partial = (float *)workspace;
     p.direct = 0;
+    MatmulParams b;
+    if (gemm && gemm_blocks_fit(p, b)) {
+        p = b;
+        p.direct = p.ksplit == 1 && ldc % 4 == 0 ? 1 : 0;
+        if (p.direct) return gemm_launch(p, (hipStream_t)stream);
+    }
     st = gemm ? gemm_launch(p, (hipStream_t)stream) : gemv_launch(p, (hipStream_t)stream);
     if (st) return st;
     SMH_REQUIRE(ldc % 4 == 0, "%s: ldc=%ld must be a multiple of 4", who, ldc);

@@ -149,11 +149,13 @@ struct TiledWeights {
 };
 // Checkpoint layout: row 8 g + r of a stage (GS_WBLOCK) and its scales (of the block's first, second 64 columns in a dword).
 // RAGGED: stage `last` is the end of K, where `dead` says that this lane's rows lie past it (their scales become zero).
+// BLOCK (q40_gemm_kg_kernel): rows of 64 bytes in the order (r, g), so that the four rows of a read lie in different banks; scales row by row.
 // (With reads that were waited for where they were issued, in us, before and now: 42 / 75 / 100 rows x 26880 x 9704 61.2 / 81.8 / 76.8 and 52.0 / 63.7 / 75.9,
 // 75 x 4096 x 11008 21.5 and 19.9, 100 x 11008 x 4096 23.9 and 23.2, 300 x 11008 x 4096 59 and 46.)
-template <bool RAGGED>
+template <bool RAGGED, bool BLOCK = false>
 struct RowWeights {
-    static constexpr int READS = 8;            // (pairs of dwords)
+    static constexpr int READS = BLOCK ? 6 : 8;            // (pairs of dwords; a block's scales: four dwords)
+    static constexpr int PITCH = BLOCK ? 256 : 128;
     NibbleConsts nib;
     int w_off, s_off;
     uint32_t sel, half;                        // picks the first byte of two rows; the scales of the nibble
@@ -166,9 +168,15 @@ struct RowWeights {
         Regs x;
         x.keep = RAGGED && stage == last && dead ? 0u : ~0u;
 #pragma unroll
-        for (int r = 0; r < 8; ++r) x.w[r] = *reinterpret_cast<const uint32_t *>(st + w_off + r * 128);
+        for (int r = 0; r < 8; ++r) x.w[r] = *reinterpret_cast<const uint32_t *>(st + w_off + r * PITCH);
+        if constexpr (BLOCK) {
+            const u32x4 lo = *reinterpret_cast<const u32x4 *>(st + s_off), hi = *reinterpret_cast<const u32x4 *>(st + s_off + 16);
 #pragma unroll
-        for (int r = 0; r < 8; ++r) x.s[r] = *reinterpret_cast<const uint32_t *>(st + s_off + r * 8);
+            for (int r = 0; r < 4; ++r) { x.s[r] = lo[r]; x.s[4 + r] = hi[r]; }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 8; ++r) x.s[r] = *reinterpret_cast<const uint32_t *>(st + s_off + r * 8);
+        }
         return x;
     }
     __device__ __forceinline__ uint32_t decode(const Regs &x, int j, int o) const {
@@ -796,7 +804,7 @@ __global__ __launch_bounds__(64 * (WAVES + (PRODUCER ? GEMM_DMA_WAVES : 0)), WAV
     }
 }
 
-// ---- two K-groups in one workgroup (tiled weights, K a multiple of 64, one workgroup per compute unit) ----------------
+// ---- two K-groups in one workgroup (tiled weights with K a multiple of 64, or the checkpoint layout; one workgroup per compute unit) ----------------
 // A workgroup owns ONE 128-column block (pieces 2 blk, 2 blk + 1 of the unit's tiles), a block of rows and a K-slice, and
 // its eight multiplying waves form two groups: group kk takes the steps 2 i + kk of the slice.  Wave (kk, hh, bp)
 // multiplies the columns of nibble hh of piece 2 blk + bp of its group's steps with all row tiles of A - the same two B
@@ -805,6 +813,8 @@ __global__ __launch_bounds__(64 * (WAVES + (PRODUCER ? GEMM_DMA_WAVES : 0)), WAV
 // + group 1, a fixed order), and all eight waves write the slab.  Against q40_gemm_kernel's 256-column units this
 // fills the GPU with half as many K-slices, i.e. half the slab bytes written here and read back by the consumer; the
 // price is that a row of A is staged for 128 columns instead of 256.
+// Checkpoint layout (gemm_blocks_fit): a step is 32 rows of 64 bytes, fetched in the order that RowWeights reads; K may end anywhere in the last stage
+// (RAGGED), and a workgroup that has all of K stores the fp16 product itself.
 constexpr int KG_W = 4096;                     // [group kk][piece bp] x 1024
 constexpr int KG_S = 512;                      // [group kk] x 256 (the whole scale block of the step)
 template <int TILES> struct KgShape {
@@ -818,7 +828,7 @@ template <int TILES> struct KgShape {
     static_assert(PER * (SLOTS - 5) <= 63 && LDS <= 160 * 1024, "ring");
 };
 
-template <int TILES>
+template <int TILES, bool TILED, bool RAGGED>
 __global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_kg_kernel(MatmulParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     typedef KgShape<TILES> S;
@@ -827,10 +837,12 @@ __global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_kg_kern
     const int wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);       // 0..7 multiply, the others issue the DMA
     const int lane = tid & 63, c = lane & 15, g = lane >> 4;
     args_ahead<sizeof(MatmulParams)>();
-    // blockIdx -> (128-column block, row block, K-slice); blocks of one unit are neighbours (same XCD every 8)
+    // blockIdx -> (128-column block, row block, K-slice).  Tiled weights: blocks of one unit are neighbours (same XCD every 8).  Checkpoint layout: the
+    // blocks of a unit are the halves of its 128-byte lines and go to one XCD, one after the other, in step.
     const int hb = blockIdx.x;
-    const int slot_u = hb >> 1, blk = hb & 1;
-    const int unit = (slot_u & 7) * (p.units_pad >> 3) + (slot_u >> 3);
+    const int slot_u = hb >> 1, raw_b = (hb & 7) * (p.units_pad >> 2) + (hb >> 3);
+    const int blk = TILED ? hb & 1 : raw_b & 1;
+    const int unit = TILED ? (slot_u & 7) * (p.units_pad >> 3) + (slot_u >> 3) : raw_b >> 1;
     if (unit >= p.units) return;
     const int mb = blockIdx.y, slice = blockIdx.z;
     int sg = 0;
@@ -841,12 +853,16 @@ __global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_kg_kern
     const int col0 = pair * GEMM_COLS + 128 * blk;
     if (col0 >= seg.N) return;                                         // a weight with an odd number of 128-column blocks
     const int m0 = mb * p.block_rows;
-    const int steps_total = p.K / 32;
+    const int steps_total = RAGGED ? (p.K + 31) / 32 : p.K / 32;
     const int step0 = slice * p.steps_per_slice, step1 = min(step0 + p.steps_per_slice, steps_total);
-    const int n_st = max(step1 - step0, 0) / 2;                        // stages (two steps each; slices are even)
-    const uint8_t *w_base = seg.w + (long)pair * tiled_steps(p.K) * TILE_BYTES + (long)step0 * TILE_BYTES;
+    // stages (two steps each; slices are even).  RAGGED: the last one of the slice that ends K may have a step that lies past it
+    const int n_st = (max(step1 - step0, 0) + (RAGGED ? 1 : 0)) / 2;
+    const bool ends = RAGGED && step1 == steps_total;
+    const long w_row = seg.N / 2, s_row = seg.N / 32;                  // checkpoint layout: bytes per k of the nibbles, of the scales
+    const uint8_t *w_base = TILED ? seg.w + (long)pair * tiled_steps(p.K) * TILE_BYTES + (long)step0 * TILE_BYTES : seg.w + (long)step0 * 32 * w_row + (long)pair * 128 + 64 * blk;
+    const uint8_t *s_base = reinterpret_cast<const uint8_t *>(seg.s) + (long)step0 * 32 * s_row + (long)pair * 8 + 4 * blk;
     const uint8_t *a_base = reinterpret_cast<const uint8_t *>(p.a) + (long)step0 * 64;
-    const int rot = n_st > 0 ? uniform_divmod(hb * 5, n_st).r : 0;             // workgroups of a K-slice start at different stages
+    const int rot = n_st > 0 ? uniform_divmod((TILED ? hb : unit) * 5, n_st).r : 0;      // workgroups of a K-slice start at different stages
 
     if (wave8 >= 8) {
         // ---- the DMA waves: a K-group's steps each ----
@@ -858,18 +874,37 @@ __global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_kg_kern
             a_voff[t] = (uint32_t)((long)min(m0 + 16 * t + (lane >> 2), p.M - 1) * p.lda * 2 + 16 * a_chunk);
         int fetch = rot;
         const int kk = wave8 - 8;
+        // checkpoint layout: lane l of instruction q moves 16 bytes of row 8 ((l / 4) % 4) + 4 q + l / 16 of a step (RowWeights), and row l % 32's scales (64 rows'
+        // in one of the two waves: 1 % slower).  `left` rows of the last stage's step lie before the end of K (none, if it is all past it): what is read in the
+        // place of others repeats valid ones.
+        const int left = RAGGED && ends ? p.K - 32 * (step0 + 2 * (n_st - 1) + kk) : 32;
+        const int raw_r = 8 * ((lane >> 2) & 3) + (lane >> 4), raw_c = 16 * (lane & 3);
+        const uint32_t raw_w[2] = {(uint32_t)(raw_r * w_row + raw_c), (uint32_t)((raw_r + 4) * w_row + raw_c)}, raw_s = (uint32_t)((lane & 31) * s_row);
+        auto back = [&](int r) { return r - min(r, left - 1); };           // rows to go back
+        const uint32_t back_w[2] = {(uint32_t)(back(raw_r) * w_row), (uint32_t)(back(raw_r + 4) * w_row)}, back_s = (uint32_t)(back(lane & 31) * s_row);
+        const uint32_t back_a = (uint32_t)(2 * (8 * a_chunk - min(8 * a_chunk, left - 8)));
         gemm_feed<PER, SLOTS>(n_st, [&](int slot_) {
             uint8_t *st = lds + slot_ * STAGE;
             {
-                const uint8_t *tile = w_base + (long)(2 * fetch + kk) * TILE_BYTES;
-                const uint8_t *arow = a_base + (long)(2 * fetch + kk) * 64;
+                const long step = 2 * fetch + kk;
+                const uint8_t *arow = a_base + step * 64;
+                const bool at_end = RAGGED && ends && fetch == n_st - 1;
+                if constexpr (TILED) {
+                    const uint8_t *tile = w_base + step * TILE_BYTES;
 #pragma unroll
-                for (int bp = 0; bp < 2; ++bp)
-                    __builtin_amdgcn_global_load_lds((gptr_t)(tile + (2 * blk + bp) * 1024 + lane * 16), (lptr_t)(st + (2 * kk + bp) * 1024), 16, 0, 0);
-                __builtin_amdgcn_global_load_lds((gptr_t)(tile + TILE_W_BYTES + lane * 4), (lptr_t)(st + KG_W + kk * 256), 4, 0, 0);
+                    for (int bp = 0; bp < 2; ++bp)
+                        __builtin_amdgcn_global_load_lds((gptr_t)(tile + (2 * blk + bp) * 1024 + lane * 16), (lptr_t)(st + (2 * kk + bp) * 1024), 16, 0, 0);
+                    __builtin_amdgcn_global_load_lds((gptr_t)(tile + TILE_W_BYTES + lane * 4), (lptr_t)(st + KG_W + kk * 256), 4, 0, 0);
+                } else {
+                    const uint8_t *rows = w_base + step * 32 * w_row;
+#pragma unroll
+                    for (int q = 0; q < 2; ++q)
+                        __builtin_amdgcn_global_load_lds((gptr_t)(rows + raw_w[q] - (at_end ? back_w[q] : 0u)), (lptr_t)(st + (2 * kk + q) * 1024), 16, 0, 0);
+                    __builtin_amdgcn_global_load_lds((gptr_t)(s_base + step * 32 * s_row + raw_s - (at_end ? back_s : 0u)), (lptr_t)(st + KG_W + kk * 256), 4, 0, 0);
+                }
 #pragma unroll
                 for (int t = 0; t < TILES; ++t)
-                    __builtin_amdgcn_global_load_lds((gptr_t)(arow + a_voff[t]), (lptr_t)(st + KG_W + KG_S + (kk * TILES + t) * 1024), 16, 0, 0);
+                    __builtin_amdgcn_global_load_lds((gptr_t)(arow + a_voff[t] - (at_end ? back_a : 0u)), (lptr_t)(st + KG_W + KG_S + (kk * TILES + t) * 1024), 16, 0, 0);
             }
             fetch = fetch + 1 == n_st ? 0 : fetch + 1;
         });
@@ -880,8 +915,12 @@ __global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_kg_kern
 
     const int kk = wave8 >> 2, hh = (wave8 >> 1) & 1, bp = wave8 & 1;
     f4 acc[2][TILES];
-    gemm_multiply<TILES, SLOTS, STAGE>(lds, n_st, TiledWeights(hh, (2 * kk + bp) * 1024 + lane * 16, KG_W + kk * 256 + g * 64 + (2 * blk + hh) * 16),
-                                       KG_W + KG_S + kk * TILES * 1024 + c * 64 + ((g ^ ((c >> 1) & 3)) << 4), acc);
+    const auto weights = [&] {
+        if constexpr (TILED) return TiledWeights(hh, (2 * kk + bp) * 1024 + lane * 16, KG_W + kk * 256 + g * 64 + (2 * blk + hh) * 16);
+        else return RowWeights<RAGGED, true>(hh, kk * 2048 + g * 64 + 4 * c, KG_W + kk * 256 + g * 32, 0x0c000c00u | (uint32_t)(2 * bp) | ((uint32_t)(4 + 2 * bp) << 16),
+                                             ends ? (n_st - 1 >= rot ? n_st - 1 - rot : 2 * n_st - 1 - rot) : -1, 32 * (step0 + 2 * (n_st - 1) + kk) + 8 * g >= p.K);
+    }();
+    gemm_multiply<TILES, SLOTS, STAGE>(lds, n_st, weights, KG_W + KG_S + kk * TILES * 1024 + c * 64 + ((g ^ ((c >> 1) & 3)) << 4), acc);
 
     // ---- both groups' sums as rows of 128 floats in LDS; then every thread adds group 0 + group 1 (a fixed order) for
     // 16-byte runs of whole rows and writes the slab: one pass, two barriers, all eight waves storing ----
@@ -905,7 +944,13 @@ __global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_kg_kern
         const int m = m0 + row;
         if (m < p.M && row < p.block_rows) {
             const f4 v = *reinterpret_cast<const f4 *>(sum0 + row * OP + cq) + *reinterpret_cast<const f4 *>(sum1 + row * OP + cq);
-            *reinterpret_cast<f4 *>(slab + (long)m * p.n_total + cq) = v;
+            if (!TILED && p.direct) {
+                const int n = col0 + cq;
+                const h4 o = {matmul_epilogue(p, v[0], m, n), matmul_epilogue(p, v[1], m, n + 1), matmul_epilogue(p, v[2], m, n + 2), matmul_epilogue(p, v[3], m, n + 3)};
+                *reinterpret_cast<h4 *>(seg.c + (long)m * seg.ldc + n) = o;
+            } else {
+                *reinterpret_cast<f4 *>(slab + (long)m * p.n_total + cq) = v;
+            }
         }
     }
 }
@@ -1465,15 +1510,49 @@ static int gemm_launch_layout(const MatmulParams &p, hipStream_t stream) {
     return gemm_launch_rows(kern, p, threads, lds, stream);
 }
 
+// The checkpoint layout's plan for q40_gemm_kg_kernel in the place of p's: one weight, 17 .. 128 rows, never more slabs than p's (whose workspace holds
+// them), none where a workgroup has all of K.
+// It has half the slabs for as many workgroups, or one workgroup a compute unit where p has two of half the waves, but fetches half a line of weights
+// and as many lines of scales for half the columns: per 64 rows of K it takes 0.15 us more than two steps of the 256-column units, and up to 20 % more where
+// rows lie a large power of two apart.  So it is taken
+//   * where p has at most 256 workgroups, of which one XCD gets more than its 32 compute units hold at a time: 21 shapes 1.24 .. 1.85 times as fast;
+//   * where p has one workgroup a compute unit: up to 20 stages (64 rows of K each) a workgroup, above 64 rows 24: 48 shapes 1.02 .. 1.41 times
+//     (above that 0.76 .. 1.07: 37 x 4096 x 11008, 22 stages, 17.1 us and 18.0, 100 x 12288 x 4096, 32 stages, 26.0 and 28.3);
+//   * where p's are more, or cut at runs of steps: up to 48 stages, above 64 rows 64: 10 shapes 1.05 .. 1.64 (20 x 24576 x 4096, 64 stages, 26.1 us and
+//     32.0; 80 x 22400 x 15208 109.6 and 133).
+// us of both launches, in turn: 100 x 4096 x 4096 18.8 and 15.5, 20 x 4096 x 4096 11.4 and 9.8, 100 x 5120 x 5120 28.5 and 17.9, 37 x 7168 x 7168 26.2 and
+// 19.1, 100 x 6400 x 3000 26.7 and 18.5, 100 x 24064 x 1928 35.3 and 24.7.
+bool gemm_blocks_fit(const MatmulParams &p, MatmulParams &b) {
+    // (half a stage past a K that is a multiple of 32 would meet an infinite activation with a zero)
+    if (p.tiled || p.nseg != 1 || p.M <= SMH_GEMV_MAX_M || p.M > GEMM_BM || p.K > 16384 || p.K % 64 == 32) return false;
+    const int blocks = p.seg[0].N / 128, mblocks = blocks <= 32 && p.M > 64 && p.K <= 4096 ? 2 : 1, steps = (p.K + 31) / 32;
+    const int on_xcd = p.units_pad / 4 * mblocks;              // workgroups of a K-slice on the busiest XCD
+    const int ks = min(min(256 / (blocks * mblocks), 32 / on_xcd), min(p.ksplit, steps / 8));
+    if (ks < 1 || blocks * mblocks * ks < 170) return false;
+    b = p;
+    b.kgroups = 2;
+    b.mblocks = mblocks;
+    b.block_rows = mblocks == 2 ? 64 : GEMM_BM;
+    b.chunk = 0;
+    b.steps_per_slice = ((steps + ks - 1) / ks + 1) / 2 * 2;   // a stage of the ring is two steps
+    b.ksplit = (steps + b.steps_per_slice - 1) / b.steps_per_slice;
+    const bool one_round = p.chunk == 0 && (long)p.units * p.mblocks * p.ksplit <= 256;
+    if (one_round && p.units_pad / 8 * p.mblocks * p.ksplit > 32) return true;
+    return b.steps_per_slice / 2 <= (one_round ? (p.M <= 64 ? 20 : 24) : (p.M <= 64 ? 48 : 64));
+}
+
 typedef void (*gemm_kg_kernel_t)(MatmulParams);
 static int gemm_kg_launch(const MatmulParams &p, hipStream_t stream) {
-    static const gemm_kg_kernel_t kern[9] = {nullptr, nullptr, q40_gemm_kg_kernel<2>, q40_gemm_kg_kernel<3>, q40_gemm_kg_kernel<4>, q40_gemm_kg_kernel<5>,
-                                             q40_gemm_kg_kernel<6>, q40_gemm_kg_kernel<7>, q40_gemm_kg_kernel<8>};
+#define KG_KERNELS(...) {nullptr, nullptr, q40_gemm_kg_kernel<2, __VA_ARGS__>, q40_gemm_kg_kernel<3, __VA_ARGS__>, q40_gemm_kg_kernel<4, __VA_ARGS__>, \
+                         q40_gemm_kg_kernel<5, __VA_ARGS__>, q40_gemm_kg_kernel<6, __VA_ARGS__>, q40_gemm_kg_kernel<7, __VA_ARGS__>, q40_gemm_kg_kernel<8, __VA_ARGS__>}
+    static const gemm_kg_kernel_t kern[3][9] = {KG_KERNELS(true, false), KG_KERNELS(false, false), KG_KERNELS(false, true)};
+#undef KG_KERNELS
     static const int lds_bytes[9] = {0, 0, KgShape<2>::LDS, KgShape<3>::LDS, KgShape<4>::LDS, KgShape<5>::LDS, KgShape<6>::LDS, KgShape<7>::LDS, KgShape<8>::LDS};
     static const hipError_t lds_ok = [] {
         hipError_t e = hipSuccess;
-        for (int t = 2; t <= 8 && e == hipSuccess; ++t)
-            e = hipFuncSetAttribute((const void *)kern[t], hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes[t]);
+        for (int t = 2; t <= 8; ++t)
+            for (int form = 0; form < 3 && e == hipSuccess; ++form)
+                e = hipFuncSetAttribute((const void *)kern[form][t], hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes[t]);
         return e;
     }();
     if (lds_ok != hipSuccess) {
@@ -1483,7 +1562,8 @@ static int gemm_kg_launch(const MatmulParams &p, hipStream_t stream) {
     SMH_REQUIRE((long)p.M * p.lda * 2 < (1L << 32), "q40 gemm: M x lda = %d x %ld exceeds the 32-bit lane offsets of A", p.M, p.lda);
     int tiles = p.mblocks > 1 ? p.block_rows / 16 : (p.M + 15) / 16;
     if (tiles < 2) tiles = 2;
-    hipLaunchKernelGGL(kern[tiles], dim3((unsigned)(2 * p.units_pad), (unsigned)p.mblocks, (unsigned)p.ksplit), dim3(64 * (8 + GEMM_DMA_WAVES)), lds_bytes[tiles], stream, p);
+    const int form = p.tiled ? 0 : p.K % 32 == 0 ? 1 : 2;
+    hipLaunchKernelGGL(kern[form][tiles], dim3((unsigned)(2 * p.units_pad), (unsigned)p.mblocks, (unsigned)p.ksplit), dim3(64 * (8 + GEMM_DMA_WAVES)), lds_bytes[tiles], stream, p);
     return launch_status();
 }
 
@@ -1634,7 +1714,7 @@ static int gemm_wide_launch(const MatmulParams &p, int pieces, hipStream_t strea
 int gemm_launch(const MatmulParams &p, hipStream_t stream) {
     MatmulParams w;
     if (const int pieces = gemm_wide_fits(p, w)) return gemm_wide_launch(w, pieces, stream);
-    if (p.kgroups == 2 && p.tiled) return gemm_kg_launch(p, stream);
+    if (p.kgroups == 2) return gemm_kg_launch(p, stream);
     return p.tiled ? gemm_launch_layout<true>(p, stream) : gemm_launch_layout<false>(p, stream);
 }
 

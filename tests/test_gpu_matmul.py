@@ -323,3 +323,30 @@ def test_checkpoint_products_at_the_end_of_k(M, K, N):
     got = Kn.matmul_q40(x, w, s, (K, N)).double()
     want = x.double() @ Kn.deq_int40(w, s, 64, (K, N)).double()
     assert bool(((got - want).abs() <= want.abs() * 2.0 ** -11 + 2.0 ** -24 * K ** 0.5 * want.abs().max()).all())
+
+
+@pytest.mark.parametrize("M", [17, 48, 64, 65, 97, 128])
+@pytest.mark.parametrize("K,N", [(4096, 4096), (4104, 3840), (1928, 24064), (3000, 6400), (2072, 5760), (7168, 7168), (1496, 21760), (1024, 2944)])
+def test_checkpoint_products_in_blocks_of_128_columns(M, K, N):
+    """Launches of 128-column blocks with two K-groups a workgroup: edges of the row tiles and of the two row blocks, odd numbers of blocks, K that ends in
+    the first or the second half of a stage, one slice (stored without slabs) and several, with and without a residual, in rows of a larger output.  Against
+    64 bits: half a unit of fp16 and the fp32 sums; with the residual another half"""
+    from spec_mcts_amd import _lib, kernels as Kn
+    g = torch.Generator(device="cuda").manual_seed(7 * M + K)
+    w, s = Kn.quantize_q40(torch.randn((K, N), device="cuda", generator=g, dtype=torch.float16) * 0.02)
+    x = torch.randn((M, K), device="cuda", generator=g, dtype=torch.float16)
+    r = torch.randn((M, N), device="cuda", generator=g, dtype=torch.float16)
+    want = x.double() @ Kn.deq_int40(w, s, 64, (K, N)).double()
+    err = want.abs() * 2.0 ** -11 + 2.0 ** -24 * K ** 0.5 * want.abs().max()
+    got = Kn.matmul_q40(x, w, s, (K, N)).double()
+    assert bool(((got - want).abs() <= err).all())
+    sum_ = want + r.double()
+    got = Kn.matmul_q40(x, w, s, (K, N), residual=r).double()
+    assert bool(((got - sum_).abs() <= err + (sum_.abs() + err) * 2.0 ** -11).all())
+    wide = torch.full((M, N + 12), float("nan"), device="cuda", dtype=torch.float16)
+    ks = Kn.matmul_plan(M, K, [N])
+    if ks > 1:                                             # (an output row of N + 12: a multiple of 4, which the slabs' sum takes)
+        ws = torch.empty(ks * M * N * 4, dtype=torch.uint8, device="cuda")
+        Kn.check(_lib.load().smh_q40_matmul(x.data_ptr(), M, K, K, w.data_ptr(), s.data_ptr(), N, wide.data_ptr(), N + 12, Kn.SMH_EPI_NONE, None, N, ws.data_ptr(),
+                                            ws.numel(), Kn._stream()), "smh_q40_matmul")
+        assert torch.equal(wide[:, :N], Kn.matmul_q40(x, w, s, (K, N))) and bool(wide[:, N:].isnan().all())
