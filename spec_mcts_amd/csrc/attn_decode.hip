@@ -321,6 +321,7 @@ __global__ __launch_bounds__(256) void attn_prefix_kernel(AttnParams p) {
 // Two tiles a workgroup where one a workgroup would be more than the 768 that run at a time (three a compute unit): 32 heads, 99 branches,
 // 512 positions, 256 of them a prompt 83.1 -> 80.7 us a call (this pass 16.3 -> 14.3), 460 of them 33.2 -> 30.9, 768 with a prompt of 600 68.2 -> 64.6;
 // 100 positions, 448 workgroups of one tile, 22.6 and 23.3 with two.  Three and four tiles: no faster, seven: slower.
+// The grid runs over the tiles first and the slices last: the first slices are the likely ones, and their workgroups start together (13.8 us before, 12.8).
 constexpr int PT_TW = 64;
 constexpr long PT_ROUND = 768;
 constexpr int PT_MAX_SLICES = 64;          // one bit a slice in the suffix kernel's mask
@@ -356,7 +357,7 @@ __global__ __launch_bounds__(256) void attn_page_tile_kernel(AttnParams p) {
     __shared__ long s_row[PT_TILES][PT_TW];        // rows of the tiles' first branches
     __shared__ float s_max[4][16], s_sum[4][16];
     __shared__ uint32_t s_bits[4];
-    const int hk = blockIdx.x, split = blockIdx.y, tiles = (p.Bq + 15) / 16, tile0 = blockIdx.z * PT_TILES, n_tiles = min(PT_TILES, tiles - tile0);
+    const int hk = blockIdx.x, split = blockIdx.z, tiles = (p.Bq + 15) / 16, tile0 = blockIdx.y * PT_TILES, n_tiles = min(PT_TILES, tiles - tile0);
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, c = lane & 15, g = lane >> 4;
     const int t0 = split * PT_TW, cnt = min(PT_TW, (int)p.suffix_batch_stride_rows - t0);
     // a tile's queries (B operand of S^T)
@@ -897,7 +898,7 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
         }
         // ---- this branch's suffix: group g takes rows g, g+4, ... in batches ----
         uint64_t tiles = 0;                                 // bit s: slice s is done
-        if (TILES) tiles = __ballot(lane < p.splits && p.tile_done[((long)hk * ((p.Bq + 15) / 16) + (qrow >> 4)) * p.splits + min(lane, p.splits - 1)] != 0);
+        constexpr int TILE_PARTS = TILES ? 2 : 0;           // partials of a group that are folded in before the walk
         if (WALK == WALK_F16 || TILES || (WALK == WALK_ANY && p.suffix_format == SMH_KV_FP16)) {
             // Batches of U rows per group, the next one (and the ids of the one after it) on its way while this one is used; one
             // maximum and one rescale a batch.
@@ -934,15 +935,45 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
                 ql = q_raw[0].lo;
                 qh = q_raw[0].hi;
             }
+            // What the walk begins with comes in as few trips as there are dependent loads: the first ids (of no use where the first slice is done) with the
+            // marks, the slices' partials with the first rows and not behind the last (us, in turn, the grid of attn_page_tile_kernel included: 32 heads,
+            // 99 branches, 512 positions, 256 of them a prompt 87.3 -> 84.8, 62 branches, 273 positions, 95 of them 37.3 -> 34.6, 4 branches, 683
+            // positions 16.0 -> 15.0; 16 branches, nothing shared over a slice, 13.2 -> 13.6).
+            if constexpr (TILES) {
+                const uint8_t mark = p.tile_done[((long)hk * ((p.Bq + 15) / 16) + (qrow >> 4)) * p.splits + min(lane, p.splits - 1)];
+                ids(0);
+                tiles = __ballot(lane < p.splits && mark != 0);
+            }
             int i0 = next(-1), i1 = n_batches;
             Batch cur;
             if (i0 < n_batches) {
-                ids(i0);
+                if (!TILES || i0 > 0) ids(i0);
                 rows(cur);
                 i1 = next(i0);
                 if (i1 < n_batches) ids(i1);
             }
+            f4 part_lo[TILE_PARTS + 1], part_hi[TILE_PARTS + 1];
+            float part_m[TILE_PARTS + 1], part_l[TILE_PARTS + 1];
+#pragma unroll
+            for (int i = 0; i < TILE_PARTS; ++i) {
+                const int sp = gg + gstride * i;
+                if (sp < p.splits && ((tiles >> sp) & 1) != 0) {
+                    const long base = ((long)sp * p.Hkv + hk) * p.Bq + qrow;
+                    part_lo[i] = *reinterpret_cast<const f4 *>(p.part_o + base * ATT_D + 4 * c);
+                    part_hi[i] = *reinterpret_cast<const f4 *>(p.part_o + base * ATT_D + 64 + 4 * c);
+                    part_m[i] = p.part_ml[base * 2];
+                    part_l[i] = p.part_ml[base * 2 + 1];
+                }
+            }
             wait_loads();
+#pragma unroll
+            for (int i = 0; i < TILE_PARTS; ++i) {
+                const int sp = gg + gstride * i;
+                if (sp < p.splits && ((tiles >> sp) & 1) != 0) {
+                    const float o2[8] = {part_lo[i][0], part_lo[i][2], part_lo[i][1], part_lo[i][3], part_hi[i][0], part_hi[i][2], part_hi[i][1], part_hi[i][3]};
+                    soft_merge(st, part_m[i], part_l[i], o2);
+                }
+            }
             while (i0 < n_batches) {
                 Batch nxt;
                 int i2 = n_batches;
@@ -1115,7 +1146,7 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
                 soft_merge(st, pre_m[i], pre_l[i], o2);
             }
         }
-        for (int sp = gg + gstride * PRE; !PARTIAL && sp < p.splits; sp += gstride) {
+        for (int sp = gg + gstride * (PRE + TILE_PARTS); !PARTIAL && sp < p.splits; sp += gstride) {
             if (TILES && ((tiles >> sp) & 1) == 0) continue;
             const long base = ((long)sp * p.Hkv + hk) * p.Bq + qrow;
             const f4 lo = *reinterpret_cast<const f4 *>(p.part_o + base * ATT_D + 4 * c);
@@ -2102,7 +2133,7 @@ static int shared_prefix_attn(const char *who, bool one, const void *q, void *ou
         const auto one = pb == 2 ? attn_page_tile_kernel<2, 1> : pb == 4 ? attn_page_tile_kernel<4, 1> : attn_page_tile_kernel<8, 1>;
         const auto two = pb == 2 ? attn_page_tile_kernel<2, 2> : pb == 4 ? attn_page_tile_kernel<4, 2> : attn_page_tile_kernel<8, 2>;
         const auto walk = pb == 2 ? attn_suffix_kernel<false, WALK_TILES, 2> : pb == 4 ? attn_suffix_kernel<false, WALK_TILES, 4> : attn_suffix_kernel<false, WALK_TILES, 8>;
-        hipLaunchKernelGGL(each == 2 ? two : one, dim3(Hkv, p.splits, (tiles + each - 1) / each), dim3(256), 0, (hipStream_t)stream, p);
+        hipLaunchKernelGGL(each == 2 ? two : one, dim3(Hkv, (tiles + each - 1) / each, p.splits), dim3(256), 0, (hipStream_t)stream, p);
         hipLaunchKernelGGL(walk, dim3(wgs), dim3(256), 0, (hipStream_t)stream, p);
         return launch_status();
     }

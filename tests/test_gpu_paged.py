@@ -315,3 +315,24 @@ def test_nan_in_a_query_stays_visible_through_pages(shared):
     assert bool(got[1, 2].isnan().all())
     got[1, 2] = clean[1, 2] = 0
     assert torch.equal(got, clean)
+
+
+@pytest.mark.parametrize("B,L,shared", [(40, 64 * 11 + 5, (0, 64 * 9)), (40, 64 * 11 + 5, (0, 64 * 11 + 5)), (40, 64 * 11 + 5, (64 * 2, 64 * 10)),
+                                        (20, 64 * 3, (64 * 2, 64 * 3)), (3, 64 * 33, (0, 64 * 32)), (17, 15, (0, 15))])
+def test_walks_over_pages_behind_shared_slices(B, L, shared):
+    """The walk of what a tile's branches do not share: first and last slices that are shared, and of few positions, shared slices in the middle,
+    nothing left to walk, and more partials than are folded in before it (two a group of lanes), with one and with several waves a query"""
+    from spec_mcts_amd import kernels as K
+    g = torch.Generator().manual_seed(L + B)
+    H, lo, hi = 8, *shared
+    own = L - (hi - lo)
+    rows = (hi - lo) + B * own + 1
+    pages = torch.zeros((B, L), dtype=torch.int32)
+    pages[:, lo:hi] = torch.randperm(hi - lo, generator=g).int()
+    rest = [i for i in range(L) if not lo <= i < hi]
+    pages[:, rest] = (hi - lo) + torch.arange(B * own, dtype=torch.int32).view(B, own)
+    k, v = (torch.empty((H, rows, 128)).normal_(0.0, 0.5, generator=g).half() for _ in range(2))
+    q = torch.empty((B, H, 128)).normal_(0.0, 0.5, generator=g).half()
+    want = sdpa(q, pages, k, v)
+    got = K.paged_prefix_attn(q.cuda(), pages.cuda(), None, k.cuda(), v.cuda(), head_major=True).cpu().float()
+    assert bool(((got - want).abs() <= 2e-3 + 1e-2 * want.abs()).all())
