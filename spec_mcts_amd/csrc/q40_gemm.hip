@@ -119,7 +119,7 @@ __device__ __forceinline__ void gemm_feed(int n, Issue issue) {
 }
 template <int N> using int_constant = std::integral_constant<int, N>;
 
-// What a multiplying wave reads of a stage's weights, and half a row pair of its operands out of that: rows (2 j, 2 j + 1) of the piece's first
+// What a multiplying wave reads of a stage's weights, and its operands out of that (gemm_decode): rows (2 j, 2 j + 1) of the piece's first
 // (o = 0) or second byte, the nibble (high: hh = 0, low) as fp16 code * scale.
 struct NibbleConsts {
     uint32_t mask, magic;
@@ -142,10 +142,11 @@ struct TiledWeights {
     __device__ __forceinline__ Regs load(const uint8_t *st, int) const {
         return Regs{*reinterpret_cast<const u32x4 *>(st + w_off), *reinterpret_cast<const u32x4 *>(st + s_off)};
     }
-    __device__ __forceinline__ uint32_t decode(const Regs &r, int j, int o) const {
+    __device__ __forceinline__ uint32_t bits(const Regs &r, int j, int o) const {
         const uint32_t w = r.w[(j & 1) + 2 * o], pr = j < 2 ? w : w >> 8;
-        return as_u32(nib.code((pr & nib.mask) | nib.magic) * as_h2(r.scales[j]));
+        return (pr & nib.mask) | nib.magic;
     }
+    __device__ __forceinline__ h2 scale(const Regs &r, int j) const { return as_h2(r.scales[j]); }
 };
 // Checkpoint layout: row 8 g + r of a stage (GS_WBLOCK) and its scales (of the block's first, second 64 columns in a dword).
 // RAGGED: stage `last` is the end of K, where `dead` says that this lane's rows lie past it (their scales become zero).
@@ -179,22 +180,50 @@ struct RowWeights {
         }
         return x;
     }
-    __device__ __forceinline__ uint32_t decode(const Regs &x, int j, int o) const {
+    __device__ __forceinline__ uint32_t bits(const Regs &x, int j, int o) const {
         const uint32_t pr = __builtin_amdgcn_perm(x.w[2 * j + 1], x.w[2 * j], o == 0 ? sel : sel + 0x00010001u);
-        const uint32_t pair = __builtin_amdgcn_perm(x.s[2 * j + 1], x.s[2 * j], half), sc = RAGGED ? pair & x.keep : pair;
-        return as_u32(nib.code((pr & nib.mask) ^ nib.magic) * as_h2(sc));
+        return (pr & nib.mask) ^ nib.magic;
+    }
+    __device__ __forceinline__ h2 scale(const Regs &x, int j) const {
+        const uint32_t pair = __builtin_amdgcn_perm(x.s[2 * j + 1], x.s[2 * j], half);
+        return as_h2(RAGGED ? pair & x.keep : pair);
     }
 };
 
+// A stage's B operands, one kind of instruction after the other: a packed product that reads the result of the packed fma before it waits (the compiler puts
+// an s_nop between them), and a row pair at a time had one such wait each.
+template <class Weights, class Regs>
+__device__ __forceinline__ void gemm_decode(const Weights &weights, const Regs &w, u32x4 (&b)[2]) {
+    uint32_t bits[8];
+    h2 scale[4], code[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) bits[u] = weights.bits(w, u >> 1, u & 1);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) scale[j] = weights.scale(w, j);
+    // (all of them, not one by one where the fma needs it)
+    asm volatile("" : "+v"(bits[0]), "+v"(bits[1]), "+v"(bits[2]), "+v"(bits[3]), "+v"(bits[4]), "+v"(bits[5]), "+v"(bits[6]), "+v"(bits[7]));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) code[u] = weights.nib.code(bits[u]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) b[u & 1][u >> 1] = as_u32(code[u] * scale[u >> 1]);
+}
+
 // The products of one multiplying wave of the kernels below: n stages of a ring of SLOTS slots, B operands (one nibble of one piece, 16 columns of either
 // byte) x TILES row tiles.  A wave keeps the A rows and the B operands of ONE stage in registers.  As soon as a row tile's two products are
-// issued its registers take the next stage's rows, and the next nibbles, read first, are decoded between the products: no read is waited for where it
+// issued its registers take the next stage's rows, and the next nibbles, read first, are decoded behind the last product: no read is waited for where it
 // was issued.  Left to the compiler each pair of products waited for its own read - with the products 780 cycles a stage of 112 rows x 128 columns x 64,
-// 448 of them on the matrix pipe.
+// 448 of them on the matrix pipe.  (Decoded between the products, row pair by row pair, us before and now: tiled weights, 512 x 4096 x 11008 45.6 and 43.9,
+// 2047 rows 155 and 149, SwiGLU at 2047 rows 339 and 335, wo at 100 rows 9.16 and 8.95.  In the middle of the products in half of the waves, so that some
+// decode while others multiply: level or up to 6 % slower.)
+// PRIO: GEMM_PRODUCTS_FIRST where two waves a SIMD share it, GEMM_DECODE_FIRST where three do (us without and with: SwiGLU at 128 rows 32.7 and 31.6, at 100
+// 29.5 and 28.9; at 512 rows 91.6 and 90.0, at 2047 353 and 349; the 256-column units are level).
 // Stages go in pairs, one barrier a pair (gemm_feed): at the barrier before stages i, i + 1 the stages up to i + 2 have landed, whose rows
 // and nibbles stage i + 1 reads; past the last stage stale bytes are read, decoded and never used.
 // Not AHEAD: a stage's rows are read in it, and the compiler puts reads and decode where it likes.
-template <int TILES, int SLOTS, int STAGE, bool AHEAD = true, class Weights>
+enum { GEMM_EVEN, GEMM_PRODUCTS_FIRST, GEMM_DECODE_FIRST };
+template <int TILES, int SLOTS, int STAGE, int PRIO = GEMM_EVEN, bool AHEAD = true, class Weights>
 __device__ __forceinline__ void gemm_multiply(const uint8_t *lds, int n, const Weights &weights, int a_off, f4 (&acc)[2][TILES]) {
 #pragma unroll
     for (int o = 0; o < 2; ++o)
@@ -210,9 +239,9 @@ __device__ __forceinline__ void gemm_multiply(const uint8_t *lds, int n, const W
 #pragma unroll
             for (int t = 0; t < TILES; ++t) av[t] = *reinterpret_cast<const h8 *>(lds + a_off + t * 1024);
         }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) bq[u & 1][u >> 1] = weights.decode(w, u >> 1, u & 1);
+        gemm_decode(weights, w, bq);
     }
+    if constexpr (PRIO == GEMM_PRODUCTS_FIRST) __builtin_amdgcn_s_setprio(1);
     int slot = 0;
     auto one_stage = [&](int next) {
         const uint8_t *here = lds + slot * STAGE;
@@ -227,31 +256,24 @@ __device__ __forceinline__ void gemm_multiply(const uint8_t *lds, int n, const W
             for (int t = 0; t < TILES; ++t)
 #pragma unroll
                 for (int o = 0; o < 2; ++o) acc[o][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[t], __builtin_bit_cast(h8, bq[o]), acc[o][t], 0, 0, 0);
-#pragma unroll
-            for (int u = 0; u < 8; ++u) bn[u & 1][u >> 1] = weights.decode(w, u >> 1, u & 1);
+            gemm_decode(weights, w, bn);
             bq[0] = bn[0];
             bq[1] = bn[1];
             return;
         }
         const auto w = weights.load(st, next);
         __builtin_amdgcn_sched_barrier(0);
-        u32x4 bn[2];
-        constexpr int FROM = TILES >= 4 ? 2 : TILES - 1;       // the row tile under whose products the decode begins
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
 #pragma unroll
             for (int o = 0; o < 2; ++o) acc[o][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[t], __builtin_bit_cast(h8, bq[o]), acc[o][t], 0, 0, 0);
             av[t] = *reinterpret_cast<const h8 *>(st + a_off + t * 1024);
-#pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (t == FROM + u * (TILES - FROM) / 8) {
-                    bn[u & 1][u >> 1] = weights.decode(w, u >> 1, u & 1);
-                    asm volatile("" : "+v"(bn[u & 1][u >> 1]));      // (here, not where it is needed)
-                }
             __builtin_amdgcn_sched_barrier(0);
         }
-        bq[0] = bn[0];
-        bq[1] = bn[1];
+        if constexpr (PRIO != GEMM_EVEN) __builtin_amdgcn_s_setprio(PRIO == GEMM_DECODE_FIRST ? 1 : 0);
+        gemm_decode(weights, w, bq);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (PRIO != GEMM_EVEN) __builtin_amdgcn_s_setprio(PRIO == GEMM_DECODE_FIRST ? 0 : 1);
     };
     // The slots that are refilled behind a barrier were read a stage ago, by reads older than the last stage's TILES + READS
     auto meet = [] {
@@ -920,7 +942,7 @@ __global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_kg_kern
         else return RowWeights<RAGGED, true>(hh, kk * 2048 + g * 64 + 4 * c, KG_W + kk * 256 + g * 32, 0x0c000c00u | (uint32_t)(2 * bp) | ((uint32_t)(4 + 2 * bp) << 16),
                                              ends ? (n_st - 1 >= rot ? n_st - 1 - rot : 2 * n_st - 1 - rot) : -1, 32 * (step0 + 2 * (n_st - 1) + kk) + 8 * g >= p.K);
     }();
-    gemm_multiply<TILES, SLOTS, STAGE>(lds, n_st, weights, KG_W + KG_S + kk * TILES * 1024 + c * 64 + ((g ^ ((c >> 1) & 3)) << 4), acc);
+    gemm_multiply<TILES, SLOTS, STAGE, GEMM_PRODUCTS_FIRST>(lds, n_st, weights, KG_W + KG_S + kk * TILES * 1024 + c * 64 + ((g ^ ((c >> 1) & 3)) << 4), acc);
 
     // ---- both groups' sums as rows of 128 floats in LDS; then every thread adds group 0 + group 1 (a fixed order) for
     // 16-byte runs of whole rows and writes the slab: one pass, two barriers, all eight waves storing ----
@@ -1029,7 +1051,7 @@ __global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_swiglu_
 
     const int kk = wave8 >> 2, hh = (wave8 >> 1) & 1, gu = wave8 & 1;       // K-group, nibble, gate (0) or up (1)
     f4 acc[2][TILES];
-    gemm_multiply<TILES, SLOTS, STAGE>(lds, n_st, TiledWeights(hh, (2 * kk + gu) * 1024 + lane * 16, KG_W + (2 * kk + gu) * 256 + g * 64 + (2 * blk + hh) * 16),
+    gemm_multiply<TILES, SLOTS, STAGE, GEMM_PRODUCTS_FIRST>(lds, n_st, TiledWeights(hh, (2 * kk + gu) * 1024 + lane * 16, KG_W + (2 * kk + gu) * 256 + g * 64 + (2 * blk + hh) * 16),
                                        KG_W + S::SC + kk * TILES * 1024 + c * 64 + ((g ^ ((c >> 1) & 3)) << 4), acc);
 
     // ---- both groups' sums as rows of 64 gate and 64 up columns in LDS, then every thread adds group 0 + group 1 (a fixed order) of four columns ----
@@ -1181,7 +1203,7 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + GEMM_DMA_WAVES), 1) void q40_gem
     f4 acc[2][TILES];
     // (Seven row tiles: reading ahead needs more than the 128 registers of four waves a SIMD, and does not gain what that costs.  In us, ahead and not:
     // w1|w3 and wq|wk|wv of the 7B shape at 400 rows 90.1, 52.9 and 86.2, 49.3, w1|w3 of the 70B shape at 540 rows 551 and 524.)
-    gemm_multiply<TILES, SLOTS, STAGE, TILES != 7>(lds, n_st, TiledWeights(hh, s * 1024 + lane * 16, S::W + s * 128 + g * 32 + hh * 16),
+    gemm_multiply<TILES, SLOTS, STAGE, GEMM_DECODE_FIRST, TILES != 7>(lds, n_st, TiledWeights(hh, s * 1024 + lane * 16, S::W + s * 128 + g * 32 + hh * 16),
                                        S::W + S::SC + (MODE == WIDE_GROUPS ? half * TILES * 1024 : 0) + c * 64 + ((g ^ ((c >> 1) & 3)) << 4), acc);
 
     // rows of 64 PIECES columns: local column 64 k3 + 32 hh + 2 c + o is column 128 (P / 2) + 64 hh + 4 c + 2 (P % 2) + o, P the piece;
