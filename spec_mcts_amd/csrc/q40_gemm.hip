@@ -191,9 +191,15 @@ struct RowWeights {
 };
 
 // A stage's B operands, one kind of instruction after the other: a packed product that reads the result of the packed fma before it waits (the compiler puts
-// an s_nop between them), and a row pair at a time had one such wait each.
+// an s_nop between them), and a row pair at a time had one such wait each.  The checkpoint layout's, whose sixteen dwords of rows arrive one after the other, go
+// as the compiler orders them (like the others 37 x 11008 x 4096 16.9 us and 16.5, 48 rows 17.6 and 17.2, 80 rows 21.3 and 20.9).
 template <class Weights, class Regs>
 __device__ __forceinline__ void gemm_decode(const Weights &weights, const Regs &w, u32x4 (&b)[2]) {
+    if constexpr (Weights::READS > 2) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) b[u & 1][u >> 1] = as_u32(weights.nib.code(weights.bits(w, u >> 1, u & 1)) * weights.scale(w, u >> 1));
+        return;
+    }
     uint32_t bits[8];
     h2 scale[4], code[8];
 #pragma unroll
