@@ -1350,7 +1350,10 @@ __global__ __launch_bounds__(256, 4) void attn_parts_kernel(AttnParams p, int pr
     attn_suffix_body<false, true, WALK_F16, PB>(p, b, min(h, p.H - 1), hq & (nsub - 1), nsub, h < p.H);
 }
 
-// One wave per query adds its splits + 1 partials up, in split order: lane d holds dims 2 d, 2 d + 1.
+// One wave per query adds its splits + 1 partials up, in split order: lane d holds dims 2 d, 2 d + 1.  N partials are on their way at a time: what another XCD
+// has just written takes ~2 us to come, so all of them are asked for at once where they are at most 17 (us a call, 64 branches after 1024 rows, nine partials,
+// of which eight came in a first trip before, 44.3 and 43.0; 13 after 1740, 64 heads over 8, 23.4 and 21.2; one after 1011 14.4 and 11.5).
+template <int N>
 __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p) {
     args_ahead<sizeof(AttnParams)>();
     const int qi = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;       // kv head * Bq + query of the kv head
@@ -1358,28 +1361,34 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p) {
     if (qi >= queries) return;
     float m = -INFINITY, l = 0.f;
     f2 o = {0.f, 0.f};
-    constexpr int N = 8;                                     // partials on their way at a time
     for (int s0 = 0; s0 <= p.splits; s0 += N) {
         f2 v[N], ml[N];
 #pragma unroll
-        for (int i = 0; i < N; ++i) {
-            ml[i] = f2{-INFINITY, 0.f};
-            v[i] = f2{0.f, 0.f};
-            if (s0 + i <= p.splits) {
-                const long base = (long)(s0 + i) * queries + qi;
-                ml[i] = *reinterpret_cast<const f2 *>(p.part_ml + base * 2);
-                v[i] = *reinterpret_cast<const f2 *>(p.part_o + base * ATT_D + 2 * lane);
-            }
+        for (int i = 0; i < N; ++i) {                        // (past the last one: it again, which weighs nothing)
+            const long base = (long)min(s0 + i, p.splits) * queries + qi;
+            ml[i] = *reinterpret_cast<const f2 *>(p.part_ml + base * 2);
+            v[i] = *reinterpret_cast<const f2 *>(p.part_o + base * ATT_D + 2 * lane);
         }
+        float m_new = m;
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-            const float m_new = fmaxf(m, ml[i][0]);
-            if (m_new == -INFINITY) continue;                // nothing yet
-            const float c1 = exp2f(m - m_new), c2 = exp2f(ml[i][0] - m_new);
-            m = m_new;
-            l = l * c1 + ml[i][1] * c2;
-            o[0] = o[0] * c1 + v[i][0] * c2;
-            o[1] = o[1] * c1 + v[i][1] * c2;
+            if (s0 + i > p.splits) {
+                ml[i] = f2{-INFINITY, 0.f};
+                v[i] = f2{0.f, 0.f};
+            }
+            m_new = fmaxf(m_new, ml[i][0]);
+        }
+        const float m_ref = m_new == -INFINITY ? 0.f : m_new, corr = exp2f(m - m_ref);       // (nothing yet: every factor is exp2(-inf) = 0)
+        m = m_new;
+        l *= corr;
+        o[0] *= corr;
+        o[1] *= corr;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const float c = exp2f(ml[i][0] - m_ref);
+            l += ml[i][1] * c;
+            o[0] += v[i][0] * c;
+            o[1] += v[i][1] * c;
         }
     }
     const int hk = qi / p.Bq, qrow = qi - hk * p.Bq;
@@ -2116,7 +2125,8 @@ static int shared_prefix_attn(const char *who, bool one, const void *q, void *ou
         const dim3 grid((unsigned)(prefix_wgs + wgs));
         const auto parts = pb == 0 ? attn_parts_kernel<0> : pb == 2 ? attn_parts_kernel<2> : pb == 4 ? attn_parts_kernel<4> : attn_parts_kernel<8>;
         hipLaunchKernelGGL(parts, grid, dim3(256), 0, (hipStream_t)stream, p, (int)prefix_wgs, rounds);
-        hipLaunchKernelGGL(attn_merge_kernel, dim3((unsigned)(((long)Hkv * p.Bq + 3) / 4)), dim3(256), 0, (hipStream_t)stream, p);
+        const auto merge = p.splits < 5 ? attn_merge_kernel<5> : p.splits < 9 ? attn_merge_kernel<9> : attn_merge_kernel<17>;
+        hipLaunchKernelGGL(merge, dim3((unsigned)(((long)Hkv * p.Bq + 3) / 4)), dim3(256), 0, (hipStream_t)stream, p);
         return launch_status();
     }
     if (p.splits > 0)

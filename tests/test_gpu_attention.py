@@ -468,3 +468,18 @@ def test_prefill_lengths_around_the_tiles(S, H, Hkv):
     g = _g(500 + S)
     q, k, v = (torch.randn((S, h, 128), generator=g).half() for h in (H, Hkv, Hkv))
     _check(K.prefill_attn(q.cuda(), k.cuda(), v.cuda()), O.causal_attention(q, k, v))
+
+
+@pytest.mark.parametrize("P", [1, 128, 129, 256, 257, 512, 513, 1050])
+def test_merge_at_every_number_of_partials_on_their_way(P):
+    """fp16 suffixes: slices of 32 prompt rows and the suffix leave 2, 5, 6, 9, 10, 17, 18 and 34 partials a query; the merge has 5, 9 or 17 of them on
+    their way at a time.  A prompt of scores that rise by 30 from slice to slice lets the last ones outweigh the first; branches without rows"""
+    from spec_mcts_amd import kernels as K
+    B, S = 5, 9
+    q, pk, pv, sk, sv, lens = _inputs(B, 1, 1, 128, P, S, 60 + P)
+    lens[0] = 0
+    for rise in (0.0, 30.0):
+        k = pk.clone()
+        k[..., 0] += rise * (torch.arange(P) // 32).half()[:, None] / 16
+        want = O.shared_prefix_attention(q, k, pv, sk, sv, lens.tolist())
+        _check(K.shared_prefix_attn(q.cuda(), k.cuda(), pv.cuda(), P, suffix_k=sk.cuda(), suffix_v=sv.cuda(), Smax=S, lens=lens.cuda(), lens_stride=1), want)
