@@ -9,8 +9,8 @@
 //   * two LOADING waves bring its tiles into a ring of 26 in LDS by DMA, linear after linear, layer after layer, as far ahead as
 //     the ring has room.  (In the multiplying waves, a ring each, the loads stopped with the multiplying: 57 us a layer against 46.)
 //   * eight MULTIPLYING waves: wave (piece q, class e) multiplies piece q (64 of the 256 columns, 1 KB of nibbles) of every third tile
-//     with the activations in LDS (16 x 16 x 32 products, decoded as in q40_gemv.hip).  Its first five tiles are in registers
-//     before the activations come, which makes the ring 15 tiles longer.
+//     with the activations in LDS (16 x 16 x 32 products, decoded as in q40_gemv.hip).  Its first five or six tiles are in registers
+//     before the activations come, which makes the ring 15 to 18 tiles longer, and two of them decoded with one or two branches.
 //   * six COMMUNICATING waves: they wait for a linear's activations, leave them in LDS, add up and publish the products, and do
 //     what lies between the linears (RMSNorm, attention, SiLU, residual adds).  Four of them multiply the third class of tiles.
 // They meet at counters in LDS: a barrier would stop the loads, too.
@@ -318,8 +318,11 @@ __device__ __forceinline__ void load_wave(const StackWave &s, uint8_t *lds, Gate
 
 // ---- multiplying -------------------------------------------------------------------------------------------------------
 // Wave (piece q, class e) multiplies piece q (64 of a tile's 256 columns) of the tiles e, e + DS_CLASSES, .. of a run.  While it waits
-// for the activations it holds its first AHEAD pieces in registers: as much room more in the ring.
-template <int M, int AHEAD>
+// for the activations it holds its first AHEAD pieces in registers: as much room more in the ring.  DECODED of them it decodes there already, which leaves
+// their products alone between the activations and the sums (us a step of the 7B architecture, five pieces, none decoded, and now, in turn: 1 branch behind 512
+// rows 1435 and 1398, behind 2047 1612 and 1582, 2 branches behind 512 1586 and 1548; three of five pieces decoded 1398, 1588, 1555, four 1436, three of six,
+// which spills, 1509).  From three branches on it gained nothing (1822 and 1830; 4: 2115 and 2145): five pieces, as they come.
+template <int M, int AHEAD, int DECODED>
 struct Multiplier {
     const StackParams &p;
     uint8_t *lds;
@@ -389,18 +392,24 @@ struct Multiplier {
 #pragma unroll
             for (int h = 0; h < 2; ++h) acc[i][h] = f4{0.f, 0.f, 0.f, 0.f};
         int pc = 0, j = cls;
+        auto decode = [&](const Piece &t, int half, u32x4 &vh, u32x4 &vl) {
+            const uint32_t pr[4] = {t.w[2 * half], t.w[2 * half + 1], t.w[2 * half] >> 8, t.w[2 * half + 1] >> 8};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                vh[k] = as_u32((as_h2((pr[k] & mask_hi) | magic_hi) + off_hi) * as_h2(t.sh[k]));
+                vl[k] = as_u32((as_h2((pr[k] & mask_lo) | magic_lo) + off_lo) * as_h2(t.sl[k]));
+            }
+        };
+        auto product = [&](int half, const u32x4 &vh, const u32x4 &vl, const h8 &xv) {
+            acc[half][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv, __builtin_bit_cast(h8, vh), acc[half][0], 0, 0, 0);
+            acc[half][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv, __builtin_bit_cast(h8, vl), acc[half][1], 0, 0, 0);
+        };
         auto multiply = [&](const Piece &t, const h8 &xv) {
 #pragma unroll
             for (int half = 0; half < 2; ++half) {
-                const uint32_t pr[4] = {t.w[2 * half], t.w[2 * half + 1], t.w[2 * half] >> 8, t.w[2 * half + 1] >> 8};
                 u32x4 vh, vl;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    vh[k] = as_u32((as_h2((pr[k] & mask_hi) | magic_hi) + off_hi) * as_h2(t.sh[k]));
-                    vl[k] = as_u32((as_h2((pr[k] & mask_lo) | magic_lo) + off_lo) * as_h2(t.sl[k]));
-                }
-                acc[half][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv, __builtin_bit_cast(h8, vh), acc[half][0], 0, 0, 0);
-                acc[half][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv, __builtin_bit_cast(h8, vl), acc[half][1], 0, 0, 0);
+                decode(t, half, vh, vl);
+                product(half, vh, vl, xv);
             }
         };
         auto next = [&](int i) { return first + (uint32_t)(i < len ? i : len + cls); };      // this wave's tile at or behind i of the run
@@ -418,6 +427,16 @@ struct Multiplier {
                 pre[u] = fetch(first + j + u * DS_CLASSES);
             }
         release(next(j + AHEAD * DS_CLASSES));
+        u32x4 ready[DECODED + 1][2][2];
+#pragma unroll
+        for (int u = 0; u < DECODED; ++u)
+            if (j + u * DS_CLASSES < len) {
+#pragma unroll
+                for (int half = 0; half < 2; ++half) {
+                    decode(pre[u], half, ready[u][half][0], ready[u][half][1]);
+                    asm volatile("" : "+v"(ready[u][half][0]), "+v"(ready[u][half][1]));       // (here, not where it is needed)
+                }
+            }
         x_due += DS_COM;
         wait_for(&gates->x, x_due);
         Piece cur = pre[0];
@@ -431,7 +450,12 @@ struct Multiplier {
                     await(first + j + DS_CLASSES);
                     cur = fetch(first + j + DS_CLASSES);
                 }
-                multiply(pre[u], xv);
+                if (u < DECODED) {
+#pragma unroll
+                    for (int half = 0; half < 2; ++half) product(half, ready[u][half][0], ready[u][half][1], xv);
+                } else {
+                    multiply(pre[u], xv);
+                }
                 j += DS_CLASSES;
                 if (another) release(next(j + DS_CLASSES));
             }
@@ -464,7 +488,7 @@ template <int M>
 __device__ __forceinline__ void multiply_waves(const StackWave &s, uint8_t *lds, Gates *gates) {
     const StackParams &p = s.p;
     const StackLds at = stack_lds(M, p.x_pitch);
-    Multiplier<M, 5> mul{p, lds, gates, s.wave & 3, s.wave >> 2, s.lane, 0u, 0u, 0u, 0u};
+    Multiplier<M, M <= 2 ? 6 : 5, M <= 2 ? 2 : 0> mul{p, lds, gates, s.wave & 3, s.wave >> 2, s.lane, 0u, 0u, 0u, 0u};
     for (int layer = 0; layer < p.layers; ++layer)
         for (int lin = 0; lin < 4; ++lin) {
             const StackLinear L = p.lin[lin];
@@ -520,7 +544,7 @@ struct StackCom {
     StackSpace sp;
     bool late;
     uint32_t met, sums_due;                    // counts of the gates
-    Multiplier<M, 1> mul;                      // of the first four waves
+    Multiplier<M, 1, 0> mul;                      // of the first four waves
     int t_now;                                 // the step's suffix index and, of this lane's dims, its rotation
     half_t cos_l, sin_l;
 
@@ -1004,7 +1028,7 @@ __global__ __launch_bounds__(DS_THREADS) void decode_stack_kernel(StackParams p)
         } else {
             constexpr int first = DS_MUL + DS_DMA;
             StackCom<M> com{p, id, n, wave - first, tid & 63, tid - first * 64, 0u, lds, gates, at, stack_space(M, p.dim, p.ffn, p.heads), false, 0u, 0u,
-                            Multiplier<M, 1>{p, lds, gates, (wave - first) & 3, 2, tid & 63, 0u, 0u, 0u, 0u}, 0, (half_t)0.f, (half_t)0.f};
+                            Multiplier<M, 1, 0>{p, lds, gates, (wave - first) & 3, 2, tid & 63, 0u, 0u, 0u, 0u}, 0, (half_t)0.f, (half_t)0.f};
             com.run(epoch);
         }
     }
