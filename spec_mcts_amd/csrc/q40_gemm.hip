@@ -1652,6 +1652,27 @@ int gemm_swiglu_columns(MatmulParams p) {
     return gemm_swiglu_rows_plan(p, w) ? 384 : 256;
 }
 
+// w.units columns of workgroups of three pieces, w.mblocks row blocks, need rounds of which the last can be a poor one (w1|w3 of the 7B shape at 2047 rows: 928
+// workgroups, 3.6 rounds): the units of a first launch where a second one of two pieces of each weight a workgroup (256 columns) for the columns behind
+// them promises 3 % less, 0: none does.  Rounds on the busiest XCD, without what full ones cost in clock.  45 launches at 430 .. 2047 rows of the 7B, 13B, 34B and
+// 70B shapes and of 4096 -> 2 x 14336, promised 0.82 .. 0.96 of one launch's time: 0.89 .. 0.99 (us, 4096 -> 2 x 11008 at 2047 rows 336 and 324, at 1720 317 and
+// 302; 8192 -> 2 x 28672 at 430 rows 442 and 395, at 1965 1607 and 1564).
+static int gemm_swiglu_split(const MatmulParams &w, int pieces, int steps) {
+    auto rounds = [&](int units) { return ((units + 7) / 8 * w.mblocks + 31) / 32; };
+    auto us = [&](const RowsCost &c) { return (float)steps * (c.step + c.per_rows * w.block_rows / GEMM_BM) + c.around; };
+    const float wide = us(ROWS_384), narrow = us(ROWS_256);
+    float least = 0.97f * rounds(w.units) * wide;
+    int first = 0;
+    for (int units = 8; units < w.units; units += 8) {
+        const float t = rounds(units) * wide + rounds((pieces - 3 * units + 1) / 2) * narrow;
+        if (t < least) {
+            least = t;
+            first = units;
+        }
+    }
+    return first;
+}
+
 int gemm_swiglu_rows_launch(MatmulParams p, hipStream_t stream) {
     // (blocks of 64 .. 128 rows)
     static const gemm_kernel_t plain[5] = {q40_gemm_kernel<4, false, true, 8, GEMM_STAGES, false, false, true>, q40_gemm_kernel<5, false, true, 8, GEMM_STAGES, false, false, true>, q40_gemm_kernel<6, false, true, 8, GEMM_STAGES, false, false, true>,
@@ -1678,9 +1699,22 @@ int gemm_swiglu_rows_launch(MatmulParams p, hipStream_t stream) {
     p.kgroups = 0;
     MatmulParams w = p;
     if (gemm_swiglu_rows_plan(p, w)) {
-        const int t = w.block_rows / 16 - 4;
+        const int t = w.block_rows / 16 - 4, pieces = p.seg[0].N / 64, first = gemm_swiglu_split(w, pieces, p.K / 32);
         w.ksplit = 1;
-        return gemm_launch_rows(wide[t], w, 64 * (WIDE_WAVES + GEMM_DMA_WAVES), wide_lds[t], stream);
+        if (first > 0) w.units = w.units_pad = first;
+        const int st = gemm_launch_rows(wide[t], w, 64 * (WIDE_WAVES + GEMM_DMA_WAVES), wide_lds[t], stream);
+        if (st || first == 0) return st;
+        // the columns behind the first launch's: 3 pieces a unit, a multiple of 12 blocks of 128
+        const int blocks = 3 * first / 2;
+        for (int i = 0; i < 2; ++i) {
+            p.seg[i].w += (long)(blocks / 2) * tiled_steps(p.K) * TILE_BYTES;
+            p.seg[i].N -= 128 * blocks;
+        }
+        p.seg[0].c += 128 * blocks;
+        p.units = p.seg[0].N / 128;
+        p.units_pad = (p.units + 7) / 8 * 8;
+        p.mblocks = w.mblocks;
+        p.block_rows = w.block_rows;
     }
     const bool one_each = (long)p.units * p.mblocks <= GEMM_DMA_WAVE_MAX_WGS;
     const int t = p.block_rows / 16 - 4;

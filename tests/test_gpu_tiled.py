@@ -373,3 +373,25 @@ def test_wide_workgroups(M, K, ns, columns):
         assert torch.allclose(o.cpu().float(), want, rtol=2e-3, atol=2e-3)
         if r is not None:
             assert torch.equal(o_r.cpu(), (r.float() + o.cpu().float()).half())
+
+
+@pytest.mark.parametrize("M,K,n_half", [(430, 256, 18560), (512, 128, 28672), (500, 1056, 18560), (866, 512, 14336)])
+def test_swiglu_in_two_launches_where_the_last_round_is_a_poor_one(M, K, n_half):
+    """Workgroups of three pieces of each weight for most columns, of two for the rest: what one weight's columns after the other give in 64 bits, to the
+    roundings of fp16 products, silu and their product; outputs in rows of a larger tensor, whose other columns stay"""
+    from spec_mcts_amd import _lib, kernels as Kn
+    g = torch.Generator(device="cuda").manual_seed(M)
+    ws = [Kn.quantize_q40(torch.randn((K, n_half), device="cuda", generator=g, dtype=torch.float16) * 0.1) for _ in range(2)]
+    tiled = [Kn.tile_q40(w, s, K, n_half) for w, s in ws]
+    x = torch.randn((M, K), device="cuda", generator=g, dtype=torch.float16)
+    assert _lib.load().smh_q40_swiglu_columns(M, K, n_half) == 384
+    wide = torch.full((M, n_half + 4), 7.0, device="cuda", dtype=torch.float16)
+    Kn.check(_lib.load().smh_q40_matmul_tiled_swiglu(x.data_ptr(), M, K, K, tiled[0].buf.data_ptr(), tiled[1].buf.data_ptr(), n_half, wide.data_ptr(), n_half + 4,
+                                                     Kn._stream()), "smh_q40_matmul_tiled_swiglu")
+    got = wide[:, :n_half]
+    assert torch.equal(got, Kn.matmul_q40_swiglu(x, *tiled)) and bool((wide[:, n_half:] == 7).all())
+    gate, up = (x.double() @ Kn.deq_int40(w, s, 64, (K, n_half)).double() for w, s in ws)
+    want = torch.nn.functional.silu(gate) * up
+    # a factor of half an fp16 unit for either product (the gate's through silu, whose derivative is at most 1.1), for silu and for their product
+    err = (0.5 * (1.1 * gate.abs() * up.abs() + 3 * want.abs()) + gate.abs() * up.abs() * 2.0 ** -10) * 2.0 ** -10 + 2.0 ** -20 * (gate.abs().max() + up.abs().max())
+    assert bool(((got.double() - want).abs() <= err).all())
