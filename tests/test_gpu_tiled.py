@@ -395,3 +395,22 @@ def test_swiglu_in_two_launches_where_the_last_round_is_a_poor_one(M, K, n_half)
     # a factor of half an fp16 unit for either product (the gate's through silu, whose derivative is at most 1.1), for silu and for their product
     err = (0.5 * (1.1 * gate.abs() * up.abs() + 3 * want.abs()) + gate.abs() * up.abs() * 2.0 ** -10) * 2.0 ** -10 + 2.0 ** -20 * (gate.abs().max() + up.abs().max())
     assert bool(((got.double() - want).abs() <= err).all())
+
+
+@pytest.mark.parametrize("M,K,ns,slabs", [(161, 4096, [4096], 4), (234, 4096, [4096], 2), (512, 4096, [4096], 2), (197, 11008, [4096], 4), (526, 4096, [2048], 3),
+                                          (175, 4096, [2048, 256, 1792], 4), (220, 8192, [3072], 4), (200, 2112, [4096], 2)])
+def test_two_k_groups_above_160_rows(M, K, ns, slabs):
+    """row blocks of 96 to 128 rows on two K-groups a workgroup: the slab count, every element of the slabs written, and their sum as close to 64 bits as the
+    fp32 sums and one rounding to fp16 leave it; several weights, odd numbers of blocks, a last block of few rows, a last slice that is shorter"""
+    from spec_mcts_amd import kernels as Kn
+    assert Kn.matmul_plan(M, K, ns, tiled=True) == slabs
+    g = torch.Generator(device="cuda").manual_seed(M)
+    ws = [Kn.quantize_q40(torch.randn((K, n), device="cuda", generator=g, dtype=torch.float16) * 0.02) for n in ns]
+    a = torch.randn((M, K), device="cuda", generator=g, dtype=torch.float16)
+    size = slabs * M * sum(ns)
+    out = torch.full((size + 64,), float("nan"), dtype=torch.float32, device="cuda")
+    p = Kn.matmul_q40_partial(a, [Kn.tile_q40(w, s, K, n) for (w, s), n in zip(ws, ns)], out)
+    assert p.ksplit == slabs and not bool(out[:size].isnan().any()) and bool(out[size:].isnan().all())
+    got = Kn.partial_reduce(p).double()
+    want = torch.cat([a.double() @ Kn.deq_int40(w, s, 64, (K, n)).double() for (w, s), n in zip(ws, ns)], 1)
+    assert bool(((got - want).abs() <= want.abs() * 2.0 ** -11 + 2.0 ** -24 * K ** 0.5 * want.abs().max()).all())
