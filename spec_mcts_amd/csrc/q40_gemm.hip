@@ -1422,8 +1422,8 @@ void gemm_fill_plan(MatmulParams &p) {
         // and 29.5); of 86 stages 0.98 and 1.00 (300 and 512 x 4096 x 11008), of one slice 0.81 .. 1.02.  Up to 160 rows (20.4 and 16.6 at 144 x 4096 x 4096) slabs
         // keep the checkpoint layout's bits.
         if (p.tiled && p.M > 160 && p.ksplit > 1 && p.K % 64 == 0 && p.K <= 16384) {
-            const int blocks = p.n_total / 128, on_xcd = p.units_pad / 4 * p.mblocks;
-            const int ks = min(min(256 / (blocks * p.mblocks), 32 / on_xcd), p.ksplit), sps = ks > 0 ? ((steps + ks - 1) / ks + 1) / 2 * 2 : 0;
+            const long blocks = p.n_total / 128, on_xcd = (long)p.units_pad / 4 * p.mblocks;
+            const int ks = (int)min(min(256 / (blocks * p.mblocks), 32 / on_xcd), (long)p.ksplit), sps = ks > 0 ? ((steps + ks - 1) / ks + 1) / 2 * 2 : 0;
             if (ks >= 2 && blocks * p.mblocks * ks >= 170 && sps <= 96) {
                 p.kgroups = 2;
                 p.steps_per_slice = sps;
@@ -1552,7 +1552,7 @@ static int gemm_launch_layout(const MatmulParams &p, hipStream_t stream) {
     return gemm_launch_rows(kern, p, threads, lds, stream);
 }
 
-// The checkpoint layout's plan for q40_gemm_kg_kernel in the place of p's: one weight, 17 .. 128 rows, never more slabs than p's (whose workspace holds
+// The checkpoint layout's plan for q40_gemm_kg_kernel in the place of p's: one weight, 17 rows and more, never more slabs than p's (whose workspace holds
 // them), none where a workgroup has all of K.
 // It has half the slabs for as many workgroups, or one workgroup a compute unit where p has two of half the waves, but fetches half a line of weights
 // and as many lines of scales for half the columns: per 64 rows of K it takes 0.15 us more than two steps of the 256-column units, and up to 20 % more where
@@ -1561,23 +1561,28 @@ static int gemm_launch_layout(const MatmulParams &p, hipStream_t stream) {
 //   * where p has one workgroup a compute unit: up to 20 stages (64 rows of K each) a workgroup, above 64 rows 24: 48 shapes 1.02 .. 1.41 times
 //     (above that 0.76 .. 1.07: 37 x 4096 x 11008, 22 stages, 17.1 us and 18.0, 100 x 12288 x 4096, 32 stages, 26.0 and 28.3);
 //   * where p's are more, or cut at runs of steps: up to 48 stages, above 64 rows 64: 10 shapes 1.05 .. 1.64 (20 x 24576 x 4096, 64 stages, 26.1 us and
-//     32.0; 80 x 22400 x 15208 109.6 and 133).
+//     32.0; 80 x 22400 x 15208 109.6 and 133);
+//   * above 128 rows, on p's row blocks, where K is cut and half the compute units get work: up to 40 stages, 46 shapes of 130 .. 512 rows 1.02 .. 1.52 times
+//     (us, 512 x 4096 x 4096 32.1 and 28.3, 300 rows 24.1 and 22.0, 242 x 5888 x 1176 20.4 and 13.4; of 41 to 45 stages 0.99 .. 1.07, of 86 0.91 and 0.92, of 191 0.81).
 // us of both launches, in turn: 100 x 4096 x 4096 18.8 and 15.5, 20 x 4096 x 4096 11.4 and 9.8, 100 x 5120 x 5120 28.5 and 17.9, 37 x 7168 x 7168 26.2 and
 // 19.1, 100 x 6400 x 3000 26.7 and 18.5, 100 x 24064 x 1928 35.3 and 24.7.
 bool gemm_blocks_fit(const MatmulParams &p, MatmulParams &b) {
     // (half a stage past a K that is a multiple of 32 would meet an infinite activation with a zero)
-    if (p.tiled || p.nseg != 1 || p.M <= SMH_GEMV_MAX_M || p.M > GEMM_BM || p.K > 16384 || p.K % 64 == 32) return false;
-    const int blocks = p.seg[0].N / 128, mblocks = blocks <= 32 && p.M > 64 && p.K <= 4096 ? 2 : 1, steps = (p.K + 31) / 32;
+    if (p.tiled || p.nseg != 1 || p.M <= SMH_GEMV_MAX_M || p.K > 16384 || p.K % 64 == 32) return false;
+    const bool many = p.M > GEMM_BM;
+    const int blocks = p.seg[0].N / 128, mblocks = many ? p.mblocks : blocks <= 32 && p.M > 64 && p.K <= 4096 ? 2 : 1, steps = (p.K + 31) / 32;
+    if ((long)blocks * mblocks > 256) return false;
     const int on_xcd = p.units_pad / 4 * mblocks;              // workgroups of a K-slice on the busiest XCD
     const int ks = min(min(256 / (blocks * mblocks), 32 / on_xcd), min(p.ksplit, steps / 8));
-    if (ks < 1 || blocks * mblocks * ks < 170) return false;
+    if (ks < 1 || blocks * mblocks * ks < (many ? 128 : 170)) return false;
     b = p;
     b.kgroups = 2;
     b.mblocks = mblocks;
-    b.block_rows = mblocks == 2 ? 64 : GEMM_BM;
+    if (!many) b.block_rows = mblocks == 2 ? 64 : GEMM_BM;
     b.chunk = 0;
     b.steps_per_slice = ((steps + ks - 1) / ks + 1) / 2 * 2;   // a stage of the ring is two steps
     b.ksplit = (steps + b.steps_per_slice - 1) / b.steps_per_slice;
+    if (many) return b.steps_per_slice <= 80;
     const bool one_round = p.chunk == 0 && (long)p.units * p.mblocks * p.ksplit <= 256;
     if (one_round && p.units_pad / 8 * p.mblocks * p.ksplit > 32) return true;
     return b.steps_per_slice / 2 <= (one_round ? (p.M <= 64 ? 20 : 24) : (p.M <= 64 ? 48 : 64));

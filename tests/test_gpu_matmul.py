@@ -325,7 +325,7 @@ def test_checkpoint_products_at_the_end_of_k(M, K, N):
     assert bool(((got - want).abs() <= want.abs() * 2.0 ** -11 + 2.0 ** -24 * K ** 0.5 * want.abs().max()).all())
 
 
-@pytest.mark.parametrize("M", [17, 48, 64, 65, 97, 128])
+@pytest.mark.parametrize("M", [17, 48, 64, 65, 97, 128, 129, 200, 273, 512])
 @pytest.mark.parametrize("K,N", [(4096, 4096), (4104, 3840), (1928, 24064), (3000, 6400), (2072, 5760), (7168, 7168), (1496, 21760), (1024, 2944)])
 def test_checkpoint_products_in_blocks_of_128_columns(M, K, N):
     """Launches of 128-column blocks with two K-groups a workgroup: edges of the row tiles and of the two row blocks, odd numbers of blocks, K that ends in
