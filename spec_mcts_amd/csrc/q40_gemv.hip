@@ -136,11 +136,14 @@ struct GemvConsts {
 // fp16(code * scale) (fp16_to_int4.py:90-96) - three packed instructions per two weights - which enters the matrix core as
 // the B operand (lane = column, 8 consecutive k per lane) against the unscaled activations: the products the reference's
 // kernel forms (triton_kernels.py:444-449), accumulated in fp32.
+// FLIP: the nibbles are the checkpoint's two's complement ones, and the magic numbers hold the bits that make u of them (one three-operand instruction, too).
+template <bool FLIP>
 __device__ __forceinline__ uint32_t gemv_weights_high(uint32_t pr, h2 scale, const GemvConsts &C) {
-    return as_u32((as_h2((pr & C.mask_hi) | C.magic_hi) + C.off_hi) * scale);
+    return as_u32((as_h2(FLIP ? (pr & C.mask_hi) ^ C.magic_hi : (pr & C.mask_hi) | C.magic_hi) + C.off_hi) * scale);
 }
+template <bool FLIP>
 __device__ __forceinline__ uint32_t gemv_weights_low(uint32_t pr, h2 scale, const GemvConsts &C) {
-    return as_u32((as_h2((pr & C.mask_lo) | C.magic_lo) + C.off_lo) * scale);
+    return as_u32((as_h2(FLIP ? (pr & C.mask_lo) ^ C.magic_lo : (pr & C.mask_lo) | C.magic_lo) + C.off_lo) * scale);
 }
 
 // acc[blk][h][b]: column 128*blk + 64*h + 4c + b.
@@ -150,8 +153,8 @@ __device__ __forceinline__ void gemv_consume(const uint8_t *stage, int k0, int K
     uint32_t u0[8], u1[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        u0[i] = *reinterpret_cast<const uint32_t *>(stage + (8 * g + i) * 128 + 4 * c) ^ NIBBLE_FLIP;
-        u1[i] = *reinterpret_cast<const uint32_t *>(stage + (8 * g + i) * 128 + 64 + 4 * c) ^ NIBBLE_FLIP;
+        u0[i] = *reinterpret_cast<const uint32_t *>(stage + (8 * g + i) * 128 + 4 * c);
+        u1[i] = *reinterpret_cast<const uint32_t *>(stage + (8 * g + i) * 128 + 64 + 4 * c);
     }
     h8 xv = *reinterpret_cast<const h8 *>(stage + STAGE_W_BYTES + STAGE_S_BYTES + c * 64 + 16 * g);
     if constexpr (RAGGED) {
@@ -178,8 +181,8 @@ __device__ __forceinline__ void gemv_consume(const uint8_t *stage, int k0, int K
         u32x4 vh, vl;                                                                            \
         _Pragma("unroll") for (int j = 0; j < 4; ++j) {                                          \
             const uint32_t pr = pair_bytes<B>(U[2 * j], U[2 * j + 1]);                           \
-            vh[j] = gemv_weights_high(pr, sc[BLK][0][j], C);                                     \
-            vl[j] = gemv_weights_low(pr, sc[BLK][1][j], C);                                      \
+            vh[j] = gemv_weights_high<true>(pr, sc[BLK][0][j], C);                                     \
+            vl[j] = gemv_weights_low<true>(pr, sc[BLK][1][j], C);                                      \
         }                                                                                        \
         acc[BLK][0][B] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv, __builtin_bit_cast(h8, vh), acc[BLK][0][B], 0, 0, 0);     \
         acc[BLK][1][B] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv, __builtin_bit_cast(h8, vl), acc[BLK][1][B], 0, 0, 0);     \
@@ -228,8 +231,8 @@ __device__ __forceinline__ void gemv_consume_tiled(const uint8_t *stage, int k0,
             u32x4 vh, vl;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                vh[j] = gemv_weights_high(pr[j], as_h2(sc[2 * blk][j]), C);
-                vl[j] = gemv_weights_low(pr[j], as_h2(sc[2 * blk + 1][j]), C);
+                vh[j] = gemv_weights_high<false>(pr[j], as_h2(sc[2 * blk][j]), C);
+                vl[j] = gemv_weights_low<false>(pr[j], as_h2(sc[2 * blk + 1][j]), C);
             }
             acc[blk][0][B] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv, __builtin_bit_cast(h8, vh), acc[blk][0][B], 0, 0, 0);
             acc[blk][1][B] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv, __builtin_bit_cast(h8, vl), acc[blk][1][B], 0, 0, 0);
@@ -298,7 +301,7 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void q40_gemv_kernel(MatmulParams 
     }
     uint8_t *ring = lds + wave * RING;
 
-    GemvConsts C{0x00F000F0u, 0x000F000Fu, 0x54005400u, 0x64006400u, h2{(half_t)-72.f, (half_t)-72.f}, h2{(half_t)-1032.f, (half_t)-1032.f}};
+    GemvConsts C{0x00F000F0u, 0x000F000Fu, TILED ? 0x54005400u : 0x54805480u, TILED ? 0x64006400u : 0x64086408u, h2{(half_t)-72.f, (half_t)-72.f}, h2{(half_t)-1032.f, (half_t)-1032.f}};
     asm volatile("" : "+s"(C.mask_hi), "+s"(C.mask_lo));
     asm volatile("" : "+v"(C.magic_hi), "+v"(C.magic_lo));
 
