@@ -29,7 +29,8 @@
 // a workgroup that has waited too long publishes nothing more and leaves NaN in its part of the result.
 //
 // A step of the 7B architecture (512 prompt rows and 63 of their own), layer by layer and in one launch, in us: 1 branch 1981 and
-// 1451, 2 branches 2100 and 1590, 3 branches 2134 and 1872, 4 branches 2161 and 2094 (after 2047 and 127 rows 3057 and 2585).  What a branch adds is the communication:
+// 1451, 2 branches 2100 and 1590, 3 branches 2134 and 1872, 4 branches 2161 and 2094 (after 2047 and 127 rows 3057 and 2585), all of it before
+// pieces were decoded ahead (Multiplier).  What a branch adds is the communication:
 // its activations go through every workgroup.  So four is where the rule of the sizes (stack_plan) ends.
 #include "attn_rows.hpp"
 #include "q40_matmul.hpp"

@@ -128,7 +128,7 @@ def tile_q40(w: torch.Tensor, s: torch.Tensor, K: int, N: int) -> TiledQ40:
 
 def matmul_q40_partial(a: torch.Tensor, linears, out: Optional[torch.Tensor] = None) -> PartialProduct:
     """One launch for up to 3 Q4_0 weights that share the input a [M,K]; `linears` is a sequence of
-    (w, s, N), or of TiledQ40 (same slabs, bit for bit).  Leaves the un-reduced product; the columns of the
+    (w, s, N), or of TiledQ40 (same slabs, bit for bit, where both have the same plan: matmul_plan).  Leaves the un-reduced product; the columns of the
     weights are concatenated."""
     import ctypes
     lib = _lib.load()
