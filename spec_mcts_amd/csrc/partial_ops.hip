@@ -585,7 +585,10 @@ static int matmul_fp16(const void *a, int M, int K, long lda, const void *b_w, c
     MatmulParams b;
     if (gemm && gemm_blocks_fit(p, b)) {
         p = b;
-        p.direct = p.ksplit == 1 && ldc % 4 == 0 ? 1 : 0;
+        // (a result written over its own activations needs the second launch that p's slabs would have given it)
+        const char *a0 = (const char *)a, *c0 = (const char *)c;
+        const bool apart = c0 + ((long)(M - 1) * ldc + N) * sizeof(half_t) <= a0 || a0 + ((long)(M - 1) * lda + K) * sizeof(half_t) <= c0;
+        p.direct = p.ksplit == 1 && ldc % 4 == 0 && apart ? 1 : 0;
         if (p.direct) return gemm_launch(p, (hipStream_t)stream);
     }
     st = gemm ? gemm_launch(p, (hipStream_t)stream) : gemv_launch(p, (hipStream_t)stream);

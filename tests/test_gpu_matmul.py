@@ -325,6 +325,19 @@ def test_checkpoint_products_at_the_end_of_k(M, K, N):
     assert bool(((got - want).abs() <= want.abs() * 2.0 ** -11 + 2.0 ** -24 * K ** 0.5 * want.abs().max()).all())
 
 
+@pytest.mark.parametrize("M,K", [(1040, 2048), (900, 1536), (300, 4096)])
+def test_checkpoint_product_over_its_own_activations(M, K):
+    """A product whose K is cut reads all of its activations before the launch that writes the result, so the result may take their place: also where the
+    plan's two slices become one slice of 128-column blocks, which would be stored without slabs.  The same bits as apart"""
+    from spec_mcts_amd import kernels as Kn
+    assert Kn.matmul_plan(M, K, [K]) > 1
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    w, s = Kn.quantize_q40(torch.randn((K, K), device="cuda", generator=g, dtype=torch.float16) * 0.02)
+    x = torch.randn((M, K), device="cuda", generator=g, dtype=torch.float16)
+    apart = Kn.matmul_q40(x, w, s, (K, K))
+    assert torch.equal(Kn.matmul_q40(x, w, s, (K, K), out=x), apart)
+
+
 @pytest.mark.parametrize("M", [17, 48, 64, 65, 97, 128, 129, 200, 273, 512])
 @pytest.mark.parametrize("K,N", [(4096, 4096), (4104, 3840), (1928, 24064), (3000, 6400), (2072, 5760), (7168, 7168), (1496, 21760), (1024, 2944)])
 def test_checkpoint_products_in_blocks_of_128_columns(M, K, N):
