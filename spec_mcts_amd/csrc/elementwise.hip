@@ -243,6 +243,9 @@ namespace smh {
 // CDF with the caller's uniform number.
 constexpr int SAMPLE_MAX_K = 1024;
 constexpr int SAMPLE_HOT_MAX = 576;            // threads whose logits are looked at again
+// Up to here the bound is guessed from sixteenths of the maxima.  The guess takes k / 14 steps and saves three rounds.  80 rows of 32016, us, without and with
+// one: k = 32 7.2 and 6.8, 65 9.0 and 8.8, 96 9.4 and 9.5.
+constexpr int SAMPLE_GUESS_MAX_K = 80;
 constexpr int SAMPLE_PICK_MAX_K = 512;         // up to here the candidates are picked by the threads' maxima (above, they would be thousands)
 
 __device__ __forceinline__ uint32_t sample_key(half_t x) {
@@ -259,6 +262,21 @@ __device__ __forceinline__ uint32_t sample_keys2(uint32_t b) {
 __device__ __forceinline__ half_t sample_unkey(uint32_t k) {
     const uint16_t b = (uint16_t)((k & 0x8000u) ? (k & 0x7FFFu) : (~k & 0xFFFFu));
     return __builtin_bit_cast(half_t, b);
+}
+
+// the largest value of a lane's row of sixteen lanes (in all of them), and of the wave
+__device__ __forceinline__ uint32_t row16_max_bits(uint32_t v) {
+    auto move = [&](auto ctrl) { v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, 0xf, 0xf, false)); };
+    move(std::integral_constant<int, DPP_QUAD_XOR1>{});
+    move(std::integral_constant<int, DPP_QUAD_XOR2>{});
+    move(std::integral_constant<int, DPP_ROW_HALF_MIRROR>{});
+    move(std::integral_constant<int, DPP_ROW_ROR8>{});
+    return v;
+}
+__device__ __forceinline__ uint32_t wave_max_bits(uint32_t v) {
+    const int r = (int)row16_max_bits(v);
+    auto of = [&](int lane) { return (uint32_t)__builtin_amdgcn_readlane(r, lane); };
+    return max(max(of(0), of(16)), max(of(32), of(48)));
 }
 
 // Inclusive prefix sums over the 1024 threads of the workgroup (thread order): inside a wave by lane shifts, across waves
@@ -296,8 +314,9 @@ __device__ __forceinline__ void sample_pick_bin(int *bins, int *s_w, int want, i
 // counts == nullptr: one draw per row, uniform[row] -> out[row].  Otherwise row r makes counts[r] draws with replacement from
 // its candidates, with the uniform numbers (and into the slots of out) that start at counts[0] + ... + counts[r-1].
 // Up to 32768 logits (a multiple of 8, rows 16-byte aligned) and k <= 512 the row is read once into registers and the candidates
-// are those not below the k-th largest of the threads' maxima (a handful more than k): no histogram of the whole row, whose LDS
-// atomics pile up on the few bins that logits fall into.  80 rows of 32016, k = 32: 35 us with histograms, 7.9 like this.
+// are those not below a bound that about k of the threads' maxima reach (a handful more than k): no histogram of the whole row, whose LDS
+// atomics pile up on the few bins that logits fall into.  80 rows of 32016, k = 32: 35 us with histograms, 7.2 with the k-th largest maximum, four bits at
+// a time, and 6.8 with a bound guessed in one round (k = 1, 16 rows: 6.5 and 5.7; k = 512, 31 and 26, by the ranking's shares).
 // Bound by its instructions (sixteen waves on a compute unit: 18 cycles each for all of them) and a chain of barriers.  So keys are made and
 // compared two to an instruction, only the few threads whose maximum reaches the bound hand their logits out, one to a thread, instead
 // of every wave looking through 32 (12.3 us with that), and what the draws need is on its way from the start.
@@ -397,18 +416,55 @@ __global__ __launch_bounds__(1024) void sample_topk_kernel(const half_t *__restr
 #pragma unroll
             for (int e = 0; e < 4; ++e) mine[4 * j + e] = v[e];
         }
-        uint32_t thr = 0;
-#pragma unroll
-        for (int shift = 12; shift >= 0; shift -= 4) {         // ... and counts those at or above one value of the next four bits
-            const uint32_t t = thr | ((uint32_t)wv << shift);
+        // A bound that at least k maxima reach: thr, where fewer than k reach over.  It need not be the k-th largest, as long as only a few threads more reach it.
+        auto reach = [&](uint32_t t) {
             int n = 0;
 #pragma unroll
             for (int j = 0; j < 16; ++j) n += __popcll(__ballot(mine[j] >= t));
-            int *slot = bins + 16 * (shift >> 2);
-            if (lane == 0) slot[wv] = n;
+            return n;
+        };
+        const int wave = __builtin_amdgcn_readfirstlane(wv);
+        int *slot = bins;
+        uint32_t thr = 0;
+        if (k <= SAMPLE_GUESS_MAX_K) {
+            // Sixteen guesses: each wave's r-th largest of a sixteenth of the maxima, r a third above k / 16 or more, of which k to k + 32 maxima reach one in
+            // two or three (unordered logits: 600 of 600 rows needed no further round).
+            uint32_t v = maxima[16 * lane + ((wave + (lane >> 2)) & 15)], t = 0, over = 0x10000u;
+            for (int r = k / 14; r >= 0; --r) {
+                t = wave_max_bits(v);
+                if (lane == __builtin_ctzll(__ballot(v == t))) v = 0u;
+            }
+            const int n = reach(t);
+            if (lane == 0) slot[wave] = (int)(t << 11 | (uint32_t)n);
             __syncthreads();
-            // (the counts fall from wave to wave, and the first one's reaches k)
-            thr |= (uint32_t)(__popcll(__ballot(slot[lane & 15] >= k) & 0xFFFFull) - 1) << shift;
+            const uint32_t g = (uint32_t)slot[lane & 15], at = g & 2047u;
+            const uint32_t best = __builtin_amdgcn_readfirstlane(row16_max_bits(at >= (uint32_t)k ? g : 0u));         // the highest that k reach
+            int reached = 1024;
+            if (best != 0) { thr = best >> 11; reached = (int)(best & 2047u); }
+            over -= __builtin_amdgcn_readfirstlane(row16_max_bits(at < (uint32_t)k ? 0x10000u - (g >> 11) : 0u));      // the lowest that fewer do
+            while (over - thr > 1 && reached > k + 32) {       // every wave counts at one of sixteen values between the two
+                slot += 16;
+                const uint32_t step = (over - thr + 14) >> 4;
+                const int m = reach(min(thr + 1 + (uint32_t)wave * step, over));
+                if (lane == 0) slot[wave] = m;
+                __syncthreads();
+                const int now = slot[lane & 15], most = __popcll(__ballot(now >= k) & 0xFFFFull);      // (the counts fall from wave to wave)
+                over = min(thr + 1 + (uint32_t)most * step, over);
+                if (most > 0) {
+                    reached = __builtin_amdgcn_readlane(now, most - 1);
+                    thr += 1 + (uint32_t)(most - 1) * step;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int shift = 12; shift >= 0; shift -= 4) {     // every wave counts at one value of the next four bits
+                const int n = reach(thr | ((uint32_t)wave << shift));
+                if (lane == 0) slot[wave] = n;
+                __syncthreads();
+                // (the counts fall from wave to wave, and the first one's reaches k)
+                thr |= (uint32_t)(__popcll(__ballot(slot[lane & 15] >= k) & 0xFFFFull) - 1) << shift;
+                slot += 16;
+            }
         }
         bool small = true;
         if (!wide) {                           // (one candidate a lane: thr - lane)
@@ -452,17 +508,22 @@ __global__ __launch_bounds__(1024) void sample_topk_kernel(const half_t *__restr
             __syncthreads();
             const int count = s_count;
             if (count <= SAMPLE_MAX_K) {
-                // rank = number of candidates that come before.  1024 / (count, rounded up to a power of two) threads share a
-                // candidate, each comparing it with every so-many-th quad of the others (the same for all lanes of a wave).
-                int pow2 = 64;
-                while (pow2 < count) pow2 <<= 1;
-                const int cand = tid & (pow2 - 1), part = tid / pow2, parts = 1024 / pow2;
+                // rank = number of candidates that come before.  `parts` waves share 64 candidates, each comparing them with every
+                // so-many-th quad of the others (the same for all lanes of a wave).
+                int part = wave, parts = 16, cand = lane;
+                if (count > 64) {
+                    const int groups = (__builtin_amdgcn_readfirstlane(count) + 63) >> 6;
+                    const int inv = __builtin_amdgcn_readfirstlane((int)(65536.0f * __builtin_amdgcn_rcpf((float)groups))) + 1;
+                    part = (wave * inv) >> 16;                 // wave / groups (both at most 16)
+                    parts = (16 * inv) >> 16;
+                    cand += 64 * (wave - part * groups);
+                }
                 const uint32_t mine_c = cand < count ? c_key[cand] : 0u;
                 if (tid < 1024 - count) c_key[count + tid] = 0u;           // (below every candidate)
                 c_idx[tid] = 0;
                 __syncthreads();
                 int rank = 0;
-                for (int j = 4 * part; j < count; j += 4 * parts) {
+                for (int j = 4 * part; j < count && part < parts; j += 4 * parts) {
                     const u32x4 v = *reinterpret_cast<const u32x4 *>(&c_key[j]);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) rank += v[e] > mine_c;

@@ -155,6 +155,41 @@ def test_sample_topk_ties_take_the_lowest_indices_and_frequencies_follow_p():
         assert abs(freq - pj) < 4 * (pj * (1 - pj) / n) ** 0.5 + 1e-3
 
 
+@pytest.mark.parametrize("k", [1, 13, 14, 32, 64, 79, 80, 81])
+@pytest.mark.parametrize("kind", ["one_sixteenth", "levels", "masked", "plain"])
+def test_sample_topk_whatever_its_guesses_of_the_bound_are(k, kind):
+    """Up to k = 80 the bound of the threads' maxima is guessed from sixteenths of them (thread 16 l + ((w + l / 4) mod 16) is in sixteenth w): rows whose
+    largest values all sit in one of these, rows of a few values (a guess that k threads reach is reached by hundreds), rows that are masked but for 40"""
+    from spec_mcts_amd import kernels as K
+    g = torch.Generator().manual_seed(100 + k)
+    rows, vocab, per = 5, 32016, 40
+    logits = torch.randn((rows, vocab), generator=g) * 2
+    if kind == "one_sixteenth":
+        for r in range(rows):
+            l = torch.arange(64)
+            logits[r, 8 * (16 * l + (((3 * r) % 16 + l // 4) % 16))] = 9 + torch.rand(64, generator=g) * 4
+    elif kind == "levels":
+        logits = (logits / 2).round()
+    elif kind == "masked":
+        kept = torch.full_like(logits, float("-inf"))
+        for r in range(rows):
+            at = torch.randperm(vocab, generator=g)[:40]
+            kept[r, at] = logits[r, at]
+        logits = kept
+    logits = logits.half()
+    counts = torch.full((rows,), per, dtype=torch.int32)
+    u = torch.rand(rows * per, generator=g)
+    p, idx = O.topk_probs(logits, 0.8, k)
+    cdf = p.float().cumsum(-1)
+    got = K.sample_topk_counts(logits.cuda(), 0.8, k, counts.cuda(), u.cuda()).cpu()
+    want = O.sample_topk_counts(logits, 0.8, k, counts.tolist(), u)
+    for i in (got != want).nonzero().flatten().tolist():         # only where the number falls on a step (as above)
+        r, pos = i // per, (idx[i // per] == int(got[i])).nonzero()
+        assert len(pos) == 1, f"draw {i}: token {int(got[i])} is not a candidate"
+        j, target = int(pos[0]), float(u[i]) * float(cdf[r, -1])
+        assert min(abs(e - target) for e in (float(cdf[r, j - 1]) if j else 0.0, float(cdf[r, j]))) < 1e-5, f"draw {i}"
+
+
 @pytest.mark.parametrize("k", [1, 32, 512])
 @pytest.mark.parametrize("hot", [1, 40, 575, 576, 577, 1000])
 @pytest.mark.parametrize("temperature", [0.7, 3000.0])
