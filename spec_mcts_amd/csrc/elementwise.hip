@@ -279,6 +279,16 @@ __device__ __forceinline__ uint32_t wave_max_bits(uint32_t v) {
     return max(max(of(0), of(16)), max(of(32), of(48)));
 }
 
+// Inclusive prefix sum over the wave (lane order) without LDS: within rows of sixteen lanes, then a row's last lane to the next row, then lane 31 to the upper half
+__device__ __forceinline__ int wave_prefix_sum(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);        // lane i - 1, - 2, - 4, - 8 of the row
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);        // rows 1 and 3
+    return v + __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // rows 2 and 3
+}
+
 // Inclusive prefix sums over the 1024 threads of the workgroup (thread order): inside a wave by lane shifts, across waves
 // through s_w[16]; two barriers.  Every thread of the workgroup must call.
 template <class T>
@@ -888,7 +898,8 @@ __global__ __launch_bounds__(256) void tree_fork_kernel(const int64_t *__restric
 // thread: a draw finds its rank among its branch's distinct tokens by comparing it with its branch's other draws (one, once the
 // tree has its full batch), the rows of the forks come from a prefix sum (a branch's first new row is c0 + the forks of the
 // branches before it, cut at the batch), and everything that depends on no other load is requested at the start.  At 80
-// branches: 28 us for tree_fork_kernel (whose first thread reads the counts and the live flags one behind the other), 4.4 here.
+// branches, us: 28 for tree_fork_kernel (whose first thread reads the counts and the live flags one behind the other), 3.9 where a draw searches for its
+// branch and the prefix sums go through LDS, 3.15 where a branch marks its draws and the sums stay in registers (256 branches: 4.2 and 3.5).
 constexpr int TREE_SMALL = 256;
 __global__ __launch_bounds__(TREE_SMALL) void tree_small_kernel(const int64_t *__restrict__ draws, int n_draws, int32_t *__restrict__ tok, int32_t *__restrict__ cnt,
                                                                 uint8_t *__restrict__ alive, int32_t *__restrict__ curr_b, int batch_size,
@@ -897,6 +908,7 @@ __global__ __launch_bounds__(TREE_SMALL) void tree_small_kernel(const int64_t *_
                                                                 int32_t *__restrict__ origin, const int32_t *__restrict__ t_dev, TreeFinish fin) {
     __shared__ uint32_t d_tok[TREE_SMALL];         // token of draw i
     __shared__ uint8_t d_head[TREE_SMALL];         // draw i is the first of its branch with its token
+    __shared__ uint8_t d_branch[TREE_SMALL];       // draw i's branch
     __shared__ int seg[TREE_SMALL + 1];            // first draw of branch i
     __shared__ int uniq[TREE_SMALL], row0[TREE_SMALL];
     __shared__ int r_tok[TREE_SMALL], r_cnt[TREE_SMALL], r_origin[TREE_SMALL];
@@ -905,11 +917,7 @@ __global__ __launch_bounds__(TREE_SMALL) void tree_small_kernel(const int64_t *_
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // inclusive prefix sum over the workgroup; every thread calls
     auto block_scan = [&](int v) {
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int u = __shfl_up(v, o, 64);
-            if (lane >= o) v += u;
-        }
+        v = wave_prefix_sum(v);
         if (lane == 63) s_w[wave] = v;
         __syncthreads();
         for (int w = 0; w < wave; ++w) v += s_w[w];
@@ -936,8 +944,9 @@ __global__ __launch_bounds__(TREE_SMALL) void tree_small_kernel(const int64_t *_
     r_set[tid] = 0;
     r_origin[tid] = -1;
     b_alive[tid] = was ? 1 : 0;
-    const int upto = block_scan(tid < c0 ? min(max(my_cnt, 0), TREE_MAX_BATCH) : 0);
+    const int own = tid < c0 ? min(max(my_cnt, 0), TREE_MAX_BATCH) : 0, upto = block_scan(own);
     seg[tid + 1] = upto;
+    for (int j = upto - own; j < min(upto, TREE_SMALL); ++j) d_branch[j] = (uint8_t)tid;
     if (tid == 0) seg[0] = 0;
     __syncthreads();
     const int total = min(seg[c0], n_draws);                     // draws the buffer does not hold do not exist
@@ -945,11 +954,7 @@ __global__ __launch_bounds__(TREE_SMALL) void tree_small_kernel(const int64_t *_
     int br = 0, lo = 0, hi = 0, mult = 0;
     bool head = tid < total;
     if (tid < total) {
-        int b1 = c0 - 1;
-        while (br < b1) {
-            const int mid = (br + b1 + 1) >> 1;
-            if (seg[mid] <= tid) br = mid; else b1 = mid - 1;
-        }
+        br = d_branch[tid];
         lo = min(seg[br], total);
         hi = min(seg[br + 1], total);
         for (int j = lo; j < hi; ++j) {

@@ -290,3 +290,28 @@ def test_tree_step_on_either_side_of_the_small_batch_kernel(B, huge):
     origin = K.tree_fork(draws.cuda(), d_oc, alive.cuda(), d_cur, d_res, t)
     assert int(d_cur) == want_cur and origin.cpu().tolist() == want_origin
     assert torch.equal(d_oc.cpu(), want_oc) and torch.equal(d_res.cpu(), want_res)
+
+
+@pytest.mark.parametrize("cur", [1, 15, 16, 17, 63, 64, 65, 128, 129])
+def test_tree_fork_of_branches_without_draws(cur):
+    """Branches with no draws or less than none between the others, at the edges of the rows and the waves of the prefix sums: the one kernel's draws go to
+    the branches that the other kernel (more than 256 rows) gives them to"""
+    from spec_mcts_amd import kernels as K
+    g = torch.Generator().manual_seed(cur)
+    cnt = torch.randint(-2, 4, (cur,), generator=g).to(torch.int32)
+    cnt[cur - 1] = 3
+    n = int(cnt.clamp(min=0).sum())
+    draws = torch.randint(0, 5, (n,), generator=g).cuda()
+    res = []
+    for B in (256, 300):
+        oc = torch.zeros((2, B), dtype=torch.int32)
+        oc[1, :cur] = cnt
+        results = torch.zeros((B, 6), dtype=torch.int64)
+        results[:cur] = torch.arange(cur * 6).view(cur, 6)
+        alive = torch.ones(B, dtype=torch.bool)
+        alive[cur // 2] = cur < 3
+        d_oc, d_res, d_cur = oc.cuda(), results.cuda(), torch.tensor([cur], dtype=torch.int32).cuda()
+        origin = K.tree_fork(draws, d_oc, alive.cuda(), d_cur, d_res, 2)
+        assert cur <= int(d_cur) <= 256
+        res.append((int(d_cur), origin.cpu()[:256], d_oc.cpu()[:, :256], d_res.cpu()[:256]))
+    assert res[0][0] == res[1][0] and all(torch.equal(a, b) for a, b in zip(res[0][1:], res[1][1:]))
