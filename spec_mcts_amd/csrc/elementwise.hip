@@ -244,7 +244,7 @@ namespace smh {
 constexpr int SAMPLE_MAX_K = 1024;
 constexpr int SAMPLE_HOT_MAX = 576;            // threads whose logits are looked at again
 // Up to here the bound is guessed from sixteenths of the maxima.  The guess takes k / 14 steps and saves three rounds.  80 rows of 32016, us, without and with
-// one: k = 32 7.2 and 6.8, 65 9.0 and 8.8, 96 9.4 and 9.5.
+// one: k = 32 7.2 and 6.8, 65 9.0 and 8.8, 96 9.4 and 9.6.
 constexpr int SAMPLE_GUESS_MAX_K = 80;
 constexpr int SAMPLE_PICK_MAX_K = 512;         // up to here the candidates are picked by the threads' maxima (above, they would be thousands)
 
@@ -326,7 +326,7 @@ __device__ __forceinline__ void sample_pick_bin(int *bins, int *s_w, int want, i
 // Up to 32768 logits (a multiple of 8, rows 16-byte aligned) and k <= 512 the row is read once into registers and the candidates
 // are those not below a bound that about k of the threads' maxima reach (a handful more than k): no histogram of the whole row, whose LDS
 // atomics pile up on the few bins that logits fall into.  80 rows of 32016, k = 32: 35 us with histograms, 7.2 with the k-th largest maximum, four bits at
-// a time, and 6.8 with a bound guessed in one round (k = 1, 16 rows: 6.5 and 5.7; k = 512, 31 and 26, by the ranking's shares).
+// a time, and 6.7 with a bound guessed in one round (k = 1, 16 rows: 6.5 and 5.6; k = 512, 31 and 26, by the ranking's shares).
 // Bound by its instructions (sixteen waves on a compute unit: 18 cycles each for all of them) and a chain of barriers.  So keys are made and
 // compared two to an instruction, only the few threads whose maximum reaches the bound hand their logits out, one to a thread, instead
 // of every wave looking through 32 (12.3 us with that), and what the draws need is on its way from the start.
@@ -372,6 +372,7 @@ __global__ __launch_bounds__(1024) void sample_topk_kernel(const half_t *__restr
     // One wave: which draws are this row's (the counts of the rows before it added up, all loads together) and the uniform numbers of the
     // first 64.  Every sum is cut at n_draws < 2^31 - counts that add up to more than the buffers hold are cut - so none of these
     // unsigned sums wraps.
+    float my_uniform = 0.f;                    // (left in s_uniform when it is there: waited for at once, it kept the others at their first barrier)
     auto find_draws = [&]() {
         int first = blockIdx.x, draws = 1;
         if (counts != nullptr) {
@@ -379,13 +380,18 @@ __global__ __launch_bounds__(1024) void sample_topk_kernel(const half_t *__restr
             uint32_t sum = 0;
             for (int r = lane; r < (int)blockIdx.x; r += 64) sum = min(sum + (uint32_t)max(counts[r], 0), most);
             const int own = counts[blockIdx.x];
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) sum = min(sum + (uint32_t)__shfl_xor((int)sum, o, 64), most);
+            auto add = [&](auto ctrl) { sum = min(sum + (uint32_t)__builtin_amdgcn_update_dpp(0, (int)sum, decltype(ctrl)::value, 0xf, 0xf, false), most); };
+            add(std::integral_constant<int, DPP_QUAD_XOR1>{});
+            add(std::integral_constant<int, DPP_QUAD_XOR2>{});
+            add(std::integral_constant<int, DPP_ROW_HALF_MIRROR>{});
+            add(std::integral_constant<int, DPP_ROW_ROR8>{});
+            auto row = [&](int l) { return (uint32_t)__builtin_amdgcn_readlane((int)sum, l); };
+            sum = min(min(row(0) + row(16), most) + min(row(32) + row(48), most), most);
             first = (int)sum;
             draws = min(max(own, 0), (int)(most - sum));
         }
         if (lane == 0) { s_first = first; s_draws = draws; }
-        if (!greedy_row && lane < draws) s_uniform[lane] = uniform[first + lane];
+        if (!greedy_row && lane < draws) my_uniform = uniform[first + lane];
     };
 
     constexpr int CH = 32;
@@ -483,6 +489,7 @@ __global__ __launch_bounds__(1024) void sample_topk_kernel(const half_t *__restr
             thr -= steps;
             small = steps < 63;
         }
+        if (wv == 0) s_uniform[lane] = my_uniform;
         const bool real = small && thr > 0;                     // (key 0: also the slots past the row)
         // the threads whose maximum reaches the bound leave their keys, in any order
         const bool hot = real && mx >= thr;
@@ -644,7 +651,10 @@ __global__ __launch_bounds__(1024) void sample_topk_kernel(const half_t *__restr
 
     // ---- order the k candidates: rank = number of candidates that come before (the last wave has none of the first 960) ----
     // (Here its loads are waited for beside the ranking; at the top of the histograms, by the first wave, 16 rows with k = 600 took 81.3 us instead of 79.0.)
-    if (!by_maxima && wv == 15) find_draws();
+    if (!by_maxima && wv == 15) {
+        find_draws();
+        s_uniform[lane] = my_uniform;
+    }
     if (tid < k) {
         const uint32_t mk = c_key[tid];
         const int mi = c_idx[tid];
