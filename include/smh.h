@@ -104,8 +104,10 @@ int smh_gq40_dequant(const void *packed, const void *scale, void *out, long bloc
  * hf_model_q40_kv_shared.py:313; w1|w3 of FeedForward.forward, :434) run as segments of one
  * launch; their outputs are concatenated along the columns (n_total = sum of n[i]).
  *
- * smh_q40_matmul_plan         ksplit the kernels will use for these dimensions on checkpoint-layout weights (depends on M, K, n only)
- * smh_q40_matmul_plan_tiled   the same for tiled weights (smh_q40_tile): equal up to 16 rows; above, tiled weights may take fewer slices
+ * smh_q40_matmul_plan         ksplit of smh_q40_matmul_partial for these dimensions (depends on M, K, n only).  smh_q40_matmul needs a workspace for as
+ *                             many slabs and may leave fewer, or none
+ * smh_q40_matmul_plan_tiled   the same for tiled weights (smh_q40_tile): equal but for 17 .. 128 rows with K a multiple of 64, where tiled weights may take
+ *                             fewer slices
  * smh_q40_matmul_partial      produce the slabs; partial_bytes >= ksplit * M * n_total * 4
  * smh_partial_reduce          c[m][j] = fp16(sum) (+ residual) for columns col0 .. col0+N-1
  * smh_partial_rmsnorm         h_out = h_in + fp16(sum) (residual add of TransformerBlock.forward,
@@ -145,8 +147,8 @@ int smh_q40_matmul_partial(const void *a, int M, int K, long lda, int nseg, cons
  * is what every entry point above takes.  smh_q40_tile rewrites one weight, once, into the order the matmul
  * kernels consume it (256-column x 32-row tiles of 4352 contiguous bytes: nibbles in MFMA operand order, then the
  * tile's scales); smh_q40_matmul_partial_tiled is smh_q40_matmul_partial on such weights and leaves bit-identical
- * slabs - it replaces the same matmul_q40 (triton_kernels.py:471-500) calls, with fewer memory requests and fewer
- * decode instructions per weight.  tiled buffers: smh_q40_tiled_bytes(K, N) bytes, 128-byte aligned. */
+ * slabs (but for 17 .. 128 rows with K a multiple of 64, where the order of the additions and the number of slabs may be others) - it replaces the same
+ * matmul_q40 (triton_kernels.py:471-500) calls, with fewer memory requests and fewer decode instructions per weight.  tiled buffers: smh_q40_tiled_bytes(K, N) bytes, 128-byte aligned. */
 size_t smh_q40_tiled_bytes(int K, int N);
 int smh_q40_tile(const void *w, const void *s, int K, int N, void *tiled, size_t tiled_bytes, smh_stream_t stream);
 int smh_q40_matmul_partial_tiled(const void *a, int M, int K, long lda, int nseg, const void *const *tiled,

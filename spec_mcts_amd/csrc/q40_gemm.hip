@@ -1417,12 +1417,12 @@ void gemm_fill_plan(MatmulParams &p) {
     const int steps = (p.K + 31) / 32;
     if (p.M > GEMM_BM) {
         gemm_plan_rows(p, steps, SMH_MAX_KSPLIT, ROWS_256);
-        // Tiled weights whose plan is cut along K: the same row blocks with 128-column blocks and two K-groups a workgroup, where they fill two thirds of the
-        // compute units in one round with at least two slices of at most 48 stages (64 rows of K each) - about half the slabs.  26 launches of 136 .. 749 rows that
-        // take it, with the RMSNorm behind them: 1.06 .. 1.23 times as fast (us, 512 x 4096 x 4096 32.4 and 30.2, 240 rows 21.7 and 19.9, 221 x 4096 x 11008 32.8
-        // and 29.5); of 86 stages 0.98 and 1.00 (300 and 512 x 4096 x 11008), of one slice 0.81 .. 1.02.  Up to 160 rows (20.4 and 16.6 at 144 x 4096 x 4096) slabs
-        // keep the checkpoint layout's bits.
-        if (p.tiled && p.M > 160 && p.ksplit > 1 && p.K % 64 == 0 && p.K <= 16384) {
+        // A plan that is cut along K: the same row blocks with 128-column blocks and two K-groups a workgroup, where they fill two thirds of the
+        // compute units in one round with at least two slices of at most 48 stages (64 rows of K each) - about half the slabs.  48 launches of 129 .. 749 rows of
+        // tiled weights that take it, with the RMSNorm behind them: 1.06 .. 1.23 times as fast (us, 512 x 4096 x 4096 32.4 and 30.2, 240 rows 21.7 and 19.9,
+        // 144 rows 20.3 and 17.0, 221 x 4096 x 11008 32.8 and 29.5), 44 of the checkpoint layout 1.08 .. 1.24; of 86 stages 0.98 and 1.00 (300 and 512 x 4096 x
+        // 11008), of one slice 0.81 .. 1.02.  Both layouts take it: above 128 rows their slabs are the same bits.
+        if (p.ksplit > 1 && p.K % 64 == 0 && p.K <= 16384) {
             const long blocks = p.n_total / 128, on_xcd = (long)p.units_pad / 4 * p.mblocks;
             const int ks = (int)min(min(256 / (blocks * p.mblocks), 32 / on_xcd), (long)p.ksplit), sps = ks > 0 ? ((steps + ks - 1) / ks + 1) / 2 * 2 : 0;
             if (ks >= 2 && blocks * p.mblocks * ks >= 170 && sps <= 96) {
@@ -1563,13 +1563,13 @@ static int gemm_launch_layout(const MatmulParams &p, hipStream_t stream) {
 //     (above that 0.76 .. 1.07: 37 x 4096 x 11008, 22 stages, 17.1 us and 18.0, 100 x 12288 x 4096, 32 stages, 26.0 and 28.3);
 //   * where p's are more, or cut at runs of steps: up to 48 stages, above 64 rows 64: 10 shapes 1.05 .. 1.64 (20 x 24576 x 4096, 64 stages, 26.1 us and
 //     32.0; 80 x 22400 x 15208 109.6 and 133);
-//   * above 128 rows, on p's row blocks, where K is cut and half the compute units get work: up to 40 stages, 46 shapes of 130 .. 512 rows 1.02 .. 1.52 times
+//   * above 128 rows, on p's row blocks, where K is cut, p has not that form already and half the compute units get work: up to 40 stages, 46 shapes of 130 .. 512 rows 1.02 .. 1.52 times
 //     (us, 512 x 4096 x 4096 32.1 and 28.3, 300 rows 24.1 and 22.0, 242 x 5888 x 1176 20.4 and 13.4; of 41 to 45 stages 0.99 .. 1.07, of 86 0.91 and 0.92, of 191 0.81).
 // us of both launches, in turn: 100 x 4096 x 4096 18.8 and 15.5, 20 x 4096 x 4096 11.4 and 9.8, 100 x 5120 x 5120 28.5 and 17.9, 37 x 7168 x 7168 26.2 and
 // 19.1, 100 x 6400 x 3000 26.7 and 18.5, 100 x 24064 x 1928 35.3 and 24.7.
 bool gemm_blocks_fit(const MatmulParams &p, MatmulParams &b) {
     // (half a stage past a K that is a multiple of 32 would meet an infinite activation with a zero)
-    if (p.tiled || p.nseg != 1 || p.M <= SMH_GEMV_MAX_M || p.K > 16384 || p.K % 64 == 32) return false;
+    if (p.tiled || p.kgroups == 2 || p.nseg != 1 || p.M <= SMH_GEMV_MAX_M || p.K > 16384 || p.K % 64 == 32) return false;
     const bool many = p.M > GEMM_BM;
     const int blocks = p.seg[0].N / 128, mblocks = many ? p.mblocks : blocks <= 32 && p.M > 64 && p.K <= 4096 ? 2 : 1, steps = (p.K + 31) / 32;
     if ((long)blocks * mblocks > 256) return false;

@@ -87,7 +87,7 @@ def matmul_q40(a: torch.Tensor, b_w: torch.Tensor, b_s: torch.Tensor, b_shape: S
 
 def matmul_plan(M: int, K: int, ns: Sequence[int], tiled: bool = False) -> int:
     """Number of K slices the matmul kernels use for a [M,K] x [K, sum(ns)] product on checkpoint-layout or on tiled
-    weights (the same up to 16 rows)."""
+    weights (the same but for 17 to 128 rows with K a multiple of 64).  matmul_q40 may leave fewer slabs."""
     import ctypes
     lib = _lib.load()
     arr = (ctypes.c_int * len(ns))(*[int(n) for n in ns])
@@ -128,8 +128,8 @@ def tile_q40(w: torch.Tensor, s: torch.Tensor, K: int, N: int) -> TiledQ40:
 
 def matmul_q40_partial(a: torch.Tensor, linears, out: Optional[torch.Tensor] = None) -> PartialProduct:
     """One launch for up to 3 Q4_0 weights that share the input a [M,K]; `linears` is a sequence of
-    (w, s, N), or of TiledQ40 (same slabs, bit for bit, where both have the same plan: matmul_plan).  Leaves the un-reduced product; the columns of the
-    weights are concatenated."""
+    (w, s, N), or of TiledQ40 (same slabs, bit for bit; 17 to 128 rows with K a multiple of 64 may be added up in another order, in fewer slabs).
+    Leaves the un-reduced product; the columns of the weights are concatenated."""
     import ctypes
     lib = _lib.load()
     assert a.is_contiguous() and a.dtype == torch.float16 and a.dim() == 2 and a.data_ptr() % 16 == 0

@@ -414,3 +414,19 @@ def test_two_k_groups_above_160_rows(M, K, ns, slabs):
     got = Kn.partial_reduce(p).double()
     want = torch.cat([a.double() @ Kn.deq_int40(w, s, 64, (K, n)).double() for (w, s), n in zip(ws, ns)], 1)
     assert bool(((got - want).abs() <= want.abs() * 2.0 ** -11 + 2.0 ** -24 * K ** 0.5 * want.abs().max()).all())
+
+
+@pytest.mark.parametrize("M,K,ns", [(129, 4096, [4096]), (144, 4096, [4096]), (160, 11008, [4096]), (161, 4096, [4096]), (175, 4096, [2048, 256, 1792]), (196, 1024, [2048]),
+                                    (200, 2112, [4096]), (220, 8192, [3072]), (234, 4096, [4096]), (526, 4096, [2048]), (600, 4096, [11008])])
+def test_slabs_of_both_layouts_above_128_rows(M, K, ns):
+    """above 128 rows both layouts take the same plan: as many slabs, the same bits.  Plans of two K-groups a workgroup with blocks of 80 to 128 rows and
+    several slices (196 x 1024 x 2048: as many as without), several weights, an odd number of blocks, a shorter last slice; one without"""
+    from spec_mcts_amd import kernels as Kn
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    lin = [(*Kn.quantize_q40(torch.randn((K, n), device="cuda", generator=g, dtype=torch.float16) * 0.02), n) for n in ns]
+    a = torch.randn((M, K), device="cuda", generator=g, dtype=torch.float16)
+    p0 = Kn.matmul_q40_partial(a, lin)
+    p1 = Kn.matmul_q40_partial(a, [Kn.tile_q40(w, s, K, n) for w, s, n in lin])
+    assert p0.ksplit == p1.ksplit == Kn.matmul_plan(M, K, ns) == Kn.matmul_plan(M, K, ns, tiled=True)
+    size = p0.ksplit * M * sum(ns)
+    assert torch.equal(p0.buf[:size].view(torch.int32), p1.buf[:size].view(torch.int32))
