@@ -471,15 +471,27 @@ def test_prefill_lengths_around_the_tiles(S, H, Hkv):
 
 
 @pytest.mark.parametrize("P", [1, 128, 129, 256, 257, 512, 513, 1050])
-def test_merge_at_every_number_of_partials_on_their_way(P):
+@pytest.mark.parametrize("order", ["level", "rising", "falling", "below the suffix"])
+def test_merge_at_every_number_of_partials_on_their_way(P, order):
     """fp16 suffixes: slices of 32 prompt rows and the suffix leave 2, 5, 6, 9, 10, 17, 18 and 34 partials a query; the merge has 5, 9 or 17 of them on
-    their way at a time.  A prompt of scores that rise by 30 from slice to slice lets the last ones outweigh the first; branches without rows"""
+    their way at a time.  Scores that rise by 30 from slice to slice let the last one outweigh all before it (e^-30 and less), which the merge has
+    scaled already; that fall by 30 leave it to the first; below the suffix the last partial, the suffix's, outweighs them.  A branch without rows"""
     from spec_mcts_amd import kernels as K
     B, S = 5, 9
     q, pk, pv, sk, sv, lens = _inputs(B, 1, 1, 128, P, S, 60 + P)
-    lens[0] = 0
-    for rise in (0.0, 30.0):
-        k = pk.clone()
-        k[..., 0] += rise * (torch.arange(P) // 32).half()[:, None] / 16
-        want = O.shared_prefix_attention(q, k, pv, sk, sv, lens.tolist())
-        _check(K.shared_prefix_attn(q.cuda(), k.cuda(), pv.cuda(), P, suffix_k=sk.cuda(), suffix_v=sv.cuda(), Smax=S, lens=lens.cuda(), lens_stride=1), want)
+    lens[:] = torch.tensor([0, 9, 1, 4, 7])
+    slices = (P + 31) // 32
+    rank = torch.arange(P) // 32
+    level = {"level": 0 * rank, "rising": rank, "falling": slices - 1 - rank, "below the suffix": -1 - rank}[order]
+    if order != "level":                                   # a score's part of dimension 0 is its key's value there
+        q[..., 0] = 128 ** 0.5
+        pk[..., 0] = (30 * level).half()[:, None]
+        sk[..., 0] = 0
+    score = torch.einsum("bhd,lhd->bl", q.float(), pk.float()) / 128 ** 0.5
+    top = torch.stack([score[:, rank == i].amax(1) for i in range(slices)], 1)
+    own = torch.einsum("bhd,blhd->bl", q.float(), sk.float()) / 128 ** 0.5
+    step = top[:, 1:] - top[:, :-1]
+    assert {"level": bool((step.abs() < 10).all()), "rising": bool((step > 20).all()), "falling": bool((step < -20).all()),
+            "below the suffix": bool((step < -20).all()) and bool((own.amin(1) > top.amax(1) + 20).all())}[order]
+    want = O.shared_prefix_attention(q, pk, pv, sk, sv, lens.tolist())
+    _check(K.shared_prefix_attn(q.cuda(), pk.cuda(), pv.cuda(), P, suffix_k=sk.cuda(), suffix_v=sv.cuda(), Smax=S, lens=lens.cuda(), lens_stride=1), want)
