@@ -121,15 +121,19 @@ int smh_gq40_dequant(const void *packed, const void *scale, void *out, long bloc
  */
 int smh_q40_matmul_plan(int M, int K, int nseg, const int *n);
 int smh_q40_matmul_plan_tiled(int M, int K, int nseg, const int *n);
+/* columns that a workgroup of smh_q40_matmul multiplies above 16 rows: 128 (two K-groups a workgroup) or 256; 0 up to 16 rows */
+int smh_q40_matmul_columns(int M, int K, int N);
 /* smh_q40_matmul_tiled_swiglu: out[M, n_half] = fp16(silu(fp16(a . gate))) * fp16(a . up) for tiled gate and up weights
- * [K, n_half] - `F.silu(self.w1(x)) * self.w3(x)` of FeedForward.forward (hf_model_q40_kv_shared.py:434) in ONE launch, with
- * the roundings of smh_q40_matmul_partial_tiled + smh_partial_silu_mul (every linear rounded to fp16 first) and no slab
+ * [K, n_half] - `F.silu(self.w1(x)) * self.w3(x)` of FeedForward.forward (hf_model_q40_kv_shared.py:434) in one launch (above 128 rows one or two, of the
+ * first and the other columns), with the roundings of smh_q40_matmul_partial_tiled + smh_partial_silu_mul (every linear rounded to fp16 first) and no slab
  * in between.  17 <= M <= 128, K a multiple of 64, n_half a multiple of 128 and at most 16384 (all of K in one workgroup,
  * one workgroup per compute unit); or M > 128, K a multiple of 32, n_half a multiple of 128.  smh_q40_swiglu_fits: 1 when the shape is supported AND wide enough (n_half >= 8192) for
  * this to be the faster way; else use the two launches. */
 int smh_q40_swiglu_fits(int M, int K, int n_half);
 /* columns of the two weights that a workgroup of that launch multiplies (128; above 128 rows 256 or 384, by an estimate); 0: not supported */
 int smh_q40_swiglu_columns(int M, int K, int n_half);
+/* columns of either weight that the first of two launches multiplies (by workgroups of 384, the rest by workgroups of 256); 0: one launch */
+int smh_q40_swiglu_first_columns(int M, int K, int n_half);
 int smh_q40_matmul_tiled_swiglu(const void *a, int M, int K, long lda, const void *tiled_gate, const void *tiled_up, int n_half,
                                 void *out, long ldo, smh_stream_t stream);
 /* smh_q40_matmul_tiled_direct: LinearQ4_0.forward (:228-236) of up to 3 tiled weights that share the input, for more than 128

@@ -363,6 +363,13 @@ extern "C" int smh_q40_matmul_plan(int M, int K, int nseg, const int *n) {
     return st < 0 ? st : p.ksplit;
 }
 
+extern "C" int smh_q40_matmul_columns(int M, int K, int N) {
+    MatmulParams p, b;
+    if (M <= SMH_GEMV_MAX_M) return 0;
+    const int st = fill_params(p, nullptr, M, K, (K + 7) / 8 * 8, 1, nullptr, nullptr, &N, "smh_q40_matmul_columns");
+    return st < 0 ? st : p.kgroups == 2 || (p.ksplit > 1 && gemm_blocks_fit(p, b)) ? 128 : 256;
+}
+
 extern "C" int smh_q40_swiglu_fits(int M, int K, int n_half) { return smh::gemm_swiglu_fits(M, K, n_half, true) ? 1 : 0; }
 
 extern "C" int smh_q40_matmul_tiled_swiglu(const void *a, int M, int K, long lda, const void *tiled_gate, const void *tiled_up, int n_half,
@@ -396,13 +403,15 @@ extern "C" int smh_q40_matmul_tiled_direct_columns(int M, int K, int nseg, const
     return st < 0 ? st : gemm_direct_columns(p);
 }
 
-extern "C" int smh_q40_swiglu_columns(int M, int K, int n_half) {
+static int swiglu_plan(int M, int K, int n_half, int (*ask)(MatmulParams)) {
     if (!gemm_swiglu_fits(M, K, n_half, false)) return 0;
     MatmulParams p = MatmulParams{};
     p.M = M; p.K = K; p.nseg = 2;
     p.seg[0].N = p.seg[1].N = n_half;
-    return gemm_swiglu_columns(p);
+    return ask(p);
 }
+extern "C" int smh_q40_swiglu_columns(int M, int K, int n_half) { return swiglu_plan(M, K, n_half, gemm_swiglu_columns); }
+extern "C" int smh_q40_swiglu_first_columns(int M, int K, int n_half) { return swiglu_plan(M, K, n_half, gemm_swiglu_first_columns); }
 
 extern "C" int smh_q40_matmul_tiled_direct(const void *a, int M, int K, long lda, int nseg, const void *const *tiled, const int *n, void *const *out,
                                            const void *residual, long ldr, smh_stream_t stream) {

@@ -1693,6 +1693,11 @@ static int gemm_swiglu_split(const MatmulParams &w, int pieces, int steps) {
     return first;
 }
 
+int gemm_swiglu_first_columns(MatmulParams p) {
+    MatmulParams w = p;
+    return p.M > GEMM_BM && gemm_swiglu_rows_plan(p, w) ? 192 * gemm_swiglu_split(w, p.seg[0].N / 64, p.K / 32) : 0;
+}
+
 int gemm_swiglu_rows_launch(MatmulParams p, hipStream_t stream) {
     // (blocks of 64 .. 128 rows)
     static const gemm_kernel_t plain[5] = {q40_gemm_kernel<4, false, true, 8, GEMM_STAGES, false, false, true>, q40_gemm_kernel<5, false, true, 8, GEMM_STAGES, false, false, true>, q40_gemm_kernel<6, false, true, 8, GEMM_STAGES, false, false, true>,

@@ -124,5 +124,7 @@ int gemm_swiglu_rows_launch(MatmulParams p, hipStream_t stream);
 // columns that a workgroup of these launches multiplies
 int gemm_direct_columns(MatmulParams p);
 int gemm_swiglu_columns(MatmulParams p);
+// columns of either weight in the first of two launches, 0: there is one
+int gemm_swiglu_first_columns(MatmulParams p);
 
 }  // namespace smh

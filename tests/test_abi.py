@@ -240,3 +240,15 @@ def test_columns_of_a_workgroup_above_128_rows():
     assert lib.smh_q40_swiglu_columns(16, 4096, 11008) == 0 and lib.smh_q40_swiglu_columns(300, 4096 + 8, 11008) == 0
     assert lib.smh_q40_swiglu_columns(100, 4096, 11008) == 128
     assert {lib.smh_q40_swiglu_columns(M, 4096, 11008) for M in range(129, 600)} == {256, 384}
+    # two launches where the last round of one would be a poor one: 48 workgroups of three pieces, then the columns behind them
+    assert lib.smh_q40_swiglu_first_columns(128, 4096, 11008) == 0 and lib.smh_q40_swiglu_first_columns(2047, 4096 + 8, 11008) == 0
+    assert lib.smh_q40_swiglu_first_columns(512, 4096, 11008) == 0 and lib.smh_q40_swiglu_first_columns(2047, 4096, 11008) == 48 * 192
+
+
+def test_columns_of_a_workgroup_on_the_checkpoint_layout():
+    """which of its two launches above 16 rows smh_q40_matmul takes"""
+    from spec_mcts_amd import _lib
+    columns = _lib.load().smh_q40_matmul_columns
+    assert columns(16, 4096, 4096) == 0 and columns(100, 4096, 100) < 0
+    assert columns(17, 4096, 4096) == 128 and columns(100, 4096, 11008) == 256 and columns(512, 4096, 4096) == 128 and columns(512, 11008, 4096) == 256
+    assert columns(100, 4096 + 32, 4096) == 256                # (half a stage past the end of K)

@@ -325,17 +325,27 @@ def test_checkpoint_products_at_the_end_of_k(M, K, N):
     assert bool(((got - want).abs() <= want.abs() * 2.0 ** -11 + 2.0 ** -24 * K ** 0.5 * want.abs().max()).all())
 
 
-@pytest.mark.parametrize("M,K", [(1040, 2048), (900, 1536), (300, 4096)])
-def test_checkpoint_product_over_its_own_activations(M, K):
+@pytest.mark.parametrize("M,K,columns,stored", [(1040, 2048, 128, True), (900, 1536, 256, False), (300, 4096, 128, False)])
+def test_checkpoint_product_over_its_own_activations(M, K, columns, stored):
     """A product whose K is cut reads all of its activations before the launch that writes the result, so the result may take their place: also where the
-    plan's two slices become one slice of 128-column blocks, which would be stored without slabs.  The same bits as apart"""
-    from spec_mcts_amd import kernels as Kn
-    assert Kn.matmul_plan(M, K, [K]) > 1
+    plan's two slices become one slice of 128-column blocks, which apart is stored without slabs.  The same bits as apart"""
+    from spec_mcts_amd import _lib, kernels as Kn
+    ks = Kn.matmul_plan(M, K, [K])
+    assert ks > 1 and _lib.load().smh_q40_matmul_columns(M, K, K) == columns
     g = torch.Generator(device="cuda").manual_seed(M + K)
     w, s = Kn.quantize_q40(torch.randn((K, K), device="cuda", generator=g, dtype=torch.float16) * 0.02)
     x = torch.randn((M, K), device="cuda", generator=g, dtype=torch.float16)
     apart = Kn.matmul_q40(x, w, s, (K, K))
+    slabs, c = torch.full((ks * M * K,), float("nan"), device="cuda"), torch.empty((M, K), device="cuda", dtype=torch.float16)
+    Kn.check(_lib.load().smh_q40_matmul(x.data_ptr(), M, K, K, w.data_ptr(), s.data_ptr(), K, c.data_ptr(), K, Kn.SMH_EPI_NONE, None, K, slabs.data_ptr(),
+                                        slabs.numel() * 4, Kn._stream()), "smh_q40_matmul")
+    assert torch.equal(c, apart) and bool(slabs.isnan().all()) == stored
     assert torch.equal(Kn.matmul_q40(x, w, s, (K, K), out=x), apart)
+
+
+# row counts of the test below that keep 256 columns a workgroup
+WIDE_ROWS = {(4104, 3840): (512,), (1928, 24064): (129, 200, 273, 512), (3000, 6400): (273, 512), (2072, 5760): (512,), (7168, 7168): (129, 200, 273, 512),
+             (1496, 21760): (129, 200, 273, 512), (1024, 2944): (17, 48, 64)}
 
 
 @pytest.mark.parametrize("M", [17, 48, 64, 65, 97, 128, 129, 200, 273, 512])
@@ -343,8 +353,9 @@ def test_checkpoint_product_over_its_own_activations(M, K):
 def test_checkpoint_products_in_blocks_of_128_columns(M, K, N):
     """Launches of 128-column blocks with two K-groups a workgroup: edges of the row tiles and of the two row blocks, odd numbers of blocks, K that ends in
     the first or the second half of a stage, one slice (stored without slabs) and several, with and without a residual, in rows of a larger output.  Against
-    64 bits: half a unit of fp16 and the fp32 sums; with the residual another half"""
+    64 bits: half a unit of fp16 and the fp32 sums; with the residual another half.  Where the other launch is planned, the same"""
     from spec_mcts_amd import _lib, kernels as Kn
+    assert _lib.load().smh_q40_matmul_columns(M, K, N) == (256 if M in WIDE_ROWS.get((K, N), ()) else 128)
     g = torch.Generator(device="cuda").manual_seed(7 * M + K)
     w, s = Kn.quantize_q40(torch.randn((K, N), device="cuda", generator=g, dtype=torch.float16) * 0.02)
     x = torch.randn((M, K), device="cuda", generator=g, dtype=torch.float16)

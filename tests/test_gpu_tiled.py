@@ -375,8 +375,8 @@ def test_wide_workgroups(M, K, ns, columns):
             assert torch.equal(o_r.cpu(), (r.float() + o.cpu().float()).half())
 
 
-@pytest.mark.parametrize("M,K,n_half", [(430, 256, 18560), (512, 128, 28672), (500, 1056, 18560), (866, 512, 14336)])
-def test_swiglu_in_two_launches_where_the_last_round_is_a_poor_one(M, K, n_half):
+@pytest.mark.parametrize("M,K,n_half,first", [(430, 256, 18560, 10752), (512, 128, 28672, 12288), (500, 1056, 18560, 10752), (866, 512, 14336, 6144)])
+def test_swiglu_in_two_launches_where_the_last_round_is_a_poor_one(M, K, n_half, first):
     """Workgroups of three pieces of each weight for most columns, of two for the rest: what one weight's columns after the other give in 64 bits, to the
     roundings of fp16 products, silu and their product; outputs in rows of a larger tensor, whose other columns stay"""
     from spec_mcts_amd import _lib, kernels as Kn
@@ -384,7 +384,7 @@ def test_swiglu_in_two_launches_where_the_last_round_is_a_poor_one(M, K, n_half)
     ws = [Kn.quantize_q40(torch.randn((K, n_half), device="cuda", generator=g, dtype=torch.float16) * 0.1) for _ in range(2)]
     tiled = [Kn.tile_q40(w, s, K, n_half) for w, s in ws]
     x = torch.randn((M, K), device="cuda", generator=g, dtype=torch.float16)
-    assert _lib.load().smh_q40_swiglu_columns(M, K, n_half) == 384
+    assert _lib.load().smh_q40_swiglu_columns(M, K, n_half) == 384 and _lib.load().smh_q40_swiglu_first_columns(M, K, n_half) == first
     wide = torch.full((M, n_half + 4), 7.0, device="cuda", dtype=torch.float16)
     Kn.check(_lib.load().smh_q40_matmul_tiled_swiglu(x.data_ptr(), M, K, K, tiled[0].buf.data_ptr(), tiled[1].buf.data_ptr(), n_half, wide.data_ptr(), n_half + 4,
                                                      Kn._stream()), "smh_q40_matmul_tiled_swiglu")
