@@ -608,8 +608,8 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
     // steps i+3 .. i+S-3 may be in flight, and the slots of steps i-2, i-1 are refilled with steps i+S-2, i+S-1.  A stage has the same two steps of time to land as
     // with a barrier per step; the waves meet half as often.
     if constexpr (PRODUCER) {
-        // (the end of K is stage `at_end` of a slice that has it)
-        const int end = (p.K - 1) / 32 - step0, at_end = RAGGED && step1 > (p.K - 1) / 32 ? (end >= rot ? end - rot : end - rot + n_steps) : -1;
+        // (the end of K, the last step of a slice that has it, is fetched as stage at_end: rot < n_steps)
+        const int at_end = RAGGED && step1 > (p.K - 1) / 32 ? n_steps - 1 - rot : -1;
         const auto weights = [&] {
             if constexpr (TILED) return TiledWeights(hh, wave * 1024 + lane * 16, GS_W + g * 64 + (2 * blk + hh) * 16);
             else return RowWeights<RAGGED>(hh, g * GS_WBLOCK + 64 * blk + 4 * c, GS_W + 64 * g + 4 * blk, sel0, at_end, (p.K - 1) / 32 * 32 + 8 * g >= p.K);
@@ -947,7 +947,7 @@ __global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_kg_kern
     const auto weights = [&] {
         if constexpr (TILED) return TiledWeights(hh, (2 * kk + bp) * 1024 + lane * 16, KG_W + kk * 256 + g * 64 + (2 * blk + hh) * 16);
         else return RowWeights<RAGGED, true>(hh, kk * 2048 + g * 64 + 4 * c, KG_W + kk * 256 + g * 32, 0x0c000c00u | (uint32_t)(2 * bp) | ((uint32_t)(4 + 2 * bp) << 16),
-                                             ends ? (n_st - 1 >= rot ? n_st - 1 - rot : 2 * n_st - 1 - rot) : -1, 32 * (step0 + 2 * (n_st - 1) + kk) + 8 * g >= p.K);
+                                             ends ? n_st - 1 - rot : -1, 32 * (step0 + 2 * (n_st - 1) + kk) + 8 * g >= p.K);     // (the end of K is that stage: rot < n_st)
     }();
     gemm_multiply<TILES, SLOTS, STAGE, GEMM_PRODUCTS_FIRST>(lds, n_st, weights, KG_W + KG_S + kk * TILES * 1024 + c * 64 + ((g ^ ((c >> 1) & 3)) << 4), acc);
 
