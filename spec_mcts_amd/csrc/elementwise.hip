@@ -243,7 +243,7 @@ namespace smh {
 // CDF with the caller's uniform number.
 constexpr int SAMPLE_MAX_K = 1024;
 constexpr int SAMPLE_HOT_MAX = 576;            // threads whose logits are looked at again
-// Up to here the bound is guessed from sixteenths of the maxima.  The guess takes k / 14 steps and saves three rounds.  80 rows of 32016, us, without and with
+// Up to here the bound is guessed from sixteenths of the maxima.  The guess takes k / 14 + 1 steps and saves three rounds.  80 rows of 32016, us, without and with
 // one: k = 32 7.2 and 6.8, 65 9.0 and 8.8, 96 9.4 and 9.6.
 constexpr int SAMPLE_GUESS_MAX_K = 80;
 constexpr int SAMPLE_PICK_MAX_K = 512;         // up to here the candidates are picked by the threads' maxima (above, they would be thousands)
@@ -443,8 +443,8 @@ __global__ __launch_bounds__(1024) void sample_topk_kernel(const half_t *__restr
         int *slot = bins;
         uint32_t thr = 0;
         if (k <= SAMPLE_GUESS_MAX_K) {
-            // Sixteen guesses: each wave's r-th largest of a sixteenth of the maxima, r a third above k / 16 or more, of which k to k + 32 maxima reach one in
-            // two or three (unordered logits: 600 of 600 rows needed no further round).
+            // Sixteen guesses: each wave's r-th largest of a sixteenth of the maxima, r = k / 14 + 1 (from k = 13 on 1.16 to 2.3 times k / 16), of which k to
+            // k + 32 maxima reach one in two or three (unordered logits, 300 rows at each k up to 80: one row needed a further round, at k = 68).
             uint32_t v = maxima[16 * lane + ((wave + (lane >> 2)) & 15)], t = 0, over = 0x10000u;
             for (int r = k / 14; r >= 0; --r) {
                 t = wave_max_bits(v);
