@@ -587,7 +587,7 @@ static int matmul_fp16(const void *a, int M, int K, long lda, const void *b_w, c
         SMH_REQUIRE(!gemm || ldc % 8 == 0, "%s: ldc=%ld must be a multiple of 8 for M > 16", who, ldc);
         return gemm ? gemm_launch(p, (hipStream_t)stream) : gemv_launch(p, (hipStream_t)stream);
     }
-    size_t need = (size_t)p.ksplit * M * N * sizeof(float);          // (what smh_q40_matmul_plan says; fewer slabs where q40_gemm_kg_kernel runs)
+    size_t need = (size_t)p.ksplit * M * N * sizeof(float);          // (what smh_q40_matmul_plan says; fewer slabs where gemm_blocks_fit has a form)
     SMH_REQUIRE(workspace && workspace_bytes >= need, "%s: workspace %zu < %zu bytes", who, workspace_bytes, need);
     p.partial = (float *)workspace;
     p.direct = 0;
