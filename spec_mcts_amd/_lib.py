@@ -51,6 +51,7 @@ SIGNATURES = {
     "smh_q40_swiglu_fits": (c_int, [c_int, c_int, c_int]),
     "smh_q40_swiglu_columns": (c_int, [c_int, c_int, c_int]),
     "smh_q40_swiglu_first_columns": (c_int, [c_int, c_int, c_int]),
+    "smh_q40_warm_span": (c_int, [c_int, c_int, c_int, ctypes.POINTER(c_int), c_int, c_int, ctypes.POINTER(c_long), ctypes.POINTER(c_long), ctypes.POINTER(c_long)]),
     "smh_q40_matmul_columns": (c_int, [c_int, c_int, c_int]),
     "smh_q40_matmul_tiled_swiglu": (c_int, [_P, c_int, c_int, c_long, _P, _P, c_int, _P, c_long, _P]),
     "smh_q40_matmul_partial": (c_int, [_P, c_int, c_int, c_long, c_int, _P, _P, _P, _P, c_size_t, _P]),

@@ -24,6 +24,7 @@
 
 #include "attn_rows.hpp"
 #include "attn_tiles.hpp"
+#include "q40_warm.hpp"
 #include "rope_kv.hpp"
 
 namespace smh {
@@ -1600,10 +1601,11 @@ __device__ __forceinline__ void kv_store_lanes(h4 x, uint8_t *row, half_t *scale
 }
 
 // QKS: most slabs of the q|k|v product, LEAST: the fewest.  QT: queries of a workgroup, 16 or 8 (then a wave's halves share one query and take
-// its rows 16 at a time in turn).  Grid: (XCD, kv head of it, tile).
+// its rows 16 at a time in turn).  Grid: (XCD, kv head of it, tile); workgroups past the tiles ask for the next launch's weights (q40_warm.hpp).
 template <bool PAGES, int LEAST, int QKS, int QT>
-__global__ __launch_bounds__(64 * AT_WAVES) void attn_tile_kernel(AttnParams p, int chunks) {
-    args_ahead<sizeof(AttnParams)>();
+__global__ __launch_bounds__(64 * AT_WAVES) void attn_tile_kernel(AttnParams p, int chunks, int tiles, WarmWeights next) {
+    args_ahead<sizeof(AttnParams) + 8>();
+    if (__builtin_expect((int)blockIdx.z >= tiles, 0)) return warm_weights(next, blockIdx.x, (blockIdx.z - tiles) * gridDim.y + blockIdx.y, threadIdx.x, 64 * AT_WAVES);
     extern __shared__ __attribute__((aligned(16))) float at_lds[];
     half_t *const s_q = reinterpret_cast<half_t *>(at_lds + AT_WAVES * AT_MINE), *const s_k = s_q + 16 * AT_QPITCH, *const s_v = s_k + 16 * AT_QPITCH;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -2358,11 +2360,10 @@ extern "C" int smh_shared_prefix_attn_qkv(const void *qkv_partial, int ksplit, v
     return launch_status();
 }
 
-extern "C" int smh_shared_prefix_attn_qkv_tiles(const void *qkv_partial, int ksplit, void *out, int B, int H, int Hkv, int D,
-                                                const void *cos_tab, const void *sin_tab, const int32_t *pos_dev,
-                                                const void *prefix_k, const void *prefix_v, int P,
-                                                void *cache_k, void *cache_ks, void *cache_v, void *cache_vs, int Smax,
-                                                const int32_t *t_dev, const int32_t *pages, int pages_stride, long cache_rows, smh_stream_t stream) {
+int smh::shared_prefix_attn_qkv_tiles(const void *qkv_partial, int ksplit, void *out, int B, int H, int Hkv, int D, const void *cos_tab, const void *sin_tab,
+                                      const int32_t *pos_dev, const void *prefix_k, const void *prefix_v, int P, void *cache_k, void *cache_ks, void *cache_v,
+                                      void *cache_vs, int Smax, const int32_t *t_dev, const int32_t *pages, int pages_stride, long cache_rows,
+                                      const smh::WarmWeights &next, smh_stream_t stream) {
     using namespace smh;
     const char *who = "smh_shared_prefix_attn_qkv_tiles";
     SMH_REQUIRE(D == ATT_D, "%s: head dim %d (only 128)", who, D);
@@ -2395,7 +2396,7 @@ extern "C" int smh_shared_prefix_attn_qkv_tiles(const void *qkv_partial, int ksp
     p.app_k = (uint8_t *)cache_k; p.app_v = (uint8_t *)cache_v;
     p.app_ks = (half_t *)cache_ks; p.app_vs = (half_t *)cache_vs;
     p.app_t = t_dev; p.app_smax = Smax;
-    typedef void (*kernel_t)(AttnParams, int);
+    typedef void (*kernel_t)(AttnParams, int, int, WarmWeights);
     static const kernel_t kern[2][2][3] = {{{attn_tile_kernel<false, 1, 2, 8>, attn_tile_kernel<false, 3, 6, 8>, attn_tile_kernel<false, 7, 16, 8>},
                                             {attn_tile_kernel<true, 1, 2, 8>, attn_tile_kernel<true, 3, 6, 8>, attn_tile_kernel<true, 7, 16, 8>}},
                                            {{attn_tile_kernel<false, 1, 2, 16>, attn_tile_kernel<false, 3, 6, 16>, attn_tile_kernel<false, 7, 16, 16>},
@@ -2409,9 +2410,21 @@ extern "C" int smh_shared_prefix_attn_qkv_tiles(const void *qkv_partial, int ksp
     if (lds_ok != hipSuccess) { set_error("%s: the kernel's LDS could not be reserved: %s", who, hipGetErrorString(lds_ok)); return (int)lds_ok; }
     const int qt = attn_tile_queries(p.Bq, Hkv), tiles = (p.Bq + qt - 1) / qt;
     const int chunks = (P + AT_CHUNK - 1) / AT_CHUNK;
-    hipLaunchKernelGGL(kern[qt == 16][pages != nullptr][ksplit <= 2 ? 0 : ksplit <= 6 ? 1 : 2], dim3(8, (Hkv + 7) / 8, tiles), dim3(64 * AT_WAVES), AT_LDS,
-                       (hipStream_t)stream, p, chunks);
+    hipLaunchKernelGGL(kern[qt == 16][pages != nullptr][ksplit <= 2 ? 0 : ksplit <= 6 ? 1 : 2], dim3(8, (Hkv + 7) / 8, tiles + next.workgroups / (8 * ((Hkv + 7) / 8))),
+                       dim3(64 * AT_WAVES), AT_LDS, (hipStream_t)stream, p, chunks, tiles, next);
     return launch_status();
+}
+int smh::attn_tiles_idle(int B, int H, int Hkv) {
+    const long queries = (long)B * (H / Hkv), qt = attn_tile_queries(queries, Hkv), row = (Hkv + 7) / 8 * 8, tiles = (queries + qt - 1) / qt;
+    return row * tiles < 256 ? (int)((256 - row * tiles) / row * row) : 0;
+}
+extern "C" int smh_shared_prefix_attn_qkv_tiles(const void *qkv_partial, int ksplit, void *out, int B, int H, int Hkv, int D,
+                                                const void *cos_tab, const void *sin_tab, const int32_t *pos_dev,
+                                                const void *prefix_k, const void *prefix_v, int P,
+                                                void *cache_k, void *cache_ks, void *cache_v, void *cache_vs, int Smax,
+                                                const int32_t *t_dev, const int32_t *pages, int pages_stride, long cache_rows, smh_stream_t stream) {
+    return smh::shared_prefix_attn_qkv_tiles(qkv_partial, ksplit, out, B, H, Hkv, D, cos_tab, sin_tab, pos_dev, prefix_k, prefix_v, P, cache_k, cache_ks, cache_v,
+                                             cache_vs, Smax, t_dev, pages, pages_stride, cache_rows, smh::WarmWeights{}, stream);
 }
 
 // Causal prefill attention: query s attends to rows 0..s of the same K/V tensors.

@@ -6,6 +6,7 @@
 // behind the other (2-3 us each), out of buffers the caller allocated once for the whole pass.  The sequence, the operators
 // and their switches are those of Transformer._forward_fused in hf_model_q40_kv_shared.py.
 #include "attn_tiles.hpp"
+#include "q40_warm.hpp"
 
 namespace smh {
 
@@ -17,6 +18,14 @@ struct LayerBuffers {
     float *sums, *slab_a, *slab_b;             // slabs of wq|wk|wv and w1|w3 (a), of wo and w2 (b)
     size_t slab_a_bytes, slab_b_bytes, total;
 };
+
+// Stages of the next launch's weights that a launch asks for (q40_warm.hpp).  Not where a layer's weights are larger and its attention brings its own long
+// prompt (three layers of 64 heads over 8, dim 8192, 17 .. 100 branches behind 1024 rows: 0.998 .. 1.001 times as fast from the norms, 0.996 .. 1.000 from the attention).
+constexpr int WARM_MAX_DIM = 8191, WARM_FROM_NORM = 3, WARM_FROM_ATTENTION = 4, WARM_FROM_SWIGLU = 16;
+
+static WarmWeights ask(const smh_layer &L, int M, int K, int nseg, const void *const *w, const int *n, bool swiglu, int stages, int workgroups) {
+    return L.dim <= WARM_MAX_DIM ? q40_warm(M, K, nseg, w, n, swiglu, stages, workgroups) : WarmWeights{};
+}
 
 static int slices(int M, int K, int nseg, const int *n) { return smh_q40_matmul_plan_tiled(M, K, nseg, n); }
 // A launch that stores its fp16 results itself (more than 128 rows, no K-split) leaves no slabs.  layer_buffers reserves none for it,
@@ -104,9 +113,9 @@ struct LayerRun {
         return 0;
     }
     // S.h += the product of the linear before (S.pending slabs in slab_b), then its RMSNorm: to b.xn
-    int norm(const void *weight, float eps) {
+    int norm(const void *weight, float eps, const WarmWeights &next = WarmWeights{}) {
         void *h_out = S.pending > 0 ? b.h[S.h == b.h[0]] : nullptr;
-        const int r = smh_partial_rmsnorm(S.pending > 0 ? b.slab_b : nullptr, S.pending > 0 ? S.pending : 1, M, L.dim, S.h, weight, eps, h_out, b.xn, stream);
+        const int r = partial_rmsnorm(S.pending > 0 ? b.slab_b : nullptr, S.pending > 0 ? S.pending : 1, M, L.dim, S.h, weight, eps, h_out, b.xn, next, stream);
         if (h_out != nullptr) S.h = h_out;
         S.pending = 0;
         return r;
@@ -147,7 +156,7 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
     // the RMSNorm of the residual stream and the linears behind it: to slab_a.  With few rows the RMSNorm is made inside the linears' launch.
     auto norm_linears = [&](const void *weight, float eps, int nseg, const void *const *w, const int *n) -> int {
         if (S.pending == 0 || M > S.norm_in_rows || smh_q40_norm_in_fits(M, L.dim, nseg, n) != 1) {
-            if (int r = run.norm(weight, eps)) return r;
+            if (int r = run.norm(weight, eps, ask(L, M, L.dim, nseg, w, n, false, WARM_FROM_NORM, 256))) return r;
             return smh_q40_matmul_partial_tiled(b.xn, M, L.dim, L.dim, nseg, w, n, b.slab_a, b.slab_a_bytes, stream);
         }
         void *h_out = b.h[S.h == b.h[0]];
@@ -188,9 +197,12 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
                                         L.prompt_len, L.cache_k, L.cache_ks, L.cache_v, L.cache_vs, S.smax, S.t_dev, S.pages, S.pages_stride, one, ws,
                                         ws_bytes, stream);
     } else if (way == ATTN_TILES) {
-        st = smh_shared_prefix_attn_qkv_tiles(b.slab_a, ks_qkv, b.att, M, L.heads, L.kv_heads, 128, S.cos_tab, S.sin_tab, S.pos_dev, L.prompt_k, L.prompt_v,
-                                              L.prompt_len, L.cache_k, L.cache_ks, L.cache_v, L.cache_vs, S.smax, S.t_dev, S.pages, S.pages_stride,
-                                              S.cache_rows, stream);
+        const int row = (L.kv_heads + 7) / 8 * 8, idle = attn_tiles_idle(M, L.heads, L.kv_heads);
+        WarmWeights wo = ask(L, M, nq, 1, run.w_o, run.n_dim, false, WARM_FROM_ATTENTION, idle);
+        wo.workgroups = wo.workgroups / row * row;
+        st = shared_prefix_attn_qkv_tiles(b.slab_a, ks_qkv, b.att, M, L.heads, L.kv_heads, 128, S.cos_tab, S.sin_tab, S.pos_dev, L.prompt_k, L.prompt_v,
+                                          L.prompt_len, L.cache_k, L.cache_ks, L.cache_v, L.cache_vs, S.smax, S.t_dev, S.pages, S.pages_stride,
+                                          S.cache_rows, wo, stream);
     } else {
         st = qkv_direct ? smh_rope_append_kv(b.q, b.k, b.v, M, L.heads, L.kv_heads, 128, S.cos_tab, S.sin_tab, S.pos_dev, L.cache_k, L.cache_ks, L.cache_v,
                                              L.cache_vs, S.smax, S.t_dev, stream)
@@ -209,8 +221,9 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
     if ((st = run.residual_linear(b.att, nq, run.w_o))) return st;
     // ---- feed forward ----
     if (S.swiglu_in != 0 && smh_q40_swiglu_fits(M, L.dim, L.ffn)) {
-        if ((st = run.norm(L.ffn_norm, L.ffn_eps))) return st;
-        if ((st = smh_q40_matmul_tiled_swiglu(b.xn, M, L.dim, L.dim, L.w1, L.w3, L.ffn, b.act, L.ffn, stream))) return st;
+        if ((st = run.norm(L.ffn_norm, L.ffn_eps, ask(L, M, L.dim, 2, run.w_gu, run.n_gu, true, WARM_FROM_NORM, 256)))) return st;
+        const WarmWeights w2 = ask(L, M, L.ffn, 1, run.w_d, run.n_dim, false, WARM_FROM_SWIGLU, swiglu_idle(L.ffn));
+        if ((st = matmul_tiled_swiglu(b.xn, M, L.dim, L.dim, L.w1, L.w3, L.ffn, b.act, L.ffn, w2, stream))) return st;
         return run.residual_linear(b.act, L.ffn, run.w_d);
     }
     if ((st = norm_linears(L.ffn_norm, L.ffn_eps, 2, run.w_gu, run.n_gu))) return st;

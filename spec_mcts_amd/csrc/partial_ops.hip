@@ -10,7 +10,9 @@
 //   partial_rope_append_kernel q,k,v = fp16(acc); RoPE(q,k); Q4_0 append of k,v to the suffix cache
 // so a decode layer is 4 weight-streaming launches plus these small ones, and no kernel ever waits
 // for another workgroup.
-#include "q40_matmul.hpp"
+#include <climits>
+
+#include "q40_warm.hpp"
 #include "rope_kv.hpp"
 #include "slab_sum.hpp"
 
@@ -40,16 +42,27 @@ __global__ __launch_bounds__(256) void partial_reduce_kernel(const void *__restr
     *reinterpret_cast<h4 *>(c + (long)m * ldc + n) = out;
 }
 
+struct Nothing {};
+
 // ---- residual add + RMSNorm ---------------------------------------------------------------------
 // one workgroup of 1024 threads per row; h_out = h_in + fp16(acc) (fp16 add), xn = fp16(fp16(h*r)*w)
 // A chain of trips to memory bounds it, so everything is requested before the first sum: KS slabs (0: none), PASSES passes of four
 // columns a thread, the residual and the norm's weights.  Up to 64 registers two workgroups share a compute unit.
-template <int PASSES, int KS>
+// Grid (rows, 1); ASK: (rows, 1 and as many times more as make next.workgroups, which ask for the next launch's weights: q40_warm.hpp).
+// (ASK: a kernel of its own, as the others have fewer arguments and a shorter way to their first load)
+template <int PASSES, int KS, bool ASK = false>
 __global__ __launch_bounds__(1024, PASSES * KS <= 8 ? 8 : 4) void partial_rmsnorm_kernel(const void *__restrict__ partial, int ks, int M, int N,
                                                                const half_t *__restrict__ h_in, const half_t *__restrict__ wt,
-                                                               float eps, half_t *__restrict__ h_out, half_t *__restrict__ xn_out) {
+                                                               float eps, half_t *__restrict__ h_out, half_t *__restrict__ xn_out,
+                                                               std::conditional_t<ASK, WarmWeights, Nothing> next) {
     __shared__ float s_part[16];
     const int m = blockIdx.x;
+    if constexpr (ASK) {
+        if (__builtin_expect(blockIdx.y > 0, 0)) {                 // (known without an argument: a row's workgroup asks for all of them at once)
+            const int e = ((int)blockIdx.y - 1) * M + m;
+            return warm_weights(next, (M + e) & 7, e >> 3, threadIdx.x, 1024);
+        }
+    }
     const long slab = (long)M * N;
     float ss = 0.f;
     // each thread owns columns 4t, 4t+1, 4t+2, 4t+3 (+ 4096 per pass); values kept for the second pass
@@ -313,13 +326,17 @@ using namespace smh;
 static_assert(SMH_MAX_KSPLIT == 16, "tables");
 #define BY_SLABS(k, ...) {__VA_ARGS__, k(1), k(2), k(3), k(4), k(5), k(6), k(8), k(8), k(10), k(10), k(12), k(12), k(16), k(16), k(16), k(16)}
 typedef void (*reduce_kernel_t)(const void *, int, int, int, int, int, int, half_t *, long, const half_t *, long);
-typedef void (*rmsnorm_kernel_t)(const void *, int, int, int, const half_t *, const half_t *, float, half_t *, half_t *);
+typedef void (*rmsnorm_kernel_t)(const void *, int, int, int, const half_t *, const half_t *, float, half_t *, half_t *, Nothing);
+typedef void (*rmsnorm_ask_t)(const void *, int, int, int, const half_t *, const half_t *, float, half_t *, half_t *, WarmWeights);
 typedef void (*sumsq_kernel_t)(const void *, int, int, int, const half_t *, half_t *, float *);
 #define K_OF(n) partial_reduce_kernel<n, RES>
 template <int RES> static const reduce_kernel_t REDUCE_KERNELS[17] = BY_SLABS(K_OF, nullptr);
 #undef K_OF
 #define K_OF(n) partial_rmsnorm_kernel<PASSES, n>
 template <int PASSES> static const rmsnorm_kernel_t RMSNORM_KERNELS[17] = BY_SLABS(K_OF, K_OF(0));
+#undef K_OF
+#define K_OF(n) partial_rmsnorm_kernel<PASSES, n, true>
+template <int PASSES> static const rmsnorm_ask_t RMSNORM_ASK_KERNELS[17] = BY_SLABS(K_OF, nullptr);
 #undef K_OF
 #define K_OF(n) partial_residual_sumsq_kernel<PASSES, n>
 template <int PASSES> static const sumsq_kernel_t SUMSQ_KERNELS[17] = BY_SLABS(K_OF, nullptr);
@@ -372,8 +389,8 @@ extern "C" int smh_q40_matmul_columns(int M, int K, int N) {
 
 extern "C" int smh_q40_swiglu_fits(int M, int K, int n_half) { return smh::gemm_swiglu_fits(M, K, n_half, true) ? 1 : 0; }
 
-extern "C" int smh_q40_matmul_tiled_swiglu(const void *a, int M, int K, long lda, const void *tiled_gate, const void *tiled_up, int n_half,
-                                           void *out, long ldo, smh_stream_t stream) {
+int smh::matmul_tiled_swiglu(const void *a, int M, int K, long lda, const void *tiled_gate, const void *tiled_up, int n_half, void *out, long ldo,
+                             const WarmWeights &next, smh_stream_t stream) {
     const char *who = "smh_q40_matmul_tiled_swiglu";
     SMH_REQUIRE(gemm_swiglu_fits(M, K, n_half, false),
                 "%s: M=%d (17 .. 128) K=%d (a multiple of 64) n_half=%d (a multiple of 128, at most 16384); or M above 128 and K a multiple of 32", who, M, K, n_half);
@@ -386,7 +403,54 @@ extern "C" int smh_q40_matmul_tiled_swiglu(const void *a, int M, int K, long lda
     p.seg[0].w = (const uint8_t *)tiled_gate; p.seg[0].N = n_half;
     p.seg[1].w = (const uint8_t *)tiled_up; p.seg[1].N = n_half;
     p.c = p.seg[0].c = (half_t *)out; p.ldc = p.seg[0].ldc = ldo; p.tiled = 1;
-    return M > 128 ? gemm_swiglu_rows_launch(p, (hipStream_t)stream) : gemm_swiglu_launch(p, (hipStream_t)stream);
+    return M > 128 ? gemm_swiglu_rows_launch(p, (hipStream_t)stream) : gemm_swiglu_launch(p, next, (hipStream_t)stream);
+}
+extern "C" int smh_q40_matmul_tiled_swiglu(const void *a, int M, int K, long lda, const void *tiled_gate, const void *tiled_up, int n_half,
+                                           void *out, long ldo, smh_stream_t stream) {
+    return matmul_tiled_swiglu(a, M, K, lda, tiled_gate, tiled_up, n_half, out, ldo, WarmWeights{}, stream);
+}
+
+WarmWeights smh::q40_warm(int M, int K, int nseg, const void *const *tiled, const int *n, bool swiglu, int stages, int workgroups) {
+    WarmWeights w = WarmWeights{};
+    MatmulParams p;
+    if (M <= SMH_GEMV_MAX_M || M > 128 || K % 64 != 0 || stages < 1) return w;
+    if (swiglu ? nseg != 2 || n[0] != n[1] || !gemm_swiglu_fits(M, K, n[0], false)
+               : fill_params(p, nullptr, M, K, K, nseg, nullptr, nullptr, n, "q40_warm", true) != 0 || p.kgroups != 2) return w;
+    for (int i = 0; i < nseg; ++i)
+        if (tiled[i] == nullptr || ((uintptr_t)tiled[i] & 127) != 0) return w;
+    for (int i = 0; i < SMH_MAX_SEGMENTS; ++i) {
+        w.w[i] = (const uint8_t *)tiled[min(i, nseg - 1)];
+        w.unit0[i] = swiglu || i >= nseg ? INT_MAX : p.seg[i].unit0;
+    }
+    w.units = swiglu ? n[0] / 128 : p.units;
+    w.units_pad = swiglu ? 0 : p.units_pad;
+    w.slices = swiglu ? 1 : p.ksplit;
+    w.steps = K / 32;
+    w.steps_per_slice = swiglu ? w.steps : p.steps_per_slice;
+    w.stages = stages;
+    w.swiglu = swiglu;
+    w.workgroups = min(workgroups, (warm_blocks(w) + 7) / 8 * 8);
+    return w;
+}
+
+extern "C" int smh_q40_warm_span(int M, int K, int nseg, const int *n, int swiglu, int stages, long *lines, long *first, long *end) {
+    SMH_REQUIRE(nseg >= 1 && nseg <= SMH_MAX_SEGMENTS && n && lines && first && end, "smh_q40_warm_span: nseg=%d or a null pointer", nseg);
+    const void *const some[SMH_MAX_SEGMENTS] = {(const void *)128, (const void *)128, (const void *)128};
+    const WarmWeights w = q40_warm(M, K, nseg, some, n, swiglu != 0, stages, 8);
+    for (int i = 0; i < nseg; ++i) { lines[i] = first[i] = end[i] = 0; }
+    for (int at = 0; w.workgroups > 0 && at < warm_blocks(w); ++at) {
+        WarmBlock b;
+        if (!warm_block(w, at, b)) continue;
+        for (int i = 0; i < min(w.stages, b.stages) * warm_lines(w); ++i) {
+            int sg;
+            const long off = warm_line(w, b, i, sg);
+            if (sg < 0 || sg >= nseg) { set_error("smh_q40_warm_span: weight %d of %d", sg, nseg); return -1; }
+            if (lines[sg] == 0 || off < first[sg]) first[sg] = off;
+            if (off + 128 > end[sg]) end[sg] = off + 128;
+            ++lines[sg];
+        }
+    }
+    return w.workgroups > 0 ? 1 : 0;
 }
 
 extern "C" int smh_q40_matmul_tiled_direct_fits(int M, int K, int nseg, const int *n) {
@@ -619,8 +683,8 @@ extern "C" int smh_q40_matmul(const void *a, int M, int K, long lda, const void 
     return matmul_fp16(a, M, K, lda, b_w, b_s, N, c, ldc, epilogue, residual, ldr, workspace, workspace_bytes, stream, "smh_q40_matmul", 0);
 }
 
-extern "C" int smh_partial_rmsnorm(const void *partial, int ksplit, int M, int N, const void *h_in, const void *weight, float eps,
-                                   void *h_out, void *xn_out, smh_stream_t stream) {
+int smh::partial_rmsnorm(const void *partial, int ksplit, int M, int N, const void *h_in, const void *weight, float eps, void *h_out, void *xn_out,
+                         const WarmWeights &next, smh_stream_t stream) {
     SMH_REQUIRE(partial == nullptr || (ksplit >= 1 && ksplit <= SMH_MAX_KSPLIT), "smh_partial_rmsnorm: ksplit=%d", ksplit);
     SMH_REQUIRE(M >= 0 && N > 0 && N % 4 == 0 && N <= 16384, "smh_partial_rmsnorm: M=%d N=%d (N must be a multiple of 4, <= 16384)", M, N);
     SMH_REQUIRE(partial != nullptr || h_in != nullptr, "smh_partial_rmsnorm: no input");
@@ -633,9 +697,19 @@ extern "C" int smh_partial_rmsnorm(const void *partial, int ksplit, int M, int N
     }
     const int ks = partial == nullptr ? 0 : ksplit;
     const auto kern = N <= 4096 ? RMSNORM_KERNELS<1>[ks] : N <= 8192 ? RMSNORM_KERNELS<2>[ks] : RMSNORM_KERNELS<4>[ks];
+    if (next.workgroups > 0 && ks > 0 && N <= 8192) {
+        const auto ask = N <= 4096 ? RMSNORM_ASK_KERNELS<1>[ks] : RMSNORM_ASK_KERNELS<2>[ks];
+        hipLaunchKernelGGL(ask, dim3(M, 1 + (next.workgroups + M - 1) / M), dim3(1024), 0, (hipStream_t)stream, partial, ks, M, N, (const half_t *)h_in,
+                           (const half_t *)weight, eps, (half_t *)h_out, (half_t *)xn_out, next);
+        return launch_status();
+    }
     hipLaunchKernelGGL(kern, dim3(M), dim3(1024), 0, (hipStream_t)stream, partial, ks, M, N, (const half_t *)h_in, (const half_t *)weight, eps, (half_t *)h_out,
-                       (half_t *)xn_out);
+                       (half_t *)xn_out, Nothing{});
     return launch_status();
+}
+extern "C" int smh_partial_rmsnorm(const void *partial, int ksplit, int M, int N, const void *h_in, const void *weight, float eps,
+                                   void *h_out, void *xn_out, smh_stream_t stream) {
+    return partial_rmsnorm(partial, ksplit, M, N, h_in, weight, eps, h_out, xn_out, WarmWeights{}, stream);
 }
 
 extern "C" int smh_partial_residual_sumsq(const void *partial, int ksplit, int M, int N, const void *h_in, void *h_out, void *sums,

@@ -26,7 +26,7 @@
 #include <type_traits>
 #include <utility>
 
-#include "q40_matmul.hpp"
+#include "q40_warm.hpp"
 
 namespace smh {
 
@@ -989,7 +989,7 @@ __global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_kg_kern
 // workgroup takes piece bp of block j of the GATE weight and the same piece of the UP weight (64 columns each, the same
 // columns), so its wave (kk, hh, gu) holds, after the K-groups are added, gate or up for exactly the columns its neighbour
 // holds the other for.  The epilogue forms fp16(silu(fp16(gate))) * fp16(up) with the roundings of partial_silu_mul_kernel
-// and stores the activations of w2: no slab leaves the launch and the SiLU launch is gone.
+// and stores the activations of w2: no slab leaves the launch and the SiLU launch is gone.  Workgroups past the columns ask for w2 (q40_warm.hpp).
 template <int TILES> struct SwigluShape {
     static constexpr int SC = 1024;                                  // scales: [group kk][gate | up] x 256
     static constexpr int STAGE = KG_W + SC + 2 * TILES * 1024;
@@ -1003,7 +1003,7 @@ template <int TILES> struct SwigluShape {
 };
 
 template <int TILES>
-__global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_swiglu_kernel(MatmulParams p) {
+__global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_swiglu_kernel(MatmulParams p, WarmWeights next) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     typedef SwigluShape<TILES> S;
     constexpr int SLOTS = S::SLOTS, PER = S::PER, STAGE = S::STAGE;
@@ -1016,7 +1016,7 @@ __global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_swiglu_
     const int blockj = hb >> 1, bp = hb & 1;
     const int pair = blockj >> 1, blk = blockj & 1;
     const int n_half = p.seg[0].N;
-    if (128 * blockj >= n_half) return;
+    if (__builtin_expect(128 * blockj >= n_half, 0)) return warm_weights(next, hb & 7, (hb - n_half / 64) >> 3, tid, 64 * (8 + GEMM_DMA_WAVES));
     constexpr int m0 = 0;
     const int n_st = p.K / 64;                                         // stages (two steps each), all of K
     const uint8_t *w_gate = p.seg[0].w + (long)pair * tiled_steps(p.K) * TILE_BYTES;
@@ -1630,8 +1630,10 @@ bool gemm_swiglu_fits(int M, int K, int n_half, bool worth_it) {
     return wgs <= 256 && (!worth_it || (wgs >= 128 && M > 32));
 }
 
-typedef void (*gemm_swiglu_kernel_t)(MatmulParams);
-int gemm_swiglu_launch(const MatmulParams &p, hipStream_t stream) {
+int swiglu_idle(int n_half) { return n_half / 64 < 256 ? (256 - n_half / 64) / 8 * 8 : 0; }
+
+typedef void (*gemm_swiglu_kernel_t)(MatmulParams, WarmWeights);
+int gemm_swiglu_launch(const MatmulParams &p, const WarmWeights &next, hipStream_t stream) {
     static const gemm_swiglu_kernel_t kern[9] = {nullptr, nullptr, q40_gemm_swiglu_kernel<2>, q40_gemm_swiglu_kernel<3>, q40_gemm_swiglu_kernel<4>,
                                                  q40_gemm_swiglu_kernel<5>, q40_gemm_swiglu_kernel<6>, q40_gemm_swiglu_kernel<7>,
                                                  q40_gemm_swiglu_kernel<8>};
@@ -1650,7 +1652,7 @@ int gemm_swiglu_launch(const MatmulParams &p, hipStream_t stream) {
     SMH_REQUIRE((long)p.M * p.lda * 2 < (1L << 32), "q40 gemm: M x lda = %d x %ld exceeds the 32-bit lane offsets of A", p.M, p.lda);
     int tiles = (p.M + 15) / 16;
     if (tiles < 2) tiles = 2;
-    hipLaunchKernelGGL(kern[tiles], dim3((unsigned)(2 * (p.seg[0].N / 128))), dim3(64 * (8 + GEMM_DMA_WAVES)), lds_bytes[tiles], stream, p);
+    hipLaunchKernelGGL(kern[tiles], dim3((unsigned)(2 * (p.seg[0].N / 128) + next.workgroups)), dim3(64 * (8 + GEMM_DMA_WAVES)), lds_bytes[tiles], stream, p, next);
     return launch_status();
 }
 

@@ -116,7 +116,8 @@ void gemm_fill_plan(MatmulParams &p);
 bool gemm_blocks_fit(const MatmulParams &p, MatmulParams &b);          // after gemm_fill_plan
 int gemm_launch(const MatmulParams &p, hipStream_t stream);
 bool gemm_swiglu_fits(int M, int K, int n_half, bool worth_it);
-int gemm_swiglu_launch(const MatmulParams &p, hipStream_t stream);     // seg[0] = gate, seg[1] = up (tiled), c / ldc = the activations
+struct WarmWeights;
+int gemm_swiglu_launch(const MatmulParams &p, const WarmWeights &next, hipStream_t stream);     // seg[0] = gate, seg[1] = up (tiled), c / ldc = the activations
 // more than 128 rows on tiled weights: can the launch write its fp16 results itself (no K-split, enough workgroups without one)
 bool gemm_direct_fits(const MatmulParams &p);
 // SiLU(gate) * up for more than 128 rows: seg[0] = gate, seg[1] = up (tiled), seg[0].c / ldc = the activations

@@ -252,3 +252,32 @@ def test_columns_of_a_workgroup_on_the_checkpoint_layout():
     assert columns(16, 4096, 4096) == 0 and columns(100, 4096, 100) < 0
     assert columns(17, 4096, 4096) == 128 and columns(100, 4096, 11008) == 256 and columns(512, 4096, 4096) == 128 and columns(512, 11008, 4096) == 256
     assert columns(100, 4096 + 32, 4096) == 256                # (half a stage past the end of K)
+
+
+@pytest.mark.parametrize("M,K,ns,swiglu", [(37, 4096, [4096, 4096, 4096], 0), (100, 4096, [4096], 0), (100, 11008, [4096], 0), (17, 4096, [4096], 0),
+                                           (128, 8192, [8192, 1024, 1024], 0), (64, 4096, [5248, 1152, 1152], 0), (48, 13824, [5120], 0),
+                                           (100, 4096, [11008, 11008], 1), (33, 5120, [13824, 13824], 1), (64, 64, [8320, 8320], 1)])
+def test_weights_asked_for_ahead_are_those_of_the_launch(M, K, ns, swiglu):
+    """a few stages stay inside the weights; all stages are every line of every tile once (the padded half of a last unit included)"""
+    from spec_mcts_amd import _lib
+    lib = _lib.load()
+    n = (ctypes.c_int * len(ns))(*ns)
+    out = [(ctypes.c_long * len(ns))() for _ in range(3)]
+    for stages in (1, 3, 16):
+        assert lib.smh_q40_warm_span(M, K, len(ns), n, swiglu, stages, *out) == 1
+        for i, N in enumerate(ns):
+            assert out[0][i] > 0 and 0 <= out[1][i] < out[2][i] <= lib.smh_q40_tiled_bytes(K, N)
+    assert lib.smh_q40_warm_span(M, K, len(ns), n, swiglu, 1 << 20, *out) == 1
+    for i, N in enumerate(ns):
+        # 34 lines a tile; its scales are asked for with each half of it (128-column blocks), with each piece (SwiGLU)
+        pieces, lines = (2 * (N // 128), 10) if swiglu else (2 * ((N + 255) // 256), 18)
+        assert out[0][i] == pieces * lines * (K // 32)
+        assert out[1][i] == 0 and (out[2][i] == lib.smh_q40_tiled_bytes(K, N) or N % 256)
+
+
+@pytest.mark.parametrize("M,K,ns,swiglu", [(16, 4096, [4096], 0), (129, 4096, [4096], 0), (100, 4096 + 32, [4096], 0), (32, 4096, [11008, 11008], 0),
+                                           (100, 28672, [8192], 0), (100, 8192, [28672, 28672], 1), (200, 4096, [11008, 11008], 1)])
+def test_nothing_is_asked_for_ahead_of_other_kernels(M, K, ns, swiglu):
+    from spec_mcts_amd import _lib
+    out = [(ctypes.c_long * len(ns))() for _ in range(3)]
+    assert _lib.load().smh_q40_warm_span(M, K, len(ns), (ctypes.c_int * len(ns))(*ns), swiglu, 3, *out) == 0
