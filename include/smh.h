@@ -148,6 +148,10 @@ int smh_q40_matmul_tiled_direct_fits(int M, int K, int nseg, const int *n);
 int smh_q40_matmul_tiled_direct_columns(int M, int K, int nseg, const int *n);
 int smh_q40_matmul_tiled_direct(const void *a, int M, int K, long lda, int nseg, const void *const *tiled, const int *n, void *const *out,
                                 const void *residual, long ldr, smh_stream_t stream);
+/* ... and RoPE (:166-203) in the same launch: the first rope_heads heads of 128 columns of the outputs laid end to end leave rotated, row m as position m of
+ * the tables [>= M, 64], which begin at multiples of 16 bytes; the same bits as smh_rope behind it. */
+int smh_q40_matmul_tiled_direct_rope(const void *a, int M, int K, long lda, int nseg, const void *const *tiled, const int *n, void *const *out,
+                                     int rope_heads, const void *cos_tab, const void *sin_tab, smh_stream_t stream);
 int smh_q40_matmul_partial(const void *a, int M, int K, long lda, int nseg, const void *const *w,
                            const void *const *s, const int *n, void *partial, size_t partial_bytes,
                            smh_stream_t stream);

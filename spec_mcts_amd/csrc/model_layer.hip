@@ -238,7 +238,7 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
 
 // One layer of a prefill of `rows` tokens (TransformerBlock.forward with start_pos == 0): k and v go straight to the prompt cache.
 // Above 128 rows the linears store their fp16 results themselves wherever their launch needs no K-split (the residual adds of
-// wo and w2 inside), and SiLU(gate) * up is made inside w1|w3's launch.
+// wo and w2 inside, and RoPE), and SiLU(gate) * up is made inside w1|w3's launch.
 extern "C" int smh_prefill_layer(const smh_layer *layer, smh_pass *pass, smh_stream_t stream) {
     const char *who = "smh_prefill_layer";
     SMH_REQUIRE(layer && pass && pass->h, "%s: null pointer", who);
@@ -252,8 +252,12 @@ extern "C" int smh_prefill_layer(const smh_layer *layer, smh_pass *pass, smh_str
     if ((st = run.norm(L.att_norm, L.att_eps))) return st;
     if (direct(M, L.dim, 3, run.n_qkv)) {
         void *out[3] = {b.q, L.prompt_k, L.prompt_v};
-        if ((st = smh_q40_matmul_tiled_direct(b.xn, M, L.dim, L.dim, 3, run.w_qkv, run.n_qkv, out, nullptr, 0, stream))) return st;
-        st = smh_rope(b.q, L.prompt_k, M, L.heads, L.kv_heads, 128, S.cos_tab, S.sin_tab, 0, stream);
+        if ((((uintptr_t)S.cos_tab | (uintptr_t)S.sin_tab) & 15) == 0 && M < 1 << 24) {
+            st = smh_q40_matmul_tiled_direct_rope(b.xn, M, L.dim, L.dim, 3, run.w_qkv, run.n_qkv, out, L.heads + L.kv_heads, S.cos_tab, S.sin_tab, stream);
+        } else {
+            if ((st = smh_q40_matmul_tiled_direct(b.xn, M, L.dim, L.dim, 3, run.w_qkv, run.n_qkv, out, nullptr, 0, stream))) return st;
+            st = smh_rope(b.q, L.prompt_k, M, L.heads, L.kv_heads, 128, S.cos_tab, S.sin_tab, 0, stream);
+        }
     } else {
         if ((st = smh_q40_matmul_partial_tiled(b.xn, M, L.dim, L.dim, 3, run.w_qkv, run.n_qkv, b.slab_a, b.slab_a_bytes, stream))) return st;
         st = smh_partial_rope_rows(b.slab_a, slices(M, L.dim, 3, run.n_qkv), M, L.heads, L.kv_heads, 128, b.q, L.prompt_k, L.prompt_v, S.cos_tab, S.sin_tab, 0,

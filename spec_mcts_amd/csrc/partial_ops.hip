@@ -477,9 +477,8 @@ static int swiglu_plan(int M, int K, int n_half, int (*ask)(MatmulParams)) {
 extern "C" int smh_q40_swiglu_columns(int M, int K, int n_half) { return swiglu_plan(M, K, n_half, gemm_swiglu_columns); }
 extern "C" int smh_q40_swiglu_first_columns(int M, int K, int n_half) { return swiglu_plan(M, K, n_half, gemm_swiglu_first_columns); }
 
-extern "C" int smh_q40_matmul_tiled_direct(const void *a, int M, int K, long lda, int nseg, const void *const *tiled, const int *n, void *const *out,
-                                           const void *residual, long ldr, smh_stream_t stream) {
-    const char *who = "smh_q40_matmul_tiled_direct";
+static int tiled_direct(const char *who, const void *a, int M, int K, long lda, int nseg, const void *const *tiled, const int *n, void *const *out,
+                        const void *residual, long ldr, int rope_heads, const void *cos_tab, const void *sin_tab, smh_stream_t stream) {
     MatmulParams p;
     const int st = fill_params(p, a, M, K, lda, nseg, tiled, nullptr, n, who, true);
     if (st) return st;
@@ -495,7 +494,27 @@ extern "C" int smh_q40_matmul_tiled_direct(const void *a, int M, int K, long lda
     p.epilogue = residual ? SMH_EPI_RESIDUAL : SMH_EPI_NONE;
     p.resid = (const half_t *)residual;
     p.ldr = ldr;
+    if (rope_heads > 0) {
+        p.rope_cols = 128 * rope_heads;
+        p.rope_cos = (const half_t *)cos_tab;
+        p.rope_sin = (const half_t *)sin_tab;
+    }
     return gemm_launch(p, (hipStream_t)stream);
+}
+extern "C" int smh_q40_matmul_tiled_direct(const void *a, int M, int K, long lda, int nseg, const void *const *tiled, const int *n, void *const *out,
+                                           const void *residual, long ldr, smh_stream_t stream) {
+    return tiled_direct("smh_q40_matmul_tiled_direct", a, M, K, lda, nseg, tiled, n, out, residual, ldr, 0, nullptr, nullptr, stream);
+}
+extern "C" int smh_q40_matmul_tiled_direct_rope(const void *a, int M, int K, long lda, int nseg, const void *const *tiled, const int *n, void *const *out,
+                                                int rope_heads, const void *cos_tab, const void *sin_tab, smh_stream_t stream) {
+    const char *who = "smh_q40_matmul_tiled_direct_rope";
+    long heads = 0;
+    SMH_REQUIRE(nseg >= 1 && nseg <= SMH_MAX_SEGMENTS && n, "%s: nseg=%d outside [1,%d]", who, nseg, SMH_MAX_SEGMENTS);
+    for (int i = 0; i < nseg; ++i) heads += n[i] / 128;
+    SMH_REQUIRE(rope_heads >= 1 && rope_heads <= heads && cos_tab && sin_tab && (((uintptr_t)cos_tab | (uintptr_t)sin_tab) & 15) == 0,
+                "%s: rope_heads=%d of %ld, or a null or misaligned table", who, rope_heads, heads);
+    SMH_REQUIRE(M < 1 << 24, "%s: M=%d (32-bit offsets of the tables)", who, M);
+    return tiled_direct(who, a, M, K, lda, nseg, tiled, n, out, nullptr, 0, rope_heads, cos_tab, sin_tab, stream);
 }
 
 extern "C" int smh_q40_matmul_plan_tiled(int M, int K, int nseg, const int *n) {

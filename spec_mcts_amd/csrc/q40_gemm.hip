@@ -118,6 +118,14 @@ __device__ __forceinline__ void gemm_feed(int n, Issue issue) {
     }
 }
 template <int N> using int_constant = std::integral_constant<int, N>;
+// f(int_constant<0>) .. f(int_constant<N - 1>)
+template <int N, class F>
+__device__ __forceinline__ void static_for(F f) {
+    if constexpr (N > 0) {
+        static_for<N - 1>(f);
+        f(int_constant<N - 1>{});
+    }
+}
 
 // What a multiplying wave reads of a stage's weights, and its operands out of that (gemm_decode): rows (2 j, 2 j + 1) of the piece's first
 // (o = 0) or second byte, the nibble (high: hh = 0, low) as fp16 code * scale.
@@ -314,7 +322,8 @@ __device__ __forceinline__ void gemm_multiply(const uint8_t *lds, int n, const W
 // tid_bias: zero (a range cut passes one the compiler cannot see, see there).
 // SWIGLU (eight waves, tiled): unit j is 128-column block j of the gate weight (seg[0], pieces 0 and 1 of a stage) next to block
 // j of the up weight (seg[1], pieces 2 and 3); all of K; the epilogue stores fp16(silu(fp16(gate))) * fp16(up).
-template <int TILES, bool RAGGED, bool TILED, int WAVES, int SLOTS, bool PRODUCER, bool SWIGLU = false>
+// ROTATE (direct products): p.rope_cos.
+template <int TILES, bool RAGGED, bool TILED, int WAVES, int SLOTS, bool PRODUCER, bool SWIGLU = false, bool ROTATE = false>
 __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int mb, int slice, int step0, int step1, bool zero_rest, bool more,
                                            int tid_bias) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -711,9 +720,28 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
     const int o_half = tid >> 8;                // eight waves: the second 256 threads store the second half of the columns
     const int o_lane = tid & 15;                // store q of this lane: columns 64q + 4*o_lane .. (fp16: 128q + 8*o_lane ..),
                                                 // so that one store instruction writes whole contiguous rows
+    // RoPE: the factors of this thread's eight dims, of three row tiles ahead
+    static_assert(!ROTATE || (TILED && WAVES == 8 && !SWIGLU), "heads in whole runs of eight columns");
+    const bool rotate = ROTATE && seg.col0 < p.rope_cols;
+    constexpr int FAR = 3;
+    h8 cs[ROTATE ? TILES : 1], sn[ROTATE ? TILES : 1];
+    auto factors = [&](auto at) {
+        constexpr int T = decltype(at)::value;
+        if constexpr (ROTATE && T < TILES) {
+            const uint32_t at_ = (uint32_t)(min(m0 + 16 * T + o_row, p.M - 1) * 128 + 16 * (o_lane & 7));
+            cs[T] = *reinterpret_cast<const h8 *>(reinterpret_cast<const uint8_t *>(p.rope_cos) + at_);
+            sn[T] = *reinterpret_cast<const h8 *>(reinterpret_cast<const uint8_t *>(p.rope_sin) + at_);
+        }
+    };
+    if (rotate) {
+        factors(int_constant<0>{});
+        factors(int_constant<1>{});
+        factors(int_constant<2>{});
+    }
     gemm_barrier();                             // every wave has left the main loop: the ring is free
-#pragma unroll
-    for (int t = 0; t < TILES; ++t) {
+    static_for<TILES>([&](auto at) {
+        constexpr int t = decltype(at)::value;
+        if (rotate) factors(int_constant<t + FAR>{});
         float *otile = reinterpret_cast<float *>(lds + (t & 1) * OTILE_BYTES);
         // operands o and o + 2 are neighbouring columns: one 8-byte LDS store for the pair
         if constexpr (WAVES == 8) {
@@ -743,7 +771,7 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
                     }
                     *reinterpret_cast<h4 *>(seg.c + (long)mr * seg.ldc + col0 + cq) = o;
                 }
-            } else if (p.direct) {
+            } else if (ROTATE || p.direct) {
 #pragma unroll
                 for (int q = (WAVES == 8 ? o_half : 0); q < (WAVES == 8 ? o_half + 1 : 2); ++q) {
                     const int n_seg = col0 + 128 * q + 8 * o_lane;
@@ -752,10 +780,18 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
                         const f4 v0 = *reinterpret_cast<const f4 *>(otile + o_row * OP + 128 * q + 8 * o_lane);
                         const f4 v1 = *reinterpret_cast<const f4 *>(otile + o_row * OP + 128 * q + 8 * o_lane + 4);
                         h8 o;
+                        if (rotate && n < p.rope_cols) {
+                            if constexpr (ROTATE) {
+                                const float *there = otile + o_row * OP + 128 * q + 8 * (o_lane ^ 8);
+                                const f4 u0 = *reinterpret_cast<const f4 *>(there), u1 = *reinterpret_cast<const f4 *>(there + 4);
+                                o = rope_eight(v0, v1, u0, u1, o_lane >= 8, cs[t], sn[t]);
+                            }
+                        } else {
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            o[e] = matmul_epilogue(p, v0[e], m, n + e);
-                            o[4 + e] = matmul_epilogue(p, v1[e], m, n + 4 + e);
+                            for (int e = 0; e < 4; ++e) {
+                                o[e] = matmul_epilogue(p, v0[e], m, n + e);
+                                o[4 + e] = matmul_epilogue(p, v1[e], m, n + 4 + e);
+                            }
                         }
                         *reinterpret_cast<h8 *>(seg.c + (long)m * seg.ldc + n_seg) = o;
                     }
@@ -769,7 +805,7 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
                 }
             }
         }
-    }
+    });
     if (zero_rest) {
         for (int sl = slice + 1; sl < p.ksplit; ++sl) {
             float *zslab = p.partial + (long)sl * p.M * p.n_total;
@@ -796,7 +832,7 @@ __device__ __forceinline__ void gemm_piece(const MatmulParams &p, int unit, int 
 // what the kernel needs).  SLOTS: slots of the ring.
 // RANGE (p.chunk > 0): the steps of all column units, laid end to end, are dealt in runs of p.chunk to the workgroups, one
 // workgroup per compute unit, so a workgroup may finish one unit and begin the next: up to two pieces, one after the other.
-template <int TILES, bool RAGGED, bool TILED, int WAVES, int SLOTS = GEMM_STAGES, bool PRODUCER = false, bool RANGE = false, bool SWIGLU = false>
+template <int TILES, bool RAGGED, bool TILED, int WAVES, int SLOTS = GEMM_STAGES, bool PRODUCER = false, bool RANGE = false, bool SWIGLU = false, bool ROTATE = false>
 // (SWIGLU without the DMA waves: at most 128 registers, so that two workgroups of eight waves fit a compute unit)
 __global__ __launch_bounds__(64 * (WAVES + (PRODUCER ? GEMM_DMA_WAVES : 0)), WAVES == 8 ? (SWIGLU && !PRODUCER ? 4 : 1) : 2) void q40_gemm_kernel(MatmulParams p) {
     static_assert(WAVES == 4 || (WAVES == 8 && (TILED ? !RAGGED : PRODUCER)), "eight waves: K a multiple of 32, or the checkpoint layout with the DMA waves");
@@ -828,7 +864,7 @@ __global__ __launch_bounds__(64 * (WAVES + (PRODUCER ? GEMM_DMA_WAVES : 0)), WAV
         const int mb = p.mb0 + (int)blockIdx.y;
         const int slice = blockIdx.z;
         const int s0 = slice * p.steps_per_slice;
-        gemm_piece<TILES, RAGGED, TILED, WAVES, SLOTS, PRODUCER, SWIGLU>(p, unit, mb, slice, s0, min(s0 + p.steps_per_slice, steps_total), false, false, 0);
+        gemm_piece<TILES, RAGGED, TILED, WAVES, SLOTS, PRODUCER, SWIGLU, ROTATE>(p, unit, mb, slice, s0, min(s0 + p.steps_per_slice, steps_total), false, false, 0);
     }
 }
 
@@ -1119,7 +1155,10 @@ template <int TILES, int MODE> struct WideShape {
     static constexpr int OTILE = (MODE == WIDE_SWIGLU ? 2 : 1) * 16 * OP * 4;      // [16][OP] fp32; SwiGLU: [gate | up][16][OP]
     static constexpr int SUMS = TILES * 16 * OP * 4;             // two K-groups: [row][OP] fp32
     static constexpr int OUT = MODE == WIDE_GROUPS ? SUMS : 2 * OTILE;
-    static constexpr int LDS = SLOTS * STAGE > OUT ? SLOTS * STAGE : OUT;
+    // RoPE: the rows' cosines, then their sines (128 bytes each), behind the sums, where the ring was, or (WIDE_SIX) behind the ring
+    static constexpr int ROPE = MODE == WIDE_SIX ? SLOTS * STAGE : OUT, ROPE_END = MODE == WIDE_SWIGLU ? 0 : ROPE + TILES * 4096;
+    static constexpr int LDS = SLOTS * STAGE > OUT ? (SLOTS * STAGE > ROPE_END ? SLOTS * STAGE : ROPE_END) : OUT > ROPE_END ? OUT : ROPE_END;
+    static_assert(ROPE % 16 == 0 && 2 * OTILE <= SLOTS * STAGE, "factors are brought by DMA");
     static_assert(LDS <= 160 * 1024, "ring");
 };
 constexpr int WIDE_WAVES = 12;
@@ -1199,9 +1238,28 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + GEMM_DMA_WAVES), 1) void q40_gem
         };
         if (wave == WIDE_WAVES) feed(int_constant<0>{});
         else feed(int_constant<1>{});
+        // RoPE: the factors of the workgroup's rows, cosines by one wave, sines by the other (eight rows an instruction)
+        const bool rotate = !SWIGLU && p.rope_cos != nullptr;
+        auto bring_factors = [&] {
+            const uint8_t *tab = reinterpret_cast<const uint8_t *>(wave == WIDE_WAVES ? p.rope_cos : p.rope_sin);
+            uint8_t *to = lds + S::ROPE + (wave == WIDE_WAVES ? 0 : TILES * 2048);
+#pragma unroll
+            for (int i = 0; i < 2 * TILES; ++i)
+                __builtin_amdgcn_global_load_lds((gptr_t)(tab + (uint32_t)(min(m0 + 8 * i + (lane >> 3), p.M - 1) * 128 + 16 * (lane & 7))), (lptr_t)(to + i * 1024), 16, 0, 0);
+        };
         // the barriers of the epilogue: ring free, one per row tile; ring free, the second group's sums in place, all sums
+        if constexpr (MODE == WIDE_GROUPS) {
+            gemm_barrier();
+            if (rotate) bring_factors();
+            gemm_barrier();
+            gemm_wait_vm<0>();
+            gemm_barrier();
+        } else {
+            if (MODE == WIDE_SIX && rotate) bring_factors();           // (under the last stages)
+            gemm_wait_vm<0>();
 #pragma unroll 1
-        for (int t = 0; t < (MODE == WIDE_GROUPS ? 3 : 1 + TILES); ++t) gemm_barrier();
+            for (int t = 0; t < 1 + TILES; ++t) gemm_barrier();
+        }
         return;
     }
 
@@ -1222,6 +1280,23 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + GEMM_DMA_WAVES), 1) void q40_gem
     const int sg = segment_of(P), out_col = 128 * (P >> 1) + 64 * (q >> 3) + 8 * (q & 7) + 2 * (P & 1);
     half_t *const out = (sg == 0 ? p.seg[0].c : sg == 1 ? p.seg[1].c : p.seg[2].c) + out_col;
     const long ldc = sg == 0 ? p.seg[0].ldc : sg == 1 ? p.seg[1].ldc : p.seg[2].ldc;
+    const bool rotate = !SWIGLU && p.rope_cos != nullptr;
+    // four sums of row r of the workgroup, with the residual or rotated, to columns n_, n_ + 1, n_ + 4 and n_ + 5 (dims 8 (q % 8) + 2 (piece % 2) + 0, 1, 4, 5)
+    auto store = [&](const float *row_sums, int piece, int n_, int m, int r, half_t *dst) {
+        const f4 v = *reinterpret_cast<const f4 *>(row_sums + 4 * o_lane);
+        h2 lo, hi;
+        if (rotate && n_ < p.rope_cols) {
+            const f4 u = *reinterpret_cast<const f4 *>(row_sums + 4 * (o_lane ^ 8));
+            const half_t *cs = reinterpret_cast<const half_t *>(lds + S::ROPE) + r * 64 + 8 * (q & 7) + 2 * (piece & 1), *sn = cs + TILES * 1024;
+            rope_pairs(v, u, (q & 8) != 0, *reinterpret_cast<const h2 *>(cs), *reinterpret_cast<const h2 *>(cs + 4), *reinterpret_cast<const h2 *>(sn),
+                       *reinterpret_cast<const h2 *>(sn + 4), lo, hi);
+        } else {
+            lo = h2{matmul_epilogue(p, v[0], m, n_), matmul_epilogue(p, v[1], m, n_ + 1)};
+            hi = h2{matmul_epilogue(p, v[2], m, n_ + 4), matmul_epilogue(p, v[3], m, n_ + 5)};
+        }
+        *reinterpret_cast<h2 *>(dst) = lo;
+        *reinterpret_cast<h2 *>(dst + 4) = hi;
+    };
     gemm_barrier();                                            // every wave has left the loop: the ring is free
     if constexpr (SWIGLU) {
 #pragma unroll
@@ -1260,16 +1335,8 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + GEMM_DMA_WAVES), 1) void q40_gem
             for (int r = 0; r < 4; ++r) *reinterpret_cast<f2 *>(&otile[(4 * g + r) * OP + 64 * k3 + 32 * hh + 2 * c]) = f2{acc[0][t][r], acc[1][t][r]};
             gemm_barrier();
             const int m = m0 + 16 * t + o_row;
-            if (m < p.M && mine) {
-                const f4 v = *reinterpret_cast<const f4 *>(otile + o_row * OP + 4 * o_lane);
-                *reinterpret_cast<h2 *>(out + (long)m * ldc) = h2{matmul_epilogue(p, v[0], m, n), matmul_epilogue(p, v[1], m, n + 1)};
-                *reinterpret_cast<h2 *>(out + (long)m * ldc + 4) = h2{matmul_epilogue(p, v[2], m, n + 4), matmul_epilogue(p, v[3], m, n + 5)};
-            }
-            if (m < p.M && mine2) {
-                const f4 v = *reinterpret_cast<const f4 *>(otile + o_row * OP + 192 + 4 * o_lane);
-                *reinterpret_cast<h2 *>(out2 + (long)m * ldc2) = h2{matmul_epilogue(p, v[0], m, n2), matmul_epilogue(p, v[1], m, n2 + 1)};
-                *reinterpret_cast<h2 *>(out2 + (long)m * ldc2 + 4) = h2{matmul_epilogue(p, v[2], m, n2 + 4), matmul_epilogue(p, v[3], m, n2 + 5)};
-            }
+            if (m < p.M && mine) store(otile + o_row * OP, P, n, m, 16 * t + o_row, out + (long)m * ldc);
+            if (m < p.M && mine2) store(otile + o_row * OP + 192, P2, n2, m, 16 * t + o_row, out2 + (long)m * ldc2);
         }
     } else {
         // the second K-group's sums, then both groups' (in their order), then whole rows
@@ -1296,11 +1363,7 @@ __global__ __launch_bounds__(64 * (WIDE_WAVES + GEMM_DMA_WAVES), 1) void q40_gem
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
             const int m = m0 + 16 * t + o_row;
-            if (m < p.M && mine) {
-                const f4 v = *reinterpret_cast<const f4 *>(reinterpret_cast<const float *>(lds) + (16 * t + o_row) * OP + 4 * o_lane);
-                *reinterpret_cast<h2 *>(out + (long)m * ldc) = h2{matmul_epilogue(p, v[0], m, n), matmul_epilogue(p, v[1], m, n + 1)};
-                *reinterpret_cast<h2 *>(out + (long)m * ldc + 4) = h2{matmul_epilogue(p, v[2], m, n + 4), matmul_epilogue(p, v[3], m, n + 5)};
-            }
+            if (m < p.M && mine) store(reinterpret_cast<const float *>(lds) + (16 * t + o_row) * OP, P, n, m, 16 * t + o_row, out + (long)m * ldc);
         }
     }
 }
@@ -1506,6 +1569,13 @@ static int gemm_launch_layout(const MatmulParams &p, hipStream_t stream) {
         q40_gemm_kernel<3, false, TILED, WD, gemm_dma_slots(3), true, true>, q40_gemm_kernel<4, false, TILED, WD, gemm_dma_slots(4), true, true>,
         q40_gemm_kernel<5, false, TILED, WD, gemm_dma_slots(5), true, true>, q40_gemm_kernel<6, false, TILED, WD, gemm_dma_slots(6), true, true>,
         q40_gemm_kernel<7, false, TILED, WD, gemm_dma_slots(7), true, true>, q40_gemm_kernel<8, false, TILED, WD, gemm_dma_slots(8), true, true>};
+    // blocks of 64 .. 128 rows with RoPE (a kernel of its own: with the factors' registers in the others' epilogue three layers of a 70B shape took 1.2 % longer at 384 rows)
+    static const gemm_kernel_t rotate[2][5] = {{q40_gemm_kernel<4, false, true, WD, GEMM_STAGES, false, false, false, true>, q40_gemm_kernel<5, false, true, WD, GEMM_STAGES, false, false, false, true>,
+                                                q40_gemm_kernel<6, false, true, WD, GEMM_STAGES, false, false, false, true>, q40_gemm_kernel<7, false, true, WD, GEMM_STAGES, false, false, false, true>,
+                                                q40_gemm_kernel<8, false, true, WD, GEMM_STAGES, false, false, false, true>},
+                                               {q40_gemm_kernel<4, false, true, WD, gemm_dma_slots(4), true, false, false, true>, q40_gemm_kernel<5, false, true, WD, gemm_dma_slots(5), true, false, false, true>,
+                                                q40_gemm_kernel<6, false, true, WD, gemm_dma_slots(6), true, false, false, true>, q40_gemm_kernel<7, false, true, WD, gemm_dma_slots(7), true, false, false, true>,
+                                                q40_gemm_kernel<8, false, true, WD, gemm_dma_slots(8), true, false, false, true>}};
     // K not a multiple of 32: on tiled weights one kernel for all row counts, on the checkpoint layout the two forms from above with
     // a masked last step (against one four-wave kernel of eight row tiles: 33
     // rows x 11008 x 4072 29.7 -> 19.4 us, 100 rows 34.5 -> 27.6, 20 x 28672 x 8200 103 -> 53, 512 x 4096 x 4104 50 -> 40)
@@ -1526,6 +1596,8 @@ static int gemm_launch_layout(const MatmulParams &p, hipStream_t stream) {
                                                           {range_cut[t], gemm_dma_slots(t) * GS_BYTES}, {ragged_dma_wave[t], gemm_dma_slots(t) * GS_BYTES}};
             for (int i = 0; i < 5 && e == hipSuccess; ++i)
                 e = hipFuncSetAttribute((const void *)all[i].first, hipFuncAttributeMaxDynamicSharedMemorySize, all[i].second);
+            for (int i = 0; TILED && t >= 4 && i < 2 && e == hipSuccess; ++i)
+                e = hipFuncSetAttribute((const void *)rotate[i][t - 4], hipFuncAttributeMaxDynamicSharedMemorySize, i == 0 ? GEMM_LDS : gemm_dma_slots(t) * GS_BYTES);
         }
         return e;
     }();
@@ -1543,7 +1615,7 @@ static int gemm_launch_layout(const MatmulParams &p, hipStream_t stream) {
     const bool crowded = !TILED && (long)(p.units_pad / 8) * p.mblocks * p.ksplit > GEMM_DMA_WAVE_MAX_WGS / 8 && p.steps_per_slice <= 24;
     const bool one_each = !(TILED && odd_k) && (p.chunk > 0 || ((long)p.units * p.mblocks * p.ksplit <= GEMM_DMA_WAVE_MAX_WGS && !crowded));
     const bool four = odd_k ? !one_each : !TILED && !one_each;
-    const gemm_kernel_t kern = odd_k ? (TILED ? ragged : (one_each ? ragged_dma_wave : ragged_four)[tiles])
+    const gemm_kernel_t kern = p.rope_cos != nullptr ? rotate[one_each][p.block_rows / 16 - 4] : odd_k ? (TILED ? ragged : (one_each ? ragged_dma_wave : ragged_four)[tiles])
                                      : (p.chunk > 0 ? range_cut : one_each ? with_dma_wave : exact)[tiles];
     const long total_steps = (long)p.units * ((p.K + 31) / 32);
     const int lds = one_each ? gemm_dma_slots(tiles) * GS_BYTES : GEMM_LDS, threads = one_each ? 64 * (WD + GEMM_DMA_WAVES) : four ? GEMM_THREADS : 64 * W;

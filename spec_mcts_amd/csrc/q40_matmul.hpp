@@ -78,6 +78,11 @@ struct MatmulParams {
     const half_t *norm_w;
     const float *norm_ss;
     float norm_eps;
+    // GEMM, direct on tiled weights: columns [0, rope_cols) of the outputs laid end to end are heads of 128 that leave rotated, row m at position m
+    // (in the place of rope_kernel behind it, 5.7 us at 512 rows and 12.6 at 2047 of the 7B shape; a prefill of 384 / 512 / 1024 / 2047 rows 6707 / 7912 / 14451 / 26706
+    // -> 6572 / 7757 / 14240 / 26392 us.  With the factors loaded by the storing threads, not brought by the DMA waves, the wide kernels gained half of that.)
+    int rope_cols;
+    const half_t *rope_cos, *rope_sin;         // [position][64]
 };
 
 // p.seg[sg] without a load that waits for sg.  GLOBAL: the kernel stores through c (held_global); one that does not schedules its first loads better
@@ -107,6 +112,26 @@ __device__ __forceinline__ half_t matmul_epilogue(const MatmulParams &p, float a
     half_t v = (half_t)acc;
     if (p.epilogue == SMH_EPI_RESIDUAL) v = (half_t)((float)p.resid[(long)m * p.ldr + n] + (float)v);
     return v;
+}
+
+// RoPE in an epilogue: four sums of a head's lower or upper half, those of the same dims of its other half, and the dims' factors in pairs.  Rounded to fp16
+// before the rotation and in it as rope_kernel does.
+__device__ __forceinline__ void rope_pairs(f4 mine, f4 other, bool upper, h2 cs0, h2 cs1, h2 sn0, h2 sn1, h2 &lo, h2 &hi) {
+#pragma clang fp contract(off)
+    const uint32_t sign = upper ? 0u : 0x80008000u;
+    auto turn = [&](float x0, float x1, float y0, float y1, h2 cs, h2 sn) {
+        const h2 x = {(half_t)x0, (half_t)x1}, y = {(half_t)y0, (half_t)y1};
+        const h2 a = x * cs, b = as_h2(as_u32(y) ^ sign) * sn;
+        return a + b;
+    };
+    lo = turn(mine[0], mine[1], other[0], other[1], cs0, sn0);
+    hi = turn(mine[2], mine[3], other[2], other[3], cs1, sn1);
+}
+__device__ __forceinline__ h8 rope_eight(f4 mine0, f4 mine1, f4 other0, f4 other1, bool upper, h8 cs, h8 sn) {
+    h2 o[4];
+    rope_pairs(mine0, other0, upper, h2{cs[0], cs[1]}, h2{cs[2], cs[3]}, h2{sn[0], sn[1]}, h2{sn[2], sn[3]}, o[0], o[1]);
+    rope_pairs(mine1, other1, upper, h2{cs[4], cs[5]}, h2{cs[6], cs[7]}, h2{sn[4], sn[5]}, h2{sn[6], sn[7]}, o[2], o[3]);
+    return h8{o[0].x, o[0].y, o[1].x, o[1].y, o[2].x, o[2].y, o[3].x, o[3].y};
 }
 
 void gemv_fill_plan(MatmulParams &p);

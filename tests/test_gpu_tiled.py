@@ -375,6 +375,41 @@ def test_wide_workgroups(M, K, ns, columns):
             assert torch.equal(o_r.cpu(), (r.float() + o.cpu().float()).half())
 
 
+@pytest.mark.parametrize("M,K,ns,columns,heads", [(400, 4096, [4096, 4096, 4096], 192, 64),       # wq|wk|wv: the values stay
+                                                  (512, 704, [7040, 128, 896], 192, 56),          # up to a weight's end
+                                                  (512, 704, [7040, 128, 896], 192, 60),          # up to the middle of one
+                                                  (1024, 64, [4096, 4096, 4096], 384, 64),
+                                                  (700, 32, [5120, 128, 5120], 384, 41),
+                                                  (700, 32, [5120, 128, 5120], 384, 81),          # all of them
+                                                  (600, 256, [4096, 4096, 4096], 256, 64),        # 256 columns a workgroup
+                                                  (1100, 128, [8192, 1024, 1024], 256, 72),
+                                                  (400, 128, [4096, 4096, 4096], 256, 96),
+                                                  (513, 64, [4096, 128, 4096], 256, 40)])
+def test_rope_in_the_launch_of_the_product(M, K, ns, columns, heads):
+    """the bits of the rotation behind the product (smh_rope), columns behind the heads as they were"""
+    from spec_mcts_amd import _lib, kernels as Kn
+    lib = _lib.load()
+    na = (ctypes.c_int * len(ns))(*ns)
+    assert lib.smh_q40_matmul_tiled_direct_columns(M, K, len(ns), na) == columns
+    g = torch.Generator(device="cuda").manual_seed(M + heads)
+    tiled = [Kn.tile_q40(*Kn.quantize_q40(torch.randn((K, n), device="cuda", generator=g, dtype=torch.float16) * 0.1), K, n) for n in ns]
+    a = torch.randn((M, K), device="cuda", generator=g, dtype=torch.float16)
+    a[M // 2, 0] = float("inf")
+    a[M - 1, K - 1] = float("nan")
+    tabs = torch.randn((2, M * 64), device="cuda", generator=g, dtype=torch.float16)
+    out = [torch.empty((M, n), device="cuda", dtype=torch.float16) for n in ns]
+    Kn.check(lib.smh_q40_matmul_tiled_direct_rope(a.data_ptr(), M, K, K, len(ns), (ctypes.c_void_p * len(ns))(*[t.buf.data_ptr() for t in tiled]), na,
+                                                  (ctypes.c_void_p * len(ns))(*[o.data_ptr() for o in out]), heads, tabs[0].data_ptr(), tabs[1].data_ptr(),
+                                                  Kn._stream()), "smh_q40_matmul_tiled_direct_rope")
+    plain = torch.cat(Kn.matmul_q40_direct(a, tiled), dim=1)
+    q, k = plain[:, :128 * (heads - 1)].contiguous(), plain[:, 128 * (heads - 1):128 * heads].contiguous()
+    Kn.check(lib.smh_rope(q.data_ptr(), k.data_ptr(), M, heads - 1, 1, 128, tabs[0].data_ptr(), tabs[1].data_ptr(), 0, Kn._stream()), "smh_rope")
+    want = torch.cat((q, k, plain[:, 128 * heads:]), dim=1)
+    got = torch.cat(out, dim=1)
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.nan_to_num(0.0).view(torch.int16), want.nan_to_num(0.0).view(torch.int16))
+
+
 @pytest.mark.parametrize("M,K,n_half,first", [(430, 256, 18560, 10752), (512, 128, 28672, 12288), (500, 1056, 18560, 10752), (866, 512, 14336, 6144)])
 def test_swiglu_in_two_launches_where_the_last_round_is_a_poor_one(M, K, n_half, first):
     """Workgroups of three pieces of each weight for most columns, of two for the rest: what one weight's columns after the other give in 64 bits, to the
