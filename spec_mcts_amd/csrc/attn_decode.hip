@@ -1992,6 +1992,12 @@ static int attn_plan_tw(int P, int Hkv) {
     return tw;
 }
 
+// The one-launch kernel.  From 32 kv heads on slices of ATT_ONE_TW rows, also where narrower ones would give each compute unit one: what they leave to the
+// merge, and the second wave of a query's own rows that they take the place of, cost more (us a step of the 7B architecture, slices of 32 rows and of 64, 10 / 60 / 120
+// rows of their own: 5 branches behind 100 rows 1905 / 1913 / 1938 and 1892 / 1896 / 1916; 16 behind 256 2072 / 2116 / 2168 and 2010 / 2026 / 2088; 10 behind 400 2085 /
+// 2188 / 2347 and 1986 / 1999 / 2066).  Below 96 rows results stay what they were (ATTN_TILES_MIN_PROMPT).
+static int attn_plan_one_tw(int P, int Hkv) { return Hkv >= 32 && P >= 96 ? ATT_ONE_TW : min(attn_plan_tw(P, Hkv), ATT_ONE_TW); }
+
 // Two launches: rows of the prefix per workgroup and the number of workgroups that share one slice's query tiles.
 // Every slice leaves a partial per query, so wide slices mean less partial traffic; the CUs are filled first by
 // dealing the rounds of query tiles (four tiles, one per wave) of a slice to several workgroups, which re-read the
@@ -2324,7 +2330,7 @@ extern "C" int smh_shared_prefix_attn_qkv(const void *qkv_partial, int ksplit, v
     p.P = P; p.suffix_format = SMH_KV_Q40;
     p.scale_log2 = LOG2E / sqrtf((float)D);
     int qgroups = 1;
-    if (single_launch) p.tw = min(attn_plan_tw(P, Hkv), ATT_ONE_TW);
+    if (single_launch) p.tw = attn_plan_one_tw(P, Hkv);
     else attn_plan(P, Hkv, p.Bq, &p.tw, &qgroups);
     p.splits = P > 0 ? (P + p.tw - 1) / p.tw : 0;
     p.qkv = (const float *)qkv_partial; p.qkv_ks = ksplit;
@@ -2342,7 +2348,8 @@ extern "C" int smh_shared_prefix_attn_qkv(const void *qkv_partial, int ksplit, v
         p.counters = (uint32_t *)workspace;
         p.part_o = (float *)((char *)workspace + ATT_COUNTER_BYTES);
         p.part_ml = p.part_o + n_part * ATT_D;
-        const auto kern = ksplit <= 8    ? (pages != nullptr ? attn_one_kernel<true, 4, 8> : attn_one_kernel<true, 0, 8>)
+        const auto kern = ksplit <= 2    ? (pages != nullptr ? attn_one_kernel<true, 4, 2> : attn_one_kernel<true, 0, 2>)
+                          : ksplit <= 8  ? (pages != nullptr ? attn_one_kernel<true, 4, 8> : attn_one_kernel<true, 0, 8>)
                           : ksplit <= 12 ? (pages != nullptr ? attn_one_kernel<true, 4, 12> : attn_one_kernel<true, 0, 12>)
                                          : (pages != nullptr ? attn_one_kernel<true, 4, 16> : attn_one_kernel<true, 0, 16>);
         hipLaunchKernelGGL(kern, dim3(p.splits + (p.Bq + 4 / p.suffix_waves - 1) / (4 / p.suffix_waves), Hkv), dim3(256), 0, (hipStream_t)stream, p);
