@@ -19,18 +19,32 @@ struct LayerBuffers {
     size_t slab_a_bytes, slab_b_bytes, total;
 };
 
-// Stages of the next launch's weights that a launch asks for (q40_warm.hpp).  Not where a layer's weights are larger and its attention brings its own long
+// Stages of the next launch's weights that a launch asks for (q40_warm.hpp).  Not in layers whose w1|w3 leaves slabs (17 .. 28 branches of the 7B shape behind 64
+// prompt rows: 0.992 .. 0.997 times as fast), nor where a layer's weights are larger and its attention brings its own long
 // prompt (three layers of 64 heads over 8, dim 8192, 17 .. 100 branches behind 1024 rows: 0.998 .. 1.001 times as fast from the norms, 0.996 .. 1.000 from the attention).
 constexpr int WARM_MAX_DIM = 8191, WARM_FROM_NORM = 3, WARM_FROM_ATTENTION = 4, WARM_FROM_SWIGLU = 16;
 
-static WarmWeights ask(const smh_layer &L, int M, int K, int nseg, const void *const *w, const int *n, bool swiglu, int stages, int workgroups) {
-    return L.dim <= WARM_MAX_DIM ? q40_warm(M, K, nseg, w, n, swiglu, stages, workgroups) : WarmWeights{};
-}
-
 static int slices(int M, int K, int nseg, const int *n) { return smh_q40_matmul_plan_tiled(M, K, nseg, n); }
+// Launches of 17 rows and more (128-column blocks, SwiGLU inside w1|w3, the norms and the attention asking for the next weights) for a layer of fewer, too,
+// where all four linears have them: bound by latency both ways, they are fewer (no SiLU launch), leave 2 to 8 slabs instead of 5 to 16, and their weights are
+// on their way earlier.  7B architecture, 512 + 50 rows, us a step with the GEMVs and so: 5 branches 2059 and 1973, 8 2142 and 2027, 10 2219 and 2042, 12 2248
+// and 2063, 16 2376 and 2150.  (4, which the launch of all layers takes with probabilities
+// of 32 bits, not 16: 2150 there and 1950 so.)  SwiGLU inside at 17 / 24 / 32 branches: 2360 / 2432 / 2495 -> 2250 /
+// 2318 / 2361.  Behind short prompts a decode step stays what it was (ATTN_TILES_MIN_PROMPT: two evaluations that differ in one rounding drift apart there).
+constexpr int BLOCKS_MIN_ROWS = 5, BLOCKS_MIN_PROMPT = 96;
+static bool as_blocks(const smh_layer &L, int M, bool swiglu_in) {
+    const int n_qkv[3] = {L.heads * 128, L.kv_heads * 128, L.kv_heads * 128}, n_dim[1] = {L.dim};
+    return M >= BLOCKS_MIN_ROWS && M <= SMH_GEMV_MAX_M && swiglu_in && gemm_swiglu_fits(M, L.dim, L.ffn, true) && blocks_plan(M, L.dim, 3, n_qkv) > 0 &&
+           blocks_plan(M, L.heads * 128, 1, n_dim) > 0 && blocks_plan(M, L.ffn, 1, n_dim) > 0;
+}
 // A launch that stores its fp16 results itself (more than 128 rows, no K-split) leaves no slabs.  layer_buffers reserves none for it,
 // so every linear below asks here before it takes the slab form.
 static bool direct(int M, int K, int nseg, const int *n) { return smh_q40_matmul_tiled_direct_fits(M, K, nseg, n) == 1; }
+
+static WarmWeights ask(const smh_layer &L, bool blocks, int M, int K, int nseg, const void *const *w, const int *n, bool swiglu, int stages, int workgroups) {
+    return L.dim <= WARM_MAX_DIM && (M > SMH_GEMV_MAX_M || blocks) ? q40_warm(M, K, nseg, w, n, swiglu, stages, workgroups) : WarmWeights{};
+}
+
 
 // The attention of a decode layer: in one launch whose last workgroups merge (ONE, up to 16 queries a kv head), in one launch of 8 or 16
 // queries a workgroup (TILES), or RoPE, prefix slices and walks (LAUNCHES).  us a call with RoPE and append, caches in HBM:
@@ -47,6 +61,9 @@ static bool direct(int M, int K, int nseg, const int *n) { return smh_q40_matmul
 //    48 / 2047                               -    31.5   32.0    |    16 / 2047                      -    24.4   26.3
 //   100 / 2047                               -    34.7   47.7    |   100 / 2047                      -    48.8   65.6
 //                                                                |  40 heads, 100 / 512 (two rounds) -   39.5   39.0
+// (Multi-head attention, with ONE's slices of 64 rows and two slabs, us a step of the 7B architecture with ONE and LAUNCHES, 10 / 60 / 120 rows of their own: 700 prompt
+// rows, 10 branches 2097 / 2112 / 2164 and 2142 / 2154 / 2206, 16 2158 / 2225 / 2382 and 2183 / 2196 / 2251; 768 rows, 8 branches 2046 / 2060 / 2124 and 2104 / 2113 /
+// 2138, 9 2093 / 2185 / 2343 and 2138 / 2150 / 2200, where its waves no longer fit one round in pairs.)
 // A long prompt wants more workgroups than few tiles are, and ONE's merge grows with the slices.  Where the table has a faster form than the rule takes,
 // the line is not drawn yet: multi-head attention of 6 to 16 branches (TILES at 16 / 256, LAUNCHES at 10 / 768) and one grouped branch behind a long
 // prompt were measured at these sizes only, and stay with ONE.  Behind fewer than 96 prompt rows results stay
@@ -57,7 +74,7 @@ constexpr int ATTN_TILES_MIN_PROMPT = 96;
 static AttnWay attn_way(int M, int heads, int kv_heads, int P, bool one, bool tiles, bool launches) {
     const int rep = heads / kv_heads;
     const long queries = (long)M * rep;                      // of a kv head
-    if (one && (rep == 1 ? P <= 768 : queries <= 8 || P <= 256)) return ATTN_ONE;
+    if (one && (rep == 1 ? P <= (M > 8 ? 704 : 768) : queries <= 8 || P <= 256)) return ATTN_ONE;
     const bool round = (kv_heads + 7) / 8 * 8 * ((queries + 15) / 16) <= 256;
     if (tiles && P >= ATTN_TILES_MIN_PROMPT && (rep > 1 || (M > SMH_GEMV_MAX_M && round)) &&
         (P <= 512 || P <= kv_heads * ((queries + 7) / 8) * (rep == 1 ? 12 : 24)))
@@ -70,12 +87,14 @@ static int layer_buffers(const smh_layer &L, int M, bool swiglu_in, char *base, 
     const int n_qkv[3] = {nq, nkv, nkv}, n_gu[2] = {L.ffn, L.ffn}, n_dim[1] = {L.dim};
     const int ks_qkv = slices(M, L.dim, 3, n_qkv), ks_gu = slices(M, L.dim, 2, n_gu), ks_o = slices(M, nq, 1, n_dim), ks_d = slices(M, L.ffn, 1, n_dim);
     if (ks_qkv < 1 || ks_gu < 1 || ks_o < 1 || ks_d < 1) return -1;
+    const bool blocks = as_blocks(L, M, swiglu_in);
     const size_t m = (size_t)M;
     auto most = [](size_t x, size_t y) { return x > y ? x : y; };
     const bool gu_slabs = !(M > 128 && swiglu_in && smh_q40_swiglu_fits(M, L.dim, L.ffn));
     const bool qkv_slabs = !direct(M, L.dim, 3, n_qkv), o_slabs = !direct(M, nq, 1, n_dim), d_slabs = !direct(M, L.ffn, 1, n_dim);
-    b.slab_a_bytes = align_up(most(qkv_slabs ? ks_qkv * m * (nq + 2 * (size_t)nkv) : 1, gu_slabs ? ks_gu * m * 2 * (size_t)L.ffn : 1) * sizeof(float));
-    b.slab_b_bytes = align_up((size_t)most(o_slabs ? ks_o : 0, d_slabs ? ks_d : 0) * m * L.dim * sizeof(float));
+    auto slabs = [&](int ks, int K, int nseg, const int *n) { return most((size_t)ks, blocks ? (size_t)blocks_plan(M, K, nseg, n) : 0); };
+    b.slab_a_bytes = align_up(most(qkv_slabs ? slabs(ks_qkv, L.dim, 3, n_qkv) * m * (nq + 2 * (size_t)nkv) : 1, gu_slabs ? ks_gu * m * 2 * (size_t)L.ffn : 1) * sizeof(float));
+    b.slab_b_bytes = align_up((size_t)most(o_slabs ? slabs(ks_o, nq, 1, n_dim) : 0, d_slabs ? slabs(ks_d, L.ffn, 1, n_dim) : 0) * m * L.dim * sizeof(float));
     size_t at = 0;
     auto take = [&](size_t bytes) { char *p = base ? base + at : nullptr; at += align_up(bytes); return p; };
     b.h[0] = take(m * L.dim * 2);
@@ -99,13 +118,16 @@ struct LayerRun {
     smh_pass &S;
     smh_stream_t stream;
     const int M, nq, nkv;
+    const bool blocks, swiglu;                 // far: not a decode step behind a short prompt
     const int n_qkv[3], n_gu[2], n_dim[1];
     const void *w_qkv[3], *w_o[1], *w_gu[2], *w_d[1];
     LayerBuffers b;
 
-    LayerRun(const smh_layer &l, smh_pass &s, smh_stream_t st)
-        : L(l), S(s), stream(st), M(s.rows), nq(l.heads * 128), nkv(l.kv_heads * 128), n_qkv{nq, nkv, nkv}, n_gu{l.ffn, l.ffn}, n_dim{l.dim},
+    LayerRun(const smh_layer &l, smh_pass &s, smh_stream_t st, bool far)
+        : L(l), S(s), stream(st), M(s.rows), nq(l.heads * 128), nkv(l.kv_heads * 128), blocks(far && as_blocks(l, s.rows, s.swiglu_in != 0)),
+          swiglu(s.swiglu_in != 0 && (s.rows > SMH_GEMV_MAX_M ? s.rows > 32 || far : blocks) && gemm_swiglu_fits(s.rows, l.dim, l.ffn, true)), n_qkv{nq, nkv, nkv}, n_gu{l.ffn, l.ffn}, n_dim{l.dim},
           w_qkv{l.wq, l.wk, l.wv}, w_o{l.wo}, w_gu{l.w1, l.w3}, w_d{l.w2} {}
+    int slabs(int K, int nseg, const int *n) const { return blocks ? blocks_plan(M, K, nseg, n) : slices(M, K, nseg, n); }
     int begin(const char *who) {
         SMH_REQUIRE(M >= 1 && L.heads > 0 && L.kv_heads > 0 && L.heads % L.kv_heads == 0, "%s: rows=%d heads=%d kv_heads=%d", who, M, L.heads, L.kv_heads);
         if (layer_buffers(L, M, S.swiglu_in != 0, (char *)S.scratch, b) != 0) return -1;
@@ -128,8 +150,8 @@ struct LayerRun {
             S.h = out[0];
             return r;
         }
-        S.pending = slices(M, K, 1, n_dim);
-        return smh_q40_matmul_partial_tiled(x, M, K, K, 1, w, n_dim, b.slab_b, b.slab_b_bytes, stream);
+        S.pending = slabs(K, 1, n_dim);
+        return matmul_partial_tiled(x, M, K, K, 1, w, n_dim, b.slab_b, b.slab_b_bytes, blocks, stream);
     }
 };
 
@@ -146,7 +168,7 @@ extern "C" size_t smh_decode_scratch_bytes(const smh_layer *layer, int rows, int
 extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stream_t stream) {
     const char *who = "smh_decode_layer";
     SMH_REQUIRE(layer && pass && pass->h, "%s: null pointer", who);
-    LayerRun run(*layer, *pass, stream);
+    LayerRun run(*layer, *pass, stream, layer->prompt_len >= BLOCKS_MIN_PROMPT);
     int st = run.begin(who);
     if (st) return st;
     const smh_layer &L = *layer;
@@ -155,9 +177,9 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
     const int M = run.M, nq = run.nq;
     // the RMSNorm of the residual stream and the linears behind it: to slab_a.  With few rows the RMSNorm is made inside the linears' launch.
     auto norm_linears = [&](const void *weight, float eps, int nseg, const void *const *w, const int *n) -> int {
-        if (S.pending == 0 || M > S.norm_in_rows || smh_q40_norm_in_fits(M, L.dim, nseg, n) != 1) {
-            if (int r = run.norm(weight, eps, ask(L, M, L.dim, nseg, w, n, false, WARM_FROM_NORM, 256))) return r;
-            return smh_q40_matmul_partial_tiled(b.xn, M, L.dim, L.dim, nseg, w, n, b.slab_a, b.slab_a_bytes, stream);
+        if (S.pending == 0 || M > S.norm_in_rows || run.blocks || smh_q40_norm_in_fits(M, L.dim, nseg, n) != 1) {
+            if (int r = run.norm(weight, eps, run.swiglu ? ask(L, run.blocks, M, L.dim, nseg, w, n, false, WARM_FROM_NORM, 256) : WarmWeights{})) return r;
+            return matmul_partial_tiled(b.xn, M, L.dim, L.dim, nseg, w, n, b.slab_a, b.slab_a_bytes, run.blocks, stream);
         }
         void *h_out = b.h[S.h == b.h[0]];
         if (int r = smh_partial_residual_sumsq(b.slab_b, S.pending, M, L.dim, S.h, h_out, b.sums, stream)) return r;
@@ -188,7 +210,7 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
         st = norm_linears(L.att_norm, L.att_eps, 3, run.w_qkv, run.n_qkv);
     }
     if (st) return st;
-    const int ks_qkv = slices(M, L.dim, 3, run.n_qkv);
+    const int ks_qkv = run.slabs(L.dim, 3, run.n_qkv);
     // (Only in one launch: in two, each of the 256 prefix workgroups adds up and rotates all queries of its kv head.  Grouped queries,
     // three layers of 64 heads over 8 kv heads: 10 branches after 2047 rows 594 us a step so, 552 with the RoPE launch in front; 3
     // branches 523 against 511, 16 branches 629 against 571.)
@@ -198,7 +220,7 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
                                         ws_bytes, stream);
     } else if (way == ATTN_TILES) {
         const int row = (L.kv_heads + 7) / 8 * 8, idle = attn_tiles_idle(M, L.heads, L.kv_heads);
-        WarmWeights wo = ask(L, M, nq, 1, run.w_o, run.n_dim, false, WARM_FROM_ATTENTION, idle);
+        WarmWeights wo = ask(L, run.blocks, M, nq, 1, run.w_o, run.n_dim, false, WARM_FROM_ATTENTION, idle);
         wo.workgroups = wo.workgroups / row * row;
         st = shared_prefix_attn_qkv_tiles(b.slab_a, ks_qkv, b.att, M, L.heads, L.kv_heads, 128, S.cos_tab, S.sin_tab, S.pos_dev, L.prompt_k, L.prompt_v,
                                           L.prompt_len, L.cache_k, L.cache_ks, L.cache_v, L.cache_vs, S.smax, S.t_dev, S.pages, S.pages_stride,
@@ -220,9 +242,9 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
     if (st) return st;
     if ((st = run.residual_linear(b.att, nq, run.w_o))) return st;
     // ---- feed forward ----
-    if (S.swiglu_in != 0 && smh_q40_swiglu_fits(M, L.dim, L.ffn)) {
-        if ((st = run.norm(L.ffn_norm, L.ffn_eps, ask(L, M, L.dim, 2, run.w_gu, run.n_gu, true, WARM_FROM_NORM, 256)))) return st;
-        const WarmWeights w2 = ask(L, M, L.ffn, 1, run.w_d, run.n_dim, false, WARM_FROM_SWIGLU, swiglu_idle(L.ffn));
+    if (run.swiglu) {
+        if ((st = run.norm(L.ffn_norm, L.ffn_eps, ask(L, run.blocks, M, L.dim, 2, run.w_gu, run.n_gu, true, WARM_FROM_NORM, 256)))) return st;
+        const WarmWeights w2 = ask(L, run.blocks, M, L.ffn, 1, run.w_d, run.n_dim, false, WARM_FROM_SWIGLU, swiglu_idle(L.ffn));
         if ((st = matmul_tiled_swiglu(b.xn, M, L.dim, L.dim, L.w1, L.w3, L.ffn, b.act, L.ffn, w2, stream))) return st;
         return run.residual_linear(b.act, L.ffn, run.w_d);
     }
@@ -242,7 +264,7 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
 extern "C" int smh_prefill_layer(const smh_layer *layer, smh_pass *pass, smh_stream_t stream) {
     const char *who = "smh_prefill_layer";
     SMH_REQUIRE(layer && pass && pass->h, "%s: null pointer", who);
-    LayerRun run(*layer, *pass, stream);
+    LayerRun run(*layer, *pass, stream, true);
     int st = run.begin(who);
     if (st) return st;
     const smh_layer &L = *layer;
@@ -259,16 +281,16 @@ extern "C" int smh_prefill_layer(const smh_layer *layer, smh_pass *pass, smh_str
             st = smh_rope(b.q, L.prompt_k, M, L.heads, L.kv_heads, 128, S.cos_tab, S.sin_tab, 0, stream);
         }
     } else {
-        if ((st = smh_q40_matmul_partial_tiled(b.xn, M, L.dim, L.dim, 3, run.w_qkv, run.n_qkv, b.slab_a, b.slab_a_bytes, stream))) return st;
-        st = smh_partial_rope_rows(b.slab_a, slices(M, L.dim, 3, run.n_qkv), M, L.heads, L.kv_heads, 128, b.q, L.prompt_k, L.prompt_v, S.cos_tab, S.sin_tab, 0,
+        if ((st = matmul_partial_tiled(b.xn, M, L.dim, L.dim, 3, run.w_qkv, run.n_qkv, b.slab_a, b.slab_a_bytes, run.blocks, stream))) return st;
+        st = smh_partial_rope_rows(b.slab_a, run.slabs(L.dim, 3, run.n_qkv), M, L.heads, L.kv_heads, 128, b.q, L.prompt_k, L.prompt_v, S.cos_tab, S.sin_tab, 0,
                                    stream);
     }
     if (st) return st;
     if ((st = smh_prefill_attn(b.q, L.prompt_k, L.prompt_v, b.att, M, L.heads, L.kv_heads, 128, stream))) return st;
     if ((st = run.residual_linear(b.att, nq, run.w_o))) return st;
     if ((st = run.norm(L.ffn_norm, L.ffn_eps))) return st;
-    if (S.swiglu_in != 0 && smh_q40_swiglu_fits(M, L.dim, L.ffn)) {
-        st = smh_q40_matmul_tiled_swiglu(b.xn, M, L.dim, L.dim, L.w1, L.w3, L.ffn, b.act, L.ffn, stream);
+    if (run.swiglu) {
+        st = matmul_tiled_swiglu(b.xn, M, L.dim, L.dim, L.w1, L.w3, L.ffn, b.act, L.ffn, WarmWeights{}, stream);
     } else if ((st = smh_q40_matmul_partial_tiled(b.xn, M, L.dim, L.dim, 2, run.w_gu, run.n_gu, b.slab_a, b.slab_a_bytes, stream)) == 0) {
         st = smh_partial_silu_mul(b.slab_a, slices(M, L.dim, 2, run.n_gu), M, L.ffn, b.act, stream);
     }

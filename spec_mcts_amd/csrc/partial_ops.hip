@@ -354,7 +354,7 @@ static const decltype(&partial_rope_rows_kernel<1>) ROPE_ROWS_KERNELS[17] = BY_S
 
 // ---- host side: plan, produce, consume ----------------------------------------------------------------
 static int fill_params(MatmulParams &p, const void *a, int M, int K, long lda, int nseg, const void *const *w,
-                       const void *const *s, const int *n, const char *who, bool tiled = false) {
+                       const void *const *s, const int *n, const char *who, bool tiled = false, bool gemm = false) {
     SMH_REQUIRE(M >= 0, "%s: M=%d", who, M);
     SMH_REQUIRE(K > 0 && K % 8 == 0, "%s: K=%d must be a positive multiple of 8", who, K);
     SMH_REQUIRE(nseg >= 1 && nseg <= SMH_MAX_SEGMENTS && n != nullptr, "%s: nseg=%d outside [1,%d]", who, nseg, SMH_MAX_SEGMENTS);
@@ -369,7 +369,7 @@ static int fill_params(MatmulParams &p, const void *a, int M, int K, long lda, i
         p.seg[i].N = n[i];
     }
     p.tiled = tiled ? 1 : 0;                   // (the plan above 16 rows depends on the layout)
-    if (M <= SMH_GEMV_MAX_M) gemv_fill_plan(p); else gemm_fill_plan(p);
+    if (M <= SMH_GEMV_MAX_M && !gemm) gemv_fill_plan(p); else gemm_fill_plan(p);
     return 0;
 }
 
@@ -387,7 +387,9 @@ extern "C" int smh_q40_matmul_columns(int M, int K, int N) {
     return st < 0 ? st : p.kgroups == 2 || (p.ksplit > 1 && gemm_blocks_fit(p, b)) ? 128 : 256;
 }
 
-extern "C" int smh_q40_swiglu_fits(int M, int K, int n_half) { return smh::gemm_swiglu_fits(M, K, n_half, true) ? 1 : 0; }
+extern "C" int smh_q40_swiglu_fits(int M, int K, int n_half) {
+    return (M > 32 && smh::gemm_swiglu_fits(M, K, n_half, true)) ? 1 : 0;
+}
 
 int smh::matmul_tiled_swiglu(const void *a, int M, int K, long lda, const void *tiled_gate, const void *tiled_up, int n_half, void *out, long ldo,
                              const WarmWeights &next, smh_stream_t stream) {
@@ -407,15 +409,16 @@ int smh::matmul_tiled_swiglu(const void *a, int M, int K, long lda, const void *
 }
 extern "C" int smh_q40_matmul_tiled_swiglu(const void *a, int M, int K, long lda, const void *tiled_gate, const void *tiled_up, int n_half,
                                            void *out, long ldo, smh_stream_t stream) {
+    SMH_REQUIRE(M > SMH_GEMV_MAX_M, "smh_q40_matmul_tiled_swiglu: M=%d (17 .. 128, or above 128)", M);
     return matmul_tiled_swiglu(a, M, K, lda, tiled_gate, tiled_up, n_half, out, ldo, WarmWeights{}, stream);
 }
 
 WarmWeights smh::q40_warm(int M, int K, int nseg, const void *const *tiled, const int *n, bool swiglu, int stages, int workgroups) {
     WarmWeights w = WarmWeights{};
     MatmulParams p;
-    if (M <= SMH_GEMV_MAX_M || M > 128 || K % 64 != 0 || stages < 1) return w;
+    if (M < 1 || M > 128 || K % 64 != 0 || stages < 1) return w;
     if (swiglu ? nseg != 2 || n[0] != n[1] || !gemm_swiglu_fits(M, K, n[0], false)
-               : fill_params(p, nullptr, M, K, K, nseg, nullptr, nullptr, n, "q40_warm", true) != 0 || p.kgroups != 2) return w;
+               : fill_params(p, nullptr, M, K, K, nseg, nullptr, nullptr, n, "q40_warm", true, true) != 0 || p.kgroups != 2) return w;
     for (int i = 0; i < nseg; ++i)
         if (tiled[i] == nullptr || ((uintptr_t)tiled[i] & 127) != 0) return w;
     for (int i = 0; i < SMH_MAX_SEGMENTS; ++i) {
@@ -436,7 +439,7 @@ WarmWeights smh::q40_warm(int M, int K, int nseg, const void *const *tiled, cons
 extern "C" int smh_q40_warm_span(int M, int K, int nseg, const int *n, int swiglu, int stages, long *lines, long *first, long *end) {
     SMH_REQUIRE(nseg >= 1 && nseg <= SMH_MAX_SEGMENTS && n && lines && first && end, "smh_q40_warm_span: nseg=%d or a null pointer", nseg);
     const void *const some[SMH_MAX_SEGMENTS] = {(const void *)128, (const void *)128, (const void *)128};
-    const WarmWeights w = q40_warm(M, K, nseg, some, n, swiglu != 0, stages, 8);
+    const WarmWeights w = M > SMH_GEMV_MAX_M ? q40_warm(M, K, nseg, some, n, swiglu != 0, stages, 8) : WarmWeights{};
     for (int i = 0; i < nseg; ++i) { lines[i] = first[i] = end[i] = 0; }
     for (int at = 0; w.workgroups > 0 && at < warm_blocks(w); ++at) {
         WarmBlock b;
@@ -468,7 +471,7 @@ extern "C" int smh_q40_matmul_tiled_direct_columns(int M, int K, int nseg, const
 }
 
 static int swiglu_plan(int M, int K, int n_half, int (*ask)(MatmulParams)) {
-    if (!gemm_swiglu_fits(M, K, n_half, false)) return 0;
+    if (M <= SMH_GEMV_MAX_M || !gemm_swiglu_fits(M, K, n_half, false)) return 0;
     MatmulParams p = MatmulParams{};
     p.M = M; p.K = K; p.nseg = 2;
     p.seg[0].N = p.seg[1].N = n_half;
@@ -550,10 +553,18 @@ extern "C" int smh_q40_matmul_partial(const void *a, int M, int K, long lda, int
     return M <= SMH_GEMV_MAX_M ? gemv_launch(p, (hipStream_t)stream) : gemm_launch(p, (hipStream_t)stream);
 }
 
+int smh::blocks_plan(int M, int K, int nseg, const int *n) {
+    MatmulParams p;
+    return fill_params(p, nullptr, M, K, (K + 7) / 8 * 8, nseg, nullptr, nullptr, n, "blocks_plan", true, true) == 0 && p.kgroups == 2 ? p.ksplit : 0;
+}
 extern "C" int smh_q40_matmul_partial_tiled(const void *a, int M, int K, long lda, int nseg, const void *const *tiled,
                                             const int *n, void *partial, size_t partial_bytes, smh_stream_t stream) {
+    return matmul_partial_tiled(a, M, K, lda, nseg, tiled, n, partial, partial_bytes, false, stream);
+}
+int smh::matmul_partial_tiled(const void *a, int M, int K, long lda, int nseg, const void *const *tiled, const int *n, void *partial, size_t partial_bytes,
+                              bool blocks, smh_stream_t stream) {
     MatmulParams p;
-    int st = fill_params(p, a, M, K, lda, nseg, tiled, nullptr, n, "smh_q40_matmul_partial_tiled", true);
+    int st = fill_params(p, a, M, K, lda, nseg, tiled, nullptr, n, "smh_q40_matmul_partial_tiled", true, blocks);
     if (st) return st;
     if (M == 0) return 0;
     SMH_REQUIRE(a && tiled && partial, "smh_q40_matmul_partial_tiled: null pointer");
@@ -564,7 +575,7 @@ extern "C" int smh_q40_matmul_partial_tiled(const void *a, int M, int K, long ld
     p.partial = (float *)partial;
     p.direct = 0;
     p.tiled = 1;
-    return M <= SMH_GEMV_MAX_M ? gemv_launch(p, (hipStream_t)stream) : gemm_launch(p, (hipStream_t)stream);
+    return M <= SMH_GEMV_MAX_M && !blocks ? gemv_launch(p, (hipStream_t)stream) : gemm_launch(p, (hipStream_t)stream);
 }
 
 extern "C" int smh_q40_matmul_partial_tiled_silu(const void *gate_up_partial, int gate_up_ksplit, int M, int K, int nseg,

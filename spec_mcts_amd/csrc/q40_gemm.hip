@@ -1664,16 +1664,16 @@ bool gemm_blocks_fit(const MatmulParams &p, MatmulParams &b) {
 
 typedef void (*gemm_kg_kernel_t)(MatmulParams);
 static int gemm_kg_launch(const MatmulParams &p, hipStream_t stream) {
-#define KG_KERNELS(...) {nullptr, nullptr, q40_gemm_kg_kernel<2, __VA_ARGS__>, q40_gemm_kg_kernel<3, __VA_ARGS__>, q40_gemm_kg_kernel<4, __VA_ARGS__>, \
+#define KG_KERNELS(one, ...) {nullptr, one, q40_gemm_kg_kernel<2, __VA_ARGS__>, q40_gemm_kg_kernel<3, __VA_ARGS__>, q40_gemm_kg_kernel<4, __VA_ARGS__>, \
                          q40_gemm_kg_kernel<5, __VA_ARGS__>, q40_gemm_kg_kernel<6, __VA_ARGS__>, q40_gemm_kg_kernel<7, __VA_ARGS__>, q40_gemm_kg_kernel<8, __VA_ARGS__>}
-    static const gemm_kg_kernel_t kern[3][9] = {KG_KERNELS(true, false), KG_KERNELS(false, false), KG_KERNELS(false, true)};
+    static const gemm_kg_kernel_t kern[3][9] = {KG_KERNELS((q40_gemm_kg_kernel<1, true, false>), true, false), KG_KERNELS(nullptr, false, false), KG_KERNELS(nullptr, false, true)};
 #undef KG_KERNELS
-    static const int lds_bytes[9] = {0, 0, KgShape<2>::LDS, KgShape<3>::LDS, KgShape<4>::LDS, KgShape<5>::LDS, KgShape<6>::LDS, KgShape<7>::LDS, KgShape<8>::LDS};
+    static const int lds_bytes[9] = {0, KgShape<1>::LDS, KgShape<2>::LDS, KgShape<3>::LDS, KgShape<4>::LDS, KgShape<5>::LDS, KgShape<6>::LDS, KgShape<7>::LDS, KgShape<8>::LDS};
     static const hipError_t lds_ok = [] {
         hipError_t e = hipSuccess;
-        for (int t = 2; t <= 8; ++t)
+        for (int t = 1; t <= 8; ++t)
             for (int form = 0; form < 3 && e == hipSuccess; ++form)
-                e = hipFuncSetAttribute((const void *)kern[form][t], hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes[t]);
+                if (kern[form][t] != nullptr) e = hipFuncSetAttribute((const void *)kern[form][t], hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes[t]);
         return e;
     }();
     if (lds_ok != hipSuccess) {
@@ -1682,7 +1682,7 @@ static int gemm_kg_launch(const MatmulParams &p, hipStream_t stream) {
     }
     SMH_REQUIRE((long)p.M * p.lda * 2 < (1L << 32), "q40 gemm: M x lda = %d x %ld exceeds the 32-bit lane offsets of A", p.M, p.lda);
     int tiles = p.mblocks > 1 ? p.block_rows / 16 : (p.M + 15) / 16;
-    if (tiles < 2) tiles = 2;
+    if (tiles < 2 && !p.tiled) tiles = 2;
     const int form = p.tiled ? 0 : p.K % 32 == 0 ? 1 : 2;
     hipLaunchKernelGGL(kern[form][tiles], dim3((unsigned)(2 * p.units_pad), (unsigned)p.mblocks, (unsigned)p.ksplit), dim3(64 * (8 + GEMM_DMA_WAVES)), lds_bytes[tiles], stream, p);
     return launch_status();
@@ -1695,25 +1695,25 @@ static int gemm_kg_launch(const MatmulParams &p, hipStream_t stream) {
 // `worth_it`: and fill at least half of them (narrower weights are faster as two kernels with a K-split), above 32 rows
 // (measured at the 7B shape, w1|w3 + SiLU: 38.1 against 44.9 us at 100 rows, 29.1 against 31.5 at 64, level at 32).
 bool gemm_swiglu_fits(int M, int K, int n_half, bool worth_it) {
-    if (M <= SMH_GEMV_MAX_M || K <= 0 || n_half <= 0 || n_half % 128 != 0) return false;
+    if (M < 1 || K <= 0 || n_half <= 0 || n_half % 128 != 0) return false;
     if (M > GEMM_BM) return K % 32 == 0;                        // gemm_swiglu_rows_launch
     if (K % 64 != 0) return false;
     const int wgs = 2 * (n_half / 128);
-    return wgs <= 256 && (!worth_it || (wgs >= 128 && M > 32));
+    return wgs <= 256 && (!worth_it || wgs >= 128);
 }
 
 int swiglu_idle(int n_half) { return n_half / 64 < 256 ? (256 - n_half / 64) / 8 * 8 : 0; }
 
 typedef void (*gemm_swiglu_kernel_t)(MatmulParams, WarmWeights);
 int gemm_swiglu_launch(const MatmulParams &p, const WarmWeights &next, hipStream_t stream) {
-    static const gemm_swiglu_kernel_t kern[9] = {nullptr, nullptr, q40_gemm_swiglu_kernel<2>, q40_gemm_swiglu_kernel<3>, q40_gemm_swiglu_kernel<4>,
+    static const gemm_swiglu_kernel_t kern[9] = {nullptr, q40_gemm_swiglu_kernel<1>, q40_gemm_swiglu_kernel<2>, q40_gemm_swiglu_kernel<3>, q40_gemm_swiglu_kernel<4>,
                                                  q40_gemm_swiglu_kernel<5>, q40_gemm_swiglu_kernel<6>, q40_gemm_swiglu_kernel<7>,
                                                  q40_gemm_swiglu_kernel<8>};
-    static const int lds_bytes[9] = {0, 0, SwigluShape<2>::LDS, SwigluShape<3>::LDS, SwigluShape<4>::LDS, SwigluShape<5>::LDS, SwigluShape<6>::LDS,
+    static const int lds_bytes[9] = {0, SwigluShape<1>::LDS, SwigluShape<2>::LDS, SwigluShape<3>::LDS, SwigluShape<4>::LDS, SwigluShape<5>::LDS, SwigluShape<6>::LDS,
                                      SwigluShape<7>::LDS, SwigluShape<8>::LDS};
     static const hipError_t lds_ok = [] {
         hipError_t e = hipSuccess;
-        for (int t = 2; t <= 8 && e == hipSuccess; ++t)
+        for (int t = 1; t <= 8 && e == hipSuccess; ++t)
             e = hipFuncSetAttribute((const void *)kern[t], hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes[t]);
         return e;
     }();
@@ -1722,8 +1722,7 @@ int gemm_swiglu_launch(const MatmulParams &p, const WarmWeights &next, hipStream
         return (int)lds_ok;
     }
     SMH_REQUIRE((long)p.M * p.lda * 2 < (1L << 32), "q40 gemm: M x lda = %d x %ld exceeds the 32-bit lane offsets of A", p.M, p.lda);
-    int tiles = (p.M + 15) / 16;
-    if (tiles < 2) tiles = 2;
+    const int tiles = (p.M + 15) / 16;
     hipLaunchKernelGGL(kern[tiles], dim3((unsigned)(2 * (p.seg[0].N / 128) + next.workgroups)), dim3(64 * (8 + GEMM_DMA_WAVES)), lds_bytes[tiles], stream, p, next);
     return launch_status();
 }

@@ -96,6 +96,10 @@ int shared_prefix_attn_qkv_tiles(const void *qkv_partial, int ksplit, void *out,
                                  const int32_t *pos_dev, const void *prefix_k, const void *prefix_v, int P, void *cache_k, void *cache_ks, void *cache_v,
                                  void *cache_vs, int Smax, const int32_t *t_dev, const int32_t *pages, int pages_stride, long cache_rows,
                                  const WarmWeights &next, smh_stream_t stream);
+// smh_q40_matmul_partial_tiled; blocks: up to 16 rows, too, on q40_gemm_kg_kernel, for which blocks_plan is not 0 (the slabs it leaves)
+int matmul_partial_tiled(const void *a, int M, int K, long lda, int nseg, const void *const *tiled, const int *n, void *partial, size_t partial_bytes,
+                         bool blocks, smh_stream_t stream);
+int blocks_plan(int M, int K, int nseg, const int *n);
 // compute units that a launch of these leaves without a workgroup, in eights
 int swiglu_idle(int n_half);
 int attn_tiles_idle(int B, int H, int Hkv);

@@ -309,7 +309,7 @@ class Transformer(nn.Module):
         self.per_branch_kv = False    # True: hf_model_q40's protocol (every position in the branch's own Q4_0 cache)
         self.fused_sampler = True          # generate(): temperature / top-k / draw as one kernel instead of five torch ops
         self.silu_in_matmul = True         # up to 2 rows: w2's launch makes its own SiLU(gate)*up activations
-        self.swiglu_in_matmul = True       # 33 .. 128 rows, wide FFN: SiLU(gate) * up inside w1|w3's launch (kernels.matmul_q40_swiglu)
+        self.swiglu_in_matmul = True       # up to 128 rows, wide FFN: SiLU(gate) * up inside w1|w3's launch (kernels.matmul_q40_swiglu)
         self.tiled_weights = True          # the fused path streams tiled copies of the weights (LinearQ4_0.operand)
         self.attn_single_launch = True     # up to 16 queries per kv head: prefix slices, suffix passes and the merge in one launch
                                            # (above, the one workgroup that merges a kv head's query tiles takes longer than a launch)

@@ -153,3 +153,32 @@ def test_passes_that_only_some_forms_of_the_attention_take(heads, kv_heads, B, P
         got = _layer_pass(model, h, t, rows, **(dict(cache_rows=0) if change == "no row count" else dict(attn_ws_bytes=256)))
     torch.cuda.synchronize()
     assert want.isfinite().all() and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("B,P", [(5, 96), (6, 130), (11, 300), (16, 100), (17, 97), (32, 96), (5, 95), (16, 95), (24, 95)])
+def test_few_branches_behind_a_prompt(B, P):
+    """Layers of the 7B shape for 5 .. 32 branches: from 96 prompt rows on 128-column blocks and SwiGLU inside w1|w3 (one row tile up to 16 branches, two from
+    17 on), before that GEMVs, or slabs of w1|w3.  In 64 bits, without any of the path's roundings: as far from that as 17 .. 48 branches of the same
+    tokens are, which take the blocks anyway."""
+    cfg = dict(LAYER_7B, max_batch_size=48, max_prompt_seq_len=320)
+    _, _, model = _build(cfg, 77, 0.02)
+    att = [layer.attention for layer in model.layers]
+    g = torch.Generator(device="cuda:0").manual_seed(B + P)
+    for a in att:
+        for c in (a.cache_prompt_k, a.cache_prompt_v):
+            c[0, :P] = torch.randn((P, 32, 128), generator=g, device="cuda:0", dtype=torch.float16)
+        a.cache_prompt_len = P
+    tok = torch.randint(0, cfg["vocab_size"], (B, 1), generator=g, device="cuda:0")
+    outs = []
+    for step in range(2):                              # (the second reads what the first appended)
+        got = model(tok, P + step)[:, 0].float()
+        rows = [(a.cache_k.clone(), a.cache_k_s.clone(), a.cache_v.clone(), a.cache_v_s.clone()) for a in att]
+        wide = model(tok.repeat(48 // B + 1, 1)[:48], P + step)[:B, 0].float()
+        for a, saved in zip(att, rows):                # (what the wider step appended, taken back)
+            for c, r in zip((a.cache_k, a.cache_k_s, a.cache_v, a.cache_v_s), saved):
+                c.copy_(r)
+        outs.append((got, wide))
+    for got, wide in outs:
+        assert got.isfinite().all()
+        # fp16 roundings at the same points, fp32 sums in another order: a flip now and then moves a logit by a few 2^-11 of the deviation, two layers deep
+        assert float((got - wide).norm() / wide.norm()) < 4e-3
