@@ -1037,6 +1037,7 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
 #pragma unroll
                 for (int k = 0; k < 8; ++k) o[j][k] = 0.f;
             Q4Chunk cur = q4_first;
+            const RowCodes codes;
             wait_loads();
             for (int n = 0; n < q4_chunks; ++n) {
                 Q4Chunk nxt;
@@ -1050,7 +1051,7 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
                     float d = 0.f;
 #pragma unroll
                     for (int j = 0; j < Q4_DW; ++j) {
-                        const RowRegs kr = row_from_q40(cur.k[u][j], cur.ks[u]);
+                        const RowRegs kr = row_from_q40(cur.k[u][j], cur.ks[u], codes);
                         d = __builtin_amdgcn_fdot2(kr.a02, qj[j].a02, d, false);
                         d = __builtin_amdgcn_fdot2(kr.a13, qj[j].a13, d, false);
                         d = __builtin_amdgcn_fdot2(kr.b02, qj[j].b02, d, false);
@@ -1082,7 +1083,7 @@ __device__ __forceinline__ void attn_suffix_body(const AttnParams &p, int b, int
                     l += pr;
 #pragma unroll
                     for (int j = 0; j < Q4_DW; ++j) {
-                        const RowRegs vr = row_from_q40(cur.v[u][j], cur.vs[u]);
+                        const RowRegs vr = row_from_q40(cur.v[u][j], cur.vs[u], codes);
                         o[j][0] += pr * (float)vr.a02.x; o[j][1] += pr * (float)vr.a02.y;
                         o[j][2] += pr * (float)vr.a13.x; o[j][3] += pr * (float)vr.a13.y;
                         o[j][4] += pr * (float)vr.b02.x; o[j][5] += pr * (float)vr.b02.y;
@@ -1884,6 +1885,7 @@ __global__ __launch_bounds__(64 * AT_WAVES) void attn_tile_kernel(AttnParams p, 
             for (int j = 0; j < 2; ++j) add(pr, j, row_from_fp16(s_v + qi * AT_QPITCH, 2 * e + j));
         }
     }
+    const RowCodes codes;
     // N passes from u0 on: one maximum, one rescale.  ends: some may lie past the last row
     auto passes = [&](int s, auto N, int u0, bool ends) {
         float sc[N];
@@ -1894,7 +1896,7 @@ __global__ __launch_bounds__(64 * AT_WAVES) void attn_tile_kernel(AttnParams p, 
             const uint32_t mine = cur.sc[u0 + i], other = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mine, DPP_ROW_HALF_MIRROR, 0xf, 0xf, false);
             const uint32_t ks = e < 4 ? mine : other;
             vs[i] = e < 4 ? other : mine;
-            sc[i] = score(row_from_q40(cur.k[u0 + i][0], ks), row_from_q40(cur.k[u0 + i][1], ks));
+            sc[i] = score(row_from_q40(cur.k[u0 + i][0], ks, codes), row_from_q40(cur.k[u0 + i][1], ks, codes));
             if (ends && row_at(s, u0 + i) >= len) sc[i] = -INFINITY;
             mx = fmaxf(mx, sc[i]);
         }
@@ -1904,7 +1906,7 @@ __global__ __launch_bounds__(64 * AT_WAVES) void attn_tile_kernel(AttnParams p, 
             const float pr = __builtin_amdgcn_exp2f(sc[i] - m_ref);
             l += pr;
 #pragma unroll
-            for (int j = 0; j < 2; ++j) add(pr, j, row_from_q40(cur.v[u0 + i][j], vs[i]));
+            for (int j = 0; j < 2; ++j) add(pr, j, row_from_q40(cur.v[u0 + i][j], vs[i], codes));
         }
     };
     for (int s = 0; s < turns; ++s) {

@@ -27,15 +27,29 @@ __device__ __forceinline__ RowRegs row_of_raw(const RawRow &t) {
     return r;
 }
 __device__ __forceinline__ RowRegs row_from_fp16(const half_t *row, int c) { return row_of_raw(raw_row(row, c)); }
-// bytes: this lane's dword of the packed row; sc: (scale of dims 0..63, scale of dims 64..127)
-__device__ __forceinline__ RowRegs row_from_q40(uint32_t bytes, uint32_t sc) {
-    const uint32_t u = bytes ^ NIBBLE_FLIP, u1 = u >> 8;
-    const h2 s_a = as_h2(pack_lo16(sc, sc)), s_b = as_h2(pack_hi16(sc, sc));
+// Q4_0 rows.  A walk of them is bound by these instructions, so masks and magic numbers stand in registers that the compiler cannot see through: the nibbles'
+// sign bits are flipped and the magic number's bits set by the instruction that masks them (v_bitop3_b32, which takes no literals), and a scale is picked
+// by the product's own operand select.  13 instructions for the eight values of a dword; with an XOR, an AND and an OR each and a permute a scale 19.
+// (us a step of the 7B architecture behind 512 rows, 10 / 64 / 127 rows of their own, before and now: 37 branches 2406 / 2490 / 2662 and 2391 / 2463 / 2643, 64
+// 2716 / 2869 / 3062 and 2691 / 2772 / 2970, 100 3317 / 3592 / 3943 and 3307 / 3551 / 3912; three layers of 64 heads over 8, 100 branches and 90 rows 994 and 972.)
+struct RowCodes {
+    uint32_t mask_hi = 0x00F000F0u, mask_lo = 0x000F000Fu, magic_hi = 0x54005400u ^ 0x00800080u, magic_lo = MAGIC_1024 ^ 0x00080008u;
+    __device__ __forceinline__ RowCodes() {
+        asm volatile("" : "+s"(mask_hi), "+s"(mask_lo));
+        asm volatile("" : "+v"(magic_hi), "+v"(magic_lo));
+    }
+};
+// bytes: this lane's dword of the packed row; sc: (scale of dims 0..63, scale of dims 64..127).  With u = code + 8: 64 + u and 1024 + u, then the code, then its
+// product, rounded once (smh_common.hpp).
+__device__ __forceinline__ RowRegs row_from_q40(uint32_t bytes, uint32_t sc, const RowCodes &C) {
+    const uint32_t next = bytes >> 8;
+    const h2 s = as_h2(sc), s_a = __builtin_shufflevector(s, s, 0, 0), s_b = __builtin_shufflevector(s, s, 1, 1);
+    const h2 off_hi = {(half_t)-72.f, (half_t)-72.f}, off_lo = {(half_t)-1032.f, (half_t)-1032.f};
     RowRegs r;
-    r.a02 = codes_high(u) * s_a;
-    r.a13 = codes_high(u1) * s_a;
-    r.b02 = codes_low(u) * s_b;
-    r.b13 = codes_low(u1) * s_b;
+    r.a02 = (as_h2((bytes & C.mask_hi) ^ C.magic_hi) + off_hi) * s_a;
+    r.a13 = (as_h2((next & C.mask_hi) ^ C.magic_hi) + off_hi) * s_a;
+    r.b02 = (as_h2((bytes & C.mask_lo) ^ C.magic_lo) + off_lo) * s_b;
+    r.b13 = (as_h2((next & C.mask_lo) ^ C.magic_lo) + off_lo) * s_b;
     return r;
 }
 __device__ __forceinline__ float row_dot(const RowRegs &k, const RowRegs &q) {
