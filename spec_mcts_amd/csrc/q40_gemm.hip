@@ -44,7 +44,8 @@ constexpr int GEMM_STAGES = 6;
 // six slots, 12.8 with eight and with twelve.  At 64 rows and more six are as good or better (wo, w2 at 512 rows 36.9, 37.4 and 37.7 us with six, eight and ten).
 constexpr int gemm_dma_slots(int tiles) { return tiles <= 3 ? 8 : 6; }
 // slots of the kernels whose stages hold two steps: up to `most`, as many as fit.  w1|w3 at 37 rows of the 7B shape 25.5 us with six, 21.6 with eight,
-// 22.0 with twelve; at 100 rows 30.0, 29.6.  The K-sliced kernel: at 37 rows 9.2 and 9.0, at 100 rows, where a slice has few stages, 16.6 and 17.0.
+// 22.0 with twelve; at 100 rows 30.0, 29.6.  The K-sliced kernel: at 37 rows 9.2 and 9.0, at 100 rows, where a slice has few stages, 16.6 and 17.0;
+// nine to twelve slots are within 0.3 % of eight from 5 to 48 rows.
 constexpr int gemm_slots(int stage, int most) { return 160 * 1024 / stage < most ? 160 * 1024 / stage : most; }
 constexpr int GEMM_DMA_WAVE_MAX_WGS = 256;
 constexpr int GS_WBLOCK = 8 * 128 + 64;        // the 8 rows one wave fetches, padded by 16 banks: the four row groups a
@@ -71,12 +72,15 @@ __device__ __forceinline__ void gemm_wait_vm() { asm volatile("s_waitcnt vmcnt(%
 template <int PER>
 __device__ __forceinline__ void gemm_wait_dma(int stages) {
     switch (stages) {
+        case 8: gemm_wait_vm<8 * PER>(); break;
+        case 7: gemm_wait_vm<7 * PER>(); break;
+        case 6: gemm_wait_vm<6 * PER>(); break;
         case 5: gemm_wait_vm<5 * PER>(); break;
         case 4: gemm_wait_vm<4 * PER>(); break;
         case 3: gemm_wait_vm<3 * PER>(); break;
         case 2: gemm_wait_vm<2 * PER>(); break;
         case 1: gemm_wait_vm<1 * PER>(); break;
-        default: gemm_wait_vm<0>(); break;              // (a ring of eight slots asks for five at most; waits for more than asked)
+        default: gemm_wait_vm<0>(); break;              // (a ring of eleven slots asks for eight at most)
     }
 }
 
@@ -1029,7 +1033,9 @@ __global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_kg_kern
 template <int TILES> struct SwigluShape {
     static constexpr int SC = 1024;                                  // scales: [group kk][gate | up] x 256
     static constexpr int STAGE = KG_W + SC + 2 * TILES * 1024;
-    static constexpr int SLOTS = gemm_slots(STAGE, 8);
+    // One row tile: eleven slots, steps behind 300 rows of the 7B model 1918, 2023 and 2046 us at 5, 10 and 16 branches with eight, 1895, 2001
+    // and 2038 with eleven (ten: the same).  Two and three: seven to eleven within 1.2 % of eight either way, by the card; from four on they are as good.
+    static constexpr int SLOTS = gemm_slots(STAGE, TILES == 1 ? 11 : 8);
     static constexpr int LDS = SLOTS * STAGE;
     static constexpr int PER = 4 + TILES;                            // DMA instructions of a step
     static constexpr int OP = 128 + 4;                               // floats per row of a group's sums in LDS
