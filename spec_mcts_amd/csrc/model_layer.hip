@@ -177,7 +177,7 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
     const int M = run.M, nq = run.nq;
     // the RMSNorm of the residual stream and the linears behind it: to slab_a.  With few rows the RMSNorm is made inside the linears' launch.
     auto norm_linears = [&](const void *weight, float eps, int nseg, const void *const *w, const int *n) -> int {
-        if (S.pending == 0 || M > S.norm_in_rows || run.blocks || smh_q40_norm_in_fits(M, L.dim, nseg, n) != 1) {
+        if (S.pending == 0 || M > S.norm_in_rows || run.blocks || !norm_inside_fits(M, L.dim, nseg, n)) {
             if (int r = run.norm(weight, eps, run.swiglu ? ask(L, run.blocks, M, L.dim, nseg, w, n, false, WARM_FROM_NORM, 256) : WarmWeights{})) return r;
             return matmul_partial_tiled(b.xn, M, L.dim, L.dim, nseg, w, n, b.slab_a, b.slab_a_bytes, run.blocks, stream);
         }
@@ -185,7 +185,7 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
         if (int r = smh_partial_residual_sumsq(b.slab_b, S.pending, M, L.dim, S.h, h_out, b.sums, stream)) return r;
         S.h = h_out;
         S.pending = 0;
-        return smh_q40_matmul_partial_tiled_norm(h_out, L.dim, b.sums, weight, eps, M, L.dim, nseg, w, n, b.slab_a, b.slab_a_bytes, stream);
+        return matmul_partial_tiled_norm(h_out, L.dim, b.sums, weight, eps, M, L.dim, nseg, w, n, b.slab_a, b.slab_a_bytes, true, stream);
     };
     // ---- attention ----
     const int rep = L.heads / L.kv_heads;

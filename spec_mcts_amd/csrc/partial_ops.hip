@@ -609,9 +609,15 @@ extern "C" int smh_q40_norm_in_fits(int M, int K, int nseg, const int *n) {
     return st < 0 ? st : (gemv_norm_in_fits(p) ? 1 : 0);
 }
 
-extern "C" int smh_q40_matmul_partial_tiled_norm(const void *h, long ldh, const void *sums, const void *norm_weight, float eps,
-                                                 int M, int K, int nseg, const void *const *tiled, const int *n,
-                                                 void *partial, size_t partial_bytes, smh_stream_t stream) {
+namespace smh {
+bool norm_inside_fits(int M, int K, int nseg, const int *n) {
+    MatmulParams p;
+    return M > 0 && M <= SMH_GEMV_MAX_M && K % 32 == 0 &&
+           fill_params(p, nullptr, M, K, K, nseg, nullptr, nullptr, n, "norm_inside_fits", true) >= 0 && (gemv_norm_in_fits(p) || gemv_norm_step_fits(p));
+}
+
+int matmul_partial_tiled_norm(const void *h, long ldh, const void *sums, const void *norm_weight, float eps, int M, int K, int nseg, const void *const *tiled,
+                              const int *n, void *partial, size_t partial_bytes, bool steps, smh_stream_t stream) {
     const char *who = "smh_q40_matmul_partial_tiled_norm";
     MatmulParams p;
     int st = fill_params(p, h, M, K, ldh, nseg, tiled, nullptr, n, who, true);
@@ -623,7 +629,7 @@ extern "C" int smh_q40_matmul_partial_tiled_norm(const void *h, long ldh, const 
     SMH_REQUIRE(((uintptr_t)h & 15) == 0 && ((uintptr_t)norm_weight & 15) == 0 && ((uintptr_t)sums & 15) == 0, "%s: h, norm_weight and sums must be 16-byte aligned", who);
     for (int i = 0; i < nseg; ++i)
         SMH_REQUIRE(tiled[i] && ((uintptr_t)tiled[i] & 127) == 0, "%s: weight %d is null or not 128-byte aligned", who, i);
-    SMH_REQUIRE(gemv_norm_in_fits(p), "%s: %d rows x K-slices of %d rows exceed %d bytes (ask smh_q40_norm_in_fits first)", who, M,
+    SMH_REQUIRE(gemv_norm_in_fits(p) || (steps && gemv_norm_step_fits(p)), "%s: %d rows x K-slices of %d rows exceed %d bytes (ask smh_q40_norm_in_fits first)", who, M,
                 p.steps_per_slice * 32, SMH_NORM_IN_MAX_XS_BYTES);
     size_t need = (size_t)p.ksplit * M * p.n_total * sizeof(float);
     SMH_REQUIRE(partial_bytes >= need, "%s: partial buffer %zu < %zu bytes", who, partial_bytes, need);
@@ -634,6 +640,13 @@ extern "C" int smh_q40_matmul_partial_tiled_norm(const void *h, long ldh, const 
     p.norm_ss = (const float *)sums;
     p.norm_eps = eps;
     return gemv_launch(p, (hipStream_t)stream);
+}
+}  // namespace smh
+
+extern "C" int smh_q40_matmul_partial_tiled_norm(const void *h, long ldh, const void *sums, const void *norm_weight, float eps,
+                                                 int M, int K, int nseg, const void *const *tiled, const int *n,
+                                                 void *partial, size_t partial_bytes, smh_stream_t stream) {
+    return matmul_partial_tiled_norm(h, ldh, sums, norm_weight, eps, M, K, nseg, tiled, n, partial, partial_bytes, false, stream);
 }
 
 static int reduce_launch(const void *partial, int ksplit, int M, int n_total, int col0, int N, void *c, long ldc,

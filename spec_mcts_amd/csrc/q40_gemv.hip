@@ -52,6 +52,8 @@ constexpr int RING_BYTES = RING_STAGES * STAGE_BYTES;                        // 
 constexpr int STAGE_BYTES_NO_X = STAGE_W_BYTES + STAGE_S_BYTES;             // 4352
 constexpr int RING_BYTES_NO_X = RING_STAGES * STAGE_BYTES_NO_X;             // 8704 per wave
 
+constexpr int NORM_STEP_OCTETS = 4;        // LAYOUT 4: k-octets of norm weights per thread, K-slices of up to 8192 rows
+
 typedef const __attribute__((address_space(1))) void *gptr_t;
 typedef __attribute__((address_space(3))) void *lptr_t;
 
@@ -202,9 +204,10 @@ __device__ __forceinline__ void gemv_consume(const uint8_t *stage, int k0, int K
 // pairs come out of (x, x2, x >> 8, x2 >> 8) and the scales arrive in the order of the row pairs.
 // Same operands into the same MFMAs in the same order as gemv_consume: the results are bit-identical.
 // `xrow`: the 8 activations k0 + 8g .. of this lane's batch row when they do not come from the stage (nullptr otherwise)
-template <bool RAGGED, bool XROW = false>
+// `norm`: the 8 norm weights of the same k when the stage holds the residual stream (nullptr otherwise), r: 1 / rms of this lane's row
+template <bool RAGGED, bool XROW = false, bool NORM = false>
 __device__ __forceinline__ void gemv_consume_tiled(const uint8_t *stage, int k0, int K, int lane, const GemvConsts &C,
-                                                   f4 (&acc)[2][2][4], const half_t *xrow = nullptr) {
+                                                   f4 (&acc)[2][2][4], const half_t *xrow = nullptr, const half_t *norm = nullptr, float r = 0.f) {
     const int c = lane & 15, g = lane >> 4;
     u32x4 wq[4];
 #pragma unroll
@@ -212,6 +215,11 @@ __device__ __forceinline__ void gemv_consume_tiled(const uint8_t *stage, int k0,
     h8 xv;
     if constexpr (XROW) xv = *reinterpret_cast<const h8 *>(xrow);      // (no select between two pointers: this stays an LDS read)
     else xv = *reinterpret_cast<const h8 *>(stage + STAGE_W_BYTES + STAGE_S_BYTES + c * 64 + 16 * g);
+    if constexpr (NORM) {
+        const h8 wv = *reinterpret_cast<const h8 *>(norm);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) xv[i] = scale_to_half(xv[i], r) * wv[i];      // the roundings of partial_rmsnorm_kernel
+    }
     if constexpr (RAGGED) {
         if (k0 + 8 * g >= K) {
 #pragma unroll
@@ -241,8 +249,13 @@ __device__ __forceinline__ void gemv_consume_tiled(const uint8_t *stage, int k0,
 
 // LAYOUT 0: checkpoint layout; 1: tiled weights (smh_q40_tile); 2: tiled weights and activations made from the
 // gate|up slabs by the workgroup itself (p.gu_partial): SiLU(gate) * up needs no launch of its own; 3: tiled weights
-// and activations made from the residual stream by the workgroup itself (p.norm_w, p.norm_ss): RMSNorm needs only
-// the small launch that adds the slabs and leaves the sums of squares
+// and activations made from the residual stream by the workgroup itself (p.norm_w, p.norm_ss), one row: RMSNorm needs only
+// the small launch that adds the slabs and leaves the sums of squares; 4: the same for 2 rows and more.  There a workgroup's share of the
+// rows grows with them, up to 80 KB for w1|w3 of dim 8192, and with it a prologue that no weight is consumed in.  So the stages bring the
+// residual stream, and every wave normalises the eight values of its operand on their way into the matrix core: 28 vector instructions more on the 190 of a step
+// that waits for HBM.  us a step of three layers of dim 8192 behind 1024 rows, w1|w3 behind a launch of RMSNorm's own and wq|wk|wv in form 3 / w1|w3 in form 4 /
+// both: 4 branches 489 / 478 / 477, 10 511 / 503 / 499, 16 527 / 522 / 515; one branch, both in form 3 and in form 4: 466 and 472.  32 layers of dim 4096 behind 64
+// rows, with launches of RMSNorm's own and in form 4: 5 branches 2006 and 1927, 10 2125 and 2020, 16 2225 and 2125.
 template <int LAYOUT>
 __global__ __launch_bounds__(GEMV_WAVES * 64) void q40_gemv_kernel(MatmulParams p) {
     constexpr int WAVES = GEMV_WAVES;
@@ -251,6 +264,7 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void q40_gemv_kernel(MatmulParams 
     constexpr bool TILED = LAYOUT != 0;
     constexpr bool SILU_IN = LAYOUT == 2;
     constexpr bool NORM_IN = LAYOUT == 3;
+    constexpr bool NORM_STEP = LAYOUT == 4;
     constexpr bool X_IN_LDS = SILU_IN || NORM_IN;                   // activations: xs[M][slice rows] behind the rings
     constexpr int PER_STAGE = X_IN_LDS ? 5 : 6;                     // vector-memory instructions per stage
     constexpr int STAGE = X_IN_LDS ? STAGE_BYTES_NO_X : STAGE_BYTES;
@@ -332,9 +346,10 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void q40_gemv_kernel(MatmulParams 
     // weight stages right behind them, so that both are in flight together.
     half_t *xs = reinterpret_cast<half_t *>(lds + WAVES * RING);
     const int slice_k0 = step0 * 32, slice_rows = (step1 - step0) * 32;
-    // a row of xs is 16 bytes longer than its data: the 16 lanes that read one k-octet of 16 different rows would
+    // a row of xs is 16 bytes longer than its data (SILU_IN; NORM_IN has one row): the 16 lanes that read one k-octet of 16 different rows would
     // otherwise hit the same LDS banks whenever the slice is a multiple of 128 bytes long
     const int xs_pitch = slice_rows + 8;
+    [[maybe_unused]] float r_c = 0.f;
     if constexpr (SILU_IN) {
         constexpr int MAXQ = SMH_SILU_IN_MAX_M * SMH_SILU_IN_MAX_K / 4 / THREADS;     // quads of columns per thread
         f4 ga[MAXQ], ua[MAXQ];
@@ -377,62 +392,60 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void q40_gemv_kernel(MatmulParams 
         }
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // xs is complete; the DMA ring stays in flight
     } else if constexpr (NORM_IN) {
-        // the loads of this thread's share of h (eight consecutive k of one row at a time), of the matching norm
-        // weights and, in the first threads, of a row's sums of squares go out first, the weight stages right
-        // behind them
+        // the loads of this thread's share of the row, of the matching norm weights and of the row's sums of squares go out first, the weight stages
+        // right behind them
         constexpr int MAXO = (SMH_NORM_IN_MAX_XS_BYTES / 16 + THREADS - 1) / THREADS;     // k-octets per thread
-        float *s_r = reinterpret_cast<float *>(xs + (long)p.M * xs_pitch);           // r[m], behind xs
         h8 hv[MAXO], wv[MAXO];
-        const int octs = slice_rows / 8, total = p.M * octs;
-        // item idx = (row idx / octs, octet idx % octs); idx < 1760 and octs <= 1760, so the quotient from a float
-        // reciprocal is exact (an integer division costs ~25 instructions per item here)
-        const float inv_octs = 1.0f / (float)max(octs, 1);
-        auto row_of = [&](int idx) { return (int)(((float)idx + 0.5f) * inv_octs); };
 #pragma unroll
         for (int i = 0; i < MAXO; ++i) {
-            const int idx = tid + i * THREADS;
-            if (idx < total) {
-                const int m = row_of(idx), k = slice_k0 + 8 * (idx - m * octs);
-                if (k < p.K) {
-                    hv[i] = *reinterpret_cast<const h8 *>(p.a + (long)m * p.lda + k);
-                    wv[i] = *reinterpret_cast<const h8 *>(p.norm_w + k);
-                } else {
-                    hv[i] = h8{0, 0, 0, 0, 0, 0, 0, 0};
-                    wv[i] = hv[i];
-                }
+            const int k = 8 * (tid + i * THREADS);
+            if (k < slice_rows) {
+                hv[i] = *reinterpret_cast<const h8 *>(p.a + slice_k0 + k);
+                wv[i] = *reinterpret_cast<const h8 *>(p.norm_w + slice_k0 + k);
             }
         }
+        const f4 *ss4 = reinterpret_cast<const f4 *>(p.norm_ss);
         f4 ssv[SMH_NORM_SUMS / 4];
-        if (tid < p.M) {
 #pragma unroll
-            for (int j = 0; j < SMH_NORM_SUMS / 4; ++j) ssv[j] = *reinterpret_cast<const f4 *>(p.norm_ss + (long)tid * SMH_NORM_SUMS + 4 * j);
-        }
+        for (int j = 0; j < SMH_NORM_SUMS / 4; ++j) ssv[j] = ss4[j];
 #pragma unroll
         for (int i = 0; i < RING_STAGES; ++i)
             if (i < n_steps) issue(ring + i * STAGE, first + i * WAVES);
-        if (tid < p.M) {
-            float sum = 0.f;
+        float sum = 0.f;
 #pragma unroll
-            for (int j = 0; j < SMH_NORM_SUMS; ++j) sum += ssv[j / 4][j % 4];
-            s_r[tid] = rms_factor(sum, p.K, p.norm_eps);
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // r[] is complete
+        for (int j = 0; j < SMH_NORM_SUMS; ++j) sum += ssv[j / 4][j % 4];
+        const float r = rms_factor(sum, p.K, p.norm_eps);
 #pragma unroll
         for (int i = 0; i < MAXO; ++i) {
-            const int idx = tid + i * THREADS;
-            if (idx < total) {
-                const int m = row_of(idx);
-                const float r = s_r[m];
+            const int k = 8 * (tid + i * THREADS);
+            if (k < slice_rows) {
                 h8 o;
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {                  // the roundings of partial_rmsnorm_kernel
-                    const half_t nv = scale_to_half(hv[i][j], r);
-                    o[j] = nv * wv[i][j];
-                }
-                *reinterpret_cast<h8 *>(xs + (long)m * xs_pitch + 8 * (idx - m * octs)) = o;
+                for (int j = 0; j < 8; ++j) o[j] = scale_to_half(hv[i][j], r) * wv[i][j];      // the roundings of partial_rmsnorm_kernel
+                *reinterpret_cast<h8 *>(xs + k) = o;
             }
         }
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // xs is complete; the DMA ring stays in flight
+    } else if constexpr (NORM_STEP) {
+        // the slice's norm weights behind the rings (K is a multiple of 32: steps are whole), 1 / rms of row c in lane (g, c)
+        f4 ssv[SMH_NORM_SUMS / 4];
+#pragma unroll
+        for (int j = 0; j < SMH_NORM_SUMS / 4; ++j) ssv[j] = *reinterpret_cast<const f4 *>(p.norm_ss + (long)min(c, p.M - 1) * SMH_NORM_SUMS + 4 * j);
+        h8 wv[NORM_STEP_OCTETS];
+#pragma unroll
+        for (int i = 0; i < NORM_STEP_OCTETS; ++i)
+            if (8 * (tid + i * THREADS) < slice_rows) wv[i] = *reinterpret_cast<const h8 *>(p.norm_w + slice_k0 + 8 * (tid + i * THREADS));
+#pragma unroll
+        for (int i = 0; i < RING_STAGES; ++i)
+            if (i < n_steps) issue(ring + i * STAGE, first + i * WAVES);
+#pragma unroll
+        for (int i = 0; i < NORM_STEP_OCTETS; ++i)
+            if (8 * (tid + i * THREADS) < slice_rows) *reinterpret_cast<h8 *>(xs + 8 * (tid + i * THREADS)) = wv[i];
+        float sum = 0.f;
+#pragma unroll
+        for (int j = 0; j < SMH_NORM_SUMS; ++j) sum += ssv[j / 4][j % 4];
+        r_c = rms_factor(sum, p.K, p.norm_eps);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // the weights are there; the DMA ring stays in flight
     } else {
 #pragma unroll
         for (int i = 0; i < RING_STAGES; ++i)
@@ -449,6 +462,7 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void q40_gemv_kernel(MatmulParams 
         else if (later == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER_STAGE) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if constexpr (X_IN_LDS) gemv_consume_tiled<false, true>(ring + stage * STAGE, 0, p.K, lane, C, acc, xlane + (first + i * WAVES - step0) * 32);
+        else if constexpr (NORM_STEP) gemv_consume_tiled<false, false, true>(ring + stage * STAGE, 0, p.K, lane, C, acc, nullptr, xs + (first + i * WAVES - step0) * 32 + 8 * g, r_c);
         else if constexpr (TILED) gemv_consume_tiled<false>(ring + stage * STAGE, 0, p.K, lane, C, acc);
         else gemv_consume<false>(ring + stage * STAGE, 0, p.K, c, g, C, acc);
         if (i + RING_STAGES < n_steps) {
@@ -544,6 +558,10 @@ void gemv_fill_plan(MatmulParams &p) {
     gemv_plan(p.units, p.K, GEMV_WAVES, &p.ksplit, &p.steps_per_slice);
 }
 
+bool gemv_norm_step_fits(const MatmulParams &p) {
+    return p.M <= SMH_GEMV_MAX_M && p.K % 32 == 0 && p.steps_per_slice * 32 <= NORM_STEP_OCTETS * 8 * GEMV_WAVES * 64;
+}
+
 bool gemv_norm_in_fits(const MatmulParams &p) {
     return p.M <= SMH_GEMV_MAX_M && (size_t)p.M * (p.steps_per_slice * 32 + 8) * sizeof(half_t) <= SMH_NORM_IN_MAX_XS_BYTES;
 }
@@ -553,8 +571,11 @@ int gemv_launch(const MatmulParams &p, hipStream_t stream) {
     dim3 grid((unsigned)p.units_pad, (unsigned)p.ksplit);
     size_t lds = (size_t)waves * RING_BYTES;                       // rings, reused for the [waves][M][256] sums
     const size_t red = (size_t)waves * p.M * GEMV_COLS * sizeof(float);
-    if (p.tiled && (p.gu_partial != nullptr || p.norm_w != nullptr))   // rings without activation tiles, xs (and r[]) behind them
-        lds = (size_t)waves * RING_BYTES_NO_X + (size_t)p.M * (p.steps_per_slice * 32 + 8) * sizeof(half_t) + SMH_GEMV_MAX_M * sizeof(float);
+    if (p.tiled && (p.gu_partial != nullptr || p.norm_w != nullptr))   // rings without activation tiles, xs behind them
+        lds = (size_t)waves * RING_BYTES_NO_X + (size_t)p.M * (p.steps_per_slice * 32 + 8) * sizeof(half_t);
+    // RMSNorm inside: one row in LDS, more step by step (figures: q40_gemv_kernel)
+    const bool norm_step = p.tiled && p.norm_w != nullptr && p.gu_partial == nullptr && (p.M > 1 || !gemv_norm_in_fits(p));
+    if (norm_step) lds = (size_t)waves * RING_BYTES + (size_t)p.steps_per_slice * 64;
     if (red > lds) lds = red;
     if (p.tiled) {
         if (p.gu_partial != nullptr) {
@@ -571,12 +592,14 @@ int gemv_launch(const MatmulParams &p, hipStream_t stream) {
                 return (int)lds_ok;
             }
             hipLaunchKernelGGL((q40_gemv_kernel<2>), grid, dim3(256), lds, stream, p);
-        } else if (p.norm_w != nullptr) {
-            if (!gemv_norm_in_fits(p)) {
+        } else if (norm_step) {
+            if (!gemv_norm_step_fits(p)) {
                 set_error("q40 gemv: %d rows x K-slices of %d rows do not fit next to the weight rings (RMSNorm inside the matmul)", p.M,
                           p.steps_per_slice * 32);
                 return -1;
             }
+            hipLaunchKernelGGL((q40_gemv_kernel<4>), grid, dim3(256), lds, stream, p);
+        } else if (p.norm_w != nullptr) {
             static const hipError_t lds_ok = hipFuncSetAttribute((const void *)q40_gemv_kernel<3>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                                                  80 * 1024);
             if (lds_ok != hipSuccess) {

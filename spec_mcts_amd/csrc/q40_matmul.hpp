@@ -136,6 +136,7 @@ __device__ __forceinline__ h8 rope_eight(f4 mine0, f4 mine1, f4 other0, f4 other
 
 void gemv_fill_plan(MatmulParams &p);
 int gemv_launch(const MatmulParams &p, hipStream_t stream);
+bool gemv_norm_step_fits(const MatmulParams &p);   // ... or, where not, step by step
 bool gemv_norm_in_fits(const MatmulParams &p);     // after gemv_fill_plan: can RMSNorm be made inside the launch
 void gemm_fill_plan(MatmulParams &p);
 bool gemm_blocks_fit(const MatmulParams &p, MatmulParams &b);          // after gemm_fill_plan

@@ -314,10 +314,8 @@ class Transformer(nn.Module):
         self.attn_single_launch = True     # up to 16 queries per kv head: prefix slices, suffix passes and the merge in one launch
                                            # (above, the one workgroup that merges a kv head's query tiles takes longer than a launch)
         self.norm_in_matmul = True         # RMSNorm made by the matmul that consumes it (a shorter launch in between) ...
-        # ... up to this many rows: at 10 rows of 4096 the matmul's longer prologue costs what it saves (2.364 against 2.358 ms a step);
-        # rows of 8192 are twice the work for the one workgroup that owns a row in the other form (3 layers, 3 branches: 499 against
-        # 511 us a step, 10: 546 against 552, 16: 568 against 571)
-        self.norm_in_max_rows = 2 if params.dim < 8192 else 16
+        # ... up to this many rows, where the linears are GEMVs (32 layers of dim 4096 behind 64 rows: 5 branches 2006 -> 1927 us a step, 16 2225 -> 2125)
+        self.norm_in_max_rows = K.SMH_GEMV_MAX_M
         self._norm_in_ok = {}
         self.attn_from_qkv = True          # where the attention is one launch it takes the wq|wk|wv product itself
         self.decode_stack = True           # up to 4 branches (multi-head attention): all layers of a decode step in one launch

@@ -85,6 +85,23 @@ def test_70b_architecture_layer(B, P):
     _steps(cfg, 74, B, P=P, std=0.02, rtol=1e-2, atol=1e-2, steps=2 if P > 100 else 3)
 
 
+def test_rmsnorm_inside_a_launch_whose_slices_do_not_fit():
+    """The 70B shape's w1|w3 (K-slices of 4096 rows): up to three branches fit next to the rings, from four on each step is normalised on its way into the
+    matrix core.  The same bits as with launches of RMSNorm's own."""
+    _, _, model = _build(ARCH_70B_LAYER, 83, 0.02)
+    gen = torch.Generator().manual_seed(84)
+    prompt = torch.randint(0, 512, (1, 9), generator=gen).cuda()
+    for B in (1, 3, 4, 10, 16):
+        tok = torch.randint(0, 512, (B, 1), generator=gen).cuda()
+        outs = []
+        for inside in (True, False):
+            model.norm_in_matmul = inside
+            model.resetSeq()
+            outs.append([model(prompt, 0).clone(), model(tok, 9).clone(), model(tok, 10).clone()])
+        for x, y in zip(*outs):
+            assert x.isfinite().all() and torch.equal(x, y), B
+
+
 LAYER_7B = dict(dim=4096, n_layers=2, n_heads=32, vocab_size=512, multiple_of=256, max_seq_len=8, max_prompt_seq_len=16)
 
 
