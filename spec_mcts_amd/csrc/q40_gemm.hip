@@ -68,19 +68,24 @@ typedef __attribute__((address_space(3))) void *lptr_t;
 template <int N>
 __device__ __forceinline__ void gemm_wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N < 63 ? N : 63) : "memory"); }
 // ... at most `stages` younger stages of PER DMA instructions each (4 with four waves, 2 with eight, 5 + row tiles in
-// a DMA wave at most).
-template <int PER>
+// a DMA wave at most).  A ring of eight slots asks for MOST = 5, one of eleven for eight.
+template <int PER, int MOST = 5>
 __device__ __forceinline__ void gemm_wait_dma(int stages) {
+    if constexpr (MOST > 5) {
+        static_assert(MOST <= 8, "a case each");
+        switch (stages) {
+            case 8: return gemm_wait_vm<8 * PER>();
+            case 7: return gemm_wait_vm<7 * PER>();
+            case 6: return gemm_wait_vm<6 * PER>();
+        }
+    }
     switch (stages) {
-        case 8: gemm_wait_vm<8 * PER>(); break;
-        case 7: gemm_wait_vm<7 * PER>(); break;
-        case 6: gemm_wait_vm<6 * PER>(); break;
         case 5: gemm_wait_vm<5 * PER>(); break;
         case 4: gemm_wait_vm<4 * PER>(); break;
         case 3: gemm_wait_vm<3 * PER>(); break;
         case 2: gemm_wait_vm<2 * PER>(); break;
         case 1: gemm_wait_vm<1 * PER>(); break;
-        default: gemm_wait_vm<0>(); break;              // (a ring of eleven slots asks for eight at most)
+        default: gemm_wait_vm<0>(); break;              // (waits for more than asked)
     }
 }
 
@@ -99,7 +104,7 @@ __device__ __forceinline__ void gemm_feed(int n, Issue issue) {
     if (n <= 0) return;
 #pragma unroll 1
     for (int i = 0; i < min(SLOTS - 2, n); ++i) issue(i);
-    gemm_wait_dma<PER>(min(SLOTS - 3, n - 1));
+    gemm_wait_dma<PER, SLOTS - 3>(min(SLOTS - 3, n - 1));
     gemm_barrier();
     int slot = 0;
     auto back = [&](int k) { return slot >= k ? slot - k : slot + SLOTS - k; };
@@ -114,7 +119,7 @@ __device__ __forceinline__ void gemm_feed(int n, Issue issue) {
     }
 #pragma unroll 1
     for (; i < n; i += 2) {
-        gemm_wait_dma<PER>(max(0, min(n - 1, i + SLOTS - 3) - (i + 2)));      // stages issued past stage i + 2
+        gemm_wait_dma<PER, SLOTS - 3>(max(0, min(n - 1, i + SLOTS - 3) - (i + 2)));      // stages issued past stage i + 2
         gemm_barrier();
         if (i + SLOTS - 2 < n) issue(back(2));
         if (i + SLOTS - 1 < n) issue(back(1));
