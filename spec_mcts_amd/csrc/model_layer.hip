@@ -27,8 +27,8 @@ constexpr int WARM_MAX_DIM = 8191, WARM_FROM_NORM = 3, WARM_FROM_ATTENTION = 4, 
 static int slices(int M, int K, int nseg, const int *n) { return smh_q40_matmul_plan_tiled(M, K, nseg, n); }
 // Launches of 17 rows and more (128-column blocks, SwiGLU inside w1|w3, the norms and the attention asking for the next weights) for a layer of fewer, too,
 // where all four linears have them: bound by latency both ways, they are fewer (no SiLU launch), leave 2 to 8 slabs instead of 5 to 16, and their weights are
-// on their way earlier.  7B architecture, 512 + 50 rows, us a step with the GEMVs and so: 5 branches 2059 and 1973, 8 2142 and 2027, 10 2219 and 2042, 12 2248
-// and 2063, 16 2376 and 2150.  (4, which the launch of all layers takes with probabilities
+// on their way earlier.  7B architecture, 512 + 50 rows, us a step with the GEMVs and so: 5 branches 1976 and 1946, 6 2009 and 1949, 8 2022 and 2007, 10 2119
+// and 2018, 12 2149 and 2040, 16 2275 and 2126.  (4, which the launch of all layers takes with probabilities
 // of 32 bits, not 16: 2150 there and 1950 so.)  SwiGLU inside at 17 / 24 / 32 branches: 2360 / 2432 / 2495 -> 2250 /
 // 2318 / 2361.  Behind short prompts a decode step stays what it was (ATTN_TILES_MIN_PROMPT: two evaluations that differ in one rounding drift apart there).
 constexpr int BLOCKS_MIN_ROWS = 5, BLOCKS_MIN_PROMPT = 96;
@@ -177,7 +177,7 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
     const int M = run.M, nq = run.nq;
     // the RMSNorm of the residual stream and the linears behind it: to slab_a.  With few rows the RMSNorm is made inside the linears' launch.
     auto norm_linears = [&](const void *weight, float eps, int nseg, const void *const *w, const int *n) -> int {
-        if (S.pending == 0 || M > S.norm_in_rows || run.blocks || !norm_inside_fits(M, L.dim, nseg, n)) {
+        if (S.pending == 0 || M > S.norm_in_rows || run.blocks || ((uintptr_t)weight & 15) != 0 || !norm_inside_fits(M, L.dim, nseg, n)) {
             if (int r = run.norm(weight, eps, run.swiglu ? ask(L, run.blocks, M, L.dim, nseg, w, n, false, WARM_FROM_NORM, 256) : WarmWeights{})) return r;
             return matmul_partial_tiled(b.xn, M, L.dim, L.dim, nseg, w, n, b.slab_a, b.slab_a_bytes, run.blocks, stream);
         }

@@ -102,6 +102,25 @@ def test_rmsnorm_inside_a_launch_whose_slices_do_not_fit():
             assert x.isfinite().all() and torch.equal(x, y), B
 
 
+@pytest.mark.parametrize("B", [2, 5, 16])
+def test_norm_weights_that_are_not_aligned_to_16_bytes(B):
+    """Launches of GEMVs that normalise themselves read 16 bytes of them at a time; such weights go to the launch of RMSNorm's own: the same bits."""
+    _, _, model = _build(MANY, 85, 0.05)
+    gen = torch.Generator().manual_seed(86)
+    prompt, tok = torch.randint(0, 320, (1, 9), generator=gen).cuda(), torch.randint(0, 320, (B, 1), generator=gen).cuda()
+    outs = []
+    for offset in (0, 4):
+        for layer in model.layers:
+            for norm in (layer.attention_norm, layer.ffn_norm):
+                buf = torch.empty(256 + offset, dtype=torch.float16, device="cuda:0")
+                buf[offset:] = norm.weight
+                norm.weight.data = buf[offset:]
+        model.resetSeq()
+        outs.append([model(prompt, 0).clone(), model(tok, 9).clone(), model(tok, 10).clone()])
+    for x, y in zip(*outs):
+        assert x.isfinite().all() and torch.equal(x, y)
+
+
 LAYER_7B = dict(dim=4096, n_layers=2, n_heads=32, vocab_size=512, multiple_of=256, max_seq_len=8, max_prompt_seq_len=16)
 
 
