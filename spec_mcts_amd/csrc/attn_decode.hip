@@ -1994,11 +1994,17 @@ static int attn_plan_tw(int P, int Hkv) {
     return tw;
 }
 
-// The one-launch kernel.  From 32 kv heads on slices of ATT_ONE_TW rows, also where narrower ones would give each compute unit one: what they leave to the
-// merge, and the second wave of a query's own rows that they take the place of, cost more (us a step of the 7B architecture, slices of 32 rows and of 64, 10 / 60 / 120
-// rows of their own: 5 branches behind 100 rows 1905 / 1913 / 1938 and 1892 / 1896 / 1916; 16 behind 256 2072 / 2116 / 2168 and 2010 / 2026 / 2088; 10 behind 400 2085 /
-// 2188 / 2347 and 1986 / 1999 / 2066).  Below 96 rows results stay what they were (ATTN_TILES_MIN_PROMPT).
-static int attn_plan_one_tw(int P, int Hkv) { return Hkv >= 32 && P >= 96 ? ATT_ONE_TW : min(attn_plan_tw(P, Hkv), ATT_ONE_TW); }
+// The one-launch kernel fed by the q|k|v product.  From 32 kv heads on slices of ATT_ONE_TW rows, also where narrower ones would give each compute unit one: what
+// they leave to the merge, and the second wave of a query's own rows that they take the place of, cost more (us a step of the 7B architecture, slices of 32 rows and of
+// 64, 10 / 60 / 120 rows of their own: 5 branches behind 100 rows 1905 / 1913 / 1938 and 1892 / 1896 / 1916; 16 behind 256 2072 / 2116 / 2168 and 2010 / 2026 / 2088; 10
+// behind 400 2085 / 2188 / 2347 and 1986 / 1999 / 2066; us a call of 32 / 40 / 64 heads, slices as narrow and of 64 rows, 10 rows of their own: one branch behind 128 rows 10.1
+// / 10.1 / 10.6 and 9.9 / 9.8 / 10.2, four behind 256 11.1 / 11.1 / 12.0 and 10.1 / 10.5 / 12.0, 16 behind 128 12.7 / 12.7 / 13.6 and 11.9 / 11.8 / 12.4; 384 sizes of 4 to 16 branches, 10 to 120 own
+// rows, with the waves below: 1.08 times as fast at the mean, slowest 0.97, 64 heads of 12 branches behind 96 rows, 11.3 and 11.7 at 10 own rows, 19.9 and 14.2 at 120.)  One query keeps three slices of 32 rows
+// behind 96: 9.2 and 9.7 us with two.  Below 96 rows results stay what they were (ATTN_TILES_MIN_PROMPT).
+// (smh_shared_prefix_attn_one, whose queries are ready and whose slices end sooner, keeps the narrow ones: with wide ones 0.91 .. 0.97 times as fast
+// at 1 to 5 branches behind 96 and 128 rows, 32 and 40 heads, 1.0 .. 1.9 behind 256 and more.)
+static bool attn_wide_slices(int P, int Hkv, int queries) { return Hkv >= 32 && P >= (queries > 1 ? 96 : 97) && attn_plan_tw(P, Hkv) < ATT_ONE_TW; }
+static int attn_plan_one_tw(int P, int Hkv, int queries) { return attn_wide_slices(P, Hkv, queries) ? ATT_ONE_TW : min(attn_plan_tw(P, Hkv), ATT_ONE_TW); }
 
 // Two launches: rows of the prefix per workgroup and the number of workgroups that share one slice's query tiles.
 // Every slice leaves a partial per query, so wide slices mean less partial traffic; the CUs are filled first by
@@ -2027,10 +2033,13 @@ static int attn_plan_suffix_waves_two(long queries) {
 }
 
 // One-launch kernel: waves that share a query's suffix rows - as many as keep the launch within one round of
-// workgroups (two fit a compute unit).
-static int attn_plan_suffix_waves(int splits, int Bq, int Hkv) {
+// workgroups (two fit a compute unit).  wide (attn_wide_slices): four only where they leave a sixteenth of the round free.  A launch that four waves fill costs
+// more than two waves' longer walks (us a call, 10 / 30 / 60 / 120 own rows, two waves and four: 32 heads, 12 branches behind 200 rows 12.1 / 12.3 / 12.9 / 14.0 and
+// 13.5 / 13.7 / 13.8 / 14.5, 14 behind 128 11.7 / 11.8 / 12.4 / 13.4 and 12.9 / 13.1 / 13.3 / 14.3; 64 heads, 6 behind 96 10.3 / 10.4 / 11.0 / 12.7 and 11.3 /
+// 11.5 / 11.6 / 12.0); two waves where one would do may fill it (64 heads, 12 behind 96, one and two: 11.1 / 11.9 / 14.0 / 18.3 and 11.7 / 11.8 / 12.4 / 14.2).
+static int attn_plan_suffix_waves(int splits, int Bq, int Hkv, bool wide) {
     int nsub = 4;
-    while (nsub > 1 && (long)(splits + (Bq + 4 / nsub - 1) / (4 / nsub)) * Hkv > 512) nsub >>= 1;
+    while (nsub > 1 && (long)(splits + (Bq + 4 / nsub - 1) / (4 / nsub)) * Hkv > (wide && nsub == 4 ? 479 : 512)) nsub >>= 1;
     return nsub;
 }
 
@@ -2106,7 +2115,7 @@ static int shared_prefix_attn(const char *who, bool one, const void *q, void *ou
     else attn_plan(P, Hkv, p.Bq, &p.tw, &qgroups);
     p.splits = P > 0 ? (P + p.tw - 1) / p.tw : 0;
     if (one) {
-        p.suffix_waves = attn_plan_suffix_waves(p.splits, p.Bq, Hkv);
+        p.suffix_waves = attn_plan_suffix_waves(p.splits, p.Bq, Hkv, false);
         const int q_tiles = (p.Bq + 15) / 16;
         SMH_REQUIRE(q_tiles <= ATT_ONE_MAX_TILES && (size_t)Hkv * q_tiles * sizeof(uint32_t) <= ATT_COUNTER_BYTES,
                     "%s: %d queries per kv head (at most %d), %d kv heads", who, p.Bq, ATT_FUSED_MAX_Q, Hkv);
@@ -2332,7 +2341,7 @@ extern "C" int smh_shared_prefix_attn_qkv(const void *qkv_partial, int ksplit, v
     p.P = P; p.suffix_format = SMH_KV_Q40;
     p.scale_log2 = LOG2E / sqrtf((float)D);
     int qgroups = 1;
-    if (single_launch) p.tw = attn_plan_one_tw(P, Hkv);
+    if (single_launch) p.tw = attn_plan_one_tw(P, Hkv, p.Bq);
     else attn_plan(P, Hkv, p.Bq, &p.tw, &qgroups);
     p.splits = P > 0 ? (P + p.tw - 1) / p.tw : 0;
     p.qkv = (const float *)qkv_partial; p.qkv_ks = ksplit;
@@ -2341,7 +2350,7 @@ extern "C" int smh_shared_prefix_attn_qkv(const void *qkv_partial, int ksplit, v
     p.app_ks = (half_t *)cache_ks; p.app_vs = (half_t *)cache_vs;
     p.app_t = t_dev; p.app_smax = Smax;
     if (single_launch) {
-        p.suffix_waves = attn_plan_suffix_waves(p.splits, p.Bq, Hkv);
+        p.suffix_waves = attn_plan_suffix_waves(p.splits, p.Bq, Hkv, attn_wide_slices(P, Hkv, p.Bq));
         // workspace = [arrival counters | partials of splits + 1 passes]
         SMH_REQUIRE((size_t)Hkv * ((p.Bq + 15) / 16) * sizeof(uint32_t) <= ATT_COUNTER_BYTES, "%s: %d kv heads x %d query tiles", who, Hkv, (p.Bq + 15) / 16);
         size_t n_part = (size_t)(p.splits + 1) * Hkv * p.Bq;

@@ -241,8 +241,8 @@ def test_attention_fed_by_the_qkv_product_matches_the_three_launch_sequence(B, H
             assert torch.equal(a, b_), "appended cache rows differ"
 
 
-def _tiles_against_launches(qkv, H, Hkv, P, t, Smax, paged, g):
-    """smh_shared_prefix_attn_qkv_tiles and smh_partial_rope_append_kv + smh_shared_prefix_attn / smh_paged_prefix_attn on the same slabs and caches, of
+def _tiles_against_launches(qkv, H, Hkv, P, t, Smax, paged, g, one=False):
+    """smh_shared_prefix_attn_qkv_tiles (one: smh_shared_prefix_attn_qkv in one launch) and smh_partial_rope_append_kv + smh_shared_prefix_attn / smh_paged_prefix_attn on the same slabs and caches, of
     which nobody's rows are alike: the same rows appended, outputs within the bound of the tests below.  Returns the call and its output."""
     from spec_mcts_amd import kernels as K
     dev, D, B = "cuda:0", 128, qkv.M
@@ -268,7 +268,8 @@ def _tiles_against_launches(qkv, H, Hkv, P, t, Smax, paged, g):
         want = K.paged_prefix_attn(q, pages, t_dev, ck.view(-1, Hkv, 64), cv.view(-1, Hkv, 64), cks.view(-1, Hkv, 2), cvs.view(-1, Hkv, 2), False, *prefix, P, **common)
     else:
         want = K.shared_prefix_attn(q, *prefix, P, suffix_k=ck, suffix_v=cv, suffix_ks=cks, suffix_vs=cvs, Smax=Smax, n_kv_heads=Hkv, **common)
-    tiles = lambda: K.shared_prefix_attn_qkv_tiles(qkv, H, Hkv, D, cos, sin, pos_dev, *prefix, P, *mine, Smax, t_dev, pages=pages)
+    call = K.shared_prefix_attn_qkv if one else K.shared_prefix_attn_qkv_tiles
+    tiles = lambda: call(qkv, H, Hkv, D, cos, sin, pos_dev, *prefix, P, *mine, Smax, t_dev, pages=pages)
     got = tiles()
     torch.cuda.synchronize()
     assert torch.isfinite(got).all()
@@ -321,6 +322,25 @@ def test_tile_attention_over_long_branches(B, H, Hkv, queries, ksplit, P, t, pag
     n = (H + 2 * Hkv) * 128
     qkv = K.PartialProduct((torch.randn((ksplit, B, n), generator=g) * 1.5 / ksplit ** 0.5).to("cuda:0"), ksplit, B, n)
     _tiles_against_launches(qkv, H, Hkv, P, t, 128, paged, g)
+
+
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("B,H,ksplit,P,t", [
+    (1, 32, 2, 96, 5), (1, 32, 1, 97, 120), (2, 32, 2, 96, 1), (5, 32, 2, 95, 64), (5, 32, 1, 96, 0), (16, 32, 2, 97, 127), (10, 32, 3, 96, 31), (10, 32, 2, 129, 32), (11, 32, 2, 200, 33),
+    (12, 32, 1, 193, 120), (14, 32, 2, 128, 16), (16, 32, 2, 256, 63), (5, 32, 5, 400, 100), (16, 32, 2, 400, 17), (13, 32, 2, 511, 90), (8, 32, 2, 512, 40), (16, 32, 2, 704, 65),
+    (10, 40, 2, 96, 70), (12, 40, 16, 320, 40), (6, 64, 2, 128, 21), (12, 64, 9, 96, 50)])
+def test_one_launch_of_many_heads(B, H, ksplit, P, t, paged):
+    """smh_shared_prefix_attn_qkv in one launch from 32 kv heads on, against the three-launch sequence (bound: the test of sixteen queries a workgroup): its kernels by the
+    number of slabs (up to two, 8, 12, 16), prompts around the rows from which slices are 64 rows wide, last slices of 1 to 64 rows, one, two and four waves a query's own
+    rows with and without a table, of 0 rows, of one and of several turns of a walk.  What lies past the prompt and past a branch's rows is NaN, and the
+    counters are left ready for the next call."""
+    from spec_mcts_amd import kernels as K
+    g = torch.Generator().manual_seed(B + P + t)
+    n = 3 * H * 128
+    qkv = K.PartialProduct((torch.randn((ksplit, B, n), generator=g) * 1.5 / ksplit ** 0.5).to("cuda:0"), ksplit, B, n)
+    again, got = _tiles_against_launches(qkv, H, H, P, t, 128, paged, g, one=True)
+    for _ in range(2):
+        assert torch.equal(again(), got)
 
 
 @pytest.mark.parametrize("B,H,Hkv,P", [(17, 4, 4, 100), (20, 8, 2, 530), (100, 32, 32, 130), (40, 64, 8, 1030)])
