@@ -178,11 +178,13 @@ int smh_q40_matmul_partial_tiled_silu(const void *gate_up_partial, int gate_up_k
  * (fp32; added in index order they are smh_partial_rmsnorm's sum bit for bit).  smh_q40_matmul_partial_tiled_norm is
  * smh_q40_matmul_partial_tiled on a = RMSNorm(h) * norm_weight, which every workgroup makes for its own K-slice from h,
  * sums and norm_weight with smh_partial_rmsnorm's roundings; the slabs it leaves equal those of smh_partial_rmsnorm +
- * smh_q40_matmul_partial_tiled.  M rows x the K-slice must fit the workgroup's LDS: smh_q40_norm_in_fits says (1 / 0)
- * whether a shape does; where it does not, smh_partial_rmsnorm is the path. */
+ * smh_q40_matmul_partial_tiled.  It takes M rows x the K-slice of at most 27.5 KB: smh_q40_norm_in_fits says (1 / 0)
+ * whether a shape is; where it is not, smh_partial_rmsnorm is the path.  smh_decode_norm_in_fits: whether smh_decode_layer makes the RMSNorm in front of
+ * such a product inside it (from two rows on only the slice's norm weights need to fit: K-slices of up to 8192 rows). */
 int smh_partial_residual_sumsq(const void *partial, int ksplit, int M, int N, const void *h_in, void *h_out, void *sums,
                                smh_stream_t stream);
 int smh_q40_norm_in_fits(int M, int K, int nseg, const int *n);
+int smh_decode_norm_in_fits(int M, int K, int nseg, const int *n);
 int smh_q40_matmul_partial_tiled_norm(const void *h, long ldh, const void *sums, const void *norm_weight, float eps,
                                       int M, int K, int nseg, const void *const *tiled, const int *n,
                                       void *partial, size_t partial_bytes, smh_stream_t stream);

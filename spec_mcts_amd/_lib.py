@@ -61,6 +61,7 @@ SIGNATURES = {
     "smh_q40_matmul_partial_tiled_silu": (c_int, [_P, c_int, c_int, c_int, c_int, _P, _P, _P, c_size_t, _P]),
     "smh_partial_residual_sumsq": (c_int, [_P, c_int, c_int, c_int, _P, _P, _P, _P]),
     "smh_q40_norm_in_fits": (c_int, [c_int, c_int, c_int, _P]),
+    "smh_decode_norm_in_fits": (c_int, [c_int, c_int, c_int, _P]),
     "smh_q40_matmul_partial_tiled_norm": (c_int, [_P, c_long, _P, _P, c_float, c_int, c_int, c_int, _P, _P, _P, c_size_t, _P]),
     "smh_sample_topk_counts": (c_int, [_P, c_int, c_int, c_long, c_float, c_int, _P, _P, _P, c_int, _P]),
     "smh_tree_fork": (c_int, [_P, c_int, _P, _P, _P, _P, c_int, _P, c_long, c_int, _P, c_long, c_int, _P, _P]),

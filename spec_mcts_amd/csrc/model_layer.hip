@@ -177,7 +177,7 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
     const int M = run.M, nq = run.nq;
     // the RMSNorm of the residual stream and the linears behind it: to slab_a.  With few rows the RMSNorm is made inside the linears' launch.
     auto norm_linears = [&](const void *weight, float eps, int nseg, const void *const *w, const int *n) -> int {
-        if (S.pending == 0 || M > S.norm_in_rows || run.blocks || ((uintptr_t)weight & 15) != 0 || !norm_inside_fits(M, L.dim, nseg, n)) {
+        if (S.pending == 0 || M > S.norm_in_rows || run.blocks || ((uintptr_t)weight & 15) != 0 || smh_decode_norm_in_fits(M, L.dim, nseg, n) != 1) {
             if (int r = run.norm(weight, eps, run.swiglu ? ask(L, run.blocks, M, L.dim, nseg, w, n, false, WARM_FROM_NORM, 256) : WarmWeights{})) return r;
             return matmul_partial_tiled(b.xn, M, L.dim, L.dim, nseg, w, n, b.slab_a, b.slab_a_bytes, run.blocks, stream);
         }

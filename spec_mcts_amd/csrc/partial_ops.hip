@@ -609,13 +609,14 @@ extern "C" int smh_q40_norm_in_fits(int M, int K, int nseg, const int *n) {
     return st < 0 ? st : (gemv_norm_in_fits(p) ? 1 : 0);
 }
 
-namespace smh {
-bool norm_inside_fits(int M, int K, int nseg, const int *n) {
+extern "C" int smh_decode_norm_in_fits(int M, int K, int nseg, const int *n) {
     MatmulParams p;
-    return M > 0 && M <= SMH_GEMV_MAX_M && K % 32 == 0 &&
-           fill_params(p, nullptr, M, K, K, nseg, nullptr, nullptr, n, "norm_inside_fits", true) >= 0 && (gemv_norm_in_fits(p) || gemv_norm_step_fits(p));
+    if (M <= 0 || M > SMH_GEMV_MAX_M || K % 32 != 0) return 0;
+    int st = fill_params(p, nullptr, M, K, K, nseg, nullptr, nullptr, n, "smh_decode_norm_in_fits", true);
+    return st < 0 ? st : (gemv_norm_in_fits(p) || gemv_norm_step_fits(p) ? 1 : 0);
 }
 
+namespace smh {
 int matmul_partial_tiled_norm(const void *h, long ldh, const void *sums, const void *norm_weight, float eps, int M, int K, int nseg, const void *const *tiled,
                               const int *n, void *partial, size_t partial_bytes, bool steps, smh_stream_t stream) {
     const char *who = "smh_q40_matmul_partial_tiled_norm";

@@ -100,10 +100,9 @@ int shared_prefix_attn_qkv_tiles(const void *qkv_partial, int ksplit, void *out,
 int matmul_partial_tiled(const void *a, int M, int K, long lda, int nseg, const void *const *tiled, const int *n, void *partial, size_t partial_bytes,
                          bool blocks, smh_stream_t stream);
 int blocks_plan(int M, int K, int nseg, const int *n);
-// smh_q40_matmul_partial_tiled_norm; steps: also where a K-slice of all rows does not fit next to the rings (they are normalised step by step).
+// smh_q40_matmul_partial_tiled_norm; steps: whatever smh_decode_norm_in_fits takes.
 int matmul_partial_tiled_norm(const void *h, long ldh, const void *sums, const void *norm_weight, float eps, int M, int K, int nseg, const void *const *tiled,
                               const int *n, void *partial, size_t partial_bytes, bool steps, smh_stream_t stream);
-bool norm_inside_fits(int M, int K, int nseg, const int *n);
 // compute units that a launch of these leaves without a workgroup, in eights
 int swiglu_idle(int n_half);
 int attn_tiles_idle(int B, int H, int Hkv);

@@ -555,15 +555,15 @@ class Transformer(nn.Module):
         return self._page_table
 
     def _norm_in(self, M: int, Kd: int, ops) -> bool:
-        """RMSNorm inside the matmul that follows it: tiled weights, few rows, and rows x K-slice small enough for the
-        kernel's LDS (asked of the library once per shape)."""
+        """RMSNorm inside the matmul that follows it: tiled weights, few rows, and a shape that the layer calls take (asked of the
+        library once per shape)."""
         if not (self.norm_in_matmul and self.tiled_weights and M <= min(self.norm_in_max_rows, K.SMH_GEMV_MAX_M)
                 and isinstance(ops[0], K.TiledQ40)):
             return False
         key = (M, Kd, tuple(t.N for t in ops))
         ok = self._norm_in_ok.get(key)
         if ok is None:
-            ok = self._norm_in_ok[key] = K.norm_in_fits(M, Kd, list(key[2]))
+            ok = self._norm_in_ok[key] = K.decode_norm_in_fits(M, Kd, list(key[2]))
         return ok
 
     @torch.inference_mode()

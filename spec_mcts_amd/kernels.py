@@ -250,6 +250,14 @@ def norm_in_fits(M: int, Kd: int, ns) -> bool:
     return st == 1
 
 
+def decode_norm_in_fits(M: int, Kd: int, ns) -> bool:
+    """Does a layer call (LayerPass.decode) make the RMSNorm in front of linears of this shape inside their launch, where it is asked to?"""
+    import ctypes
+    st = _lib.load().smh_decode_norm_in_fits(M, Kd, len(ns), (ctypes.c_int * len(ns))(*ns))
+    check(min(st, 0), "smh_decode_norm_in_fits")
+    return st == 1
+
+
 def partial_residual_sumsq(p: PartialProduct, h_in: Optional[torch.Tensor]):
     """h = h_in + fp16(product), sums[m][0..15] = partial sums of squares of h's row m.  Returns (h, sums)."""
     lib = _lib.load()

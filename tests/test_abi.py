@@ -220,6 +220,24 @@ def test_layer_scratch_holds_every_slab_of_a_pass():
                 assert lib.smh_decode_scratch_bytes(layer, M, swiglu) >= need, (dim, swiglu, M)
 
 
+def test_rmsnorm_inside_the_launches_of_a_layer():
+    """up to 16 rows wherever a K-slice's norm weights fit, one row where they do or the row does; _norm_in of the model asks the same"""
+    from spec_mcts_amd import ModelArgs, Transformer, _lib, kernels as K
+    lib = _lib.load()
+    fits = lambda M, Kd, *ns: lib.smh_decode_norm_in_fits(M, Kd, len(ns), (ctypes.c_int * len(ns))(*ns))
+    for M in range(1, 17):
+        for Kd, ns in ((4096, (4096,) * 3), (6656, (6656,) * 3), (8192, (8192,) * 3), (8192, (28672, 28672)), (7168, (7168, 1024, 1024)), (14336, (512,))):
+            assert fits(M, Kd, *ns) == 1
+            assert lib.smh_q40_norm_in_fits(M, Kd, len(ns), (ctypes.c_int * len(ns))(*ns)) in (0, 1)
+        assert fits(M, 16384, 131072) == 0                 # (one K-slice of 16384 rows)
+    assert fits(1, 12288, 131072) == 1 and fits(2, 12288, 131072) == 0
+    assert fits(0, 4096, 4096) == fits(17, 4096, 4096) == fits(4, 4096 + 8, 4096) == 0 and fits(4, 4096, 100) < 0
+    model = Transformer(ModelArgs(dim=256, n_layers=1, n_heads=2, vocab_size=320, multiple_of=128))
+    for M, Kd in ((1, 4096), (12, 6144), (16, 6656), (9, 8192), (16, 8192)):
+        assert model._norm_in(M, Kd, [K.TiledQ40(None, Kd, Kd)] * 3)
+    assert not model._norm_in(17, 4096, [K.TiledQ40(None, 4096, 4096)] * 3)
+
+
 def test_columns_of_a_workgroup_above_128_rows():
     """which of the launches above 128 rows a shape takes (the GPU tests of each ask here), 0 where there is none"""
     from spec_mcts_amd import _lib

@@ -102,6 +102,22 @@ def test_rmsnorm_inside_a_launch_whose_slices_do_not_fit():
             assert x.isfinite().all() and torch.equal(x, y), B
 
 
+def test_rmsnorm_inside_wq_wk_wv_of_many_rows():
+    """16 rows of 6144: more than fits next to the rings row by row.  The same bits as with launches of RMSNorm's own."""
+    _, _, model = _build(dict(dim=6144, n_layers=2, n_heads=48, vocab_size=512, multiple_of=256, ffn_dim_multiplier=0.25, max_batch_size=16, max_seq_len=8,
+                              max_prompt_seq_len=16), 87, 0.02)
+    gen = torch.Generator().manual_seed(88)
+    prompt, tok = torch.randint(0, 512, (1, 9), generator=gen).cuda(), torch.randint(0, 512, (16, 1), generator=gen).cuda()
+    outs = []
+    for inside in (True, False):
+        model.norm_in_matmul = inside
+        model.resetSeq()
+        outs.append([model(prompt, 0).clone(), model(tok, 9).clone(), model(tok, 10).clone()])
+    assert model._norm_in_ok and all(model._norm_in_ok.values())
+    for x, y in zip(*outs):
+        assert x.isfinite().all() and torch.equal(x, y)
+
+
 @pytest.mark.parametrize("B", [2, 5, 16])
 def test_norm_weights_that_are_not_aligned_to_16_bytes(B):
     """Launches of GEMVs that normalise themselves read 16 bytes of them at a time; such weights go to the launch of RMSNorm's own: the same bits."""
