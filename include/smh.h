@@ -134,10 +134,11 @@ int smh_q40_swiglu_fits(int M, int K, int n_half);
 int smh_q40_swiglu_columns(int M, int K, int n_half);
 /* columns of either weight that the first of two launches multiplies (by workgroups of 384, the rest by workgroups of 256); 0: one launch */
 int smh_q40_swiglu_first_columns(int M, int K, int n_half);
-/* What the launch in front of a product of 17 .. 128 rows on tiled weights asks for ahead of it (swiglu: of smh_q40_matmul_tiled_swiglu, else of
- * smh_q40_matmul_partial_tiled): per weight the number of 128-byte lines of the first `stages` stages of all workgroups, the first byte and the byte behind
+/* What the launch in front of a product of 17 .. 128 rows on tiled weights asks for ahead of it (form bit 0: of smh_q40_matmul_tiled_swiglu, else of
+ * smh_q40_matmul_partial_tiled; bit 1: of the same products in a layer call that takes them on 128-column blocks from fewer rows on, smh_decode_layer_form):
+ * per weight the number of 128-byte lines of the first `stages` stages of all workgroups, the first byte and the byte behind
  * the last.  1: it does, 0: the product takes another kernel and nothing is asked for.  Host arithmetic only. */
-int smh_q40_warm_span(int M, int K, int nseg, const int *n, int swiglu, int stages, long *lines, long *first, long *end);
+int smh_q40_warm_span(int M, int K, int nseg, const int *n, int form, int stages, long *lines, long *first, long *end);
 int smh_q40_matmul_tiled_swiglu(const void *a, int M, int K, long lda, const void *tiled_gate, const void *tiled_up, int n_half,
                                 void *out, long ldo, smh_stream_t stream);
 /* smh_q40_matmul_tiled_direct: LinearQ4_0.forward (:228-236) of up to 3 tiled weights that share the input, for more than 128

@@ -436,10 +436,10 @@ WarmWeights smh::q40_warm(int M, int K, int nseg, const void *const *tiled, cons
     return w;
 }
 
-extern "C" int smh_q40_warm_span(int M, int K, int nseg, const int *n, int swiglu, int stages, long *lines, long *first, long *end) {
+extern "C" int smh_q40_warm_span(int M, int K, int nseg, const int *n, int form, int stages, long *lines, long *first, long *end) {
     SMH_REQUIRE(nseg >= 1 && nseg <= SMH_MAX_SEGMENTS && n && lines && first && end, "smh_q40_warm_span: nseg=%d or a null pointer", nseg);
     const void *const some[SMH_MAX_SEGMENTS] = {(const void *)128, (const void *)128, (const void *)128};
-    const WarmWeights w = M > SMH_GEMV_MAX_M ? q40_warm(M, K, nseg, some, n, swiglu != 0, stages, 8) : WarmWeights{};
+    const WarmWeights w = M > SMH_GEMV_MAX_M || (form & 2) ? q40_warm(M, K, nseg, some, n, form & 1, stages, 8) : WarmWeights{};
     for (int i = 0; i < nseg; ++i) { lines[i] = first[i] = end[i] = 0; }
     for (int at = 0; w.workgroups > 0 && at < warm_blocks(w); ++at) {
         WarmBlock b;

@@ -274,7 +274,9 @@ def test_columns_of_a_workgroup_on_the_checkpoint_layout():
 
 @pytest.mark.parametrize("M,K,ns,swiglu", [(37, 4096, [4096, 4096, 4096], 0), (100, 4096, [4096], 0), (100, 11008, [4096], 0), (17, 4096, [4096], 0),
                                            (128, 8192, [8192, 1024, 1024], 0), (64, 4096, [5248, 1152, 1152], 0), (48, 13824, [5120], 0),
-                                           (100, 4096, [11008, 11008], 1), (33, 5120, [13824, 13824], 1), (64, 64, [8320, 8320], 1)])
+                                           (100, 4096, [11008, 11008], 1), (33, 5120, [13824, 13824], 1), (64, 64, [8320, 8320], 1),
+                                           (5, 4096, [4096, 4096, 4096], 2), (10, 4096, [4096, 1024, 1024], 2), (16, 11008, [4096], 2), (5, 14336, [4096], 2), (16, 4096, [4096], 2),
+                                           (5, 4096, [11008, 11008], 3), (16, 4096, [14336, 14336], 3), (10, 5120, [13824, 13824], 3)])
 def test_weights_asked_for_ahead_are_those_of_the_launch(M, K, ns, swiglu):
     """a few stages stay inside the weights; all stages are every line of every tile once (the padded half of a last unit included)"""
     from spec_mcts_amd import _lib
@@ -288,7 +290,7 @@ def test_weights_asked_for_ahead_are_those_of_the_launch(M, K, ns, swiglu):
     assert lib.smh_q40_warm_span(M, K, len(ns), n, swiglu, 1 << 20, *out) == 1
     for i, N in enumerate(ns):
         # 34 lines a tile; its scales are asked for with each half of it (128-column blocks), with each piece (SwiGLU)
-        pieces, lines = (2 * (N // 128), 10) if swiglu else (2 * ((N + 255) // 256), 18)
+        pieces, lines = (2 * (N // 128), 10) if swiglu & 1 else (2 * ((N + 255) // 256), 18)
         assert out[0][i] == pieces * lines * (K // 32)
         assert out[1][i] == 0 and (out[2][i] == lib.smh_q40_tiled_bytes(K, N) or N % 256)
 
