@@ -165,6 +165,24 @@ extern "C" size_t smh_decode_scratch_bytes(const smh_layer *layer, int rows, int
     return b.total;
 }
 
+extern "C" int smh_decode_layer_form(const smh_layer *layer, int rows, int swiglu_in, int *slabs) {
+    const char *who = "smh_decode_layer_form";
+    SMH_REQUIRE(layer && slabs, "%s: null pointer", who);
+    smh_pass pass{};
+    pass.rows = rows;
+    pass.swiglu_in = swiglu_in != 0;
+    LayerBuffers b;
+    SMH_REQUIRE(rows >= 1 && layer->heads > 0 && layer->kv_heads > 0 && layer->heads % layer->kv_heads == 0, "%s: rows=%d heads=%d kv_heads=%d", who, rows, layer->heads, layer->kv_heads);
+    if (layer_buffers(*layer, rows, pass.swiglu_in, nullptr, b) != 0) return -1;
+    const LayerRun run(*layer, pass, nullptr, layer->prompt_len >= BLOCKS_MIN_PROMPT);
+    auto left = [&](int K, int nseg, const int *n) { return direct(rows, K, nseg, n) ? 0 : run.slabs(K, nseg, n); };
+    slabs[0] = left(layer->dim, 3, run.n_qkv);
+    slabs[1] = left(run.nq, 1, run.n_dim);
+    slabs[2] = run.swiglu ? 0 : slices(rows, layer->dim, 2, run.n_gu);
+    slabs[3] = left(layer->ffn, 1, run.n_dim);
+    return (run.blocks ? 1 : 0) | (run.swiglu ? 2 : 0);
+}
+
 extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stream_t stream) {
     const char *who = "smh_decode_layer";
     SMH_REQUIRE(layer && pass && pass->h, "%s: null pointer", who);

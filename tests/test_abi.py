@@ -238,6 +238,38 @@ def test_rmsnorm_inside_the_launches_of_a_layer():
     assert not model._norm_in(17, 4096, [K.TiledQ40(None, 4096, 4096)] * 3)
 
 
+def test_form_of_a_layer():
+    """5 .. 16 branches on 128-column blocks, and up to 32 with SwiGLU inside w1|w3, behind 96 prompt rows and more where all linears have them; whatever the
+    form leaves, the scratch holds"""
+    from spec_mcts_amd import _lib
+    lib = _lib.load()
+
+    def form(dim, heads, kv_heads, ffn, P, M, swiglu=1):
+        layer, slabs = _lib.SmhLayer(), (ctypes.c_int * 4)()
+        layer.dim, layer.heads, layer.kv_heads, layer.ffn, layer.prompt_len = dim, heads, kv_heads, ffn, P
+        f = lib.smh_decode_layer_form(layer, M, swiglu, slabs)
+        n = (heads + 2 * kv_heads) * 128
+        need = 2 * M * (3 * dim + n + heads * 128 + ffn) + 4 * M * (max(slabs[0] * n, slabs[2] * 2 * ffn) + max(slabs[1], slabs[3]) * dim)
+        assert f < 0 or lib.smh_decode_scratch_bytes(layer, M, swiglu) >= need
+        return f, list(slabs)
+
+    L7, L8, L13, L70 = (4096, 32, 32, 11008), (4096, 32, 8, 14336), (5120, 40, 40, 13824), (8192, 64, 8, 28672)
+    for L, wide in ((L7, [2, 8, 0, 8]), (L8, [5, 8, 0, 8])):
+        for M in (1, 4, 5, 10, 16, 17, 32, 33, 100):
+            for P in (0, 95, 96, 512):
+                f, slabs = form(*L, P, M)
+                assert f == (3 if 5 <= M <= 16 and P >= 96 else 2 if M > 32 or (M > 16 and P >= 96) else 0), (L, M, P)
+                assert f == 0 or M == 100 or slabs == wide
+                assert form(*L, P, M, 0)[0] == 0           # (SwiGLU switched off: as before, whatever the rows)
+    assert [form(*L13, 96, M)[0] for M in (5, 16, 17, 32)] == [0, 0, 2, 2]             # (wo and w2 of 5120 columns have no such blocks)
+    assert [form(*L70, 512, M)[0] for M in (1, 5, 16, 17, 100, 129)] == [0, 0, 0, 0, 0, 2]
+    for L in (L7, L8, L13, L70, (256, 2, 2, 768)):
+        for P in (0, 100):
+            for M in range(1, 700, 3):
+                assert form(*L, P, M)[0] >= 0
+    assert form(*L7, 96, 0)[0] < 0 and form(4096, 32, 5, 11008, 96, 8)[0] < 0 and form(100, 32, 32, 11008, 96, 8)[0] < 0
+
+
 def test_columns_of_a_workgroup_above_128_rows():
     """which of the launches above 128 rows a shape takes (the GPU tests of each ask here), 0 where there is none"""
     from spec_mcts_amd import _lib

@@ -4,6 +4,8 @@ configs[4]: dim 8192, 64 heads over 8 KV heads, FFN 28672), each against the ora
 
 Branches are given DIFFERENT tokens, so a row mix-up between branches cannot cancel out, and several decode
 steps are taken, so the later ones read suffix rows the earlier ones appended."""
+import ctypes
+
 import pytest
 import torch
 
@@ -210,8 +212,8 @@ def test_passes_that_only_some_forms_of_the_attention_take(heads, kv_heads, B, P
 @pytest.mark.parametrize("B,P", [(5, 96), (6, 130), (11, 300), (16, 100), (17, 97), (32, 96), (5, 95), (16, 95), (24, 95)])
 def test_few_branches_behind_a_prompt(B, P):
     """Layers of the 7B shape for 5 .. 32 branches: from 96 prompt rows on 128-column blocks and SwiGLU inside w1|w3 (one row tile up to 16 branches, two from
-    17 on), before that GEMVs, or slabs of w1|w3.  In 64 bits, without any of the path's roundings: as far from that as 17 .. 48 branches of the same
-    tokens are, which take the blocks anyway."""
+    17 on), before that GEMVs, or slabs of w1|w3.  Against the same tokens among 48 branches, which take the blocks anyway: no more than flips of a
+    rounding apart.  (Against the oracle: the test below.)"""
     cfg = dict(LAYER_7B, max_batch_size=48, max_prompt_seq_len=320)
     _, _, model = _build(cfg, 77, 0.02)
     att = [layer.attention for layer in model.layers]
@@ -234,3 +236,33 @@ def test_few_branches_behind_a_prompt(B, P):
         assert got.isfinite().all()
         # fp16 roundings at the same points, fp32 sums in another order: a flip now and then moves a logit by a few 2^-11 of the deviation, two layers deep
         assert float((got - wide).norm() / wide.norm()) < 4e-3
+
+
+LAYER_8B = dict(LAYER_7B, n_kv_heads=8, multiple_of=1024, ffn_dim_multiplier=1.3)
+
+
+def _form(cfg, B, P):
+    """smh_decode_layer_form of a model's layers behind P prompt rows, and the slabs of wq|wk|wv, wo, w1|w3 and w2"""
+    from spec_mcts_amd import _lib
+    layer, slabs = _lib.SmhLayer(), (ctypes.c_int * 4)()
+    layer.dim, layer.heads, layer.kv_heads, layer.prompt_len = cfg["dim"], cfg["n_heads"], cfg.get("n_kv_heads") or cfg["n_heads"], P
+    layer.ffn = O.ffn_hidden_dim(cfg["dim"], cfg["multiple_of"], cfg.get("ffn_dim_multiplier"))
+    return _lib.load().smh_decode_layer_form(layer, B, 1, slabs), list(slabs)
+
+
+@pytest.mark.parametrize("forked", [False, True])
+@pytest.mark.parametrize("cfg,B,P,form,slabs", [(LAYER_7B, 5, 96, 3, [2, 8, 0, 8]), (LAYER_7B, 10, 130, 3, [2, 8, 0, 8]), (LAYER_7B, 16, 97, 3, [2, 8, 0, 8]), (LAYER_7B, 24, 100, 2, [2, 8, 0, 8]),
+                                                (LAYER_7B, 10, 95, 0, [10, 16, 5, 16]), (LAYER_8B, 5, 96, 3, [5, 8, 0, 8]), (LAYER_8B, 16, 129, 3, [5, 8, 0, 8]),
+                                                (LAYER_8B, 9, 260, 3, [5, 8, 0, 8])])
+def test_decode_logits_of_few_branches_behind_longer_prompts(cfg, B, P, form, slabs, forked):
+    """5 .. 32 branches of the 7B shape, and of 32 heads over 8, on 128-column blocks with SwiGLU inside w1|w3 from 96 prompt rows on (asked of the library): per
+    branch and step against the oracle, branches with rows of their own and branches that share an ancestor's."""
+    assert _form(cfg, B, P) == (form, slabs)
+    cfg = dict(cfg, n_layers=1, max_batch_size=B, max_prompt_seq_len=P)
+    _steps(cfg, 91, B, P, std=0.02, rtol=1e-2, atol=1e-2, steps=5, forks={2: (1, 3, B - 3), 4: (B - 1, 0, 1)} if forked else {})
+
+
+@pytest.mark.parametrize("cfg,P", [(LAYER_7B, 4), (LAYER_7B, 5), (LAYER_7B, 16), (LAYER_7B, 17), (LAYER_7B, 32), (LAYER_8B, 13)])
+def test_prefill_of_few_rows(cfg, P):
+    """Prompts of 5 .. 32 rows take the launches that as many branches behind a longer prompt do."""
+    _steps(dict(cfg, n_layers=1, max_batch_size=2, max_prompt_seq_len=32), 92, 2, P, std=0.02, rtol=1e-2, atol=1e-2, steps=1)
