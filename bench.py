@@ -93,8 +93,8 @@ def time_region(torch, fn, iters):
 
 
 def step_matmuls(model):
-    """The weight-streaming launches of one decode step as the model issues them: per layer the fused
-    wq|wk|wv, wo, the fused w1|w3 and w2 (128 launches for 32 layers)."""
+    """The weight products of one decode step: per layer the fused wq|wk|wv, wo, the fused w1|w3 and w2 (128 launches for 32 layers
+    where each is a launch of its own)."""
     out = []
     for layer in model.layers:
         a, f = layer.attention, layer.feed_forward
@@ -107,9 +107,10 @@ def step_matmuls(model):
 
 
 def matmul_roofline(torch, model, M, iters):
-    """Only the Q4_0 matmul kernels (q40_gemv_kernel for M <= 16; above, the kernels the model launches at that batch:
-    q40_gemm_kg_kernel, q40_gemm_swiglu_kernel for w1|w3 where it applies, q40_gemm_kernel otherwise), launched once per
-    weight launch of a decode step at batch M, back to back in one HIP graph; timed with HIP events on the
+    """Only the Q4_0 matmul kernels as the operators launch them (q40_gemv_kernel for M <= 16, whatever a decode step of as many branches takes: all layers
+    in one launch, or the kernels of more rows; above, those the model launches at that batch:
+    q40_gemm_kg_kernel, q40_gemm_swiglu_kernel for w1|w3 where it applies, q40_gemm_kernel otherwise), once per
+    weight product of a decode step at batch M, back to back in one HIP graph; timed with HIP events on the
     stream the graph runs on.  Every launch reads different weights (3.4 GB per pass, the Infinity Cache
     holds 256 MB)."""
     from spec_mcts_amd import kernels as K
@@ -523,13 +524,13 @@ def main():
         rf10 = matmul_roofline(torch, model, 10, 5)
         rf100 = matmul_roofline(torch, model, 100, 3)
         result["roofline"] = {
-            "kernel": "q40_gemv_kernel at M=1: the %d weight launches of one %s decode step (wq|wk|wv, wo, w1|w3, w2 per layer)"
+            "kernel": "q40_gemv_kernel at M=1: the %d weight products of one %s decode step (wq|wk|wv, wo, w1|w3, w2 per layer), a launch each"
                       % (rf1["launches"], a.arch.upper()),
             "bound": "hbm", "achieved": round(rf1["gbs"], 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(rf1["gbs"] / HBM_PEAK_GBS, 4), "traffic": GEMV_TRAFFIC_BYTES_PER_LAUNCH if a.arch == "7b" else None,
             "avg_launch_us": round(rf1["avg_us"], 3), "bytes_per_launch": round(rf1["bytes_per_launch"])}
         result["rooflines_other"] = [
-            {"kernel": "q40_gemv_kernel at M=10", "bound": "hbm", "achieved": round(rf10["gbs"], 1), "peak": HBM_PEAK_GBS,
+            {"kernel": "q40_gemv_kernel at M=10: the same products as operators (a 7B step of 10 branches behind 96 prompt rows has them on 128-column blocks)", "bound": "hbm", "achieved": round(rf10["gbs"], 1), "peak": HBM_PEAK_GBS,
              "unit": "GB/s", "frac": round(rf10["gbs"] / HBM_PEAK_GBS, 4), "avg_launch_us": round(rf10["avg_us"], 3)},
             {"kernel": "Q4_0 GEMM at M=100: q40_gemm_kg_kernel (wq|wk|wv, wo, w2) and q40_gemm_swiglu_kernel (w1|w3), the 128 weight launches of a step", "bound": "mfma", "achieved": round(rf100["tflops"], 1),
              "peak": MFMA_F16_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": round(rf100["tflops"] / MFMA_F16_PEAK_TFLOPS, 4),

@@ -1999,7 +1999,8 @@ static int attn_plan_tw(int P, int Hkv) {
 // 64, 10 / 60 / 120 rows of their own: 5 branches behind 100 rows 1905 / 1913 / 1938 and 1892 / 1896 / 1916; 16 behind 256 2072 / 2116 / 2168 and 2010 / 2026 / 2088; 10
 // behind 400 2085 / 2188 / 2347 and 1986 / 1999 / 2066; us a call of 32 / 40 / 64 heads, slices as narrow and of 64 rows, 10 rows of their own: one branch behind 128 rows 10.1
 // / 10.1 / 10.6 and 9.9 / 9.8 / 10.2, four behind 256 11.1 / 11.1 / 12.0 and 10.1 / 10.5 / 12.0, 16 behind 128 12.7 / 12.7 / 13.6 and 11.9 / 11.8 / 12.4; 384 sizes of 4 to 16 branches, 10 to 120 own
-// rows, with the waves below: 1.08 times as fast at the mean, slowest 0.97, 64 heads of 12 branches behind 96 rows, 11.3 and 11.7 at 10 own rows, 19.9 and 14.2 at 120.)  One query keeps three slices of 32 rows
+// rows, with the waves below: 1.08 times as fast at the mean, slowest 0.97, 64 heads of 12 branches behind 96 rows, 11.3 and 11.7 at 10 own rows, 19.9 and 14.2 at 120;
+// 64 and 80 heads over 32 and 40, 1 to 8 branches: 0.97 .. 1.7.)  One query keeps three slices of 32 rows
 // behind 96: 9.2 and 9.7 us with two.  Below 96 rows results stay what they were (ATTN_TILES_MIN_PROMPT).
 // (smh_shared_prefix_attn_one, whose queries are ready and whose slices end sooner, keeps the narrow ones: with wide ones 0.91 .. 0.97 times as fast
 // at 1 to 5 branches behind 96 and 128 rows, 32 and 40 heads, 1.0 .. 1.9 behind 256 and more.)

@@ -3,8 +3,8 @@
 // Issued operator by operator from Python a decode layer costs ~90 us of host time (eight or nine operators, each with its
 // checks, its output tensors and a foreign call), which at one branch is more than the GPU needs for it: a step of the
 // 32-layer model took 3.0 ms where a captured graph of the same launches takes 2.0.  Here the layer's launches are issued one
-// behind the other (2-3 us each), out of buffers the caller allocated once for the whole pass.  The sequence, the operators
-// and their switches are those of Transformer._forward_fused in hf_model_q40_kv_shared.py.
+// behind the other (2-3 us each), out of buffers the caller allocated once for the whole pass.  The operators and their roundings are those of
+// Transformer._forward_fused in hf_model_q40_kv_shared.py; which launches they share is decided here (as_blocks, attn_way, norm_linears, LayerRun::swiglu).
 #include "attn_tiles.hpp"
 #include "q40_warm.hpp"
 
@@ -19,18 +19,19 @@ struct LayerBuffers {
     size_t slab_a_bytes, slab_b_bytes, total;
 };
 
-// Stages of the next launch's weights that a launch asks for (q40_warm.hpp).  Not in layers whose w1|w3 leaves slabs (17 .. 28 branches of the 7B shape behind 64
-// prompt rows: 0.992 .. 0.997 times as fast), nor where a layer's weights are larger and its attention brings its own long
-// prompt (three layers of 64 heads over 8, dim 8192, 17 .. 100 branches behind 1024 rows: 0.998 .. 1.001 times as fast from the norms, 0.996 .. 1.000 from the attention).
+// Stages of the next launch's weights that a launch asks for (q40_warm.hpp).  The norms of layers whose w1|w3 leaves slabs do not ask (17 .. 28 branches of the 7B
+// shape behind 64 prompt rows: 0.992 .. 0.997 times as fast); their attention does (17 .. 100 branches behind 256 and 512 rows, SwiGLU switched off: 1.001 .. 1.009).
+// Nothing is asked for where a layer's weights are larger and its attention brings its own long prompt (three layers of 64 heads over 8, dim 8192, 17 .. 100 branches behind 1024 rows: 0.998 .. 1.001 times as fast from the norms, 0.996 .. 1.000 from the attention).
 constexpr int WARM_MAX_DIM = 8191, WARM_FROM_NORM = 3, WARM_FROM_ATTENTION = 4, WARM_FROM_SWIGLU = 16;
 
 static int slices(int M, int K, int nseg, const int *n) { return smh_q40_matmul_plan_tiled(M, K, nseg, n); }
 // Launches of 17 rows and more (128-column blocks, SwiGLU inside w1|w3, the norms and the attention asking for the next weights) for a layer of fewer, too,
 // where all four linears have them: bound by latency both ways, they are fewer (no SiLU launch), leave 2 to 8 slabs instead of 5 to 16, and their weights are
 // on their way earlier.  7B architecture, 512 + 50 rows, us a step with the GEMVs and so: 5 branches 1976 and 1946, 6 2009 and 1949, 8 2022 and 2007, 10 2119
-// and 2018, 12 2149 and 2040, 16 2275 and 2126.  (4, which the launch of all layers takes with probabilities
+// and 2018, 12 2149 and 2040, 16 2275 and 2126; 32 heads over 8 with FFN 14336 (five slabs of wq|wk|wv) the step is 1.07 .. 1.15 times as fast, eight layers, 5 to
+// 16 branches behind 100 to 1024 rows, 20 and 110 of their own (5 branches behind 256 560 and 513, 16 596 and 522).  (4, which the launch of all layers takes with probabilities
 // of 32 bits, not 16: 2150 there and 1950 so.)  SwiGLU inside at 17 / 24 / 32 branches: 2360 / 2432 / 2495 -> 2250 /
-// 2318 / 2361.  Behind short prompts a decode step stays what it was (ATTN_TILES_MIN_PROMPT: two evaluations that differ in one rounding drift apart there).
+// 2318 / 2361, with FFN 14336 and 8 kv heads 1.03 .. 1.07 times as fast, with dim 5120 and FFN 13824 1.02 .. 1.03.  Behind short prompts a decode step stays what it was (ATTN_TILES_MIN_PROMPT: two evaluations that differ in one rounding drift apart there).
 constexpr int BLOCKS_MIN_ROWS = 5, BLOCKS_MIN_PROMPT = 96;
 static bool as_blocks(const smh_layer &L, int M, bool swiglu_in) {
     const int n_qkv[3] = {L.heads * 128, L.kv_heads * 128, L.kv_heads * 128}, n_dim[1] = {L.dim};
@@ -45,15 +46,14 @@ static WarmWeights ask(const smh_layer &L, bool blocks, int M, int K, int nseg, 
     return L.dim <= WARM_MAX_DIM && (M > SMH_GEMV_MAX_M || blocks) ? q40_warm(M, K, nseg, w, n, swiglu, stages, workgroups) : WarmWeights{};
 }
 
-
 // The attention of a decode layer: in one launch whose last workgroups merge (ONE, up to 16 queries a kv head), in one launch of 8 or 16
-// queries a workgroup (TILES), or RoPE, prefix slices and walks (LAUNCHES).  us a call with RoPE and append, caches in HBM:
+// queries a workgroup (TILES), or RoPE, prefix slices and walks (LAUNCHES).  us a call with RoPE and append, caches in HBM (32 heads, up to 16 branches: two slabs, 10 own rows):
 //   32 heads, branches after prompt rows   ONE   TILES LAUNCHES  |  64 heads over 8                ONE   TILES LAUNCHES
-//     5 /  512                             12.8   14.9   15.1    |     1 /  512 (8 queries)        12.2   13.7   13.6
-//    16 /  256                             16.7   14.1   15.9    |     1 / 2047                    17.0   22.6   16.6
-//    10 /  768                             19.9   20.2   19.3    |     2 /  128 (16 queries)       10.7   11.2   12.7
-//    10 / 1024                             24.9   23.3   20.5    |     2 /  512                    15.6   13.7   14.1
-//    10 / 2047                             38.9   33.8   24.5    |     2 / 2047                    24.2   22.4   17.9
+//     5 /  512                             11.7   13.4   14.2    |     1 /  512 (8 queries)        12.2   13.7   13.6
+//    16 /  256                             12.1    9.8   14.4    |     1 / 2047                    17.0   22.6   16.6
+//    10 /  768                             15.7   14.1   16.9    |     2 /  128 (16 queries)       10.7   11.2   12.7
+//    10 / 1024                             21.8   17.3   17.9    |     2 /  512                    15.6   13.7   14.1
+//    10 / 2047                             36.2   25.8   20.8    |     2 / 2047                    24.2   22.4   17.9
 //    17 /  512                               -    16.9   18.9    |     3 /  512                      -    11.8   14.9
 //    17 / 1024                               -    21.5   21.8    |     3 / 1024                      -    18.6   17.5
 //    17 / 2047                               -    29.3   26.0    |    10 / 1024                      -    18.0   21.4
@@ -63,10 +63,12 @@ static WarmWeights ask(const smh_layer &L, bool blocks, int M, int K, int nseg, 
 //                                                                |  40 heads, 100 / 512 (two rounds) -   39.5   39.0
 // (Multi-head attention, with ONE's slices of 64 rows and two slabs, us a step of the 7B architecture with ONE and LAUNCHES, 10 / 60 / 120 rows of their own: 700 prompt
 // rows, 10 branches 2097 / 2112 / 2164 and 2142 / 2154 / 2206, 16 2158 / 2225 / 2382 and 2183 / 2196 / 2251; 768 rows, 8 branches 2046 / 2060 / 2124 and 2104 / 2113 /
-// 2138, 9 2093 / 2185 / 2343 and 2138 / 2150 / 2200, where its waves no longer fit one round in pairs.)
+// 2138, 9 2093 / 2185 / 2343 and 2138 / 2150 / 2200, where its waves no longer fit one round in pairs.  With more heads they stop fitting earlier, but LAUNCHES is the
+// faster way behind 705 .. 768 rows there too: eight layers of 40 heads behind 730, 9 / 16 branches, 110 own rows 801 / 903 and 732 / 778, four of 64 heads behind 720 696 / 774
+// and 676 / 701, quotients above those of the same trees behind 704.)
 // A long prompt wants more workgroups than few tiles are, and ONE's merge grows with the slices.  Where the table has a faster form than the rule takes,
-// the line is not drawn yet: multi-head attention of 6 to 16 branches (TILES at 16 / 256, LAUNCHES at 10 / 768) and one grouped branch behind a long
-// prompt were measured at these sizes only, and stay with ONE.  Behind fewer than 96 prompt rows results stay
+// the line is not drawn yet: multi-head attention of 6 to 16 branches (with TILES the step is faster at 10 own rows and slower at 120) and one grouped branch
+// behind a long prompt stay with ONE up to the lines of the rule.  Behind fewer than 96 prompt rows results stay
 // where they are: there two evaluations that differ in one rounding drift 3e-2 (40 rows) to 6e-2 (16 rows) apart within eight steps of the 7B
 // architecture, 1.5e-2 behind 96.
 enum AttnWay { ATTN_ONE, ATTN_TILES, ATTN_LAUNCHES };

@@ -1029,7 +1029,7 @@ __global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_kg_kern
     }
 }
 
-// ---- SwiGLU inside the launch of w1|w3 (tiled weights, 17 .. 128 rows, all of K in one workgroup) -----------------------
+// ---- SwiGLU inside the launch of w1|w3 (tiled weights, up to 128 rows, all of K in one workgroup) -----------------------
 // q40_gemm_kg_kernel with the roles of a workgroup's waves changed: instead of the two pieces of one 128-column block, a
 // workgroup takes piece bp of block j of the GATE weight and the same piece of the UP weight (64 columns each, the same
 // columns), so its wave (kk, hh, gu) holds, after the K-groups are added, gate or up for exactly the columns its neighbour
@@ -1701,10 +1701,11 @@ static int gemm_kg_launch(const MatmulParams &p, hipStream_t stream) {
 
 // Can w1|w3 of these dimensions run with SwiGLU inside the launch, and is it the faster way?  Above 128 rows always (K a multiple
 // of 32; the two-launch form writes and reads 8 bytes of slabs per gate and up value: 62 of 426 us at 2047 rows of the 7B
-// shape).  17 .. 128 rows: K a multiple of
+// shape).  Up to 128 rows: K a multiple of
 // 64, two weights of n_half columns (a multiple of 128) whose 2 * n_half / 128 workgroups fit the compute units in one round;
-// `worth_it`: and fill at least half of them (narrower weights are faster as two kernels with a K-split), above 32 rows
-// (measured at the 7B shape, w1|w3 + SiLU: 38.1 against 44.9 us at 100 rows, 29.1 against 31.5 at 64, level at 32).
+// `worth_it`: and fill at least half of them (narrower weights are faster as two kernels with a K-split; w1|w3 + SiLU of the 7B shape 38.1 against
+// 44.9 us at 100 rows, 29.1 against 31.5 at 64, level at 32).  From how many rows on is for the caller: smh_q40_swiglu_fits says 33, layer calls behind a longer
+// prompt, whose norms ask for the weights, 5 (as_blocks) and 17.
 bool gemm_swiglu_fits(int M, int K, int n_half, bool worth_it) {
     if (M < 1 || K <= 0 || n_half <= 0 || n_half % 128 != 0) return false;
     if (M > GEMM_BM) return K % 32 == 0;                        // gemm_swiglu_rows_launch

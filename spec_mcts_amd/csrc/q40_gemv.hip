@@ -254,7 +254,8 @@ __device__ __forceinline__ void gemv_consume_tiled(const uint8_t *stage, int k0,
 // rows grows with them, up to 80 KB for w1|w3 of dim 8192, and with it a prologue that no weight is consumed in.  So the stages bring the
 // residual stream, and every wave normalises the eight values of its operand on their way into the matrix core: 28 vector instructions more on the 190 of a step
 // that waits for HBM.  us a step of three layers of dim 8192 behind 1024 rows, w1|w3 behind a launch of RMSNorm's own and wq|wk|wv in form 3 / w1|w3 in form 4 /
-// both: 4 branches 489 / 478 / 477, 10 511 / 503 / 499, 16 527 / 522 / 515; one branch, both in form 3 and in form 4: 466 and 472.  32 layers of dim 4096 behind 64
+// both: 4 branches 489 / 478 / 477, 10 511 / 503 / 499, 16 527 / 522 / 515; 2 and 3, both in form 3 and in form 4: 485 / 480 and 480 / 475, behind 64 rows 463 / 473 and 465 / 468; one
+// branch 466 and 472.  32 layers of dim 4096 behind 64
 // rows, with launches of RMSNorm's own and in form 4: 5 branches 2006 and 1927, 10 2125 and 2020, 16 2225 and 2125.
 template <int LAYOUT>
 __global__ __launch_bounds__(GEMV_WAVES * 64) void q40_gemv_kernel(MatmulParams p) {

@@ -1,4 +1,5 @@
-// The weights that a launch of 17 .. 128 rows will read first, asked for by workgroups of the launch in front of it.
+// The weights that a launch of q40_gemm_kg_kernel or q40_gemm_swiglu_kernel (17 .. 128 rows, in layer calls 5 .. 128) will read first, asked for by workgroups of the
+// launch in front of it.
 //
 // A workgroup of q40_gemm_kg_kernel or q40_gemm_swiglu_kernel waits ~2.5 us for its first stage (cold translations and HBM), a quarter of a launch at 37
 // rows, and HBM idles meanwhile, as it does under the RMSNorm (a workgroup a row) and the attention.  Those launches, and SwiGLU's on 172 compute units, get
@@ -8,8 +9,8 @@
 // 2720 and 2616) 1.028 .. 1.043, 65 .. 100 (3494 and 3434, 3676 and 3665) 1.002 .. 1.018.
 // How many stages (us a step of the 7B architecture, 37 forked and 100 branches, 2418 and 3440 without): wq|wk|wv and w1|w3 from the norms 2: 2408 and 3427,
 // 3: 2404 and 3425, 8: 2416 and 3446 (the norms end later), wo from the attention 4 more: 2395 and 3422, w2 from SwiGLU, too, all of its 22 stages: 2332 and
-// 3387, 16: 2335 and 3367, 8: 2369 and 3384.  The prompt's rows for the attention, from wq|wk|wv's idle compute units: no gain.  Up to 16 rows (GEMV), whose
-// launches stream from their first microsecond on: none (7B and 70B, 10 branches).
+// 3387, 16: 2335 and 3367, 8: 2369 and 3384.  The prompt's rows for the attention, from wq|wk|wv's idle compute units: no gain.  GEMVs, which
+// stream from their first microsecond on: no gain (7B and 70B, 10 branches).
 #pragma once
 
 #include "q40_matmul.hpp"

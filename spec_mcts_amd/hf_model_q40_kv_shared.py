@@ -437,8 +437,8 @@ class Transformer(nn.Module):
         return self._lm_head(hn.view(bsz, seqlen, p.dim))
 
     def _decode(self, tokens: torch.Tensor, step_state) -> torch.Tensor:
-        """A decode step on tiled weights: the launches of _forward_fused, a layer per library call (smh_decode_layer) instead of
-        an operator per call - at a few branches the host, not the GPU, is what the operators' way waits for."""
+        """A decode step on tiled weights: the operators of _forward_fused with their roundings, a layer per library call (smh_decode_layer, which has
+        several of them in one launch) instead of an operator per call - at a few branches the host, not the GPU, is what the operators' way waits for."""
         p = self.params
         B = tokens.shape[0]
         h = K.embedding(tokens, self.tok_embeddings.weight)

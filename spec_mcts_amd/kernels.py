@@ -171,7 +171,7 @@ def matmul_q40_partial(a: torch.Tensor, linears, out: Optional[torch.Tensor] = N
 
 
 def swiglu_fits(M: int, K: int, n_half: int) -> bool:
-    """Is matmul_q40_swiglu the faster way for these dimensions (17 .. 128 rows, a wide gate / up pair)?"""
+    """Is matmul_q40_swiglu the faster way for these dimensions (33 rows and more, up to 128 a wide gate / up pair)?"""
     return bool(_lib.load().smh_q40_swiglu_fits(int(M), int(K), int(n_half)))
 
 
