@@ -42,8 +42,6 @@ __global__ __launch_bounds__(256) void partial_reduce_kernel(const void *__restr
     *reinterpret_cast<h4 *>(c + (long)m * ldc + n) = out;
 }
 
-struct Nothing {};
-
 // ---- residual add + RMSNorm ---------------------------------------------------------------------
 // one workgroup of 1024 threads per row; h_out = h_in + fp16(acc) (fp16 add), xn = fp16(fp16(h*r)*w)
 // A chain of trips to memory bounds it, so everything is requested before the first sum: KS slabs (0: none), PASSES passes of four
