@@ -1602,14 +1602,19 @@ __device__ __forceinline__ void kv_store_lanes(h4 x, uint8_t *row, half_t *scale
 }
 
 // QKS: most slabs of the q|k|v product, LEAST: the fewest.  QT: queries of a workgroup, 16 or 8 (then a wave's halves share one query and take
-// its rows 16 at a time in turn).  Grid: (XCD, kv head of it, tile); ASK: workgroups past the tiles ask for the next launch's weights (q40_warm.hpp).
+// its rows 16 at a time in turn).  Grid: (XCD, kv head of it, tile); Ask = TileAsk: workgroups past the tiles ask for the next launch's weights (q40_warm.hpp).
 // (A kernel of its own: with the arguments and the branch in every launch calls that ask for nothing took 0.2 to 0.4 us longer, 32 heads, 17 branches behind 256 rows
 // without rows of their own 8.04 us and 7.65 so; 64 over 8 7.63 and 7.36.)
-template <bool PAGES, int LEAST, int QKS, int QT, bool ASK>
-__global__ __launch_bounds__(64 * AT_WAVES) void attn_tile_kernel(AttnParams p, int chunks, std::conditional_t<ASK, int, Nothing> tiles, std::conditional_t<ASK, WarmWeights, Nothing> next) {
-    args_ahead<sizeof(AttnParams) + 8>();
-    if constexpr (ASK) {
-        if (__builtin_expect((int)blockIdx.z >= tiles, 0)) return warm_weights(next, blockIdx.x, (blockIdx.z - tiles) * gridDim.y + blockIdx.y, threadIdx.x, 64 * AT_WAVES);
+struct TileAsk {
+    int tiles;
+    WarmWeights next;
+};
+template <bool PAGES, int LEAST, int QKS, int QT, class... Ask>
+__global__ __launch_bounds__(64 * AT_WAVES) void attn_tile_kernel(AttnParams p, int chunks, Ask... ask) {
+    args_ahead<sizeof(AttnParams) + (sizeof...(Ask) > 0 ? 16 : 4)>();
+    if constexpr (sizeof...(Ask) > 0) {
+        const TileAsk &a = (ask, ...);
+        if (__builtin_expect((int)blockIdx.z >= a.tiles, 0)) return warm_weights(a.next, blockIdx.x, (blockIdx.z - a.tiles) * gridDim.y + blockIdx.y, threadIdx.x, 64 * AT_WAVES);
     }
     extern __shared__ __attribute__((aligned(16))) float at_lds[];
     half_t *const s_q = reinterpret_cast<half_t *>(at_lds + AT_WAVES * AT_MINE), *const s_k = s_q + 16 * AT_QPITCH, *const s_v = s_k + 16 * AT_QPITCH;
@@ -2419,14 +2424,14 @@ int smh::shared_prefix_attn_qkv_tiles(const void *qkv_partial, int ksplit, void 
     p.app_k = (uint8_t *)cache_k; p.app_v = (uint8_t *)cache_v;
     p.app_ks = (half_t *)cache_ks; p.app_vs = (half_t *)cache_vs;
     p.app_t = t_dev; p.app_smax = Smax;
-#define TILE_KERNELS(ask) {{{attn_tile_kernel<false, 1, 2, 8, ask>, attn_tile_kernel<false, 3, 6, 8, ask>, attn_tile_kernel<false, 7, 16, 8, ask>}, \
-                            {attn_tile_kernel<true, 1, 2, 8, ask>, attn_tile_kernel<true, 3, 6, 8, ask>, attn_tile_kernel<true, 7, 16, 8, ask>}}, \
-                           {{attn_tile_kernel<false, 1, 2, 16, ask>, attn_tile_kernel<false, 3, 6, 16, ask>, attn_tile_kernel<false, 7, 16, 16, ask>}, \
-                            {attn_tile_kernel<true, 1, 2, 16, ask>, attn_tile_kernel<true, 3, 6, 16, ask>, attn_tile_kernel<true, 7, 16, 16, ask>}}}
-    typedef void (*plain_t)(AttnParams, int, Nothing, Nothing);
-    typedef void (*ask_t)(AttnParams, int, int, WarmWeights);
-    static const plain_t plain[2][2][3] = TILE_KERNELS(false);
-    static const ask_t asking[2][2][3] = TILE_KERNELS(true);
+#define TILE_KERNELS(...) {{{attn_tile_kernel<false, 1, 2, 8 __VA_ARGS__>, attn_tile_kernel<false, 3, 6, 8 __VA_ARGS__>, attn_tile_kernel<false, 7, 16, 8 __VA_ARGS__>}, \
+                            {attn_tile_kernel<true, 1, 2, 8 __VA_ARGS__>, attn_tile_kernel<true, 3, 6, 8 __VA_ARGS__>, attn_tile_kernel<true, 7, 16, 8 __VA_ARGS__>}}, \
+                           {{attn_tile_kernel<false, 1, 2, 16 __VA_ARGS__>, attn_tile_kernel<false, 3, 6, 16 __VA_ARGS__>, attn_tile_kernel<false, 7, 16, 16 __VA_ARGS__>}, \
+                            {attn_tile_kernel<true, 1, 2, 16 __VA_ARGS__>, attn_tile_kernel<true, 3, 6, 16 __VA_ARGS__>, attn_tile_kernel<true, 7, 16, 16 __VA_ARGS__>}}}
+    typedef void (*plain_t)(AttnParams, int);
+    typedef void (*ask_t)(AttnParams, int, TileAsk);
+    static const plain_t plain[2][2][3] = TILE_KERNELS();
+    static const ask_t asking[2][2][3] = TILE_KERNELS(, TileAsk);
 #undef TILE_KERNELS
     static const hipError_t lds_ok = [] {
         hipError_t e = hipSuccess;
@@ -2440,8 +2445,8 @@ int smh::shared_prefix_attn_qkv_tiles(const void *qkv_partial, int ksplit, void 
     const int qt = attn_tile_queries(p.Bq, Hkv), tiles = (p.Bq + qt - 1) / qt, rows = (Hkv + 7) / 8, slabs = ksplit <= 2 ? 0 : ksplit <= 6 ? 1 : 2;
     const int chunks = (P + AT_CHUNK - 1) / AT_CHUNK;
     const dim3 grid(8, rows, tiles + next.workgroups / (8 * rows)), threads(64 * AT_WAVES);
-    if (next.workgroups >= 8 * rows) hipLaunchKernelGGL(asking[qt == 16][pages != nullptr][slabs], grid, threads, AT_LDS, (hipStream_t)stream, p, chunks, tiles, next);
-    else hipLaunchKernelGGL(plain[qt == 16][pages != nullptr][slabs], grid, threads, AT_LDS, (hipStream_t)stream, p, chunks, Nothing{}, Nothing{});
+    if (next.workgroups >= 8 * rows) hipLaunchKernelGGL(asking[qt == 16][pages != nullptr][slabs], grid, threads, AT_LDS, (hipStream_t)stream, p, chunks, TileAsk{tiles, next});
+    else hipLaunchKernelGGL(plain[qt == 16][pages != nullptr][slabs], grid, threads, AT_LDS, (hipStream_t)stream, p, chunks);
     return launch_status();
 }
 int smh::attn_tiles_idle(int B, int H, int Hkv) {

@@ -46,19 +46,20 @@ __global__ __launch_bounds__(256) void partial_reduce_kernel(const void *__restr
 // one workgroup of 1024 threads per row; h_out = h_in + fp16(acc) (fp16 add), xn = fp16(fp16(h*r)*w)
 // A chain of trips to memory bounds it, so everything is requested before the first sum: KS slabs (0: none), PASSES passes of four
 // columns a thread, the residual and the norm's weights.  Up to 64 registers two workgroups share a compute unit.
-// Grid (rows, 1); ASK: (rows, 1 and as many times more as make next.workgroups, which ask for the next launch's weights: q40_warm.hpp).
-// (ASK: a kernel of its own, as the others have fewer arguments and a shorter way to their first load)
-template <int PASSES, int KS, bool ASK = false>
+// Grid (rows, 1); Ask = WarmWeights: (rows, 1 and as many times more as make next.workgroups, which ask for the next launch's weights: q40_warm.hpp).
+// (A kernel of its own, as the others have fewer arguments and a shorter way to their first load: one more, be it empty, makes 68 bytes of them
+// in the place of one line, and 100 rows of 4096 behind four slabs 3.34 us and not 3.27)
+template <int PASSES, int KS, class... Ask>
 __global__ __launch_bounds__(1024, PASSES * KS <= 8 ? 8 : 4) void partial_rmsnorm_kernel(const void *__restrict__ partial, int ks, int M, int N,
                                                                const half_t *__restrict__ h_in, const half_t *__restrict__ wt,
                                                                float eps, half_t *__restrict__ h_out, half_t *__restrict__ xn_out,
-                                                               std::conditional_t<ASK, WarmWeights, Nothing> next) {
+                                                               Ask... next) {
     __shared__ float s_part[16];
     const int m = blockIdx.x;
-    if constexpr (ASK) {
+    if constexpr (sizeof...(Ask) > 0) {
         if (__builtin_expect(blockIdx.y > 0, 0)) {                 // (known without an argument: a row's workgroup asks for all of them at once)
             const int e = ((int)blockIdx.y - 1) * M + m;
-            return warm_weights(next, (M + e) & 7, e >> 3, threadIdx.x, 1024);
+            return warm_weights(next..., (M + e) & 7, e >> 3, threadIdx.x, 1024);
         }
     }
     const long slab = (long)M * N;
@@ -324,7 +325,7 @@ using namespace smh;
 static_assert(SMH_MAX_KSPLIT == 16, "tables");
 #define BY_SLABS(k, ...) {__VA_ARGS__, k(1), k(2), k(3), k(4), k(5), k(6), k(8), k(8), k(10), k(10), k(12), k(12), k(16), k(16), k(16), k(16)}
 typedef void (*reduce_kernel_t)(const void *, int, int, int, int, int, int, half_t *, long, const half_t *, long);
-typedef void (*rmsnorm_kernel_t)(const void *, int, int, int, const half_t *, const half_t *, float, half_t *, half_t *, Nothing);
+typedef void (*rmsnorm_kernel_t)(const void *, int, int, int, const half_t *, const half_t *, float, half_t *, half_t *);
 typedef void (*rmsnorm_ask_t)(const void *, int, int, int, const half_t *, const half_t *, float, half_t *, half_t *, WarmWeights);
 typedef void (*sumsq_kernel_t)(const void *, int, int, int, const half_t *, half_t *, float *);
 #define K_OF(n) partial_reduce_kernel<n, RES>
@@ -333,7 +334,7 @@ template <int RES> static const reduce_kernel_t REDUCE_KERNELS[17] = BY_SLABS(K_
 #define K_OF(n) partial_rmsnorm_kernel<PASSES, n>
 template <int PASSES> static const rmsnorm_kernel_t RMSNORM_KERNELS[17] = BY_SLABS(K_OF, K_OF(0));
 #undef K_OF
-#define K_OF(n) partial_rmsnorm_kernel<PASSES, n, true>
+#define K_OF(n) partial_rmsnorm_kernel<PASSES, n, WarmWeights>
 template <int PASSES> static const rmsnorm_ask_t RMSNORM_ASK_KERNELS[17] = BY_SLABS(K_OF, nullptr);
 #undef K_OF
 #define K_OF(n) partial_residual_sumsq_kernel<PASSES, n>
@@ -746,7 +747,7 @@ int smh::partial_rmsnorm(const void *partial, int ksplit, int M, int N, const vo
         return launch_status();
     }
     hipLaunchKernelGGL(kern, dim3(M), dim3(1024), 0, (hipStream_t)stream, partial, ks, M, N, (const half_t *)h_in, (const half_t *)weight, eps, (half_t *)h_out,
-                       (half_t *)xn_out, Nothing{});
+                       (half_t *)xn_out);
     return launch_status();
 }
 extern "C" int smh_partial_rmsnorm(const void *partial, int ksplit, int M, int N, const void *h_in, const void *weight, float eps,

@@ -1034,7 +1034,7 @@ __global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_kg_kern
 // workgroup takes piece bp of block j of the GATE weight and the same piece of the UP weight (64 columns each, the same
 // columns), so its wave (kk, hh, gu) holds, after the K-groups are added, gate or up for exactly the columns its neighbour
 // holds the other for.  The epilogue forms fp16(silu(fp16(gate))) * fp16(up) with the roundings of partial_silu_mul_kernel
-// and stores the activations of w2: no slab leaves the launch and the SiLU launch is gone.  ASK: workgroups past the columns ask for w2 (q40_warm.hpp).
+// and stores the activations of w2: no slab leaves the launch and the SiLU launch is gone.  Ask = WarmWeights: workgroups past the columns ask for w2 (q40_warm.hpp).
 // (A kernel of its own: calls that ask for nothing took 19.04 us at 33 rows of 4096 -> 2 x 11008 before there were such workgroups, 19.32 with them, 19.04 so.)
 template <int TILES> struct SwigluShape {
     static constexpr int SC = 1024;                                  // scales: [group kk][gate | up] x 256
@@ -1050,8 +1050,8 @@ template <int TILES> struct SwigluShape {
     static_assert(PER * (SLOTS - 5) <= 63 && LDS <= 160 * 1024, "ring");
 };
 
-template <int TILES, bool ASK>
-__global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_swiglu_kernel(MatmulParams p, std::conditional_t<ASK, WarmWeights, Nothing> next) {
+template <int TILES, class... Ask>
+__global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_swiglu_kernel(MatmulParams p, Ask... next) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     typedef SwigluShape<TILES> S;
     constexpr int SLOTS = S::SLOTS, PER = S::PER, STAGE = S::STAGE;
@@ -1064,8 +1064,8 @@ __global__ __launch_bounds__(64 * (8 + GEMM_DMA_WAVES), 1) void q40_gemm_swiglu_
     const int blockj = hb >> 1, bp = hb & 1;
     const int pair = blockj >> 1, blk = blockj & 1;
     const int n_half = p.seg[0].N;
-    if constexpr (ASK) {
-        if (__builtin_expect(128 * blockj >= n_half, 0)) return warm_weights(next, hb & 7, (hb - n_half / 64) >> 3, tid, 64 * (8 + GEMM_DMA_WAVES));
+    if constexpr (sizeof...(Ask) > 0) {
+        if (__builtin_expect(128 * blockj >= n_half, 0)) return warm_weights(next..., hb & 7, (hb - n_half / 64) >> 3, tid, 64 * (8 + GEMM_DMA_WAVES));
     } else if (128 * blockj >= n_half) return;
     constexpr int m0 = 0;
     const int n_st = p.K / 64;                                         // stages (two steps each), all of K
@@ -1720,12 +1720,13 @@ bool gemm_swiglu_fits(int M, int K, int n_half, bool worth_it) {
 int swiglu_idle(int n_half) { return n_half / 64 < 256 ? (256 - n_half / 64) / 8 * 8 : 0; }
 
 int gemm_swiglu_launch(const MatmulParams &p, const WarmWeights &next, hipStream_t stream) {
-#define SWIGLU_KERNELS(ask) {nullptr, q40_gemm_swiglu_kernel<1, ask>, q40_gemm_swiglu_kernel<2, ask>, q40_gemm_swiglu_kernel<3, ask>, q40_gemm_swiglu_kernel<4, ask>, \
-                             q40_gemm_swiglu_kernel<5, ask>, q40_gemm_swiglu_kernel<6, ask>, q40_gemm_swiglu_kernel<7, ask>, q40_gemm_swiglu_kernel<8, ask>}
-    typedef void (*plain_t)(MatmulParams, Nothing);
+#define SWIGLU_KERNELS(...) {nullptr, q40_gemm_swiglu_kernel<1 __VA_ARGS__>, q40_gemm_swiglu_kernel<2 __VA_ARGS__>, q40_gemm_swiglu_kernel<3 __VA_ARGS__>, \
+                             q40_gemm_swiglu_kernel<4 __VA_ARGS__>, q40_gemm_swiglu_kernel<5 __VA_ARGS__>, q40_gemm_swiglu_kernel<6 __VA_ARGS__>, \
+                             q40_gemm_swiglu_kernel<7 __VA_ARGS__>, q40_gemm_swiglu_kernel<8 __VA_ARGS__>}
+    typedef void (*plain_t)(MatmulParams);
     typedef void (*ask_t)(MatmulParams, WarmWeights);
-    static const plain_t plain[9] = SWIGLU_KERNELS(false);
-    static const ask_t asking[9] = SWIGLU_KERNELS(true);
+    static const plain_t plain[9] = SWIGLU_KERNELS();
+    static const ask_t asking[9] = SWIGLU_KERNELS(, WarmWeights);
 #undef SWIGLU_KERNELS
     static const int lds_bytes[9] = {0, SwigluShape<1>::LDS, SwigluShape<2>::LDS, SwigluShape<3>::LDS, SwigluShape<4>::LDS, SwigluShape<5>::LDS, SwigluShape<6>::LDS,
                                      SwigluShape<7>::LDS, SwigluShape<8>::LDS};
@@ -1745,7 +1746,7 @@ int gemm_swiglu_launch(const MatmulParams &p, const WarmWeights &next, hipStream
     const int tiles = (p.M + 15) / 16;
     const dim3 grid((unsigned)(2 * (p.seg[0].N / 128) + next.workgroups)), threads(64 * (8 + GEMM_DMA_WAVES));
     if (next.workgroups > 0) hipLaunchKernelGGL(asking[tiles], grid, threads, lds_bytes[tiles], stream, p, next);
-    else hipLaunchKernelGGL(plain[tiles], grid, threads, lds_bytes[tiles], stream, p, Nothing{});
+    else hipLaunchKernelGGL(plain[tiles], grid, threads, lds_bytes[tiles], stream, p);
     return launch_status();
 }
 

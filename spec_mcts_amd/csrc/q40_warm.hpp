@@ -17,7 +17,6 @@
 
 namespace smh {
 
-struct Nothing {};                          // in its place: a kernel that asks for nothing has fewer arguments
 struct WarmWeights {
     const uint8_t *w[SMH_MAX_SEGMENTS];        // tiled
     int unit0[SMH_MAX_SEGMENTS];               // first column unit of each
