@@ -159,7 +159,7 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const half_t *__restr
 // ---- residual add + sums of squares (the first half of partial_rmsnorm_kernel, spread over 16 workgroups a row) ----
 // grid (16, M), one wave each: wave w of a row is wave w of partial_rmsnorm_kernel's workgroup (same columns per
 // thread, same order of additions), so sums[m][0..15] added in index order give that kernel's sum of squares bit
-// for bit.  The consumer (the matmul that follows, q40_gemv_kernel LAYOUT 3 and 4) normalises what it multiplies.
+// for bit.  The consumer (the matmul that follows, q40_gemv_kernel LAYOUT 3, 4 and 5) normalises what it multiplies.
 template <int PASSES, int KS>
 __global__ __launch_bounds__(64) void partial_residual_sumsq_kernel(const void *__restrict__ partial, int ks, int M, int N,
                                                                     const half_t *__restrict__ h_in, half_t *__restrict__ h_out,

@@ -48,7 +48,7 @@ constexpr int STAGE_S_BYTES = 32 * 8;
 constexpr int STAGE_X_BYTES = 16 * 64;
 constexpr int STAGE_BYTES = STAGE_W_BYTES + STAGE_S_BYTES + STAGE_X_BYTES;   // 5376
 constexpr int RING_BYTES = RING_STAGES * STAGE_BYTES;                        // 10752 per wave
-// kernels that keep their activations in LDS outside the ring (LAYOUT 2 and 3) have no activation tile in a stage
+// kernels that keep their activations in LDS outside the ring (LAYOUT 2, 3 and 5) have no activation tile in a stage
 constexpr int STAGE_BYTES_NO_X = STAGE_W_BYTES + STAGE_S_BYTES;             // 4352
 constexpr int RING_BYTES_NO_X = RING_STAGES * STAGE_BYTES_NO_X;             // 8704 per wave
 
@@ -250,13 +250,15 @@ __device__ __forceinline__ void gemv_consume_tiled(const uint8_t *stage, int k0,
 // LAYOUT 0: checkpoint layout; 1: tiled weights (smh_q40_tile); 2: tiled weights and activations made from the
 // gate|up slabs by the workgroup itself (p.gu_partial): SiLU(gate) * up needs no launch of its own; 3: tiled weights
 // and activations made from the residual stream by the workgroup itself (p.norm_w, p.norm_ss), one row: RMSNorm needs only
-// the small launch that adds the slabs and leaves the sums of squares; 4: the same for 2 rows and more.  There a workgroup's share of the
+// the small launch that adds the slabs and leaves the sums of squares; 5: two rows; 4: the same for 3 rows and more.  There a workgroup's share of the
 // rows grows with them, up to 80 KB for w1|w3 of dim 8192, and with it a prologue that no weight is consumed in.  So the stages bring the
 // residual stream, and every wave normalises the eight values of its operand on their way into the matrix core: 28 vector instructions more on the 190 of a step
 // that waits for HBM.  us a step of three layers of dim 8192 behind 1024 rows, w1|w3 behind a launch of RMSNorm's own and wq|wk|wv in form 3 / w1|w3 in form 4 /
-// both: 4 branches 489 / 478 / 477, 10 511 / 503 / 499, 16 527 / 522 / 515; 2 and 3, both in form 3 and in form 4: 485 / 480 and 480 / 475, behind 64 rows 463 / 473 and 465 / 468; one
-// branch 466 and 472.  32 layers of dim 4096 behind 64
+// both: 4 branches 489 / 478 / 477, 10 511 / 503 / 499, 16 527 / 522 / 515; one branch, both in form 3 and in form 4: 466 and 472.  32 layers of dim 4096 behind 64
 // rows, with launches of RMSNorm's own and in form 4: 5 branches 2006 and 1927, 10 2125 and 2020, 16 2225 and 2125.
+// Two rows, us a launch in form 5 and in form 4: 4096 -> 2 x 11008 13.5 and 13.9, 2 x 14336 15.5 and 15.9, 8192 -> 8192 + 2 x 1024 (slices of 704 rows) 12.7 and
+// 13.0, 2 x 28672 50.2 and 51.2, 5120 -> 3 x 5120 (640 rows) 11.85 and 11.9, 4096 -> 3 x 4096 (416) 10.1 both; 4096 -> 4096 + 2 x 1024 (256) 8.2 and 7.7.  Three
+// rows, form 4 and the rows in LDS: 14.2 and 14.5, 16.7 and 16.8, 13.2 and 13.7, 51.5 and 51.6, 12.15 and 12.2, 10.2 and 10.3, 7.9 and 8.4.
 template <int LAYOUT>
 __global__ __launch_bounds__(GEMV_WAVES * 64) void q40_gemv_kernel(MatmulParams p) {
     constexpr int WAVES = GEMV_WAVES;
@@ -264,7 +266,8 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void q40_gemv_kernel(MatmulParams 
     constexpr int THREADS = WAVES * 64;
     constexpr bool TILED = LAYOUT != 0;
     constexpr bool SILU_IN = LAYOUT == 2;
-    constexpr bool NORM_IN = LAYOUT == 3;
+    constexpr bool NORM_IN = LAYOUT == 3 || LAYOUT == 5;
+    constexpr int NORM_ROWS = LAYOUT == 5 ? 2 : 1;
     constexpr bool NORM_STEP = LAYOUT == 4;
     constexpr bool X_IN_LDS = SILU_IN || NORM_IN;                   // activations: xs[M][slice rows] behind the rings
     constexpr int PER_STAGE = X_IN_LDS ? 5 : 6;                     // vector-memory instructions per stage
@@ -347,7 +350,7 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void q40_gemv_kernel(MatmulParams 
     // weight stages right behind them, so that both are in flight together.
     half_t *xs = reinterpret_cast<half_t *>(lds + WAVES * RING);
     const int slice_k0 = step0 * 32, slice_rows = (step1 - step0) * 32;
-    // a row of xs is 16 bytes longer than its data (SILU_IN; NORM_IN has one row): the 16 lanes that read one k-octet of 16 different rows would
+    // a row of xs is 16 bytes longer than its data (NORM_IN has one or two): the 16 lanes that read one k-octet of 16 different rows would
     // otherwise hit the same LDS banks whenever the slice is a multiple of 128 bytes long
     const int xs_pitch = slice_rows + 8;
     [[maybe_unused]] float r_c = 0.f;
@@ -393,37 +396,41 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void q40_gemv_kernel(MatmulParams 
         }
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // xs is complete; the DMA ring stays in flight
     } else if constexpr (NORM_IN) {
-        // the loads of this thread's share of the row, of the matching norm weights and of the row's sums of squares go out first, the weight stages
+        // the loads of this thread's share of the rows, of the matching norm weights and of the rows' sums of squares go out first, the weight stages
         // right behind them
-        constexpr int MAXO = (SMH_NORM_IN_MAX_XS_BYTES / 16 + THREADS - 1) / THREADS;     // k-octets per thread
-        h8 hv[MAXO], wv[MAXO];
+        constexpr int MAXO = (SMH_NORM_IN_MAX_XS_BYTES / 16 / NORM_ROWS + THREADS - 1) / THREADS;     // k-octets per thread
+        h8 hv[NORM_ROWS][MAXO], wv[MAXO];
 #pragma unroll
         for (int i = 0; i < MAXO; ++i) {
             const int k = 8 * (tid + i * THREADS);
             if (k < slice_rows) {
-                hv[i] = *reinterpret_cast<const h8 *>(p.a + slice_k0 + k);
+#pragma unroll
+                for (int m = 0; m < NORM_ROWS; ++m) hv[m][i] = *reinterpret_cast<const h8 *>(p.a + m * p.lda + slice_k0 + k);
                 wv[i] = *reinterpret_cast<const h8 *>(p.norm_w + slice_k0 + k);
             }
         }
         const f4 *ss4 = reinterpret_cast<const f4 *>(p.norm_ss);
-        f4 ssv[SMH_NORM_SUMS / 4];
+        f4 ssv[NORM_ROWS * SMH_NORM_SUMS / 4];
 #pragma unroll
-        for (int j = 0; j < SMH_NORM_SUMS / 4; ++j) ssv[j] = ss4[j];
+        for (int j = 0; j < NORM_ROWS * SMH_NORM_SUMS / 4; ++j) ssv[j] = ss4[j];
 #pragma unroll
         for (int i = 0; i < RING_STAGES; ++i)
             if (i < n_steps) issue(ring + i * STAGE, first + i * WAVES);
-        float sum = 0.f;
 #pragma unroll
-        for (int j = 0; j < SMH_NORM_SUMS; ++j) sum += ssv[j / 4][j % 4];
-        const float r = rms_factor(sum, p.K, p.norm_eps);
+        for (int m = 0; m < NORM_ROWS; ++m) {
+            float sum = 0.f;
 #pragma unroll
-        for (int i = 0; i < MAXO; ++i) {
-            const int k = 8 * (tid + i * THREADS);
-            if (k < slice_rows) {
-                h8 o;
+            for (int j = 0; j < SMH_NORM_SUMS; ++j) sum += ssv[m * (SMH_NORM_SUMS / 4) + j / 4][j % 4];
+            const float r = rms_factor(sum, p.K, p.norm_eps);
 #pragma unroll
-                for (int j = 0; j < 8; ++j) o[j] = scale_to_half(hv[i][j], r) * wv[i][j];      // the roundings of partial_rmsnorm_kernel
-                *reinterpret_cast<h8 *>(xs + k) = o;
+            for (int i = 0; i < MAXO; ++i) {
+                const int k = 8 * (tid + i * THREADS);
+                if (k < slice_rows) {
+                    h8 o;
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) o[j] = scale_to_half(hv[m][i][j], r) * wv[i][j];      // the roundings of partial_rmsnorm_kernel
+                    *reinterpret_cast<h8 *>(xs + m * xs_pitch + k) = o;
+                }
             }
         }
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // xs is complete; the DMA ring stays in flight
@@ -574,8 +581,8 @@ int gemv_launch(const MatmulParams &p, hipStream_t stream) {
     const size_t red = (size_t)waves * p.M * GEMV_COLS * sizeof(float);
     if (p.tiled && (p.gu_partial != nullptr || p.norm_w != nullptr))   // rings without activation tiles, xs behind them
         lds = (size_t)waves * RING_BYTES_NO_X + (size_t)p.M * (p.steps_per_slice * 32 + 8) * sizeof(half_t);
-    // RMSNorm inside: one row in LDS, more step by step (figures: q40_gemv_kernel)
-    const bool norm_step = p.tiled && p.norm_w != nullptr && p.gu_partial == nullptr && (p.M > 1 || !gemv_norm_in_fits(p));
+    // RMSNorm inside: one and two rows in LDS, more, and two of a short K-slice, step by step (figures: q40_gemv_kernel)
+    const bool norm_step = p.tiled && p.norm_w != nullptr && p.gu_partial == nullptr && (p.M > 2 || (p.M == 2 && p.steps_per_slice <= 8) || !gemv_norm_in_fits(p));
     if (norm_step) lds = (size_t)waves * RING_BYTES + (size_t)p.steps_per_slice * 64;
     if (red > lds) lds = red;
     if (p.tiled) {
@@ -601,13 +608,16 @@ int gemv_launch(const MatmulParams &p, hipStream_t stream) {
             }
             hipLaunchKernelGGL((q40_gemv_kernel<4>), grid, dim3(256), lds, stream, p);
         } else if (p.norm_w != nullptr) {
-            static const hipError_t lds_ok = hipFuncSetAttribute((const void *)q40_gemv_kernel<3>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                                 80 * 1024);
+            static const hipError_t lds_ok = [] {
+                const hipError_t e = hipFuncSetAttribute((const void *)q40_gemv_kernel<3>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
+                return e != hipSuccess ? e : hipFuncSetAttribute((const void *)q40_gemv_kernel<5>, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
+            }();
             if (lds_ok != hipSuccess) {
                 set_error("q40 gemv: the kernel's LDS could not be reserved: %s", hipGetErrorString(lds_ok));
                 return (int)lds_ok;
             }
-            hipLaunchKernelGGL((q40_gemv_kernel<3>), grid, dim3(256), lds, stream, p);
+            if (p.M == 1) hipLaunchKernelGGL((q40_gemv_kernel<3>), grid, dim3(256), lds, stream, p);
+            else hipLaunchKernelGGL((q40_gemv_kernel<5>), grid, dim3(256), lds, stream, p);
         } else {
             hipLaunchKernelGGL((q40_gemv_kernel<1>), grid, dim3(256), lds, stream, p);
         }
