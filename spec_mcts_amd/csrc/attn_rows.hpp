@@ -52,6 +52,17 @@ __device__ __forceinline__ RowRegs row_from_q40(uint32_t bytes, uint32_t sc, con
     r.b13 = (as_h2((next & C.mask_lo) ^ C.magic_lo) + off_lo) * s_b;
     return r;
 }
+// The same with the masks as literals, for a kernel that lacks the registers (decode_stack_kernel<4>)
+__device__ __forceinline__ RowRegs row_from_q40(uint32_t bytes, uint32_t sc) {
+    const uint32_t u = bytes ^ NIBBLE_FLIP, u1 = u >> 8;
+    const h2 s_a = as_h2(pack_lo16(sc, sc)), s_b = as_h2(pack_hi16(sc, sc));
+    RowRegs r;
+    r.a02 = codes_high(u) * s_a;
+    r.a13 = codes_high(u1) * s_a;
+    r.b02 = codes_low(u) * s_b;
+    r.b13 = codes_low(u1) * s_b;
+    return r;
+}
 __device__ __forceinline__ float row_dot(const RowRegs &k, const RowRegs &q) {
     float s = __builtin_amdgcn_fdot2(k.a02, q.a02, 0.f, false);
     s = __builtin_amdgcn_fdot2(k.a13, q.a13, s, false);

@@ -818,9 +818,15 @@ struct StackCom {
             v.a02 = as_h2(pack_lo16(r.vl[0], r.vl[1])); v.a13 = as_h2(pack_hi16(r.vl[0], r.vl[1]));
             v.b02 = as_h2(pack_lo16(r.vh[0], r.vh[1])); v.b13 = as_h2(pack_hi16(r.vh[0], r.vh[1]));
         } else {
-            const RowCodes codes;
-            k = row_from_q40(r.kl[0], r.kh[0], codes);
-            v = row_from_q40(r.kl[1], r.kh[1], codes);
+            // us a step of the 7B architecture behind 128 rows, 60 of their own, masks in registers and as literals: 3 branches 1751 and 1775, 4 2045 and 2030
+            if constexpr (M == 4) {
+                k = row_from_q40(r.kl[0], r.kh[0]);
+                v = row_from_q40(r.kl[1], r.kh[1]);
+            } else {
+                const RowCodes codes;
+                k = row_from_q40(r.kl[0], r.kh[0], codes);
+                v = row_from_q40(r.kl[1], r.kh[1], codes);
+            }
             if (!in) v.a02 = v.a13 = v.b02 = v.b13 = h2{(half_t)0.f, (half_t)0.f};
         }
 #pragma unroll
