@@ -38,6 +38,16 @@ static bool as_blocks(const smh_layer &L, int M, bool swiglu_in) {
     return M >= BLOCKS_MIN_ROWS && M <= SMH_GEMV_MAX_M && swiglu_in && gemm_swiglu_fits(M, L.dim, L.ffn, true) && blocks_plan(M, L.dim, 3, n_qkv) > 0 &&
            blocks_plan(M, L.heads * 128, 1, n_dim) > 0 && blocks_plan(M, L.ffn, 1, n_dim) > 0;
 }
+// SwiGLU inside w1|w3 of a layer (far: a prefill, or a decode step behind a longer prompt).  17 .. 32 rows want more workgroups than more rows do, as the slabs
+// they save are smaller: two thirds of the compute units up to 24 rows, the half and a sixteenth from there on.  Times as long as with slabs, decode behind 96 to 1024 rows at 17 / 24 /
+// 32 branches and prefills of 17 / 24 / 32: 4096 -> 8192 (128 workgroups) 1.04 / 1.02 / 1.02 and 1.05 / 1.05 / 1.05, 3072 -> 8192 1.04 / 1.03 / 1.03 and 1.02 / 1.04 / 1.01,
+// 4096 -> 9216 (144) 1.00 / 0.98 / 0.97 and level / 1.01 / level, 3584 -> 9728 (152) 1.01 / 1.01 / 1.00 and 1.03 / level / level, 4096 -> 10240 (160, 8 kv heads) 1.01 / 1.00 / 0.99 and
+// 1.015 / 1.01 / level, 5120 -> 10240 1.01 / 1.00 / 0.99; 4096 -> 11008 (172) 0.94 / 0.93 / 0.93, 3072 -> 12288 0.93 / 0.92 / 0.90.
+static bool swiglu_inside(const smh_layer &L, int M, bool blocks, bool far) {
+    if (!gemm_swiglu_fits(M, L.dim, L.ffn, true)) return false;
+    if (M <= SMH_GEMV_MAX_M) return blocks;
+    return M > 32 || (far && 2 * (L.ffn / 128) >= (M <= 24 ? 171 : 144));
+}
 // A launch that stores its fp16 results itself (more than 128 rows, no K-split) leaves no slabs.  layer_buffers reserves none for it,
 // so every linear below asks here before it takes the slab form.
 static bool direct(int M, int K, int nseg, const int *n) { return smh_q40_matmul_tiled_direct_fits(M, K, nseg, n) == 1; }
@@ -127,7 +137,7 @@ struct LayerRun {
 
     LayerRun(const smh_layer &l, smh_pass &s, smh_stream_t st, bool far)
         : L(l), S(s), stream(st), M(s.rows), nq(l.heads * 128), nkv(l.kv_heads * 128), blocks(far && as_blocks(l, s.rows, s.swiglu_in != 0)),
-          swiglu(s.swiglu_in != 0 && (s.rows > SMH_GEMV_MAX_M ? s.rows > 32 || far : blocks) && gemm_swiglu_fits(s.rows, l.dim, l.ffn, true)), n_qkv{nq, nkv, nkv}, n_gu{l.ffn, l.ffn}, n_dim{l.dim},
+          swiglu(s.swiglu_in != 0 && swiglu_inside(l, s.rows, blocks, far)), n_qkv{nq, nkv, nkv}, n_gu{l.ffn, l.ffn}, n_dim{l.dim},
           w_qkv{l.wq, l.wk, l.wv}, w_o{l.wo}, w_gu{l.w1, l.w3}, w_d{l.w2} {}
     int slabs(int K, int nseg, const int *n) const { return blocks ? blocks_plan(M, K, nseg, n) : slices(M, K, nseg, n); }
     int begin(const char *who) {

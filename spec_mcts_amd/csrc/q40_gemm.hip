@@ -1708,7 +1708,7 @@ static int gemm_kg_launch(const MatmulParams &p, hipStream_t stream) {
 // 64, two weights of n_half columns (a multiple of 128) whose 2 * n_half / 128 workgroups fit the compute units in one round;
 // `worth_it`: and fill at least half of them (narrower weights are faster as two kernels with a K-split; w1|w3 + SiLU of the 7B shape 38.1 against
 // 44.9 us at 100 rows, 29.1 against 31.5 at 64, level at 32).  From how many rows on is for the caller: smh_q40_swiglu_fits says 33, layer calls behind a longer
-// prompt, whose norms ask for the weights, 5 (as_blocks) and 17.
+// prompt 5 (as_blocks) and 17 (swiglu_inside).
 bool gemm_swiglu_fits(int M, int K, int n_half, bool worth_it) {
     if (M < 1 || K <= 0 || n_half <= 0 || n_half % 128 != 0) return false;
     if (M > GEMM_BM) return K % 32 == 0;                        // gemm_swiglu_rows_launch

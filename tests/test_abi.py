@@ -270,6 +270,21 @@ def test_form_of_a_layer():
     assert form(*L7, 96, 0)[0] < 0 and form(4096, 32, 5, 11008, 96, 8)[0] < 0 and form(100, 32, 32, 11008, 96, 8)[0] < 0
 
 
+@pytest.mark.parametrize("dim,heads,kv_heads,ffn,wide_from", [(4096, 32, 32, 8192, 33), (3072, 24, 8, 8192, 33), (4096, 32, 32, 9088, 33), (4096, 32, 32, 9216, 25), (3584, 28, 28, 9728, 25),
+                                                              (4096, 32, 8, 10240, 25), (5120, 40, 8, 10240, 25), (4096, 32, 32, 10880, 25), (4096, 32, 32, 11008, 17), (3072, 24, 24, 12288, 17)])
+def test_swiglu_of_17_to_32_rows_wants_wide_weights(dim, heads, kv_heads, ffn, wide_from):
+    """SwiGLU inside w1|w3 up to 32 rows only where its workgroups fill the compute units far enough; slabs below, as behind short prompts"""
+    from spec_mcts_amd import _lib
+    lib, layer, slabs = _lib.load(), _lib.SmhLayer(), (ctypes.c_int * 4)()
+    layer.dim, layer.heads, layer.kv_heads, layer.ffn = dim, heads, kv_heads, ffn
+    for P in (95, 96, 1024):
+        layer.prompt_len = P
+        for M in (17, 20, 24, 25, 31, 32, 33, 100):
+            inside = M > 32 or (P >= 96 and M >= wide_from)
+            assert lib.smh_decode_layer_form(layer, M, 1, slabs) == (2 if inside else 0), (P, M)
+            assert (slabs[2] == 0) == inside
+
+
 def test_columns_of_a_workgroup_above_128_rows():
     """which of the launches above 128 rows a shape takes (the GPU tests of each ask here), 0 where there is none"""
     from spec_mcts_amd import _lib
