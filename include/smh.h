@@ -473,6 +473,9 @@ size_t smh_decode_scratch_bytes(const smh_layer *layer, int rows, int swiglu_in)
 /* How smh_decode_layer runs a layer (its sizes and prompt_len) for `rows` branches: bit 0: 5 .. 16 rows on the 128-column blocks that more rows take, bit 1:
  * SwiGLU inside w1|w3; slabs: K-slices that wq|wk|wv, wo, w1|w3 and w2 leave (0: none, the launch stores fp16).  Negative: refused.  Host arithmetic only. */
 int smh_decode_layer_form(const smh_layer *layer, int rows, int swiglu_in, int *slabs);
+/* Which launches of such a layer ask for the next one's weights ahead of it (smh_q40_warm_span): bit 0: the RMSNorm for wq|wk|wv, bit 1: for w1|w3, bit 2: the
+ * attention, where smh_shared_prefix_attn_qkv_tiles makes it, for wo, bit 3: SwiGLU for w2.  Negative: refused.  Host arithmetic only. */
+int smh_decode_layer_asks(const smh_layer *layer, int rows, int swiglu_in);
 int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stream_t stream);
 int smh_prefill_layer(const smh_layer *layer, smh_pass *pass, smh_stream_t stream);
 /* All layers of a decode step of a few branches in one launch (of up to 32 layers): what smh_decode_layer does layer by layer, with sums in

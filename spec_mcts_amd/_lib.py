@@ -112,6 +112,7 @@ SIGNATURES = {
     "smh_q40_matmul_tiled_direct_rope": (c_int, [_P, c_int, c_int, c_long, c_int, _P, _P, _P, c_int, _P, _P, _P]),
     "smh_partial_rope_rows": (c_int, [_P, c_int, c_int, c_int, c_int, c_int, _P, _P, _P, _P, _P, c_int, _P]),
     "smh_decode_layer": (c_int, [_LAYER, _PASS, _P]),
+    "smh_decode_layer_asks": (c_int, [_LAYER, c_int, c_int]),
     "smh_decode_layer_form": (c_int, [_LAYER, c_int, c_int, ctypes.POINTER(c_int)]),
     "smh_decode_stack_workspace_bytes": (c_size_t, [_LAYER, c_int]),
     "smh_decode_stack_fits": (c_int, [_P, c_int, c_int]),

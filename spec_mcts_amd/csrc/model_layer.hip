@@ -21,8 +21,13 @@ struct LayerBuffers {
 
 // Stages of the next launch's weights that a launch asks for (q40_warm.hpp).  The norms of layers whose w1|w3 leaves slabs do not ask (17 .. 28 branches of the 7B
 // shape behind 64 prompt rows: 0.992 .. 0.997 times as fast); their attention does (17 .. 100 branches behind 256 and 512 rows, SwiGLU switched off: 1.001 .. 1.009).
-// Nothing is asked for where a layer's weights are larger and its attention brings its own long prompt (three layers of 64 heads over 8, dim 8192, 17 .. 100 branches behind 1024 rows: 0.998 .. 1.001 times as fast from the norms, 0.996 .. 1.000 from the attention).
-constexpr int WARM_MAX_DIM = 8191, WARM_FROM_NORM = 3, WARM_FROM_ATTENTION = 4, WARM_FROM_SWIGLU = 16;
+// Nothing is asked for outside of dims 3585 .. 4096.  A wider RMSNorm takes two passes, and one of its workgroups a compute unit's registers, so that the asking ones wait
+// for the rows or the rows for them; narrower layers' launches are shorter than the asking.  Times as long with the asking as without it, decode behind 96 to 1024
+// rows at 33 / 48 / 65 / 100 branches: dim 4096, FFN 11008 0.97 / 0.96 / 0.985 / 0.995, dim 3840, FFN 10240 (32 branches) 0.98 / 0.97 / 0.995 / 0.98; dim 3584, FFN 9728
+// 1.01 / 1.00 / 0.99 / 0.985, 3072, 8192 1.015 / 1.015 / 1.02 / 1.015, 2048, 8192 1.01 / 1.01 / 1.015 / 1.015, 2048, 5632 level / level / 1.01 / 1.01; 4608, 12288 1.03 / 1.02 / 1.02 / 1.01, 5120, 13824
+// 1.025 / 1.015 / 1.015 / 1.005, 5120, 10240 1.01 / 1.07 / 0.985 / 0.985, 6144, 16384 1.01 / 1.01 / level / level; three layers of 64 heads over 8, dim 8192, 17 .. 100 branches behind
+// 1024 rows 0.999 .. 1.002 from the norms, 1.000 .. 1.004 from the attention.
+constexpr int WARM_MIN_DIM = 3585, WARM_MAX_DIM = 4096, WARM_FROM_NORM = 3, WARM_FROM_ATTENTION = 4, WARM_FROM_SWIGLU = 16;
 
 static int slices(int M, int K, int nseg, const int *n) { return smh_q40_matmul_plan_tiled(M, K, nseg, n); }
 // Launches of 17 rows and more (128-column blocks, SwiGLU inside w1|w3, the norms and the attention asking for the next weights) for a layer of fewer, too,
@@ -51,10 +56,6 @@ static bool swiglu_inside(const smh_layer &L, int M, bool blocks, bool far) {
 // A launch that stores its fp16 results itself (more than 128 rows, no K-split) leaves no slabs.  layer_buffers reserves none for it,
 // so every linear below asks here before it takes the slab form.
 static bool direct(int M, int K, int nseg, const int *n) { return smh_q40_matmul_tiled_direct_fits(M, K, nseg, n) == 1; }
-
-static WarmWeights ask(const smh_layer &L, bool blocks, int M, int K, int nseg, const void *const *w, const int *n, bool swiglu, int stages, int workgroups) {
-    return L.dim <= WARM_MAX_DIM && (M > SMH_GEMV_MAX_M || blocks) ? q40_warm(M, K, nseg, w, n, swiglu, stages, workgroups) : WarmWeights{};
-}
 
 // The attention of a decode layer: in one launch whose last workgroups merge (ONE, up to 16 queries a kv head), in one launch of 8 or 16
 // queries a workgroup (TILES), or RoPE, prefix slices and walks (LAUNCHES).  us a call with RoPE and append, caches in HBM (32 heads, up to 16 branches: two slabs, 10 own rows):
@@ -139,6 +140,17 @@ struct LayerRun {
         : L(l), S(s), stream(st), M(s.rows), nq(l.heads * 128), nkv(l.kv_heads * 128), blocks(far && as_blocks(l, s.rows, s.swiglu_in != 0)),
           swiglu(s.swiglu_in != 0 && swiglu_inside(l, s.rows, blocks, far)), n_qkv{nq, nkv, nkv}, n_gu{l.ffn, l.ffn}, n_dim{l.dim},
           w_qkv{l.wq, l.wk, l.wv}, w_o{l.wo}, w_gu{l.w1, l.w3}, w_d{l.w2} {}
+    // What the launches of a decode layer ask for ahead: the norms, where SwiGLU is inside, for the product behind them, the attention of tiles for wo, SwiGLU for w2
+    bool asks() const { return L.dim >= WARM_MIN_DIM && L.dim <= WARM_MAX_DIM && (M > SMH_GEMV_MAX_M || blocks); }
+    WarmWeights ask_qkv() const { return asks() && swiglu ? q40_warm(M, L.dim, 3, w_qkv, n_qkv, false, WARM_FROM_NORM, 256) : WarmWeights{}; }
+    WarmWeights ask_gu() const { return asks() && swiglu ? q40_warm(M, L.dim, 2, w_gu, n_gu, true, WARM_FROM_NORM, 256) : WarmWeights{}; }
+    WarmWeights ask_o() const {
+        const int row = (L.kv_heads + 7) / 8 * 8;
+        WarmWeights wo = asks() ? q40_warm(M, nq, 1, w_o, n_dim, false, WARM_FROM_ATTENTION, attn_tiles_idle(M, L.heads, L.kv_heads)) : WarmWeights{};
+        wo.workgroups = wo.workgroups / row * row;
+        return wo;
+    }
+    WarmWeights ask_d() const { return asks() && swiglu ? q40_warm(M, L.ffn, 1, w_d, n_dim, false, WARM_FROM_SWIGLU, swiglu_idle(L.ffn)) : WarmWeights{}; }
     int slabs(int K, int nseg, const int *n) const { return blocks ? blocks_plan(M, K, nseg, n) : slices(M, K, nseg, n); }
     int begin(const char *who) {
         SMH_REQUIRE(M >= 1 && L.heads > 0 && L.kv_heads > 0 && L.heads % L.kv_heads == 0, "%s: rows=%d heads=%d kv_heads=%d", who, M, L.heads, L.kv_heads);
@@ -195,6 +207,22 @@ extern "C" int smh_decode_layer_form(const smh_layer *layer, int rows, int swigl
     return (run.blocks ? 1 : 0) | (run.swiglu ? 2 : 0);
 }
 
+extern "C" int smh_decode_layer_asks(const smh_layer *layer, int rows, int swiglu_in) {
+    const char *who = "smh_decode_layer_asks";
+    SMH_REQUIRE(layer, "%s: null pointer", who);
+    int slabs[4];
+    const int form = smh_decode_layer_form(layer, rows, swiglu_in, slabs);
+    if (form < 0) return form;
+    smh_layer L = *layer;
+    const void *const some = (const void *)128;             // (weights that a product would take)
+    L.wq = L.wk = L.wv = L.wo = L.w1 = L.w2 = L.w3 = some;
+    smh_pass pass{};
+    pass.rows = rows;
+    pass.swiglu_in = swiglu_in != 0;
+    const LayerRun run(L, pass, nullptr, L.prompt_len >= BLOCKS_MIN_PROMPT);
+    return (run.ask_qkv().workgroups > 0 ? 1 : 0) | (run.ask_gu().workgroups > 0 ? 2 : 0) | (run.ask_o().workgroups > 0 ? 4 : 0) | (run.ask_d().workgroups > 0 ? 8 : 0);
+}
+
 extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stream_t stream) {
     const char *who = "smh_decode_layer";
     SMH_REQUIRE(layer && pass && pass->h, "%s: null pointer", who);
@@ -208,7 +236,7 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
     // the RMSNorm of the residual stream and the linears behind it: to slab_a.  With few rows the RMSNorm is made inside the linears' launch.
     auto norm_linears = [&](const void *weight, float eps, int nseg, const void *const *w, const int *n) -> int {
         if (S.pending == 0 || M > S.norm_in_rows || run.blocks || ((uintptr_t)weight & 15) != 0 || smh_decode_norm_in_fits(M, L.dim, nseg, n) != 1) {
-            if (int r = run.norm(weight, eps, run.swiglu ? ask(L, run.blocks, M, L.dim, nseg, w, n, false, WARM_FROM_NORM, 256) : WarmWeights{})) return r;
+            if (int r = run.norm(weight, eps, nseg == 3 ? run.ask_qkv() : WarmWeights{})) return r;
             return matmul_partial_tiled(b.xn, M, L.dim, L.dim, nseg, w, n, b.slab_a, b.slab_a_bytes, run.blocks, stream);
         }
         void *h_out = b.h[S.h == b.h[0]];
@@ -249,12 +277,9 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
                                         L.prompt_len, L.cache_k, L.cache_ks, L.cache_v, L.cache_vs, S.smax, S.t_dev, S.pages, S.pages_stride, one, ws,
                                         ws_bytes, stream);
     } else if (way == ATTN_TILES) {
-        const int row = (L.kv_heads + 7) / 8 * 8, idle = attn_tiles_idle(M, L.heads, L.kv_heads);
-        WarmWeights wo = ask(L, run.blocks, M, nq, 1, run.w_o, run.n_dim, false, WARM_FROM_ATTENTION, idle);
-        wo.workgroups = wo.workgroups / row * row;
         st = shared_prefix_attn_qkv_tiles(b.slab_a, ks_qkv, b.att, M, L.heads, L.kv_heads, 128, S.cos_tab, S.sin_tab, S.pos_dev, L.prompt_k, L.prompt_v,
                                           L.prompt_len, L.cache_k, L.cache_ks, L.cache_v, L.cache_vs, S.smax, S.t_dev, S.pages, S.pages_stride,
-                                          S.cache_rows, wo, stream);
+                                          S.cache_rows, run.ask_o(), stream);
     } else {
         st = qkv_direct ? smh_rope_append_kv(b.q, b.k, b.v, M, L.heads, L.kv_heads, 128, S.cos_tab, S.sin_tab, S.pos_dev, L.cache_k, L.cache_ks, L.cache_v,
                                              L.cache_vs, S.smax, S.t_dev, stream)
@@ -273,9 +298,8 @@ extern "C" int smh_decode_layer(const smh_layer *layer, smh_pass *pass, smh_stre
     if ((st = run.residual_linear(b.att, nq, run.w_o))) return st;
     // ---- feed forward ----
     if (run.swiglu) {
-        if ((st = run.norm(L.ffn_norm, L.ffn_eps, ask(L, run.blocks, M, L.dim, 2, run.w_gu, run.n_gu, true, WARM_FROM_NORM, 256)))) return st;
-        const WarmWeights w2 = ask(L, run.blocks, M, L.ffn, 1, run.w_d, run.n_dim, false, WARM_FROM_SWIGLU, swiglu_idle(L.ffn));
-        if ((st = matmul_tiled_swiglu(b.xn, M, L.dim, L.dim, L.w1, L.w3, L.ffn, b.act, L.ffn, w2, stream))) return st;
+        if ((st = run.norm(L.ffn_norm, L.ffn_eps, run.ask_gu()))) return st;
+        if ((st = matmul_tiled_swiglu(b.xn, M, L.dim, L.dim, L.w1, L.w3, L.ffn, b.act, L.ffn, run.ask_d(), stream))) return st;
         return run.residual_linear(b.act, L.ffn, run.w_d);
     }
     if ((st = norm_linears(L.ffn_norm, L.ffn_eps, 2, run.w_gu, run.n_gu))) return st;

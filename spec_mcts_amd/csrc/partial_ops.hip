@@ -334,8 +334,8 @@ template <int RES> static const reduce_kernel_t REDUCE_KERNELS[17] = BY_SLABS(K_
 #define K_OF(n) partial_rmsnorm_kernel<PASSES, n>
 template <int PASSES> static const rmsnorm_kernel_t RMSNORM_KERNELS[17] = BY_SLABS(K_OF, K_OF(0));
 #undef K_OF
-#define K_OF(n) partial_rmsnorm_kernel<PASSES, n, WarmWeights>
-template <int PASSES> static const rmsnorm_ask_t RMSNORM_ASK_KERNELS[17] = BY_SLABS(K_OF, nullptr);
+#define K_OF(n) partial_rmsnorm_kernel<1, n, WarmWeights>
+static const rmsnorm_ask_t RMSNORM_ASK_KERNELS[17] = BY_SLABS(K_OF, nullptr);
 #undef K_OF
 #define K_OF(n) partial_residual_sumsq_kernel<PASSES, n>
 template <int PASSES> static const sumsq_kernel_t SUMSQ_KERNELS[17] = BY_SLABS(K_OF, nullptr);
@@ -740,9 +740,8 @@ int smh::partial_rmsnorm(const void *partial, int ksplit, int M, int N, const vo
     }
     const int ks = partial == nullptr ? 0 : ksplit;
     const auto kern = N <= 4096 ? RMSNORM_KERNELS<1>[ks] : N <= 8192 ? RMSNORM_KERNELS<2>[ks] : RMSNORM_KERNELS<4>[ks];
-    if (next.workgroups > 0 && ks > 0 && N <= 8192) {
-        const auto ask = N <= 4096 ? RMSNORM_ASK_KERNELS<1>[ks] : RMSNORM_ASK_KERNELS<2>[ks];
-        hipLaunchKernelGGL(ask, dim3(M, 1 + (next.workgroups + M - 1) / M), dim3(1024), 0, (hipStream_t)stream, partial, ks, M, N, (const half_t *)h_in,
+    if (next.workgroups > 0 && ks > 0 && N <= 4096) {
+        hipLaunchKernelGGL(RMSNORM_ASK_KERNELS[ks], dim3(M, 1 + (next.workgroups + M - 1) / M), dim3(1024), 0, (hipStream_t)stream, partial, ks, M, N, (const half_t *)h_in,
                            (const half_t *)weight, eps, (half_t *)h_out, (half_t *)xn_out, next);
         return launch_status();
     }

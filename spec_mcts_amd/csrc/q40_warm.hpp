@@ -7,6 +7,7 @@
 // (from another one, through the Infinity Cache, half of the gain of w2's stages is left) - and drop it.  Nothing waits for them but the end of the launch.
 // A step of the 7B architecture behind 512 rows, in turn with the launches without, two cards: 17 .. 32 branches 1.003 .. 1.009 times as fast, 33 .. 64 (us, 48:
 // 2720 and 2616) 1.028 .. 1.043, 65 .. 100 (3494 and 3434, 3676 and 3665) 1.002 .. 1.018.
+// (Dims of 3585 .. 4096; of others in model_layer.hip.)
 // How many stages (us a step of the 7B architecture, 37 forked and 100 branches, 2418 and 3440 without): wq|wk|wv and w1|w3 from the norms 2: 2408 and 3427,
 // 3: 2404 and 3425, 8: 2416 and 3446 (the norms end later), wo from the attention 4 more: 2395 and 3422, w2 from SwiGLU, too, all of its 22 stages: 2332 and
 // 3387, 16: 2335 and 3367, 8: 2369 and 3384.  The prompt's rows for the attention, from wq|wk|wv's idle compute units: no gain.  GEMVs, which

@@ -285,6 +285,27 @@ def test_swiglu_of_17_to_32_rows_wants_wide_weights(dim, heads, kv_heads, ffn, w
             assert (slabs[2] == 0) == inside
 
 
+def _asks(dim, heads, kv_heads, ffn, P, M, swiglu=1):
+    from spec_mcts_amd import _lib
+    layer = _lib.SmhLayer()
+    layer.dim, layer.heads, layer.kv_heads, layer.ffn, layer.prompt_len = dim, heads, kv_heads, ffn, P
+    return _lib.load().smh_decode_layer_asks(layer, M, swiglu)
+
+
+@pytest.mark.parametrize("dim,heads,kv_heads,ffn,some", [(4096, 32, 32, 11008, True), (3840, 30, 30, 10240, True), (3584, 28, 28, 9728, False), (3072, 24, 8, 8192, False),
+                                                         (2048, 16, 16, 5632, False), (4608, 36, 36, 12288, False), (5120, 40, 40, 13824, False), (5120, 40, 8, 10240, False),
+                                                         (6144, 48, 48, 16384, False), (8192, 64, 8, 28672, False)])
+def test_dims_whose_launches_ask_for_weights_ahead(dim, heads, kv_heads, ffn, some):
+    """where asking was the slower way nothing is asked for, whatever the rows and the prompt; nor of up to 16 rows on GEMVs"""
+    for P in (0, 96, 1024):
+        for M in (1, 5, 16, 17, 33, 48, 65, 100, 128):
+            asks = _asks(dim, heads, kv_heads, ffn, P, M)
+            assert asks == 0 or (some and (M > 16 or P >= 96)), (P, M, asks)
+        assert (_asks(dim, heads, kv_heads, ffn, P, 33) == 15) == some
+        assert _asks(dim, heads, kv_heads, ffn, P, 33, 0) == (4 if some else 0)
+    assert _asks(dim, heads, kv_heads, ffn, 96, 0) < 0
+
+
 def test_columns_of_a_workgroup_above_128_rows():
     """which of the launches above 128 rows a shape takes (the GPU tests of each ask here), 0 where there is none"""
     from spec_mcts_amd import _lib
