@@ -20,14 +20,17 @@ struct LayerBuffers {
 };
 
 // Stages of the next launch's weights that a launch asks for (q40_warm.hpp).  The norms of layers whose w1|w3 leaves slabs do not ask (17 .. 28 branches of the 7B
-// shape behind 64 prompt rows: 0.992 .. 0.997 times as fast); their attention does (17 .. 100 branches behind 256 and 512 rows, SwiGLU switched off: 1.001 .. 1.009).
+// shape behind 64 prompt rows: 0.992 .. 0.997 times as fast); their attention does (17 .. 48 branches behind 256 and 512 rows, SwiGLU switched off: 1.001 .. 1.009).
+// Up to three row tiles, that is: above, the attention's workgroups are many and long themselves (dim 4096, times as long with its asking as without, 17 / 32 / 48 / 64 / 65 / 80 / 100
+// branches: FFN 11008 0.995 / 0.99 / level / level / 1.005 / 1.002 / 1.003, 8192 1.001 / 1.004 / 0.999 / - / 1.005 / 1.002 / 1.006, 12288 0.996 / 0.999 / 0.997 / - / 1.004 / 1.003 / 1.002, 16384
+// 1.003 / 1.002 / 1.003 / - / 1.004 / 1.005 / 1.027).
 // Nothing is asked for outside of dims 3585 .. 4096.  A wider RMSNorm takes two passes, and one of its workgroups a compute unit's registers, so that the asking ones wait
 // for the rows or the rows for them; narrower layers' launches are shorter than the asking.  Times as long with the asking as without it, decode behind 96 to 1024
 // rows at 33 / 48 / 65 / 100 branches: dim 4096, FFN 11008 0.97 / 0.96 / 0.985 / 0.995, dim 3840, FFN 10240 (32 branches) 0.98 / 0.97 / 0.995 / 0.98; dim 3584, FFN 9728
 // 1.01 / 1.00 / 0.99 / 0.985, 3072, 8192 1.015 / 1.015 / 1.02 / 1.015, 2048, 8192 1.01 / 1.01 / 1.015 / 1.015, 2048, 5632 level / level / 1.01 / 1.01; 4608, 12288 1.03 / 1.02 / 1.02 / 1.01, 5120, 13824
 // 1.025 / 1.015 / 1.015 / 1.005, 5120, 10240 1.01 / 1.07 / 0.985 / 0.985, 6144, 16384 1.01 / 1.01 / level / level; three layers of 64 heads over 8, dim 8192, 17 .. 100 branches behind
 // 1024 rows 0.999 .. 1.002 from the norms, 1.000 .. 1.004 from the attention.
-constexpr int WARM_MIN_DIM = 3585, WARM_MAX_DIM = 4096, WARM_FROM_NORM = 3, WARM_FROM_ATTENTION = 4, WARM_FROM_SWIGLU = 16;
+constexpr int WARM_MIN_DIM = 3585, WARM_MAX_DIM = 4096, WARM_FROM_NORM = 3, WARM_FROM_ATTENTION = 4, WARM_FROM_ATTENTION_ROWS = 48, WARM_FROM_SWIGLU = 16;
 
 static int slices(int M, int K, int nseg, const int *n) { return smh_q40_matmul_plan_tiled(M, K, nseg, n); }
 // Launches of 17 rows and more (128-column blocks, SwiGLU inside w1|w3, the norms and the attention asking for the next weights) for a layer of fewer, too,
@@ -146,7 +149,7 @@ struct LayerRun {
     WarmWeights ask_gu() const { return asks() && swiglu ? q40_warm(M, L.dim, 2, w_gu, n_gu, true, WARM_FROM_NORM, 256) : WarmWeights{}; }
     WarmWeights ask_o() const {
         const int row = (L.kv_heads + 7) / 8 * 8;
-        WarmWeights wo = asks() ? q40_warm(M, nq, 1, w_o, n_dim, false, WARM_FROM_ATTENTION, attn_tiles_idle(M, L.heads, L.kv_heads)) : WarmWeights{};
+        WarmWeights wo = asks() && M <= WARM_FROM_ATTENTION_ROWS ? q40_warm(M, nq, 1, w_o, n_dim, false, WARM_FROM_ATTENTION, attn_tiles_idle(M, L.heads, L.kv_heads)) : WarmWeights{};
         wo.workgroups = wo.workgroups / row * row;
         return wo;
     }

@@ -306,6 +306,15 @@ def test_dims_whose_launches_ask_for_weights_ahead(dim, heads, kv_heads, ffn, so
     assert _asks(dim, heads, kv_heads, ffn, 96, 0) < 0
 
 
+@pytest.mark.parametrize("ffn", [8192, 11008, 16384])
+def test_attention_of_many_branches_asks_for_nothing(ffn):
+    """wo's weights are asked for up to three row tiles, with 32 kv heads and with 8"""
+    for kv_heads in (32, 8):
+        for M in (17, 32, 47, 48, 49, 64, 65, 100, 128):
+            for swiglu in (0, 1):
+                assert (_asks(4096, 32, kv_heads, ffn, 512, M, swiglu) & 4 != 0) == (M <= 48), (kv_heads, M)
+
+
 def test_columns_of_a_workgroup_above_128_rows():
     """which of the launches above 128 rows a shape takes (the GPU tests of each ask here), 0 where there is none"""
     from spec_mcts_amd import _lib
