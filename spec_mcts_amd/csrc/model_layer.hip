@@ -30,7 +30,10 @@ struct LayerBuffers {
 // 1.01 / 1.00 / 0.99 / 0.985, 3072, 8192 1.015 / 1.015 / 1.02 / 1.015, 2048, 8192 1.01 / 1.01 / 1.015 / 1.015, 2048, 5632 level / level / 1.01 / 1.01; 4608, 12288 1.03 / 1.02 / 1.02 / 1.01, 5120, 13824
 // 1.025 / 1.015 / 1.015 / 1.005, 5120, 10240 1.01 / 1.07 / 0.985 / 0.985, 6144, 16384 1.01 / 1.01 / level / level; three layers of 64 heads over 8, dim 8192, 17 .. 100 branches behind
 // 1024 rows 0.999 .. 1.002 from the norms, 1.000 .. 1.004 from the attention.
-constexpr int WARM_MIN_DIM = 3585, WARM_MAX_DIM = 4096, WARM_FROM_NORM = 3, WARM_FROM_ATTENTION = 4, WARM_FROM_ATTENTION_ROWS = 48, WARM_FROM_SWIGLU = 16;
+// SwiGLU's launch asks for w2 where 40 compute units and more are left to do it (dim 4096, times as long with its asking as without at 17 / 24 / 32 / 48 branches: FFN 13312, 48 units
+// 1.00 / 0.99 / 0.995 / 0.98, 13824, 40 units 0.995 / - / 0.99 / 0.985; 14336, 32 units 1.00 / 1.02 / 1.03 / 1.015), and the norms do where it leaves 32 (14336, without w2's,
+// 0.995 / 0.985 / 0.985 / 0.985; 16384, where it fills the chip, 1.01 / 1.01 / 1.02 / 1.00, at 5 and 16 branches 1.01 and 1.005).
+constexpr int WARM_MIN_DIM = 3585, WARM_MAX_DIM = 4096, WARM_FROM_NORM = 3, WARM_FROM_ATTENTION = 4, WARM_FROM_ATTENTION_ROWS = 48, WARM_FROM_SWIGLU = 16, WARM_NORM_MIN_IDLE = 32, WARM_SWIGLU_MIN_IDLE = 40;
 
 static int slices(int M, int K, int nseg, const int *n) { return smh_q40_matmul_plan_tiled(M, K, nseg, n); }
 // Launches of 17 rows and more (128-column blocks, SwiGLU inside w1|w3, the norms and the attention asking for the next weights) for a layer of fewer, too,
@@ -145,15 +148,15 @@ struct LayerRun {
           w_qkv{l.wq, l.wk, l.wv}, w_o{l.wo}, w_gu{l.w1, l.w3}, w_d{l.w2} {}
     // What the launches of a decode layer ask for ahead: the norms, where SwiGLU is inside, for the product behind them, the attention of tiles for wo, SwiGLU for w2
     bool asks() const { return L.dim >= WARM_MIN_DIM && L.dim <= WARM_MAX_DIM && (M > SMH_GEMV_MAX_M || blocks); }
-    WarmWeights ask_qkv() const { return asks() && swiglu ? q40_warm(M, L.dim, 3, w_qkv, n_qkv, false, WARM_FROM_NORM, 256) : WarmWeights{}; }
-    WarmWeights ask_gu() const { return asks() && swiglu ? q40_warm(M, L.dim, 2, w_gu, n_gu, true, WARM_FROM_NORM, 256) : WarmWeights{}; }
+    WarmWeights ask_qkv() const { return asks() && swiglu && swiglu_idle(L.ffn) >= WARM_NORM_MIN_IDLE ? q40_warm(M, L.dim, 3, w_qkv, n_qkv, false, WARM_FROM_NORM, 256) : WarmWeights{}; }
+    WarmWeights ask_gu() const { return asks() && swiglu && swiglu_idle(L.ffn) >= WARM_NORM_MIN_IDLE ? q40_warm(M, L.dim, 2, w_gu, n_gu, true, WARM_FROM_NORM, 256) : WarmWeights{}; }
     WarmWeights ask_o() const {
         const int row = (L.kv_heads + 7) / 8 * 8;
         WarmWeights wo = asks() && M <= WARM_FROM_ATTENTION_ROWS ? q40_warm(M, nq, 1, w_o, n_dim, false, WARM_FROM_ATTENTION, attn_tiles_idle(M, L.heads, L.kv_heads)) : WarmWeights{};
         wo.workgroups = wo.workgroups / row * row;
         return wo;
     }
-    WarmWeights ask_d() const { return asks() && swiglu ? q40_warm(M, L.ffn, 1, w_d, n_dim, false, WARM_FROM_SWIGLU, swiglu_idle(L.ffn)) : WarmWeights{}; }
+    WarmWeights ask_d() const { return asks() && swiglu && swiglu_idle(L.ffn) >= WARM_SWIGLU_MIN_IDLE ? q40_warm(M, L.ffn, 1, w_d, n_dim, false, WARM_FROM_SWIGLU, swiglu_idle(L.ffn)) : WarmWeights{}; }
     int slabs(int K, int nseg, const int *n) const { return blocks ? blocks_plan(M, K, nseg, n) : slices(M, K, nseg, n); }
     int begin(const char *who) {
         SMH_REQUIRE(M >= 1 && L.heads > 0 && L.kv_heads > 0 && L.heads % L.kv_heads == 0, "%s: rows=%d heads=%d kv_heads=%d", who, M, L.heads, L.kv_heads);

@@ -315,6 +315,14 @@ def test_attention_of_many_branches_asks_for_nothing(ffn):
                 assert (_asks(4096, 32, kv_heads, ffn, 512, M, swiglu) & 4 != 0) == (M <= 48), (kv_heads, M)
 
 
+@pytest.mark.parametrize("ffn,asks", [(9216, 11), (11008, 11), (13824, 11), (13952, 3), (14336, 3), (14464, 0), (16384, 0)])
+def test_swiglu_that_fills_the_chip_asks_for_nothing(ffn, asks):
+    """w2 is asked for from 40 idle compute units on, by the norms where 32 are idle in SwiGLU's launch (bits: wq|wk|wv, w1|w3, wo, w2)"""
+    for kv_heads in (32, 8):
+        for M in (5, 16, 25, 33, 100):
+            assert _asks(4096, 32, kv_heads, ffn, 512, M) & ~4 == asks, (kv_heads, M)
+
+
 def test_columns_of_a_workgroup_above_128_rows():
     """which of the launches above 128 rows a shape takes (the GPU tests of each ask here), 0 where there is none"""
     from spec_mcts_amd import _lib
