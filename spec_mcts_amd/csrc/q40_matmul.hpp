@@ -71,18 +71,17 @@ struct MatmulParams {
     // its own K-slice from the slabs of the gate|up product, a[m][k] = silu(gate[m][k]) * up[m][k] (gate = columns
     // 0..K-1, up = columns K..2K-1 of the slabs), with the roundings of partial_silu_mul_kernel
     const float *gu_partial;
-    int gu_ksplit;
     // GEMV, norm_w != nullptr: `a` holds the un-normalised residual stream h; every workgroup makes its K-slice of
     // RMSNorm(h) * norm_w itself, a[m][k] = fp16(fp16(h[m][k] * r[m]) * norm_w[k]) with r[m] = 1 / sqrt(sum / K + eps)
     // and sum = norm_ss[m][0] + ... + norm_ss[m][SMH_NORM_SUMS - 1] added in that order (partial_rmsnorm_kernel's roundings)
-    const half_t *norm_w;
-    const float *norm_ss;
-    float norm_eps;
-    // GEMM, direct on tiled weights: columns [0, rope_cols) of the outputs laid end to end are heads of 128 that leave rotated, row m at position m
+    // GEMM, direct on tiled weights, rope_cos != nullptr: columns [0, rope_cols) of the outputs laid end to end are heads of 128 that leave rotated, row m at position m
     // (in the place of rope_kernel behind it, 5.7 us at 512 rows and 12.6 at 2047 of the 7B shape; a prefill of 384 / 512 / 1024 / 2047 rows 6707 / 7912 / 14451 / 26706
     // -> 6572 / 7757 / 14240 / 26392 us.  With the factors loaded by the storing threads, not brought by the DMA waves, the wide kernels gained half of that.)
-    int rope_cols;
-    const half_t *rope_cos, *rope_sin;         // [position][64]
+    // (In one place, as no launch has both: with 16 bytes more of arguments products of 129 .. 512 rows took 1.003 times as long with slabs, 1.002 without, means of 89 and 61 sizes)
+    union { int gu_ksplit, rope_cols; };
+    union { const half_t *norm_w, *rope_cos; };        // rope_cos, rope_sin: [position][64]
+    union { const float *norm_ss; const half_t *rope_sin; };
+    float norm_eps;
 };
 
 // p.seg[sg] without a load that waits for sg.  GLOBAL: the kernel stores through c (held_global); one that does not schedules its first loads better
